@@ -20,8 +20,8 @@
 // pre-activation z [T, H*d] in a buffer of its own.
 //
 // Two kernels, one workgroup per (head, sequence), thread c owns column c of the state: decode
-// steps stream the state through registers (read once, written once); portions keep it in
-// LDS and walk their tokens in chunks (the walk is sequential in time by the recurrence's
+// steps stream the state through registers (read once, written once); portions that the matrix-core
+// form (recurrent_chunk.hip) does not take keep it in LDS and walk their tokens in chunks (the walk is sequential in time by the recurrence's
 // per-channel decay; the gates and the norm of a chunk are computed in parallel).
 #include "common.h"
 

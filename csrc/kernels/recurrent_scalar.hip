@@ -15,6 +15,7 @@
 //     n_t . q_t = A_t (n_0 . q_t) + sum_{j <= t} b_j (prod_{j < i <= t} a_i) (k_j . q_t),
 //   A_t = prod_{i <= t} a_i, so the chunk's key-query products and the carried vector n_0 (LDS,
 //   updated once a chunk) give every token's normaliser in parallel, beside the walk.
+// Portions of both at the usual sizes run recurrent_chunk.hip instead.
 // FORM 2, retention: as FORM 0 without activations; the first `rot` dims of q and k rotate
 //   (dimension i with i + rot/2, by the step's table of cosines | sines), k times d^(-1/2); o_t
 //   is divided by its RMS per head and multiplied by silu(gate_t) -> S. Portions of more than

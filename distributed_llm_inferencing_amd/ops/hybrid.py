@@ -403,6 +403,30 @@ def window_attention(q, k_cache, v_cache, dq, dv, H, G, cu_seqlens, max_seqlen, 
     return out
 
 
+_CHUNK_HGRN2, _CHUNK_GLA, _CHUNK_FIXED, _CHUNK_MLSTM = range(4)
+# shortest step whose portions run 16 tokens at a time on the matrix cores (recurrent_chunk.hip)
+# instead of the token-by-token walk. 64 sequences, 32 heads of 128: at 8 tokens each the walk takes
+# 58 / 91 / 57 us (hgrn2 / gla / lightning) and a block 85 / 89 / 71; at 16 tokens 96 / 144 / 81 and
+# 87 / 92 / 73.
+CHUNK_MIN_TOKENS = 16
+
+
+def _recurrence_chunks(mode: int, proj, state, slots, cu_seqlens, positions, out, max_seqlen, H, d,
+                       dv, dtype, z=None, bias=None, lower=None, inv_tau=0.0, qscale=1.0,
+                       decays=None, if_b=None, cap=0.0, norm_w=None, eps=0.0, nstate=None,
+                       out_scale=1.0) -> bool:
+    """The chunk form of a recurrence over a step's portions, where it takes the sizes: heads of at
+    most 128 channels, normed ones of at most 128 columns. False: nothing was launched."""
+    if int(max_seqlen) < CHUNK_MIN_TOKENS or d > 128 or (dv > 128 and mode != _CHUNK_FIXED):
+        return False
+    _call("dli_recurrence_chunks", mode, _p(proj), proj.stride(0), _p(z),
+          z.stride(0) if z is not None else 0, _p(bias), _p(lower), float(inv_tau), float(qscale),
+          _p(decays), _p(if_b), float(cap), _p(norm_w), float(eps), _p(state), _p(nstate), _p(slots),
+          _p(cu_seqlens), _p(positions), _p(out), out.stride(0), float(out_scale),
+          cu_seqlens.shape[0] - 1, H, d, dv, _dt(dtype), _st())
+    return True
+
+
 def hgrn2(proj, f_bias, lower, norm_w, eps, state, slots, cu_seqlens, max_seqlen, positions,
           H, d, dv):
     dtype = norm_w.dtype
@@ -412,6 +436,9 @@ def hgrn2(proj, f_bias, lower, norm_w, eps, state, slots, cu_seqlens, max_seqlen
     T = proj.shape[0]
     S = cu_seqlens.shape[0] - 1
     out = torch.empty(T, H * dv, dtype=dtype, device=proj.device)
+    if _recurrence_chunks(_CHUNK_HGRN2, proj, state, slots, cu_seqlens, positions, out, max_seqlen,
+                          H, d, dv, dtype, bias=f_bias, lower=lower, norm_w=norm_w, eps=eps):
+        return out
     _call("dli_hgrn2", _p(proj), proj.stride(0), _p(f_bias), _p(lower), _p(norm_w), float(eps),
           _p(state), _p(slots), _p(cu_seqlens), _p(positions), _p(out), out.stride(0), S,
           int(max_seqlen), H, d, dv, _dt(dtype), _st())
@@ -650,6 +677,10 @@ def gla(proj, z, a_bias, tau: float, norm_w, eps, state, slots, cu_seqlens, max_
     T = proj.shape[0]
     S = cu_seqlens.shape[0] - 1
     out = torch.empty(T, H * dv, dtype=dtype, device=proj.device)
+    if _recurrence_chunks(_CHUNK_GLA, proj, state, slots, cu_seqlens, positions, out, max_seqlen, H,
+                          d, dv, dtype, z=z, bias=a_bias, inv_tau=1.0 / tau, qscale=d ** -0.5,
+                          norm_w=norm_w, eps=eps):
+        return out
     _call("dli_gla", _p(proj), proj.stride(0), _p(z), z.stride(0), _p(a_bias), float(1.0 / tau),
           float(d ** -0.5), _p(norm_w), float(eps), _p(state), _p(slots), _p(cu_seqlens),
           _p(positions), _p(out), out.stride(0), S, int(max_seqlen), H, d, dv, _dt(dtype), _st())
@@ -743,6 +774,9 @@ def lightning(proj, decays, state, slots, cu_seqlens, max_seqlen, positions, H, 
     T = proj.shape[0]
     S = cu_seqlens.shape[0] - 1
     out = torch.empty(T, H * dv, dtype=torch.float32, device=proj.device)
+    if _recurrence_chunks(_CHUNK_FIXED, proj, state, slots, cu_seqlens, positions, out, max_seqlen,
+                          H, d, dv, torch.float32, decays=decays):
+        return out
     _call("dli_scalar_recurrence", _p(proj), proj.stride(0), 0, _p(decays), None, 0.0, None, 0.0,
           _p(state), None, _p(slots), _p(cu_seqlens), _p(positions), _p(out), out.stride(0), 1.0,
           S, int(max_seqlen), H, d, dv, _column_block(S, H, d, dv, max_seqlen), None, 1, _st())
@@ -771,6 +805,10 @@ def mlstm(proj, if_b, cap: float, norm_w, eps: float, state, mstate, slots, cu_s
         return R.mlstm(proj, if_b, cap, norm_w, eps, state, mstate, slots, cu_seqlens, positions,
                        H, d, dv, out, out_scale)
     S = cu_seqlens.shape[0] - 1
+    if _recurrence_chunks(_CHUNK_MLSTM, proj, state, slots, cu_seqlens, positions, out, max_seqlen,
+                          H, d, dv, norm_w.dtype, qscale=d ** -0.5, if_b=if_b, cap=cap,
+                          norm_w=norm_w, eps=eps, nstate=mstate, out_scale=out_scale):
+        return out
     cw = _column_block(S, H, d, dv, max_seqlen)
     # with column blocks no workgroup sees a whole head: the read-outs leave in fp32 and the
     # per-head norm, gate and scale run as a row kernel

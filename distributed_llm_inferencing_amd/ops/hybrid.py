@@ -356,9 +356,8 @@ def window_attention(q, k_cache, v_cache, dq, dv, H, G, cu_seqlens, max_seqlen, 
     hg = int(bool(head_gate))
     if q.dtype == torch.bfloat16 and MFMA_ATTENTION:
         lib = N.require_native()
-        if (Gk == G and not chunk and slopes is None and talk is None and not head_gate
-                and sink is None and out_scale == 1.0):
-            # grouped-query attention, plain or with an elementwise output gate: the dedicated
+        if Gk == G and not chunk and slopes is None and talk is None:
+            # grouped-query attention, with or without output gate and sink: the dedicated
             # kernels (a few pairs of key and value widths)
             nb = lib.dli_swa_attention_workspace_bytes(S, int(max_seqlen), H, G, dv, int(window),
                                                        int(keep_first))
@@ -368,7 +367,8 @@ def window_attention(q, k_cache, v_cache, dq, dv, H, G, cu_seqlens, max_seqlen, 
                 v_cache.stride(0), _p(out), out.stride(0), _p(cu_seqlens), _p(positions),
                 _p(block_tables), block_tables.stride(0), block_size, S, int(max_seqlen), H, G, dq,
                 dv, int(window), int(keep_first), float(scale), _p(gate),
-                gate.stride(0) if gate is not None else 0, _p(ws), _st())
+                gate.stride(0) if gate is not None else 0, hg, _p(sink), float(out_scale), _p(ws),
+                _st())
             if rc == 0:
                 return out
             if rc != _NOT_SUPPORTED:

@@ -1,0 +1,49 @@
+"""Attention with a sink logit and a gate a head on the dedicated grouped-query kernels: decode rows
+(one and several key splits), short and long portions, against the reference in float64."""
+import pytest
+import torch
+
+from distributed_llm_inferencing_amd.ops import hybrid as H
+from distributed_llm_inferencing_amd.ops import reference as R
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,dv,G", [(128, 128, 2), (64, 64, 6)])
+@pytest.mark.parametrize("lens,before", [([1] * 9, [0, 1, 31, 32, 127, 300, 1500, 4000, 5]),
+                                         ([1] * 300, list(range(300))),      # one key split
+                                         ([17, 64, 191, 1, 2], [0, 70, 5, 40, 0]),
+                                         ([256, 192, 513, 3], [0, 100, 0, 700])])
+def test_sink_and_head_gate(gpu, d, dv, G, lens, before):
+    heads, block, scale = 6, 16, d ** -0.5
+    g = torch.Generator().manual_seed(sum(lens) + d)
+    S, T, ctx = len(lens), sum(lens), [a + b for a, b in zip(lens, before)]
+    W = max(-(-c // block) for c in ctx)
+    need = [-(-c // block) for c in ctx]
+    perm = torch.randperm(sum(need), generator=g).int()
+    bt, o = torch.zeros(S, W, dtype=torch.int32), 0
+    for s, n in enumerate(need):
+        bt[s, :n] = perm[o:o + n]
+        o += n
+    kc, vc = (torch.randn(sum(need) * block, G * w, generator=g).bfloat16() for w in (d, dv))
+    q = torch.randn(T, heads * d, generator=g).bfloat16()
+    gate = torch.randn(T, heads + 3, generator=g)[:, 1:1 + heads]
+    # far below and far above every score too: exp(sink) alone would leave fp32's range
+    sink = torch.tensor([-200.0, -3.0, 0.0, 2.0, 6.0, 300.0])
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist()).int()
+    pos = torch.cat([torch.arange(n) + b for n, b in zip(lens, before)]).int()
+    want = R.window_attention(q, kc, vc, d, dv, heads, G, cu, pos, bt, block, 1 << 30, scale,
+                              gate=gate, out_dtype=torch.float32, sink=sink, head_gate=True,
+                              out_scale=0.7).double()
+    wide = torch.zeros(T, heads * dv + 8, dtype=torch.bfloat16, device=gpu)
+    buf = torch.zeros(T, heads + 3, device=gpu)
+    buf[:, 1:1 + heads] = gate.to(gpu)
+    got = H.window_attention(q.to(gpu), kc.to(gpu), vc.to(gpu), d, dv, heads, G, cu.to(gpu), max(lens),
+                             pos.to(gpu), bt.to(gpu), block, max(ctx), scale, gate=buf[:, 1:1 + heads],
+                             sink=sink.to(gpu), head_gate=True, out_scale=0.7,
+                             out=wide[:, :heads * dv])
+    assert (wide[:, heads * dv:] == 0).all()
+    got = got.double().cpu()
+    assert torch.isfinite(got).all()
+    # weights and outputs rounded to bf16, half an ulp (2^-9) each
+    assert float((got - want).norm() / want.norm()) < 2 * 2.0 ** -9
+    assert float(got.view(T, heads, dv)[:, 5].abs().max()) < 1e-30        # the sink takes it all

@@ -17,6 +17,7 @@
 //                   the softmax is lane-local but for one exchange; K / V tiles of 64 keys by
 //                   LDS-DMA into three buffers, one barrier a tile; the list's cache rows looked
 //                   up once (LDS). The structure of attention_prefill.hip's long-prompt kernel.
+//                   Latent attention runs it too, expanded: [k_h | shared rotated key] rows of 192.
 //  * swa_prefill16  4 waves x 16 query rows: portions shorter than the above is worth
 //  * swa_decode     one query token a sequence: a workgroup per (sequence, kv head, key split).
 //                   Scores on the matrix cores with K rows straight from the cache (the heads
@@ -51,6 +52,12 @@ struct SwaArgs {
   int table_cap;                       // prefill32: list entries that fit the LDS table
   int nsplit;                          // decode: key splits
   float* ws;                           // decode, nsplit > 1: [nsplit][S][H][2], [nsplit][S][H][HD]
+  // shared tail of queries and keys (prefill32 with DR > 0): head h of token t has its DR dims at q2 +
+  // t * ldq2 + h * q2_head, a key row has them once for all heads; the key and value rows of sequence
+  // s are then rows cu_ctx[s] + position of plain matrices
+  const u16* q2; long ldq2; int q2_head;
+  const u16* k2; long k2_stride;
+  const int* cu_ctx;
 };
 
 // floats of the decode splits' (max, sum) pairs, in front of their partial sums
@@ -92,10 +99,10 @@ constexpr float RESCALE_THR = 8.f;     // log2 units: the running max moves only
 
 // One tile of rows (D wide) by LDS-DMA: 1-KiB pieces of two subtiles in a row, wave w of 8 takes
 // pieces w, w + 8, ... The DMA writes lane-linearly, so each lane loads the logical chunk that
-// lands at its place.
-template <int D, typename RowOf>
-__device__ __forceinline__ void stage_rows(const u16* src, long stride, char* dst, int x0, int wid,
-                                           int lane, const RowOf& row_of) {
+// lands at its place. Columns from D1 on come from a second matrix (its rows alike).
+template <int D, int D1, typename RowOf>
+__device__ __forceinline__ void stage_rows(const u16* src, long stride, const u16* src2, long stride2,
+                                           char* dst, int x0, int wid, int lane, const RowOf& row_of) {
   constexpr int NP = D / 8;
 #pragma unroll
   for (int j = 0; j < (NP + 7) / 8; ++j) {
@@ -105,19 +112,20 @@ __device__ __forceinline__ void stage_rows(const u16* src, long stride, char* ds
     const int rg = b / (D * 16), in = b % (D * 16);
     const int r = 8 * rg + ((lane & 31) >> 2);
     const int c = 4 * (in / 512) + ((lane & 3) ^ ((r >> 2) & 3));
-    const u16* p = src + row_of(x0 + r) * stride + c * 8;
+    const long row = row_of(x0 + r);
+    const u16* p = D1 < D && c * 8 >= D1 ? src2 + row * stride2 + (c * 8 - D1) : src + row * stride + c * 8;
     __builtin_amdgcn_global_load_lds((gbl_void*)p, (lds_void*)(dst + piece * 1024), 16, 0, 0);
   }
 }
 
 // Tile image: 8-row x 32-column subtiles of 512 B with the chunks of a row rotated by its row
-// group: conflict-free for row reads and for transposed reads. DK, DV: multiples of 32.
-template <int DK, int DV>
+// group: conflict-free for row reads and for transposed reads. DK, DR, DV: multiples of 32.
+template <int DK, int DR, int DV>
 __global__ void __launch_bounds__(512) swa_prefill32_kernel(SwaArgs a) {
-  constexpr int KC = DK / 16, DBK = DV / 32;
-  constexpr int RGK = DK * 16, RGV = DV * 16;                  // bytes of an 8-row group
-  constexpr int TILE_K = KT * DK * 2, TILE_B = KT * (DK + DV) * 2, NBUF = 3;
-  constexpr int NPK = DK / 8, NPV = DV / 8;                    // 1-KiB pieces of a tile
+  constexpr int KW = DK + DR, KC = KW / 16, DBK = DV / 32;
+  constexpr int RGK = KW * 16, RGV = DV * 16;                  // bytes of an 8-row group
+  constexpr int TILE_K = KT * KW * 2, TILE_B = KT * (KW + DV) * 2, NBUF = 3;
+  constexpr int NPK = KW / 8, NPV = DV / 8;                    // 1-KiB pieces of a tile
   extern __shared__ __attribute__((aligned(16))) char lds[];   // [NBUF][K tile | V tile], slot table
   int* table = (int*)(lds + NBUF * TILE_B);
   const int s = blockIdx.y, h = blockIdx.z;
@@ -134,21 +142,24 @@ __global__ void __launch_bounds__(512) swa_prefill32_kernel(SwaArgs a) {
   const int kvh = h / (a.H / a.G);
   const KeyList kl(p0 + wg_q0, p0 + min(wg_q0 + LROWS, len) - 1, a.window, a.keep);
   const int ntiles = (kl.n + KT - 1) / KT;
-  const int* bt = a.block_tables + (long)s * a.bt_stride;
+  const int* bt = DR ? nullptr : a.block_tables + (long)s * a.bt_stride;
+  const int base = DR ? a.cu_ctx[s] : 0;
   const auto row_of = [&](int x) {
     const int j = kl.key(x);
-    return bt[j / a.block_size] * a.block_size + j % a.block_size;
+    return DR ? base + j : bt[j / a.block_size] * a.block_size + j % a.block_size;
   };
-  const bool use_table = kl.n <= a.table_cap;
+  const bool use_table = !DR && kl.n <= a.table_cap;
   if (use_table)
     for (int x = tid; x < kl.n; x += 512) table[x] = row_of(x);
 
   bf16x8 qf[KC];
   {
-    const u16* qp = a.q + (long)(t0 + min(q0 + qc, len - 1)) * a.ldq + (long)h * DK + 8 * hi;
+    const long qt = t0 + min(q0 + qc, len - 1);
+    const u16* qp = a.q + qt * a.ldq + (long)h * DK + 8 * hi;
+    const u16* qp2 = DR ? a.q2 + qt * a.ldq2 + (long)h * a.q2_head + 8 * hi : nullptr;
 #pragma unroll
     for (int c = 0; c < KC; ++c) {
-      const uint4 v = *reinterpret_cast<const uint4*>(qp + 16 * c);
+      const uint4 v = *reinterpret_cast<const uint4*>(16 * c < DK ? qp + 16 * c : qp2 + (16 * c - DK));
       qf[c] = *reinterpret_cast<const bf16x8*>(&v);
     }
   }
@@ -168,8 +179,8 @@ __global__ void __launch_bounds__(512) swa_prefill32_kernel(SwaArgs a) {
   };
   const auto stage = [&](int buf, int x0) {
     char* kd = lds + buf * TILE_B;
-    stage_rows<DK>(a.k + kvh * DK, a.k_stride, kd, x0, wid, lane, row_in_list);
-    stage_rows<DV>(a.v + kvh * DV, a.v_stride, kd + TILE_K, x0, wid, lane, row_in_list);
+    stage_rows<KW, DK>(a.k + kvh * DK, a.k_stride, a.k2, a.k2_stride, kd, x0, wid, lane, row_in_list);
+    stage_rows<DV, DV>(a.v + kvh * DV, a.v_stride, nullptr, 0, kd + TILE_K, x0, wid, lane, row_in_list);
   };
   const auto wait_one_tile = [&]() {                           // all but the youngest tile landed
     constexpr int LO = NPK / 8 + NPV / 8, RK = NPK % 8, RV = NPV % 8;
@@ -678,6 +689,25 @@ int decode_splits(int num_seqs, int H, int G, long keys) {
 // key / value widths this file is built for
 #define SWA_WIDTHS(F) F(64, 64) F(128, 128) F(64, 128) F(96, 192) F(128, 256)
 
+template <int DK, int DR, int DV>
+int launch_prefill32(SwaArgs a, int num_seqs, int max_seqlen, hipStream_t st) {
+  const long list = (long)a.window + LROWS + a.keep;
+  constexpr int TILES = 3 * KT * (DK + DR + DV) * 2;
+  a.table_cap = !DR && list <= 6144 && TILES + list * 4 + 16 <= 160 * 1024 ? (int)list : 0;
+  const int sh = TILES + a.table_cap * 4 + 16;
+  static bool raised = false;
+  if (!raised) {
+    const hipError_t e = hipFuncSetAttribute((const void*)swa_prefill32_kernel<DK, DR, DV>,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             160 * 1024);
+    if (e != hipSuccess) return (int)e;
+    raised = true;
+  }
+  dim3 grid((max_seqlen + LROWS - 1) / LROWS, num_seqs, a.H);
+  swa_prefill32_kernel<DK, DR, DV><<<grid, 512, sh, st>>>(a);
+  DLI_RETURN_LAUNCH();
+}
+
 template <int DK, int DV>
 int launch_swa(SwaArgs a, int num_seqs, int max_seqlen, hipStream_t st) {
   if (max_seqlen == 1) {
@@ -696,24 +726,62 @@ int launch_swa(SwaArgs a, int num_seqs, int max_seqlen, hipStream_t st) {
     swa_prefill16_kernel<DK, DV><<<grid, 256, 0, st>>>(a);
     DLI_RETURN_LAUNCH();
   }
-  const long list = (long)a.window + LROWS + a.keep;
-  constexpr int TILES = 3 * KT * (DK + DV) * 2;
-  a.table_cap = list <= 6144 && TILES + list * 4 + 16 <= 160 * 1024 ? (int)list : 0;
-  const int sh = TILES + a.table_cap * 4 + 16;
-  static bool raised = false;
-  if (!raised) {
-    const hipError_t e = hipFuncSetAttribute((const void*)swa_prefill32_kernel<DK, DV>,
-                                             hipFuncAttributeMaxDynamicSharedMemorySize,
-                                             160 * 1024);
-    if (e != hipSuccess) return (int)e;
-    raised = true;
+  return launch_prefill32<DK, 0, DV>(a, num_seqs, max_seqlen, st);
+}
+
+
+// Rows cu_ctx[s] + j of out <- the cache row of position j of sequence s, `chunks` 16-byte pieces each
+__global__ void __launch_bounds__(256) gather_rows_kernel(uint4* out, const uint4* cache,
+                                                          const int* cu_ctx, const int* block_tables,
+                                                          int bt_stride, int block_size, int chunks) {
+  const int s = blockIdx.y, o0 = cu_ctx[s], n = cu_ctx[s + 1] - o0;
+  const int* bt = block_tables + (long)s * bt_stride;
+  const int j0 = blockIdx.x * 64, rows = min(64, n - j0);
+  for (int i = threadIdx.x; i < rows * chunks; i += 256) {
+    const int j = j0 + i / chunks, c = i % chunks;
+    const long row = (long)bt[j / block_size] * block_size + j % block_size;
+    out[(long)(o0 + j) * chunks + c] = cache[row * chunks + c];
   }
-  dim3 grid((max_seqlen + LROWS - 1) / LROWS, num_seqs, a.H);
-  swa_prefill32_kernel<DK, DV><<<grid, 512, sh, st>>>(a);
-  DLI_RETURN_LAUNCH();
 }
 
 }  // namespace
+
+// The cached rows (width bf16 elements, a multiple of 8) of every sequence's context, in order
+extern "C" int dli_gather_context(void* out, const void* cache, int width, const int* cu_ctx,
+                                  const int* block_tables, int bt_stride, int block_size, int num_seqs,
+                                  int max_context, hipStream_t st) {
+  if (num_seqs <= 0 || max_context <= 0) return 0;
+  if (width < 8 || width % 8 || block_size < 1 || num_seqs > 65535 ||
+      (((uintptr_t)out | (uintptr_t)cache) & 15))
+    return (int)hipErrorInvalidValue;
+  dim3 grid((max_context + 63) / 64, num_seqs);
+  gather_rows_kernel<<<grid, 256, 0, st>>>((uint4*)out, (const uint4*)cache, cu_ctx, block_tables,
+                                           bt_stride, block_size, width / 8);
+  DLI_RETURN_LAUNCH();
+}
+
+// Portions whose keys share their last dr dims (latent attention, expanded): q [T, H*dk] and its tail
+// q2 (row stride ldq2, head stride q2_head); k and v are rows cu_ctx[s] + position of matrices with one
+// column block a head, k2 [.., dr] of a third. hipErrorNotSupported (801): widths or alignment that this
+// form does not take.
+extern "C" int dli_shared_tail_attention(const void* q, int ldq, const void* q2, long ldq2, int q2_head,
+                                         const void* k, long k_stride, const void* k2, long k2_stride,
+                                         const void* v, long v_stride, void* out, int ldo, const int* cu,
+                                         const int* positions, const int* cu_ctx, int num_seqs,
+                                         int max_seqlen, int H, int dk, int dr, int dv, int window,
+                                         float scale, const float* gate, int ldg, hipStream_t st) {
+  if (num_seqs <= 0 || max_seqlen <= 0) return 0;
+  if (H < 1 || window < 1 || cu_ctx == nullptr) return (int)hipErrorInvalidValue;
+  const bool aligned = (((uintptr_t)q | (uintptr_t)q2 | (uintptr_t)k | (uintptr_t)k2 | (uintptr_t)v) & 15) == 0 &&
+                       (uintptr_t)out % 8 == 0 && ldq % 8 == 0 && ldq2 % 8 == 0 && q2_head % 8 == 0 &&
+                       k_stride % 8 == 0 && k2_stride % 8 == 0 && v_stride % 8 == 0 && ldo % 4 == 0;
+  if (!aligned || !(scale > 0.f) || num_seqs > 65535 || H > 65535 || dk != 128 || dr != 64 || dv != 128)
+    return (int)hipErrorNotSupported;
+  SwaArgs a{(const u16*)q, ldq, (const u16*)k, k_stride, (const u16*)v, v_stride, (u16*)out, ldo,
+            gate, ldg, gate != nullptr, nullptr, 1.f, cu, positions, nullptr, 0, 1, H, H, window, 0,
+            scale * LOG2E, 0, 1, nullptr, (const u16*)q2, ldq2, q2_head, (const u16*)k2, k2_stride, cu_ctx};
+  return launch_prefill32<128, 64, 128>(a, num_seqs, max_seqlen, st);
+}
 
 // Workspace bytes of a decode step (0: not split over keys)
 extern "C" long dli_swa_attention_workspace_bytes(int num_seqs, int max_seqlen, int H, int G,
@@ -745,7 +813,7 @@ extern "C" int dli_swa_attention(const void* q, int ldq, const void* k, long k_s
     return (int)hipErrorNotSupported;
   SwaArgs a{(const u16*)q, ldq, (const u16*)k, k_stride, (const u16*)v, v_stride, (u16*)out, ldo,
             gate, ldg, head_gate != 0, sink, out_scale, cu, positions, block_tables, bt_stride, block_size, H, G, window, keep,
-            scale * LOG2E, 0, 1, (float*)ws};
+            scale * LOG2E, 0, 1, (float*)ws, nullptr, 0, 0, nullptr, 0, nullptr};
   if (max_seqlen == 1) {
     a.nsplit = decode_splits(num_seqs, H, G, (long)window + keep);
     if (a.nsplit > 1 && ws == nullptr) return (int)hipErrorInvalidValue;

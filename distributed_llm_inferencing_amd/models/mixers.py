@@ -34,6 +34,11 @@ class StepView:
     block_size: int
     state_slots: Optional[torch.Tensor]   # [S] int32 recurrent-state slot (-1: padding row)
     max_context: int = 1 << 30      # no position of this step is at or beyond this
+    # of a prefill step (``DeviceBatch``): cumulative context lengths [S+1] int32, their sum, and the
+    # pairs of a new token and a position before it; unknown without the first
+    cu_context: Optional[torch.Tensor] = None
+    total_context: int = 0
+    context_pairs: int = 0
     tables: dict = field(default_factory=dict)      # rotation tables made so far in this step
 
     def rotation(self, spec: LayerSpec, lp: dict):
@@ -59,6 +64,12 @@ def derive_constants(spec: LayerSpec, lp: dict, device) -> None:
         # float64: the angle position * frequency is formed in double and rounded once
         i = torch.arange(spec.rot_dims // 2, dtype=torch.float64)
         lp["inv_freq"] = torch.pow(spec.rot_base, -2.0 * i / max(1, spec.rot_dims)).to(device)
+        w = lp["w_ukT"]
+        if w.is_cuda and H.expanded_latent_ok(w.dtype, spec.dim, spec.rot_dim, spec.vdim, spec.kv_rank):
+            # every head's W_uk over every head's W_uv, [1, H (d + dv), r]: expands cached latents
+            # (a batch of one: not among the matrices that a decode step's plans are made for)
+            lp["w_ukv"] = torch.cat([w.transpose(1, 2).reshape(-1, spec.kv_rank),
+                                     lp["w_uv"].reshape(-1, spec.kv_rank)]).unsqueeze(0).contiguous()
     elif spec.kind == "talk_attention":
         lp["talk"] = lp["talk"].float().contiguous()
     elif spec.kind == "lightning":
@@ -149,8 +160,9 @@ def latent_attention_mixer(spec: LayerSpec, lp: dict, h, step: StepView, cache, 
     key are cached. With k_h = W_uk,h c and v_h = W_uv,h c,
         q_h . k_h = (W_uk,h^T q_h) . c      and      sum_j w_j v_h,j = W_uv,h (sum_j w_j c_j),
     so every head attends the same cached row [c | k_rot] with the query [W_uk,h^T q_h | q_rot]
-    and its output is expanded afterwards: one multi-query attention over the latent, for
-    prompts and decoding alike, and no per-step expansion of the window's keys."""
+    and its output is expanded afterwards: one multi-query attention over the latent. Steps with
+    enough new tokens for their context (``H.latent_expansion_pays``) expand k_h and v_h of the whole
+    context instead: the pairs of a query and a key cost 3.4 times less then."""
     Hh, d, dr, dv, r = spec.heads, spec.dim, spec.rot_dim, spec.vdim, spec.kv_rank
     (c,) = cache
     T = h.shape[0]
@@ -173,10 +185,17 @@ def latent_attention_mixer(spec: LayerSpec, lp: dict, h, step: StepView, cache, 
     else:                                   # fp32 [T, q heads | ckv | k_rot]
         q_nope, q_full = H.mla_prepare(proj, lp["c_norm"], eps, Hh, d, dr, r, spec.rot_dims,
                                        lp["inv_freq"], step.positions, step.slot_mapping, c)
-    H.head_linear(q_nope, lp["w_ukT"], q_full)               # q_full[:, h, :r] = W_uk,h^T q_h
     # a window no shorter than the step's longest context masks nothing: the tight bound lets
     # the kernel size its slot table and key splits for the keys that exist
     win = min(spec.window, max(1, step.max_context))
+    if ("w_ukv" in lp and step.cu_context is not None and H.latent_expansion_pays(
+            T, step.max_seqlen, step.total_context, step.context_pairs, Hh * (d + dv))):
+        o = H.expanded_latent_attention(q_nope, q_full[:, :, r:], c, lp["w_ukv"][0], Hh, r,
+                                        step.cu_seqlens, step.max_seqlen, step.positions,
+                                        step.block_tables, step.block_size, step.cu_context,
+                                        step.total_context, step.max_context, win, spec.scale, gates)
+        return H.linear_any(o, lp["wo"])
+    H.head_linear(q_nope, lp["w_ukT"], q_full)               # q_full[:, h, :r] = W_uk,h^T q_h
     ol = H.window_attention(q_full.view(T, Hh * (r + dr)), c, c, r + dr, r, Hh, 1,
                             step.cu_seqlens, step.max_seqlen, step.positions,
                             step.block_tables, step.block_size, win, spec.scale)

@@ -403,6 +403,46 @@ def window_attention(q, k_cache, v_cache, dq, dv, H, G, cu_seqlens, max_seqlen, 
     return out
 
 
+# ----------------------------------------------------------------------------- latent attention, expanded
+def expanded_latent_ok(dtype, d: int, dr: int, dv: int, r: int) -> bool:
+    """Whether the expanded form takes these widths."""
+    return dtype == torch.bfloat16 and (d, dr, dv) == (128, 64, 128) and r % 64 == 0
+
+
+def latent_expansion_pays(tokens: int, max_seqlen: int, context: int, pairs: int, width: int) -> bool:
+    """Whether a step expands the context's keys and values (``width`` columns of them) instead of
+    attending the latent itself: ``context`` rows to expand, some 14 ns each at width 8192, against
+    0.44 ns for each of ``pairs`` (a key and a row of the absorbed kernel, which takes a sequence's
+    rows 16 at a time) and 75 ns a token for absorbing its query and expanding its output. A layer of
+    32 heads, absorbed -> expanded: 4 x 2048 tokens 5.6 -> 1.2 ms, 32 x 64 0.48 -> 0.31, 512 tokens
+    at 4096 1.04 -> 0.37, 512 beside 64 single ones at 1000 10.3 -> 1.6; 64 at 4096 0.23 -> 0.26."""
+    if max_seqlen < 64 or (max_seqlen < 96 and context > 8 * tokens) or context * width > 1 << 30:
+        return False
+    return 14 * context < 75 * tokens + 0.44 * pairs
+
+
+def expanded_latent_attention(q, q_rot, cache, w_ukv, H, r, cu_seqlens, max_seqlen, positions,
+                              block_tables, block_size, cu_context, context, max_context, window,
+                              scale, gates=None) -> torch.Tensor:
+    """Latent attention over portions with keys and values expanded from the cached rows [latent r |
+    shared rotated key]: q [T, H, d] and its rotated tails q_rot [T, H, dr] (rows of a wider buffer),
+    w_ukv [H (d + dv), r]; sigmoid(gates [T, H]) multiplies the heads. -> [T, H*dv] in q's dtype."""
+    T, _, d = q.shape
+    dr, dv = q_rot.shape[2], w_ukv.shape[0] // H - d
+    rows = torch.empty(context, r + dr, dtype=q.dtype, device=q.device)
+    _call("dli_gather_context", _p(rows), _p(cache), r + dr, _p(cu_context), _p(block_tables),
+          block_tables.stride(0), block_size, cu_seqlens.shape[0] - 1, int(max_context), _st())
+    kv = linear_any(rows[:, :r], w_ukv, out_f32=False)
+    out = torch.empty(T, H * dv, dtype=q.dtype, device=q.device)
+    k_rot, v = rows[:, r:], kv[:, H * d:]
+    _call("dli_shared_tail_attention", _p(q), q.stride(0), _p(q_rot), q_rot.stride(0),
+          q_rot.stride(1), _p(kv), kv.stride(0), _p(k_rot), k_rot.stride(0), _p(v), kv.stride(0),
+          _p(out), out.stride(0), _p(cu_seqlens), _p(positions), _p(cu_context),
+          cu_seqlens.shape[0] - 1, int(max_seqlen), H, d, dr, dv, int(window), float(scale),
+          _p(gates), gates.stride(0) if gates is not None else 0, _st())
+    return out
+
+
 _CHUNK_HGRN2, _CHUNK_GLA, _CHUNK_FIXED, _CHUNK_MLSTM = range(4)
 # shortest step whose portions run 16 tokens at a time on the matrix cores (recurrent_chunk.hip)
 # instead of the token-by-token walk. 64 sequences, 32 heads of 128: at 8 tokens each the walk takes

@@ -17,6 +17,7 @@ up before hipGraph capture so no allocation happens inside a capture.
 """
 from __future__ import annotations
 
+import functools
 import math
 import os
 import threading
@@ -152,12 +153,13 @@ def workspace(device: torch.device, nbytes: int) -> torch.Tensor:
 LARGE_M = 1024
 
 
+@functools.lru_cache(maxsize=8192)
 def _heuristic(M: int, N: int, K: int, epi: str) -> GemmPlan:
     """Fitted to profiles/r1_gemm/gemm_bench.json and profiles/r1_gemm8p/ (MI355X, random
     bf16 operands): skinny decode GEMMs (M <= 512) on the 2/3-stage tiles below (autotuned
-    at capture); fat prefill GEMMs (M >= LARGE_M) on the 256x256 8-phase ping-pong kernel
-    (tile 22) with its fused epilogue (SiLU*up, bias+GELU, fp32); the prefill autotune
-    (``prefill_candidates``) may pin the 4-wave tile instead."""
+    at capture); fat prefill GEMMs (M >= LARGE_M) on the 256x256 kernels, the 8-phase ping-pong one
+    (tile 22) or the persistent 4-wave one (tile 55), with their fused epilogues (SiLU*up, bias+GELU,
+    fp32); the prefill autotune (``prefill_candidates``) measures them per bucket."""
     # M > 512: mixed prefill+decode steps of a full batch and prefill — 256x256 8-phase
     # tiles (the 128-row tiles below ran a 512 + 300-token mixed step's GEMMs ~2.5x slower
     # than the tuned decode step: 26.7 ms per mixed step end to end, profiles/r3/e2e/)
@@ -166,11 +168,25 @@ def _heuristic(M: int, N: int, K: int, epi: str) -> GemmPlan:
         # most CUs idle on the N = 4096 / 6144 projections (M = 1200: 80 / 120 tiles), so
         # split K while the grid stays within one wave of the chip
         tiles = -(-M // 256) * -(-N // 256)
+        if (epi == "f32" and tiles * 2 <= NUM_CUS and K <= 6144
+                and -(-M // 256) * -(-N // 128) > NUM_CUS // 2):
+            # half-width tiles fill the chip without a split and its reduce over fp32 slabs: M = 1100 /
+            # 1536, N = K = 4096: 60 / 62 us against 78 / 80 unsplit
+            return GemmPlan("dli", 28, 1)
         splits = 1
-        if epi in ("none", "splitk"):
+        if epi in ("none", "splitk", "f32"):
+            # (f32, M = 1100, N = 4096, K = 14336: 240 us unsplit, 153 in two)
             while (tiles * splits * 2 <= NUM_CUS and K % (64 * splits * 2) == 0
                    and K // (splits * 2) >= 1024 and splits < 4):
                 splits *= 2
+        # the persistent kernel hides a tile's prologue and epilogue, which counts for short K: 8192
+        # rows, K = 4096: N = 4096 / 6144 / 12288 / 28672 in 185 / 274 / 556 / 1284 us against 192 / 288 /
+        # 582 / 1337; at K = 14336 it is 5 % ahead for 1536 to 3000 rows (251 against 267) and 4 % behind
+        # from 4096 on (643 against 619 at 8192). 16384 rows: 2538 against 2672 at N = 28672, within 2 %
+        # at 6144
+        if (splits == 1 and M >= LARGE_M and K % 128 == 0 and (K <= 8192 or M < 4096)
+                and (M < 16384 or N >= 16384) and tile_ok(55, epi)):
+            return GemmPlan("dli", 55, 1)
         return GemmPlan("dli", 22, splits)
     if epi == "res":
         # residual-adding GEMV (full K): 4 rows a workgroup, 8 K-steps in flight per lane
@@ -195,7 +211,9 @@ def _heuristic(M: int, N: int, K: int, epi: str) -> GemmPlan:
     elif M <= 256:
         tile = 1 if N <= 8192 else 2
     else:
-        tile = 2
+        # (the last rows of a prefill wave through the head, M = 512, N = 128256: 513 us on 256x256
+        # tiles, 630 on 128x128)
+        tile = 22 if -(-M // 256) * -(-N // 256) >= 2 * NUM_CUS else 2
     bm, bn = TILES[tile]
     tiles = -(-M // bm) * -(-N // bn)
     splits = 1
@@ -306,12 +324,9 @@ def _bucket(M: int) -> int:
 
 def plan(M: int, N: int, K: int, epi: str) -> GemmPlan:
     key = (_bucket(M), N, K, epi)
-    p = _plan_cache.get(key)
-    if p is not None:
-        return p
-    p = _heuristic(M, N, K, epi)
-    _plan_cache[key] = p
-    return p
+    # tuned and pinned plans by bucket; a fitted one by its own M (a bucket of prefill sizes spans a
+    # factor of two, in which the best split differs)
+    return _plan_cache.get(key) or _heuristic(M, N, K, epi)
 
 
 def set_plan(M: int, N: int, K: int, epi: str, p: GemmPlan) -> None:
@@ -497,8 +512,10 @@ def prefill_candidates(M: int, N: int, K: int, epi: str):
     two-barrier schedule) at the same split, 1-4 % apart on the square / QKV / gate-up /
     down prefill shapes (profiles/r4/gemm4w/), measured per shape and bucket. At these sizes
     the GEMM is MFMA-bound, so the autotuner times them warm (``cold_bytes`` 1)."""
-    out = [_heuristic(M, N, K, epi)]
-    base = out[0]
+    base = _heuristic(M, N, K, epi)
+    if base.tile == 55:                  # (its 8-phase and 4-wave counterparts)
+        base = GemmPlan("dli", 22, 1)
+    out = [base]
     if base.tile == 22 and PREFILL_4W_TILE > 0:
         out.append(GemmPlan("dli", PREFILL_4W_TILE, base.splits))
     if base.tile == 22 and base.splits == 1 and K % 128 == 0 and PREFILL_PERSIST:

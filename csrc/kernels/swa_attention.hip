@@ -4,7 +4,7 @@
 // mixing — those run window_attention_mfma.hip). The sink and the head's gate only touch the epilogue
 // and cost nothing: 5 prompts of 900 to 2601 tokens, 32 heads of 128 on 8 kv heads, took 2.12 ms in
 // window_attention_mfma.hip (16 queries x 8 heads a workgroup, barrier-separated phases) and take
-// 0.34 ms here; decode of 64 rows at 984 keys 59 us instead of 252.
+// 0.25 ms here; decode of 64 rows at 984 keys 59 us instead of 252.
 // Position i sees j <= i with i - j < window or j < keep.
 //
 // The keys that a group of queries can see are at most two runs, [0, kf) and [lo, last], walked
@@ -128,18 +128,21 @@ __global__ void __launch_bounds__(512) swa_prefill32_kernel(SwaArgs a) {
   constexpr int NPK = KW / 8, NPV = DV / 8;                    // 1-KiB pieces of a tile
   extern __shared__ __attribute__((aligned(16))) char lds[];   // [NBUF][K tile | V tile], slot table
   int* table = (int*)(lds + NBUF * TILE_B);
-  const int s = blockIdx.y, h = blockIdx.z;
+  // key heads fastest, then the query heads of a group, then row blocks, longest lists first
+  // (attention_prefill.hip's order): 5 prompts of 900 to 2601 tokens, 32 heads of 128 on 8 kv heads,
+  // 339 -> 250 us; expanded latent heads, 6 prompts of 301 to 3000, 416 -> 278
+  const int s = blockIdx.y, kvh = blockIdx.x % a.G, rep = a.H / a.G;
+  const int h = kvh * rep + blockIdx.x / a.G % rep;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int qc = lane & 31, hi = lane >> 5;
   const int t0 = a.cu[s], len = a.cu[s + 1] - t0;
-  const int blk = (int)(gridDim.x - 1 - blockIdx.x);           // longest lists first
+  const int blk = (int)((gridDim.x - 1 - blockIdx.x) / a.H);
   const int wg_q0 = blk * LROWS;
   if (wg_q0 >= len) return;                                    // workgroup-uniform
   const int p0 = a.positions[t0];
   const int q0 = wg_q0 + wid * 32;
   const bool active = q0 < len;
-  const int kvh = h / (a.H / a.G);
   const KeyList kl(p0 + wg_q0, p0 + min(wg_q0 + LROWS, len) - 1, a.window, a.keep);
   const int ntiles = (kl.n + KT - 1) / KT;
   const int* bt = DR ? nullptr : a.block_tables + (long)s * a.bt_stride;
@@ -703,7 +706,7 @@ int launch_prefill32(SwaArgs a, int num_seqs, int max_seqlen, hipStream_t st) {
     if (e != hipSuccess) return (int)e;
     raised = true;
   }
-  dim3 grid((max_seqlen + LROWS - 1) / LROWS, num_seqs, a.H);
+  dim3 grid((max_seqlen + LROWS - 1) / LROWS * a.H, num_seqs);
   swa_prefill32_kernel<DK, DR, DV><<<grid, 512, sh, st>>>(a);
   DLI_RETURN_LAUNCH();
 }

@@ -22,9 +22,13 @@ enum { EPI_BF16 = 0, EPI_F32 = 1, EPI_SILU = 2, EPI_BIAS_GELU = 3, EPI_BIAS = 4,
        // clamp(up, -L, L); `bias` points to the fp32 constant L on the device
        EPI_CLAMP = 7,
        // relu(gate) * up over the interleaved gate/up weight
-       EPI_RELU = 8 };
+       EPI_RELU = 8,
+       // tanh-approximate gelu(gate) * up over the interleaved gate/up weight
+       EPI_GELU_MUL = 9 };
 // epilogues that pair a gate block with the up block beside it (output width N / 2)
-constexpr bool epi_pairs(int epi) { return epi == EPI_SILU || epi == EPI_CLAMP || epi == EPI_RELU; }
+constexpr bool epi_pairs(int epi) {
+  return epi == EPI_SILU || epi == EPI_CLAMP || epi == EPI_RELU || epi == EPI_GELU_MUL;
+}
 
 typedef __attribute__((address_space(3))) void lds_void;
 typedef const __attribute__((address_space(1))) void gbl_void;
@@ -210,7 +214,8 @@ __device__ __forceinline__ float clamp_swish_f(float g, float u, float lim) {
 }
 template <int EPI> __device__ __forceinline__ float pair_f(float g, float u, float lim) {
   return EPI == EPI_CLAMP ? clamp_swish_f(g, u, lim)
-                          : EPI == EPI_RELU ? fmaxf(g, 0.f) * u : silu_f(g) * u;
+                          : EPI == EPI_RELU ? fmaxf(g, 0.f) * u
+                          : EPI == EPI_GELU_MUL ? gelu_f(g) * u : silu_f(g) * u;
 }
 // the constant of a pairing epilogue
 template <int EPI> __device__ __forceinline__ float pair_const(const u16* bias) {
@@ -320,6 +325,7 @@ int gemm_4w_set_slab_store(int mode);
 #define DLI_EPI_SWITCH_S16(FN)                                                     \
   if (epi == EPI_CLAMP) return FN<EPI_CLAMP>(tile_cfg, DLI_GEMM_PASS);             \
   if (epi == EPI_RELU) return FN<EPI_RELU>(tile_cfg, DLI_GEMM_PASS);               \
+  if (epi == EPI_GELU_MUL) return FN<EPI_GELU_MUL>(tile_cfg, DLI_GEMM_PASS);       \
   if (epi == EPI_SLAB16) {                                                         \
     if (C != nullptr || splits < 2) return (int)hipErrorInvalidValue;              \
     return FN<EPI_SLAB16>(tile_cfg, DLI_GEMM_PASS);                                \

@@ -6,6 +6,7 @@ int gemm_tiles_pairs_dispatch(int epi, int tile_cfg, DLI_GEMM_ARGS) {
     case EPI_SILU: return dispatch_tiles<EPI_SILU>(tile_cfg, DLI_GEMM_PASS);
     case EPI_CLAMP: return dispatch_tiles<EPI_CLAMP>(tile_cfg, DLI_GEMM_PASS);
     case EPI_RELU: return dispatch_tiles<EPI_RELU>(tile_cfg, DLI_GEMM_PASS);
+    case EPI_GELU_MUL: return dispatch_tiles<EPI_GELU_MUL>(tile_cfg, DLI_GEMM_PASS);
     default: return DLI_NOT_MINE;
   }
 }

@@ -245,7 +245,7 @@ __device__ __forceinline__ float act_pair(int kind, float g, float u, float limi
     return g / (1.f + expf(-1.702f * g)) * (u + 1.f);
   }
   if (kind == 6) return fmaxf(g, 0.f) * u;
-  if (kind == 0) return gelu_tanh32(g) * u;
+  if (kind == 0 || kind == 7) return gelu_tanh32(g) * u;
   if (kind == 1) return g / (1.f + expf(-g)) * u;
   if (kind == 3) return 0.5f * g * (1.f + erff(g * 0.7071067811865476f));
   if (kind == 4) return g;
@@ -255,7 +255,8 @@ __device__ __forceinline__ float act_pair(int kind, float g, float u, float limi
 // kind 0: gelu_tanh(gu[:, c]) * gu[:, F + c]; 1: silu(..) * ..; 2: gelu_tanh(gu[:, c]);
 // 3: the exact (erf) GELU of gu[:, c]; 4: gu[:, c] itself (a rounding copy of a column slice);
 // 5: g sigmoid(1.702 g) (u + 1) with g = min(gu[:, c], limit), u = clamp(gu[:, F + c], +-limit);
-// 6: relu(gu[:, c]) * gu[:, F + c].
+// 6: relu(gu[:, c]) * gu[:, F + c]; 7: as 0 over a projection by the interleaved weight (16 gate, 16 up
+// columns in turn).
 // nrows (nullable, device): rows from *nrows on hold no data and are skipped.
 // I: the projection's type (fp32, or bf16 bits when a tuned GEMM wrote it).
 template <typename I> __device__ __forceinline__ f32x4 ldin4(const I* p);
@@ -268,6 +269,10 @@ template <> __device__ __forceinline__ f32x4 ldin4<u16>(const u16* p) {
                __uint_as_float(b.y << 16), __uint_as_float(b.y & 0xffff0000u)};
 }
 
+// columns of feature c's gate and up values in a projection row
+__device__ __forceinline__ int gate_col(int kind, int c) { return kind == 7 ? (c & ~15) + c : c; }
+__device__ __forceinline__ int up_col(int kind, int c, int F) { return kind == 7 ? (c & ~15) + c + 16 : F + c; }
+
 template <typename S, typename I>
 __global__ void __launch_bounds__(256) act_mul_kernel(
     S* __restrict__ out, int ldo, const I* __restrict__ gu, int ldg, int T, int F, int kind,
@@ -278,7 +283,8 @@ __global__ void __launch_bounds__(256) act_mul_kernel(
   if (nrows != nullptr && t >= *nrows) return;
   const I* r = gu + (long)t * ldg;
   stf(out + (long)t * ldo + c,
-      act_pair(kind, ldf(r + c), (kind >= 2 && kind < 5) ? 0.f : ldf(r + F + c), limit));
+      act_pair(kind, ldf(r + gate_col(kind, c)), (kind >= 2 && kind < 5) ? 0.f : ldf(r + up_col(kind, c, F)),
+               limit));
 }
 
 // 4 features a thread (F, ldg multiples of 4, 16-byte aligned rows): 16-byte loads
@@ -292,9 +298,9 @@ __global__ void __launch_bounds__(256) act_mul4_kernel(
   const int t = (int)(gid / f4), c = (int)(gid % f4) * 4;
   if (nrows != nullptr && t >= *nrows) return;
   const I* r = gu + (long)t * ldg;
-  const f32x4 g = ldin4(r + c);
+  const f32x4 g = ldin4(r + gate_col(kind, c));
   f32x4 u = f32x4{0.f, 0.f, 0.f, 0.f};
-  if (kind < 2 || kind >= 5) u = ldin4(r + F + c);
+  if (kind < 2 || kind >= 5) u = ldin4(r + up_col(kind, c, F));
 #pragma unroll
   for (int i = 0; i < 4; ++i)
     stf(out + (long)t * ldo + c + i, act_pair(kind, g[i], u[i], limit));
@@ -532,7 +538,7 @@ extern "C" int dli_token_shift(const float* h, const void* mu, float* state, con
 extern "C" int dli_act_mul(void* out, int ldo, const void* gu, int ldg, int T, int F, int kind,
                            const int* nrows, float limit, int in_dt, int dt, hipStream_t st) {
   if (T <= 0) return 0;
-  if (kind < 0 || kind > 6 || in_dt < 0 || in_dt > 1 || (in_dt == 0 && dt != 0))
+  if (kind < 0 || kind > 7 || (kind == 7 && F % 16) || in_dt < 0 || in_dt > 1 || (in_dt == 0 && dt != 0))
     return (int)hipErrorInvalidValue;
   const bool v4 = F % 4 == 0 && ldg % 4 == 0 && (uintptr_t)gu % 16 == 0;
   const int nb = (int)(((long)T * (v4 ? F / 4 : F) + 255) / 256);

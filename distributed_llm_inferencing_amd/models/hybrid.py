@@ -53,6 +53,7 @@ from typing import Dict, List, Optional
 import torch
 
 from ..engine.batch import DeviceBatch
+from ..ops import gemm as G
 from ..ops import hybrid as H
 from .configs import ModelConfig
 from .mixers import (FEED_FORWARDS, MIXERS, StepView, derive_constants,
@@ -309,6 +310,9 @@ class HybridLM(TransformerLM):
                     fused[id(lp["w_gu"])] = "clamp_mul"
                 elif spec.ff_kind == "gated_relu":
                     fused[id(lp["w_gu"])] = "relu_mul"
+                elif spec.ff_kind == "gated_gelu":
+                    if M > G.GEMV_MAX_M:
+                        fused[id(lp["w_gu"])] = "gelu_mul"
                 elif spec.ff_kind == "gated_silu":
                     fused[id(lp["w_gu"])] = "silu_mul"
                 elif spec.shared_ff and spec.expert_act == "gelu_erf":

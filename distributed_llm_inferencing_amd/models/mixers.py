@@ -370,7 +370,7 @@ MIXERS = {"attention": attention_mixer, "hgrn2": hgrn2_mixer,
 # Two layouts of a feed-forward's weights. The plain one ([gate | up] stacked) runs the
 # shape-agnostic GEMM with fp32 outputs and separate activation kernels: any sizes, bf16 or
 # fp32. The tuned one (``prepare_feed_forward``: bf16, sizes the tile family takes) fuses the
-# activation into the first GEMM's epilogue — SiLU * up or the clamped swish over the 16-row interleaved gate/up
+# activation into the first GEMM's epilogue — SiLU * up, GELU * up or the clamped swish over the 16-row interleaved gate/up
 # weight, bias + GELU for the ungated form — and runs the experts as the grouped GEMMs of the
 # framework's other mixture model.
 def prepare_feed_forward(spec: LayerSpec, params: dict, pre: str) -> None:
@@ -382,12 +382,12 @@ def prepare_feed_forward(spec: LayerSpec, params: dict, pre: str) -> None:
     w = params.get(pre + "w_down")
     if (not spec.ff or w is None or pre + "ff_tuned" in params or w.dtype != torch.bfloat16
             or not w.is_cuda
-            or spec.ff_kind not in ("gelu", "moe", "gated_silu", "clamp_swish", "gated_relu")
+            or spec.ff_kind not in ("gelu", "moe", "gated_silu", "gated_gelu", "clamp_swish", "gated_relu")
             or w.shape[-2] % 64 or spec.ff % 64 or spec.shared_ff % 64):
         return
     if spec.ff_kind == "gelu":
         params[pre + "b_up"] = torch.zeros(spec.ff, dtype=w.dtype, device=w.device)
-    elif spec.ff_kind in ("gated_silu", "clamp_swish", "gated_relu"):
+    elif spec.ff_kind in ("gated_silu", "gated_gelu", "clamp_swish", "gated_relu"):
         if spec.ff_kind == "clamp_swish":            # read by the GEMM's epilogue
             params[pre + "act_limit"] = torch.full((1,), spec.act_limit, dtype=torch.float32,
                                                    device=w.device)
@@ -406,7 +406,14 @@ def prepare_feed_forward(spec: LayerSpec, params: dict, pre: str) -> None:
 
 
 def gated_gelu_ff(spec: LayerSpec, lp: dict, h):
-    act = H.act_mul(H.linear_any(h, lp["w_gu"]), spec.ff, h.dtype, "gelu_mul")
+    from .. import ops
+    from ..ops.gemm import GEMV_MAX_M
+    if "ff_tuned" in lp and h.shape[0] > GEMV_MAX_M:
+        # the activation in the epilogue: 8192 rows, width 4096 -> 14336, 1426 + 222 us -> 1382 us
+        act = ops.linear(h, lp["w_gu"], epi="gelu_mul")
+    else:                               # (a few rows: the weight-streaming kernel, fp32 out)
+        act = H.act_mul(H.linear_any(h, lp["w_gu"]), spec.ff, h.dtype,
+                        "gelu_mul_pairs" if "ff_tuned" in lp else "gelu_mul")
     return H.linear_any(act, lp["w_down"])
 
 

@@ -238,7 +238,7 @@ def _gemm_native(x, w, epi: str, bias=None, out=None, plan: Optional[G.GemmPlan]
 
 def linear(x, w, bias=None, epi: str = "none", out=None):
     """y = epi(x @ w.T (+bias)). epi in {none, f32, silu_mul, bias_gelu, bias, gelu_erf,
-    clamp_mul, relu_mul}. silu_mul, clamp_mul and relu_mul expect the 16-row interleaved gate/up
+    clamp_mul, relu_mul, gelu_mul}. silu_mul, clamp_mul, relu_mul and gelu_mul expect the 16-row interleaved gate/up
     weight and return width N/2; clamp_mul takes its limit as ``bias``, one fp32 number on the device."""
     if bias is not None and epi == "none":
         epi = "bias"
@@ -264,6 +264,9 @@ def linear(x, w, bias=None, epi: str = "none", out=None):
         elif epi == "relu_mul":
             g, u = R.split_gate_up(R.linear(x, w, out_dtype=torch.float32))
             y = (torch.relu(g) * u).to(x.dtype)
+        elif epi == "gelu_mul":
+            g, u = R.split_gate_up(R.linear(x, w, out_dtype=torch.float32))
+            y = (torch.nn.functional.gelu(g, approximate="tanh") * u).to(x.dtype)
         elif epi == "gelu_erf":
             y = torch.nn.functional.gelu(R.linear(x, w, out_dtype=torch.float32)).to(x.dtype)
         else:

@@ -251,7 +251,7 @@ def concat_cast(a: torch.Tensor, b: torch.Tensor, dtype) -> torch.Tensor:
 
 
 _ACT_KINDS = {"gelu_mul": 0, "silu_mul": 1, "gelu": 2, "gelu_erf": 3, "copy": 4,
-              "clamp_swish": 5, "relu_mul": 6}
+              "clamp_swish": 5, "relu_mul": 6, "gelu_mul_pairs": 7}
 
 
 def act_mul(gu: torch.Tensor, F_: int, dtype, kind: str = "gelu_mul",
@@ -260,10 +260,13 @@ def act_mul(gu: torch.Tensor, F_: int, dtype, kind: str = "gelu_mul",
     ``relu_mul`` = act(gu[:, :F]) * gu[:, F:2F]; ``gelu`` = gelu_tanh(gu[:, :F]); ``gelu_erf`` = the exact GELU
     of gu[:, :F]; ``copy`` = gu[:, :F] rounded to the storage dtype; ``clamp_swish`` = g
     sigmoid(1.702 g) (u + 1) with g = min(gu[:, :F], limit), u = clamp(gu[:, F:2F], +-limit).
+    ``gelu_mul_pairs``: ``gelu_mul`` for a projection by the 16-row interleaved weight.
     ``gu`` may also be a bf16 projection (a tuned GEMM's output) when ``dtype`` is bf16.
     ``rows`` (device int32
     scalar): only that many leading rows hold data (routed rows of a mixture)."""
     if not gu.is_cuda:
+        if kind == "gelu_mul_pairs":
+            gu, kind = torch.cat(R.split_gate_up(gu), -1), "gelu_mul"
         return R.act_mul(gu, F_, dtype, kind, limit)
     T = gu.shape[0]
     out = torch.empty(T, F_, dtype=dtype, device=gu.device)

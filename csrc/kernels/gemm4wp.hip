@@ -207,7 +207,7 @@ __global__ void __launch_bounds__(256, 1) gemm4wp_kernel(
     // acc[I][J][r] = C[m0 + 128 wm + 16I + fr][n0 + 128 wn + 16J + 4fq + r]
     const int wr0 = m0 + 128 * wm, wc0 = n0 + 128 * wn;
     const bool vec = out_vec<EPI>(C, ldc, N, bias);
-    if (EPI == EPI_SILU) {
+    if (epi_pairs(EPI)) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const int row = wr0 + 16 * i + fr;
@@ -216,7 +216,7 @@ __global__ void __launch_bounds__(256, 1) gemm4wp_kernel(
           const f32x4 g = vget(acc[i][j]), u = vget(acc[i][j + 1]);
           const int gcol = wc0 + 16 * j;
           if (row < M && gcol < N)
-            store_pair_quad(C, ldc, row, (gcol >> 5) * 16 + 4 * fq, g, u, vec);
+            store_pair_quad<EPI>(C, ldc, row, (gcol >> 5) * 16 + 4 * fq, g, u, vec);
         }
       }
     } else {
@@ -247,7 +247,7 @@ static int launch_4wp(const void* A, int lda, const void* W, int ldw, void* C, i
                       int N, int K, int splits, const void* bias, const int* group_off,
                       hipStream_t st) {
   if (splits != 1 || group_off != nullptr || K % (2 * BK) || C == nullptr ||
-      (EPI == EPI_SILU && N % 32))
+      (epi_pairs(EPI) && N % 32))
     return (int)hipErrorInvalidValue;
   constexpr size_t lds = 4 * (size_t)256 * BK * 2;
   static int cus = 0;
@@ -277,4 +277,7 @@ static int dispatch_4wp(int tile_cfg, DLI_GEMM_ARGS) {
   return launch_4wp<EPI>(A, lda, W, ldw, C, ldc, M, N, K, splits, bias, go, st);
 }
 
-int gemm_4wp_dispatch(int epi, int tile_cfg, DLI_GEMM_ARGS) { DLI_EPI_SWITCH_BASE(dispatch_4wp) }
+int gemm_4wp_dispatch(int epi, int tile_cfg, DLI_GEMM_ARGS) {
+  if (epi == EPI_GELU_MUL) return dispatch_4wp<EPI_GELU_MUL>(tile_cfg, DLI_GEMM_PASS);
+  DLI_EPI_SWITCH_BASE(dispatch_4wp)
+}

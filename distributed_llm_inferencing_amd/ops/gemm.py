@@ -90,7 +90,7 @@ def tile_ok(tile: int, epi: str) -> bool:
     if epi == "res":
         return tile in GEMV_RES_TILES
     if epi in ("gelu_erf", "clamp_mul", "relu_mul", "gelu_mul") and tile in (34, 41, 45, 55):
-        return False            # the 4-wave families are built without these epilogues
+        return epi == "gelu_mul" and tile == 55     # the 4-wave families lack the others
     if tile in (29, 58, 59):
         return epi == "silu_mul"
     if tile in GEMV_TILES:

@@ -24,7 +24,8 @@ def close(got, want):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("tile,splits", [(0, 1), (0, 2), (1, 4), (2, 1), (13, 1), (22, 1), (22, 2), (26, 1), (28, 2)])
+@pytest.mark.parametrize("tile,splits", [(0, 1), (0, 2), (1, 4), (2, 1), (13, 1), (22, 1), (22, 2), (26, 1), (28, 2),
+                                         (55, 1)])
 @pytest.mark.parametrize("M", [5, 70, 300])
 def test_epilogue(gpu, tile, splits, M):
     x, w, want = case(M, 448, 256, gpu)

@@ -4,11 +4,12 @@
 // -> multinomial. One 512-thread workgroup per row (vocab up to ~256k), no full-vocab sort:
 //   * greedy (temperature <= 0 or top_k == 1): block argmax (first index on ties, like torch).
 //   * top_k <= 0 and top_p >= 1: exact Gumbel-max sampling over the whole row in one pass.
-//   * otherwise: radix select (8-bit digits, early exit) finds the bin holding the k-th
-//     largest logit; every element at or above it (<= CAP) is gathered into LDS, bitonic-
-//     sorted, cut to the top-k (ties kept, as HF's `scores < kth` mask keeps them), then
-//     temperature-softmax, top-p truncation (keep j while the mass of strictly larger tokens
-//     < top_p, i.e. HF's `cumsum_asc <= 1-top_p` removal) and an inverse-CDF draw.
+//   * otherwise the top-k set (ties with the k-th kept, as HF's `scores < kth` mask keeps them):
+//     up to k = 256 from the elements above a bound on the k-th largest, found from per-thread
+//     maxima; larger k and rows this does not take by radix select (8-bit digits, early exit) and
+//     a gather of <= CAP elements. The set is sorted, then temperature-softmax, top-p truncation
+//     (keep j while the mass of strictly larger tokens < top_p, i.e. HF's `cumsum_asc <=
+//     1-top_p` removal) and an inverse-CDF draw.
 // top_k is capped at CAP (2048). Randomness: Philox4x32-10 keyed by a per-row 64-bit seed
 // supplied by the engine (seed = f(request seed, output index)), so a request samples the
 // same tokens regardless of how it is batched.
@@ -16,6 +17,8 @@
 
 #define SMP_THREADS 512
 #define SMP_CAP 2048
+// candidates ranked by counting; more go through the bitonic sort
+#define SMP_RANK_MAX 128
 
 __device__ __forceinline__ uint32_t f2key(float f) {
   uint32_t u = __float_as_uint(f);
@@ -123,68 +126,113 @@ __device__ uint32_t radix_kth(const uint32_t* keys, int n, uint32_t k, uint32_t*
   return prefix;
 }
 
+// A threshold t with at least k of the wave's 64 * NR keys at or above it, the largest one unless
+// exactly k keys are: bit by bit, one ballot per register and bit, no LDS and no barrier. 0 when
+// fewer than k keys are non-zero. low: every key but empty (0) ones is at least that, so the bits
+// it shares with the largest key need no step. steps: bits to find; fewer leave a lower threshold.
+// (512 keys by four histogram passes: some 4 us in 20 barriers; by some 12 bits of 8 ballots 1 us,
+// every wave for itself.)
+template <int NR>
+__device__ __forceinline__ uint32_t wave_kth(const uint32_t (&keys)[NR], int k, uint32_t low = 0u,
+                                              int steps = 32) {
+  uint32_t t = 0u;
+  int bit = 31;
+  if (low != 0u) {
+    uint32_t top = low;
+#pragma unroll
+    for (int j = 0; j < NR; ++j) top = max(top, keys[j]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, o, 64));
+    const uint32_t diff = top ^ low;
+    if (diff == 0u) return low;
+    bit = 31 - __builtin_clz(diff);
+    t = bit == 31 ? 0u : low >> (bit + 1) << (bit + 1);
+  }
+  for (; bit >= 0 && steps > 0; --bit, --steps) {
+    const uint32_t c = t | (1u << bit);
+    int cnt = 0;
+#pragma unroll
+    for (int j = 0; j < NR; ++j) cnt += __popcll(__ballot(keys[j] >= c));
+    if (cnt >= k) t = c;
+    if (cnt == k) break;
+  }
+  return t;
+}
+
 // Logits arrive as fp32 or as bf16 (u16: the LM head's output in the model dtype, as HF's
 // `lm_head(hidden).float()` produces them); every comparison runs on the exact fp32 value.
 __device__ __forceinline__ float ldv(const float* x, int i) { return x[i]; }
 __device__ __forceinline__ float ldv(const u16* x, int i) { return bf2f(x[i]); }
 
-// Visit every element of a row with 16-B loads, 4 loads in flight per thread (the sampler is
-// one workgroup per row, so memory-level parallelism per CU comes from ILP, not occupancy).
+// Visit every element of a row with 16-B loads, 8 in flight per thread, the last partial round
+// too (the sampler is one workgroup per row, so memory-level parallelism per CU comes from ILP,
+// not occupancy).
 template <typename F>
-__device__ __forceinline__ void row_scan(const u16* __restrict__ x, int V, F&& f) {
-  const int tid = threadIdx.x, nt = blockDim.x;
-  int done = 0;
-  if ((reinterpret_cast<uintptr_t>(x) & 15) == 0) {
-    const int V8 = V >> 3;
-    const uint4* x8 = reinterpret_cast<const uint4*>(x);
-    auto eight = [&](const uint4 v, int base) {
-      f(__uint_as_float(v.x << 16), base);     f(__uint_as_float(v.x & 0xffff0000u), base + 1);
-      f(__uint_as_float(v.y << 16), base + 2); f(__uint_as_float(v.y & 0xffff0000u), base + 3);
-      f(__uint_as_float(v.z << 16), base + 4); f(__uint_as_float(v.z & 0xffff0000u), base + 5);
-      f(__uint_as_float(v.w << 16), base + 6); f(__uint_as_float(v.w & 0xffff0000u), base + 7);
-    };
-    int i = tid;
-    for (; i + 3 * nt < V8; i += 4 * nt) {
-      const uint4 a = x8[i], b = x8[i + nt], c = x8[i + 2 * nt], d = x8[i + 3 * nt];
-      eight(a, 8 * i); eight(b, 8 * (i + nt)); eight(c, 8 * (i + 2 * nt)); eight(d, 8 * (i + 3 * nt));
-    }
-    for (; i < V8; i += nt) eight(x8[i], 8 * i);
-    done = V8 * 8;
-  }
-  for (int j = done + tid; j < V; j += nt) f(bf2f(x[j]), j);
+__device__ __forceinline__ void visit16(const uint4 v, int base, const u16*, F&& f) {
+  f(__uint_as_float(v.x << 16), base);     f(__uint_as_float(v.x & 0xffff0000u), base + 1);
+  f(__uint_as_float(v.y << 16), base + 2); f(__uint_as_float(v.y & 0xffff0000u), base + 3);
+  f(__uint_as_float(v.z << 16), base + 4); f(__uint_as_float(v.z & 0xffff0000u), base + 5);
+  f(__uint_as_float(v.w << 16), base + 6); f(__uint_as_float(v.w & 0xffff0000u), base + 7);
+}
+template <typename F>
+__device__ __forceinline__ void visit16(const uint4 v, int base, const float*, F&& f) {
+  f(__uint_as_float(v.x), base);     f(__uint_as_float(v.y), base + 1);
+  f(__uint_as_float(v.z), base + 2); f(__uint_as_float(v.w), base + 3);
 }
 
+// with a floor: only groups holding an element that is not below it
 template <typename F>
-__device__ __forceinline__ void row_scan(const float* __restrict__ x, int V, F&& f) {
+__device__ __forceinline__ void visit16(const uint4 v, int base, const u16* x, F&& f, float lo) {
+  bool any = false;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const uint32_t w = j == 0 ? v.x : j == 1 ? v.y : j == 2 ? v.z : v.w;
+    any |= !(__uint_as_float(w << 16) < lo) | !(__uint_as_float(w & 0xffff0000u) < lo);
+  }
+  if (any) visit16(v, base, x, f);
+}
+template <typename F>
+__device__ __forceinline__ void visit16(const uint4 v, int base, const float* x, F&& f, float lo) {
+  if (!(__uint_as_float(v.x) < lo) | !(__uint_as_float(v.y) < lo) |
+      !(__uint_as_float(v.z) < lo) | !(__uint_as_float(v.w) < lo))
+    visit16(v, base, x, f);
+}
+
+template <typename LT, typename F, typename... G>
+__device__ __forceinline__ void row_scan(const LT* __restrict__ x, int V, F&& f, G... floor) {
+  constexpr int E = 16 / sizeof(LT), U = 8;
   const int tid = threadIdx.x, nt = blockDim.x;
   int done = 0;
   if ((reinterpret_cast<uintptr_t>(x) & 15) == 0) {
-    const int V4 = V >> 2;
-    const float4* x4 = reinterpret_cast<const float4*>(x);
+    const int VE = V / E;
+    const uint4* xe = reinterpret_cast<const uint4*>(x);
+    uint4 a[U];
     int i = tid;
-    for (; i + 3 * nt < V4; i += 4 * nt) {
-      const float4 a = x4[i], b = x4[i + nt], c = x4[i + 2 * nt], d = x4[i + 3 * nt];
-      f(a.x, 4 * i); f(a.y, 4 * i + 1); f(a.z, 4 * i + 2); f(a.w, 4 * i + 3);
-      const int ib = 4 * (i + nt), ic = 4 * (i + 2 * nt), id = 4 * (i + 3 * nt);
-      f(b.x, ib); f(b.y, ib + 1); f(b.z, ib + 2); f(b.w, ib + 3);
-      f(c.x, ic); f(c.y, ic + 1); f(c.z, ic + 2); f(c.w, ic + 3);
-      f(d.x, id); f(d.y, id + 1); f(d.z, id + 2); f(d.w, id + 3);
+    for (; i + (U - 1) * nt < VE; i += U * nt) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) a[u] = xe[i + u * nt];
+#pragma unroll
+      for (int u = 0; u < U; ++u) visit16(a[u], E * (i + u * nt), x, f, floor...);
     }
-    for (; i < V4; i += nt) {
-      const float4 a = x4[i];
-      f(a.x, 4 * i); f(a.y, 4 * i + 1); f(a.z, 4 * i + 2); f(a.w, 4 * i + 3);
+    if (i < VE) {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (i + u * nt < VE) a[u] = xe[i + u * nt];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (i + u * nt < VE) visit16(a[u], E * (i + u * nt), x, f, floor...);
     }
-    done = V4 * 4;
+    done = VE * E;
   }
-  for (int j = done + tid; j < V; j += nt) f(x[j], j);
+  for (int j = done + tid; j < V; j += nt) f(ldv(x, j), j);
 }
 
 // ---------------------------------------------------------------------------------------
 // Small batches (B <= SMP_SPLIT_MAX_B): one workgroup per row leaves ~255 CUs idle while it
-// walks a 128k-entry row several times (~45 us at batch 1, profiles/r3/b1_p). Two phases
+// walks a 128k-entry row (23 us at batch 1; two phases 18). Two phases
 // instead: sample_chunk_kernel splits each row into P chunks (P workgroups per row); a chunk
-// keeps every logit >= its own Keff-th largest (radix select in LDS), in index order, in a
-// CAPC-slot candidate list (pads: -inf). The row's top-Keff is contained in the union of the
+// keeps every logit >= its own Keff-th largest (16 keys a thread in registers, the threshold by
+// ballots as in sample_kernel), in index order, in a CAPC-slot candidate list (pads: -inf). The row's top-Keff is contained in the union of the
 // chunks' lists, which keep index order, so sample_kernel then runs its unchanged algorithm
 // over the P*CAPC candidates (ties still break on the lower vocab index) and maps the pick
 // back to a vocab id. Rows whose Keff exceeds CAPC, plain-temperature rows and rows where a
@@ -206,10 +254,9 @@ __global__ void __launch_bounds__(256) sample_chunk_kernel(
     const LT* __restrict__ logits, long row_stride, int V, int L,
     const float* __restrict__ temperature, const int* __restrict__ top_k,
     const float* __restrict__ top_p) {
-  __shared__ uint32_t keys[SMP_CHUNK_MAX];
-  __shared__ uint32_t hist[256];
-  __shared__ float tmp[16];
-  __shared__ uint32_t sel[3];
+  constexpr int NE = SMP_CHUNK_MAX / 256, LIST = 512;
+  __shared__ uint32_t lk[LIST], s_tau[4];
+  __shared__ int li[LIST], s_cnt;
   const int row = blockIdx.y, c = blockIdx.x, tid = threadIdx.x, P = gridDim.x;
   const float T = temperature[row];
   const int K = top_k[row];
@@ -217,32 +264,69 @@ __global__ void __launch_bounds__(256) sample_chunk_kernel(
   const int keff = (T <= 0.f || K == 1) ? 1 : K;
   const int lo = c * L, n = max(0, min(V, lo + L) - lo);
   const LT* x = logits + (long)row * row_stride + lo;
-  for (int e = tid; e < n; e += 256) keys[e] = f2key(ldv(x, e));
-  __syncthreads();
-  // the chunk's keff-th largest key (0: fewer than keff entries -> keep them all)
-  const uint32_t tau = n > 0 ? radix_kth(keys, n, (uint32_t)min(keff, n), hist, tmp, sel) : 0u;
-  // ordered compaction: thread t owns a contiguous slice, a block scan of the counts gives
-  // each survivor its slot
-  const int per = (n + 255) / 256, b0 = min(n, tid * per), b1 = min(n, b0 + per);
-  int cnt = 0;
-  for (int e = b0; e < b1; ++e) cnt += keys[e] >= tau && keys[e] != 0u;
-  const int incl = (int)block_scan((float)cnt, tmp);   // exact: counts < 2^24
-  int pos = incl - cnt;
-  const long base = ((long)row * P + c) * SMP_CAPC;
-  for (int e = b0; e < b1; ++e)
-    if (keys[e] >= tau && keys[e] != 0u) {
-      if (pos < SMP_CAPC) { cand_v[base + pos] = key2f(keys[e]); cand_i[base + pos] = lo + e; }
-      ++pos;
-    }
-  __shared__ int s_total;
-  if (tid == 255) s_total = incl;
-  __syncthreads();
-  if (s_total > SMP_CAPC) {
-    if (tid == 0) overflow[row] = 1;                   // the row falls back to the full scan
+  uint32_t key[NE];
+  uint32_t mk[1] = {0u};
+#pragma unroll
+  for (int j = 0; j < NE; ++j) {
+    const int e = tid + 256 * j;
+    key[j] = e < n ? f2key(ldv(x, e)) : 0u;
   }
-  for (int e = s_total + tid; e < SMP_CAPC; e += 256) {
-    cand_v[base + e] = -INFINITY;
-    cand_i[base + e] = 0;
+#pragma unroll
+  for (int j = 0; j < NE; ++j) mk[0] = max(mk[0], key[j]);
+  // a lower bound of the chunk's keff-th largest key, as in sample_kernel: the least of the
+  // waves' ceil(keff / 4)-th largest per-thread maxima
+  const uint32_t tw = wave_kth(mk, (keff + 3) / 4);
+  if ((tid & 63) == 0) s_tau[tid >> 6] = tw;
+  if (tid == 0) s_cnt = 0;
+  __syncthreads();
+  const uint32_t tau0 = max(min(min(s_tau[0], s_tau[1]), min(s_tau[2], s_tau[3])), 1u);
+#pragma unroll
+  for (int j = 0; j < NE; ++j)
+    if (key[j] >= tau0) {
+      const int pos = atomicAdd(&s_cnt, 1);
+      if (pos < LIST) { lk[pos] = key[j]; li[pos] = lo + tid + 256 * j; }
+    }
+  __syncthreads();
+  const int nc = s_cnt;
+  if (nc > LIST) {                                     // ties by the hundred: the row's full scan
+    if (tid == 0) overflow[row] = 1;
+    return;
+  }
+  if (tid >= 64) return;                               // one wave orders what is left
+  uint32_t ck[LIST / 64];
+  int ci[LIST / 64];
+#pragma unroll
+  for (int j = 0; j < LIST / 64; ++j) {
+    const int e = j * 64 + tid;
+    ck[j] = e < nc ? lk[e] : 0u;
+    ci[j] = e < nc ? li[e] : 0;
+  }
+  // (fewer than keff entries: keep them all)
+  const uint32_t tau = nc > keff ? wave_kth(ck, keff, tau0) : 1u;
+  int m = 0;
+  const unsigned long long below = (1ull << tid) - 1ull;
+#pragma unroll
+  for (int j = 0; j < LIST / 64; ++j) {
+    const unsigned long long keep = __ballot(ck[j] >= tau);
+    const int pos = m + __popcll(keep & below);
+    if (ck[j] >= tau) { lk[pos] = ck[j]; li[pos] = ci[j]; }   // every entry is in registers
+    m += __popcll(keep);
+  }
+  if (m > SMP_CAPC) {
+    if (tid == 0) overflow[row] = 1;                   // the row falls back to the full scan
+    return;
+  }
+  __builtin_amdgcn_wave_barrier();
+  const long base = ((long)row * P + c) * SMP_CAPC;
+  if (tid < m) {
+    const int id = li[tid];
+    int rank = 0;                                      // index order within the chunk
+    for (int j = 0; j < m; ++j) rank += li[j] < id;
+    cand_v[base + rank] = key2f(lk[tid]);
+    cand_i[base + rank] = id;
+  } else {
+    cand_v[base + tid] = -INFINITY;
+    cand_i[base + tid] = 0;
   }
 }
 
@@ -254,14 +338,14 @@ __global__ void __launch_bounds__(SMP_THREADS) sample_kernel(
     const float* __restrict__ cand_v, const int* __restrict__ cand_i,
     int* __restrict__ overflow, int ncand) {
   __shared__ uint32_t hist[256];
-  __shared__ uint32_t ckey[2 * SMP_CAP];      // fast path: 512 threads x top-8 candidates
+  __shared__ uint32_t ckey[2 * SMP_CAP];      // fast path: the list of candidates
   __shared__ int cidx[2 * SMP_CAP];
   __shared__ uint32_t skey[512];
   __shared__ int sidx[512];
-  __shared__ float cprob[SMP_CAP];
+  __shared__ __attribute__((aligned(8))) float cprob[SMP_CAP];
   __shared__ float sv[16];
   __shared__ int si[16];
-  __shared__ uint32_t s_sel[3], s_cnt;
+  __shared__ uint32_t s_sel[3], s_tau[SMP_THREADS / 64], s_cnt;
   const int row = blockIdx.x, tid = threadIdx.x;
   const LT* xl = logits + (long)row * row_stride;
   const float* xc = nullptr;                     // two-phase mode: the row's candidate list
@@ -319,63 +403,131 @@ __global__ void __launch_bounds__(SMP_THREADS) sample_kernel(
   if (Keff > Vfull) Keff = Vfull;
 
   int n = 0;
-  bool fast_ok = false;
+  bool fast_ok = false, sorted = false;
   // ---- fast path, no full-row select:
-  //  (1) tau0 = the Keff-th largest of the 512 per-thread maxima over the row's first
-  //      quarter. At least Keff elements are >= tau0, so tau0 <= the row's Keff-th largest.
-  //  (2) one pass over the row; each thread keeps its top-8 (key, index) in registers
-  //      (static-index insertion network) among the elements >= tau0 only. Unguarded, the
-  //      network ran for nearly every element: some lane of the wave almost always had a
-  //      new local top-8 entry, and the whole wave pays for it.
-  //  The Keff-th largest of the candidates (tau) is exact iff no thread dropped an element
-  //  >= tau, i.e. every thread's 8th kept key is < tau — one block-wide OR. Otherwise the
-  //  full radix select below.
+  //  (1) tau0: each of the 8 waves takes the ceil(Keff / 8)-th largest of its 64 per-thread
+  //      maxima over the row's first quarter (fewer waves on a short row); the least of them,
+  //      brought nearer to the Keff-th largest of all 512 by a few steps, is tau0. At least Keff elements are >= tau0, so
+  //      tau0 <= the row's Keff-th largest. (Without the steps the list runs to 300 - 600.)
+  //  (2) one pass over the row; each thread keeps the elements >= tau0 it meets, a few hundred
+  //      of 128k over all, in 8 slots of its own in LDS (a shared counter would cost a round trip
+  //      per element). A row that needs more in one thread goes through the full radix select.
+  //  (3) the list's Keff-th largest key is the row's; what reaches it is ranked by counting.
+  // 24 rows of 32k / 128k logits, top-k 50: 32 / 42 us with the 512 maxima and the list's 4096 slots
+  // selected by histograms and a bitonic sort of the rest -> 16 / 25.
   if (Keff <= 256) {
     uint32_t mk = 0u;
-    scan((V >> 4) << 2, [&](float v, int) { mk = max(mk, f2key(v)); });
-    ckey[tid] = mk;
+    // (a short row whole: every thread needs elements)
+    const int first = max((V >> 4) << 2, min(V, 16 * SMP_THREADS));
+    scan(first, [&](float v, int) { mk = max(mk, f2key(v)); });
+    constexpr int NWV = SMP_THREADS / 64, SLOTS = 2 * SMP_CAP / SMP_THREADS;
+    const uint32_t mk1[1] = {mk};
+    const int nw = min(NWV, (first + 255) >> 8);  // waves that met elements
+    const uint32_t tw = wave_kth(mk1, (Keff + nw - 1) / nw);
+    if ((tid & 63) == 0) s_tau[tid >> 6] = (tid >> 6) < nw ? tw : 0xffffffffu;
+    if (tid == 0) s_cnt = 0;
+    skey[tid] = mk;
     __syncthreads();
-    const uint32_t tau0 = radix_kth(ckey, SMP_THREADS, (uint32_t)Keff, hist, sv, s_sel);
-    uint32_t tk[8];
-    int ti[8];
+    uint32_t tau0 = s_tau[0];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) { tk[j] = 0u; ti[j] = 0x7fffffff; }
-    scan(V, [&](float v, int i) {
-      uint32_t k = f2key(v);
-      if (k >= tau0 && k > tk[7]) {
-        int id = i;
+    for (int w = 1; w < NWV; ++w) tau0 = min(tau0, s_tau[w]);
+    if (xc == nullptr) {                          // (a candidate list is short enough)
+      uint32_t ck[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) ck[j] = skey[j * 64 + (tid & 63)];
+      tau0 = max(tau0, wave_kth(ck, Keff, tau0, 7));
+    }
+    tau0 = max(tau0, 1u);                         // key 0 is no element
+    // !(v < tf) is true of every element with a key >= tau0 (and of NaNs and zeros below it): one
+    // compare an element, the keys only where one of 16 bytes passes
+    const float tf = key2f(tau0);
+    int cnt = 0;
+    auto hit = [&](float v, int i) {
+      const uint32_t k = f2key(v);
+      if (k >= tau0) {
+        if (cnt < SLOTS) {                        // thread-strided slots: no bank conflicts
+          ckey[tid + SMP_THREADS * cnt] = k;
+          cidx[tid + SMP_THREADS * cnt] = i;
+        }
+        ++cnt;
+      }
+    };
+    if (xc != nullptr) row_scan(xc, V, hit, tf);
+    else row_scan(xl, V, hit, tf);
+    const uint32_t at = cnt ? atomicAdd(&s_cnt, (uint32_t)cnt) : 0u;
+    const int dropped = __syncthreads_or(cnt > SLOTS ? 1 : 0);
+    const uint32_t nc = s_cnt;
+    if (!dropped && nc >= (uint32_t)Keff) {
+      if (nc <= 512) {
+        for (int j = 0; j < cnt; ++j) {
+          skey[at + j] = ckey[tid + SMP_THREADS * j];
+          sidx[at + j] = cidx[tid + SMP_THREADS * j];
+        }
+      } else {
+        for (int j = cnt; j < SLOTS; ++j) ckey[tid + SMP_THREADS * j] = 0u;
+      }
+      __syncthreads();
+      if (nc <= 512) {
+        // every wave holds the whole list and finds the threshold for itself; the first packs
+        // and ranks what reaches it
+        uint32_t ck[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-          if (k > tk[j]) {
-            const uint32_t t = tk[j]; tk[j] = k; k = t;
-            const int u = ti[j]; ti[j] = id; id = u;
+          const uint32_t e = j * 64 + (tid & 63);
+          ck[j] = e < nc ? skey[e] : 0u;
+        }
+        const uint32_t(&half)[4] = *reinterpret_cast<const uint32_t(*)[4]>(ck);
+        const uint32_t tau = nc <= 256 ? wave_kth(half, Keff, tau0) : wave_kth(ck, Keff, tau0);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) n += __popcll(__ballot(ck[j] >= tau));
+        sorted = n <= SMP_RANK_MAX;
+        unsigned long long* both = reinterpret_cast<unsigned long long*>(cprob);
+        if (tid < 64) {
+          int m = 0;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            const unsigned long long keep = __ballot(ck[j] >= tau);
+            if (ck[j] >= tau) {
+              const int pos = m + __popcll(keep & ((1ull << tid) - 1ull));
+              const int id = sidx[j * 64 + tid];
+              if (sorted) {
+                both[pos] = (unsigned long long)ck[j] << 32 | (uint32_t)~id;
+              } else {
+                ckey[pos] = ck[j];
+                cidx[pos] = id;
+              }
+            }
+            m += __popcll(keep);
+          }
+          __builtin_amdgcn_wave_barrier();
+          if (sorted) {
+            for (int e = tid; e < n; e += 64) {
+              const unsigned long long own = both[e];   // larger key first, then smaller index
+              int rank = 0;
+#pragma unroll 8
+              for (int j = 0; j < n; ++j) rank += both[j] > own;
+              ckey[rank] = (uint32_t)(own >> 32);
+              cidx[rank] = ~(int)(uint32_t)own;
+            }
           }
         }
-      }
-    });
-    __syncthreads();                              // every thread is past radix_kth's reads
-#pragma unroll
-    for (int j = 0; j < 8; ++j) { ckey[tid * 8 + j] = tk[j]; cidx[tid * 8 + j] = ti[j]; }
-    __syncthreads();
-    // key of the Keff-th largest candidate (0: fewer than Keff candidates)
-    const uint32_t tau = radix_kth(ckey, 8 * SMP_THREADS, (uint32_t)Keff, hist, sv, s_sel);
-    const int dropped = __syncthreads_or(tk[7] >= tau ? 1 : 0);
-    fast_ok = tau != 0u && !dropped;
-    if (fast_ok) {
-      if (tid == 0) s_cnt = 0;
-      __syncthreads();
-      for (int e = tid; e < 8 * SMP_THREADS; e += blockDim.x) {
-        if (ckey[e] >= tau) {
-          const uint32_t pos = atomicAdd(&s_cnt, 1u);
-          if (pos < 512) { skey[pos] = ckey[e]; sidx[pos] = cidx[e]; }
-        }
-      }
-      __syncthreads();
-      if (s_cnt > 512) {
-        fast_ok = false;                          // absurd tie count: take the slow path
+        fast_ok = true;
       } else {
-        n = (int)s_cnt;
-        for (int e = tid; e < n; e += blockDim.x) { ckey[e] = skey[e]; cidx[e] = sidx[e]; }
+        const uint32_t tau = radix_kth(ckey, SLOTS * SMP_THREADS, (uint32_t)Keff, hist, sv, s_sel);
+        if (tid == 0) s_cnt = 0;
+        __syncthreads();
+        for (int e = tid; e < SLOTS * SMP_THREADS; e += blockDim.x) {
+          if (ckey[e] >= tau) {
+            const uint32_t pos = atomicAdd(&s_cnt, 1u);
+            if (pos < 512) { skey[pos] = ckey[e]; sidx[pos] = cidx[e]; }
+          }
+        }
+        __syncthreads();
+        fast_ok = s_cnt <= 512;                   // absurd tie count: take the slow path
+        if (fast_ok) {
+          n = (int)s_cnt;
+          for (int e = tid; e < n; e += blockDim.x) { ckey[e] = skey[e]; cidx[e] = sidx[e]; }
+        }
       }
       __syncthreads();
     }
@@ -438,9 +590,11 @@ __global__ void __launch_bounds__(SMP_THREADS) sample_kernel(
   }
   }
   int npow = 1;
-  while (npow < n) npow <<= 1;
-  for (int i = n + tid; i < npow; i += blockDim.x) { ckey[i] = 0u; cidx[i] = 0x7fffffff; }
-  __syncthreads();
+  if (!sorted) {
+    while (npow < n) npow <<= 1;
+    for (int i = n + tid; i < npow; i += blockDim.x) { ckey[i] = 0u; cidx[i] = 0x7fffffff; }
+    __syncthreads();
+  }
   // ---- bitonic sort descending by key (ties: smaller index first)
   for (int size = 2; size <= npow; size <<= 1) {
     for (int stride = size >> 1; stride > 0; stride >>= 1) {
@@ -463,6 +617,47 @@ __global__ void __launch_bounds__(SMP_THREADS) sample_kernel(
   const uint32_t tau = ckey[kk - 1];
   int m = kk;
   while (m < n && ckey[m] == tau) ++m;
+  if (m <= 256) {
+    // the first wave's entries are all there are: the sums below in the same order, in its
+    // registers, and no barriers (7k -> 2k cycles)
+    if (tid >= 64) return;
+    const float xm = key2f(ckey[0]);
+    float cp[4], ls = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int e = tid * 4 + j;
+      cp[j] = e < m ? __expf((key2f(ckey[e]) - xm) * invT) : 0.f;
+      ls += cp[j];
+    }
+    float inc = ls;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const float t = __shfl_up(inc, o, 64);
+      if (tid >= o) inc += t;
+    }
+    float run = inc - ls;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) { run += cp[j]; cp[j] = run; }
+    auto at = [&](int e) {                        // e is the same in every lane
+      const float v = (e & 2) ? ((e & 1) ? cp[3] : cp[2]) : ((e & 1) ? cp[1] : cp[0]);
+      return __shfl(v, e >> 2, 64);
+    };
+    auto first = [&](int end, auto&& pass) {      // first e < end that passes, else end
+      int e = end;
+#pragma unroll
+      for (int j = 3; j >= 0; --j)
+        if (tid * 4 + j < end && pass(cp[j])) e = tid * 4 + j;
+      const unsigned long long any = __ballot(e < end);
+      return any ? __shfl(e, __ffsll(any) - 1, 64) : end;
+    };
+    const float lim = P * at(m - 1);
+    const int c = first(m - 1, [&](float v) { return v >= lim; }) + 1;
+    const uint4 r = philox(key, make_uint4(0xfffffffu, 1u, 0xa5a5a5a5u, 7u));
+    const float u = u01(r.x) * at(c - 1);
+    const int pick = first(c - 1, [&](float v) { return v > u; });
+    if (tid == 0) out_tokens[row] = vocab_id(cidx[pick]);
+    return;
+  }
   // ---- temperature softmax over the m survivors, top-p, inverse CDF
   const float xmax = key2f(ckey[0]);
   constexpr int PER = SMP_CAP / SMP_THREADS;                 // 4 consecutive entries / thread

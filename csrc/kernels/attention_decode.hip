@@ -23,9 +23,12 @@
 #include "common.h"
 #include <limits.h>
 #include <stdlib.h>
+#include <type_traits>
 
 #define DEC_WAVES 4
 #define DEC_TILE 32
+#define DEC_TARGET 3072
+#define DEC_MIN_TILES 2
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
@@ -51,6 +54,82 @@ __device__ __forceinline__ void decode_wg_range(int ctx, int wv, int& s_begin, i
   const int per = (tiles + WPI - 1) / WPI;
   s_begin = min(ctx, wv * per * DEC_TILE);
   s_end = min(ctx, s_begin + per * DEC_TILE);
+}
+
+// KV splits of a step, from its contexts. Ragged ones: split_tokens (whole tiles) deals the step's
+// tiles to about DEC_TARGET waves, so that one long context among short ones is cut as finely as the
+// step can use; near-equal ones (the mean at least 3/4 of the longest) are cut in the power of two
+// that gives 2048 waves or more, which leaves no short last split and CUs with equal shares (64 x
+// 1000 tokens: 59 us, by DEC_TARGET 62; 24 of 500 - 8000: 62 us, cut like equal ones 101). At least
+// DEC_MIN_TILES tiles a split, and no sequence takes more than num_splits. Sequence b has
+// max(1, ceil(context / split_tokens)) of them, listed sequence by sequence: `pair` of that list is
+// (b, split); b = -1 past its end. Every wave works this out for itself (B * hkv < 2048 where there
+// are splits): a few loads and scans.
+__host__ __device__ static inline int decode_even_splits(int items) {
+  int n = 1;
+  while ((long)items * n < 2048) n *= 2;
+  return n;
+}
+struct DecSplit { int b, split, split_tokens, last; };
+// inclusive scan over the wave's lanes (values >= 0) by lane shifts in the registers
+template <bool MAX>
+__device__ __forceinline__ int wave_scan(int v) {
+  const auto step = [&](int t) { v = MAX ? max(v, t) : v + t; };
+  step(__builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false));   // row_shr 1, 2, 4, 8
+  step(__builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false));
+  step(__builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false));
+  step(__builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false));
+  step(__builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));   // row_bcast 15, 31
+  step(__builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));
+  return v;
+}
+__device__ __forceinline__ DecSplit decode_split(const int* __restrict__ context_lens, int B, int hkv,
+                                                 int num_splits, int pair, int lane) {
+  // the first 256 contexts stay in registers
+  int ctx[4], sum = 0, longest = 0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) ctx[k] = 64 * k + lane < B ? context_lens[64 * k + lane] : 0;
+  const auto count = [&](int c) {
+    const int tiles = (c + DEC_TILE - 1) / DEC_TILE;
+    sum += tiles;
+    longest = max(longest, tiles);
+  };
+#pragma unroll
+  for (int k = 0; k < 4; ++k) count(ctx[k]);
+  for (int i = 256 + lane; i < B; i += 64) count(context_lens[i]);
+  sum = __builtin_amdgcn_readlane(wave_scan<false>(sum), 63);
+  longest = __builtin_amdgcn_readlane(wave_scan<true>(longest), 63);
+  const int even = decode_even_splits(B * hkv);
+  const int share = 4l * sum >= 3l * longest * B ? (longest + even - 1) / even
+                                                 : (sum * hkv + DEC_TARGET - 1) / DEC_TARGET;
+  const int per = max(max(share, (longest + num_splits - 1) / num_splits), DEC_MIN_TILES);
+  DecSplit r{-1, 0, per * DEC_TILE, 0};
+  const auto find = [&](int i0, int c) {
+    const int n = i0 + lane < B ? max(1, (c + r.split_tokens - 1) / r.split_tokens) : 0;
+    const int upto = wave_scan<false>(n);
+    const unsigned long long past = __ballot(upto > pair);
+    if (past) {
+      const int l = __ffsll(past) - 1;
+      r.b = i0 + l;
+      r.last = __builtin_amdgcn_readlane(n, l) - 1;
+      r.split = pair - (__builtin_amdgcn_readlane(upto, l) - 1 - r.last);
+    }
+    pair -= __builtin_amdgcn_readlane(upto, 63);
+    return past != 0;
+  };
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    if (64 * k >= B || find(64 * k, ctx[k])) return r;
+  for (int i0 = 256; i0 < B; i0 += 64)
+    if (find(i0, i0 + lane < B ? context_lens[i0 + lane] : 0)) return r;
+  return r;
+}
+// waves a split launch needs at most: the even splits, or DEC_TARGET and the rounding up of every
+// sequence
+static inline long decode_split_items(int items, int num_splits) {
+  const long even = (long)items * decode_even_splits(items), ragged = DEC_TARGET + items;
+  const long all = (long)items * num_splits, most = even > ragged ? even : ragged;
+  return all < most ? all : most;
 }
 
 template <int HD>
@@ -231,10 +310,12 @@ __global__ void __launch_bounds__(256, MINW) decode_attn_kernel(
   // one WAVE per work item (sequence, kv head, KV split): no LDS, no barriers, so every
   // resident wave of the chip streams a different (seq, head) pair concurrently
   const int item = blockIdx.x * DEC_WAVES + (threadIdx.x >> 6);
-  if (item >= B * hkv * num_splits) return;                    // wave-uniform exit
-  const int split = item % num_splits;
-  const int bh = item / num_splits;
-  const int kvh = bh % hkv, b = bh / hkv;
+  const int kvh = item % hkv;
+  DecSplit sp{item / hkv, 0, split_tokens, 0};
+  if (num_splits > 1) sp = decode_split(context_lens, B, hkv, num_splits, item / hkv, lane);
+  if (sp.b < 0 || sp.b >= B) return;                           // wave-uniform exit
+  const int b = sp.b, split = sp.split;
+  split_tokens = sp.split_tokens;
   const int col = lane & 15, grp = lane >> 4;
   const int G = hq / hkv;
   const int ctx = context_lens[b];
@@ -255,7 +336,11 @@ __global__ void __launch_bounds__(256, MINW) decode_attn_kernel(
   }
   decode_attn_core<HD>(qf, vt, lane, b, kvh, split, G, ctx, s_begin, s_end, out, k_cache,
                        v_cache, block_tables, max_blocks, hq, hkv, block_size, scale_log2,
-                       num_splits, ws_o, ws_ml);
+                       sp.last == 0 ? 1 : num_splits, ws_o, ws_ml);
+  // l = -1 ends the list for the reduce; a single split is the output itself and its list empty
+  const int end = sp.last == 0 ? 0 : split + 1;
+  if (num_splits > 1 && split == sp.last && end < num_splits && lane < G)
+    ws_ml[(((long)b * hq + kvh * G + lane) * num_splits + end) * 2 + 1] = -1.f;
 }
 
 // One (sequence, kv head) item per workgroup of WPI waves: wave wv walks the wv-th of WPI
@@ -748,34 +833,68 @@ __global__ void __launch_bounds__(256, 2) decode_attn_pipe_kernel(
   }
 }
 
-// out[b, h, :] = sum_s w_s o_s / sum_s w_s,  w_s = exp2(m_s - M) * l_s
+// out[b, h, :] = sum_s w_s o_s / sum_s w_s,  w_s = exp2(m_s - M) * l_s, over the splits before the
+// first one with l = -1; none: the row is there already. A wave per row, the splits' (m, l) one per
+// lane, up to 16 splits' outputs in flight: what another XCD wrote comes from memory, and a row has
+// up to 64 of them
 template <int HD>
 __global__ void __launch_bounds__(256) decode_reduce_kernel(u16* __restrict__ out,
                                                             const float* __restrict__ ws_o,
                                                             const float* __restrict__ ws_ml,
                                                             int B, int hq, int num_splits) {
-  const int per_row = HD / 8;
-  const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= (long)B * hq * per_row) return;
-  const long bh = gid / per_row;
-  const int d0 = (int)(gid % per_row) * 8;
+  constexpr int E = HD / 64;                      // dims per lane
+  const int lane = threadIdx.x & 63;
+  const long bh = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (bh >= (long)B * hq) return;
   const float* ml = ws_ml + bh * num_splits * 2;
-  float M = -INFINITY;
-  for (int s = 0; s < num_splits; ++s) M = fmaxf(M, ml[2 * s]);
-  float den = 0.f, acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  if (M != -INFINITY) {
-    for (int s = 0; s < num_splits; ++s) {
-      const float w = exp2f(ml[2 * s] - M) * ml[2 * s + 1];
-      den += w;
-      const float* o = ws_o + (bh * num_splits + s) * HD + d0;
+  float M = -INFINITY, den = 0.f, acc[E];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) acc[j] += w * o[j];
+  for (int j = 0; j < E; ++j) acc[j] = 0.f;
+  for (int s0 = 0; s0 < num_splits; s0 += 64) {
+    float m = -INFINITY, l = -1.f;
+    if (s0 + lane < num_splits) { m = ml[2 * (s0 + lane)]; l = ml[2 * (s0 + lane) + 1]; }
+    const unsigned long long end = __ballot(l == -1.f);
+    const int ns = end ? __ffsll(end) - 1 : 64;
+    if (ns == 0) {
+      if (s0 == 0) return;
+      break;
     }
+    if (lane >= ns) m = -INFINITY;
+    float top = m;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) top = fmaxf(top, __shfl_xor(top, o, 64));
+    top = fmaxf(top, M);
+    const float old = top == -INFINITY ? 1.f : exp2f(M - top);
+    den *= old;
+#pragma unroll
+    for (int j = 0; j < E; ++j) acc[j] *= old;
+    M = top;
+    const float w = lane >= ns || l == 0.f ? 0.f : exp2f(m - M) * l;
+    const float* o = ws_o + (bh * num_splits + s0) * HD + lane * E;
+    const auto batch = [&](auto depth, int s) {
+      constexpr int U = decltype(depth)::value;
+      float v[U][E];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int j = 0; j < E; ++j) v[u][j] = o[(long)min(s + u, ns - 1) * HD + j];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const float ws = s + u < ns ? __shfl(w, (s + u) & 63, 64) : 0.f;
+        den += ws;
+#pragma unroll
+        for (int j = 0; j < E; ++j) acc[j] += ws * v[u][j];
+      }
+      return s + U;
+    };
+    for (int s = 0; s < ns;)
+      s = ns - s > 4 ? batch(std::integral_constant<int, 16>{}, s)
+                     : batch(std::integral_constant<int, 4>{}, s);
+    if (ns < 64) break;
   }
   const float inv = den > 0.f ? 1.f / den : 0.f;
 #pragma unroll
-  for (int j = 0; j < 8; ++j) acc[j] *= inv;
-  store8(out + bh * HD + d0, acc);
+  for (int j = 0; j < E; ++j) out[bh * HD + lane * E + j] = f2bf(acc[j] * inv);
 }
 
 // pipelined (1), one-tile-per-round (0) or automatic (2, the default) decode kernel for hd 128
@@ -836,7 +955,8 @@ extern "C" int dli_decode_attention(void* out, const void* q, int q_stride, cons
         (u16*)out, (const u16*)q, q_stride, (const u16*)k_cache, (const u16*)v_cache,
         block_tables, max_blocks, context_lens, B, hq, hkv, block_size, scale_log2);
   } else {
-  dim3 grid((int)((items + DEC_WAVES - 1) / DEC_WAVES));
+  const long listed = num_splits > 1 ? decode_split_items(B * hkv, num_splits) : items;
+  dim3 grid((int)((listed + DEC_WAVES - 1) / DEC_WAVES));
   if (hd == 128)
     decode_attn_kernel<128, 4><<<grid, 64 * DEC_WAVES, 0, st>>>(
         (u16*)out, (const u16*)q, q_stride, (const u16*)k_cache, (const u16*)v_cache,
@@ -849,8 +969,7 @@ extern "C" int dli_decode_attention(void* out, const void* q, int q_stride, cons
         split_tokens, ws_o, ws_ml);
   }
   if (num_splits > 1) {
-    const long total = (long)B * hq * (hd / 8);
-    const int blocks = (int)((total + 255) / 256);
+    const int blocks = (int)(((long)B * hq + 3) / 4);
     if (hd == 128)
       decode_reduce_kernel<128><<<blocks, 256, 0, st>>>((u16*)out, ws_o, ws_ml, B, hq, num_splits);
     else

@@ -556,8 +556,8 @@ def prefill_attention_paged(qkv, cu_seqlens, max_seqlen: int, context_lens, bloc
 
 
 def decode_num_splits(B: int, hkv: int, max_context: int) -> int:
-    """KV splits so that the B*Hkv*splits work items (one wave each) fill the chip's ~2048
-    resident waves for long contexts, keeping >= 128 tokens per split."""
+    """KV split slots per sequence: 1 where the B*Hkv items (one wave each) or short contexts fill
+    the chip unsplit, else what the longest context may need."""
     items = B * hkv
     splits = 1
     # tiny batches (batch-1 latency): >= 512 tokens per split, so graphs captured for a
@@ -567,7 +567,11 @@ def decode_num_splits(B: int, hkv: int, max_context: int) -> int:
     min_tok = 512 if B <= 4 else 128
     while items * splits < 2048 and max_context // (splits * 2) >= min_tok and splits < 64:
         splits *= 2
-    return splits
+    if splits == 1:
+        return 1
+    # slots a sequence may use, of at least 64 tokens: the kernel deals the step's actual contexts
+    # to 2048 - 4096 waves, so one long context among short ones takes many slots
+    return max(splits, min(64, max_context // 64, 8192 // items))
 
 
 def decode_attention(qkv, k_cache, v_cache, block_tables, context_lens, max_context: int,

@@ -3,6 +3,7 @@
 // 128-wide slice of the value dimension), all heads in the workgroup because the head-mixing
 // matrix needs every head's normalised weights at the same (query, key).
 //
+// (Portions of 32 mixed heads of 128 channels run mix_attention.hip.)
 // With head mixing, two passes over the window in tiles of 32 keys (without it an unsplit
 // launch runs the usual single pass with rescaled accumulators):
 //   pass 1   S^T = K . Q^T per head (v_mfma_f32_16x16x32_bf16, K rows as operand A, so a lane

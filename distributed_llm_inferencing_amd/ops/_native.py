@@ -88,6 +88,9 @@ _SIGS = {
                              I, I, I, I, I, I, I, I, I, F, I, I, P, I, F, I, I, P],
     "dli_window_attention_mfma": [P, I, P, L, P, L, P, I, P, I, P, P, P, P, P,
                                   I, I, I, I, I, I, I, I, I, F, I, P, I, I, I, P, I, F, I, P],
+    "dli_mix_attention": [P, I, P, L, P, L, P, I, P, I, P, P, P, P, P, I, I, I, I, I, I, I, I, I, F,
+                          P, I, F, P],
+    "dli_mix_attention_workspace_bytes": [I],
     "dli_window_attention_mfma_workspace_bytes": [I, I, I, I, I, I, I, I],
     "dli_hgrn2": [P, I, P, P, P, F, P, P, P, P, P, I, I, I, I, I, I, I, P],
     "dli_gla": [P, I, P, I, P, F, F, P, F, P, P, P, P, P, I, I, I, I, I, I, I, P],

@@ -376,6 +376,19 @@ def window_attention(q, k_cache, v_cache, dq, dv, H, G, cu_seqlens, max_seqlen, 
                 return out
             if rc != _NOT_SUPPORTED:
                 raise RuntimeError(f"dli_swa_attention failed with hipError {rc}")
+        if talk is not None and Gk == G and not chunk and not keep_first and sink is None:
+            # portions of 32 mixed heads
+            rc = lib.dli_mix_attention(
+                _p(q), q.stride(0), _p(k_cache), k_cache.stride(0), _p(v_cache), v_cache.stride(0),
+                _p(out), out.stride(0), _p(gate), gate.stride(0) if gate is not None else 0,
+                _p(slopes), _p(talk), _p(cu_seqlens), _p(positions), _p(block_tables),
+                block_tables.stride(0), block_size, S, int(max_seqlen), H, G, dq, dv, int(window),
+                float(scale), _p(_gemm.workspace(q.device, lib.dli_mix_attention_workspace_bytes(T))),
+                hg, float(out_scale), _st())
+            if rc == 0:
+                return out
+            if rc != _NOT_SUPPORTED:
+                raise RuntimeError(f"dli_mix_attention failed with hipError {rc}")
         # the MFMA form; shapes it does not take (odd head sizes, > 32 heads) fall through
         # decode steps of heads that share one cached row per position (latent attention):
         # the heads become the query rows of a one-head problem

@@ -14,9 +14,17 @@
 //     S  <- diag(G) S + sum_j (B_j k_j) v_j^T
 // are four products of v_mfma_f32_16x16x4_f32. A block's 72 MFMAs of 32 cycles a wave at d = 128 are its
 // floor (1.9 us with two waves a SIMD); it takes 4 to 7 us, the rest being the gates and the LDS image.
-// The walk's floor is one token after another: 0.5 to 1.2 us each. 4 prompts of 2048 tokens, d = dv =
-// 128: HGRN2 1667 -> 621 us, GLA 2342 -> 704, FIXED 976 -> 517 (32 heads), MLSTM 1938 -> 895 (16 heads);
-// 32 prompts of 256: 680 -> 354, 824 -> 397, 508 -> 295, 423 -> 240.
+// The walk's floor is one token after another: 0.5 to 1.2 us each.
+//
+// A workgroup fills a CU, and there are as many as heads times sequences. Where that leaves CUs idle the
+// portions are cut in segments: a first launch forms each segment's state from nothing (no read-outs:
+// less than half the work), the second starts every segment from the fold of the states before it.
+//
+// d = dv = 128, HGRN2 / GLA / FIXED of 32 heads / MLSTM of 16, us; the walk, whole portions, segments:
+//   4 x 2048 tokens     1667  2342   976  1938     621   704   517   895     483   523   403   326
+//   998 to 2601 (5)                                768   891   650  1133     551   587   478   392
+//   1 x 8000                                      2325  2688  1972  3441     462   523   419   525
+//   32 x 256             680   824   508   423     354   397   295   240    (not cut)        211
 //
 // One workgroup of 8 waves per (head, sequence, 128 state columns); a wave owns 16 columns and all d
 // rows of S in its accumulators for the whole portion. The summation index of an MFMA may be permuted
@@ -122,25 +130,34 @@ struct ChunkArgs {
   const int* slots; const int* cu; const int* positions;
   void* out; int ldo; float out_scale;
   int H, d, dv;
+  const float* gates;                           // MLSTM: [T][H][4] = a, b, exp(-m)
+  // nseg > 1: the portions are cut in segments of seg_tokens, (sequence s, segment k, head h) being
+  // unit (s nseg + k) H + h of: the state after a segment, from nothing (from the portion's start for
+  // k = 0); its decay (a number a channel, or the first); its normaliser (MLSTM). Segment nseg - 1
+  // has no successor: its unit keeps the portion's first state.
+  int seg_tokens, nseg;
+  float* seg_state; float* seg_decay; float* seg_n;
 };
+constexpr int UNIT = 128;                       // floats of seg_decay and seg_n a unit
 
 // scalar decays of a block: A_i, b_j B_j, exp(-m_i), G, and D_ij = b_j prod_{j < t <= i} a_t
 struct Gates { float A[TB], kb[TB], em[TB], G[4], D[TB * LT]; };   // G as a sum of two floats
 
-template <int ND> struct Smem {
+// STATE: the image of a launch that forms the segments' states only
+template <int ND, bool STATE> struct Smem {
   static constexpr int DP = ND * 16, LQ = DP + 8;
-  float Q[2][TB * LQ];              // q (per-channel decays: A_i q_i), token-major
-  float K[2][TB * LQ];              // k (per-channel decays: k_j / A_j), token-major
   float Kb[2][DP * LT];             // B_j k_j, channel-major
   float V[2][COLS * LT];            // v, column-major
-  float P[2][ND][256];              // partial sums of P^T, an accumulator a lane
+  float Q[2][STATE ? 4 : TB * LQ];  // q (per-channel decays: A_i q_i), token-major
+  float K[2][STATE ? 4 : TB * LQ];  // k (per-channel decays: k_j / A_j), token-major
+  float P[2][ND][STATE ? 4 : 256];  // partial sums of P^T, an accumulator a lane
   float ss[2][TB][8];               // partial sums of squares of a row
 };
-template <int ND> struct ChannelSmem {          // per-channel decays
+template <int ND, bool STATE> struct ChannelSmem {          // per-channel decays
   float G[2][ND * 16];              // over the block
   float part[2][4][ND * 16];        // over 4 tokens
-  float raw[2][ND * 16][3 * TB + 4];  // q, k and decays of a channel below MIN_DECAY
-  float xP[2][256];                 // such channels' share of P, [j][i]
+  float raw[2][STATE ? 1 : ND * 16][3 * TB + 4];  // q, k and decays of a channel below MIN_DECAY
+  float xP[2][STATE ? 2 : 256];     // such channels' share of P, [j][i]
   unsigned long long bad[2][2];     // which channels
 };
 template <int ND> struct ScalarSmem {           // one decay a token
@@ -149,18 +166,26 @@ template <int ND> struct ScalarSmem {           // one decay a token
 };
 
 // ND * 16 >= d
-template <typename S, int ND, int MODE>
+// STATE: only the states after the segments that have a successor
+template <typename S, int ND, int MODE, bool STATE>
 __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
   constexpr bool CHANNEL = MODE == HGRN2 || MODE == GLA;
   constexpr int DP = ND * 16, LQ = DP + 8;
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
-  Smem<ND>& sm = *reinterpret_cast<Smem<ND>*>(smem_raw);
-  ChannelSmem<ND>& cm = *reinterpret_cast<ChannelSmem<ND>*>(smem_raw + sizeof(Smem<ND>));
-  ScalarSmem<ND>& gm = *reinterpret_cast<ScalarSmem<ND>*>(smem_raw + sizeof(Smem<ND>));
+  using Image = Smem<ND, STATE>;
+  using Channels = ChannelSmem<ND, STATE>;
+  Image& sm = *reinterpret_cast<Image*>(smem_raw);
+  Channels& cm = *reinterpret_cast<Channels*>(smem_raw + sizeof(Image));
+  ScalarSmem<ND>& gm = *reinterpret_cast<ScalarSmem<ND>*>(smem_raw + sizeof(Image));
   const int H = a.H, d = a.d, dv = a.dv;
-  const int h = blockIdx.x, s = blockIdx.y, c0 = blockIdx.z * COLS;
-  const int slot = a.slots[s], t0 = a.cu[s], t1 = a.cu[s + 1];
-  if (t1 <= t0) return;
+  const int segs = STATE ? a.nseg - 1 : a.nseg;
+  const int h = blockIdx.x, s = blockIdx.y / segs, seg = blockIdx.y % segs, c0 = blockIdx.z * COLS;
+  const int end = a.cu[s + 1], first = a.cu[s];
+  const int slot = a.slots[s], t0 = first + seg * a.seg_tokens;
+  if (end <= t0) return;
+  const int t1 = seg + 1 < a.nseg && end - t0 > a.seg_tokens ? t0 + a.seg_tokens : end;
+  const bool last = t1 == end, cut = end - first > a.seg_tokens;
+  if (STATE && (last || slot < 0)) return;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int fr = lane & 15, q = lane >> 4;
   const int col = c0 + w * 16 + fr;             // this lane's state column
@@ -175,22 +200,76 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
       }
     return;
   }
-  const bool fresh = a.positions[t0] == 0;
+  const bool fresh = a.positions[first] == 0;
   float* sp = a.state + ((long)slot * H + h) * d * dv + col;
   float* np = MODE == MLSTM ? a.nstate + ((long)slot * H + h) * (d + 1) : nullptr;
+  const auto unit = [&](int k) { return ((long)s * a.nseg + k) * H + h; };
+  const auto seg_st = [&](int k) { return a.seg_state + unit(k) * d * dv + col; };
   f32x4 st[ND];
+  const auto load_state = [&](const float* p, auto&& put) {
 #pragma unroll
-  for (int t = 0; t < ND; ++t)
+    for (int t = 0; t < ND; ++t)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int c = 16 * t + 4 * q + r;
-      st[t][r] = (!fresh && on && c < d) ? sp[(long)c * dv] : 0.f;
+      for (int r = 0; r < 4; ++r) {
+        const int c = 16 * t + 4 * q + r;
+        put(t, r, p != nullptr && on && c < d ? p[(long)c * dv] : 0.f);
+      }
+  };
+  const auto store_state = [&](float* p) {
+    if (on) {
+#pragma unroll
+      for (int t = 0; t < ND; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int c = 16 * t + 4 * q + r;
+          if (c < d) p[(long)c * dv] = st[t][r];
+        }
     }
-  float m_run = 0.f;                            // the gate wave's running maximum
-  if (MODE == MLSTM) {
-    if (!fresh) m_run = np[d];
-    if (w < ND && q == 0) gm.n[16 * w + fr] = (!fresh && 16 * w + fr < d) ? np[16 * w + fr] : 0.f;
+  };
+  // The first state. Where the portion is cut, the output launch's last segment replaces the state
+  // that the first one starts from, in any order: the first reads the copy that the state launch
+  // took. Later segments fold the states before them.
+  const int nc = w * 16 + fr;                   // this lane's channel of the normaliser
+  float n0 = 0.f;
+  if (seg == 0) {
+    const bool copied = !STATE && cut;
+    load_state(fresh ? nullptr : copied ? seg_st(a.nseg - 1) : sp,
+               [&](int t, int r, float x) { st[t][r] = x; });
+    if (MODE == MLSTM && !fresh && nc < d) n0 = copied ? a.seg_n[unit(a.nseg - 1) * UNIT + nc] : np[nc];
+    if (STATE && !fresh) {
+      store_state(seg_st(a.nseg - 1));
+      if (MODE == MLSTM && q == 0 && nc < d) a.seg_n[unit(a.nseg - 1) * UNIT + nc] = n0;
+    }
+  } else {
+    load_state(STATE ? nullptr : seg_st(0), [&](int t, int r, float x) { st[t][r] = x; });
+    if (!STATE) {
+      if (MODE == MLSTM && nc < d) n0 = a.seg_n[unit(0) * UNIT + nc];
+      float Gs = 0.f, Gl = 0.f;
+      if (MODE == FIXED) {                      // a segment's decay, as in scalar_gates
+        double p = 1.0, x = (double)a.decays[h];
+        for (int e = a.seg_tokens; e; e >>= 1, x *= x)
+          if (e & 1) p *= x;
+        Gs = (float)p;
+        Gl = (float)(p - (double)Gs);
+      }
+      for (int k = 1; k < seg; ++k) {
+        const float* dec = a.seg_decay + unit(k) * UNIT;
+        if (MODE == MLSTM) {
+          Gs = dec[0];
+          if (nc < d) n0 = Gs * n0 + a.seg_n[unit(k) * UNIT + nc];
+        }
+#pragma unroll
+        for (int t = 0; t < ND; ++t) {
+          if (CHANNEL) st[t] *= *reinterpret_cast<const f32x4*>(dec + 16 * t + 4 * q);
+          else if (MODE == FIXED) st[t] = st[t] * Gs + st[t] * Gl;
+          else st[t] *= Gs;
+        }
+        load_state(seg_st(k), [&](int t, int r, float x) { st[t][r] += x; });
+      }
+    }
   }
+  if (MODE == MLSTM && w < ND && q == 0) gm.n[nc] = n0;
+  float G_seg = 1.f;                            // STATE: this thread's channel's, or the gate wave's
   // staging: thread = (channel sc and column sc of the block's 128, tokens 4 tg .. 4 tg + 3)
   const int sc = tid & 127, tg = tid >> 7;
   const bool chan = sc < d, scol = c0 + sc < dv;
@@ -200,11 +279,11 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
     if (MODE == HGRN2) low = ldf((const S*)a.lower + h * d + sc);
   }
   const int goff = 2 * H * d + H * dv + h * dv + col;           // output gate
-  const int ioff = 2 * H * d + 2 * H * dv + h;                  // MLSTM gates
   constexpr int GW = 7;                                         // the gate wave
   const int nb = (t1 - t0 + TB - 1) / TB;
   auto tokens = [&](int b) { return min(TB, t1 - t0 - b * TB); };
-  float rq[4], rk[4], rz[4], rv[4], ra[4], gin = 0.f;
+  float rq[4], rk[4], rz[4], rv[4], ra[4];
+  f32x4 gin = {1.f, 0.f, 0.f, 0.f};
   auto load = [&](int b) {
     const int tc = t0 + b * TB, n = tokens(b);
 #pragma unroll
@@ -214,7 +293,7 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
       if (t < n) {
         const float* row = a.proj + (long)(tc + t) * a.ldp;
         if (chan) {
-          rq[u] = row[h * d + sc];
+          if (!STATE) rq[u] = row[h * d + sc];
           rk[u] = row[H * d + h * d + sc];
           if (MODE == GLA) rz[u] = a.z[(long)(tc + t) * a.ldz + h * d + sc];
         }
@@ -222,9 +301,9 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
       }
     }
   };
-  auto load_gates = [&](int b) {                // MLSTM: the gate wave's rows of 16 lanes, i | f | i | f
+  auto load_gates = [&](int b) {                // MLSTM: the gate wave's
     if (MODE == MLSTM && w == GW && b < nb && fr < tokens(b))
-      gin = a.proj[(long)(t0 + b * TB + fr) * a.ldp + ioff + (q & 1) * H];
+      gin = *reinterpret_cast<const f32x4*>(a.gates + ((long)(t0 + b * TB + fr) * H + h) * 4);
   };
   // per-channel decays of the block in the registers, and their products over 4 tokens
   auto channel_gates = [&](int b) {
@@ -270,21 +349,9 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
       }
       return;
     }
-    const float y = a.cap * tanhf((gin + a.if_b[(q & 1) * H + h]) / a.cap);      // odd rows: forget gates
-    const float ls = logsigmoid32(y);
-    const float ig = fr < n ? __shfl(y, fr, 64) : -INFINITY;
-    const float fg = fr < n ? __shfl(ls, 16 + fr, 64) : 0.f;
-    float ft = 0.f, mt = 0.f;
-#pragma unroll
-    for (int t = 0; t < TB; ++t) {
-      const float f = from_lane(fg, t) + m_run;
-      m_run = fmaxf(f, from_lane(ig, t));
-      ft = fr == t ? f : ft;
-      mt = fr == t ? m_run : mt;
-    }
-    at = expf(ft - mt);
-    bt = expf(ig - mt);
-    em = expf(-mt);
+    at = fr < n ? gin[0] : 1.f;
+    bt = fr < n ? gin[1] : 0.f;
+    em = fr < n ? gin[2] : 0.f;
     float A = at, B = at;                       // products up to a token, and from it on
 #define PRODUCTS(N) A *= row<0x110 + N>(1.f, A), B *= row<0x100 + N>(1.f, B)
     PRODUCTS(1); PRODUCTS(2); PRODUCTS(4); PRODUCTS(8);
@@ -313,6 +380,7 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
       gt.em[lane] = em;
     }
     if (lane == 0) gt.G[0] = G;
+    G_seg *= G;
   };
   // fixed decays: table 0 for full blocks, 1 for a shorter last one
   auto table = [&](int b) -> Gates& { return gm.g[MODE == FIXED ? int(tokens(b) < TB) : (b & 3)]; };
@@ -335,16 +403,18 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
         const bool bad = !(G >= MIN_DECAY);
         if (tg == 0) {
           cm.G[buf][sc] = G;
+          if (STATE) G_seg *= G;
           const unsigned long long m = __ballot(bad);
           if (lane == 0) cm.bad[buf][w] = m;
         }
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           const int t = 4 * tg + u;
+          kb[u] = rk[u] * B[u];
+          if (STATE) continue;
           const float qq = MODE == HGRN2 ? silu1(rq[u]) : rq[u] * a.qscale;
           sm.Q[buf][t * LQ + sc] = qq * A[u];
           sm.K[buf][t * LQ + sc] = bad ? 0.f : rk[u] * rcp1(A[u]);
-          kb[u] = rk[u] * B[u];
           if (bad) {
             cm.raw[buf][sc][t] = qq;
             cm.raw[buf][sc][TB + t] = rk[u];
@@ -356,11 +426,12 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           const int t = 4 * tg + u;
-          const float qq = MODE == FIXED ? silu1(rq[u]) : rq[u] * a.qscale;
           const float kk = MODE == FIXED ? silu1(rk[u]) : rk[u];
+          kb[u] = kk * kw[u];
+          if (STATE) continue;
+          const float qq = MODE == FIXED ? silu1(rq[u]) : rq[u] * a.qscale;
           sm.Q[buf][t * LQ + sc] = qq;
           sm.K[buf][t * LQ + sc] = kk;
-          kb[u] = kk * kw[u];
         }
       }
       *reinterpret_cast<f32x4*>(sm.Kb[buf] + sc * LT + 4 * tg) = kb;
@@ -376,17 +447,22 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
   auto products = [&](int b) {
     const int buf = b & 1;
     const float* Q = sm.Q[buf];
-    if (w < ND) {                               // this wave's 16 channels of P^T
-      const f32x4 qf = *reinterpret_cast<const f32x4*>(Q + fr * LQ + 16 * w + 4 * q);
-      const f32x4 kf = *reinterpret_cast<const f32x4*>(sm.K[buf] + fr * LQ + 16 * w + 4 * q);
-      const f32x4 p = mfma4(kf, qf, f32x4{0.f, 0.f, 0.f, 0.f});
-      *reinterpret_cast<f32x4*>(&sm.P[buf][w][4 * lane]) = p;
+    if (w < ND && (!STATE || MODE == MLSTM)) {  // this wave's 16 channels of P^T
+      f32x4 qf;
+      if (!STATE) {
+        qf = *reinterpret_cast<const f32x4*>(Q + fr * LQ + 16 * w + 4 * q);
+        const f32x4 kf = *reinterpret_cast<const f32x4*>(sm.K[buf] + fr * LQ + 16 * w + 4 * q);
+        const f32x4 p = mfma4(kf, qf, f32x4{0.f, 0.f, 0.f, 0.f});
+        *reinterpret_cast<f32x4*>(&sm.P[buf][w][4 * lane]) = p;
+      }
       if (MODE == MLSTM) {                      // n . q_i over them, then n after the block
-        const f32x4 nf = *reinterpret_cast<const f32x4*>(gm.n + 16 * w + 4 * q);
-        float x = (nf[0] * qf[0] + nf[1] * qf[1]) + (nf[2] * qf[2] + nf[3] * qf[3]);
-        x += __shfl_xor(x, 16, 64);
-        x += __shfl_xor(x, 32, 64);
-        if (q == 0) gm.nq[buf][w][fr] = x;
+        if (!STATE) {
+          const f32x4 nf = *reinterpret_cast<const f32x4*>(gm.n + 16 * w + 4 * q);
+          float x = (nf[0] * qf[0] + nf[1] * qf[1]) + (nf[2] * qf[2] + nf[3] * qf[3]);
+          x += __shfl_xor(x, 16, 64);
+          x += __shfl_xor(x, 32, 64);
+          if (q == 0) gm.nq[buf][w][fr] = x;
+        }
         const f32x4 kb = *reinterpret_cast<const f32x4*>(sm.Kb[buf] + (16 * w + fr) * LT + 4 * q);
         float y = (kb[0] + kb[1]) + (kb[2] + kb[3]);
         y += __shfl_xor(y, 16, 64);
@@ -394,7 +470,7 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
         if (q == 0) gm.n[16 * w + fr] = table(b).G[0] * gm.n[16 * w + fr] + y;
       }
     }
-    if constexpr (CHANNEL) {
+    if constexpr (CHANNEL && !STATE) {
       bad0n = cm.bad[buf][0];
       bad1n = DP > 64 ? cm.bad[buf][1] : 0;
       if ((bad0n | bad1n) != 0 && tid < 256) {
@@ -422,7 +498,8 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
       if (MODE == FIXED) Gl = table(b).G[1];
 #pragma unroll
       for (int t = 0; t < ND; ++t) {            // tile t's read-out and update side by side
-        const f32x4 qf = *reinterpret_cast<const f32x4*>(Q + fr * LQ + 16 * t + 4 * q);
+        f32x4 qf;
+        if (!STATE) qf = *reinterpret_cast<const f32x4*>(Q + fr * LQ + 16 * t + 4 * q);
         const f32x4 kb = *reinterpret_cast<const f32x4*>(sm.Kb[buf] + (16 * t + fr) * LT + 4 * q);
         f32x4 sn;
         if constexpr (CHANNEL) sn = st[t] * *reinterpret_cast<const f32x4*>(cm.G[buf] + 16 * t + 4 * q);
@@ -430,7 +507,8 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
         if (MODE == FIXED) sn += st[t] * Gl;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          part[t & 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[r], st[t][r], part[t & 3], 0, 0, 0);
+          if (!STATE)
+            part[t & 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[r], st[t][r], part[t & 3], 0, 0, 0);
           sn = __builtin_amdgcn_mfma_f32_16x16x4f32(kb[r], vfn[r], sn, 0, 0, 0);
         }
         st[t] = sn;
@@ -440,7 +518,7 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
   };
   f32x4 o = {0.f, 0.f, 0.f, 0.f}, gate = o;
   float nw = 0.f;
-  if (MODE != FIXED && on) nw = ldf((const S*)a.norm_w + (MODE == MLSTM ? h * dv + col : col));
+  if (!STATE && MODE != FIXED && on) nw = ldf((const S*)a.norm_w + (MODE == MLSTM ? h * dv + col : col));
   // o = the read-outs of block b (rows 4 q + r, this lane's column) from vf, acc and P
   auto finish = [&](int b) {
     const int buf = b & 1;
@@ -535,7 +613,7 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
   }
   __syncthreads();
 #pragma unroll 1
-  for (int b = 0; b < nb + 2; ++b) {
+  for (int b = 0; b < nb + (STATE ? 0 : 2); ++b) {
     if (b + 1 < nb) stage(b + 1);
     if (b + 2 < nb) {
       load(b + 2);
@@ -544,43 +622,101 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
         load_gates(b + 3);
       }
     }
-    if (w < 4 && b < nb) products(b);
-    if (b >= 2) write_out(b - 2);
-    if (b >= 1 && b <= nb) finish(b - 1);
-    if (w >= 4 && b < nb) products(b);
-    vf = vfn; acc = accn; bad0 = bad0n; bad1 = bad1n;
+    if constexpr (STATE) {
+      products(b);
+    } else {
+      if (w < 4 && b < nb) products(b);
+      if (b >= 2) write_out(b - 2);
+      if (b >= 1 && b <= nb) finish(b - 1);
+      if (w >= 4 && b < nb) products(b);
+      vf = vfn; acc = accn; bad0 = bad0n; bad1 = bad1n;
+    }
     if constexpr (CHANNEL) {
       if (b + 2 < nb) channel_gates(b + 2);
     }
     lds_barrier();
   }
-  if (on) {
-#pragma unroll
-    for (int t = 0; t < ND; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int c = 16 * t + 4 * q + r;
-        if (c < d) sp[(long)c * dv] = st[t][r];
-      }
-  }
-  if (MODE == MLSTM) {
-    if (w < ND && q == 0 && 16 * w + fr < d) np[16 * w + fr] = gm.n[16 * w + fr];
-    if (w == GW && lane == 0) np[d] = m_run;
+  if constexpr (STATE) {
+    store_state(seg_st(seg));
+    if (CHANNEL && tg == 0 && blockIdx.z == 0) a.seg_decay[unit(seg) * UNIT + sc] = sc < DP ? G_seg : 1.f;
+    if (MODE == MLSTM) {
+      if (w < ND && q == 0 && nc < d) a.seg_n[unit(seg) * UNIT + nc] = gm.n[nc];
+      if (w == GW && lane == 0) a.seg_decay[unit(seg) * UNIT] = G_seg;
+    }
+  } else if (last) {
+    store_state(sp);
+    if (MODE == MLSTM && w < ND && q == 0 && nc < d) np[nc] = gm.n[nc];
   }
 }
 
-template <typename S, int ND, int MODE>
+// MLSTM's gates: a_t = exp(f_t + m_{t-1} - m_t), b_t = exp(i_t - m_t) and exp(-m_t) of every token of a
+// (head, sequence), and the state's m after the portion. Only m is a walk, of an addition and a maximum
+// a token (2600 tokens some 20 us); inside the products' launch, where one wave did this for a block
+// beside its share of the products, it was what the other waves waited for.
+__global__ void __launch_bounds__(512) mlstm_gates_kernel(ChunkArgs a, float* gates) {
+  constexpr int N = 1024;
+  __shared__ float ig[N], fg[N], m[N + 1];
+  const int h = blockIdx.x, s = blockIdx.y, H = a.H, tid = threadIdx.x, lane = tid & 63;
+  const int slot = a.slots[s], first = a.cu[s], end = a.cu[s + 1];
+  if (slot < 0 || end <= first) return;
+  float* mp = a.nstate + ((long)slot * H + h) * (a.d + 1) + a.d;
+  const int ioff = 2 * H * a.d + 2 * H * a.dv + h;
+  if (tid == 0) m[0] = a.positions[first] == 0 ? 0.f : *mp;
+  for (int t0 = first; t0 < end; t0 += N) {
+    const int n = min(N, end - t0);
+    for (int t = tid; t < n; t += 512) {
+      const float* row = a.proj + (long)(t0 + t) * a.ldp + ioff;
+      ig[t] = a.cap * tanhf((row[0] + a.if_b[h]) / a.cap);
+      fg[t] = logsigmoid32(a.cap * tanhf((row[H] + a.if_b[H + h]) / a.cap));
+    }
+    __syncthreads();
+    if (tid < 64) {
+      float run = m[0];
+      for (int t = 0; t < n; t += 64) {
+        const float i = t + lane < n ? ig[t + lane] : -INFINITY, f = t + lane < n ? fg[t + lane] : 0.f;
+        float own = 0.f;
+#pragma unroll
+        for (int u = 0; u < 64; ++u) {
+          run = fmaxf(from_lane(f, u) + run, from_lane(i, u));
+          own = lane == u ? run : own;
+        }
+        if (t + lane < n) m[t + lane + 1] = own;
+      }
+    }
+    __syncthreads();
+    for (int t = tid; t < n; t += 512) {
+      const float mt = m[t + 1];
+      *reinterpret_cast<f32x4*>(gates + ((long)(t0 + t) * H + h) * 4) =
+          f32x4{expf(fg[t] + m[t] - mt), expf(ig[t] - mt), expf(-mt), 0.f};
+    }
+    __syncthreads();
+    if (tid == 0) m[0] = m[n];
+    __syncthreads();
+  }
+  if (tid == 0) *mp = m[0];
+}
+
+template <typename S, int ND, int MODE, bool STATE>
 int launch_chunks(const ChunkArgs& a, int num_seqs, hipStream_t st) {
-  constexpr size_t sh = sizeof(Smem<ND>) + (MODE <= GLA ? sizeof(ChannelSmem<ND>) : sizeof(ScalarSmem<ND>));
-  static_assert(sh <= 160 * 1024 && sizeof(Smem<ND>) % 16 == 0, "LDS image");
+  constexpr size_t sh = sizeof(Smem<ND, STATE>) +
+                        (MODE <= GLA ? sizeof(ChannelSmem<ND, STATE>) : sizeof(ScalarSmem<ND>));
+  static_assert(sh <= 160 * 1024 && sizeof(Smem<ND, STATE>) % 16 == 0, "LDS image");
   if (sh > 48 * 1024) {
-    hipError_t e = hipFuncSetAttribute((const void*)recurrence_chunk_kernel<S, ND, MODE>,
+    hipError_t e = hipFuncSetAttribute((const void*)recurrence_chunk_kernel<S, ND, MODE, STATE>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh);
     if (e != hipSuccess) return (int)e;
   }
-  dim3 grid(a.H, num_seqs, (a.dv + COLS - 1) / COLS);
-  recurrence_chunk_kernel<S, ND, MODE><<<grid, NTH, sh, st>>>(a);
+  dim3 grid(a.H, num_seqs * (STATE ? a.nseg - 1 : a.nseg), (a.dv + COLS - 1) / COLS);
+  recurrence_chunk_kernel<S, ND, MODE, STATE><<<grid, NTH, sh, st>>>(a);
   DLI_RETURN_LAUNCH();
+}
+template <typename S, int ND, int MODE>
+int launch_chunks(const ChunkArgs& a, int num_seqs, hipStream_t st) {
+  if (a.nseg > 1) {
+    const int rc = launch_chunks<S, ND, MODE, true>(a, num_seqs, st);
+    if (rc) return rc;
+  }
+  return launch_chunks<S, ND, MODE, false>(a, num_seqs, st);
 }
 
 template <typename S, int MODE>
@@ -590,7 +726,41 @@ int launch_by_width(const ChunkArgs& a, int num_seqs, hipStream_t st) {
   return launch_chunks<S, 8, MODE>(a, num_seqs, st);
 }
 
+// Segments of a portion of at most max_seqlen tokens (T in all): a CU takes one workgroup, so few heads
+// and sequences, or ragged ones, leave most of the chip idle for as long as the longest portion takes.
+// Cut, every segment but the last runs twice, the first time (states only, several workgroups a CU) at
+// some 0.4 of a block's time. In block times, with 3 to fill and drain a workgroup and the fold.
+static int pick_segments(int H, int dv, int num_seqs, int max_seqlen, int T) {
+  const long wg = (long)H * ((dv + COLS - 1) / COLS);
+  const auto rounds = [&](long units) { return (units * wg + 255) / 256; };
+  float best = 0.9f * rounds(num_seqs) * (max_seqlen / 16 + 3.f);
+  int pick = 1;
+  for (int n = 2; n <= 16 && (long)num_seqs * n <= 65535; ++n) {
+    const int len = ((max_seqlen + n - 1) / n + TB - 1) / TB * TB;
+    if (len < 128) break;
+    const int k = (max_seqlen + len - 1) / len;
+    const long all = (long)num_seqs * k, most = T / len + num_seqs, units = all < most ? all : most;
+    const float cost = rounds(units) * (len / 16 + 3.f) * 1.4f + 0.4f * k;
+    if (cost < best) { best = cost; pick = k; }
+  }
+  return pick;
+}
+static int segment_tokens(int max_seqlen, int nseg) {
+  return ((max_seqlen + nseg - 1) / nseg + TB - 1) / TB * TB;
+}
+
 }  // namespace
+
+static size_t unit_floats(int d, int dv) { return (size_t)d * dv + 2 * UNIT; }
+
+// scratch that dli_recurrence_chunks takes for a step of T tokens (nullptr there: portions stay whole,
+// which MLSTM does not take)
+extern "C" long dli_recurrence_workspace_bytes(int mode, int num_seqs, int max_seqlen, int T, int H,
+                                               int d, int dv) {
+  const int n = pick_segments(H, dv, num_seqs, max_seqlen, T);
+  const size_t gates = mode == MLSTM ? (size_t)T * H * 4 : 0;
+  return (long)((gates + (n > 1 ? (size_t)num_seqs * n * H * unit_floats(d, dv) : 0)) * 4);
+}
 
 // Portions of a step's sequences (mode as above). hipErrorNotSupported: a size that the walk takes
 // (d > 128, or a normed head wider than 128).
@@ -599,15 +769,31 @@ extern "C" int dli_recurrence_chunks(int mode, const float* proj, int ldp, const
                                      const float* decays, const float* if_b, float cap,
                                      const void* norm_w, float eps, float* state, float* nstate,
                                      const int* slots, const int* cu, const int* positions, void* out,
-                                     int ldo, float out_scale, int num_seqs, int H, int d, int dv,
-                                     int dt, hipStream_t st) {
-  if (num_seqs <= 0) return 0;
+                                     int ldo, float out_scale, int num_seqs, int max_seqlen, int T,
+                                     int H, int d, int dv, int dt, void* ws, hipStream_t st) {
+  if (num_seqs <= 0 || max_seqlen <= 0) return 0;
   if (H < 1 || d < 1 || dv < 1 || num_seqs > 65535 || state == nullptr || slots == nullptr ||
       out == nullptr || (dt != 0 && dt != 1))
     return (int)hipErrorInvalidValue;
   if (d > 128 || (mode != FIXED && dv > COLS)) return (int)hipErrorNotSupported;
   ChunkArgs a{proj, ldp, z, ldz, bias, lower, inv_tau, qscale, decays, if_b, cap, norm_w, eps, state,
-              nstate, slots, cu, positions, out, ldo, out_scale, H, d, dv};
+              nstate, slots, cu, positions, out, ldo, out_scale, H, d, dv, nullptr, 1 << 30, 1,
+              nullptr, nullptr, nullptr};
+  const int nseg = ws != nullptr ? pick_segments(H, dv, num_seqs, max_seqlen, T) : 1;
+  float* scratch = (float*)ws;
+  float* gates = scratch;
+  if (mode == MLSTM) {
+    a.gates = gates;
+    scratch += (size_t)T * H * 4;
+  }
+  if (nseg > 1) {
+    a.nseg = nseg;
+    a.seg_tokens = segment_tokens(max_seqlen, nseg);
+    const size_t units = (size_t)num_seqs * nseg * H;
+    a.seg_decay = scratch;
+    a.seg_n = a.seg_decay + units * UNIT;
+    a.seg_state = a.seg_n + units * UNIT;
+  }
   switch (mode) {
     case HGRN2:
       if (bias == nullptr || lower == nullptr || norm_w == nullptr) break;
@@ -619,7 +805,8 @@ extern "C" int dli_recurrence_chunks(int mode, const float* proj, int ldp, const
       if (decays == nullptr) break;
       return launch_by_width<float, FIXED>(a, num_seqs, st);
     case MLSTM:
-      if (if_b == nullptr || norm_w == nullptr || nstate == nullptr || !(cap > 0.f)) break;
+      if (if_b == nullptr || norm_w == nullptr || nstate == nullptr || !(cap > 0.f) || ws == nullptr) break;
+      mlstm_gates_kernel<<<dim3(H, num_seqs), 512, 0, st>>>(a, gates);
       return dt == 0 ? launch_by_width<u16, MLSTM>(a, num_seqs, st) : launch_by_width<float, MLSTM>(a, num_seqs, st);
   }
   return (int)hipErrorInvalidValue;

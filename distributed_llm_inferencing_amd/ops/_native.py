@@ -96,7 +96,8 @@ _SIGS = {
     "dli_gla": [P, I, P, I, P, F, F, P, F, P, P, P, P, P, I, I, I, I, I, I, I, P],
     # portions of the linear recurrences (recurrent_chunk.hip)
     "dli_recurrence_chunks": [I, P, I, P, I, P, P, F, F, P, P, F, P, F, P, P, P, P, P, P, I, F, I, I, I,
-                              I, I, P],
+                              I, I, I, I, P, P],
+    "dli_recurrence_workspace_bytes": [I, I, I, I, I, I, I],
     # post-norm designs (postnorm.hip)
     "dli_prev_tokens": [P, P, P, P, P, P, I, I, P],
     "dli_embedding_bigram": [P, P, P, P, P, P, I, I, I, I, I, I, I, P],

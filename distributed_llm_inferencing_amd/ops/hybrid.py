@@ -475,11 +475,14 @@ def _recurrence_chunks(mode: int, proj, state, slots, cu_seqlens, positions, out
     most 128 channels, normed ones of at most 128 columns. False: nothing was launched."""
     if int(max_seqlen) < CHUNK_MIN_TOKENS or d > 128 or (dv > 128 and mode != _CHUNK_FIXED):
         return False
+    S, T = cu_seqlens.shape[0] - 1, proj.shape[0]
+    nb = N.require_native().dli_recurrence_workspace_bytes(mode, S, int(max_seqlen), T, H, d, dv)
+    ws = _gemm.workspace(proj.device, nb) if nb else None
     _call("dli_recurrence_chunks", mode, _p(proj), proj.stride(0), _p(z),
           z.stride(0) if z is not None else 0, _p(bias), _p(lower), float(inv_tau), float(qscale),
           _p(decays), _p(if_b), float(cap), _p(norm_w), float(eps), _p(state), _p(nstate), _p(slots),
           _p(cu_seqlens), _p(positions), _p(out), out.stride(0), float(out_scale),
-          cu_seqlens.shape[0] - 1, H, d, dv, _dt(dtype), _st())
+          S, int(max_seqlen), T, H, d, dv, _dt(dtype), _p(ws), _st())
     return True
 
 

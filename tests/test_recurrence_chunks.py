@@ -75,10 +75,28 @@ def oracle(mode, proj, extra, state, nstate, lens, slots, first, heads, d, dv, e
                                          (24, 20, False), (16, 128, True)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_portions_match_a_float64_walk(gpu, mode, d, dv, strong, dtype):
-    heads, eps = 3, 1e-6
     if mode == "lightning" and dv == 48:
         dv = 200                                     # raw read-outs: more than one column block
-    lens, slots, first = [1, 16, 0, 17, 100, 33, 5], [4, 0, 1, 2, 5, 3, -1], [0, 1, 0, 0, 1, 0, 0]
+    check(gpu, mode, d, dv, strong, dtype, [1, 16, 0, 17, 100, 33, 5], [4, 0, 1, 2, 5, 3, -1],
+          [0, 1, 0, 0, 1, 0, 0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["hgrn2", "gla", "lightning", "mlstm"])
+@pytest.mark.parametrize("d,dv,strong", [(128, 128, False), (32, 48, True)])
+@pytest.mark.parametrize("lens,slots,first", [
+    # segments of 144 tokens: last ones of 1 and 16 tokens, portions of one segment and of exactly
+    # one, new and continued states, padding
+    ([289, 144, 704, 1, 400, 145], [4, 0, 1, 2, -1, 3], [0, 1, 0, 0, 1, 1]),
+    ([1500], [3], [0]), ([1500], [3], [1])])
+def test_portions_cut_in_segments(gpu, mode, d, dv, strong, lens, slots, first):
+    if mode == "lightning" and dv == 48:
+        dv = 200
+    check(gpu, mode, d, dv, strong, torch.float32, lens, slots, first)
+
+
+def check(gpu, mode, d, dv, strong, dtype, lens, slots, first):
+    heads, eps = 3, 1e-6
     g = torch.Generator().manual_seed(d * 7 + dv + strong)
     rnd = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
     T, wide = sum(lens), 2 * heads * (d + dv) + 2 * heads

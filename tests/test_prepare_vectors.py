@@ -68,3 +68,23 @@ def test_mla_prepare(heads, d, dr, r, rot, pad, dtype):
 def test_concat_cast(D, dtype):
     a, b = torch.randn(5, D), torch.randn(5, D)
     assert torch.equal(H.concat_cast(a.cuda(), b.cuda(), dtype).cpu(), torch.cat([a, b], 1).to(dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("heads,G,d,dv,rot,pad", [(32, 8, 128, 128, 64, 4), (4, 2, 24, 20, 24, 0), (4, 1, 32, 8, 8, 0),
+                                                  (6, 3, 64, 64, 0, 0), (4, 2, 24, 20, 20, 0), (4, 2, 24, 18, 8, 1)])
+def test_sink_prepare(heads, G, d, dv, rot, pad, dtype):
+    g = torch.Generator().manual_seed(d + rot)
+    T, W = 6, (heads + G) * d + G * dv
+    proj = torch.randn(T, W + pad, generator=g)
+    qw, kw = (torch.randn(n * d, generator=g).to(dtype) for n in (heads, G))
+    slots, pos = torch.tensor([3, -1, 0, 7, 1, 2]).int(), torch.tensor([0, 1, 5, 4000, 31000, 7]).int()
+    freq = torch.pow(10000.0, -torch.arange(max(1, rot // 2)).double() / max(1, rot // 2))
+    kc, vc = torch.full((8, G * d), 5.0, dtype=dtype), torch.full((8, G * dv), 5.0, dtype=dtype)
+    kd, vd = kc.cuda(), vc.cuda()
+    want = R.sink_prepare(proj[:, :W], qw, kw, 1e-6, heads, G, d, dv, rot, freq[:rot // 2], 1.3, pos, kc, vc,
+                          slots, dtype)
+    got = H.sink_prepare(proj.cuda()[:, :W], qw.cuda(), kw.cuda(), 1e-6, heads, G, d, dv, rot, freq.cuda(), 1.3,
+                         pos.cuda(), kd, vd, slots.cuda())
+    for a, b in ((got, want), (kd, kc), (vd, vc)):
+        close(a.reshape(-1), b.reshape(-1), dtype)

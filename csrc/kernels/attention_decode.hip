@@ -62,7 +62,7 @@ __device__ __forceinline__ void decode_wg_range(int ctx, int wv, int& s_begin, i
 // that gives 2048 waves or more, which leaves no short last split and CUs with equal shares (64 x
 // 1000 tokens: 59 us, by DEC_TARGET 62; 24 of 500 - 8000: 62 us, cut like equal ones 101). At least
 // DEC_MIN_TILES tiles a split, and no sequence takes more than num_splits. Sequence b has
-// max(1, ceil(context / split_tokens)) of them, listed sequence by sequence: `pair` of that list is
+// max(1, ceil(context / split_tokens)) equal ones, listed sequence by sequence: `pair` of that list is
 // (b, split); b = -1 past its end. Every wave works this out for itself (B * hkv < 2048 where there
 // are splits): a few loads and scans.
 __host__ __device__ static inline int decode_even_splits(int items) {
@@ -113,6 +113,10 @@ __device__ __forceinline__ DecSplit decode_split(const int* __restrict__ context
       r.b = i0 + l;
       r.last = __builtin_amdgcn_readlane(n, l) - 1;
       r.split = pair - (__builtin_amdgcn_readlane(upto, l) - 1 - r.last);
+      // equal splits: a short last one, at the same place of every sequence's list, would fall to the
+      // same XCDs (200 contexts of 700 - 1000, two splits each: 169 -> 164 us)
+      const int tiles = (__builtin_amdgcn_readlane(c, l) + DEC_TILE - 1) / DEC_TILE;
+      r.split_tokens = DEC_TILE * max(1, (tiles + r.last) / (r.last + 1));
     }
     pair -= __builtin_amdgcn_readlane(upto, 63);
     return past != 0;

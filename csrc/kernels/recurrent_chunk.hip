@@ -729,8 +729,10 @@ int launch_by_width(const ChunkArgs& a, int num_seqs, hipStream_t st) {
 // Segments of a portion of at most max_seqlen tokens (T in all): a CU takes one workgroup, so few heads
 // and sequences, or ragged ones, leave most of the chip idle for as long as the longest portion takes.
 // Cut, every segment but the last runs twice, the first time (states only, several workgroups a CU) at
-// some 0.4 of a block's time. In block times, with 3 to fill and drain a workgroup and the fold.
-static int pick_segments(int H, int dv, int num_seqs, int max_seqlen, int T) {
+// some 0.4 of a block's time. In block times, with 3 to fill and drain a workgroup and the fold. The
+// segments' states take at most 256 MB of scratch.
+static size_t unit_floats(int d, int dv) { return (size_t)d * dv + 2 * UNIT; }
+static int pick_segments(int H, int d, int dv, int num_seqs, int max_seqlen, int T) {
   const long wg = (long)H * ((dv + COLS - 1) / COLS);
   const auto rounds = [&](long units) { return (units * wg + 255) / 256; };
   float best = 0.9f * rounds(num_seqs) * (max_seqlen / 16 + 3.f);
@@ -739,6 +741,7 @@ static int pick_segments(int H, int dv, int num_seqs, int max_seqlen, int T) {
     const int len = ((max_seqlen + n - 1) / n + TB - 1) / TB * TB;
     if (len < 128) break;
     const int k = (max_seqlen + len - 1) / len;
+    if ((size_t)num_seqs * k * H * unit_floats(d, dv) > (64u << 20)) break;
     const long all = (long)num_seqs * k, most = T / len + num_seqs, units = all < most ? all : most;
     const float cost = rounds(units) * (len / 16 + 3.f) * 1.4f + 0.4f * k;
     if (cost < best) { best = cost; pick = k; }
@@ -751,13 +754,11 @@ static int segment_tokens(int max_seqlen, int nseg) {
 
 }  // namespace
 
-static size_t unit_floats(int d, int dv) { return (size_t)d * dv + 2 * UNIT; }
-
 // scratch that dli_recurrence_chunks takes for a step of T tokens (nullptr there: portions stay whole,
 // which MLSTM does not take)
 extern "C" long dli_recurrence_workspace_bytes(int mode, int num_seqs, int max_seqlen, int T, int H,
                                                int d, int dv) {
-  const int n = pick_segments(H, dv, num_seqs, max_seqlen, T);
+  const int n = pick_segments(H, d, dv, num_seqs, max_seqlen, T);
   const size_t gates = mode == MLSTM ? (size_t)T * H * 4 : 0;
   return (long)((gates + (n > 1 ? (size_t)num_seqs * n * H * unit_floats(d, dv) : 0)) * 4);
 }
@@ -779,7 +780,7 @@ extern "C" int dli_recurrence_chunks(int mode, const float* proj, int ldp, const
   ChunkArgs a{proj, ldp, z, ldz, bias, lower, inv_tau, qscale, decays, if_b, cap, norm_w, eps, state,
               nstate, slots, cu, positions, out, ldo, out_scale, H, d, dv, nullptr, 1 << 30, 1,
               nullptr, nullptr, nullptr};
-  const int nseg = ws != nullptr ? pick_segments(H, dv, num_seqs, max_seqlen, T) : 1;
+  const int nseg = ws != nullptr ? pick_segments(H, d, dv, num_seqs, max_seqlen, T) : 1;
   float* scratch = (float*)ws;
   float* gates = scratch;
   if (mode == MLSTM) {

@@ -304,6 +304,50 @@ __global__ void __launch_bounds__(256) rmsnorm_cols_block_kernel(
   }
 }
 
+// The same for rows of at most 4096 columns in whole 16-byte pieces: a thread's pieces of the row, the
+// weight and the gate are all requested at once and stay in registers, so the row costs one round trip to
+// memory instead of one for each column of a thread, twice. 64 gated rows of 4096: 18.8 -> 6.3 us.
+template <typename S>
+__global__ void __launch_bounds__(256) rmsnorm_cols_block4_kernel(
+    S* __restrict__ out, const float* __restrict__ src, int lds, const S* __restrict__ w, int n,
+    float eps, const float* __restrict__ gate, int ldg, int groups, int ldo, float out_scale,
+    bool silu) {
+  constexpr int U = 4;
+  __shared__ float red[16];
+  const int t = blockIdx.x / groups, go = (blockIdx.x % groups) * n, c0 = threadIdx.x * 4;
+  const float* r = src + (long)t * lds + go;
+  const f32x4 one = {1.f, 1.f, 1.f, 1.f};
+  f32x4 v[U], wt[U], g[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int c = c0 + u * 1024;
+    v[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    wt[u] = g[u] = one;
+    if (c < n) {
+      v[u] = *reinterpret_cast<const f32x4*>(r + c);
+      if (w != nullptr) wt[u] = ld4(w + go + c);
+      if (gate != nullptr) g[u] = *reinterpret_cast<const f32x4*>(gate + (long)t * ldg + go + c);
+    }
+  }
+  float s = 0.f;
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    s += (v[u][0] * v[u][0] + v[u][1] * v[u][1]) + (v[u][2] * v[u][2] + v[u][3] * v[u][3]);
+  s = block_sum(s, red);
+  const float rs = 1.f / sqrtf(s / (float)n + eps);
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int c = c0 + u * 1024;
+    if (c >= n) continue;
+    f32x4 y = v[u] * rs * wt[u];
+    if (gate != nullptr) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) y[i] *= gate_of(g[u][i], silu);
+    }
+    st4(out + (long)t * ldo + go + c, y * out_scale);
+  }
+}
+
 // The rotation of element c of a rotated part `v` (length >= rot_dims): with `half` dimension
 // i < rot_dims/2 pairs with i + rot_dims/2, else pairs are (2i, 2i+1). The pair (u, v) at angle
 // a becomes (u cos a - v sin a, v cos a + u sin a); the angle position * frequency is formed in
@@ -541,7 +585,19 @@ extern "C" int dli_rmsnorm_cols(void* out, const float* src, int lds, const void
                                 float out_scale, int silu, int dt, hipStream_t st) {
   if (T <= 0) return 0;
   if (n < 1 || groups < 1) return (int)hipErrorInvalidValue;
+  const bool vec4 = n % 4 == 0 && lds % 4 == 0 && ldg % 4 == 0 && ldo % 4 == 0 &&
+                    (((uintptr_t)out | (uintptr_t)src | (uintptr_t)w | (uintptr_t)gate) & 15) == 0;
   if ((long)T * groups <= 512 && n >= 1024) {
+    if (vec4 && n <= 4096) {
+      DT_SWITCH(dt,
+                (rmsnorm_cols_block4_kernel<u16><<<T * groups, 256, 0, st>>>(
+                    (u16*)out, src, lds, (const u16*)w, n, eps, gate, ldg, groups, ldo, out_scale,
+                    silu != 0)),
+                (rmsnorm_cols_block4_kernel<float><<<T * groups, 256, 0, st>>>(
+                    (float*)out, src, lds, (const float*)w, n, eps, gate, ldg, groups, ldo,
+                    out_scale, silu != 0)));
+      DLI_RETURN_LAUNCH();
+    }
     DT_SWITCH(dt,
               (rmsnorm_cols_block_kernel<u16><<<T * groups, 256, 0, st>>>(
                   (u16*)out, src, lds, (const u16*)w, n, eps, gate, ldg, groups, ldo, out_scale,
@@ -552,8 +608,6 @@ extern "C" int dli_rmsnorm_cols(void* out, const float* src, int lds, const void
     DLI_RETURN_LAUNCH();
   }
   const int nb = (int)(((long)T * groups + 3) / 4);
-  const bool vec4 = n % 4 == 0 && lds % 4 == 0 && ldg % 4 == 0 && ldo % 4 == 0 &&
-                    (((uintptr_t)out | (uintptr_t)src | (uintptr_t)w | (uintptr_t)gate) & 15) == 0;
   if (vec4 && n <= 128) {
     const int lpr = n <= 32 ? 8 : n <= 64 ? 16 : 32;
     const int nh = (int)(((long)T * groups + 256 / lpr - 1) / (256 / lpr));

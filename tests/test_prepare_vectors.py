@@ -88,3 +88,21 @@ def test_sink_prepare(heads, G, d, dv, rot, pad, dtype):
                          pos.cuda(), kd, vd, slots.cuda())
     for a, b in ((got, want), (kd, kc), (vd, vc)):
         close(a.reshape(-1), b.reshape(-1), dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n,groups,gated,pad", [(4096, 1, True, 4), (1024, 3, True, 0), (2052, 1, False, 0), (4100, 1, True, 0),
+                                                (1030, 2, True, 0), (3000, 1, True, 3)])
+def test_rmsnorm_of_few_wide_rows(n, groups, gated, pad, dtype):
+    T, W = 5, n * groups
+    src, gate = torch.randn(T, W + pad)[:, :W], torch.randn(T, W + pad)[:, :W]
+    w = torch.randn(W).to(dtype)
+    want = torch.cat([R.rmsnorm_cols(src[:, i * n:(i + 1) * n], w[i * n:(i + 1) * n], 1e-6, torch.float32,
+                                     gate[:, i * n:(i + 1) * n] if gated else None) for i in range(groups)], 1) * 0.5
+
+    def wide(x):                                 # rows of a wider buffer there too
+        b = torch.zeros(T, W + pad, device="cuda")
+        b[:, :W] = x.cuda()
+        return b[:, :W]
+    got = H.rmsnorm_cols(wide(src), w.cuda(), 1e-6, gate=wide(gate) if gated else None, groups=groups, out_scale=0.5)
+    close(got, want, dtype)

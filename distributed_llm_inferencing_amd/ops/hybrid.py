@@ -1,11 +1,12 @@
 """Ops of the hybrid model family (models/hybrid.py): fp32 residual stream and norms, grouped
 RMS norm, windowed attention with distance bias / head mixing / output gate over token-major
-paged caches, latent (compressed-kv) attention in the absorbed form, a gated linear recurrence
-with per-sequence state slots, and a shape-agnostic GEMM.
+paged caches, latent (compressed-kv) attention in the absorbed and the expanded form, linear
+recurrences with per-sequence state slots, and a shape-agnostic GEMM.
 
 Dispatch is the package's: CUDA (HIP) tensors run the gfx950 kernels (``csrc/kernels``:
-hybrid_elementwise.hip, window_attention.hip, recurrent.hip, gemm_any.hip), CPU tensors the
-PyTorch reference (``ops/reference.py``). The storage dtype (bf16 when serving, fp32 in the
+hybrid_elementwise.hip, gemm_any.hip; attention: swa_attention.hip, mix_attention.hip,
+window_attention_mfma.hip, window_attention.hip; recurrences: recurrent_chunk.hip, recurrent.hip,
+recurrent_scalar.hip), CPU tensors the PyTorch reference (``ops/reference.py``). The storage dtype (bf16 when serving, fp32 in the
 exact mode) is the dtype of the weights; kernels take it as ``dt``.
 """
 from __future__ import annotations

@@ -942,10 +942,14 @@ extern "C" int dli_decode_attention(void* out, const void* q, int q_stride, cons
   float* ws_ml = ws_o ? ws_o + (long)B * hq * num_splits * hd : nullptr;
   const float scale_log2 = scale * 1.4426950408889634f;
   const long items = (long)B * hkv * num_splits;
-  // 2 = automatic: the pipelined kernel for splits of >= 768 tokens (measured: +18 % at ctx
-  // 1000, B 64; within 3 % slower at ctx 33-100, B 512, where the per-item dependent loads
-  // (context length -> block table -> K/V) rather than tile rounds bound the time)
-  const bool use_pipe = g_decode_pipe == 1 || (g_decode_pipe == 2 && split_tokens >= 768);
+  // 2 = automatic: the pipelined kernel where a sequence is one item of up to 768 tokens or more
+  // (max_context is a bound, in a captured step the table's width): +18 % at 1000 tokens, 64 rows;
+  // within 3 % slower at 33 - 100, 512 rows, where the per-item dependent loads (context length ->
+  // block table -> K/V) rather than tile rounds bound the time. Split sequences are dealt whatever
+  // the bound: 128 rows of 100 - 1000 tokens on an 8192-token table 54 us, pipelined over the same 8
+  // static slots 231, over two 93; 24 of 500 - 8000 on 32768 64 us, 98, 304; 128 of 8000 731, 780, 755.
+  const bool use_pipe = g_decode_pipe == 1 ||
+                        (g_decode_pipe == 2 && num_splits == 1 && split_tokens >= 768);
   if (hd == 128 && use_pipe) {
     // 8 waves per CU x 256 CUs; each wave walks items gw, gw + nw, ...
     const long wgs = (items + DEC_WAVES - 1) / DEC_WAVES;

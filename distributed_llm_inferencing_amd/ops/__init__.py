@@ -506,7 +506,7 @@ def prefill_attention(qkv, cu_seqlens, max_seqlen: int, hq, hkv, hd, scale, out=
 
 def decode_pipelined(v: int) -> int:
     """Select the pipelined (1), one-tile-per-round (0) or automatic (2, the default: pipelined
-    for KV splits of >= 768 tokens) decode attention kernel for head_dim 128. Returns the
+    for unsplit contexts of up to 768 tokens or more) decode attention kernel for head_dim 128. Returns the
     previous setting (tests force either kernel with it)."""
     return int(N.require_native().dli_decode_set_pipe(int(v)))
 
@@ -570,7 +570,8 @@ def decode_num_splits(B: int, hkv: int, max_context: int) -> int:
     if splits == 1:
         return 1
     # slots a sequence may use, of at least 64 tokens: the kernel deals the step's actual contexts
-    # to 2048 - 4096 waves, so one long context among short ones takes many slots
+    # to at most max(even splits, 3072 + B * hkv) waves, fewer where contexts or slots run out, so
+    # one long context among short ones takes many slots
     return max(splits, min(64, max_context // 64, 8192 // items))
 
 

@@ -67,3 +67,26 @@ def test_contexts_dealt_to_splits(name, hq, hkv, splits):
         # probabilities are rounded to bf16 (2^-9 relative) before the value sum, whose terms are at
         # most |v| < 6 with weights summing to 1, and the result is rounded to bf16
         assert (got - want).abs().max() <= 6 * 2 ** -9 + 2 ** -8 * want.abs().max()
+
+
+@pytest.mark.parametrize("B,bound", [(24, 32768), (64, 16384), (8, 65536)])
+def test_a_wide_table_does_not_change_the_split(B, bound):
+    """The bound is a table's width: contexts of 100 tokens take two slots at most, whatever it is,
+    and nothing is written for the others."""
+    hq, hkv = 32, 8
+    splits = ops.decode_num_splits(B, hkv, bound)
+    assert splits > 4 and bound // splits >= 768
+    kc, vc = (torch.randn(B * 7, hkv, BS, HD, device="cuda").bfloat16() for _ in range(2))
+    tables = torch.zeros(B, bound // BS, dtype=torch.int32, device="cuda")
+    tables[:, :7] = torch.arange(B * 7, device="cuda").view(B, 7)
+    qkv = torch.randn(B, (hq + 2 * hkv) * HD, device="cuda").bfloat16()
+    ctx = torch.full((B,), 100, dtype=torch.int32, device="cuda")
+    used = B * hq * splits * (HD + 2) * 4
+    ws = ops.G.workspace(qkv.device, used)
+    ws.fill_(0xff)
+    got = ops.decode_attention(qkv, kc, vc, tables, ctx, bound, hq, hkv, HD, HD ** -0.5)
+    partials = ws[:B * hq * splits * HD * 4].view(torch.int32).view(B * hq, splits, HD)
+    assert (partials[:, 2:] == -1).all()
+    want = reference(qkv[:, :hq * HD].view(B, hq, HD).float(), kc.float(), vc.float(), tables[:, :7],
+                     [100] * B, HD ** -0.5)
+    assert (got.view(B, hq, HD).float() - want).abs().max() <= 6 * 2 ** -9 + 2 ** -8 * want.abs().max()

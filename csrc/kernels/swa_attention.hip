@@ -54,7 +54,7 @@ struct SwaArgs {
   float* ws;                           // decode, nsplit > 1: [nsplit][S][H][2], [nsplit][S][H][HD]
   // shared tail of queries and keys (prefill32 with DR > 0): head h of token t has its DR dims at q2 +
   // t * ldq2 + h * q2_head, a key row has them once for all heads; the key and value rows of sequence
-  // s are then rows cu_ctx[s] + position of plain matrices
+  // s are then rows [cu_ctx[s], cu_ctx[s + 1]) of plain matrices, its last positions in order
   const u16* q2; long ldq2; int q2_head;
   const u16* k2; long k2_stride;
   const int* cu_ctx;
@@ -146,7 +146,7 @@ __global__ void __launch_bounds__(512) swa_prefill32_kernel(SwaArgs a) {
   const KeyList kl(p0 + wg_q0, p0 + min(wg_q0 + LROWS, len) - 1, a.window, a.keep);
   const int ntiles = (kl.n + KT - 1) / KT;
   const int* bt = DR ? nullptr : a.block_tables + (long)s * a.bt_stride;
-  const int base = DR ? a.cu_ctx[s] : 0;
+  const int base = DR ? a.cu_ctx[s + 1] - (p0 + len) : 0;
   const auto row_of = [&](int x) {
     const int j = kl.key(x);
     return DR ? base + j : bt[j / a.block_size] * a.block_size + j % a.block_size;
@@ -733,39 +733,45 @@ int launch_swa(SwaArgs a, int num_seqs, int max_seqlen, hipStream_t st) {
 }
 
 
-// Rows cu_ctx[s] + j of out <- the cache row of position j of sequence s, `chunks` 16-byte pieces each
+// Rows [cu_ctx[s], cu_ctx[s + 1]) of out <- the cache rows of the last positions of sequence s, whose
+// new tokens are rows [cu[s], cu[s + 1]), `chunks` 16-byte pieces each
 __global__ void __launch_bounds__(256) gather_rows_kernel(uint4* out, const uint4* cache,
-                                                          const int* cu_ctx, const int* block_tables,
+                                                          const int* cu_ctx, const int* cu,
+                                                          const int* positions, const int* block_tables,
                                                           int bt_stride, int block_size, int chunks) {
   const int s = blockIdx.y, o0 = cu_ctx[s], n = cu_ctx[s + 1] - o0;
   const int* bt = block_tables + (long)s * bt_stride;
   const int j0 = blockIdx.x * 64, rows = min(64, n - j0);
+  if (rows <= 0 || cu[s + 1] <= cu[s]) return;
+  const int first = positions[cu[s + 1] - 1] + 1 - n;
   for (int i = threadIdx.x; i < rows * chunks; i += 256) {
-    const int j = j0 + i / chunks, c = i % chunks;
-    const long row = (long)bt[j / block_size] * block_size + j % block_size;
+    const int j = j0 + i / chunks, c = i % chunks, p = first + j;
+    const long row = (long)bt[p / block_size] * block_size + p % block_size;
     out[(long)(o0 + j) * chunks + c] = cache[row * chunks + c];
   }
 }
 
 }  // namespace
 
-// The cached rows (width bf16 elements, a multiple of 8) of every sequence's context, in order
+// The cached rows (width bf16 elements, a multiple of 8) of every sequence's last cu_ctx[s + 1] -
+// cu_ctx[s] <= max_rows positions, in order
 extern "C" int dli_gather_context(void* out, const void* cache, int width, const int* cu_ctx,
-                                  const int* block_tables, int bt_stride, int block_size, int num_seqs,
-                                  int max_context, hipStream_t st) {
-  if (num_seqs <= 0 || max_context <= 0) return 0;
+                                  const int* cu, const int* positions, const int* block_tables,
+                                  int bt_stride, int block_size, int num_seqs, int max_rows,
+                                  hipStream_t st) {
+  if (num_seqs <= 0 || max_rows <= 0) return 0;
   if (width < 8 || width % 8 || block_size < 1 || num_seqs > 65535 ||
       (((uintptr_t)out | (uintptr_t)cache) & 15))
     return (int)hipErrorInvalidValue;
-  dim3 grid((max_context + 63) / 64, num_seqs);
-  gather_rows_kernel<<<grid, 256, 0, st>>>((uint4*)out, (const uint4*)cache, cu_ctx, block_tables,
-                                           bt_stride, block_size, width / 8);
+  dim3 grid((max_rows + 63) / 64, num_seqs);
+  gather_rows_kernel<<<grid, 256, 0, st>>>((uint4*)out, (const uint4*)cache, cu_ctx, cu, positions,
+                                           block_tables, bt_stride, block_size, width / 8);
   DLI_RETURN_LAUNCH();
 }
 
 // Portions whose keys share their last dr dims (latent attention, expanded): q [T, H*dk] and its tail
-// q2 (row stride ldq2, head stride q2_head); k and v are rows cu_ctx[s] + position of matrices with one
-// column block a head, k2 [.., dr] of a third. hipErrorNotSupported (801): widths or alignment that this
+// q2 (row stride ldq2, head stride q2_head); k and v are rows [cu_ctx[s], cu_ctx[s + 1]), a sequence's
+// last positions (every one that a query sees), of matrices with one column block a head, k2 [.., dr] of a third. hipErrorNotSupported (801): widths or alignment that this
 // form does not take.
 extern "C" int dli_shared_tail_attention(const void* q, int ldq, const void* q2, long ldq2, int q2_head,
                                          const void* k, long k_stride, const void* k2, long k2_stride,

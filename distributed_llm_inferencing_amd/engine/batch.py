@@ -202,11 +202,9 @@ class DeviceBatch:
     max_seqlen_prefill: int = 0
     state_slots: Optional[torch.Tensor] = None
     logit_rows: Optional[torch.Tensor] = None
-    # steps that attend over the paged cache: cumulative context lengths [S + 1], their sum, and the
-    # pairs of a new token (a sequence's rounded up to 16) and a position before it
-    cu_context: Optional[torch.Tensor] = None
-    total_context: int = 0
-    context_pairs: int = 0
+    # a prefill step over the paged cache: new tokens and context lengths of its sequences, on the host
+    host_lens: Optional[np.ndarray] = None
+    host_context: Optional[np.ndarray] = None
 
     @property
     def is_prefill(self) -> bool:
@@ -256,11 +254,6 @@ def to_device(meta: StepMeta, device, pin: bool = True) -> DeviceBatch:
         paged = meta.block_tables is not None and np.shape(meta.block_tables)[1] > 0
         if nd:
             add("cu_seqlens_prefill", cu[nd:] - nd, torch.int32)
-    if paged:
-        ctx = np.asarray(meta.context_lens, dtype=np.int64)
-        cuc = np.zeros(S + 1, dtype=np.int32)
-        cuc[1:] = np.cumsum(ctx)
-        add("cu_context", cuc, torch.int32)
     if meta.kind != PREFILL or paged:
         add("block_tables", meta.block_tables, torch.int32)
         add("context_lens", meta.context_lens, torch.int32)
@@ -296,9 +289,7 @@ def to_device(meta: StepMeta, device, pin: bool = True) -> DeviceBatch:
             db.block_tables = v["block_tables"]
             db.context_lens = v["context_lens"]
             db.max_context = int(np.max(meta.context_lens)) if S else 0
-            db.cu_context = v["cu_context"]
-            db.total_context = int(ctx.sum())
-            db.context_pairs = int(((lens + 15) // 16 * 16 * ctx - lens * (lens - 1) // 2).sum())
+            db.host_lens, db.host_context = lens.copy(), np.array(meta.context_lens, dtype=np.int64)
         if nd:
             ctx = np.asarray(meta.context_lens)
             db.num_decode = nd

@@ -123,7 +123,7 @@ class HybridLM(TransformerLM):
                              "no block tables")
         return StepView(cu, mx, b.positions, b.slot_mapping, b.block_tables, block_size,
                         b.state_slots, b.max_context if b.max_context > 0 else 1 << 30,
-                        b.cu_context, b.total_context, b.context_pairs)
+                        b.host_lens, b.host_context)
 
     def _all_rows(self, n: int) -> torch.Tensor:
         r = self._rows.get(n)

@@ -15,6 +15,7 @@ from __future__ import annotations
 from dataclasses import dataclass, field
 from typing import Optional
 
+import numpy as np
 import torch
 
 from ..ops import hybrid as H
@@ -34,12 +35,10 @@ class StepView:
     block_size: int
     state_slots: Optional[torch.Tensor]   # [S] int32 recurrent-state slot (-1: padding row)
     max_context: int = 1 << 30      # no position of this step is at or beyond this
-    # of a prefill step (``DeviceBatch``): cumulative context lengths [S+1] int32, their sum, and the
-    # pairs of a new token and a position before it; unknown without the first
-    cu_context: Optional[torch.Tensor] = None
-    total_context: int = 0
-    context_pairs: int = 0
-    tables: dict = field(default_factory=dict)      # rotation tables made so far in this step
+    # of a prefill step: the sequences' new tokens and context lengths (int64 [S], on the host)
+    host_lens: Optional[np.ndarray] = None
+    host_context: Optional[np.ndarray] = None
+    tables: dict = field(default_factory=dict)      # rotation tables and the like made so far in this step
 
     def rotation(self, spec: LayerSpec, lp: dict):
         """fp32 [T, rot_dims] = cosines | sines of the step's positions, made once per step for
@@ -51,6 +50,23 @@ class StepView:
         if t is None:
             t = self.tables[key] = H.rotation_table(self.positions, lp["rot_freq"])
         return t
+
+    def visible(self, window: int):
+        """(rows [S], pairs) of ``H.visible_context``, once per step for all layers of a window."""
+        key = ("visible", window)
+        if key not in self.tables:
+            self.tables[key] = H.visible_context(self.host_lens, self.host_context, window)
+        return self.tables[key]
+
+    def cu_visible(self, window: int) -> torch.Tensor:
+        """The visible rows' cumulative counts [S+1] int32 on the step's device."""
+        key = ("cu_visible", window)
+        if key not in self.tables:
+            rows = self.visible(window)[0]
+            cu = torch.zeros(len(rows) + 1, dtype=torch.int32, pin_memory=self.positions.is_cuda)
+            np.cumsum(rows, dtype=np.int32, out=cu.numpy()[1:])
+            self.tables[key] = cu.to(self.positions.device, non_blocking=True)
+        return self.tables[key]
 
 
 def derive_constants(spec: LayerSpec, lp: dict, device) -> None:
@@ -161,8 +177,8 @@ def latent_attention_mixer(spec: LayerSpec, lp: dict, h, step: StepView, cache, 
         q_h . k_h = (W_uk,h^T q_h) . c      and      sum_j w_j v_h,j = W_uv,h (sum_j w_j c_j),
     so every head attends the same cached row [c | k_rot] with the query [W_uk,h^T q_h | q_rot]
     and its output is expanded afterwards: one multi-query attention over the latent. Steps with
-    enough new tokens for their context (``H.latent_expansion_pays``) expand k_h and v_h of the whole
-    context instead: the pairs of a query and a key cost 3.4 times less then."""
+    enough new tokens for the context they see (``H.latent_expansion_pays``) expand its k_h and v_h
+    instead: the pairs of a query and a key cost 3.4 times less then."""
     Hh, d, dr, dv, r = spec.heads, spec.dim, spec.rot_dim, spec.vdim, spec.kv_rank
     (c,) = cache
     T = h.shape[0]
@@ -188,13 +204,15 @@ def latent_attention_mixer(spec: LayerSpec, lp: dict, h, step: StepView, cache, 
     # a window no shorter than the step's longest context masks nothing: the tight bound lets
     # the kernel size its slot table and key splits for the keys that exist
     win = min(spec.window, max(1, step.max_context))
-    if ("w_ukv" in lp and step.cu_context is not None and H.latent_expansion_pays(
-            T, step.max_seqlen, step.total_context, step.context_pairs, Hh * (d + dv))):
-        o = H.expanded_latent_attention(q_nope, q_full[:, :, r:], c, lp["w_ukv"][0], Hh, r,
-                                        step.cu_seqlens, step.max_seqlen, step.positions,
-                                        step.block_tables, step.block_size, step.cu_context,
-                                        step.total_context, step.max_context, win, spec.scale, gates)
-        return H.linear_any(o, lp["wo"])
+    if "w_ukv" in lp and step.host_context is not None:
+        rows, pairs = step.visible(win)
+        total = int(rows.sum())
+        if H.latent_expansion_pays(T, step.max_seqlen, total, pairs, Hh * (d + dv)):
+            o = H.expanded_latent_attention(q_nope, q_full[:, :, r:], c, lp["w_ukv"][0], Hh, r,
+                                            step.cu_seqlens, step.max_seqlen, step.positions,
+                                            step.block_tables, step.block_size, step.cu_visible(win),
+                                            total, int(rows.max()), win, spec.scale, gates)
+            return H.linear_any(o, lp["wo"])
     H.head_linear(q_nope, lp["w_ukT"], q_full)               # q_full[:, h, :r] = W_uk,h^T q_h
     ol = H.window_attention(q_full.view(T, Hh * (r + dr)), c, c, r + dr, r, Hh, 1,
                             step.cu_seqlens, step.max_seqlen, step.positions,

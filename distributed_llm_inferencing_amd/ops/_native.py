@@ -117,7 +117,7 @@ _SIGS = {
     "dli_swa_attention": [P, I, P, L, P, L, P, I, P, P, P, I, I, I, I, I, I, I, I, I, I, F, P, I, I,
                           P, F, P, P],
     "dli_swa_attention_workspace_bytes": [I, I, I, I, I, I, I],
-    "dli_gather_context": [P, P, I, P, P, I, I, I, I, P],
+    "dli_gather_context": [P, P, I, P, P, P, P, I, I, I, I, P],
     "dli_shared_tail_attention": [P, I, P, L, I, P, L, P, L, P, L, P, I, P, P, P, I, I, I, I, I, I, I, F,
                                   P, I, P],
     "dli_sandwich_add": [P, P, I, I, L, P, I, P, P, F, P, I, I, P, P, P, I, I, F, F, I, P],

@@ -15,6 +15,7 @@ import os
 from dataclasses import dataclass
 from typing import Optional
 
+import numpy as np
 import torch
 
 from . import _native as N
@@ -426,35 +427,57 @@ def expanded_latent_ok(dtype, d: int, dr: int, dv: int, r: int) -> bool:
     return dtype == torch.bfloat16 and (d, dr, dv) == (128, 64, 128) and r % 64 == 0
 
 
-def latent_expansion_pays(tokens: int, max_seqlen: int, context: int, pairs: int, width: int) -> bool:
-    """Whether a step expands the context's keys and values (``width`` columns of them) instead of
-    attending the latent itself: ``context`` rows to expand, some 14 ns each at width 8192, against
-    0.44 ns for each of ``pairs`` (a key and a row of the absorbed kernel, which takes a sequence's
-    rows 16 at a time) and 75 ns a token for absorbing its query and expanding its output. A layer of
-    32 heads, absorbed -> expanded: 4 x 2048 tokens 5.6 -> 1.2 ms, 32 x 64 0.48 -> 0.31, 512 tokens
-    at 4096 1.04 -> 0.37, 512 beside 64 single ones at 1000 10.3 -> 1.6; 64 at 4096 0.23 -> 0.26."""
-    if max_seqlen < 64 or (max_seqlen < 96 and context > 8 * tokens) or context * width > 1 << 30:
+def visible_context(lens, context, window: int):
+    """Of a step whose sequences bring ``lens`` new tokens, contexts of ``context`` positions with
+    them (int64 arrays): the last positions of each that any of its queries sees, and the pairs of a
+    row and a key that the absorbed kernel's time goes with. Its workgroups take 16 rows, and the
+    step has ceil(longest / 16) for every sequence, dealt to the 8 XCDs in turn. Where that is too many
+    to split the keys too, the busiest XCD counts: 64 single tokens beside a portion of 512 (32 to
+    a sequence) are all on the same one, 10.1 ms at 1000 keys each where the pairs alone make 0.7."""
+    rows = np.where(lens > 0, np.minimum(context, lens + (window - 1)), 0)
+    n = -(-lens // 16)
+    seq = np.repeat(np.arange(len(lens)), n)
+    tile = np.arange(len(seq)) - np.repeat(np.cumsum(n) - n, n)
+    end = np.minimum(16 * tile + 16, lens[seq])
+    keys = np.minimum(context[seq] - lens[seq] + end, end - 16 * tile + window - 1)
+    slots = int(n.max(initial=0))
+    if slots * len(lens) <= 128:
+        return rows, 16 * int(keys.sum())
+    return rows, 128 * int(np.bincount((seq * slots + tile) % 8, keys, 8).max())
+
+
+def latent_expansion_pays(tokens: int, max_seqlen: int, rows: int, pairs: int, width: int) -> bool:
+    """Whether a step expands its visible context's keys and values (``width`` columns of them) instead
+    of attending the latent itself: ``rows`` to expand, some 14 ns each at width 8192, against
+    0.44 ns for each of ``pairs`` (``visible_context``) and 75 ns a token for absorbing its query and
+    expanding its output. A layer of 32 heads, absorbed -> expanded: 4 x 2048 tokens 5.6 -> 1.2 ms, 32 x 64
+    0.48 -> 0.31, 512 tokens at 4096 1.04 -> 0.37, 512 beside 64 single ones at 1000 10.3 -> 1.6; 64 at
+    4096 0.23 -> 0.26."""
+    if max_seqlen < 64 or (max_seqlen < 96 and rows > 8 * tokens) or rows * width > 1 << 30:
         return False
-    return 14 * context < 75 * tokens + 0.44 * pairs
+    return 14 * rows < 75 * tokens + 0.44 * pairs
 
 
 def expanded_latent_attention(q, q_rot, cache, w_ukv, H, r, cu_seqlens, max_seqlen, positions,
-                              block_tables, block_size, cu_context, context, max_context, window,
+                              block_tables, block_size, cu_rows, rows, max_rows, window,
                               scale, gates=None) -> torch.Tensor:
     """Latent attention over portions with keys and values expanded from the cached rows [latent r |
     shared rotated key]: q [T, H, d] and its rotated tails q_rot [T, H, dr] (rows of a wider buffer),
-    w_ukv [H (d + dv), r]; sigmoid(gates [T, H]) multiplies the heads. -> [T, H*dv] in q's dtype."""
+    w_ukv [H (d + dv), r]; sigmoid(gates [T, H]) multiplies the heads. ``cu_rows`` [S+1] int32: the
+    last positions of each sequence that are expanded, cumulative; ``rows`` in all, ``max_rows`` at
+    most; those before are in no query's window. -> [T, H*dv] in q's dtype."""
     T, _, d = q.shape
     dr, dv = q_rot.shape[2], w_ukv.shape[0] // H - d
-    rows = torch.empty(context, r + dr, dtype=q.dtype, device=q.device)
-    _call("dli_gather_context", _p(rows), _p(cache), r + dr, _p(cu_context), _p(block_tables),
-          block_tables.stride(0), block_size, cu_seqlens.shape[0] - 1, int(max_context), _st())
-    kv = linear_any(rows[:, :r], w_ukv, out_f32=False)
+    ctx = torch.empty(rows, r + dr, dtype=q.dtype, device=q.device)
+    _call("dli_gather_context", _p(ctx), _p(cache), r + dr, _p(cu_rows), _p(cu_seqlens),
+          _p(positions), _p(block_tables), block_tables.stride(0), block_size,
+          cu_seqlens.shape[0] - 1, int(max_rows), _st())
+    kv = linear_any(ctx[:, :r], w_ukv, out_f32=False)
     out = torch.empty(T, H * dv, dtype=q.dtype, device=q.device)
-    k_rot, v = rows[:, r:], kv[:, H * d:]
+    k_rot, v = ctx[:, r:], kv[:, H * d:]
     _call("dli_shared_tail_attention", _p(q), q.stride(0), _p(q_rot), q_rot.stride(0),
           q_rot.stride(1), _p(kv), kv.stride(0), _p(k_rot), k_rot.stride(0), _p(v), kv.stride(0),
-          _p(out), out.stride(0), _p(cu_seqlens), _p(positions), _p(cu_context),
+          _p(out), out.stride(0), _p(cu_seqlens), _p(positions), _p(cu_rows),
           cu_seqlens.shape[0] - 1, int(max_seqlen), H, d, dr, dv, int(window), float(scale),
           _p(gates), gates.stride(0) if gates is not None else 0, _st())
     return out

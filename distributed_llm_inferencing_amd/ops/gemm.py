@@ -138,14 +138,18 @@ _retired: list = []
 
 
 def workspace(device: torch.device, nbytes: int) -> torch.Tensor:
-    """Grow-only scratch (bytes) per device. Never freed: see ``_retired``."""
+    """Grow-only scratch (bytes) per device. Never freed: see ``_retired``. It at least doubles, so
+    that all outgrown buffers together are smaller than the one in use: the sizes asked for follow
+    the steps' lengths, and by exact sizes rising steps of recurrences (2.1 MB a segment and
+    sequence, up to 256 MB) would leave 15 GB behind."""
     key = (device.type, device.index)
     with _ws_lock:
         ws = _workspaces.get(key)
         if ws is None or ws.numel() < nbytes:
             if ws is not None:
                 _retired.append(ws)
-            ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
+            grown = max(nbytes, 1 << 20, 2 * ws.numel() if ws is not None else 0)
+            ws = torch.empty(grown, dtype=torch.uint8, device=device)
             _workspaces[key] = ws
         return ws
 

@@ -389,6 +389,21 @@ def test_gemm_workspace_growth_keeps_the_replaced_buffer_alive():
             G._workspaces.pop(key, None)
 
 
+def test_gemm_workspace_of_rising_sizes_stays_bounded(monkeypatch):
+    """Every step may ask for a little more than the last one: what is retained in all stays within a
+    small multiple of the largest request."""
+    from distributed_llm_inferencing_amd.ops import gemm as G
+    monkeypatch.setattr(G, "_workspaces", {})
+    monkeypatch.setattr(G, "_retired", [])
+    dev, most = torch.device("cpu"), 0
+    for i in range(1, 200):
+        most = (1 << 20) + i * 70001
+        assert G.workspace(dev, most).numel() >= most
+        held = sum(t.numel() for t in G._retired)
+        live = G._workspaces[("cpu", None)].numel()
+        assert held <= live <= 2 * most
+
+
 def test_autotune_final_round_picks_the_lowest_median():
     """ops.gemm._final_round: finalists within the band are re-timed round-robin and the lowest
     median wins, so one lucky first-pass sample cannot pin a plan."""

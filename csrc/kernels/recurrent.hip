@@ -58,7 +58,8 @@ __global__ void __launch_bounds__(1024) hgrn2_kernel(const float* __restrict__ p
                              float* __restrict__ state, const int* __restrict__ slots,
                              const int* __restrict__ cu, const int* __restrict__ positions,
                              S* __restrict__ out, int ldo, int H, int d, int dv,
-                             const float* __restrict__ zp, int ldz, float inv_tau, float qscale) {
+                             const float* __restrict__ zp, int ldz, float inv_tau, float qscale,
+                             int max_len) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
   float* St = sm;                 // [d][dv] (D == 0 only)
   float* qv = St + (D ? 0 : d * dv);   // [TC][d] silu(qz) (GLA: q * qscale)
@@ -70,6 +71,7 @@ __global__ void __launch_bounds__(1024) hgrn2_kernel(const float* __restrict__ p
   const int h = blockIdx.x, s = blockIdx.y;
   const int slot = slots[s];
   const int t0 = cu[s], t1 = cu[s + 1];
+  if (t1 - t0 > max_len) return;
   const int dvp = blockDim.x / P;
   const int c = threadIdx.x % dvp, part = threadIdx.x / dvp;
   if (slot < 0) {                        // padding rows: defined (zero) output, no state
@@ -187,7 +189,7 @@ __global__ void __launch_bounds__(1024) hgrn2_kernel(const float* __restrict__ p
   for (int i = threadIdx.x; i < d * dv; i += blockDim.x) sp[i] = St[i];
 }
 
-// Decode steps (every sequence brings one token): the state streams through registers, one
+// Sequences that bring one token (others are skipped): the state streams through registers, one
 // read and one write per element, no LDS copy. One workgroup per (head, sequence), thread c
 // owns column c: consecutive threads touch consecutive addresses of every state row.
 template <typename S, bool GLA>
@@ -208,7 +210,7 @@ __global__ void hgrn2_step_kernel(const float* __restrict__ proj, int ldp,
   const int slot = slots[s];
   const int t = cu[s];
   const int c = threadIdx.x;
-  if (cu[s + 1] <= t) return;
+  if (cu[s + 1] != t + 1) return;
   if (slot < 0) {
     if (c < dv) stf(out + (long)t * ldo + h * dv + c, 0.f);
     return;
@@ -268,12 +270,12 @@ static int launch_recurrence(const float* proj, int ldp, const void* f_bias, con
                              const void* norm_w, float eps, float* state, const int* slots,
                              const int* cu, const int* positions, void* out, int ldo,
                              int num_seqs, int max_seqlen, int H, int d, int dv, int dt,
-                             const float* zp, int ldz, float inv_tau, float qscale,
+                             const float* zp, int ldz, float inv_tau, float qscale, int max_len,
                              hipStream_t st) {
   if (num_seqs <= 0) return 0;
   const int threads = ((dv + 63) / 64) * 64;
   if (H < 1 || d < 1 || dv < 1 || threads > 1024) return (int)hipErrorInvalidValue;
-  if (max_seqlen == 1) {                 // a decode step: stream the state, no LDS copy
+  if (max_seqlen == 1 || max_len == 1) { // single tokens: stream the state, no LDS copy
     dim3 grid1(H, num_seqs);
     const size_t sh1 = ((size_t)(GLA ? 3 : 2) * d + 16) * 4;
     if (sh1 > 48 * 1024) return (int)hipErrorInvalidValue;
@@ -306,7 +308,7 @@ static int launch_recurrence(const float* proj, int ldp, const void* f_bias, con
     }                                                                                          \
     hgrn2_kernel<ST, DD, PP, GLA><<<grid, nthreads, sh, st>>>(                                 \
         proj, ldp, (const ST*)f_bias, (const ST*)lower, (const ST*)norm_w, eps, state, slots,  \
-        cu, positions, (ST*)out, ldo, H, d, dv, zp, ldz, inv_tau, qscale);                     \
+        cu, positions, (ST*)out, ldo, H, d, dv, zp, ldz, inv_tau, qscale, max_len);            \
   } while (0)
 #define HGRN2_BY_D(ST)                                   \
   do {                                                   \
@@ -324,13 +326,14 @@ static int launch_recurrence(const float* proj, int ldp, const void* f_bias, con
   DLI_RETURN_LAUNCH();
 }
 
+// max_len: sequences that bring more tokens are left alone (recurrent_chunk.hip takes them)
 extern "C" int dli_hgrn2(const float* proj, int ldp, const void* f_bias, const void* lower,
                          const void* norm_w, float eps, float* state, const int* slots,
                          const int* cu, const int* positions, void* out, int ldo, int num_seqs,
-                         int max_seqlen, int H, int d, int dv, int dt, hipStream_t st) {
+                         int max_seqlen, int max_len, int H, int d, int dv, int dt, hipStream_t st) {
   return launch_recurrence<false>(proj, ldp, f_bias, lower, norm_w, eps, state, slots, cu,
                                   positions, out, ldo, num_seqs, max_seqlen, H, d, dv, dt,
-                                  nullptr, 0, 0.f, 0.f, st);
+                                  nullptr, 0, 0.f, 0.f, max_len, st);
 }
 
 // Gated linear attention: proj row [H*d q | H*d k | H*dv v | H*dv gate | ...] (fp32), z
@@ -338,10 +341,10 @@ extern "C" int dli_hgrn2(const float* proj, int ldp, const void* f_bias, const v
 extern "C" int dli_gla(const float* proj, int ldp, const float* z, int ldz, const void* a_bias,
                        float inv_tau, float qscale, const void* norm_w, float eps, float* state,
                        const int* slots, const int* cu, const int* positions, void* out, int ldo,
-                       int num_seqs, int max_seqlen, int H, int d, int dv, int dt,
+                       int num_seqs, int max_seqlen, int max_len, int H, int d, int dv, int dt,
                        hipStream_t st) {
   if (z == nullptr || a_bias == nullptr) return (int)hipErrorInvalidValue;
   return launch_recurrence<true>(proj, ldp, a_bias, nullptr, norm_w, eps, state, slots, cu,
                                  positions, out, ldo, num_seqs, max_seqlen, H, d, dv, dt, z, ldz,
-                                 inv_tau, qscale, st);
+                                 inv_tau, qscale, max_len, st);
 }

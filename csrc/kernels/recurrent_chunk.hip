@@ -130,6 +130,7 @@ struct ChunkArgs {
   const int* slots; const int* cu; const int* positions;
   void* out; int ldo; float out_scale;
   int H, d, dv;
+  int min_len;                                  // sequences that bring fewer tokens are left alone
   const float* gates;                           // MLSTM: [T][H][4] = a, b, exp(-m)
   // nseg > 1: the portions are cut in segments of seg_tokens, (sequence s, segment k, head h) being
   // unit (s nseg + k) H + h of: the state after a segment, from nothing (from the portion's start for
@@ -182,7 +183,7 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
   const int h = blockIdx.x, s = blockIdx.y / segs, seg = blockIdx.y % segs, c0 = blockIdx.z * COLS;
   const int end = a.cu[s + 1], first = a.cu[s];
   const int slot = a.slots[s], t0 = first + seg * a.seg_tokens;
-  if (end <= t0) return;
+  if (end <= t0 || end - first < a.min_len) return;
   const int t1 = seg + 1 < a.nseg && end - t0 > a.seg_tokens ? t0 + a.seg_tokens : end;
   const bool last = t1 == end, cut = end - first > a.seg_tokens;
   if (STATE && (last || slot < 0)) return;
@@ -658,7 +659,7 @@ __global__ void __launch_bounds__(512) mlstm_gates_kernel(ChunkArgs a, float* ga
   __shared__ float ig[N], fg[N], m[N + 1];
   const int h = blockIdx.x, s = blockIdx.y, H = a.H, tid = threadIdx.x, lane = tid & 63;
   const int slot = a.slots[s], first = a.cu[s], end = a.cu[s + 1];
-  if (slot < 0 || end <= first) return;
+  if (slot < 0 || end <= first || end - first < a.min_len) return;
   float* mp = a.nstate + ((long)slot * H + h) * (a.d + 1) + a.d;
   const int ioff = 2 * H * a.d + 2 * H * a.dv + h;
   if (tid == 0) m[0] = a.positions[first] == 0 ? 0.f : *mp;
@@ -732,17 +733,20 @@ int launch_by_width(const ChunkArgs& a, int num_seqs, hipStream_t st) {
 // some 0.4 of a block's time. In block times, with 3 to fill and drain a workgroup and the fold. The
 // segments' states take at most 256 MB of scratch.
 static size_t unit_floats(int d, int dv) { return (size_t)d * dv + 2 * UNIT; }
-static int pick_segments(int H, int d, int dv, int num_seqs, int max_seqlen, int T) {
+static int pick_segments(int H, int d, int dv, int num_seqs, int max_seqlen, int T, int min_len) {
+  // the sequences that min_len leaves count for nothing: beside the longest at most this many others
+  const int others = (T - max_seqlen) / (min_len > 1 ? min_len : 1);
+  const int seqs = others < 0 ? 1 : others < num_seqs ? 1 + others : num_seqs;
   const long wg = (long)H * ((dv + COLS - 1) / COLS);
   const auto rounds = [&](long units) { return (units * wg + 255) / 256; };
-  float best = 0.9f * rounds(num_seqs) * (max_seqlen / 16 + 3.f);
+  float best = 0.9f * rounds(seqs) * (max_seqlen / 16 + 3.f);
   int pick = 1;
   for (int n = 2; n <= 16 && (long)num_seqs * n <= 65535; ++n) {
     const int len = ((max_seqlen + n - 1) / n + TB - 1) / TB * TB;
     if (len < 128) break;
     const int k = (max_seqlen + len - 1) / len;
     if ((size_t)num_seqs * k * H * unit_floats(d, dv) > (64u << 20)) break;
-    const long all = (long)num_seqs * k, most = T / len + num_seqs, units = all < most ? all : most;
+    const long all = (long)seqs * k, most = T / len + seqs, units = all < most ? all : most;
     const float cost = rounds(units) * (len / 16 + 3.f) * 1.4f + 0.4f * k;
     if (cost < best) { best = cost; pick = k; }
   }
@@ -756,14 +760,15 @@ static int segment_tokens(int max_seqlen, int nseg) {
 
 // scratch that dli_recurrence_chunks takes for a step of T tokens (nullptr there: portions stay whole,
 // which MLSTM does not take)
-extern "C" long dli_recurrence_workspace_bytes(int mode, int num_seqs, int max_seqlen, int T, int H,
-                                               int d, int dv) {
-  const int n = pick_segments(H, d, dv, num_seqs, max_seqlen, T);
+extern "C" long dli_recurrence_workspace_bytes(int mode, int num_seqs, int max_seqlen, int T,
+                                               int min_len, int H, int d, int dv) {
+  const int n = pick_segments(H, d, dv, num_seqs, max_seqlen, T, min_len);
   const size_t gates = mode == MLSTM ? (size_t)T * H * 4 : 0;
   return (long)((gates + (n > 1 ? (size_t)num_seqs * n * H * unit_floats(d, dv) : 0)) * 4);
 }
 
-// Portions of a step's sequences (mode as above). hipErrorNotSupported: a size that the walk takes
+// Portions of a step's sequences that bring at least min_len tokens (mode as above; the others' rows and
+// states are left alone). hipErrorNotSupported: a size that the walk takes
 // (d > 128, or a normed head wider than 128).
 extern "C" int dli_recurrence_chunks(int mode, const float* proj, int ldp, const float* z, int ldz,
                                      const void* bias, const void* lower, float inv_tau, float qscale,
@@ -771,16 +776,16 @@ extern "C" int dli_recurrence_chunks(int mode, const float* proj, int ldp, const
                                      const void* norm_w, float eps, float* state, float* nstate,
                                      const int* slots, const int* cu, const int* positions, void* out,
                                      int ldo, float out_scale, int num_seqs, int max_seqlen, int T,
-                                     int H, int d, int dv, int dt, void* ws, hipStream_t st) {
+                                     int min_len, int H, int d, int dv, int dt, void* ws, hipStream_t st) {
   if (num_seqs <= 0 || max_seqlen <= 0) return 0;
   if (H < 1 || d < 1 || dv < 1 || num_seqs > 65535 || state == nullptr || slots == nullptr ||
       out == nullptr || (dt != 0 && dt != 1))
     return (int)hipErrorInvalidValue;
   if (d > 128 || (mode != FIXED && dv > COLS)) return (int)hipErrorNotSupported;
   ChunkArgs a{proj, ldp, z, ldz, bias, lower, inv_tau, qscale, decays, if_b, cap, norm_w, eps, state,
-              nstate, slots, cu, positions, out, ldo, out_scale, H, d, dv, nullptr, 1 << 30, 1,
+              nstate, slots, cu, positions, out, ldo, out_scale, H, d, dv, min_len, nullptr, 1 << 30, 1,
               nullptr, nullptr, nullptr};
-  const int nseg = ws != nullptr ? pick_segments(H, d, dv, num_seqs, max_seqlen, T) : 1;
+  const int nseg = ws != nullptr ? pick_segments(H, d, dv, num_seqs, max_seqlen, T, min_len) : 1;
   float* scratch = (float*)ws;
   float* gates = scratch;
   if (mode == MLSTM) {

@@ -72,6 +72,7 @@ struct ScalarRecArgs {
   const float* table; int rot;    // FORM 2: [T, rot] cosines | sines
   const float* dt; int ldt;       // FORM 3: [T, H]
   const float* dt_bias; const float* rate; const float* skip; int G;
+  int max_len = 1 << 30;          // sequences that bring more tokens are left alone
 };
 
 __device__ __forceinline__ float softplus32(float z) {
@@ -101,6 +102,7 @@ __global__ void __launch_bounds__(1024) scalar_recurrence_kernel(ScalarRecArgs a
   const int h = blockIdx.x, s = blockIdx.y;
   const int slot = a.slots[s];
   const int t0 = a.cu[s], t1 = a.cu[s + 1];
+  if (t1 - t0 > a.max_len) return;
   const int c = threadIdx.x % dvp, part = threadIdx.x / dvp;
   constexpr bool PLAIN_OUT = FORM == 0 || FORM == 3;
   const bool fused_norm = !PLAIN_OUT && a.raw == nullptr;
@@ -358,19 +360,20 @@ int launch_scalar_recurrence(const ScalarRecArgs& a, int num_seqs, hipStream_t s
 // with exponential gating (out in the storage type dt, norm_w likewise). cw > 0 deals the
 // state's columns to workgroups in blocks of cw (a multiple of 64); form 1 then writes o_t
 // (before the head norm) to raw [T, H*dv] in fp32 and leaves norm, gate and scale to the caller.
+// max_len: sequences that bring more tokens are left alone (recurrent_chunk.hip takes them).
 extern "C" int dli_scalar_recurrence(const float* proj, int ldp, int form, const float* decays,
                                      const float* if_b, float cap, const void* norm_w, float eps,
                                      float* state, float* nstate, const int* slots, const int* cu,
                                      const int* positions, void* out, int ldo, float out_scale,
-                                     int num_seqs, int max_seqlen, int H, int d, int dv, int cw,
-                                     float* raw, int dt, hipStream_t st) {
+                                     int num_seqs, int max_seqlen, int max_len, int H, int d, int dv,
+                                     int cw, float* raw, int dt, hipStream_t st) {
   if (num_seqs <= 0 || max_seqlen <= 0) return 0;
   if (H < 1 || d < 1 || dv < 1 || state == nullptr || cw < 0 || (cw > 0 && cw % 64))
     return (int)hipErrorInvalidValue;
   if (cw == 0 || cw >= dv) { cw = dv; raw = form == 1 ? nullptr : raw; }
   ScalarRecArgs a{proj, ldp, decays, if_b, cap, norm_w, eps, state, nstate, slots, cu, positions,
                   out, ldo, out_scale, raw, H, d, dv, cw, 1, nullptr, 0, nullptr, 0, nullptr, nullptr,
-                  nullptr, 1};
+                  nullptr, 1, max_len};
   if (form == 0) {
     if (decays == nullptr || out == nullptr) return (int)hipErrorInvalidValue;
     return launch_scalar_recurrence<float, 0>(a, num_seqs, st);

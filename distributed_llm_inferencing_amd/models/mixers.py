@@ -51,6 +51,11 @@ class StepView:
             t = self.tables[key] = H.rotation_table(self.positions, lp["rot_freq"])
         return t
 
+    @property
+    def min_seqlen(self) -> int:
+        """Tokens of the step's shortest sequence (0: unknown)."""
+        return int(self.host_lens.min(initial=1 << 30)) if self.host_lens is not None else 0
+
     def visible(self, window: int):
         """(rows [S], pairs) of ``H.visible_context``, once per step for all layers of a window."""
         key = ("visible", window)
@@ -167,7 +172,7 @@ def hgrn2_mixer(spec: LayerSpec, lp: dict, h, step: StepView, cache, eps: float)
     proj = H.linear_any(h, lp["w_in"])                       # fp32 [T, q | f | v]
     o = H.hgrn2(proj, lp["f_b"], lp["lower"], lp["o_norm"], eps, state, step.state_slots,
                 step.cu_seqlens, step.max_seqlen, step.positions, spec.heads, spec.dim,
-                spec.vdim)
+                spec.vdim, step.min_seqlen)
     return H.linear_any(o, lp["wo"])
 
 
@@ -237,7 +242,7 @@ def gla_mixer(spec: LayerSpec, lp: dict, h, step: StepView, cache, eps: float):
     a1 = H.act_mul(proj[:, a0:], spec.decay_rank, h.dtype, "copy")
     z = H.linear_any(a1, lp["w_a2"])
     o = H.gla(proj, z, lp["a_b"], spec.tau, lp["o_norm"], eps, state, step.state_slots,
-              step.cu_seqlens, step.max_seqlen, step.positions, Hh, d, dv)
+              step.cu_seqlens, step.max_seqlen, step.positions, Hh, d, dv, step.min_seqlen)
     return H.linear_any(o, lp["wo"])
 
 
@@ -265,7 +270,7 @@ def lightning_mixer(spec: LayerSpec, lp: dict, h, step: StepView, cache, eps: fl
     Hh, d, dv = spec.heads, spec.dim, spec.vdim
     proj = H.linear_any(h, lp["w_in"])                       # fp32 [T, q | k | v | gate]
     o = H.lightning(proj, lp["decays"], state, step.state_slots, step.cu_seqlens,
-                    step.max_seqlen, step.positions, Hh, d, dv)
+                    step.max_seqlen, step.positions, Hh, d, dv, step.min_seqlen)
     g0 = 2 * Hh * d + Hh * dv
     return H.linear_any(H.rmsnorm_cols(o, lp["o_norm"], eps, gate=proj[:, g0:g0 + Hh * dv]),
                         lp["wo"])
@@ -294,7 +299,7 @@ def parallel_mixer(spec: LayerSpec, lp: dict, h, step: StepView, cache, eps: flo
                        head_gate=True, out_scale=spec.left_scale, out=o[:, :wl])
     H.mlstm(proj[:, nl + l.heads:], lp["if_b"], r.gate_cap, lp["o_norm"], eps, state, mstate,
             step.state_slots, step.cu_seqlens, step.max_seqlen, step.positions, r.heads, r.dim,
-            r.vdim, o[:, wl:], spec.right_scale)
+            r.vdim, o[:, wl:], spec.right_scale, step.min_seqlen)
     return H.linear_any(o, lp["wo"])
 
 

@@ -92,12 +92,12 @@ _SIGS = {
                           P, I, F, P],
     "dli_mix_attention_workspace_bytes": [I],
     "dli_window_attention_mfma_workspace_bytes": [I, I, I, I, I, I, I, I],
-    "dli_hgrn2": [P, I, P, P, P, F, P, P, P, P, P, I, I, I, I, I, I, I, P],
-    "dli_gla": [P, I, P, I, P, F, F, P, F, P, P, P, P, P, I, I, I, I, I, I, I, P],
+    "dli_hgrn2": [P, I, P, P, P, F, P, P, P, P, P, I, I, I, I, I, I, I, I, P],
+    "dli_gla": [P, I, P, I, P, F, F, P, F, P, P, P, P, P, I, I, I, I, I, I, I, I, P],
     # portions of the linear recurrences (recurrent_chunk.hip)
     "dli_recurrence_chunks": [I, P, I, P, I, P, P, F, F, P, P, F, P, F, P, P, P, P, P, P, I, F, I, I, I,
-                              I, I, I, I, P, P],
-    "dli_recurrence_workspace_bytes": [I, I, I, I, I, I, I],
+                              I, I, I, I, I, P, P],
+    "dli_recurrence_workspace_bytes": [I, I, I, I, I, I, I, I],
     # post-norm designs (postnorm.hip)
     "dli_prev_tokens": [P, P, P, P, P, P, I, I, P],
     "dli_embedding_bigram": [P, P, P, P, P, P, I, I, I, I, I, I, I, P],
@@ -112,7 +112,7 @@ _SIGS = {
     "dli_hyper_mix": [P, P, I, P, P, P, P, I, I, I, F, F, I, P],
     "dli_sink_prepare": [P, I, P, P, F, I, I, I, I, I, I, P, F, P, P, P, P, P, I, P],
     "dli_scalar_recurrence": [P, I, I, P, P, F, P, F, P, P, P, P, P, P, I, F, I, I, I, I, I,
-                              I, P, I, P],
+                              I, I, P, I, P],
     # rotated designs (rotary.hip, retention.hip, swa_attention.hip)
     "dli_swa_attention": [P, I, P, L, P, L, P, I, P, P, P, I, I, I, I, I, I, I, I, I, I, F, P, I, I,
                           P, F, P, P],

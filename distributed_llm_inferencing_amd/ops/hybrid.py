@@ -484,34 +484,70 @@ def expanded_latent_attention(q, q_rot, cache, w_ukv, H, r, cu_seqlens, max_seql
 
 
 _CHUNK_HGRN2, _CHUNK_GLA, _CHUNK_FIXED, _CHUNK_MLSTM = range(4)
-# shortest step whose portions run 16 tokens at a time on the matrix cores (recurrent_chunk.hip)
-# instead of the token-by-token walk. 64 sequences, 32 heads of 128: at 8 tokens each the walk takes
-# 58 / 91 / 57 us (hgrn2 / gla / lightning) and a block 85 / 89 / 71; at 16 tokens 96 / 144 / 81 and
-# 87 / 92 / 73.
-CHUNK_MIN_TOKENS = 16
+_ANY = 1 << 30                          # no limit to a sequence's tokens
 
 
-def _recurrence_chunks(mode: int, proj, state, slots, cu_seqlens, positions, out, max_seqlen, H, d,
-                       dv, dtype, z=None, bias=None, lower=None, inv_tau=0.0, qscale=1.0,
-                       decays=None, if_b=None, cap=0.0, norm_w=None, eps=0.0, nstate=None,
-                       out_scale=1.0) -> bool:
-    """The chunk form of a recurrence over a step's portions, where it takes the sizes: heads of at
-    most 128 channels, normed ones of at most 128 columns. False: nothing was launched."""
-    if int(max_seqlen) < CHUNK_MIN_TOKENS or d > 128 or (dv > 128 and mode != _CHUNK_FIXED):
-        return False
-    S, T = cu_seqlens.shape[0] - 1, proj.shape[0]
-    nb = N.require_native().dli_recurrence_workspace_bytes(mode, S, int(max_seqlen), T, H, d, dv)
+def chunk_min_tokens(mode: int, S: int, T: int, longest: int, mixed: bool, H: int, d: int) -> int:
+    """Fewest tokens of a sequence that run 16 at a time on the matrix cores (recurrent_chunk.hip)
+    instead of token by token, in a step of T tokens in S sequences of at most ``longest``; ``mixed``:
+    some have fewer than 16. A block of the former fills a CU, whatever it holds; the walk leaves room for others (more of
+    them, the narrower a head) but goes token by token. So where CUs are left over 16 tokens are
+    enough, walk -> blocks, us: hgrn2, 4 x 16 tokens, 32 heads of 128 channels 19 -> 14, of 64 14 -> 11;
+    where a CU has several (sequence, head) in turn it takes 2 blocks at d = 128 (64 x 20 111 and 134,
+    64 x 32 178 and 143; GLA's walk is the slower one from 2 tokens on, 99 and 95) and more of narrower
+    heads (32 of 64: hgrn2 64 x 64 104 and 126, GLA 147 and 150, fixed decay 64 x 48 72 and 69; 16 of
+    32: GLA 64 x 64 70 and 69). Shorter sequences beside longer ones are a launch of their own, unless
+    one round of workgroups takes them all."""
+    # at most this many sequences have 16 tokens or more
+    units = H * min(S, 1 + max(0, T - longest - (S - 1)) // 15)
+    if mixed and S * H <= (288 if mode in (_CHUNK_GLA, _CHUNK_MLSTM) else 256):
+        return 1
+    if d > 64:
+        if mode == _CHUNK_GLA:
+            return 2
+        few = mode == _CHUNK_MLSTM or units <= 512 or T == 16 * S
+    else:
+        few = units <= (512 if d <= 32 or mode == _CHUNK_MLSTM else 256)
+    if few:
+        # (a walk of few tokens is over as soon as the short ones'; the matrix memory's is slower)
+        return 32 if mixed and mode != _CHUNK_MLSTM else 16
+    if d > 64:
+        return 32
+    if d > 32:
+        if units <= 768:
+            return 48 if mode in (_CHUNK_HGRN2, _CHUNK_MLSTM) else 32
+        return {_CHUNK_HGRN2: 192, _CHUNK_GLA: 96}.get(mode, 48)
+    return 64 if units <= 1536 else 128
+
+
+def _recurrence(mode: int, proj, state, slots, cu_seqlens, positions, out, max_seqlen, min_seqlen, H, d,
+                dv, dtype, walk, z=None, bias=None, lower=None, inv_tau=0.0, qscale=1.0,
+                decays=None, if_b=None, cap=0.0, norm_w=None, eps=0.0, nstate=None,
+                out_scale=1.0) -> None:
+    """A recurrence over a step's portions: ``walk(max_len, longest)`` for the sequences of at most
+    ``max_len`` tokens, the blocks' form for the others where it takes the sizes (heads of at most 128
+    channels, normed ones of at most 128 columns). Short sequences beside long ones run the walk as they do without them.
+    ``min_seqlen``: no sequence is shorter (0: unknown)."""
+    S, T, longest = cu_seqlens.shape[0] - 1, proj.shape[0], int(max_seqlen)
+    if longest < 16 or d > 128 or (dv > 128 and mode != _CHUNK_FIXED):
+        return walk(_ANY, longest)
+    equal = T == S * longest
+    least = chunk_min_tokens(mode, S, T, longest, min_seqlen < 16 and not equal, H, d)
+    if longest < least:
+        return walk(_ANY, longest)
+    if min_seqlen < least and least > 1 and not equal:
+        walk(least - 1, least - 1)
+    nb = N.require_native().dli_recurrence_workspace_bytes(mode, S, longest, T, least, H, d, dv)
     ws = _gemm.workspace(proj.device, nb) if nb else None
     _call("dli_recurrence_chunks", mode, _p(proj), proj.stride(0), _p(z),
           z.stride(0) if z is not None else 0, _p(bias), _p(lower), float(inv_tau), float(qscale),
           _p(decays), _p(if_b), float(cap), _p(norm_w), float(eps), _p(state), _p(nstate), _p(slots),
           _p(cu_seqlens), _p(positions), _p(out), out.stride(0), float(out_scale),
-          S, int(max_seqlen), T, H, d, dv, _dt(dtype), _p(ws), _st())
-    return True
+          S, longest, T, least, H, d, dv, _dt(dtype), _p(ws), _st())
 
 
 def hgrn2(proj, f_bias, lower, norm_w, eps, state, slots, cu_seqlens, max_seqlen, positions,
-          H, d, dv):
+          H, d, dv, min_seqlen: int = 0):
     dtype = norm_w.dtype
     if not proj.is_cuda:
         return R.hgrn2(proj, f_bias, lower, norm_w, eps, state, slots, cu_seqlens, positions,
@@ -519,12 +555,13 @@ def hgrn2(proj, f_bias, lower, norm_w, eps, state, slots, cu_seqlens, max_seqlen
     T = proj.shape[0]
     S = cu_seqlens.shape[0] - 1
     out = torch.empty(T, H * dv, dtype=dtype, device=proj.device)
-    if _recurrence_chunks(_CHUNK_HGRN2, proj, state, slots, cu_seqlens, positions, out, max_seqlen,
-                          H, d, dv, dtype, bias=f_bias, lower=lower, norm_w=norm_w, eps=eps):
-        return out
-    _call("dli_hgrn2", _p(proj), proj.stride(0), _p(f_bias), _p(lower), _p(norm_w), float(eps),
-          _p(state), _p(slots), _p(cu_seqlens), _p(positions), _p(out), out.stride(0), S,
-          int(max_seqlen), H, d, dv, _dt(dtype), _st())
+
+    def walk(max_len, longest):
+        _call("dli_hgrn2", _p(proj), proj.stride(0), _p(f_bias), _p(lower), _p(norm_w), float(eps),
+              _p(state), _p(slots), _p(cu_seqlens), _p(positions), _p(out), out.stride(0), S, longest,
+              max_len, H, d, dv, _dt(dtype), _st())
+    _recurrence(_CHUNK_HGRN2, proj, state, slots, cu_seqlens, positions, out, max_seqlen, min_seqlen, H,
+                d, dv, dtype, walk, bias=f_bias, lower=lower, norm_w=norm_w, eps=eps)
     return out
 
 
@@ -749,7 +786,7 @@ def head_gate(o, g, dtype) -> torch.Tensor:
 
 
 def gla(proj, z, a_bias, tau: float, norm_w, eps, state, slots, cu_seqlens, max_seqlen,
-        positions, H, d, dv):
+        positions, H, d, dv, min_seqlen: int = 0):
     """Gated linear attention over per-sequence state slots (``reference.gla``): proj fp32
     [T, q | k | v | gate | ...], z fp32 [T, H*d]; returns the normed, gated read-out
     [T, H*dv] in the storage dtype."""
@@ -760,13 +797,14 @@ def gla(proj, z, a_bias, tau: float, norm_w, eps, state, slots, cu_seqlens, max_
     T = proj.shape[0]
     S = cu_seqlens.shape[0] - 1
     out = torch.empty(T, H * dv, dtype=dtype, device=proj.device)
-    if _recurrence_chunks(_CHUNK_GLA, proj, state, slots, cu_seqlens, positions, out, max_seqlen, H,
-                          d, dv, dtype, z=z, bias=a_bias, inv_tau=1.0 / tau, qscale=d ** -0.5,
-                          norm_w=norm_w, eps=eps):
-        return out
-    _call("dli_gla", _p(proj), proj.stride(0), _p(z), z.stride(0), _p(a_bias), float(1.0 / tau),
-          float(d ** -0.5), _p(norm_w), float(eps), _p(state), _p(slots), _p(cu_seqlens),
-          _p(positions), _p(out), out.stride(0), S, int(max_seqlen), H, d, dv, _dt(dtype), _st())
+
+    def walk(max_len, longest):
+        _call("dli_gla", _p(proj), proj.stride(0), _p(z), z.stride(0), _p(a_bias), float(1.0 / tau),
+              float(d ** -0.5), _p(norm_w), float(eps), _p(state), _p(slots), _p(cu_seqlens),
+              _p(positions), _p(out), out.stride(0), S, longest, max_len, H, d, dv, _dt(dtype), _st())
+    _recurrence(_CHUNK_GLA, proj, state, slots, cu_seqlens, positions, out, max_seqlen, min_seqlen, H, d,
+                dv, dtype, walk, z=z, bias=a_bias, inv_tau=1.0 / tau, qscale=d ** -0.5, norm_w=norm_w,
+                eps=eps)
     return out
 
 
@@ -849,7 +887,8 @@ def sink_prepare(proj, qw, kw, eps, H, G, d, dv, rot_dims, freq, mscale, positio
     return q
 
 
-def lightning(proj, decays, state, slots, cu_seqlens, max_seqlen, positions, H, d, dv):
+def lightning(proj, decays, state, slots, cu_seqlens, max_seqlen, positions, H, d, dv,
+              min_seqlen: int = 0):
     """Linear attention with one fixed decay per head over per-sequence state slots
     (``reference.lightning``): the raw read-outs fp32 [T, H*dv]."""
     if not proj.is_cuda:
@@ -857,12 +896,13 @@ def lightning(proj, decays, state, slots, cu_seqlens, max_seqlen, positions, H, 
     T = proj.shape[0]
     S = cu_seqlens.shape[0] - 1
     out = torch.empty(T, H * dv, dtype=torch.float32, device=proj.device)
-    if _recurrence_chunks(_CHUNK_FIXED, proj, state, slots, cu_seqlens, positions, out, max_seqlen,
-                          H, d, dv, torch.float32, decays=decays):
-        return out
-    _call("dli_scalar_recurrence", _p(proj), proj.stride(0), 0, _p(decays), None, 0.0, None, 0.0,
-          _p(state), None, _p(slots), _p(cu_seqlens), _p(positions), _p(out), out.stride(0), 1.0,
-          S, int(max_seqlen), H, d, dv, _column_block(S, H, d, dv, max_seqlen), None, 1, _st())
+
+    def walk(max_len, longest):
+        _call("dli_scalar_recurrence", _p(proj), proj.stride(0), 0, _p(decays), None, 0.0, None, 0.0,
+              _p(state), None, _p(slots), _p(cu_seqlens), _p(positions), _p(out), out.stride(0), 1.0,
+              S, longest, max_len, H, d, dv, _column_block(S, H, d, dv, longest), None, 1, _st())
+    _recurrence(_CHUNK_FIXED, proj, state, slots, cu_seqlens, positions, out, max_seqlen, min_seqlen, H,
+                d, dv, torch.float32, walk, decays=decays)
     return out
 
 
@@ -879,7 +919,7 @@ def _column_block(S: int, H: int, d: int, dv: int, max_seqlen: int) -> int:
 
 
 def mlstm(proj, if_b, cap: float, norm_w, eps: float, state, mstate, slots, cu_seqlens,
-          max_seqlen, positions, H, d, dv, out, out_scale: float = 1.0):
+          max_seqlen, positions, H, d, dv, out, out_scale: float = 1.0, min_seqlen: int = 0):
     """Matrix memory with exponential gating over per-sequence state slots
     (``reference.mlstm``); the normed, gated, scaled read-out is written to ``out`` [T, H*dv]
     (storage dtype; may be a column slice of a wider buffer). ``state`` fp32 [slots, H, d, dv];
@@ -888,22 +928,23 @@ def mlstm(proj, if_b, cap: float, norm_w, eps: float, state, mstate, slots, cu_s
         return R.mlstm(proj, if_b, cap, norm_w, eps, state, mstate, slots, cu_seqlens, positions,
                        H, d, dv, out, out_scale)
     S = cu_seqlens.shape[0] - 1
-    if _recurrence_chunks(_CHUNK_MLSTM, proj, state, slots, cu_seqlens, positions, out, max_seqlen,
-                          H, d, dv, norm_w.dtype, qscale=d ** -0.5, if_b=if_b, cap=cap,
-                          norm_w=norm_w, eps=eps, nstate=mstate, out_scale=out_scale):
-        return out
-    cw = _column_block(S, H, d, dv, max_seqlen)
-    # with column blocks no workgroup sees a whole head: the read-outs leave in fp32 and the
-    # per-head norm, gate and scale run as a row kernel
-    raw = torch.empty(proj.shape[0], H * dv, dtype=torch.float32, device=proj.device) if cw else None
-    _call("dli_scalar_recurrence", _p(proj), proj.stride(0), 1, None, _p(if_b), float(cap),
-          _p(norm_w), float(eps), _p(state), _p(mstate), _p(slots), _p(cu_seqlens),
-          _p(positions), _p(out), out.stride(0), float(out_scale), S, int(max_seqlen), H, d, dv,
-          cw, _p(raw), _dt(norm_w.dtype), _st())
-    if cw:
-        g0 = 2 * H * d + H * dv
-        rmsnorm_cols(raw, norm_w, eps, gate=proj[:, g0:g0 + H * dv], groups=H, out=out,
-                     out_scale=out_scale)
+
+    def walk(max_len, longest):
+        # with column blocks no workgroup sees a whole head: the read-outs leave in fp32 and the
+        # per-head norm, gate and scale run as a row kernel over all rows (so not beside the blocks' form)
+        cw = _column_block(S, H, d, dv, longest) if max_len == _ANY else 0
+        raw = torch.empty(proj.shape[0], H * dv, dtype=torch.float32, device=proj.device) if cw else None
+        _call("dli_scalar_recurrence", _p(proj), proj.stride(0), 1, None, _p(if_b), float(cap),
+              _p(norm_w), float(eps), _p(state), _p(mstate), _p(slots), _p(cu_seqlens),
+              _p(positions), _p(out), out.stride(0), float(out_scale), S, longest, max_len, H, d, dv,
+              cw, _p(raw), _dt(norm_w.dtype), _st())
+        if cw:
+            g0 = 2 * H * d + H * dv
+            rmsnorm_cols(raw, norm_w, eps, gate=proj[:, g0:g0 + H * dv], groups=H, out=out,
+                         out_scale=out_scale)
+    _recurrence(_CHUNK_MLSTM, proj, state, slots, cu_seqlens, positions, out, max_seqlen, min_seqlen, H,
+                d, dv, norm_w.dtype, walk, qscale=d ** -0.5, if_b=if_b, cap=cap, norm_w=norm_w, eps=eps,
+                nstate=mstate, out_scale=out_scale)
     return out
 
 

@@ -154,3 +154,65 @@ def check(gpu, mode, d, dv, strong, dtype, lens, slots, first):
     assert off(st, want_s) < 1e-5
     if ns is not None:
         assert off(ns, want_n) < 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["hgrn2", "gla", "lightning", "mlstm"])
+@pytest.mark.parametrize("d,dv,known", [(128, 128, False), (64, 64, True), (24, 20, False)])
+def test_a_short_sequence_does_not_feel_its_neighbours(gpu, mode, d, dv, known):
+    """Single tokens and portions of one step, each alone and all together: a sequence runs the form of
+    its own length, so that its rows and its state are the same to the bit (at d = 128 GLA's portions of
+    2 tokens and more run the blocks' form beside longer ones)."""
+    heads, dtype = 48, torch.bfloat16                 # (few heads: one round of blocks takes them all)
+    lens, rnd = [1, 40, 1, 5, 33, 1, 15], lambda *s: torch.randn(*s, device=gpu)
+    if mode == "gla" and d > 64:
+        lens[3] = lens[6] = 1
+    T, S = sum(lens), len(lens)
+    proj, z = rnd(T, 2 * heads * (d + dv) + 2 * heads), rnd(T, heads * d)
+    bias, low = rnd(heads * d).to(dtype), torch.rand(heads * d, device=gpu).to(dtype)
+    nw = rnd(heads * dv if mode == "mlstm" else dv).to(dtype)
+    ifb, decays = torch.cat([rnd(heads) - 1, rnd(heads) + 3]), torch.linspace(0.5, 0.99, heads, device=gpu)
+    state, nstate = rnd(S, heads, d, dv), rnd(S, heads, d + 1).abs()
+
+    def step(which):
+        rows = torch.cat([torch.arange(sum(lens[:s]), sum(lens[:s + 1])) for s in which]).to(gpu)
+        ls = [lens[s] for s in which]
+        st, ns = state.clone(), nstate.clone()
+        cu = torch.tensor([0] + ls).cumsum(0).int().to(gpu)
+        pos = torch.cat([torch.arange(n) + 9 for n in ls]).int().to(gpu)
+        tail = (torch.tensor(which).int().to(gpu), cu, max(ls), pos, heads, d, dv)
+        more = dict(min_seqlen=min(ls)) if known else {}
+        p = proj[rows].contiguous()
+        if mode == "hgrn2":
+            got = H.hgrn2(p, bias, low, nw, 1e-6, st, *tail, **more)
+        elif mode == "gla":
+            got = H.gla(p, z[rows].contiguous(), bias, 8.0, nw, 1e-6, st, *tail, **more)
+        elif mode == "lightning":
+            got = H.lightning(p, decays, st, *tail, **more)
+        else:
+            got = torch.full((len(rows), heads * dv), float("nan"), dtype=dtype, device=gpu)
+            H.mlstm(p, ifb, 15.0, nw, 1e-6, st, ns, *tail, got, 0.6, **more)
+        return got, st, ns
+    got, st, ns = step(list(range(S)))
+    assert torch.isfinite(got).all()
+    for s in range(S):
+        if lens[s] == 1 and (mode == "hgrn2" or mode == "gla" and d <= 64):
+            continue                              # alone a decode step, whose sums are dealt otherwise
+        alone, sa, na = step([s])
+        at = sum(lens[:s])
+        assert torch.equal(got[at:at + lens[s]], alone), lens[s]
+        assert torch.equal(st[s], sa[s]) and torch.equal(ns[s], na[s]), lens[s]
+
+
+def test_blocks_rule():
+    G, X, L, M = H._CHUNK_GLA, H._CHUNK_HGRN2, H._CHUNK_FIXED, H._CHUNK_MLSTM
+
+    def least(mode, lens, heads, d):
+        return H.chunk_min_tokens(mode, len(lens), sum(lens), max(lens), min(lens) < 16, heads, d)
+    for mode in (G, X, L, M):
+        assert least(mode, [8000], 8, 64) == least(mode, [16] * 4, 32, 64) == 16     # CUs are left over
+        assert least(mode, [20] * 64, 32, 64) > 40 and least(mode, [32] * 256, 16, 32) > 32
+        assert least(mode, [1] * 16 + [2048], 8, 128) == 1            # one round of workgroups
+        assert least(mode, [1] * 64 + [512], 32, 64) in (16, 32)      # one portion beside single tokens
+    assert [least(m, [20] * 64, 32, 128) for m in (X, G, L, M)] == [32, 2, 32, 16]
+    assert [least(m, [1] * 64 + [512], 32, 128) for m in (X, G, L, M)] == [32, 2, 32, 16]

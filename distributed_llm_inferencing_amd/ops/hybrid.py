@@ -330,6 +330,36 @@ def mla_prepare(proj, cw, eps, H, d, dr, r, rot_dims, inv_freq, positions, slots
     return qn, qf
 
 
+def split_attention_pays(S: int, T: int, longest: int, H: int, G: int, dv: int, keys: int) -> bool:
+    """Whether attention with a sink, a gate a head or an output scale over portions runs the general
+    form (window_attention_mfma.hip) instead of the dedicated one (swa_attention.hip), which does not
+    split a step of few portions over its ``keys``: 2 tokens at 8000 keys, 32 heads of 128 on 8 kv heads,
+    124 us against 280, 16 in each of 4 sequences 128 and 281. From measurements over 1 to 64 sequences of
+    2 to 2048 tokens at 200 to 8000 keys: the general form walks ``keys`` in some 0.2 us each (more, the
+    more kv heads the 8 heads of a workgroup have) divided by its splits, in rounds of 256
+    workgroups of 16 queries; the dedicated one in 0.035 us (64 queries a workgroup; 0.027 at a value
+    width of 64, 0.05 at 192, 0.1 at 256) or 0.049 (256 queries), all at once up to a workgroup a CU.
+    Of 255 steps drawn from 10 head layouts it picks the slower form for 8, 0.6 % lost in the mean."""
+    if longest == 1:
+        return False
+    wgs, most = S * -(-longest // 16) * -(-H // 8), (keys + 14) // 32 + 2
+    splits = 1
+    if most >= 4 and (wgs < 256 or wgs < 1024 and most >= 8):
+        splits = max(1, min((1024 if wgs >= 256 else 512) // wgs, 16, most // 2))
+    walk = 0.19 + 0.03 * max(1, min(8, H) * G // H)
+    walk *= 1.5 if dv > 192 else 1.15 if dv > 128 else 1.0
+    general = 17 + keys * walk * -(-wgs * splits // 256) / splits
+    rows = 256 if longest >= 192 else 64
+    fill = min(S * -(-longest // rows), S + T // rows) * H / 256
+    if rows == 256:
+        walk = 0.049 if dv > 64 else 0.027
+    else:
+        walk = 0.1 if dv > 192 else 0.05 if dv > 128 else 0.035 if dv > 64 else 0.027
+    if fill > 1 and dv <= 128:
+        return False
+    return general < 6 + keys * walk * max(1.0, 1.2 * fill)
+
+
 def window_attention(q, k_cache, v_cache, dq, dv, H, G, cu_seqlens, max_seqlen, positions,
                      block_tables, block_size, window, scale, slopes=None, talk=None, gate=None,
                      chunk: int = 0, k_groups: Optional[int] = None, sink=None,
@@ -361,7 +391,9 @@ def window_attention(q, k_cache, v_cache, dq, dv, H, G, cu_seqlens, max_seqlen, 
     hg = int(bool(head_gate))
     if q.dtype == torch.bfloat16 and MFMA_ATTENTION:
         lib = N.require_native()
-        if Gk == G and not chunk and slopes is None and talk is None:
+        if (Gk == G and not chunk and slopes is None and talk is None
+                and not ((sink is not None or head_gate or out_scale != 1.0) and split_attention_pays(
+                    S, T, int(max_seqlen), H, G, dv, int(window) + int(keep_first)))):
             # grouped-query attention, with or without output gate and sink: the dedicated
             # kernels (a few pairs of key and value widths)
             nb = lib.dli_swa_attention_workspace_bytes(S, int(max_seqlen), H, G, dv, int(window),

@@ -47,3 +47,48 @@ def test_sink_and_head_gate(gpu, d, dv, G, lens, before):
     # weights and outputs rounded to bf16, half an ulp (2^-9) each
     assert float((got - want).norm() / want.norm()) < 2 * 2.0 ** -9
     assert float(got.view(T, heads, dv)[:, 5].abs().max()) < 1e-30        # the sink takes it all
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("split", [False, True])
+@pytest.mark.parametrize("d,dv", [(64, 64), (128, 128), (64, 128), (96, 192), (128, 256)])
+@pytest.mark.parametrize("lens,before", [([1] * 5, [0, 31, 300, 1500, 7]), ([17, 64, 191, 1, 2], [0, 70, 5, 40, 0]),
+                                         ([256, 192, 3], [0, 100, 700])])
+@pytest.mark.parametrize("window,keep,gated", [(1 << 30, 0, True), (100, 3, False)])
+def test_widths_and_kept_tokens(gpu, monkeypatch, split, d, dv, lens, before, window, keep, gated):
+    """Every pair of widths with a sink, an elementwise or a head's gate and kept first tokens, in both
+    forms that a step of few portions may run."""
+    monkeypatch.setattr(H, "split_attention_pays", lambda *a: split)
+    heads, G, block, scale = 4, 2, 16, d ** -0.5
+    g = torch.Generator().manual_seed(sum(lens) + d + dv)
+    S, T, ctx = len(lens), sum(lens), [a + b for a, b in zip(lens, before)]
+    need = [-(-c // block) for c in ctx]
+    perm = torch.randperm(sum(need), generator=g).int()
+    bt, o = torch.zeros(S, max(need), dtype=torch.int32), 0
+    for s, n in enumerate(need):
+        bt[s, :n] = perm[o:o + n]
+        o += n
+    kc, vc = (torch.randn(sum(need) * block, G * w, generator=g).bfloat16() for w in (d, dv))
+    q = torch.randn(T, heads * d, generator=g).bfloat16()
+    gate = torch.randn(T, heads if gated else heads * dv, generator=g)
+    sink = torch.tensor([-3.0, 0.0, 2.0, 4.0])
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist()).int()
+    pos = torch.cat([torch.arange(n) + b for n, b in zip(lens, before)]).int()
+    more = dict(head_gate=gated, out_scale=0.7, keep_first=keep)
+    want = R.window_attention(q, kc, vc, d, dv, heads, G, cu, pos, bt, block, window, scale, gate=gate,
+                              out_dtype=torch.float32, sink=sink, **more).double()
+    got = H.window_attention(q.to(gpu), kc.to(gpu), vc.to(gpu), d, dv, heads, G, cu.to(gpu), max(lens),
+                             pos.to(gpu), bt.to(gpu), block, min(window, max(ctx)), scale,
+                             gate=gate.to(gpu), sink=sink.to(gpu), **more).double().cpu()
+    assert torch.isfinite(got).all()
+    # weights and outputs rounded to bf16, half an ulp (2^-9) each
+    assert float((got - want).norm() / want.norm()) < 2 * 2.0 ** -9
+
+
+def test_few_portions_over_many_keys_are_split():
+    pays = H.split_attention_pays
+    for S, L in ((1, 2), (1, 64), (4, 16), (2, 33)):
+        assert pays(S, S * L, L, 32, 8, 128, 8000) and not pays(S, S * L, L, 32, 8, 128, 300)
+    assert pays(1, 256, 256, 8, 8, 128, 8000) and not pays(1, 1024, 1024, 8, 8, 128, 8000)
+    assert not pays(65, 576, 512, 32, 8, 128, 8000)                  # single tokens beside a portion
+    assert not pays(64, 1024, 16, 32, 8, 128, 8000) and not pays(64, 64, 1, 32, 8, 128, 8000)

@@ -18,7 +18,7 @@
 // waves of a SIMD, in the same phase, wait for each other; the registers allow no third.
 // 4 x 2048 tokens, window 1024: the general form, which stages all heads' keys behind barriers, loads
 // the queries for every tile and transposes the values by 2-byte stores, 2264 us; this 147 + 496.
-// 8000 tokens, window 4096: 8141 -> 2052 us; 64 single ones at 500 keys 182 -> 105.
+// 8000 tokens, window 4096: 8141 -> 2052 us; 64 single ones at 1000 keys 306 -> 167.
 #include "common.h"
 
 typedef __attribute__((address_space(3))) void mix_lds_void;
@@ -34,7 +34,8 @@ constexpr int WROW = TK + 8;       // padded row of the mixed weights [(head, qu
 constexpr int SLOTS_MAX = 4096;    // keys a query tile may see: their cache rows are kept in LDS
 constexpr float LOG2E = 1.4426950408889634f;
 // Fewest query tiles; the general form splits a step of fewer over the keys. This / the general form, us,
-// at ~1000 visible keys: 8 tiles 159 / 151, 16 160 / 157, 20 158 / 238, 32 163 / 304.
+// at ~1000 visible keys: 8 tiles 159 / 151, 16 160 / 157, 20 158 / 238, 32 163 / 304; of single rows 20 at
+// 500, 1000, 2000, 4000 keys 103 / 99, 193 / 203, 290 / 319, 590 / 602, 32 at 4000 612 / 605, 64 630 / 1093.
 constexpr int MIX_MIN_TILES = 20;
 
 struct MixArgs {
@@ -143,7 +144,8 @@ __global__ void __launch_bounds__(STATS ? 256 : 512) mix_attention_kernel(MixArg
 
   for (int tile = 0; tile < ntiles; ++tile) {
     const int j0 = lo + tile * TK;
-    const bool interior = nq == TQ && j0 + TK - 1 <= p0 && j0 > p_last - a.window;
+    // (rows past the last query keep m = l = 0 or are not stored: whatever they hold stays theirs)
+    const bool interior = j0 + TK - 1 <= p0 && j0 > p_last - a.window;
     f32x4 sc[2][HW];
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {

@@ -810,9 +810,9 @@ extern "C" int dli_swa_attention(const void* q, int ldq, const void* k, long k_s
                                  const float* gate, int ldg, int head_gate, const float* sink,
                                  float out_scale, void* ws, hipStream_t st) {
   if (num_seqs <= 0 || max_seqlen <= 0) return 0;
-  if (H < 1 || G < 1 || H % G || window < 1 || keep < 0 || block_size < 1 ||
-      (head_gate && gate == nullptr))
+  if (H < 1 || G < 1 || H % G || window < 1 || keep < 0 || block_size < 1)
     return (int)hipErrorInvalidValue;
+  head_gate = head_gate && gate != nullptr;
   const bool aligned = (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15) == 0 &&
                        (uintptr_t)out % 8 == 0 && ldq % 8 == 0 && k_stride % 8 == 0 &&
                        v_stride % 8 == 0 && ldo % 4 == 0 &&

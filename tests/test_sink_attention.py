@@ -85,6 +85,20 @@ def test_widths_and_kept_tokens(gpu, monkeypatch, split, d, dv, lens, before, wi
     assert float((got - want).norm() / want.norm()) < 2 * 2.0 ** -9
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens", [[1, 1, 1], [17, 3], [200]])
+def test_no_gate_is_no_gate(gpu, lens):
+    """``head_gate`` says how a gate is read; without one it says nothing."""
+    heads, d, block = 4, 64, 16
+    T, S, W = sum(lens), len(lens), -(-max(lens) // block)
+    q, kc, vc = (torch.randn(n, heads * d, device=gpu).bfloat16() for n in (T, S * W * block, S * W * block))
+    bt = torch.arange(S * W, device=gpu).int().view(S, W)
+    cu = torch.tensor([0] + lens).cumsum(0).int().to(gpu)
+    pos = torch.cat([torch.arange(n) for n in lens]).int().to(gpu)
+    args = (q, kc, vc, d, d, heads, heads, cu, max(lens), pos, bt, block, 1000, d ** -0.5)
+    assert torch.equal(H.window_attention(*args, head_gate=True), H.window_attention(*args))
+
+
 def test_few_portions_over_many_keys_are_split():
     pays = H.split_attention_pays
     for S, L in ((1, 2), (1, 64), (4, 16), (2, 33)):

@@ -243,7 +243,8 @@ __device__ __forceinline__ void st4(u16* p, const f32x4 v) {
 __device__ __forceinline__ void st4(float* p, const f32x4 v) { *reinterpret_cast<f32x4*>(p) = v; }
 
 // the same, 4 columns a thread, a row of both halves a workgroup row: 16-byte loads and no division
-// per element. 8192 rows of 2 x 4096 (0.4 GB): 170 -> 63 us.
+// per element. 8192 rows of 2 x 4096 (0.4 GB): 170 -> 63 us. A few wide rows leave CUs idle: 64 of 2 x 8192
+// 3.3 us by columns, 4.8 so; 192 of them 6.6 and 5.9.
 template <typename S>
 __global__ void __launch_bounds__(256) concat_cast4_kernel(
     S* __restrict__ out, const float* __restrict__ a, const float* __restrict__ b, int dim) {
@@ -426,7 +427,10 @@ __global__ void __launch_bounds__(256) attn_prepare_kernel(
 }
 
 // the same, a workgroup a token and d / 4 lanes (a power of two, at most 64) a head, read once in 16-byte
-// pieces, 4 heads of a lane group in flight: 8192 tokens of 32 + 8 heads of 128 (0.27 GB) 146 -> 68 us.
+// pieces, 4 heads of a lane group in flight: 8192 tokens of 32 + 8 heads of 128 (0.27 GB) 146 -> 68 us. A
+// step of few tokens leaves CUs idle and few wide heads leave lane groups idle: a wave per head and
+// token is faster there (32 + 8 heads of 128, this / by waves: 64 tokens 6.5 / 3.2 us, 320 7.2 / 5.9, 512 7.5 / 7.9;
+// 8 + 2 of 64 at 512 4.0 / 3.3, 1024 4.5 / 4.6; 8 + 1 of 128 at 2048 1.06 times, 4 + 1 of 256 at 8192 1.10).
 template <typename S>
 __global__ void __launch_bounds__(256) attn_prepare4_kernel(
     const float* __restrict__ proj, int ldp, const S* __restrict__ qw, const S* __restrict__ kw,
@@ -629,7 +633,8 @@ extern "C" int dli_concat_cast(void* out, const float* a, const float* b, int T,
                                hipStream_t st) {
   if (T <= 0) return 0;
   const int nb = (int)(((long)T * 2 * dim + 255) / 256);
-  if (dim % 4 == 0 && (((uintptr_t)out | (uintptr_t)a | (uintptr_t)b) & 15) == 0) {
+  if ((T >= 160 || dim <= 1024) && dim % 4 == 0 &&
+      (((uintptr_t)out | (uintptr_t)a | (uintptr_t)b) & 15) == 0) {
     DT_SWITCH(dt, (concat_cast4_kernel<u16><<<T, 256, 0, st>>>((u16*)out, a, b, dim)),
               (concat_cast4_kernel<float><<<T, 256, 0, st>>>((float*)out, a, b, dim)));
     DLI_RETURN_LAUNCH();
@@ -710,7 +715,9 @@ extern "C" int dli_attn_prepare(const float* proj, int ldp, const void* qw, cons
   if (T <= 0) return 0;
   const long units = (long)T * (H + G);
   const int nb = (int)((units + 3) / 4);
-  if (d % 4 == 0 && d <= 256 && (d & (d - 1)) == 0 && ldp % 4 == 0 &&
+  const bool many = d <= 64 ? units >= 10240
+                            : (H + G) * d >= 2048 && (units >= 32768 || (T >= 512 && H + G >= 32));
+  if (many && d % 4 == 0 && d <= 256 && (d & (d - 1)) == 0 && ldp % 4 == 0 &&
       (((uintptr_t)proj | (uintptr_t)q_out | (uintptr_t)kcache | (uintptr_t)vcache) & 15) == 0) {
     DT_SWITCH(dt,
               (attn_prepare4_kernel<u16><<<T, 256, 0, st>>>(

@@ -35,6 +35,25 @@ def test_attn_prepare(heads, G, d, pad, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,heads,G,d,pad", [(511, 32, 8, 128, 0), (513, 32, 8, 128, 4), (1707, 5, 1, 64, 4),
+                                             (1639, 16, 4, 256, 0), (245, 40, 2, 4, 0), (1600, 16, 5, 32, 8)])
+def test_attn_prepare_of_many_rows(T, heads, G, d, pad, dtype):
+    """On both sides of the number of rows from which the 16-byte form runs."""
+    g = torch.Generator().manual_seed(T)
+    W = (heads + G) * d
+    proj = torch.randn(T, W + pad, generator=g)
+    qw, kw = (torch.randn(d, generator=g).to(dtype) for _ in range(2))
+    slots = torch.randperm(T + 3, generator=g)[:T].int()
+    slots[::7] = -1
+    kc, vc = (torch.full((T + 3, G * d), 5.0, dtype=dtype) for _ in range(2))
+    kd, vd = kc.cuda(), vc.cuda()
+    want = R.attn_prepare(proj[:, :W], qw, kw, 1e-6, heads, G, d, kc, vc, slots, dtype)
+    got = H.attn_prepare(proj.cuda()[:, :W], qw.cuda(), kw.cuda(), 1e-6, heads, G, d, kd, vd, slots.cuda())
+    for a, b in ((got, want), (kd, kc), (vd, vc)):
+        close(a, b, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("heads,d,dr,r,rot,pad", [(32, 128, 64, 512, 64, 0), (3, 20, 12, 36, 6, 4),
                                                   (2, 64, 32, 48, 0, 0), (4, 16, 10, 48, 8, 0), (1, 8, 4, 4, 2, 1)])
 def test_mla_prepare(heads, d, dr, r, rot, pad, dtype):
@@ -67,6 +86,13 @@ def test_mla_prepare(heads, d, dr, r, rot, pad, dtype):
 @pytest.mark.parametrize("D", [4, 33, 1024, 4100])
 def test_concat_cast(D, dtype):
     a, b = torch.randn(5, D), torch.randn(5, D)
+    assert torch.equal(H.concat_cast(a.cuda(), b.cuda(), dtype).cpu(), torch.cat([a, b], 1).to(dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,D", [(159, 1028), (160, 1028), (170, 4100), (300, 33)])
+def test_concat_cast_of_many_rows(T, D, dtype):
+    a, b = torch.randn(T, D), torch.randn(T, D)
     assert torch.equal(H.concat_cast(a.cuda(), b.cuda(), dtype).cpu(), torch.cat([a, b], 1).to(dtype))
 
 

@@ -198,10 +198,12 @@ __device__ __forceinline__ void visit16(const uint4 v, int base, const float* x,
     visit16(v, base, x, f);
 }
 
-template <typename LT, typename F, typename... G>
-__device__ __forceinline__ void row_scan(const LT* __restrict__ x, int V, F&& f, G... floor) {
-  constexpr int E = 16 / sizeof(LT), U = 8;
-  const int tid = threadIdx.x, nt = blockDim.x;
+// Every step-th round of the workgroup over a row, from the first on (a sample leaves the row's last
+// partial piece out)
+template <int U, typename LT, typename F, typename... G>
+__device__ __forceinline__ void row_rounds(const LT* __restrict__ x, int V, int step, F&& f, G... floor) {
+  constexpr int E = 16 / sizeof(LT);
+  const int tid = threadIdx.x, nt = blockDim.x * step;
   int done = 0;
   if ((reinterpret_cast<uintptr_t>(x) & 15) == 0) {
     const int VE = V / E;
@@ -223,8 +225,13 @@ __device__ __forceinline__ void row_scan(const LT* __restrict__ x, int V, F&& f,
         if (i + u * nt < VE) visit16(a[u], E * (i + u * nt), x, f, floor...);
     }
     done = VE * E;
+    if (step > 1) return;
   }
   for (int j = done + tid; j < V; j += nt) f(ldv(x, j), j);
+}
+template <typename LT, typename F, typename... G>
+__device__ __forceinline__ void row_scan(const LT* __restrict__ x, int V, F&& f, G... floor) {
+  row_rounds<8>(x, V, 1, f, floor...);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -274,9 +281,10 @@ __global__ void __launch_bounds__(256) sample_chunk_kernel(
 #pragma unroll
   for (int j = 0; j < NE; ++j) mk[0] = max(mk[0], key[j]);
   // a lower bound of the chunk's keff-th largest key, as in sample_kernel: the least of the
-  // waves' ceil(keff / 4)-th largest per-thread maxima
-  const uint32_t tw = wave_kth(mk, (keff + 3) / 4);
-  if ((tid & 63) == 0) s_tau[tid >> 6] = tw;
+  // ceil(keff / waves)-th largest per-thread maxima of the waves that have elements
+  const int nw = max(1, min(4, (n + 63) >> 6));
+  const uint32_t tw = wave_kth(mk, (keff + nw - 1) / nw);
+  if ((tid & 63) == 0) s_tau[tid >> 6] = (tid >> 6) < nw ? tw : 0xffffffffu;
   if (tid == 0) s_cnt = 0;
   __syncthreads();
   const uint32_t tau0 = max(min(min(s_tau[0], s_tau[1]), min(s_tau[2], s_tau[3])), 1u);
@@ -368,14 +376,18 @@ __global__ void __launch_bounds__(SMP_THREADS) sample_kernel(
   }
   auto vocab_id = [&](int j) { return map != nullptr ? map[j] : j; };
   // every pass over the row: the candidate list (fp32) or the logits row (fp32 / bf16)
-  auto scan = [&](int n, auto&& f) {
-    if (xc != nullptr) row_scan(xc, n, f);
-    else row_scan(xl, n, f);
+  auto scan = [&](auto&& f) {
+    if (xc != nullptr) row_scan(xc, V, f);
+    else row_scan(xl, V, f);
   };
 
   if (T <= 0.f || K == 1) {                                  // greedy
     ArgMax a{-INFINITY, 0x7fffffff};
-    scan(V, [&](float v, int i) { a = amax(a, ArgMax{v, i}); });
+    const auto larger = [&](float v, int i) { a = amax(a, ArgMax{v, i}); };
+    // (fewer loads in flight where more rows than CUs are walked: 512 rows of 128k bf16 logits 24 us, 27)
+    if (xc != nullptr) row_scan(xc, V, larger);
+    else if (sizeof(LT) == 2 || gridDim.x > 128) row_rounds<4>(xl, V, 1, larger);
+    else row_scan(xl, V, larger);
     a = block_argmax(a, sv, si);
     if (tid == 0) out_tokens[row] = a.i < V ? vocab_id(a.i) : 0;
     return;
@@ -406,23 +418,36 @@ __global__ void __launch_bounds__(SMP_THREADS) sample_kernel(
   bool fast_ok = false, sorted = false;
   // ---- fast path, no full-row select:
   //  (1) tau0: each of the 8 waves takes the ceil(Keff / 8)-th largest of its 64 per-thread
-  //      maxima over the row's first quarter (fewer waves on a short row); the least of them,
+  //      maxima over a sample of the row (fewer waves on a short row); the least of them,
   //      brought nearer to the Keff-th largest of all 512 by a few steps, is tau0. At least Keff elements are >= tau0, so
   //      tau0 <= the row's Keff-th largest. (Without the steps the list runs to 300 - 600.)
+  //      The sample is spread over the row, which may rise or fall with the index, and larger for
+  //      a larger Keff: the list takes -512 ln(1 - Keff / 512) times the row's part in it elements,
+  //      211 for 50 of a quarter, 295 for 128 and 507 for 200 of a half, 355 for 256 of all; a quarter
+  //      would take 1014 for 200, and some thread more than its slots.
   //  (2) one pass over the row; each thread keeps the elements >= tau0 it meets, a few hundred
   //      of 128k over all, in 8 slots of its own in LDS (a shared counter would cost a round trip
-  //      per element). A row that needs more in one thread goes through the full radix select.
+  //      per element). Where a thread needs more (many ties, a row with its large elements in one
+  //      thread's columns) the Keff-th largest of what was kept is a nearer bound for a second pass;
+  //      a row that needs more again goes through the full radix select.
   //  (3) the list's Keff-th largest key is the row's; what reaches it is ranked by counting.
   // 24 rows of 32k / 128k logits, top-k 50: 32 / 42 us with the 512 maxima and the list's 4096 slots
   // selected by histograms and a bitonic sort of the rest -> 16 / 25.
   if (Keff <= 256) {
     uint32_t mk = 0u;
+    int step = Keff <= 64 ? 4 : Keff <= 208 ? 2 : 1;
     // (a short row whole: every thread needs elements)
-    const int first = max((V >> 4) << 2, min(V, 16 * SMP_THREADS));
-    scan(first, [&](float v, int) { mk = max(mk, f2key(v)); });
+    while (step > 1 && V < step * 16 * SMP_THREADS) step >>= 1;
+    int pieces;                                   // of a first round over the row
+    const auto sample = [&](auto* x) {
+      row_rounds<8>(x, V, step, [&](float v, int) { mk = max(mk, f2key(v)); });
+      pieces = (reinterpret_cast<uintptr_t>(x) & 15) ? V : V / (int)(16 / sizeof(*x));
+    };
+    if (xc != nullptr) sample(xc);
+    else sample(xl);
     constexpr int NWV = SMP_THREADS / 64, SLOTS = 2 * SMP_CAP / SMP_THREADS;
     const uint32_t mk1[1] = {mk};
-    const int nw = min(NWV, (first + 255) >> 8);  // waves that met elements
+    const int nw = max(1, min(NWV, (pieces + 63) >> 6));   // waves that met elements
     const uint32_t tw = wave_kth(mk1, (Keff + nw - 1) / nw);
     if ((tid & 63) == 0) s_tau[tid >> 6] = (tid >> 6) < nw ? tw : 0xffffffffu;
     if (tid == 0) s_cnt = 0;
@@ -438,10 +463,7 @@ __global__ void __launch_bounds__(SMP_THREADS) sample_kernel(
       tau0 = max(tau0, wave_kth(ck, Keff, tau0, 7));
     }
     tau0 = max(tau0, 1u);                         // key 0 is no element
-    // !(v < tf) is true of every element with a key >= tau0 (and of NaNs and zeros below it): one
-    // compare an element, the keys only where one of 16 bytes passes
-    const float tf = key2f(tau0);
-    int cnt = 0;
+    int cnt;
     auto hit = [&](float v, int i) {
       const uint32_t k = f2key(v);
       if (k >= tau0) {
@@ -452,11 +474,28 @@ __global__ void __launch_bounds__(SMP_THREADS) sample_kernel(
         ++cnt;
       }
     };
-    if (xc != nullptr) row_scan(xc, V, hit, tf);
-    else row_scan(xl, V, hit, tf);
-    const uint32_t at = cnt ? atomicAdd(&s_cnt, (uint32_t)cnt) : 0u;
-    const int dropped = __syncthreads_or(cnt > SLOTS ? 1 : 0);
-    const uint32_t nc = s_cnt;
+    uint32_t at, nc;
+    int dropped;
+    for (bool again = false;; again = true) {
+      // !(v < tf) is true of every element with a key >= tau0 (and of NaNs and zeros below it): one
+      // compare an element, the keys only where one of 16 bytes passes
+      const float tf = key2f(tau0);
+      cnt = 0;
+      if (xc != nullptr) row_scan(xc, V, hit, tf);
+      else row_scan(xl, V, hit, tf);
+      at = cnt ? atomicAdd(&s_cnt, (uint32_t)cnt) : 0u;
+      dropped = __syncthreads_or(cnt > SLOTS ? 1 : 0);
+      nc = s_cnt;
+      if (!dropped || again) break;
+      for (int j = cnt; j < SLOTS; ++j) ckey[tid + SMP_THREADS * j] = 0u;
+      __syncthreads();
+      const uint32_t t = radix_kth(ckey, SLOTS * SMP_THREADS, (uint32_t)Keff, hist, sv, s_sel);
+      if (t <= tau0) break;                       // (0: fewer than Keff were kept)
+      __syncthreads();
+      tau0 = t;
+      if (tid == 0) s_cnt = 0;
+      __syncthreads();
+    }
     if (!dropped && nc >= (uint32_t)Keff) {
       if (nc <= 512) {
         for (int j = 0; j < cnt; ++j) {
@@ -539,7 +578,7 @@ __global__ void __launch_bounds__(SMP_THREADS) sample_kernel(
     const int shift = 24 - 8 * pass;
     for (int i = tid; i < 256; i += blockDim.x) hist[i] = 0;
     __syncthreads();
-    scan(V, [&](float v, int) {
+    scan([&](float v, int) {
       const uint32_t k = f2key(v);
       if ((k & pmask) == prefix) atomicAdd(&hist[(k >> shift) & 255u], 1u);
     });
@@ -559,7 +598,7 @@ __global__ void __launch_bounds__(SMP_THREADS) sample_kernel(
   const bool overflow_ties = above_total + s_sel[2] > SMP_CAP;
   if (tid == 0) s_cnt = 0;
   __syncthreads();
-  scan(V, [&](float v, int i) {
+  scan([&](float v, int i) {
     const uint32_t k = f2key(v);
     if (overflow_ties ? k > prefix : (k & pmask) >= prefix) {
       const uint32_t pos = atomicAdd(&s_cnt, 1u);

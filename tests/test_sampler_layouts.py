@@ -43,3 +43,24 @@ def test_same_values_in_any_layout(V, B, dtype):
             got.append(x.gather(1, tok.long()[:, None]).cpu())
             assert (got[-1] >= down[min(K, V) - 1]).all(), (T, K, P)
         assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2]), (T, K, P)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("V", [8191, 8192, 16384, 32768, 32776, 128256, 128257])
+def test_rows_that_rise_with_the_index(V, dtype):
+    """The threshold comes from a sample that is spread over the row, at sizes around those where it is
+    the whole row, a half and a quarter; rows of odd lengths are not aligned."""
+    B = 12
+    g = torch.Generator().manual_seed(V)
+    x = (torch.randn(V, generator=g) + torch.linspace(0, 8, V)).to(dtype)
+    order = torch.randperm(V, generator=g)
+    for K, P in ((1, 1.0), (50, 0.9), (64, 1.0), (65, 1.0), (128, 0.95), (129, 1.0), (256, 1.0)):
+        picked = []
+        for row in (x, x.flip(0), x[order]):
+            rows = row[None].repeat(B, 1).cuda()
+            tok = ops.sample(rows, torch.full((B,), 3.0, device="cuda"), torch.full((B,), K, dtype=torch.int32, device="cuda"),
+                             torch.full((B,), P, device="cuda"), torch.arange(B, dtype=torch.int64, device="cuda") * 77 + K)
+            picked.append(rows.gather(1, tok.long()[:, None]).cpu())
+            assert (picked[-1] >= x.sort(descending=True).values[K - 1]).all(), (K, P)
+        if dtype == torch.float32:               # (bf16 values tie, and ties count in the top k)
+            assert torch.equal(picked[0], picked[1]) and torch.equal(picked[0], picked[2]), (K, P)

@@ -265,14 +265,18 @@ __global__ void __launch_bounds__(512) prefill_attn32_kernel(
   // holds one head's K and V), then the query heads of a group, then row blocks, longest first over
   // all heads. With the blocks of a head fastest the last heads' long blocks started when other CUs
   // ran dry: 1 x 7993 tokens 880 -> 636 us, 4 x 2048 262 -> 176, 8 of 300 to 2000 224 -> 120.
-  const int seq = blockIdx.y, kvh = blockIdx.x % hkv, G = hq / hkv;
-  const int h = kvh * G + blockIdx.x / hkv % G;
+  // Up to 4 heads leave too few of a sequence's blocks in flight before its empty ones come; there a
+  // head's blocks of all sequences follow each other (4 heads, 20 of 100 and 3000 tokens over 1000
+  // cached ones each 150 us, so 137; 32 of 300 22.9, 21.2; 6 heads 128 and 163, 85 and 106).
+  const bool by_head = gridDim.z > 1;
+  const int seq = blockIdx.y, G = hq / hkv;
+  const int h = by_head ? blockIdx.z : blockIdx.x % hkv * G + blockIdx.x / hkv % G, kvh = h / G;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int qc = lane & 31, hi = lane >> 5;
   const int s0 = cu_seqlens[seq], len = cu_seqlens[seq + 1] - s0;
   const int nblk = (len + PL_ROWS - 1) / PL_ROWS;
-  const int blk = (int)((gridDim.x - 1 - blockIdx.x) / hq);
+  const int blk = (int)((gridDim.x - 1 - blockIdx.x) / (by_head ? 1 : hq));
   if (blk >= nblk) return;                                       // workgroup-uniform
   const int nkeys = PAGED ? ctx_lens[seq] : len;
   const int qoff = nkeys - len;
@@ -479,7 +483,8 @@ static int launch_prefill(void* out, int out_stride, const void* qkv, int row_st
   if (hq % hkv || (hd != 64 && hd != 128)) return (int)hipErrorInvalidValue;
   const float sl2 = scale * 1.4426950408889634f;
   if (hd == 128 && max_seqlen >= g_pl_min_len) {     // long sequences: 256-row workgroups
-    dim3 grid32((max_seqlen + PL_ROWS - 1) / PL_ROWS * hq, num_seqs);
+    const int blocks = (max_seqlen + PL_ROWS - 1) / PL_ROWS;
+    const dim3 grid32 = hq <= 4 ? dim3(blocks, num_seqs, hq) : dim3(blocks * hq, num_seqs);
     prefill_attn32_kernel<128, PAGED><<<grid32, 512, 0, st>>>(
         (u16*)out, out_stride, (const u16*)qkv, row_stride, cu_seqlens, hq, hkv, sl2, ctx_lens,
         (const u16*)k_cache, (const u16*)v_cache, block_tables, bt_stride, block_size);

@@ -131,13 +131,14 @@ __global__ void __launch_bounds__(512) swa_prefill32_kernel(SwaArgs a) {
   // key heads fastest, then the query heads of a group, then row blocks, longest lists first
   // (attention_prefill.hip's order): 5 prompts of 900 to 2601 tokens, 32 heads of 128 on 8 kv heads,
   // 339 -> 250 us; expanded latent heads, 6 prompts of 301 to 3000, 416 -> 278
-  const int s = blockIdx.y, kvh = blockIdx.x % a.G, rep = a.H / a.G;
-  const int h = kvh * rep + blockIdx.x / a.G % rep;
+  const bool by_head = gridDim.z > 1;                          // (up to 4 heads, as there)
+  const int s = blockIdx.y, rep = a.H / a.G;
+  const int h = by_head ? blockIdx.z : blockIdx.x % a.G * rep + blockIdx.x / a.G % rep, kvh = h / rep;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int qc = lane & 31, hi = lane >> 5;
   const int t0 = a.cu[s], len = a.cu[s + 1] - t0;
-  const int blk = (int)((gridDim.x - 1 - blockIdx.x) / a.H);
+  const int blk = (int)((gridDim.x - 1 - blockIdx.x) / (by_head ? 1 : a.H));
   const int wg_q0 = blk * LROWS;
   if (wg_q0 >= len) return;                                    // workgroup-uniform
   const int p0 = a.positions[t0];
@@ -706,7 +707,8 @@ int launch_prefill32(SwaArgs a, int num_seqs, int max_seqlen, hipStream_t st) {
     if (e != hipSuccess) return (int)e;
     raised = true;
   }
-  dim3 grid((max_seqlen + LROWS - 1) / LROWS * a.H, num_seqs);
+  const int blocks = (max_seqlen + LROWS - 1) / LROWS;
+  const dim3 grid = a.H <= 4 ? dim3(blocks, num_seqs, a.H) : dim3(blocks * a.H, num_seqs);
   swa_prefill32_kernel<DK, DR, DV><<<grid, 512, sh, st>>>(a);
   DLI_RETURN_LAUNCH();
 }

@@ -887,7 +887,7 @@ __global__ void __launch_bounds__(256) decode_reduce_kernel(u16* __restrict__ ou
         const float ws = s + u < ns ? __shfl(w, (s + u) & 63, 64) : 0.f;
         den += ws;
 #pragma unroll
-        for (int j = 0; j < E; ++j) acc[j] += ws * v[u][j];
+        for (int j = 0; j < E; ++j) acc[j] += s + u < ns ? ws * v[u][j] : 0.f;   // (0 x inf is NaN)
       }
       return s + U;
     };

@@ -90,3 +90,22 @@ def test_a_wide_table_does_not_change_the_split(B, bound):
     want = reference(qkv[:, :hq * HD].view(B, hq, HD).float(), kc.float(), vc.float(), tables[:, :7],
                      [100] * B, HD ** -0.5)
     assert (got.view(B, hq, HD).float() - want).abs().max() <= 6 * 2 ** -9 + 2 ** -8 * want.abs().max()
+
+
+@pytest.mark.parametrize("splits", [2, 3, 5, 17, 21, 64])
+def test_infinite_values_stay_infinite(splits):
+    """A value that overflowed bf16 in the first or the last split: its channel is infinite and no other
+    one is touched, whatever the number of splits leaves of the reduce's batches."""
+    hq, hkv, n = 4, 1, 64 * splits
+    kc = torch.randn(n // BS, hkv, BS, HD, device="cuda").bfloat16()
+    vc = torch.randn_like(kc)
+    vc[0, 0, 0, 5] = float("inf")
+    vc[-1, 0, 0, 9] = float("-inf")
+    tables = torch.arange(n // BS, device="cuda", dtype=torch.int32)[None]
+    qkv = 0.1 * torch.randn(1, (hq + 2 * hkv) * HD, device="cuda").bfloat16()
+    ctx = torch.tensor([n], dtype=torch.int32, device="cuda")
+    got = ops.decode_attention(qkv, kc, vc, tables, ctx, n, hq, hkv, HD, HD ** -0.5,
+                               num_splits=splits).view(hq, HD).float()
+    assert (got[:, 5] == float("inf")).all() and (got[:, 9] == float("-inf")).all()
+    rest = [c for c in range(HD) if c not in (5, 9)]
+    assert torch.isfinite(got[:, rest]).all()

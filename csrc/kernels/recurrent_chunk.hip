@@ -556,7 +556,24 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
         inv = 1.f / (fmaxf(fabsf(x + gt.A[fr] * y), gt.em[fr]) + 1e-6f);
       }
     }
-    o = mfma4(p, vf, acc);
+    // a masked P_ij is zero, but zero times a value that is not finite is not: such a block's terms are
+    // added one by one, so that no token feels a later one
+    if (__ballot(((vf[0] - vf[0]) + (vf[1] - vf[1])) + ((vf[2] - vf[2]) + (vf[3] - vf[3])) != 0.f) == 0) {
+      o = mfma4(p, vf, acc);
+    } else {
+      o = acc;
+#pragma unroll 1
+      for (int g = 0; g < 4; ++g)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const float v = __shfl(vf[u], 16 * g + fr, 64);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float pij = __shfl(p[u], 16 * g + 4 * q + r, 64);
+            if (4 * g + u <= 4 * q + r) o[r] = fmaf(pij, v, o[r]);
+          }
+        }
+    }
     if (MODE != FIXED) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {

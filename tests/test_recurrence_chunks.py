@@ -204,6 +204,42 @@ def test_a_short_sequence_does_not_feel_its_neighbours(gpu, mode, d, dv, known):
         assert torch.equal(st[s], sa[s]) and torch.equal(ns[s], na[s]), lens[s]
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["hgrn2", "gla", "lightning", "mlstm"])
+@pytest.mark.parametrize("d,dv", [(128, 128), (24, 20)])
+@pytest.mark.parametrize("what", [float("nan"), float("inf")])
+@pytest.mark.parametrize("part", ["key", "value"])
+def test_no_token_feels_a_later_one(gpu, mode, d, dv, what, part):
+    """A key or value that is not finite changes nothing before its own token, in its block of 16 either."""
+    heads, T, bad = 2, 60, 37
+    rnd = lambda *s: torch.randn(*s, device=gpu)  # noqa: E731
+    proj, z, state, nstate = rnd(T, 2 * heads * (d + dv) + 2 * heads), rnd(T, heads * d), rnd(1, heads, d, dv), rnd(1, heads, d + 1).abs()
+    bias, low, nw = rnd(heads * d), torch.rand(heads * d, device=gpu), rnd(heads * dv if mode == "mlstm" else dv)
+    ifb, decays = torch.cat([rnd(heads) - 1, rnd(heads) + 3]), torch.tensor([0.5, 0.99], device=gpu)
+    tail = (torch.zeros(1, dtype=torch.int32, device=gpu), torch.tensor([0, T]).int().to(gpu), T,
+            torch.arange(T, device=gpu).int() + 3, heads, d, dv)
+
+    def step(p):
+        st, ns = state.clone(), nstate.clone()
+        if mode == "hgrn2":
+            return H.hgrn2(p, bias, low, nw, 1e-6, st, *tail), st
+        if mode == "gla":
+            return H.gla(p, z, bias, 8.0, nw, 1e-6, st, *tail), st
+        if mode == "lightning":
+            return H.lightning(p, decays, st, *tail), st
+        got = torch.empty(T, heads * dv, device=gpu)
+        H.mlstm(p, ifb, 15.0, nw, 1e-6, st, ns, *tail, got, 0.6)
+        return got, st
+    good, _ = step(proj)
+    proj[bad, heads * d + 3 if part == "key" else 2 * heads * d + 3] = what
+    got, st = step(proj)
+    assert torch.isfinite(got[:bad]).all()
+    # (fp32 sums of 16 terms in another order)
+    assert (got[:bad] - good[:bad]).abs().max() <= 1e-5 * good.abs().max()
+    if not (mode == "hgrn2" and part == "key" and what == float("inf")):        # (a saturated gate)
+        assert not torch.isfinite(got[bad]).all() and not torch.isfinite(st).all()
+
+
 def test_blocks_rule():
     G, X, L, M = H._CHUNK_GLA, H._CHUNK_HGRN2, H._CHUNK_FIXED, H._CHUNK_MLSTM
 

@@ -187,8 +187,15 @@ def _heuristic(M: int, N: int, K: int, epi: str) -> GemmPlan:
         # rows, K = 4096: N = 4096 / 6144 / 12288 / 28672 in 185 / 274 / 556 / 1284 us against 192 / 288 /
         # 582 / 1337; at K = 14336 it is 5 % ahead for 1536 to 3000 rows (251 against 267) and 4 % behind
         # from 4096 on (643 against 619 at 8192). 16384 rows: 2538 against 2672 at N = 28672, within 2 %
-        # at 6144
-        if (splits == 1 and M >= LARGE_M and K % 128 == 0 and (K <= 8192 or M < 4096)
+        # at 6144. Its biased epilogues are slower, GELU's most (4096 x 3072, K = 768: 48 us against 33,
+        # bias alone 38 and 33; 8192 x 12288, K = 4096 684 and 637), and a pairing one pays where tiles
+        # follow each other or K is long (1024 x 8192, K = 1024, one round of 128 tiles: 27.2 against 26.3,
+        # 8192 x 8192 114 against 116; 4096 x 8192, K = 512 38.0 against 37.1)
+        if epi in PAIR_EPIS:
+            pays = K > 2048 or (K >= 1024 and tiles > NUM_CUS) or N % 64 != 0   # (tile 22 takes no such N)
+        else:
+            pays = epi not in ("bias", "bias_gelu")
+        if (pays and splits == 1 and M >= LARGE_M and K % 128 == 0 and (K <= 8192 or M < 4096)
                 and (M < 16384 or N >= 16384) and tile_ok(55, epi)):
             return GemmPlan("dli", 55, 1)
         return GemmPlan("dli", 22, splits)
@@ -215,9 +222,13 @@ def _heuristic(M: int, N: int, K: int, epi: str) -> GemmPlan:
     elif M <= 256:
         tile = 1 if N <= 8192 else 2
     else:
-        # (the last rows of a prefill wave through the head, M = 512, N = 128256: 513 us on 256x256
-        # tiles, 630 on 128x128)
-        tile = 22 if -(-M // 256) * -(-N // 256) >= 2 * NUM_CUS else 2
+        # (the last rows of a prefill wave through the head, K = 4096, N = 128256: 512 rows 447 us on
+        # 256x256 tiles, 619 on 128x128. Up to 384 rows, which are three tiles of 128, where the last
+        # round of tiles is nearly full and K is not short: 257 rows 419 and 438, but 1.05 times as long
+        # at N = 102400, K = 2048 and 1.14 at 65536, K = 1024)
+        tiles = -(-M // 256) * -(-N // 256)
+        full = 10 * tiles >= 9 * NUM_CUS * -(-tiles // NUM_CUS) and K >= 2048
+        tile = 22 if tiles >= 2 * NUM_CUS and (M > 384 or full) else 2
     bm, bn = TILES[tile]
     tiles = -(-M // bm) * -(-N // bn)
     splits = 1

@@ -1,0 +1,80 @@
+"""The fitted GEMM plans for steps above the decode sizes (ops.gemm.plan): each side of every line, and
+the products that run on them against float64."""
+import pytest
+import torch
+
+from distributed_llm_inferencing_amd import ops
+from distributed_llm_inferencing_amd.ops import gemm as G
+from distributed_llm_inferencing_amd.ops.reference import interleave_gate_up
+
+
+@pytest.fixture(autouse=True)
+def fitted():
+    """No tuned or pinned plan while a test runs."""
+    kept = dict(G._plan_cache), set(G._tuned)
+    G.clear_plans()
+    yield
+    G.clear_plans()
+    G._plan_cache.update(kept[0])
+    G._tuned.update(kept[1])
+
+
+@pytest.mark.parametrize("M,N,K,epi,tile,splits", [
+    # fp32 outputs: half-width tiles where they fill the chip unsplit, else K split as for bf16
+    (1100, 4096, 4096, "f32", 28, 1), (2048, 4096, 6144, "f32", 28, 1), (520, 8192, 4096, "f32", 28, 1),
+    (1024, 4096, 4096, "f32", 22, 4), (1100, 4096, 14336, "f32", 22, 2), (1100, 4096, 6272, "f32", 22, 2),
+    (1100, 4096, 6208, "f32", 22, 1), (2049, 4096, 4096, "f32", 55, 1), (520, 12288, 4096, "f32", 22, 1),
+    # the persistent kernel: from 1024 rows, K in whole pairs of steps, long K for few rows only
+    (1023, 28672, 4096, "none", 22, 1), (1024, 28672, 4096, "none", 55, 1), (8192, 4096, 4160, "none", 22, 1),
+    (4095, 4096, 14336, "none", 55, 1), (4096, 4096, 14336, "none", 22, 1), (16384, 16384, 4096, "none", 55, 1),
+    # not with a bias, nor for a pairing epilogue over short K (but several rounds of tiles of 1024)
+    (4096, 3072, 768, "bias_gelu", 22, 1), (8192, 12288, 4096, "bias_gelu", 22, 1),
+    (4096, 2304, 768, "bias", 22, 1), (1024, 8192, 1024, "silu_mul", 22, 1), (8192, 8192, 1024, "silu_mul", 55, 1),
+    (8192, 8192, 512, "silu_mul", 22, 1), (1024, 8192, 4096, "silu_mul", 55, 1), (1024, 8192, 2048, "gelu_mul", 22, 1),
+    (1024, 8224, 1024, "silu_mul", 55, 1),
+    # the head over a wave's last rows: 256x256 tiles above 384 rows, below in nearly full rounds
+    (512, 128256, 4096, "f32", 22, 1), (385, 102400, 768, "f32", 22, 1), (257, 128256, 4096, "f32", 22, 1),
+    (384, 102400, 4096, "f32", 2, 1), (300, 128256, 1024, "f32", 2, 1), (512, 65280, 4096, "f32", 2, 1)])
+def test_fitted_plan(M, N, K, epi, tile, splits):
+    assert G.plan(M, N, K, epi) == G.GemmPlan("dli", tile, splits)
+
+
+def test_a_fitted_plan_is_of_its_own_rows_and_a_pinned_one_of_its_bucket():
+    assert G._bucket(1100) == G._bucket(2048)
+    assert G.plan(1100, 4096, 14336, "none").splits == 2
+    assert G.plan(2048, 4096, 14336, "none").splits == 2
+    assert G.plan(1024, 4096, 14336, "none").splits == 4
+    assert G.plan(2049, 4096, 14336, "none") == G.GemmPlan("dli", 55, 1)       # the bucket of 4096
+    assert G.plan(4096, 4096, 14336, "none") == G.GemmPlan("dli", 22, 1)
+    G.set_plan(4096, 4096, 14336, "none", G.GemmPlan("dli", 34, 1))
+    for rows in (2049, 3000, 4096):
+        assert G.plan(rows, 4096, 14336, "none") == G.GemmPlan("dli", 34, 1)
+    assert G.plan(2048, 4096, 14336, "none").splits == 2
+
+
+# sizes with partial tiles in both directions; the sums are fp32 in 64 to 4096 steps of 32 exact products
+# (1e-6), bf16 results are rounded once, half an ulp (2^-9) a value
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,epi", [
+    (1100, 4000, 2048, "f32"), (1025, 4104, 4096, "f32"), (1030, 4096, 14336, "f32"), (1500, 1032, 6208, "f32"),
+    (2100, 4104, 1024, "f32"), (300, 65544, 2048, "f32"), (400, 65544, 768, "f32"), (1100, 2312, 768, "bias"),
+    (1100, 3080, 768, "bias_gelu"), (1030, 8224, 1024, "silu_mul"), (1030, 8256, 1024, "silu_mul"), (4100, 4160, 1024, "gelu_mul")])
+def test_products_on_fitted_plans(gpu, M, N, K, epi):
+    g = torch.Generator(device=gpu).manual_seed(M + N)
+    x, w = (torch.randn(r, K, device=gpu, generator=g).bfloat16() for r in (M, N))
+    w = w * K ** -0.5
+    bias = torch.randn(N, device=gpu, generator=g).bfloat16() if epi.startswith("bias") else None
+    pairs = epi in G.PAIR_EPIS
+    want = x.double() @ w.double().t()
+    if epi.startswith("bias"):
+        want += bias.double()
+    if epi == "bias_gelu":
+        want = torch.nn.functional.gelu(want, approximate="tanh")
+    if pairs:
+        gate, up = want[:, :N // 2], want[:, N // 2:]
+        act = torch.nn.functional.silu(gate) if epi == "silu_mul" else torch.nn.functional.gelu(
+            gate, approximate="tanh")
+        want, w = act * up, interleave_gate_up(w[:N // 2], w[N // 2:]).contiguous()
+    got = ops.linear(x, w, bias, epi=epi)
+    assert got.shape == want.shape and got.dtype == (torch.float32 if epi == "f32" else torch.bfloat16)
+    assert float((got.double() - want).norm() / want.norm()) < (1e-5 if epi == "f32" else 2.0 ** -8)

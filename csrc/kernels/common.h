@@ -55,6 +55,15 @@ __device__ __forceinline__ void store8(u16* p, const float* f) {
   *reinterpret_cast<uint4*>(p) = v;
 }
 
+// four consecutive elements (8-byte aligned bf16, 16-byte aligned fp32)
+__device__ __forceinline__ void st4(u16* p, const f32x4 v) {
+  uint2 pk;
+  pk.x = pack2bf(v[0], v[1]);
+  pk.y = pack2bf(v[2], v[3]);
+  *reinterpret_cast<uint2*>(p) = pk;
+}
+__device__ __forceinline__ void st4(float* p, const f32x4 v) { *reinterpret_cast<f32x4*>(p) = v; }
+
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);

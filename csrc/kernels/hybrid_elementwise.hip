@@ -234,14 +234,6 @@ __global__ void __launch_bounds__(256) concat_cast_kernel(
   stf(out + gid, c < dim ? a[(long)t * dim + c] : b[(long)t * dim + c - dim]);
 }
 
-__device__ __forceinline__ void st4(u16* p, const f32x4 v) {
-  uint2 pk;
-  pk.x = pack2bf(v[0], v[1]);
-  pk.y = pack2bf(v[2], v[3]);
-  *reinterpret_cast<uint2*>(p) = pk;
-}
-__device__ __forceinline__ void st4(float* p, const f32x4 v) { *reinterpret_cast<f32x4*>(p) = v; }
-
 // the same, 4 columns a thread, a row of both halves a workgroup row: 16-byte loads and no division
 // per element. 8192 rows of 2 x 4096 (0.4 GB): 170 -> 63 us. A few wide rows leave CUs idle: 64 of 2 x 8192
 // 3.3 us by columns, 4.8 so; 192 of them 6.6 and 5.9.

@@ -41,16 +41,6 @@ template <> __device__ __forceinline__ f32x4 ld4<u16>(const u16* p) {
   return f32x4{__uint_as_float(b.x << 16), __uint_as_float(b.x & 0xffff0000u),
                __uint_as_float(b.y << 16), __uint_as_float(b.y & 0xffff0000u)};
 }
-template <typename S> __device__ __forceinline__ void st4(S* p, f32x4 v);
-template <> __device__ __forceinline__ void st4<float>(float* p, f32x4 v) {
-  *reinterpret_cast<f32x4*>(p) = v;
-}
-template <> __device__ __forceinline__ void st4<u16>(u16* p, f32x4 v) {
-  uint2 pk;
-  pk.x = pack2bf(v[0], v[1]);
-  pk.y = pack2bf(v[2], v[3]);
-  *reinterpret_cast<uint2*>(p) = pk;
-}
 
 // Grid: one workgroup per sequence. Every row's predecessor is read before the slot is
 // overwritten (the barrier), so a one-token portion sees the token of the step before.

@@ -109,14 +109,6 @@ __global__ void __launch_bounds__(1024) hyper_mix_kernel(
     stf((S*)h + (long)t * dim + c, urow[c] * rs * (ldf(w + c) + w_offset));
 }
 
-__device__ __forceinline__ void st4(u16* p, const f32x4 v) {
-  uint2 pk;
-  pk.x = pack2bf(v[0], v[1]);
-  pk.y = pack2bf(v[2], v[3]);
-  *reinterpret_cast<uint2*>(p) = pk;
-}
-__device__ __forceinline__ void st4(float* p, const f32x4 v) { *reinterpret_cast<f32x4*>(p) = v; }
-
 // One workgroup per token. proj row (fp32): [H*d q | G*d k | G*dv v | ...].
 template <typename S>
 __global__ void __launch_bounds__(1024) sink_prepare_kernel(

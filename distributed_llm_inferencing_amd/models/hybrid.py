@@ -42,9 +42,10 @@ the sum of a token's routed experts.
 * The residual stream and every norm are fp32; GEMM operands use the storage dtype of the
   weights (bf16 when serving; fp32 weights give an all-fp32 model). Each residual add is fused
   with the norm that follows it (``ops.hybrid.resadd_groupnorm``).
-* Every step kind — whole prompts, prompt portions, decode rows, mixed — runs the same path:
-  new tokens are written to the paged caches, then attend through the block tables, so a
-  position's logits do not depend on how its sequence was cut into steps.
+* Every step kind — whole prompts, prompt portions, decode rows, mixed — writes its new tokens to
+  the paged caches, attends through the block tables and continues a recurrence from its slot, so
+  a position's logits depend on how its sequence was cut into steps, and on what shares a step, in
+  rounding only (a step's sizes choose kernels and splits).
 """
 from __future__ import annotations
 

@@ -54,20 +54,37 @@ class StepView:
     @property
     def min_seqlen(self) -> int:
         """Tokens of the step's shortest sequence (0: unknown)."""
-        return int(self.host_lens.min(initial=1 << 30)) if self.host_lens is not None else 0
+        if self.host_lens is None:
+            return 0
+        if "min_seqlen" not in self.tables:
+            self.tables["min_seqlen"] = int(self.host_lens.min(initial=1 << 30))
+        return self.tables["min_seqlen"]
 
-    def visible(self, window: int):
-        """(rows [S], pairs) of ``H.visible_context``, once per step for all layers of a window."""
-        key = ("visible", window)
+    def visible_rows(self, window: int):
+        """The rows [S] of ``H.visible_context``, their sum and the most of one sequence, once per step
+        for all layers of a window."""
+        key = ("visible_rows", window)
         if key not in self.tables:
-            self.tables[key] = H.visible_context(self.host_lens, self.host_context, window)
+            rows = H.visible_rows(self.host_lens, self.host_context, window)
+            self.tables[key] = rows, int(rows.sum()), int(rows.max(initial=0))
+        return self.tables[key]
+
+    def visible_pairs(self, window: int) -> int:
+        """The pairs of ``H.visible_context``."""
+        key = ("visible_pairs", window)
+        if key not in self.tables:
+            self.tables[key] = H.visible_context(self.host_lens, self.host_context, window)[1]
         return self.tables[key]
 
     def cu_visible(self, window: int) -> torch.Tensor:
-        """The visible rows' cumulative counts [S+1] int32 on the step's device."""
+        """The visible rows' cumulative counts [S+1] int32 on the step's device (whole prompts': the
+        new tokens')."""
         key = ("cu_visible", window)
         if key not in self.tables:
-            rows = self.visible(window)[0]
+            rows = self.visible_rows(window)[0]
+            if np.array_equal(rows, self.host_lens):
+                self.tables[key] = self.cu_seqlens
+                return self.cu_seqlens
             cu = torch.zeros(len(rows) + 1, dtype=torch.int32, pin_memory=self.positions.is_cuda)
             np.cumsum(rows, dtype=np.int32, out=cu.numpy()[1:])
             self.tables[key] = cu.to(self.positions.device, non_blocking=True)
@@ -210,13 +227,12 @@ def latent_attention_mixer(spec: LayerSpec, lp: dict, h, step: StepView, cache, 
     # the kernel size its slot table and key splits for the keys that exist
     win = min(spec.window, max(1, step.max_context))
     if "w_ukv" in lp and step.host_context is not None:
-        rows, pairs = step.visible(win)
-        total = int(rows.sum())
-        if H.latent_expansion_pays(T, step.max_seqlen, total, pairs, Hh * (d + dv)):
+        _, total, most = step.visible_rows(win)
+        if H.latent_expansion_pays(T, step.max_seqlen, total, lambda: step.visible_pairs(win), Hh * (d + dv)):
             o = H.expanded_latent_attention(q_nope, q_full[:, :, r:], c, lp["w_ukv"][0], Hh, r,
                                             step.cu_seqlens, step.max_seqlen, step.positions,
                                             step.block_tables, step.block_size, step.cu_visible(win),
-                                            total, int(rows.max()), win, spec.scale, gates)
+                                            total, most, win, spec.scale, gates)
             return H.linear_any(o, lp["wo"])
     H.head_linear(q_nope, lp["w_ukT"], q_full)               # q_full[:, h, :r] = W_uk,h^T q_h
     ol = H.window_attention(q_full.view(T, Hh * (r + dr)), c, c, r + dr, r, Hh, 1,

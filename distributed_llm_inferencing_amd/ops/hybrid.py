@@ -459,6 +459,11 @@ def expanded_latent_ok(dtype, d: int, dr: int, dv: int, r: int) -> bool:
     return dtype == torch.bfloat16 and (d, dr, dv) == (128, 64, 128) and r % 64 == 0
 
 
+def visible_rows(lens, context, window: int):
+    """The rows of ``visible_context`` alone."""
+    return np.where(lens > 0, np.minimum(context, lens + (window - 1)), 0)
+
+
 def visible_context(lens, context, window: int):
     """Of a step whose sequences bring ``lens`` new tokens, contexts of ``context`` positions with
     them (int64 arrays): the last positions of each that any of its queries sees, and the pairs of a
@@ -466,7 +471,7 @@ def visible_context(lens, context, window: int):
     step has ceil(longest / 16) for every sequence, dealt to the 8 XCDs in turn. Where that is too many
     to split the keys too, the busiest XCD counts: 64 single tokens beside a portion of 512 (32 to
     a sequence) are all on the same one, 10.1 ms at 1000 keys each where the pairs alone make 0.7."""
-    rows = np.where(lens > 0, np.minimum(context, lens + (window - 1)), 0)
+    rows = visible_rows(lens, context, window)
     n = -(-lens // 16)
     seq = np.repeat(np.arange(len(lens)), n)
     tile = np.arange(len(seq)) - np.repeat(np.cumsum(n) - n, n)
@@ -478,16 +483,18 @@ def visible_context(lens, context, window: int):
     return rows, 128 * int(np.bincount((seq * slots + tile) % 8, keys, 8).max())
 
 
-def latent_expansion_pays(tokens: int, max_seqlen: int, rows: int, pairs: int, width: int) -> bool:
+def latent_expansion_pays(tokens: int, max_seqlen: int, rows: int, pairs, width: int) -> bool:
     """Whether a step expands its visible context's keys and values (``width`` columns of them) instead
     of attending the latent itself: ``rows`` to expand, some 14 ns each at width 8192, against
-    0.44 ns for each of ``pairs`` (``visible_context``) and 75 ns a token for absorbing its query and
-    expanding its output. A layer of 32 heads, absorbed -> expanded: 4 x 2048 tokens 5.6 -> 1.2 ms, 32 x 64
+    0.44 ns for each of ``pairs`` (``visible_context``; or a function that gives them, called where rows
+    and tokens do not decide) and 75 ns a token for absorbing its query and expanding its output. A layer of 32 heads, absorbed -> expanded: 4 x 2048 tokens 5.6 -> 1.2 ms, 32 x 64
     0.48 -> 0.31, 512 tokens at 4096 1.04 -> 0.37, 512 beside 64 single ones at 1000 10.3 -> 1.6; 64 at
     4096 0.23 -> 0.26."""
     if max_seqlen < 64 or (max_seqlen < 96 and rows > 8 * tokens) or rows * width > 1 << 30:
         return False
-    return 14 * rows < 75 * tokens + 0.44 * pairs
+    if 14 * rows < 75 * tokens:
+        return True
+    return 14 * rows < 75 * tokens + 0.44 * (pairs() if callable(pairs) else pairs)
 
 
 def expanded_latent_attention(q, q_rot, cache, w_ukv, H, r, cu_seqlens, max_seqlen, positions,

@@ -119,3 +119,25 @@ def test_expansion_counts_what_a_window_shows():
     # single tokens beside a portion: 10.1 ms absorbed, 1.2 expanded (2.8 and 0.5 at 256)
     for window in (64, 256, 1024, 1 << 30):
         assert pays([512] + [1] * 64, [2000] + [1000] * 64, window)
+
+
+def test_the_pairs_are_asked_for_only_where_they_decide():
+    def never():
+        raise AssertionError
+    assert H.latent_expansion_pays(2048, 2048, 2048, never, 8192)         # a whole prompt
+    assert not H.latent_expansion_pays(33, 33, 33, never, 8192)
+    assert not H.latent_expansion_pays(64, 64, 4160, lambda: 64 * 4160, 8192)
+    assert H.latent_expansion_pays(512, 512, 4608, lambda: 512 * 4608, 8192)
+
+
+def test_cumulative_rows_of_a_step():
+    from distributed_llm_inferencing_amd.models.mixers import StepView
+
+    def view(lens, before):
+        cu = torch.tensor([0] + np.cumsum(lens).tolist(), dtype=torch.int32)
+        lens = np.array(lens, dtype=np.int64)
+        return StepView(cu, int(lens.max()), cu, cu, cu, 16, None, 1 << 30, lens, lens + np.array(before))
+    whole = view([5, 0, 70], [0, 0, 0])
+    assert whole.cu_visible(64) is whole.cu_seqlens and whole.cu_visible(1) is whole.cu_seqlens
+    part = view([5, 70, 0], [3, 40, 9])
+    assert part.cu_visible(10).tolist() == [0, 8, 87, 87] and part.cu_visible(1).tolist() == [0, 5, 75, 75]

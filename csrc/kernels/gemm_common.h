@@ -312,11 +312,13 @@ static __global__ void __launch_bounds__(256) splitk_reduce_kernel(void* __restr
 constexpr int DLI_NOT_MINE = -0x4d494e45;
 
 int gemm_tiles_dispatch(int epi, int tile_cfg, DLI_GEMM_ARGS);
+int gemm_stream_dispatch(int epi, int tile_cfg, DLI_GEMM_ARGS);
 int gemm_8p_dispatch(int epi, int tile_cfg, DLI_GEMM_ARGS);
 int gemm_4w_dispatch(int epi, int tile_cfg, DLI_GEMM_ARGS);
 int gemm_4wp_dispatch(int epi, int tile_cfg, DLI_GEMM_ARGS);
 int gemm_gemv_dispatch(int epi, int tile_cfg, DLI_GEMM_ARGS);
 int gemm_tiles_set_slab_store(int mode);
+int gemm_stream_set_slab_store(int mode);
 int gemm_8p_set_slab_store(int mode);
 int gemm_4w_set_slab_store(int mode);
 

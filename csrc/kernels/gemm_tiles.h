@@ -6,7 +6,7 @@
 #pragma once
 #include "gemm_common.h"
 
-template <int BM, int BN, int EPI, int NS, int WM, int WN>
+template <int BM, int BN, int EPI, int NS, int WM, int WN, int BKT = BK, bool STREAM = false>
 __global__ void __launch_bounds__(64 * WM * WN) gemm_bf16_kernel(
     const u16* __restrict__ A, int lda, const u16* __restrict__ W, int ldw,
     void* __restrict__ C, int ldc, int M, int N, int K, int k_split_len,
@@ -14,7 +14,7 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_bf16_kernel(
   constexpr int NW = WM * WN;                      // waves: WM along M x WN along N
   constexpr int TM = BM / WM, TN = BN / WN;        // wave tile
   constexpr int MI = TM / 16, NI = TN / 16;        // 16x16 MFMA blocks per wave
-  constexpr int A_BYTES = BM * BK * 2, W_BYTES = BN * BK * 2;
+  constexpr int A_BYTES = BM * BKT * 2, W_BYTES = BN * BKT * 2;
   constexpr int BUF = A_BYTES + W_BYTES;
   extern __shared__ __attribute__((aligned(16))) char smem[];
 
@@ -35,7 +35,7 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_bf16_kernel(
   const int m0 = tm * BM, n0 = tn * BN;
   if (m0 >= Mg) return;                             // grouped: empty tile (block-uniform)
   const int kb = ks * k_split_len;
-  const int nk = min(k_split_len, K - kb) / BK;
+  const int nk = min(k_split_len, K - kb) / BKT;
 
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const int wm = wid / WN, wn = wid % WN;
@@ -47,37 +47,48 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_bf16_kernel(
                         ? reinterpret_cast<const int*>(bias) : nullptr;
 
   // ---- per-lane glds source pointers (row clamped in range; swizzled chunk)
-  // one glds wave-instruction stages 8 rows x 128 B; all NW waves share each tile
-  constexpr int A_INSTR = BM / (8 * NW), W_INSTR = BN / (8 * NW);
-  static_assert(A_INSTR * 8 * NW == BM && W_INSTR * 8 * NW == BN, "tile vs waves");
+  // one glds wave-instruction stages 8 rows x 128 B (deeper K-tiles: 4 x 256 B, 2 x 512 B); all NW
+  // waves share each tile. A row's 16-B chunks are XOR-swizzled so that the 16 rows of a fragment read
+  // spread over the banks
+  constexpr int LPR = BKT / 8, RPI = 64 / LPR;     // lanes a row, rows an instruction
+  constexpr int A_INSTR = BM / (RPI * NW), W_INSTR = BN / (RPI * NW);
+  static_assert(A_INSTR * RPI * NW == BM && W_INSTR * RPI * NW == BN, "tile vs waves");
+  auto swz = [](int r) { return BKT == 64 ? (r >> 1) & 7 : r & 15; };
   const u16* a_src[A_INSTR];
   const u16* w_src[W_INSTR];
 #pragma unroll
   for (int i = 0; i < A_INSTR; ++i) {
-    const int r = (i * NW + wid) * 8 + (lane >> 3);
-    const int c = (lane & 7) ^ ((r >> 1) & 7);
+    const int r = (i * NW + wid) * RPI + lane / LPR;
+    const int c = (lane % LPR) ^ swz(r);
     const int gr = min(m0 + r, Mg - 1);
     a_src[i] = (arow != nullptr ? A + (long)arow[row0 + gr] * lda : Ab + (long)gr * lda) + kb +
                c * 8;
   }
 #pragma unroll
   for (int i = 0; i < W_INSTR; ++i) {
-    const int r = (i * NW + wid) * 8 + (lane >> 3);
-    const int c = (lane & 7) ^ ((r >> 1) & 7);
+    const int r = (i * NW + wid) * RPI + lane / LPR;
+    const int c = (lane % LPR) ^ swz(r);
     const int gr = min(n0 + r, N - 1);
     w_src[i] = Wg + (long)gr * ldw + kb + c * 8;
   }
+  // STREAM: tile t starts at K-tile t mod nk and wraps around (see gemm_stream.h)
+  const int rot = STREAM && nk > 0 ? tile % nk : 0;
+  constexpr int W_AUX = STREAM ? 2 : 0;            // nt: each weight line is read once
   auto stage = [&](int buf, int kt) {
     char* base = smem + buf * BUF;
+    if (STREAM) {
+      kt += rot;
+      if (kt >= nk) kt -= nk;
+    }
 #pragma unroll
     for (int i = 0; i < A_INSTR; ++i)
-      __builtin_amdgcn_global_load_lds((gbl_void*)(a_src[i] + kt * BK),
+      __builtin_amdgcn_global_load_lds((gbl_void*)(a_src[i] + kt * BKT),
                                        (lds_void*)(base + (i * NW + wid) * 1024), 16, 0, 0);
 #pragma unroll
     for (int i = 0; i < W_INSTR; ++i)
-      __builtin_amdgcn_global_load_lds((gbl_void*)(w_src[i] + kt * BK),
+      __builtin_amdgcn_global_load_lds((gbl_void*)(w_src[i] + kt * BKT),
                                        (lds_void*)(base + A_BYTES + (i * NW + wid) * 1024), 16,
-                                       0, 0);
+                                       0, W_AUX);
   };
 
   f32x4 acc[MI][NI];
@@ -98,18 +109,18 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_bf16_kernel(
     const char* abuf = smem + buf * BUF;
     const char* wbuf = abuf + A_BYTES;
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
+    for (int kk = 0; kk < BKT / 32; ++kk) {
       const int c = kk * 4 + fq;
       bf16x8 af[MI], bfr[NI];
 #pragma unroll
       for (int i = 0; i < MI; ++i) {
         const int r = a_row[i];
-        af[i] = *reinterpret_cast<const bf16x8*>(abuf + r * 128 + ((c ^ ((r >> 1) & 7)) << 4));
+        af[i] = *reinterpret_cast<const bf16x8*>(abuf + r * (BKT * 2) + ((c ^ swz(r)) << 4));
       }
 #pragma unroll
       for (int j = 0; j < NI; ++j) {
         const int r = w_row[j];
-        bfr[j] = *reinterpret_cast<const bf16x8*>(wbuf + r * 128 + ((c ^ ((r >> 1) & 7)) << 4));
+        bfr[j] = *reinterpret_cast<const bf16x8*>(wbuf + r * (BKT * 2) + ((c ^ swz(r)) << 4));
       }
 #pragma unroll
       for (int i = 0; i < MI; ++i)
@@ -212,24 +223,24 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_bf16_kernel(
   }
 }
 
-template <int BM, int BN, int EPI, int NS, int WM = 2, int WN = 2>
+template <int BM, int BN, int EPI, int NS, int WM = 2, int WN = 2, int BKT = BK, bool STREAM = false>
 static int launch_cfg(const void* A, int lda, const void* W, int ldw, void* C, int ldc, int M,
                       int N, int K, int splits, const void* bias, void* ws,
                       const int* group_off, int groups, hipStream_t st) {
   if (epi_pairs(EPI) && (BN / WN) % 32) return (int)hipErrorInvalidValue;  // gate/up pairs
   const int tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
   int ksl = K / splits;
-  ksl = (ksl / BK) * BK;
+  ksl = (ksl / BKT) * BKT;
   if (ksl * splits != K) return (int)hipErrorInvalidValue;
-  const size_t lds = NS * (size_t)(BM + BN) * BK * 2;
+  const size_t lds = NS * (size_t)(BM + BN) * BKT * 2;
   static bool attr_done = false;                   // > 64 KiB dynamic LDS needs the opt-in
   if (!attr_done) {
-    hipFuncSetAttribute((const void*)gemm_bf16_kernel<BM, BN, EPI, NS, WM, WN>,
+    hipFuncSetAttribute((const void*)gemm_bf16_kernel<BM, BN, EPI, NS, WM, WN, BKT, STREAM>,
                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     attr_done = true;
   }
   dim3 grid(tiles, splits, groups);
-  gemm_bf16_kernel<BM, BN, EPI, NS, WM, WN><<<grid, 64 * WM * WN, lds, st>>>(
+  gemm_bf16_kernel<BM, BN, EPI, NS, WM, WN, BKT, STREAM><<<grid, 64 * WM * WN, lds, st>>>(
       (const u16*)A, lda, (const u16*)W, ldw, C, ldc, M, N, K, ksl, (const u16*)bias,
       (float*)ws, group_off);
   if (splits > 1 && C != nullptr) {       // C == nullptr: leave the fp32 partial slabs for a

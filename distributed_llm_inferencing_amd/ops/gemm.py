@@ -54,7 +54,14 @@ TILES = {0: (64, 64), 1: (64, 128), 2: (128, 128), 3: (128, 256), 4: (256, 128),
          34: (256, 256), 41: (256, 256), 45: (256, 256),
          # 55 = 45 persistent: one workgroup per CU walks its tiles, the next tile's first two
          # K-tiles staged in the current tile's last two (gemm4wp.hip); no split-K / grouped
-         55: (256, 256)}
+         55: (256, 256),
+         # weight-streaming tiles for up to 128 rows (gemm_stream.h): weights nontemporal, K loops
+         # turned from tile to tile, 3 or 4 stages
+         60: (16, 128), 61: (32, 128), 62: (32, 64), 63: (64, 128), 64: (64, 64), 65: (64, 256),
+         66: (96, 128), 67: (128, 128), 68: (128, 256)}
+# their K-tiles
+STREAM_K = {60: 128, 61: 64, 62: 256, 63: 128, 64: 128, 65: 64, 66: 64, 67: 64, 68: 64}
+STREAM_MAX_M = 128
 # the 4-wave plan raced against the 8-phase one in the prefill autotune
 PREFILL_4W_TILE = 45
 # the persistent 4-wave tile (55) raced too
@@ -81,7 +88,7 @@ GEMV_PRO_M1_ONLY = (32, 33)
 DEFER_NORM = os.environ.get("DLI_DEFER_NORM", "1") == "1"
 TILE_WAVES = {13: (2, 4), 14: (4, 2), 15: (2, 4), 16: (4, 2), 17: (2, 4),
               22: (2, 4), 23: (2, 4), 24: (2, 4), 25: (4, 2),
-              26: (4, 2), 28: (4, 2)}
+              26: (4, 2), 28: (4, 2), 60: (1, 4), 66: (1, 4), 68: (2, 4)}
 
 
 def tile_ok(tile: int, epi: str) -> bool:
@@ -112,11 +119,11 @@ PAIR_EPIS = ("silu_mul", "clamp_mul", "relu_mul", "gelu_mul")
 # tiles whose slab-only split-K call can store fp16 partials (EPI "slab16": the generic tile
 # family and the 8-phase kernels); the fused consumers then read half the bytes. The
 # weight-streaming GEMVs and the 4-wave family keep fp32 slabs.
-SLAB16_TILES = frozenset(list(range(0, 22)) + [22, 23, 24, 25, 26, 28])
+SLAB16_TILES = frozenset(list(range(0, 22)) + [22, 23, 24, 25, 26, 28] + list(STREAM_K))
 SLAB16 = os.environ.get("DLI_SLAB_FP32", "0") != "1"      # A/B: fp32 partials everywhere
 # tiles whose grouped SiLU*up GEMM can read its rows through a permutation (the generic
 # family: dli_gemm_grouped_gather), so the MoE gate/up skips the gathered copy of its input
-GATHER_TILES = frozenset(list(range(0, 22)) + [23, 24, 25])
+GATHER_TILES = frozenset(list(range(0, 22)) + [23, 24, 25] + list(STREAM_K))
 NUM_CUS = 256
 
 
@@ -155,6 +162,42 @@ def workspace(device: torch.device, nbytes: int) -> torch.Tensor:
 
 
 LARGE_M = 1024
+
+
+def _stream_plan(M: int, N: int, K: int, epi: str):
+    """Few rows: the weights' read is the product's time. One row of the weight-streaming tiles, narrow
+    ones split over K until about one workgroup a CU, wide ones where N alone gives that many; None for a K of
+    no whole K-tiles. fp32 outputs, us on these against the best other tile:
+    24 rows: 4096 x 4096 11.9 / 13.2, 4096 x 14336 24.3 / 27.2, 12288 x 4096 19.1 / 23.6, 32000 x 4096
+    41.5 / 56.3, 128256 x 4096 167 / 197; 64 rows 13.9 / 14.2, 28.5 / 29.1, 28.2 / 28.2, 45.3 / 59.5, 177 / 209; 2 and 4 rows of the last 157 and 155
+    against 164 on the plain weight stream. From
+    65 rows on the narrow weights stay on two rows of tile 5 or one of tile 7 (96 rows, 4096 x 4096
+    15.6, on tile 66 20.3), the wide ones do not (32000 x 4096 47.2 / 61.7)."""
+    wide = -(-N // 128) >= 3 * NUM_CUS // 4
+    if M <= 32:
+        # (the head: 62's long K-tiles, 24 rows 167 us against 174)
+        tile = 62 if K % 256 == 0 and (not wide or N >= 256 * NUM_CUS) else 61
+    elif M <= 64 and K % 128:
+        tile = 6 if wide else 5
+    elif M <= 64:
+        tile = (65 if N >= 256 * NUM_CUS else 63) if wide else 64
+    elif wide:
+        tile = 68 if N >= 256 * NUM_CUS else 66 if M <= 96 else 67
+    else:
+        tile = 7 if N >= 8192 or K > 8192 else 5
+    step = STREAM_K.get(tile, 64)
+    if K % step:
+        return None
+    bm, bn = TILES[tile]
+    tiles, splits = -(-M // bm) * -(-N // bn), 1
+    most = 2 * NUM_CUS if tile == 5 else NUM_CUS
+    # (K <= 1024: the second launch costs more than the shorter loop saves, 4096 x 1024 at 24 rows 6.1 / 7.8)
+    while (K > 1024 and tiles * splits * 2 <= most and K % (step * splits * 2) == 0
+           and K // (splits * 2) >= 512 and splits < 8):
+        splits *= 2
+    if epi == "splitk" and splits == 1 and K % (2 * step) == 0 and K >= 1024:
+        splits = 2            # the fused reduce consumes partial slabs: need >= 2 slices
+    return GemmPlan("dli", tile, splits)
 
 
 @functools.lru_cache(maxsize=8192)
@@ -205,6 +248,10 @@ def _heuristic(M: int, N: int, K: int, epi: str) -> GemmPlan:
         # residual-adding GEMV (full K): 4 rows a workgroup, 8 K-steps in flight per lane
         # (1024 workgroups on a 4096-wide projection)
         return GemmPlan("dli", 56, 1)
+    if 1 < M <= STREAM_MAX_M and (M > GEMV_MAX_M or epi not in ("splitk", "none")):
+        p = _stream_plan(M, N, K, epi)
+        if p is not None:
+            return p
     if M <= GEMV_MAX_M and epi not in ("clamp_mul", "relu_mul", "gelu_mul"):   # (no GEMV has them)
         # batch-1 / tiny batches: stream the weights (gemv_kernel) with enough workgroups
         # (>= 512, two per CU) to keep ~64 KB of loads in flight per CU
@@ -266,7 +313,17 @@ _grouped_cache: dict = {}
 
 def grouped_plan(rows: int, N: int, K: int, epi: str, groups: int) -> GemmPlan:
     p = _grouped_cache.get((_bucket(rows), N, K, epi, groups))
-    return p if p is not None else GemmPlan("dli", grouped_tile(rows, groups), 1)
+    if p is not None:
+        return p
+    tile = grouped_tile(rows, groups)
+    # experts of few rows: the streaming tile that covers them
+    need = 1.25 * rows / max(1, groups)
+    for t in (61, 63, 66) if "DLI_MOE_TILE" not in os.environ else ():
+        if need <= TILES[t][0]:
+            if K % STREAM_K[t] == 0 and tile_ok(t, epi):
+                tile = t
+            break
+    return GemmPlan("dli", tile, 1)
 
 
 def autotune_grouped(rows: int, w: torch.Tensor, epi: str, iters: int = 5, log=None):
@@ -297,8 +354,11 @@ def autotune_grouped(rows: int, w: torch.Tensor, epi: str, iters: int = 5, log=N
     for tile in sorted(TILES):
         if TILES[tile][0] > 2 * max(64, rows // E + 32) or not tile_ok(tile, epi):
             continue                                  # far taller than an expert's rows
+        if tile in STREAM_K and TILES[tile][0] < rows // E:
+            continue                                  # streams the weights once or not at all
+        step = STREAM_K.get(tile, 64)
         for splits in (1, 2, 4):                      # split-K for long-K expert GEMMs
-            if splits == 1 or (K % (64 * splits) == 0 and K // splits >= 2048):
+            if K % (step * splits) == 0 and (splits == 1 or K // splits >= 2048):
                 cands.append(GemmPlan("dli", tile, splits))
     for p in cands:
         fused = epi == "none" and ops.moe_slab_plan(p)
@@ -576,8 +636,16 @@ def candidate_plans(M: int, N: int, K: int, epi: str):
             continue
         if M > 512 and bm < 128:
             continue
+        if tile in STREAM_K:
+            # one row of tiles; for 2 to 4 rows beside the weight stream's own kernels, but for the
+            # products whose partial sums those keep in fp32
+            if (M > bm or bm >= 2 * max(M, 32) or M < 2
+                    or (M <= GEMV_MAX_M and epi in ("splitk", "none"))):
+                continue
+        elif M <= 64 and tile in (0, 1) and K % 128 == 0:
+            continue                     # slower than their 3-stage and streaming forms
         for splits in (1, 2, 4, 8):
-            if K % (64 * splits) or K // splits < 256:
+            if K % (STREAM_K.get(tile, 64) * splits) or K // splits < 256:
                 continue
             tiles = -(-M // bm) * -(-N // bn)
             if splits > 1 and tiles * splits > 4 * NUM_CUS:

@@ -1,0 +1,95 @@
+"""The weight-streaming GEMM tiles (2 to 128 rows): the fitted plans at each side of their lines, and every
+tile against float64 at the sizes where it can go wrong."""
+import pytest
+import torch
+
+from distributed_llm_inferencing_amd import ops
+from distributed_llm_inferencing_amd.ops import gemm as G
+from distributed_llm_inferencing_amd.ops.reference import interleave_gate_up
+
+
+@pytest.mark.parametrize("M,N,K,epi,tile,splits", [
+    (5, 4096, 4096, "f32", 62, 4), (32, 4096, 4096, "f32", 62, 4), (32, 4096, 4160, "f32", 61, 1),
+    (33, 4096, 4096, "f32", 64, 4), (64, 4096, 4160, "f32", 5, 1), (65, 4096, 4096, "f32", 5, 4),
+    (128, 8192, 4096, "f32", 7, 4), (128, 4096, 14336, "f32", 7, 8), (129, 4096, 4096, "f32", 1, 8),
+    # wide: unsplit on 128 columns, the head on its own tiles
+    (24, 24480, 4096, "silu_mul", 61, 1), (24, 24448, 4096, "silu_mul", 62, 1),
+    (64, 28672, 4096, "silu_mul", 63, 1), (96, 28672, 4096, "silu_mul", 66, 1), (97, 28672, 4096, "silu_mul", 67, 1),
+    (24, 128256, 4096, "f32", 62, 1), (64, 128256, 4096, "f32", 65, 1), (65, 128256, 4096, "f32", 68, 1),
+    # short K is not split, but where a fused reduce follows
+    (24, 4096, 1024, "f32", 62, 1), (24, 4096, 1024, "splitk", 62, 2), (24, 4096, 768, "splitk", 62, 1),
+    # 2 to 4 rows: only what keeps no partial sums in 32 bits; one row stays on the plain weight stream
+    (4, 28672, 4096, "silu_mul", 61, 1), (4, 4096, 4096, "splitk", 30, 2), (2, 28672, 4096, "silu_mul", 61, 1),
+    (1, 28672, 4096, "silu_mul", 29, 1)])
+def test_fitted_plan(M, N, K, epi, tile, splits):
+    assert G._heuristic(M, N, K, epi) == G.GemmPlan("dli", tile, splits)
+
+
+def test_every_candidate_fits_its_rows_and_k():
+    for M in (1, 2, 3, 4, 5, 16, 17, 32, 33, 64, 65, 96, 97, 128, 129, 512):
+        for K in (64, 192, 768, 4096, 4160):
+            for epi in ("f32", "splitk", "silu_mul", "none"):
+                for p in G.candidate_plans(M, 4096, K, epi):
+                    step = G.STREAM_K.get(p.tile)
+                    if step:
+                        assert K % (step * p.splits) == 0 and 2 <= M <= G.TILES[p.tile][0]
+                        assert M > G.GEMV_MAX_M or epi not in ("splitk", "none")
+
+
+# Sums are fp32 in up to 64 steps of 32 exact products (1e-6); bf16 results are rounded once, half an ulp
+# (2^-9) a value; fp16 partial sums likewise (2^-11 each)
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", sorted(G.STREAM_K))
+@pytest.mark.parametrize("rows", ["one", "full", "two rows of tiles"])
+def test_tiles_match_float64(gpu, tile, rows):
+    bm, bn = G.TILES[tile]
+    M = {"one": 1, "full": bm, "two rows of tiles": bm + 3}[rows]
+    step = G.STREAM_K[tile]
+    g = torch.Generator(device=gpu).manual_seed(tile)
+    for N, K, epi, splits in ((bn + 3, step, "f32", 1), (3 * bn - 1, 2 * step, "none", 1), (96, 3 * step, "silu_mul", 1),
+                              (5 * bn + 32, 9 * step, "silu_mul", 1), (bn * 2, 8 * step, "f32", 4),
+                              (260, 4 * step, "slab16", 2), (bn + 16, 5 * step, "bias_gelu", 1)):
+        x = torch.randn(M, K, device=gpu, generator=g).bfloat16()
+        w = (torch.randn(N, K, device=gpu, generator=g) * K ** -0.5).bfloat16()
+        bias = torch.randn(N, device=gpu, generator=g).bfloat16() if epi == "bias_gelu" else None
+        want, plan, tol = x.double() @ w.double().t(), G.GemmPlan("dli", tile, splits), 2.0 ** -8
+        if epi == "slab16":
+            ws = torch.full((splits, M, N), 7.0, dtype=torch.float16, device=gpu)
+            ops._native_call("dli_gemm", x.data_ptr(), K, w.data_ptr(), K, None, N, M, N, K, G.EPI[epi], tile, splits,
+                             None, ws.data_ptr(), None, 1, ops._st())
+            got, tol = ws.double().sum(0) * 16, 2.0 ** -10
+        else:
+            if epi == "silu_mul":
+                gate, up = want[:, :N // 2], want[:, N // 2:]
+                want, w = torch.nn.functional.silu(gate) * up, interleave_gate_up(w[:N // 2], w[N // 2:]).contiguous()
+            elif bias is not None:
+                want = torch.nn.functional.gelu(want + bias.double(), approximate="tanh")
+            got = ops._gemm_native(x, w, epi, bias=bias, plan=plan).double()
+            tol = 1e-5 if epi == "f32" else tol
+        err = float((got - want).norm() / want.norm())
+        assert err < tol, (N, K, epi, splits, err)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", (61, 63, 66))
+def test_grouped_tiles_match_float64(gpu, tile):
+    """Experts of no, one, a full tile's and more rows, gathered and in place."""
+    bm, _ = G.TILES[tile]
+    counts, K, N = [3, 0, bm, 1, bm + 5], 2 * G.STREAM_K[tile], 160
+    off = [sum(counts[:i]) for i in range(len(counts) + 1)]
+    g = torch.Generator(device=gpu).manual_seed(tile)
+    x = torch.randn(off[-1], K, device=gpu, generator=g).bfloat16()
+    w = (torch.randn(len(counts), N, K, device=gpu, generator=g) * K ** -0.5).bfloat16()
+    offs = torch.tensor(off, dtype=torch.int32, device=gpu)
+    want = torch.cat([x[a:b].double() @ w[e].double().t() for e, (a, b) in enumerate(zip(off, off[1:]))])
+    got = ops._gemm_native(x, w, "none", plan=G.GemmPlan("dli", tile, 1), groups=len(counts), group_off=offs,
+                           rows_per_group=off[-1]).double()
+    assert float((got - want).norm() / want.norm()) < 2.0 ** -8
+    rows = torch.randperm(off[-1], device=gpu, generator=g).to(torch.int32)
+    out = torch.empty(off[-1], N // 2, dtype=torch.bfloat16, device=gpu)
+    ops._native_call("dli_gemm_grouped_gather", x.data_ptr(), K, w.data_ptr(), K, out.data_ptr(), N // 2, off[-1], N, K,
+                     tile, rows.data_ptr(), offs.data_ptr(), len(counts), ops._st())
+    want = torch.cat([x[rows[a:b].long()].double() @ w[e].double().t() for e, (a, b) in enumerate(zip(off, off[1:]))])
+    want = want.view(off[-1], N // 32, 2, 16)
+    want = (torch.nn.functional.silu(want[:, :, 0]) * want[:, :, 1]).reshape(off[-1], N // 2)
+    assert float((out.double() - want).norm() / want.norm()) < 2.0 ** -8

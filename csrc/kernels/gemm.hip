@@ -22,7 +22,7 @@
 // gate/up weight (output width N/2), 3 bias + tanh-GELU, 4 bias.
 //
 // Files: gemm_common.h (shared epilogue / split-K pieces), gemm_tiles.hip (ids 0-21, 23-25),
-// gemm_stream.hip (60-68: few rows, weights streamed), gemm8p.hip (22, 26-28), gemm4w.h +
+// gemm_stream.hip (60-72: few rows, weights streamed), gemm8p.hip (22, 26-28), gemm4w.h +
 // gemm4w.hip (34, 41, 45), gemm4wp.hip (55: persistent 45), gemv.hip (29-33 and the fused batch-1
 // combine). The losing 4-wave A/B variants of round 4 are documented, not built
 // (profiles/r4/gemm4w/).
@@ -54,7 +54,7 @@ extern "C" int dli_gemm_set_slab_store_family(int family, int mode) {
 // 20/21 = 128x64 with 2/3 stages; 22 = 256x256 8-phase ping-pong; 23/24 = 128x192 (3/2
 // stages), 25 = 256x192, 8 waves; 26 = 256x224 ping-pong; 29-33 = the M <= 4 weight
 // stream (16 / 32 rows per workgroup, dispatch_gemv); 55 = tile 45 persistent (one workgroup
-// per CU walks its tiles, no split-K / grouped mode); 60-68 = weight-streaming tiles
+// per CU walks its tiles, no split-K / grouped mode); 60-72 = weight-streaming tiles
 // (gemm_stream.h). ws: fp32 [splits, M, N] when splits>1.
 // group_off (nullable): int[groups+1] row offsets; M is then the max rows of any group.
 // Grouped SiLU*up GEMM whose permuted row p reads activation row arow[p] (the MoE gate/up
@@ -65,7 +65,7 @@ extern "C" int dli_gemm_grouped_gather(const void* A, int lda, const void* W, in
                                        const int* arow, const int* group_off, int groups,
                                        hipStream_t st) {
   if (M <= 0 || N <= 0) return 0;
-  const bool stream = tile_cfg >= 60 && tile_cfg <= 68;
+  const bool stream = tile_cfg >= 60 && tile_cfg <= 72;
   const bool generic = (tile_cfg >= 0 && tile_cfg <= 21) || (tile_cfg >= 23 && tile_cfg <= 25);
   if (!(generic || stream) || arow == nullptr || group_off == nullptr || groups < 1 || K % BK ||
       lda % 8 || ldw % 8 || N % 32)

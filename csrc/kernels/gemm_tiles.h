@@ -19,19 +19,31 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_bf16_kernel(
   extern __shared__ __attribute__((aligned(16))) char smem[];
 
   // ---- tile coordinates
+  // STREAM: x = column tile + K split, y = group, z = row tile. Row tiles past an expert's rows, of
+  // which a launch for the worst case has several times as many as it fills, come last: one that
+  // only reads its offsets and leaves holds a workgroup's LDS meanwhile
+  const int grp = STREAM ? blockIdx.y : blockIdx.z;
   int row0 = 0, Mg = M;
   const u16* Wg = W;
   if (group_off != nullptr) {
-    row0 = group_off[blockIdx.z];
-    Mg = group_off[blockIdx.z + 1] - row0;
-    Wg = W + (long)blockIdx.z * N * ldw;
+    row0 = group_off[grp];
+    Mg = group_off[grp + 1] - row0;
+    Wg = W + (long)grp * N * ldw;
   }
   const int tiles_m = (M + BM - 1) / BM;           // M = max rows per group in grouped mode
   const int tiles_n = (N + BN - 1) / BN;
   const int nwg = tiles_m * tiles_n;
-  int tile, ks;
-  split_tile(nwg, group_off != nullptr, tile, ks);
-  const int tn = tile / tiles_m, tm = tile % tiles_m;
+  int tile, ks, tn, tm;
+  if (STREAM) {
+    tile = blockIdx.x;
+    ks = tile / tiles_n;
+    tn = tile - ks * tiles_n;
+    tm = blockIdx.z;
+  } else {
+    split_tile(nwg, group_off != nullptr, tile, ks);
+    tn = tile / tiles_m;
+    tm = tile % tiles_m;
+  }
   const int m0 = tm * BM, n0 = tn * BN;
   if (m0 >= Mg) return;                             // grouped: empty tile (block-uniform)
   const int kb = ks * k_split_len;
@@ -71,8 +83,8 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_bf16_kernel(
     const int gr = min(n0 + r, N - 1);
     w_src[i] = Wg + (long)gr * ldw + kb + c * 8;
   }
-  // STREAM: tile t starts at K-tile t mod nk and wraps around (see gemm_stream.h)
-  const int rot = STREAM && nk > 0 ? tile % nk : 0;
+  // STREAM: column tile t starts at K-tile t mod nk and wraps around (see gemm_stream.h)
+  const int rot = STREAM && nk > 0 ? (tn + grp) % nk : 0;
   constexpr int W_AUX = STREAM ? 2 : 0;            // nt: each weight line is read once
   auto stage = [&](int buf, int kt) {
     char* base = smem + buf * BUF;
@@ -173,7 +185,7 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_bf16_kernel(
 
   // ---- epilogue (transposed accumulators):
   // acc[i][j][r] = C[m0 + wm*TM + 16i + fr][n0 + wn*TN + 16j + 4fq + r]
-  const bool split = gridDim.y > 1;
+  const bool split = STREAM ? k_split_len < K : gridDim.y > 1;
   if (split) {
     float* slab = ws + (long)ks * M * N;
     const int sm = g_slab_store;
@@ -239,7 +251,8 @@ static int launch_cfg(const void* A, int lda, const void* W, int ldw, void* C, i
                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     attr_done = true;
   }
-  dim3 grid(tiles, splits, groups);
+  const dim3 grid = STREAM ? dim3((N + BN - 1) / BN * splits, groups, (M + BM - 1) / BM)
+                           : dim3(tiles, splits, groups);
   gemm_bf16_kernel<BM, BN, EPI, NS, WM, WN, BKT, STREAM><<<grid, 64 * WM * WN, lds, st>>>(
       (const u16*)A, lda, (const u16*)W, ldw, C, ldc, M, N, K, ksl, (const u16*)bias,
       (float*)ws, group_off);

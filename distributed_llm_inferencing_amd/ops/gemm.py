@@ -56,11 +56,13 @@ TILES = {0: (64, 64), 1: (64, 128), 2: (128, 128), 3: (128, 256), 4: (256, 128),
          # K-tiles staged in the current tile's last two (gemm4wp.hip); no split-K / grouped
          55: (256, 256),
          # weight-streaming tiles for up to 128 rows (gemm_stream.h): weights nontemporal, K loops
-         # turned from tile to tile, 3 or 4 stages
-         60: (16, 128), 61: (32, 128), 62: (32, 64), 63: (64, 128), 64: (64, 64), 65: (64, 256),
-         66: (96, 128), 67: (128, 128), 68: (128, 256)}
+         # turned from tile to tile, 3 to 6 stages
+         60: (32, 32), 61: (32, 128), 62: (32, 64), 63: (64, 128), 64: (64, 64), 65: (64, 256),
+         66: (96, 128), 67: (128, 128), 68: (128, 256), 69: (64, 32), 70: (96, 64), 71: (128, 64),
+         72: (128, 32)}
 # their K-tiles
-STREAM_K = {60: 128, 61: 64, 62: 256, 63: 128, 64: 128, 65: 64, 66: 64, 67: 64, 68: 64}
+STREAM_K = {60: 256, 61: 64, 62: 256, 63: 64, 64: 64, 65: 64, 66: 64, 67: 64, 68: 64, 69: 256, 70: 64,
+            71: 64, 72: 128}
 STREAM_MAX_M = 128
 # the 4-wave plan raced against the 8-phase one in the prefill autotune
 PREFILL_4W_TILE = 45
@@ -88,7 +90,7 @@ GEMV_PRO_M1_ONLY = (32, 33)
 DEFER_NORM = os.environ.get("DLI_DEFER_NORM", "1") == "1"
 TILE_WAVES = {13: (2, 4), 14: (4, 2), 15: (2, 4), 16: (4, 2), 17: (2, 4),
               22: (2, 4), 23: (2, 4), 24: (2, 4), 25: (4, 2),
-              26: (4, 2), 28: (4, 2), 60: (1, 4), 66: (1, 4), 68: (2, 4)}
+              26: (4, 2), 28: (4, 2), 60: (2, 1), 66: (1, 4), 68: (2, 4), 69: (4, 1), 72: (4, 1)}
 
 
 def tile_ok(tile: int, epi: str) -> bool:
@@ -164,35 +166,49 @@ def workspace(device: torch.device, nbytes: int) -> torch.Tensor:
 LARGE_M = 1024
 
 
+# (rows up to, tiles of 32, 64 and 128 columns, the head's)
+STREAM_BANDS = ((32, 60, 62, 61, 62), (64, 69, 64, 63, 65), (96, 72, 70, 66, 68), (128, 72, 71, 67, 68))
+
+
 def _stream_plan(M: int, N: int, K: int, epi: str):
-    """Few rows: the weights' read is the product's time. One row of the weight-streaming tiles, narrow
-    ones split over K until about one workgroup a CU, wide ones where N alone gives that many; None for a K of
-    no whole K-tiles. fp32 outputs, us on these against the best other tile:
-    24 rows: 4096 x 4096 11.9 / 13.2, 4096 x 14336 24.3 / 27.2, 12288 x 4096 19.1 / 23.6, 32000 x 4096
-    41.5 / 56.3, 128256 x 4096 167 / 197; 64 rows 13.9 / 14.2, 28.5 / 29.1, 28.2 / 28.2, 45.3 / 59.5, 177 / 209; 2 and 4 rows of the last 157 and 155
-    against 164 on the plain weight stream. From
-    65 rows on the narrow weights stay on two rows of tile 5 or one of tile 7 (96 rows, 4096 x 4096
-    15.6, on tile 66 20.3), the wide ones do not (32000 x 4096 47.2 / 61.7)."""
-    wide = -(-N // 128) >= 3 * NUM_CUS // 4
-    if M <= 32:
-        # (the head: 62's long K-tiles, 24 rows 167 us against 174)
-        tile = 62 if K % 256 == 0 and (not wide or N >= 256 * NUM_CUS) else 61
-    elif M <= 64 and K % 128:
-        tile = 6 if wide else 5
-    elif M <= 64:
-        tile = (65 if N >= 256 * NUM_CUS else 63) if wide else 64
-    elif wide:
-        tile = 68 if N >= 256 * NUM_CUS else 66 if M <= 96 else 67
-    else:
-        tile = 7 if N >= 8192 or K > 8192 else 5
-    step = STREAM_K.get(tile, 64)
-    if K % step:
+    """Few rows: the weights' read is the product's time. One row of the weight-streaming tiles, as wide
+    as still gives three quarters of the CUs a workgroup (a narrower one reads the rows more often, a
+    second round costs as much as the first); where 32 columns are too wide too, 64 and K split until
+    about one workgroup a CU. fp32 outputs, us on these against the best other tile: 24 rows: 4096 x 4096
+    11.6 / 13.2, 8192 x 4096 13.9 / 17.6, 16384 x 4096 23.7 / 30.7, 4096 x 14336 24.2 / 27.4, 32000 x 4096 41.5 /
+    56.3, 128256 x 4096 167 / 197 (4 rows 155, on the plain weight stream 164); 64 rows: 14.1 / 13.8, 16.5 /
+    20.0, 26.5 / 35.2, 28.5 / 29.0, 45 / 60, 177 / 209; 96 rows: 16.3 / 16.2, 23.8 / 24.4, 30.1 / 38.3, 31.9 / 33.0,
+    47.5 / 63.5, 190 / 215. Above 96 rows the narrowest weights stay on two rows of tile 6 or one of tile 7
+    (128 rows, 4096 x 4096 17.6 / 19.8, 4096 x 14336 35 / 39), from 65 rows the small ones on tile 5 (96 rows,
+    2048 x 2048 11.2 / 14.0)."""
+    if K % 64:
         return None
+    _, narrow, mid, wide, head = next(b for b in STREAM_BANDS if M <= b[0])
+    fill = 3 * NUM_CUS // 4
+    split = False
+    if N >= 256 * NUM_CUS:
+        tile = head
+    elif -(-N // 128) >= fill:
+        tile = wide
+    elif -(-N // 64) >= fill:
+        tile = mid
+    elif -(-N // 32) >= fill and K % STREAM_K[narrow] == 0:
+        tile = narrow
+    else:
+        split = True
+        tile = mid
+        if M > 64 and N < 3072:
+            tile = 5
+        elif M > 96 and N < 6144:
+            tile = 7 if K > 8192 else 6
+    if K % STREAM_K.get(tile, 64):
+        tile = wide
+    step = STREAM_K.get(tile, 64)
     bm, bn = TILES[tile]
     tiles, splits = -(-M // bm) * -(-N // bn), 1
     most = 2 * NUM_CUS if tile == 5 else NUM_CUS
     # (K <= 1024: the second launch costs more than the shorter loop saves, 4096 x 1024 at 24 rows 6.1 / 7.8)
-    while (K > 1024 and tiles * splits * 2 <= most and K % (step * splits * 2) == 0
+    while (split and K > 1024 and tiles * splits * 2 <= most and K % (step * splits * 2) == 0
            and K // (splits * 2) >= 512 and splits < 8):
         splits *= 2
     if epi == "splitk" and splits == 1 and K % (2 * step) == 0 and K >= 1024:
@@ -248,7 +264,7 @@ def _heuristic(M: int, N: int, K: int, epi: str) -> GemmPlan:
         # residual-adding GEMV (full K): 4 rows a workgroup, 8 K-steps in flight per lane
         # (1024 workgroups on a 4096-wide projection)
         return GemmPlan("dli", 56, 1)
-    if 1 < M <= STREAM_MAX_M and (M > GEMV_MAX_M or epi not in ("splitk", "none")):
+    if 2 < M <= STREAM_MAX_M and (M > GEMV_MAX_M or epi not in ("splitk", "none")):
         p = _stream_plan(M, N, K, epi)
         if p is not None:
             return p
@@ -639,7 +655,8 @@ def candidate_plans(M: int, N: int, K: int, epi: str):
         if tile in STREAM_K:
             # one row of tiles; for 2 to 4 rows beside the weight stream's own kernels, but for the
             # products whose partial sums those keep in fp32
-            if (M > bm or bm >= 2 * max(M, 32) or M < 2
+            band = next((b for b in STREAM_BANDS if M <= b[0]), ())
+            if (tile not in band[1:] or M < 2
                     or (M <= GEMV_MAX_M and epi in ("splitk", "none"))):
                 continue
         elif M <= 64 and tile in (0, 1) and K % 128 == 0:

@@ -9,18 +9,17 @@ from distributed_llm_inferencing_amd.ops.reference import interleave_gate_up
 
 
 @pytest.mark.parametrize("M,N,K,epi,tile,splits", [
-    (5, 4096, 4096, "f32", 62, 4), (32, 4096, 4096, "f32", 62, 4), (32, 4096, 4160, "f32", 61, 1),
-    (33, 4096, 4096, "f32", 64, 4), (64, 4096, 4160, "f32", 5, 1), (65, 4096, 4096, "f32", 5, 4),
-    (128, 8192, 4096, "f32", 7, 4), (128, 4096, 14336, "f32", 7, 8), (129, 4096, 4096, "f32", 1, 8),
-    # wide: unsplit on 128 columns, the head on its own tiles
-    (24, 24480, 4096, "silu_mul", 61, 1), (24, 24448, 4096, "silu_mul", 62, 1),
-    (64, 28672, 4096, "silu_mul", 63, 1), (96, 28672, 4096, "silu_mul", 66, 1), (97, 28672, 4096, "silu_mul", 67, 1),
-    (24, 128256, 4096, "f32", 62, 1), (64, 128256, 4096, "f32", 65, 1), (65, 128256, 4096, "f32", 68, 1),
+    # 32, 64 and 128 columns, each where it fills three quarters of the chip; below, 64 and K split
+    (3, 6112, 4096, "f32", 62, 2), (32, 6144, 4096, "f32", 60, 1), (32, 6144, 4160, "f32", 61, 1), (24, 12224, 4096, "f32", 60, 1),
+    (24, 12288, 4096, "f32", 62, 1), (24, 24448, 4096, "silu_mul", 62, 1), (24, 24480, 4096, "silu_mul", 61, 1),
+    (33, 4096, 4096, "f32", 64, 4), (33, 8192, 4096, "f32", 69, 1), (64, 16384, 4160, "f32", 64, 1), (64, 28672, 4096, "silu_mul", 63, 1),
+    (65, 4096, 4096, "f32", 70, 4), (65, 3008, 4096, "f32", 5, 4), (96, 8192, 4096, "f32", 72, 1), (96, 28672, 4096, "silu_mul", 66, 1),
+    (97, 4096, 4096, "f32", 6, 4), (128, 4096, 14336, "f32", 7, 8), (97, 12288, 4096, "f32", 71, 1), (97, 28672, 4096, "silu_mul", 67, 1),
+    (24, 128256, 4096, "f32", 62, 1), (64, 128256, 4096, "f32", 65, 1), (65, 128256, 4096, "f32", 68, 1), (129, 4096, 4096, "f32", 1, 8),
     # short K is not split, but where a fused reduce follows
     (24, 4096, 1024, "f32", 62, 1), (24, 4096, 1024, "splitk", 62, 2), (24, 4096, 768, "splitk", 62, 1),
     # 2 to 4 rows: only what keeps no partial sums in 32 bits; one row stays on the plain weight stream
-    (4, 28672, 4096, "silu_mul", 61, 1), (4, 4096, 4096, "splitk", 30, 2), (2, 28672, 4096, "silu_mul", 61, 1),
-    (1, 28672, 4096, "silu_mul", 29, 1)])
+    (4, 28672, 4096, "silu_mul", 61, 1), (4, 4096, 4096, "splitk", 30, 2), (1, 28672, 4096, "silu_mul", 29, 1)])
 def test_fitted_plan(M, N, K, epi, tile, splits):
     assert G._heuristic(M, N, K, epi) == G.GemmPlan("dli", tile, splits)
 
@@ -71,7 +70,7 @@ def test_tiles_match_float64(gpu, tile, rows):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("tile", (61, 63, 66))
+@pytest.mark.parametrize("tile", (60, 61, 63, 66))
 def test_grouped_tiles_match_float64(gpu, tile):
     """Experts of no, one, a full tile's and more rows, gathered and in place."""
     bm, _ = G.TILES[tile]

@@ -174,7 +174,7 @@ __device__ __forceinline__ void decode_attn_loop(
       const u16* kp = k_cache + ((long)blk * hkv + kvh) * kv_head_stride + (long)off * HD;
 #pragma unroll
       for (int kk = 0; kk < KK; ++kk)
-        kreg[s][kk] = *reinterpret_cast<const uint4*>(kp + kk * 32 + grp * 8);
+        kreg[s][kk] = load16_once(kp + kk * 32 + grp * 8);
     }
     // V rows t0 .. t0+31 (row-major, 16-B chunks; piece lane + 64m = row r, chunk c)
     uint4 vreg[DB];
@@ -183,7 +183,7 @@ __device__ __forceinline__ void decode_attn_loop(
       const int piece = lane + 64 * m, r = piece / VCH, c = piece % VCH;
       const int tok = min(t0 + r, s_end - 1);                  // clamp: always-written rows
       const int blk = __shfl(bt_lane, tok / block_size - win, 64), off = tok % block_size;
-      vreg[m] = *reinterpret_cast<const uint4*>(
+      vreg[m] = load16_once(
           v_cache + ((long)blk * hkv + kvh) * kv_head_stride + (long)off * HD + c * 8);
     }
     // ---- S^T = K . Q^T for the two 16-token subtiles
@@ -297,6 +297,14 @@ __device__ __forceinline__ void decode_attn_core(
     }
   }}
 
+// l = -1 ends the list for the reduce; a single split is the output itself and its list empty
+__device__ __forceinline__ void decode_end_list(float* __restrict__ ws_ml, int b, int hq, int kvh,
+                                                int G, int num_splits, int split, int last, int lane) {
+  const int end = last == 0 ? 0 : split + 1;
+  if (split == last && end < num_splits && lane < G)
+    ws_ml[(((long)b * hq + kvh * G + lane) * num_splits + end) * 2 + 1] = -1.f;
+}
+
 // MINW = 4 waves per SIMD: <= 128 VGPRs, so every item of a 512-sequence batch (4096 waves)
 // is resident at once (measured 7 % faster than the 166-VGPR / 2-waves build at ctx 66)
 template <int HD, int MINW>
@@ -313,7 +321,7 @@ __global__ void __launch_bounds__(256, MINW) decode_attn_kernel(
   const int lane = threadIdx.x & 63;
   // one WAVE per work item (sequence, kv head, KV split): no LDS, no barriers, so every
   // resident wave of the chip streams a different (seq, head) pair concurrently
-  const int item = blockIdx.x * DEC_WAVES + (threadIdx.x >> 6);
+  const int item = blockIdx.x * DEC_WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int kvh = item % hkv;
   DecSplit sp{item / hkv, 0, split_tokens, 0};
   if (num_splits > 1) sp = decode_split(context_lens, B, hkv, num_splits, item / hkv, lane);
@@ -341,10 +349,7 @@ __global__ void __launch_bounds__(256, MINW) decode_attn_kernel(
   decode_attn_core<HD>(qf, vt, lane, b, kvh, split, G, ctx, s_begin, s_end, out, k_cache,
                        v_cache, block_tables, max_blocks, hq, hkv, block_size, scale_log2,
                        sp.last == 0 ? 1 : num_splits, ws_o, ws_ml);
-  // l = -1 ends the list for the reduce; a single split is the output itself and its list empty
-  const int end = sp.last == 0 ? 0 : split + 1;
-  if (num_splits > 1 && split == sp.last && end < num_splits && lane < G)
-    ws_ml[(((long)b * hq + kvh * G + lane) * num_splits + end) * 2 + 1] = -1.f;
+  if (num_splits > 1) decode_end_list(ws_ml, b, hq, kvh, G, num_splits, split, sp.last, lane);
 }
 
 // One (sequence, kv head) item per workgroup of WPI waves: wave wv walks the wv-th of WPI
@@ -436,54 +441,28 @@ __global__ void __launch_bounds__(256) decode_attn_wg_kernel(
                             block_size, scale_log2);
 }
 
-// Fused variant for the decode graph (one KV split per item): the QKV GEMM's split-K fp32
-// slabs go straight into the attention wave instead of through dli_splitk_rope_cache.
-// Prologue of item (sequence b, kv head h): lane l sums the slabs of this token's k and v
-// for dims l and l + 64 of head h, rounds to bf16, rotates k (RoPE) and writes both into
-// the paged cache at slot_mapping[b]; then each lane builds its Q^T fragments (head col of
-// the GQA group, dims 32kk + 8grp .. +7 and their RoPE partners 64 apart, which the same
-// lane holds) from the slabs. Numerics equal the unfused kernels: sum -> bf16 -> rotate ->
-// bf16. The q rows never go to memory, and one kernel per layer and its slab pass are gone.
-//
-// WPI = 1: one wave per (sequence, kv head) item, 4 items per workgroup (large batches).
-// WPI = DEC_WAVES: one workgroup per item for small batches, where 4 items per workgroup
-// leave most of the chip idle and each wave walks the whole context serially (one HBM round
-// trip per 32-token tile): wave 0 writes the new k/v row, every wave builds the Q fragments,
-// wave w takes the w-th quarter of the context's tiles, and the four partial (m, l, O) merge
-// through LDS (the V-tile rows are reused for the O partials).
-template <int SPL, int WPI, bool S16 = false>
-__global__ void __launch_bounds__(256, 4) decode_attn_fused_kernel(
-    u16* __restrict__ out, const void* __restrict__ src, int N,
-    const int* __restrict__ positions, const int* __restrict__ slot_mapping,
-    const float* __restrict__ cos_sin, u16* __restrict__ k_cache, u16* __restrict__ v_cache,
-    const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ context_lens,
-    int B, int hq, int hkv, int block_size, float scale_log2) {
-  constexpr int HD = 128, HALF = 64, KK = HD / 32, VROW = HD + 16, DB = HD / 16;
-  // SPL > 0: src = the QKV GEMM's fp32 split-K slabs [SPL, B, N]; SPL == 0: the bf16 QKV rows
-  // [B, N] of an unsplit GEMM (the same prologue minus the slab sum)
-  // S16: the slabs are fp16 x 1/16 (EPI_SLAB16), read as 16-bit words
+// Fused variants for the decode graph: the QKV GEMM's split-K slabs go straight into the attention
+// wave instead of through dli_splitk_rope_cache. The item that holds the new token (sequence b, kv
+// head h): lane l sums the slabs of this token's k and v for dims l and l + 64 of head h, rounds to
+// bf16, rotates k (RoPE) and writes both into the paged cache at slot_mapping[b]. Every item builds
+// its Q^T fragments (head col of the GQA group, dims 32kk + 8grp .. +7 and their RoPE partners 64
+// apart, which the same lane holds) from the slabs. Numerics equal the unfused kernels: sum -> bf16
+// -> rotate -> bf16. The q rows never go to memory, and one kernel per layer and its slab pass are
+// gone.
+// SPL > 0: src = the QKV GEMM's fp32 split-K slabs [SPL, B, N]; SPL == 0: the bf16 QKV rows [B, N] of
+// an unsplit GEMM (the same prologue minus the slab sum). S16: the slabs are fp16 x 1/16 (EPI_SLAB16),
+// read as 16-bit words.
+template <int SPL, bool S16>
+__device__ __forceinline__ void fused_query(bf16x8 (&qf)[4], const void* __restrict__ src,
+                                            long rowoff, long splitstride,
+                                            const float* __restrict__ cs, int kvh, int G, int lane) {
+  constexpr int HD = 128, HALF = 64, KK = HD / 32;
   const float* ws = static_cast<const float*>(src);
   const u16* qkv = static_cast<const u16*>(src);
   const u16* ws16 = static_cast<const u16*>(src);
-  static_assert(WPI == 1 || WPI == DEC_WAVES, "one item per wave or per workgroup");
-  __shared__ __attribute__((aligned(16))) u16 vtile_all[DEC_WAVES][DEC_TILE * VROW];
-  __shared__ float ml_all[WPI > 1 ? WPI : 1][16][2];
-  const int wv = threadIdx.x >> 6;
-  u16* vt = vtile_all[wv];
-  const int lane = threadIdx.x & 63;
-  const int item = WPI > 1 ? (int)blockIdx.x : (int)blockIdx.x * DEC_WAVES + wv;
-  if (item >= B * hkv) return;                                 // wave-uniform exit (WPI 1)
-  const int kvh = item % hkv, b = item / hkv;
   const int col = lane & 15, grp = lane >> 4;
-  const int G = hq / hkv;
-  const int ctx = context_lens[b];
-  const float* cs = cos_sin + (long)positions[b] * HD;
-  const long rowoff = (long)b * N;
-  const long splitstride = (long)B * N;
-  // ---- Q^T fragments (first: their slab loads do not wait on the cache write below): head
-  // col of the group, dims 32kk + 8grp .. +7 (kk < 2: first half, its RoPE partner is
+  // head col of the group, dims 32kk + 8grp .. +7 (kk < 2: first half, its RoPE partner is
   // fragment kk + 2 of the same lane)
-  bf16x8 qf[KK];
   if (col < G) {
     const float* qp = ws + rowoff + (long)(kvh * G + col) * HD;
 #pragma unroll
@@ -537,50 +516,96 @@ __global__ void __launch_bounds__(256, 4) decode_attn_fused_kernel(
       qf[kk] = *reinterpret_cast<bf16x8*>(&z);
     }
   }
+}
+
+// this token's k (rotated) and v -> paged cache (lane: dims lane, lane + 64)
+template <int SPL, bool S16>
+__device__ __forceinline__ void fused_cache_row(const void* __restrict__ src, long rowoff,
+                                                long splitstride, const float* __restrict__ cs,
+                                                int slot, int kvh, int hq, int hkv, int block_size,
+                                                u16* __restrict__ k_cache, u16* __restrict__ v_cache,
+                                                int lane) {
+  constexpr int HD = 128, HALF = 64;
+  const float* ws = static_cast<const float*>(src);
+  const u16* qkv = static_cast<const u16*>(src);
+  const u16* ws16 = static_cast<const u16*>(src);
+  const float* kp = ws + rowoff + (long)(hq + kvh) * HD;
+  const float* vp = ws + rowoff + (long)(hq + hkv + kvh) * HD;
+  float k1 = 0.f, k2 = 0.f, v1 = 0.f, v2 = 0.f;
+  if constexpr (S16) {
+    const u16* kh = ws16 + rowoff + (long)(hq + kvh) * HD;
+    const u16* vh = ws16 + rowoff + (long)(hq + hkv + kvh) * HD;
+#pragma unroll
+    for (int s = 0; s < SPL; ++s) {
+      k1 += h2f(kh[s * splitstride + lane]) * SLAB16_UNSCALE;
+      k2 += h2f(kh[s * splitstride + HALF + lane]) * SLAB16_UNSCALE;
+      v1 += h2f(vh[s * splitstride + lane]) * SLAB16_UNSCALE;
+      v2 += h2f(vh[s * splitstride + HALF + lane]) * SLAB16_UNSCALE;
+    }
+  } else if constexpr (SPL > 0) {
+#pragma unroll
+    for (int s = 0; s < SPL; ++s) {
+      k1 += kp[s * splitstride + lane];
+      k2 += kp[s * splitstride + HALF + lane];
+      v1 += vp[s * splitstride + lane];
+      v2 += vp[s * splitstride + HALF + lane];
+    }
+  } else {
+    const u16* kr = qkv + rowoff + (long)(hq + kvh) * HD;
+    const u16* vr = qkv + rowoff + (long)(hq + hkv + kvh) * HD;
+    k1 = bf2f(kr[lane]); k2 = bf2f(kr[HALF + lane]);
+    v1 = bf2f(vr[lane]); v2 = bf2f(vr[HALF + lane]);
+  }
+  k1 = bf2f(f2bf(k1)); k2 = bf2f(f2bf(k2));
+  const float co = cs[lane], si = cs[HALF + lane];
+  const int blk = slot / block_size, off = slot - blk * block_size;
+  const long dst = (((long)blk * hkv + kvh) * block_size + off) * HD;
+  k_cache[dst + lane] = f2bf(k1 * co - k2 * si);
+  k_cache[dst + HALF + lane] = f2bf(k2 * co + k1 * si);
+  v_cache[dst + lane] = f2bf(v1);
+  v_cache[dst + HALF + lane] = f2bf(v2);
+}
+
+// One KV split per item. WPI = 1: one wave per (sequence, kv head) item, 4 items per workgroup
+// (large batches). WPI = DEC_WAVES: one workgroup per item for small batches, where 4 items per
+// workgroup leave most of the chip idle and each wave walks the whole context serially (one HBM
+// round trip per 32-token tile): wave 0 writes the new k/v row, every wave builds the Q fragments,
+// wave w takes the w-th quarter of the context's tiles, and the four partial (m, l, O) merge
+// through LDS (the V-tile rows are reused for the O partials).
+template <int SPL, int WPI, bool S16 = false>
+__global__ void __launch_bounds__(256, 4) decode_attn_fused_kernel(
+    u16* __restrict__ out, const void* __restrict__ src, int N,
+    const int* __restrict__ positions, const int* __restrict__ slot_mapping,
+    const float* __restrict__ cos_sin, u16* __restrict__ k_cache, u16* __restrict__ v_cache,
+    const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ context_lens,
+    int B, int hq, int hkv, int block_size, float scale_log2) {
+  constexpr int HD = 128, KK = HD / 32, VROW = HD + 16;
+  static_assert(WPI == 1 || WPI == DEC_WAVES, "one item per wave or per workgroup");
+  __shared__ __attribute__((aligned(16))) u16 vtile_all[DEC_WAVES][DEC_TILE * VROW];
+  __shared__ float ml_all[WPI > 1 ? WPI : 1][16][2];
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  u16* vt = vtile_all[wv];
+  const int lane = threadIdx.x & 63;
+  const int item = WPI > 1 ? (int)blockIdx.x : (int)blockIdx.x * DEC_WAVES + wv;
+  if (item >= B * hkv) return;                                 // wave-uniform exit (WPI 1)
+  const int kvh = item % hkv, b = item / hkv;
+  const int G = hq / hkv;
+  const int ctx = context_lens[b];
+  const float* cs = cos_sin + (long)positions[b] * HD;
+  const long rowoff = (long)b * N;
+  const long splitstride = (long)B * N;
+  // first the query: its slab loads do not wait on the cache write below
+  bf16x8 qf[KK];
+  fused_query<SPL, S16>(qf, src, rowoff, splitstride, cs, kvh, G, lane);
   // the block-table window too: every load the tile loop's first tile waits on except the
   // new cache row is issued before the fence below
   int s_begin = 0, s_end = ctx;
   if constexpr (WPI > 1) decode_wg_range<WPI>(ctx, wv, s_begin, s_end);
   const int bt0 = decode_bt_window(block_tables, max_blocks, b, s_begin, s_end, block_size, lane);
-  // ---- this token's k (rotated) and v -> paged cache (lane: dims lane, lane + 64)
   const int slot = slot_mapping[b];
-  if (slot >= 0 && (WPI == 1 || wv == 0)) {
-    const float* kp = ws + rowoff + (long)(hq + kvh) * HD;
-    const float* vp = ws + rowoff + (long)(hq + hkv + kvh) * HD;
-    float k1 = 0.f, k2 = 0.f, v1 = 0.f, v2 = 0.f;
-    if constexpr (S16) {
-      const u16* kh = ws16 + rowoff + (long)(hq + kvh) * HD;
-      const u16* vh = ws16 + rowoff + (long)(hq + hkv + kvh) * HD;
-#pragma unroll
-      for (int s = 0; s < SPL; ++s) {
-        k1 += h2f(kh[s * splitstride + lane]) * SLAB16_UNSCALE;
-        k2 += h2f(kh[s * splitstride + HALF + lane]) * SLAB16_UNSCALE;
-        v1 += h2f(vh[s * splitstride + lane]) * SLAB16_UNSCALE;
-        v2 += h2f(vh[s * splitstride + HALF + lane]) * SLAB16_UNSCALE;
-      }
-    } else if constexpr (SPL > 0) {
-#pragma unroll
-      for (int s = 0; s < SPL; ++s) {
-        k1 += kp[s * splitstride + lane];
-        k2 += kp[s * splitstride + HALF + lane];
-        v1 += vp[s * splitstride + lane];
-        v2 += vp[s * splitstride + HALF + lane];
-      }
-    } else {
-      const u16* kr = qkv + rowoff + (long)(hq + kvh) * HD;
-      const u16* vr = qkv + rowoff + (long)(hq + hkv + kvh) * HD;
-      k1 = bf2f(kr[lane]); k2 = bf2f(kr[HALF + lane]);
-      v1 = bf2f(vr[lane]); v2 = bf2f(vr[HALF + lane]);
-    }
-    k1 = bf2f(f2bf(k1)); k2 = bf2f(f2bf(k2));
-    const float co = cs[lane], si = cs[HALF + lane];
-    const int blk = slot / block_size, off = slot - blk * block_size;
-    const long dst = (((long)blk * hkv + kvh) * block_size + off) * HD;
-    k_cache[dst + lane] = f2bf(k1 * co - k2 * si);
-    k_cache[dst + HALF + lane] = f2bf(k2 * co + k1 * si);
-    v_cache[dst + lane] = f2bf(v1);
-    v_cache[dst + HALF + lane] = f2bf(v2);
-  }
+  if (slot >= 0 && (WPI == 1 || wv == 0))
+    fused_cache_row<SPL, S16>(src, rowoff, splitstride, cs, slot, kvh, hq, hkv, block_size, k_cache,
+                              v_cache, lane);
   // the tile loop below reads this row back (other lanes of this wave): order the stores
   // before those loads
   __threadfence_block();
@@ -594,6 +619,47 @@ __global__ void __launch_bounds__(256, 4) decode_attn_fused_kernel(
                         k_cache, v_cache, block_tables, max_blocks, hq, hkv, block_size,
                         scale_log2);
   }
+}
+
+// Several KV splits per sequence, dealt as in decode_attn_kernel: the split that holds the new token
+// writes its cache row, the others do not read it. Against a kernel for the rotation and the cache write
+// and one for the attention: 1 context of 75 tokens 5.1 + 9.2 -> 11.0 us, 24 of 500 to 8000 5.5 + 55.3 ->
+// 54.1 (the query's sums run beside the first block-table and cache requests).
+template <int SPL, bool S16>
+__global__ void __launch_bounds__(256, 4) decode_attn_fused_split_kernel(
+    u16* __restrict__ out, const void* __restrict__ src, int N,
+    const int* __restrict__ positions, const int* __restrict__ slot_mapping,
+    const float* __restrict__ cos_sin, u16* __restrict__ k_cache, u16* __restrict__ v_cache,
+    const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ context_lens,
+    int B, int hq, int hkv, int block_size, float scale_log2, int num_splits,
+    float* __restrict__ ws_o, float* __restrict__ ws_ml) {
+  constexpr int HD = 128, KK = HD / 32, VROW = HD + 16;
+  __shared__ __attribute__((aligned(16))) u16 vtile_all[DEC_WAVES][DEC_TILE * VROW];
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int item = blockIdx.x * DEC_WAVES + wv;
+  const int kvh = item % hkv;
+  const DecSplit sp = decode_split(context_lens, B, hkv, num_splits, item / hkv, lane);
+  if (sp.b < 0) return;                                        // wave-uniform exit
+  const int b = sp.b, split = sp.split, G = hq / hkv;
+  const int ctx = context_lens[b];
+  const int s_begin = split * sp.split_tokens;
+  const int s_end = min(ctx, s_begin + sp.split_tokens);
+  const float* cs = cos_sin + (long)positions[b] * HD;
+  const long rowoff = (long)b * N;
+  const long splitstride = (long)B * N;
+  const int bt0 = decode_bt_window(block_tables, max_blocks, b, s_begin, s_end, block_size, lane);
+  bf16x8 qf[KK];
+  fused_query<SPL, S16>(qf, src, rowoff, splitstride, cs, kvh, G, lane);
+  const int slot = slot_mapping[b];
+  if (slot >= 0 && split == max(ctx - 1, 0) / sp.split_tokens) {
+    fused_cache_row<SPL, S16>(src, rowoff, splitstride, cs, slot, kvh, hq, hkv, block_size, k_cache,
+                              v_cache, lane);
+    __threadfence_block();                 // read back by other lanes of this wave
+  }
+  decode_attn_core<HD>(qf, vtile_all[wv], lane, b, kvh, split, G, ctx, s_begin, s_end, out, k_cache,
+                       v_cache, block_tables, max_blocks, hq, hkv, block_size, scale_log2,
+                       sp.last == 0 ? 1 : num_splits, ws_o, ws_ml, bt0);
+  decode_end_list(ws_ml, b, hq, kvh, G, num_splits, split, sp.last, lane);
 }
 
 // Software-pipelined variant: a wave walks a list of work units (item = (sequence, kv head,
@@ -986,8 +1052,8 @@ extern "C" int dli_decode_attention(void* out, const void* q, int q_stride, cons
   DLI_RETURN_LAUNCH();
 }
 
-// Fused split-K QKV reduce + RoPE + KV-cache write + decode attention (one KV split, head
-// dim 128, RoPE models): ws = the QKV GEMM's fp32 slabs [splits, B, (hq + 2 hkv) * 128], or
+// Fused split-K QKV reduce + RoPE + KV-cache write + decode attention (head dim 128, RoPE models;
+// workspace as dli_decode_attention's where num_splits > 1, apart from ws): ws = the QKV GEMM's fp32 slabs [splits, B, (hq + 2 hkv) * 128], or
 // with splits == 0 the bf16 QKV rows [B, (hq + 2 hkv) * 128] of an unsplit GEMM.
 // fmt: 0 = fp32 slabs (or the bf16 rows when splits == 0), 1 = fp16 x 1/16 slabs (EPI_SLAB16)
 extern "C" int dli_decode_attention_fused(void* out, const void* ws, int splits,
@@ -996,15 +1062,32 @@ extern "C" int dli_decode_attention_fused(void* out, const void* ws, int splits,
                                           const int* block_tables, int max_blocks,
                                           const int* context_lens, int B, int hq, int hkv,
                                           int hd, int block_size, float scale, int fmt,
-                                          hipStream_t st) {
+                                          int num_splits, void* workspace, hipStream_t st) {
   if (B <= 0) return 0;
   if (hd != 128 || hq % hkv || hq / hkv > 16 || block_size % 16 ||
       (splits != 0 && splits != 2 && splits != 4) || fmt < 0 || fmt > 1 ||
-      (fmt == 1 && splits == 0))
+      (fmt == 1 && splits == 0) || num_splits < 1 || (num_splits > 1 && workspace == nullptr))
     return (int)hipErrorInvalidValue;
   const int N = (hq + 2 * hkv) * hd;
   const float scale_log2 = scale * 1.4426950408889634f;
   const long items = (long)B * hkv;
+  if (num_splits > 1) {
+    float* ws_o = (float*)workspace;
+    float* ws_ml = ws_o + (long)B * hq * num_splits * hd;
+    const long listed = decode_split_items(B * hkv, num_splits);
+    const dim3 gs((int)((listed + DEC_WAVES - 1) / DEC_WAVES));
+#define DLI_DAS(S, F) decode_attn_fused_split_kernel<S, F><<<gs, 64 * DEC_WAVES, 0, st>>>(     \
+      (u16*)out, ws, N, positions, slot_mapping, cos_sin, (u16*)k_cache, (u16*)v_cache,      \
+      block_tables, max_blocks, context_lens, B, hq, hkv, block_size, scale_log2, num_splits,  \
+      ws_o, ws_ml)
+    if (splits == 0) DLI_DAS(0, false);
+    else if (splits == 2) { if (fmt) DLI_DAS(2, true); else DLI_DAS(2, false); }
+    else { if (fmt) DLI_DAS(4, true); else DLI_DAS(4, false); }
+#undef DLI_DAS
+    decode_reduce_kernel<128><<<(int)(((long)B * hq + 3) / 4), 256, 0, st>>>(
+        (u16*)out, ws_o, ws_ml, B, hq, num_splits);
+    DLI_RETURN_LAUNCH();
+  }
   const bool per_wg = wg_form(items);
   dim3 grid((int)(per_wg ? items : (items + DEC_WAVES - 1) / DEC_WAVES));
 #define DLI_DAF(S, W, F) decode_attn_fused_kernel<S, W, F><<<grid, 64 * DEC_WAVES, 0, st>>>(   \

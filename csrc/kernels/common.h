@@ -55,6 +55,13 @@ __device__ __forceinline__ void store8(u16* p, const float* f) {
   *reinterpret_cast<uint4*>(p) = v;
 }
 
+// 16 bytes that this launch reads once: they leave what is read again in the L2
+__device__ __forceinline__ uint4 load16_once(const u16* p) {
+  typedef unsigned v4 __attribute__((ext_vector_type(4)));
+  const v4 v = __builtin_nontemporal_load(reinterpret_cast<const v4*>(p));
+  return uint4{v[0], v[1], v[2], v[3]};
+}
+
 // four consecutive elements (8-byte aligned bf16, 16-byte aligned fp32)
 __device__ __forceinline__ void st4(u16* p, const f32x4 v) {
   uint2 pk;

@@ -522,8 +522,7 @@ __global__ void __launch_bounds__(256) swa_decode_kernel(SwaArgs a) {
       const long r = __shfl(row, 16 * u + fr, 64);
 #pragma unroll
       for (int kk = 0; kk < KK; ++kk) {
-        const uint4 v = *reinterpret_cast<const uint4*>(a.k + r * a.k_stride + kvh * DK + kk * 32 +
-                                                        fq * 8);
+        const uint4 v = load16_once(a.k + r * a.k_stride + kvh * DK + kk * 32 + fq * 8);
         kf[u][kk] = *reinterpret_cast<const bf16x8*>(&v);
       }
     }
@@ -533,7 +532,7 @@ __global__ void __launch_bounds__(256) swa_decode_kernel(SwaArgs a) {
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       const long r = __shfl(row, i * KPI + vk, 64);
-      vv[i] = *reinterpret_cast<const uint4*>(a.v + r * a.v_stride + kvh * DV + (lane % LPR) * 8);
+      vv[i] = load16_once(a.v + r * a.v_stride + kvh * DV + (lane % LPR) * 8);
     }
     f32x4 sa[2];
     float tmax = -INFINITY;

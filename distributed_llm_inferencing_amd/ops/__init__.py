@@ -388,8 +388,7 @@ def linear_rope_attention(x, w, positions, slot_mapping, cos_sin, k_cache, v_cac
     attention computed by ONE kernel per layer (``dli_decode_attention_fused``) instead of
     ``linear_rope_cache`` + ``decode_attention``. Returns the attention output [B, hq*hd], or
     None where the fused kernel does not apply (the caller then runs the two-kernel path):
-    split counts other than 2 / 4, KV-split attention (long contexts at small batch), the
-    pipelined long-context kernel, head dim != 128."""
+    split counts other than 2 / 4, the pipelined long-context kernel, head dim != 128."""
     xr = x.residual if isinstance(x, NormedRows) else x
     if hd != 128 or k_cache is None or not _use_native(xr):
         return None
@@ -397,17 +396,21 @@ def linear_rope_attention(x, w, positions, slot_mapping, cos_sin, k_cache, v_cac
     if p is not None and p.splits not in (2, 4):
         return None
     B, K = x.shape
-    if decode_num_splits(B, hkv, max_context) != 1:
-        return None
+    ns = decode_num_splits(B, hkv, max_context)
     mode = int(N.require_native().dli_decode_get_pipe())
-    if mode == 1 or (mode == 2 and -(-max_context // 32) * 32 >= 768):
+    if mode == 1 or (mode == 2 and ns == 1 and -(-max_context // 32) * 32 >= 768):
         return None                       # dli_decode_attention picks the pipelined kernel
     Nn = w.shape[0]
     fmt = 0
+    slabs = p.splits * B * Nn * 4 if p is not None else 0
+    # the QKV slabs, then the attention splits' partial results
+    scratch = B * hq * ns * (hd + 2) * 4 if ns > 1 else 0
+    ws = G.workspace(xr.device, slabs + scratch) if slabs + scratch else None
+    parts = ws.data_ptr() + slabs if scratch else None
     if p is None:                         # unsplit plan: the prologue reads the bf16 rows
         src, splits = linear(x, w), 0
     else:
-        src, splits = G.workspace(xr.device, p.splits * B * Nn * 4), p.splits
+        src, splits = ws, p.splits
         if not (isinstance(x, NormedRows)
                 and _gemv_prologue(x, w, "splitk", p, None, Nn, ws=src)):
             if isinstance(x, NormedRows):
@@ -417,7 +420,7 @@ def linear_rope_attention(x, w, positions, slot_mapping, cos_sin, k_cache, v_cac
     _native_call("dli_decode_attention_fused", _p(out), _p(src), splits, _p(positions),
                  _p(slot_mapping), _p(cos_sin), _p(k_cache), _p(v_cache), _p(block_tables),
                  block_tables.stride(0), _p(context_lens), B, hq, hkv, hd, k_cache.shape[2],
-                 scale, fmt, _st())
+                 scale, fmt, ns, parts, _st())
     return out
 
 

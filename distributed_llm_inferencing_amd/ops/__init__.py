@@ -216,15 +216,20 @@ def _gemm_native(x, w, epi: str, bias=None, out=None, plan: Optional[G.GemmPlan]
                  groups: int = 1, group_off=None, rows_per_group: Optional[int] = None):
     M, K = x.shape
     Nn = w.shape[-2]
-    if plan is None:
-        if group_off is None:
-            plan = G.plan(M, Nn, K, epi)
-        else:
-            plan = G.grouped_plan(M, Nn, K, epi, groups)
     out_n = Nn // 2 if epi in G.PAIR_EPIS else Nn
     if out is None:
         dt = torch.float32 if epi == "f32" else x.dtype
         out = torch.empty(M, out_n, dtype=dt, device=x.device)
+    if plan is None:
+        if group_off is None:
+            cut = G.row_cut(M, Nn, K)
+            if cut:
+                _gemm_native(x[:cut], w, epi, bias, out[:cut], G.plan(cut, Nn, K, epi))
+                _gemm_native(x[cut:], w, epi, bias, out[cut:], G.plan(M - cut, Nn, K, epi))
+                return out
+            plan = G.plan(M, Nn, K, epi)
+        else:
+            plan = G.grouped_plan(M, Nn, K, epi, groups)
     splits = plan.splits
     ws = None
     if splits > 1:

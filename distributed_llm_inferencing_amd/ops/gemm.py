@@ -422,6 +422,25 @@ def plan(M: int, N: int, K: int, epi: str) -> GemmPlan:
     return _plan_cache.get(key) or _heuristic(M, N, K, epi)
 
 
+@functools.lru_cache(maxsize=8192)
+def row_cut(M: int, N: int, K: int) -> int:
+    """Rows of a large product that run by themselves, in whole 256-row tiles, where the up to 128 rows
+    past them would begin a round of the chip that they cannot fill; those then run on a streaming tile,
+    bound by the weights' read. 0: all rows together. K = 4096, fp32 outputs, us together and cut: 4104 x
+    4096 172 and 120, 8256 x 4096 265 and 212, 8199 x 16384 852 and 796, 1312 x 12288 172 and 121;
+    8199 x 28672 (SiLU pairs) 1366 and 1332; K = 14336: 8199 x 4096 907 and 710. Not where as many rounds remain: 8199
+    x 6144 is 3.09 rounds, 355 and 307, but 4104 x 6144 1.59, 181 and 193. The last round's price is
+    0.73 of a full one even if nearly empty (fewer busy CUs clock higher): 0.017 us a K on one, the other
+    side the weights at 5.5 TB/s and a launch."""
+    rest = M % 256
+    if M <= 512 or not 0 < rest <= STREAM_MAX_M or K % 64:
+        return 0
+    rows, cols = M // 256, -(-N // 256)
+    rounds = -(-(rows + 1) * cols // NUM_CUS) - -(-rows * cols // NUM_CUS)
+    apart = (N * K * 2 / 5.5e6 + 8.0) * (1.0 if rest <= 64 else 1.25)
+    return M - rest if rows * cols >= NUM_CUS // 2 and rounds * 0.017 * K > apart else 0
+
+
 def set_plan(M: int, N: int, K: int, epi: str, p: GemmPlan) -> None:
     _plan_cache[(_bucket(M), N, K, epi)] = p
 

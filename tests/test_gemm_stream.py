@@ -92,3 +92,40 @@ def test_grouped_tiles_match_float64(gpu, tile):
     want = want.view(off[-1], N // 32, 2, 16)
     want = (torch.nn.functional.silu(want[:, :, 0]) * want[:, :, 1]).reshape(off[-1], N // 2)
     assert float((out.double() - want).norm() / want.norm()) < 2.0 ** -8
+
+
+@pytest.mark.parametrize("M,N,K,cut", [
+    (4104, 4096, 4096, 4096), (4224, 4096, 4096, 4096), (4225, 4096, 4096, 0), (4096, 4096, 4096, 0), (4353, 4096, 4096, 0),
+    (8199, 28672, 4096, 8192), (4104, 6144, 4096, 0), (8199, 6144, 4096, 8192), (1312, 12288, 4096, 1280),
+    (513, 65536, 4096, 0), (300, 32768, 4096, 0), (2049, 128256, 4096, 0), (4104, 4096, 512, 0), (4104, 4096, 4104, 0)])
+def test_rows_that_would_begin_a_round_run_apart(M, N, K, cut):
+    assert G.row_cut(M, N, K) == cut
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rest", (1, 3, 33, 128))
+@pytest.mark.parametrize("epi", ("f32", "none", "silu_mul", "bias_gelu", "gelu_mul"))
+def test_products_cut_by_rows(gpu, rest, epi):
+    M, N, K = 4096 + rest, 4096, 1024
+    kept = dict(G._plan_cache), set(G._tuned)
+    G.clear_plans()
+    assert G.row_cut(M, N, K) == 4096
+    g = torch.Generator(device=gpu).manual_seed(rest)
+    x = torch.randn(M, 2 * K, device=gpu, generator=g).bfloat16()[:, K:]      # (rows of a wider tensor)
+    w = (torch.randn(N, K, device=gpu, generator=g) * K ** -0.5).bfloat16()
+    bias = torch.randn(N, device=gpu, generator=g).bfloat16() if epi == "bias_gelu" else None
+    want = x.double() @ w.double().t()
+    if epi in G.PAIR_EPIS:
+        act = torch.nn.functional.silu if epi == "silu_mul" else lambda v: torch.nn.functional.gelu(v, approximate="tanh")
+        want, w = act(want[:, :N // 2]) * want[:, N // 2:], interleave_gate_up(w[:N // 2], w[N // 2:]).contiguous()
+    elif bias is not None:
+        want = torch.nn.functional.gelu(want + bias.double(), approximate="tanh")
+    try:
+        got = ops.linear(x, w, bias, epi=epi).double()
+    finally:
+        G.clear_plans()
+        G._plan_cache.update(kept[0])
+        G._tuned.update(kept[1])
+    tol = 1e-5 if epi == "f32" else 2.0 ** -8
+    for rows in (slice(0, 4096), slice(4096, M)):
+        assert float((got[rows] - want[rows]).norm() / want[rows].norm()) < tol

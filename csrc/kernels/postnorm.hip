@@ -86,11 +86,11 @@ __global__ void __launch_bounds__(256) embedding_bigram_kernel(
   stf(xs + gid, v);
 }
 
-// One workgroup per row: v = keep * x + y; mean and variance (of the deviations, two passes
+// One workgroup per row: v = keep * x + y, y the sum of nsplit slabs of a split-K product; mean and variance (of the deviations, two passes
 // over the row held in LDS); x = (v - mean) * rsqrt(var + eps) * w + b.
 template <typename S>
 __global__ void __launch_bounds__(256) postnorm_kernel(
-    float* __restrict__ x, const float* __restrict__ y, int ldy, float keep,
+    float* __restrict__ x, const float* __restrict__ y, int ldy, int nsplit, long ysplit, float keep,
     const S* __restrict__ w, const S* __restrict__ b, S* __restrict__ h, int dim, float eps,
     const long* __restrict__ rows_idx, bool vec4) {
   extern __shared__ __attribute__((aligned(16))) float row[];   // dim floats + 16 reduction slots
@@ -104,7 +104,12 @@ __global__ void __launch_bounds__(256) postnorm_kernel(
       f32x4 v = *reinterpret_cast<const f32x4*>(xr + c);
       if (rows_idx == nullptr) {
         v *= keep;
-        if (y != nullptr) v += *reinterpret_cast<const f32x4*>(y + (long)r * ldy + c);
+        if (y != nullptr) {
+          const float* yr = y + (long)r * ldy + c;
+          f32x4 sum = *reinterpret_cast<const f32x4*>(yr);
+          for (int k = 1; k < nsplit; ++k) sum += *reinterpret_cast<const f32x4*>(yr + k * ysplit);
+          v += sum;
+        }
       }
       *reinterpret_cast<f32x4*>(row + c) = v;
       s += (v[0] + v[1]) + (v[2] + v[3]);
@@ -128,7 +133,11 @@ __global__ void __launch_bounds__(256) postnorm_kernel(
     float v = xr[c];
     if (rows_idx == nullptr) {
       v *= keep;
-      if (y != nullptr) v += y[(long)r * ldy + c];
+      if (y != nullptr) {
+        float sum = y[(long)r * ldy + c];
+        for (int k = 1; k < nsplit; ++k) sum += y[k * ysplit + (long)r * ldy + c];
+        v += sum;
+      }
     }
     row[c] = v;
     s += v;
@@ -522,20 +531,20 @@ extern "C" int dli_embedding_bigram(float* x, void* xs, const int* ids, const in
   DLI_RETURN_LAUNCH();
 }
 
-extern "C" int dli_postnorm(float* x, const float* y, int ldy, float keep, const void* w,
-                            const void* b, void* h, int rows, int dim, float eps,
+extern "C" int dli_postnorm(float* x, const float* y, int ldy, int nsplit, long ysplit, float keep,
+                            const void* w, const void* b, void* h, int rows, int dim, float eps,
                             const long* rows_idx, int dt, hipStream_t st) {
   if (rows <= 0) return 0;
   const size_t sh = (size_t)(dim + 16) * 4;
-  if (dim < 1 || sh > 60000 || w == nullptr || b == nullptr || h == nullptr)
+  if (dim < 1 || sh > 60000 || w == nullptr || b == nullptr || h == nullptr || nsplit < 1)
     return (int)hipErrorInvalidValue;
-  const bool vec4 = dim % 4 == 0 && ldy % 4 == 0 &&
+  const bool vec4 = dim % 4 == 0 && ldy % 4 == 0 && ysplit % 4 == 0 &&
                     (((uintptr_t)x | (uintptr_t)y | (uintptr_t)w | (uintptr_t)b | (uintptr_t)h) & 15) == 0;
   DT_SWITCH(dt,
-            (postnorm_kernel<u16><<<rows, 256, sh, st>>>(x, y, ldy, keep, (const u16*)w,
+            (postnorm_kernel<u16><<<rows, 256, sh, st>>>(x, y, ldy, nsplit, ysplit, keep, (const u16*)w,
                                                          (const u16*)b, (u16*)h, dim, eps,
                                                          rows_idx, vec4)),
-            (postnorm_kernel<float><<<rows, 256, sh, st>>>(x, y, ldy, keep, (const float*)w,
+            (postnorm_kernel<float><<<rows, 256, sh, st>>>(x, y, ldy, nsplit, ysplit, keep, (const float*)w,
                                                            (const float*)b, (float*)h, dim, eps,
                                                            rows_idx, vec4)));
   DLI_RETURN_LAUNCH();

@@ -26,30 +26,31 @@ template <> __device__ __forceinline__ void stf<float>(float* p, float v) { *p =
 constexpr int MAXS = 8;          // streams
 
 // One workgroup per token (256 threads; 1024 for the few wide rows of a decode step, which
-// are bound by latency). VEC = 4: 16-byte accesses of the fp32 rows (dim % 4 == 0).
-template <typename S, int VEC>
+// are bound by latency). VEC = 4: 16-byte accesses of the fp32 rows (dim % 4 == 0). NS: the number of
+// streams where it is 2 to 4 (0: any). y may be nsplit partial sums, ysplit elements apart, of a
+// split-K product: the launch and the pass of its reduce are spared. The coefficients are the same
+// for the whole launch: read as scalars, beside the rows' requests and without a barrier before them.
+// Decode step, 64 rows of 3 x 4096: 7.5 us with a reduce launch of 5.4 before it -> 6.2. Prefill is bound
+// by memory: 8199 rows 173 us, 1.0 GB at 5.8 TB/s.
+template <typename S, int VEC, int NS>
 __global__ void __launch_bounds__(1024) hyper_mix_kernel(
-    float* __restrict__ xs, const float* __restrict__ y, int ldy, const float* __restrict__ prev,
-    const float* __restrict__ read, const S* __restrict__ w, void* __restrict__ h, int ns,
-    int dim, float eps, float w_offset) {
+    float* __restrict__ xs, const float* __restrict__ y, int ldy, int nsplit, long ysplit,
+    const float* __restrict__ prev, const float* __restrict__ read, const S* __restrict__ w,
+    void* __restrict__ h, int ns_any, int dim, float eps, float w_offset) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
+  constexpr int MS = NS ? NS : MAXS;
+  const int ns = NS ? NS : ns_any;
   float* urow = sm;                        // [dim]
   float* red = urow + dim;                 // [16]
-  float* cf = red + 16;                    // [ns*(ns+2)] prev, then [ns] read
   const int t = blockIdx.x;
-  const int nc = ns * (ns + 2);
   float* xr = xs + (long)t * ns * dim;
-  for (int i = threadIdx.x; i < nc + ns; i += blockDim.x)
-    cf[i] = i < nc ? (prev != nullptr ? prev[i] : 0.f) : (read != nullptr ? read[i - nc] : 0.f);
-  __syncthreads();
-  const float* wr = cf + ns;               // write weights
-  const float* mix = cf + 2 * ns;          // [from][to]
-  const float* rd = cf + nc;
+  const float* wr = prev + ns;             // write weights
+  const float* mix = prev + 2 * ns;        // [from][to]
   float ss = 0.f;
   for (int c = threadIdx.x * VEC; c < dim; c += blockDim.x * VEC) {
-    float x[MAXS][VEC];
+    float x[MS][VEC];
 #pragma unroll
-    for (int s = 0; s < MAXS; ++s) {
+    for (int s = 0; s < MS; ++s) {
       if (s < ns) {
         if (VEC == 4) {
           const f32x4 v = *reinterpret_cast<const f32x4*>(xr + (long)s * dim + c);
@@ -61,17 +62,25 @@ __global__ void __launch_bounds__(1024) hyper_mix_kernel(
       }
     }
     if (y != nullptr) {
-      float yv[VEC], nx[MAXS][VEC];
+      float yv[VEC], nx[MS][VEC];
+      const float* yr = y + (long)t * ldy + c;
+      if constexpr (VEC == 4) {
+        f32x4 v = *reinterpret_cast<const f32x4*>(yr);
+        for (int s = 1; s < nsplit; ++s) v += *reinterpret_cast<const f32x4*>(yr + s * ysplit);
 #pragma unroll
-      for (int u = 0; u < VEC; ++u) yv[u] = y[(long)t * ldy + c + u];
+        for (int u = 0; u < VEC; ++u) yv[u] = v[u];
+      } else {
+        yv[0] = yr[0];
+        for (int s = 1; s < nsplit; ++s) yv[0] += yr[s * ysplit];
+      }
 #pragma unroll
-      for (int r = 0; r < MAXS; ++r) {
+      for (int r = 0; r < MS; ++r) {
         if (r < ns) {
 #pragma unroll
           for (int u = 0; u < VEC; ++u) {
             float acc = 0.f;
 #pragma unroll
-            for (int s = 0; s < MAXS; ++s)
+            for (int s = 0; s < MS; ++s)
               if (s < ns) acc += mix[s * ns + r] * x[s][u];
             nx[r][u] = acc + wr[r] * yv[u];
           }
@@ -83,7 +92,7 @@ __global__ void __launch_bounds__(1024) hyper_mix_kernel(
         }
       }
 #pragma unroll
-      for (int r = 0; r < MAXS; ++r)
+      for (int r = 0; r < MS; ++r)
         if (r < ns) {
 #pragma unroll
           for (int u = 0; u < VEC; ++u) x[r][u] = nx[r][u];
@@ -94,8 +103,8 @@ __global__ void __launch_bounds__(1024) hyper_mix_kernel(
       for (int u = 0; u < VEC; ++u) {
         float acc = 0.f;
 #pragma unroll
-        for (int s = 0; s < MAXS; ++s)
-          if (s < ns) acc += rd[s] * x[s][u];
+        for (int s = 0; s < MS; ++s)
+          if (s < ns) acc += read[s] * x[s][u];
         if (w == nullptr) ((float*)h)[(long)t * dim + c + u] = acc;
         else urow[c + u] = acc;
         ss += acc * acc;
@@ -105,6 +114,15 @@ __global__ void __launch_bounds__(1024) hyper_mix_kernel(
   if (read == nullptr || w == nullptr) return;
   const float tot = block_sum(ss, red);
   const float rs = 1.f / sqrtf(tot / (float)dim + eps);
+  if (VEC == 4 && ((uintptr_t)h | (uintptr_t)w) % 16 == 0) {
+    for (int c = threadIdx.x * 4; c < dim; c += blockDim.x * 4) {
+      f32x4 v = *reinterpret_cast<const f32x4*>(urow + c);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = v[u] * rs * (ldf(w + c + u) + w_offset);
+      st4((S*)h + (long)t * dim + c, v);
+    }
+    return;
+  }
   for (int c = threadIdx.x; c < dim; c += blockDim.x)
     stf((S*)h + (long)t * dim + c, urow[c] * rs * (ldf(w + c) + w_offset));
 }
@@ -230,23 +248,28 @@ __global__ void __launch_bounds__(1024) sink_prepare4_kernel(
     else return (int)hipErrorInvalidValue;        \
   } while (0)
 
-extern "C" int dli_hyper_mix(float* xs, const float* y, int ldy, const float* prev,
-                             const float* read, const void* w, void* h, int T, int ns, int dim,
-                             float eps, float w_offset, int dt, hipStream_t st) {
+// y: nsplit slabs, ysplit elements apart, whose sum is the sublayer's output (1: the output itself)
+extern "C" int dli_hyper_mix(float* xs, const float* y, int ldy, int nsplit, long ysplit,
+                             const float* prev, const float* read, const void* w, void* h, int T,
+                             int ns, int dim, float eps, float w_offset, int dt, hipStream_t st) {
   if (T <= 0) return 0;
-  if (ns < 1 || ns > MAXS || dim < 1 || (y != nullptr) != (prev != nullptr) ||
+  if (ns < 1 || ns > MAXS || dim < 1 || (y != nullptr) != (prev != nullptr) || nsplit < 1 ||
       (read != nullptr && h == nullptr) || (read == nullptr && y == nullptr))
     return (int)hipErrorInvalidValue;
-  const size_t sh = ((size_t)dim + 16 + (size_t)ns * (ns + 3)) * 4;
+  const size_t sh = ((size_t)dim + 16) * 4;
   if (sh > 60000) return (int)hipErrorInvalidValue;
   const bool v4 = dim % 4 == 0 && (uintptr_t)xs % 16 == 0 &&
-                  (y == nullptr || ((uintptr_t)y % 16 == 0 && ldy % 4 == 0));
+                  (y == nullptr || ((uintptr_t)y % 16 == 0 && ldy % 4 == 0 && ysplit % 4 == 0));
   const int nt = (T <= 1024 && dim >= 2048) ? 1024 : 256;
-#define HM_LAUNCH(S, V)                                                                       \
-  hyper_mix_kernel<S, V><<<T, nt, sh, st>>>(xs, y, ldy, prev, read, (const S*)w, h, ns, dim,  \
-                                            eps, w_offset)
-  if (v4) DT_SWITCH2(dt, HM_LAUNCH(u16, 4), HM_LAUNCH(float, 4));
-  else DT_SWITCH2(dt, HM_LAUNCH(u16, 1), HM_LAUNCH(float, 1));
+#define HM_LAUNCH(S, V, N)                                                                    \
+  hyper_mix_kernel<S, V, N><<<T, nt, sh, st>>>(xs, y, ldy, nsplit, ysplit, prev, read,         \
+                                               (const S*)w, h, ns, dim, eps, w_offset)
+#define HM_STREAMS(S)                                                                         \
+  (ns == 2 ? (void)HM_LAUNCH(S, 4, 2) : ns == 3 ? (void)HM_LAUNCH(S, 4, 3)                     \
+   : ns == 4 ? (void)HM_LAUNCH(S, 4, 4) : (void)HM_LAUNCH(S, 4, 0))
+  if (v4) DT_SWITCH2(dt, HM_STREAMS(u16), HM_STREAMS(float));
+  else DT_SWITCH2(dt, (HM_LAUNCH(u16, 1, 0)), (HM_LAUNCH(float, 1, 0)));
+#undef HM_STREAMS
 #undef HM_LAUNCH
   DLI_RETURN_LAUNCH();
 }

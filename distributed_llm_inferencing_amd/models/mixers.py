@@ -179,7 +179,7 @@ def attention_mixer(spec: LayerSpec, lp: dict, h, step: StepView, cache, eps: fl
     o = H.window_attention(q, kc, vc, d, d, Hh, G, step.cu_seqlens, step.max_seqlen,
                            step.positions, step.block_tables, step.block_size, spec.window,
                            spec.scale, slopes=lp["slopes"], talk=lp["talk"], gate=gate)
-    return H.linear_any(o, lp["wo"])
+    return H.linear_out(o, lp["wo"])
 
 
 def hgrn2_mixer(spec: LayerSpec, lp: dict, h, step: StepView, cache, eps: float):
@@ -190,7 +190,7 @@ def hgrn2_mixer(spec: LayerSpec, lp: dict, h, step: StepView, cache, eps: float)
     o = H.hgrn2(proj, lp["f_b"], lp["lower"], lp["o_norm"], eps, state, step.state_slots,
                 step.cu_seqlens, step.max_seqlen, step.positions, spec.heads, spec.dim,
                 spec.vdim, step.min_seqlen)
-    return H.linear_any(o, lp["wo"])
+    return H.linear_out(o, lp["wo"])
 
 
 def latent_attention_mixer(spec: LayerSpec, lp: dict, h, step: StepView, cache, eps: float):
@@ -233,7 +233,7 @@ def latent_attention_mixer(spec: LayerSpec, lp: dict, h, step: StepView, cache, 
                                             step.cu_seqlens, step.max_seqlen, step.positions,
                                             step.block_tables, step.block_size, step.cu_visible(win),
                                             total, most, win, spec.scale, gates)
-            return H.linear_any(o, lp["wo"])
+            return H.linear_out(o, lp["wo"])
     H.head_linear(q_nope, lp["w_ukT"], q_full)               # q_full[:, h, :r] = W_uk,h^T q_h
     ol = H.window_attention(q_full.view(T, Hh * (r + dr)), c, c, r + dr, r, Hh, 1,
                             step.cu_seqlens, step.max_seqlen, step.positions,
@@ -241,10 +241,10 @@ def latent_attention_mixer(spec: LayerSpec, lp: dict, h, step: StepView, cache, 
     if gates is not None:                   # one sigmoid gate per head, on the fp32 expansion
         o32 = torch.empty(T, Hh, dv, dtype=torch.float32, device=h.device)
         H.head_linear(ol.view(T, Hh, r), lp["w_uv"], o32)
-        return H.linear_any(H.head_gate(o32, gates, h.dtype), lp["wo"])
+        return H.linear_out(H.head_gate(o32, gates, h.dtype), lp["wo"])
     o = torch.empty(T, Hh, dv, dtype=h.dtype, device=h.device)
     H.head_linear(ol.view(T, Hh, r), lp["w_uv"], o)
-    return H.linear_any(o.view(T, Hh * dv), lp["wo"])
+    return H.linear_out(o.view(T, Hh * dv), lp["wo"])
 
 
 def gla_mixer(spec: LayerSpec, lp: dict, h, step: StepView, cache, eps: float):
@@ -259,7 +259,7 @@ def gla_mixer(spec: LayerSpec, lp: dict, h, step: StepView, cache, eps: float):
     z = H.linear_any(a1, lp["w_a2"])
     o = H.gla(proj, z, lp["a_b"], spec.tau, lp["o_norm"], eps, state, step.state_slots,
               step.cu_seqlens, step.max_seqlen, step.positions, Hh, d, dv, step.min_seqlen)
-    return H.linear_any(o, lp["wo"])
+    return H.linear_out(o, lp["wo"])
 
 
 def talk_attention_mixer(spec: LayerSpec, lp: dict, h, step: StepView, cache, eps: float):
@@ -276,7 +276,7 @@ def talk_attention_mixer(spec: LayerSpec, lp: dict, h, step: StepView, cache, ep
     o = H.window_attention(q, kc, vc, G * d, dv, Hh, G, step.cu_seqlens, step.max_seqlen,
                            step.positions, step.block_tables, step.block_size,
                            spec.window or (1 << 30), spec.scale, chunk=spec.chunk, k_groups=1)
-    return H.linear_any(o, lp["wo"])
+    return H.linear_out(o, lp["wo"])
 
 
 def lightning_mixer(spec: LayerSpec, lp: dict, h, step: StepView, cache, eps: float):
@@ -288,7 +288,7 @@ def lightning_mixer(spec: LayerSpec, lp: dict, h, step: StepView, cache, eps: fl
     o = H.lightning(proj, lp["decays"], state, step.state_slots, step.cu_seqlens,
                     step.max_seqlen, step.positions, Hh, d, dv, step.min_seqlen)
     g0 = 2 * Hh * d + Hh * dv
-    return H.linear_any(H.rmsnorm_cols(o, lp["o_norm"], eps, gate=proj[:, g0:g0 + Hh * dv]),
+    return H.linear_out(H.rmsnorm_cols(o, lp["o_norm"], eps, gate=proj[:, g0:g0 + Hh * dv]),
                         lp["wo"])
 
 
@@ -316,7 +316,7 @@ def parallel_mixer(spec: LayerSpec, lp: dict, h, step: StepView, cache, eps: flo
     H.mlstm(proj[:, nl + l.heads:], lp["if_b"], r.gate_cap, lp["o_norm"], eps, state, mstate,
             step.state_slots, step.cu_seqlens, step.max_seqlen, step.positions, r.heads, r.dim,
             r.vdim, o[:, wl:], spec.right_scale, step.min_seqlen)
-    return H.linear_any(o, lp["wo"])
+    return H.linear_out(o, lp["wo"])
 
 
 def retention_mixer(spec: LayerSpec, lp: dict, h, step: StepView, cache, eps: float):
@@ -453,7 +453,7 @@ def gated_gelu_ff(spec: LayerSpec, lp: dict, h):
     else:                               # (a few rows: the weight-streaming kernel, fp32 out)
         act = H.act_mul(H.linear_any(h, lp["w_gu"]), spec.ff, h.dtype,
                         "gelu_mul_pairs" if "ff_tuned" in lp else "gelu_mul")
-    return H.linear_any(act, lp["w_down"])
+    return H.linear_out(act, lp["w_down"])
 
 
 def gelu_ff(spec: LayerSpec, lp: dict, h):
@@ -462,7 +462,7 @@ def gelu_ff(spec: LayerSpec, lp: dict, h):
         act = ops.linear(h, lp["w_up"], lp["b_up"], epi="bias_gelu")
     else:
         act = H.act_mul(H.linear_any(h, lp["w_up"]), spec.ff, h.dtype, "gelu")
-    return H.linear_any(act, lp["w_down"])
+    return H.linear_out(act, lp["w_down"])
 
 
 def gated_silu_ff(spec: LayerSpec, lp: dict, h):
@@ -471,7 +471,7 @@ def gated_silu_ff(spec: LayerSpec, lp: dict, h):
         act = ops.linear(h, lp["w_gu"], epi="silu_mul")
     else:
         act = H.act_mul(H.linear_any(h, lp["w_gu"]), spec.ff, h.dtype, "silu_mul")
-    return H.linear_any(act, lp["w_down"])
+    return H.linear_out(act, lp["w_down"])
 
 
 def gated_relu_ff(spec: LayerSpec, lp: dict, h):

@@ -101,7 +101,7 @@ _SIGS = {
     # post-norm designs (postnorm.hip)
     "dli_prev_tokens": [P, P, P, P, P, P, I, I, P],
     "dli_embedding_bigram": [P, P, P, P, P, P, I, I, I, I, I, I, I, P],
-    "dli_postnorm": [P, P, I, F, P, P, P, I, I, F, P, I, P],
+    "dli_postnorm": [P, P, I, I, L, F, P, P, P, I, I, F, P, I, P],
     "dli_add_rmsnormed": [P, P, I, P, P, I, I, F, I, P],
     "dli_side_gate": [P, P, I, P, P, I, I, I, I, I, I, P],
     "dli_rmsnorm_cols": [P, P, I, P, I, I, F, P, I, I, I, F, I, I, P],
@@ -109,9 +109,9 @@ _SIGS = {
     "dli_head_gate": [P, P, P, I, I, I, I, I, P],
     "dli_logit_router": [P, P, P, I, P, P, I, I, I, I, I, P],
     # hyper-connected designs (streams.hip, recurrent_scalar.hip)
-    "dli_hyper_mix": [P, P, I, P, P, P, P, I, I, I, F, F, I, P],
+    "dli_hyper_mix": [P, P, I, I, L, P, P, P, P, I, I, I, F, F, I, P],
     "dli_sink_prepare": [P, I, P, P, F, I, I, I, I, I, I, P, F, P, P, P, P, P, I, P],
-    "dli_scalar_recurrence": [P, I, I, P, P, F, P, F, P, P, P, P, P, P, I, F, I, I, I, I, I,
+    "dli_scalar_recurrence": [P, I, I, P, P, F, P, F, P, P, P, P, P, P, I, F, I, I, I, I, I, I,
                               I, I, P, I, P],
     # rotated designs (rotary.hip, retention.hip, swa_attention.hip)
     "dli_swa_attention": [P, I, P, L, P, L, P, I, P, P, P, I, I, I, I, I, I, I, I, I, I, F, P, I, I,

@@ -74,8 +74,8 @@ def linear_any(x: torch.Tensor, w: torch.Tensor, out_f32: bool = True,
 
 
 def linear_out(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """x @ w^T in fp32 for a consumer that adds it to the residual (``resadd_groupnorm``, or any
-    through ``rows_of``): [M, N], or, where the planned GEMM splits K, its partial sums
+    """x @ w^T in fp32 for a consumer that adds it to the residual (``resadd_groupnorm``, ``postnorm``,
+    ``hyper_mix``, or any through ``rows_of``): [M, N], or, where the planned GEMM splits K, its partial sums
     [splits, M, N] in the shared workspace, which the add sums itself (one launch and one pass
     less). They must be consumed before the next GEMM."""
     if (x.is_cuda and x.dtype == torch.bfloat16 and x.shape[1] % 64 == 0 and w.shape[0] % 4 == 0
@@ -113,6 +113,14 @@ class RoutedRows:
     k: int
     shared: Optional[torch.Tensor]
     tokens: int
+
+
+def slabs_of(y) -> tuple:
+    """(row stride, number, distance in elements) of the partial sums that ``y`` [M, N] or
+    [splits, M, N] holds, as the kernels that sum them take them."""
+    if y is None:
+        return 0, 1, 0
+    return (y.stride(0), 1, 0) if y.dim() == 2 else (y.stride(1), y.shape[0], y.stride(0))
 
 
 def rows_of(y) -> Optional[torch.Tensor]:
@@ -206,10 +214,9 @@ def resadd_groupnorm(x: torch.Tensor, y: Optional[torch.Tensor], w: Optional[tor
          if w is not None else None)
     if add is not None and (add.shape != x.shape or not add.is_contiguous()):
         raise ValueError("resadd_groupnorm: add must have the stream's shape")
-    slabs = y is not None and y.dim() == 3
-    _call("dli_resadd_groupnorm", _p(x), _p(y), y.stride(-2) if y is not None else 0,
-          y.shape[0] if slabs else 1, y.stride(0) if slabs else 0, _p(bias), _p(add), float(keep), float(mult), _p(w), _p(h), dim, rows, dim, groups, float(eps), None,
-          float(gain), int(out_f32), float(w_offset), _dt(dtype), _st())
+    _call("dli_resadd_groupnorm", _p(x), _p(y), *slabs_of(y), _p(bias), _p(add), float(keep), float(mult),
+          _p(w), _p(h), dim, rows, dim, groups, float(eps), None, float(gain), int(out_f32),
+          float(w_offset), _dt(dtype), _st())
     return h
 
 
@@ -721,16 +728,17 @@ def embedding_bigram(ids, prev, table, bigram, buckets: int, mul_prev: int, mul_
 
 def postnorm(x, y, w, b, eps: float, keep: float = 1.0,
              rows_idx: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """x = LayerNorm(keep * x + y) * w + b on the fp32 stream, in place (y optional, fp32);
-    returns the new rows in the storage dtype (w's). With ``rows_idx`` (int64) only those rows
+    """x = LayerNorm(keep * x + y) * w + b on the fp32 stream, in place (y optional, fp32, or a
+    GEMM's partial sums, see ``linear_out``); returns the new rows in the storage dtype (w's). With ``rows_idx`` (int64) only those rows
     are normed and returned and x is left alone."""
-    y = rows_of(y)
+    if not isinstance(y, (torch.Tensor, type(None))):
+        y = rows_of(y)
     if not x.is_cuda:
         return R.postnorm(x, y, w, b, eps, keep, w.dtype, rows_idx)
     dim = x.shape[1]
     rows = x.shape[0] if rows_idx is None else rows_idx.shape[0]
     h = torch.empty(rows, dim, dtype=w.dtype, device=x.device)
-    _call("dli_postnorm", _p(x), _p(y), y.stride(0) if y is not None else 0, float(keep), _p(w),
+    _call("dli_postnorm", _p(x), _p(y), *slabs_of(y), float(keep), _p(w),
           _p(b), _p(h), rows, dim, float(eps), _p(rows_idx), _dt(w.dtype), _st())
     return h
 
@@ -893,18 +901,19 @@ def moe_gelu_experts_f32(x, w_up, w_down, topk_w, topk_ids, shared=None) -> torc
 def hyper_mix(xs, y, prev, read, w, eps: float = 0.0, w_offset: float = 0.0, dtype=None):
     """One step of hyper-connections on the fp32 streams xs [T, S, D], in place
     (``reference.hyper_mix``): with y (a sublayer's fp32 output) and ``prev`` (that sublayer's
-    fp32 vector read | write | mix) the streams are mixed and receive y; with ``read`` (the next
+    fp32 vector read | write | mix) the streams are mixed and receive y (or, of a GEMM's partial sums,
+    see ``linear_out``, their sum); with ``read`` (the next
     sublayer's vector, or ones for the plain sum) the weighted sum of the new streams is
     returned — RMS-normed times (w + w_offset) in the storage dtype when w is given, else fp32."""
-    y = rows_of(y)
+    if not isinstance(y, (torch.Tensor, type(None))):
+        y = rows_of(y)
     if not xs.is_cuda:
         return R.hyper_mix(xs, y, prev, read, w, eps, w_offset, dtype or (w.dtype if w is not None else None))
     T, S, D = xs.shape
     h = None
     if read is not None:
         h = torch.empty(T, D, dtype=torch.float32 if w is None else w.dtype, device=xs.device)
-    _call("dli_hyper_mix", _p(xs), _p(y), y.stride(0) if y is not None else 0, _p(prev),
-          _p(read), _p(w), _p(h), T, S, D, float(eps), float(w_offset),
+    _call("dli_hyper_mix", _p(xs), _p(y), *slabs_of(y), _p(prev), _p(read), _p(w), _p(h), T, S, D, float(eps), float(w_offset),
           _dt(w.dtype) if w is not None else 1, _st())
     return h
 
@@ -939,7 +948,8 @@ def lightning(proj, decays, state, slots, cu_seqlens, max_seqlen, positions, H, 
     def walk(max_len, longest):
         _call("dli_scalar_recurrence", _p(proj), proj.stride(0), 0, _p(decays), None, 0.0, None, 0.0,
               _p(state), None, _p(slots), _p(cu_seqlens), _p(positions), _p(out), out.stride(0), 1.0,
-              S, longest, max_len, H, d, dv, _column_block(S, H, d, dv, longest), None, 1, _st())
+              S, 1 if longest == 1 else min_seqlen, longest, max_len, H, d, dv,
+              _column_block(S, H, d, dv, longest), None, 1, _st())
     _recurrence(_CHUNK_FIXED, proj, state, slots, cu_seqlens, positions, out, max_seqlen, min_seqlen, H,
                 d, dv, torch.float32, walk, decays=decays)
     return out
@@ -975,8 +985,8 @@ def mlstm(proj, if_b, cap: float, norm_w, eps: float, state, mstate, slots, cu_s
         raw = torch.empty(proj.shape[0], H * dv, dtype=torch.float32, device=proj.device) if cw else None
         _call("dli_scalar_recurrence", _p(proj), proj.stride(0), 1, None, _p(if_b), float(cap),
               _p(norm_w), float(eps), _p(state), _p(mstate), _p(slots), _p(cu_seqlens),
-              _p(positions), _p(out), out.stride(0), float(out_scale), S, longest, max_len, H, d, dv,
-              cw, _p(raw), _dt(norm_w.dtype), _st())
+              _p(positions), _p(out), out.stride(0), float(out_scale), S, 1 if longest == 1 else min_seqlen,
+              longest, max_len, H, d, dv, cw, _p(raw), _dt(norm_w.dtype), _st())
         if cw:
             g0 = 2 * H * d + H * dv
             rmsnorm_cols(raw, norm_w, eps, gate=proj[:, g0:g0 + H * dv], groups=H, out=out,

@@ -83,8 +83,9 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_bf16_kernel(
     const int gr = min(n0 + r, N - 1);
     w_src[i] = Wg + (long)gr * ldw + kb + c * 8;
   }
-  // STREAM: column tile t starts at K-tile t mod nk and wraps around (see gemm_stream.h)
-  const int rot = STREAM && nk > 0 ? (tn + grp) % nk : 0;
+  // STREAM: column tile t starts at K-tile t mod nk and wraps around (see gemm_stream.h); not over less
+  // than 2 KB of a row, whose sums then are the other tiles' to the bit
+  const int rot = STREAM && nk * BKT >= 1024 ? (tn + grp) % nk : 0;
   constexpr int W_AUX = STREAM ? 2 : 0;            // nt: each weight line is read once
   auto stage = [&](int buf, int kt) {
     char* base = smem + buf * BUF;

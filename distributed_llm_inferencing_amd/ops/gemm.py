@@ -54,15 +54,13 @@ TILES = {0: (64, 64), 1: (64, 128), 2: (128, 128), 3: (128, 256), 4: (256, 128),
          34: (256, 256), 41: (256, 256), 45: (256, 256),
          # 55 = 45 persistent: one workgroup per CU walks its tiles, the next tile's first two
          # K-tiles staged in the current tile's last two (gemm4wp.hip); no split-K / grouped
-         55: (256, 256),
-         # weight-streaming tiles for up to 128 rows (gemm_stream.h): weights nontemporal, K loops
-         # turned from tile to tile, 3 to 6 stages
-         60: (32, 32), 61: (32, 128), 62: (32, 64), 63: (64, 128), 64: (64, 64), 65: (64, 256),
-         66: (96, 128), 67: (128, 128), 68: (128, 256), 69: (64, 32), 70: (96, 64), 71: (128, 64),
-         72: (128, 32)}
-# their K-tiles
-STREAM_K = {60: 256, 61: 64, 62: 256, 63: 64, 64: 64, 65: 64, 66: 64, 67: 64, 68: 64, 69: 256, 70: 64,
-            71: 64, 72: 128}
+         55: (256, 256)}
+# weight-streaming tiles for up to 128 rows (gemm_stream.h): weights nontemporal, K loops turned from
+# tile to tile, 3 to 6 stages; (BM, BN, K-tile: a split of K holds whole ones), so kept apart
+STREAM_TILES = {60: (32, 32, 256), 61: (32, 128, 64), 62: (32, 64, 256), 63: (64, 128, 64),
+                64: (64, 64, 64), 65: (64, 256, 64), 66: (96, 128, 64), 67: (128, 128, 64),
+                68: (128, 256, 64), 69: (64, 32, 256), 70: (96, 64, 64), 71: (128, 64, 64),
+                72: (128, 32, 128)}
 STREAM_MAX_M = 128
 # the 4-wave plan raced against the 8-phase one in the prefill autotune
 PREFILL_4W_TILE = 45
@@ -93,6 +91,16 @@ TILE_WAVES = {13: (2, 4), 14: (4, 2), 15: (2, 4), 16: (4, 2), 17: (2, 4),
               26: (4, 2), 28: (4, 2), 60: (2, 1), 66: (1, 4), 68: (2, 4), 69: (4, 1), 72: (4, 1)}
 
 
+def tile_shape(tile: int):
+    """(BM, BN) of an MFMA tile."""
+    return STREAM_TILES[tile][:2] if tile in STREAM_TILES else TILES[tile]
+
+
+def tile_step(tile: int) -> int:
+    """The K-tile of an MFMA tile."""
+    return STREAM_TILES[tile][2] if tile in STREAM_TILES else 64
+
+
 def tile_ok(tile: int, epi: str) -> bool:
     """The SiLU*up epilogue pairs 16-column gate/up blocks inside a wave's column range,
     which must therefore be a multiple of 32."""
@@ -108,7 +116,7 @@ def tile_ok(tile: int, epi: str) -> bool:
         return True
     if tile == 26:              # the straddling gate/up pair meets through LDS
         return True
-    bn = TILES[tile][1]
+    bn = tile_shape(tile)[1]
     return (bn // TILE_WAVES.get(tile, (2, 2))[1]) % 32 == 0
 
 
@@ -121,11 +129,11 @@ PAIR_EPIS = ("silu_mul", "clamp_mul", "relu_mul", "gelu_mul")
 # tiles whose slab-only split-K call can store fp16 partials (EPI "slab16": the generic tile
 # family and the 8-phase kernels); the fused consumers then read half the bytes. The
 # weight-streaming GEMVs and the 4-wave family keep fp32 slabs.
-SLAB16_TILES = frozenset(list(range(0, 22)) + [22, 23, 24, 25, 26, 28] + list(STREAM_K))
+SLAB16_TILES = frozenset(list(range(0, 22)) + [22, 23, 24, 25, 26, 28] + list(STREAM_TILES))
 SLAB16 = os.environ.get("DLI_SLAB_FP32", "0") != "1"      # A/B: fp32 partials everywhere
 # tiles whose grouped SiLU*up GEMM can read its rows through a permutation (the generic
 # family: dli_gemm_grouped_gather), so the MoE gate/up skips the gathered copy of its input
-GATHER_TILES = frozenset(list(range(0, 22)) + [23, 24, 25] + list(STREAM_K))
+GATHER_TILES = frozenset(list(range(0, 22)) + [23, 24, 25] + list(STREAM_TILES))
 NUM_CUS = 256
 
 
@@ -176,7 +184,7 @@ def _stream_plan(M: int, N: int, K: int, epi: str):
     second round costs as much as the first); where 32 columns are too wide too, 64 and K split until
     about one workgroup a CU. fp32 outputs, us on these against the best other tile: 24 rows: 4096 x 4096
     11.6 / 13.2, 8192 x 4096 13.9 / 17.6, 16384 x 4096 23.7 / 30.7, 4096 x 14336 24.2 / 27.4, 32000 x 4096 41.5 /
-    56.3, 128256 x 4096 167 / 197 (4 rows 155, on the plain weight stream 164); 64 rows: 14.1 / 13.8, 16.5 /
+    56.3, 128256 x 4096 167 / 197; 64 rows: 14.1 / 13.8, 16.5 /
     20.0, 26.5 / 35.2, 28.5 / 29.0, 45 / 60, 177 / 209; 96 rows: 16.3 / 16.2, 23.8 / 24.4, 30.1 / 38.3, 31.9 / 33.0,
     47.5 / 63.5, 190 / 215. Above 96 rows the narrowest weights stay on two rows of tile 6 or one of tile 7
     (128 rows, 4096 x 4096 17.6 / 19.8, 4096 x 14336 35 / 39), from 65 rows the small ones on tile 5 (96 rows,
@@ -192,7 +200,7 @@ def _stream_plan(M: int, N: int, K: int, epi: str):
         tile = wide
     elif -(-N // 64) >= fill:
         tile = mid
-    elif -(-N // 32) >= fill and K % STREAM_K[narrow] == 0:
+    elif -(-N // 32) >= fill and K % tile_step(narrow) == 0:
         tile = narrow
     else:
         split = True
@@ -201,10 +209,10 @@ def _stream_plan(M: int, N: int, K: int, epi: str):
             tile = 5
         elif M > 96 and N < 6144:
             tile = 7 if K > 8192 else 6
-    if K % STREAM_K.get(tile, 64):
+    if K % tile_step(tile):
         tile = wide
-    step = STREAM_K.get(tile, 64)
-    bm, bn = TILES[tile]
+    step = tile_step(tile)
+    bm, bn = tile_shape(tile)
     tiles, splits = -(-M // bm) * -(-N // bn), 1
     most = 2 * NUM_CUS if tile == 5 else NUM_CUS
     # (K <= 1024: the second launch costs more than the shorter loop saves, 4096 x 1024 at 24 rows 6.1 / 7.8)
@@ -264,7 +272,9 @@ def _heuristic(M: int, N: int, K: int, epi: str) -> GemmPlan:
         # residual-adding GEMV (full K): 4 rows a workgroup, 8 K-steps in flight per lane
         # (1024 workgroups on a 4096-wide projection)
         return GemmPlan("dli", 56, 1)
-    if 2 < M <= STREAM_MAX_M and (M > GEMV_MAX_M or epi not in ("splitk", "none")):
+    # (up to 4 rows the fitted plans stay on the plain weight stream, whose sums do not depend on the
+    # number of rows; a capture's timing may choose otherwise)
+    if GEMV_MAX_M < M <= STREAM_MAX_M:
         p = _stream_plan(M, N, K, epi)
         if p is not None:
             return p
@@ -335,8 +345,8 @@ def grouped_plan(rows: int, N: int, K: int, epi: str, groups: int) -> GemmPlan:
     # experts of few rows: the streaming tile that covers them
     need = 1.25 * rows / max(1, groups)
     for t in (61, 63, 66) if "DLI_MOE_TILE" not in os.environ else ():
-        if need <= TILES[t][0]:
-            if K % STREAM_K[t] == 0 and tile_ok(t, epi):
+        if need <= tile_shape(t)[0]:
+            if K % tile_step(t) == 0 and tile_ok(t, epi):
                 tile = t
             break
     return GemmPlan("dli", tile, 1)
@@ -367,12 +377,13 @@ def autotune_grouped(rows: int, w: torch.Tensor, epi: str, iters: int = 5, log=N
     comb = torch.empty(max(rows, 1), N, dtype=w.dtype, device=dev)
     best = None
     cands = []
-    for tile in sorted(TILES):
-        if TILES[tile][0] > 2 * max(64, rows // E + 32) or not tile_ok(tile, epi):
+    for tile in sorted(TILES) + sorted(STREAM_TILES):
+        bm = tile_shape(tile)[0]
+        if bm > 2 * max(64, rows // E + 32) or not tile_ok(tile, epi):
             continue                                  # far taller than an expert's rows
-        if tile in STREAM_K and TILES[tile][0] < rows // E:
+        if tile in STREAM_TILES and bm < rows // E:
             continue                                  # streams the weights once or not at all
-        step = STREAM_K.get(tile, 64)
+        step = tile_step(tile)
         for splits in (1, 2, 4):                      # split-K for long-K expert GEMMs
             if K % (step * splits) == 0 and (splits == 1 or K // splits >= 2048):
                 cands.append(GemmPlan("dli", tile, splits))
@@ -664,14 +675,15 @@ def candidate_plans(M: int, N: int, K: int, epi: str):
         t224 = -(-M // 256) * -(-N // 224)
         if t256 > NUM_CUS and t224 % NUM_CUS == 0:
             excl.discard(26)
-    for tile, (bm, bn) in TILES.items():
+    for tile in [*TILES, *STREAM_TILES]:
+        bm, bn = tile_shape(tile)
         if not tile_ok(tile, epi) or tile in excl:
             continue
         if M <= 64 and bm > 64:
             continue
         if M > 512 and bm < 128:
             continue
-        if tile in STREAM_K:
+        if tile in STREAM_TILES:
             # one row of tiles; for 2 to 4 rows beside the weight stream's own kernels, but for the
             # products whose partial sums those keep in fp32
             band = next((b for b in STREAM_BANDS if M <= b[0]), ())
@@ -681,7 +693,7 @@ def candidate_plans(M: int, N: int, K: int, epi: str):
         elif M <= 64 and tile in (0, 1) and K % 128 == 0:
             continue                     # slower than their 3-stage and streaming forms
         for splits in (1, 2, 4, 8):
-            if K % (STREAM_K.get(tile, 64) * splits) or K // splits < 256:
+            if K % (tile_step(tile) * splits) or K // splits < 256:
                 continue
             tiles = -(-M // bm) * -(-N // bn)
             if splits > 1 and tiles * splits > 4 * NUM_CUS:

@@ -796,12 +796,8 @@ def moe_mlp(x, w_gu, w_down, topk_w, topk_ids, expert_offset: int = 0,
     p_dn = G.grouped_plan(rows, D, Fa, "none", E_local)
     if moe_slab_plan(p_dn):
         if defer_combine:
-            # the down projection's slabs; the combine runs with the next layer's add + norm
-            ws = G.workspace(dev, p_dn.splits * max(n, 1) * D * 2)
-            _native_call("dli_gemm", _p(act), act.stride(0), _p(w_down), w_down.stride(-2),
-                         None, D, n, D, Fa, G.EPI["slab16"], p_dn.tile, p_dn.splits, None,
-                         _p(ws), _p(offsets), E_local, _st())
-            return MoEPending(ws, p_dn.splits, n, topk_w, pos, (T, D), x.dtype, dev)
+            # the combine runs with the next layer's add + norm
+            return moe_down_pending(act, w_down, offsets, n, p_dn, topk_w, pos, (T, D))
         out = torch.empty_like(x)
         moe_down_combine(act, w_down, offsets, n, p_dn, topk_w, pos, out)
         return out
@@ -846,6 +842,16 @@ def moe_slab_plan(p: Optional[G.GemmPlan]) -> bool:
     combine (``moe_down_combine``) instead of GEMM -> fp32 slab reduce -> bf16 y -> combine."""
     return (p is not None and G.SLAB16 and p.splits in (2, 4, 8)
             and p.tile in G.SLAB16_TILES)
+
+
+def moe_down_pending(act, w_down, offsets, n: int, p: G.GemmPlan, topk_w, pos, shape) -> MoEPending:
+    """The grouped down projection's fp16 split-K slabs, for a consumer that combines them."""
+    E_local, D, F = w_down.shape
+    ws = G.workspace(act.device, p.splits * max(n, 1) * D * 2)
+    _native_call("dli_gemm", _p(act), act.stride(0), _p(w_down), w_down.stride(-2), None, D,
+                 n, D, F, G.EPI["slab16"], p.tile, p.splits, None, _p(ws), _p(offsets),
+                 E_local, _st())
+    return MoEPending(ws, p.splits, n, topk_w, pos, shape, act.dtype, act.device)
 
 
 def moe_down_combine(act, w_down, offsets, n: int, p: G.GemmPlan, topk_w, pos, out):

@@ -370,11 +370,14 @@ def autotune_grouped(rows: int, w: torch.Tensor, epi: str, iters: int = 5, log=N
     off = torch.tensor([0] + list(__import__("itertools").accumulate(counts)),
                        dtype=torch.int32, device=dev)
     x = (torch.randn(max(rows, 1), K, device=dev) * 0.5).to(w.dtype)
-    # the down projection's split plans on the fp16-slab tiles run fused with the combine
-    # (ops.moe_down_combine): time them that way (one pick per row, weight 1)
+    # the down projection is timed with what follows it (one pick per row, weight 1): the split plans on
+    # the fp16-slab tiles fused with the combine, the residual add and, at the widths that take it, the
+    # next norm (ops.MoEPending); the others with their kernels for the same. Timed alone, an unsplit
+    # plan won at 64 tokens x 2 of 8 experts and cost the step 10 us a layer
     ones = torch.ones(max(rows, 1), 1, dtype=torch.float32, device=dev)
     ident = torch.arange(max(rows, 1), dtype=torch.int32, device=dev).view(-1, 1)
     comb = torch.empty(max(rows, 1), N, dtype=w.dtype, device=dev)
+    res, nw = torch.zeros_like(comb), torch.ones(N, dtype=w.dtype, device=dev)
     best = None
     cands = []
     for tile in sorted(TILES) + sorted(STREAM_TILES):
@@ -392,10 +395,13 @@ def autotune_grouped(rows: int, w: torch.Tensor, epi: str, iters: int = 5, log=N
 
         def run(p=p, fused=fused):
             if fused:
-                ops.moe_down_combine(x, w, off, rows, p, ones, ident, comb)
-            else:
-                ops._gemm_native(x, w, epi, plan=p, groups=E, group_off=off,
-                                 rows_per_group=rows)
+                ops.moe_down_pending(x, w, off, rows, p, ones, ident, comb.shape).add_rmsnorm(res, nw, 1e-5)
+                return
+            y = ops._gemm_native(x, w, epi, plan=p, groups=E, group_off=off, rows_per_group=rows)
+            if epi == "none":
+                ops._native_call("dli_moe_combine", comb.data_ptr(), y.data_ptr(), ones.data_ptr(),
+                                 ident.data_ptr(), rows, 1, N, ops._st())
+                ops.add_rmsnorm(comb, res, nw, 1e-5)
         try:
             ms = ops.benchmark(run, iters=iters, warmup=1, graph=_GRAPH_TUNE)
         except Exception:  # noqa: BLE001

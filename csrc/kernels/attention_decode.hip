@@ -47,27 +47,27 @@ __device__ __forceinline__ int decode_bt_window(const int* __restrict__ block_ta
   return block_tables[(long)b * max_blocks + min(s_begin / block_size + lane, last_blk)];
 }
 
-// [s_begin, s_end) of wave wv when WPI waves split a context of ctx tokens by whole tiles
+// [s_begin, s_end) of wave wv when WPI waves split the tokens [from, to) by whole tiles
 template <int WPI>
-__device__ __forceinline__ void decode_wg_range(int ctx, int wv, int& s_begin, int& s_end) {
-  const int tiles = (ctx + DEC_TILE - 1) / DEC_TILE;
+__device__ __forceinline__ void decode_wg_range(int from, int to, int wv, int& s_begin, int& s_end) {
+  const int tiles = (max(to - from, 0) + DEC_TILE - 1) / DEC_TILE;
   const int per = (tiles + WPI - 1) / WPI;
-  s_begin = min(ctx, wv * per * DEC_TILE);
-  s_end = min(ctx, s_begin + per * DEC_TILE);
+  s_begin = min(to, from + wv * per * DEC_TILE);
+  s_end = min(to, s_begin + per * DEC_TILE);
 }
 
-// KV splits of a step, from its contexts. Ragged ones: split_tokens (whole tiles) deals the step's
-// tiles to about DEC_TARGET waves, so that one long context among short ones is cut as finely as the
-// step can use; near-equal ones (the mean at least 3/4 of the longest) are cut in the power of two
-// that gives 2048 waves or more, which leaves no short last split and CUs with equal shares (64 x
-// 1000 tokens: 59 us, by DEC_TARGET 62; 24 of 500 - 8000: 62 us, cut like equal ones 101). At least
-// DEC_MIN_TILES tiles a split, and no sequence takes more than num_splits. Sequence b has
-// max(1, ceil(context / split_tokens)) equal ones, listed sequence by sequence: `pair` of that list is
-// (b, split); b = -1 past its end. Every wave works this out for itself (B * hkv < 2048 where there
-// are splits): a few loads and scans.
-__host__ __device__ static inline int decode_even_splits(int items) {
+// KV splits of a step, from its contexts, for units of W waves (a workgroup of 4, or a wave). Ragged
+// contexts: split_tokens (whole tiles) deals the step's tiles to about DEC_TARGET waves, so that one
+// long context among short ones is cut as finely as the step can use; near-equal ones (the mean at
+// least 3/4 of the longest) are cut in the power of two that gives 2048 waves or more, which leaves no
+// short last split and CUs with equal shares (64 x 1000 tokens: 59 us, by DEC_TARGET 62; 24 of 500 -
+// 8000: 62 us, cut like equal ones 101). At least DEC_MIN_TILES tiles a split, and no sequence takes
+// more than num_splits. Sequence b has max(1, ceil(context / split_tokens)) equal ones, listed sequence
+// by sequence: `pair` of that list is (b, split); b = -1 past its end. Every wave works this out for
+// itself: a few loads and scans.
+template <int W> __host__ __device__ static inline int decode_even_splits(int items) {
   int n = 1;
-  while ((long)items * n < 2048) n *= 2;
+  while ((long)items * n < 2048 / W) n *= 2;
   return n;
 }
 struct DecSplit { int b, split, split_tokens, last; };
@@ -83,6 +83,7 @@ __device__ __forceinline__ int wave_scan(int v) {
   step(__builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));
   return v;
 }
+template <int W>
 __device__ __forceinline__ DecSplit decode_split(const int* __restrict__ context_lens, int B, int hkv,
                                                  int num_splits, int pair, int lane) {
   // the first 256 contexts stay in registers
@@ -99,10 +100,10 @@ __device__ __forceinline__ DecSplit decode_split(const int* __restrict__ context
   for (int i = 256 + lane; i < B; i += 64) count(context_lens[i]);
   sum = __builtin_amdgcn_readlane(wave_scan<false>(sum), 63);
   longest = __builtin_amdgcn_readlane(wave_scan<true>(longest), 63);
-  const int even = decode_even_splits(B * hkv);
+  const int even = decode_even_splits<W>(B * hkv);
   const int share = 4l * sum >= 3l * longest * B ? (longest + even - 1) / even
-                                                 : (sum * hkv + DEC_TARGET - 1) / DEC_TARGET;
-  const int per = max(max(share, (longest + num_splits - 1) / num_splits), DEC_MIN_TILES);
+                                                 : (sum * hkv + DEC_TARGET / W - 1) / (DEC_TARGET / W);
+  const int per = max(max(share, (longest + num_splits - 1) / num_splits), max(W, DEC_MIN_TILES));
   DecSplit r{-1, 0, per * DEC_TILE, 0};
   const auto find = [&](int i0, int c) {
     const int n = i0 + lane < B ? max(1, (c + r.split_tokens - 1) / r.split_tokens) : 0;
@@ -128,10 +129,10 @@ __device__ __forceinline__ DecSplit decode_split(const int* __restrict__ context
     if (find(i0, i0 + lane < B ? context_lens[i0 + lane] : 0)) return r;
   return r;
 }
-// waves a split launch needs at most: the even splits, or DEC_TARGET and the rounding up of every
+// units a split launch needs at most: the even splits, or DEC_TARGET and the rounding up of every
 // sequence
-static inline long decode_split_items(int items, int num_splits) {
-  const long even = (long)items * decode_even_splits(items), ragged = DEC_TARGET + items;
+template <int W> static inline long decode_split_items(int items, int num_splits) {
+  const long even = (long)items * decode_even_splits<W>(items), ragged = DEC_TARGET / W + items;
   const long all = (long)items * num_splits, most = even > ragged ? even : ragged;
   return all < most ? all : most;
 }
@@ -341,7 +342,7 @@ __global__ void __launch_bounds__(256, MINW) decode_attn_kernel(
   const int item = blockIdx.x * DEC_WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int kvh = item % hkv;
   DecSplit sp{item / hkv, 0, split_tokens, 0};
-  if (num_splits > 1) sp = decode_split(context_lens, B, hkv, num_splits, item / hkv, lane);
+  if (num_splits > 1) sp = decode_split<1>(context_lens, B, hkv, num_splits, item / hkv, lane);
   if (sp.b < 0 || sp.b >= B) return;                           // wave-uniform exit
   const int b = sp.b, split = sp.split;
   split_tokens = sp.split_tokens;
@@ -369,8 +370,8 @@ __global__ void __launch_bounds__(256, MINW) decode_attn_kernel(
   if (num_splits > 1) decode_end_list(ws_ml, b, hq, kvh, G, num_splits, split, sp.last, lane);
 }
 
-// One (sequence, kv head) item per workgroup of WPI waves: wave wv walks the wv-th of WPI
-// equal slices of the context's 32-token tiles, then the partial (m, l, O) merge through
+// One (sequence, kv head) item, or one KV split of it, per workgroup of WPI waves: wave wv walks the
+// wv-th of WPI equal slices of its 32-token tiles, then the partial (m, l, O) merge through
 // LDS (each wave's V-tile rows are reused for its O partial) and the workgroup writes the
 // GQA group's output rows. Small batches: with one item per wave most of the chip idles and
 // each wave pays one HBM round trip per tile of the whole context.
@@ -380,7 +381,8 @@ __device__ __forceinline__ void decode_attn_wg(
     int lane, int b, int kvh, int G, int s_begin, int s_end, int bt_lane0,
     u16* __restrict__ out, const u16* __restrict__ k_cache, const u16* __restrict__ v_cache,
     const int* __restrict__ block_tables, int max_blocks, int hq, int hkv, int block_size,
-    float scale_log2) {
+    float scale_log2, int num_splits = 1, int split = 0, float* __restrict__ ws_o = nullptr,
+    float* __restrict__ ws_ml = nullptr) {
   constexpr int HD = 128, DB = HD / 16;
   static_assert(16 * HD * 4 <= DEC_TILE * 144 * 2, "O partials fit a wave's V tile");
   const int col = lane & 15, grp = lane >> 4;
@@ -422,11 +424,22 @@ __device__ __forceinline__ void decode_attn_wg(
   const float inv = den > 0.f ? 1.f / den : 0.f;
 #pragma unroll
   for (int j = 0; j < 8; ++j) acc[j] *= inv;
-  store8(out + ((long)b * hq + kvh * G + h) * HD + d0, acc);
+  if (num_splits == 1) {
+    store8(out + ((long)b * hq + kvh * G + h) * HD + d0, acc);
+    return;
+  }
+  const long base = ((long)b * hq + kvh * G + h) * num_splits + split;
+  float4* wo = reinterpret_cast<float4*>(ws_o + base * HD + d0);
+  wo[0] = make_float4(acc[0], acc[1], acc[2], acc[3]);
+  wo[1] = make_float4(acc[4], acc[5], acc[6], acc[7]);
+  if (d0 == 0) {
+    ws_ml[base * 2] = den > 0.f ? M : -INFINITY;
+    ws_ml[base * 2 + 1] = den;
+  }
 }
 
 // Small-batch form of decode_attn_kernel (head dim 128, one KV split): a workgroup per item.
-__global__ void __launch_bounds__(256) decode_attn_wg_kernel(
+__global__ void __launch_bounds__(256, 2) decode_attn_wg_kernel(
     u16* __restrict__ out, const u16* __restrict__ q, int q_stride,
     const u16* __restrict__ k_cache, const u16* __restrict__ v_cache,
     const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ context_lens,
@@ -434,7 +447,7 @@ __global__ void __launch_bounds__(256) decode_attn_wg_kernel(
   constexpr int HD = 128, KK = HD / 32, VROW = HD + 16;
   __shared__ __attribute__((aligned(16))) u16 vtile_all[DEC_WAVES][DEC_TILE * VROW];
   __shared__ float ml_all[DEC_WAVES][16][2];
-  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int item = blockIdx.x;
   const int kvh = item % hkv, b = item / hkv;
   const int col = lane & 15, grp = lane >> 4;
@@ -451,7 +464,7 @@ __global__ void __launch_bounds__(256) decode_attn_wg_kernel(
     }
   }
   int s_begin, s_end;
-  decode_wg_range<DEC_WAVES>(context_lens[b], wv, s_begin, s_end);
+  decode_wg_range<DEC_WAVES>(0, context_lens[b], wv, s_begin, s_end);
   const int bt0 = decode_bt_window(block_tables, max_blocks, b, s_begin, s_end, block_size, lane);
   decode_attn_wg<DEC_WAVES>(qf, vtile_all, ml_all, wv, lane, b, kvh, G, s_begin, s_end, bt0,
                             out, k_cache, v_cache, block_tables, max_blocks, hq, hkv,
@@ -587,7 +600,7 @@ __device__ __forceinline__ void fused_cache_row(const void* __restrict__ src, lo
 // (large batches). WPI = DEC_WAVES: one workgroup per item for small batches, where 4 items per
 // workgroup leave most of the chip idle and each wave walks the whole context serially (one HBM
 // round trip per 32-token tile): wave 0 writes the new k/v row, every wave builds the Q fragments,
-// wave w takes the w-th quarter of the context's tiles, and the four partial (m, l, O) merge
+// wave w takes the w-th quarter of the context's tiles, and the partial (m, l, O) merge
 // through LDS (the V-tile rows are reused for the O partials).
 template <int SPL, int WPI, bool S16 = false>
 __global__ void __launch_bounds__(256, WPI > 1 ? 2 : 4) decode_attn_fused_kernel(
@@ -617,7 +630,7 @@ __global__ void __launch_bounds__(256, WPI > 1 ? 2 : 4) decode_attn_fused_kernel
   // the block-table window too: every load the tile loop's first tile waits on except the
   // new cache row is issued before the fence below
   int s_begin = 0, s_end = ctx;
-  if constexpr (WPI > 1) decode_wg_range<WPI>(ctx, wv, s_begin, s_end);
+  if constexpr (WPI > 1) decode_wg_range<WPI>(0, ctx, wv, s_begin, s_end);
   const int bt0 = decode_bt_window(block_tables, max_blocks, b, s_begin, s_end, block_size, lane);
   const int slot = slot_mapping[b];
   if (slot >= 0 && (WPI == 1 || wv == 0))
@@ -638,12 +651,14 @@ __global__ void __launch_bounds__(256, WPI > 1 ? 2 : 4) decode_attn_fused_kernel
   }
 }
 
-// Several KV splits per sequence, dealt as in decode_attn_kernel: the split that holds the new token
-// writes its cache row, the others do not read it. Against a kernel for the rotation and the cache write
-// and one for the attention: 1 context of 75 tokens 5.1 + 9.2 -> 11.0 us, 24 of 500 to 8000 5.5 + 55.3 ->
-// 54.1 (the query's sums run beside the first block-table and cache requests).
+// Several KV splits per sequence, dealt to workgroups from the step's contexts: a split's 4 waves merge
+// through LDS, so a context of up to 4 tiles is one split and its output, and a longer one leaves a
+// quarter of the partial results. SPL >= 0, fused: the wave with the new token writes its cache row, the
+// others do not read it; SPL < 0: src = the q rows (stride N), already rotated, the cache written.
+// With its reduce, from a wave a split: 1 context of 75 tokens 12.0 -> 8.1 us, 1 of 2000 14.2 -> 10.9, 16 of
+// 1000 22.6 -> 20.1, 32 of 2000 54.2 -> 52.5.
 template <int SPL, bool S16>
-__global__ void __launch_bounds__(256, 3) decode_attn_fused_split_kernel(
+__global__ void __launch_bounds__(256, 2) decode_attn_split_kernel(
     u16* __restrict__ out, const void* __restrict__ src, int N,
     const int* __restrict__ positions, const int* __restrict__ slot_mapping,
     const float* __restrict__ cos_sin, u16* __restrict__ k_cache, u16* __restrict__ v_cache,
@@ -652,31 +667,42 @@ __global__ void __launch_bounds__(256, 3) decode_attn_fused_split_kernel(
     float* __restrict__ ws_o, float* __restrict__ ws_ml) {
   constexpr int HD = 128, KK = HD / 32, VROW = HD + 16;
   __shared__ __attribute__((aligned(16))) u16 vtile_all[DEC_WAVES][DEC_TILE * VROW];
+  __shared__ float ml_all[DEC_WAVES][16][2];
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int item = blockIdx.x * DEC_WAVES + wv;
-  const int kvh = item % hkv;
-  const DecSplit sp = decode_split(context_lens, B, hkv, num_splits, item / hkv, lane);
-  if (sp.b < 0) return;                                        // wave-uniform exit
+  const int kvh = blockIdx.x % hkv;
+  const DecSplit sp = decode_split<DEC_WAVES>(context_lens, B, hkv, num_splits, blockIdx.x / hkv, lane);
+  if (sp.b < 0) return;                                        // workgroup-uniform exit
   const int b = sp.b, split = sp.split, G = hq / hkv;
   const int ctx = context_lens[b];
-  const int s_begin = split * sp.split_tokens;
-  const int s_end = min(ctx, s_begin + sp.split_tokens);
-  const float* cs = cos_sin + (long)positions[b] * HD;
-  const long rowoff = (long)b * N;
-  const long splitstride = (long)B * N;
+  const int from = split * sp.split_tokens;
+  int s_begin, s_end;
+  decode_wg_range<DEC_WAVES>(from, min(ctx, from + sp.split_tokens), wv, s_begin, s_end);
   const int bt0 = decode_bt_window(block_tables, max_blocks, b, s_begin, s_end, block_size, lane);
   bf16x8 qf[KK];
-  fused_query<SPL, S16>(qf, src, rowoff, splitstride, cs, kvh, G, lane);
-  const int slot = slot_mapping[b];
-  if (slot >= 0 && split == max(ctx - 1, 0) / sp.split_tokens) {
-    fused_cache_row<SPL, S16>(src, rowoff, splitstride, cs, slot, kvh, hq, hkv, block_size, k_cache,
-                              v_cache, lane);
-    __threadfence_block();                 // read back by other lanes of this wave
+  if constexpr (SPL < 0) {
+    const int col = lane & 15, grp = lane >> 4;
+    const u16* qp = static_cast<const u16*>(src) + (long)b * N + (long)(kvh * G + (col < G ? col : 0)) * HD;
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) {
+      uint4 v = col < G ? *reinterpret_cast<const uint4*>(qp + kk * 32 + grp * 8) : make_uint4(0, 0, 0, 0);
+      qf[kk] = *reinterpret_cast<bf16x8*>(&v);
+    }
+  } else {
+    const float* cs = cos_sin + (long)positions[b] * HD;
+    const long rowoff = (long)b * N;
+    const long splitstride = (long)B * N;
+    fused_query<SPL, S16>(qf, src, rowoff, splitstride, cs, kvh, G, lane);
+    const int slot = slot_mapping[b];
+    if (slot >= 0 && (ctx > 0 ? s_begin < ctx && s_end == ctx : wv == 0)) {
+      fused_cache_row<SPL, S16>(src, rowoff, splitstride, cs, slot, kvh, hq, hkv, block_size, k_cache,
+                                v_cache, lane);
+      __threadfence_block();               // read back by other lanes of this wave
+    }
   }
-  decode_attn_core<HD, true>(qf, vtile_all[wv], lane, b, kvh, split, G, ctx, s_begin, s_end, out, k_cache,
-                       v_cache, block_tables, max_blocks, hq, hkv, block_size, scale_log2,
-                       sp.last == 0 ? 1 : num_splits, ws_o, ws_ml, bt0);
-  decode_end_list(ws_ml, b, hq, kvh, G, num_splits, split, sp.last, lane);
+  decode_attn_wg<DEC_WAVES>(qf, vtile_all, ml_all, wv, lane, b, kvh, G, s_begin, s_end, bt0, out,
+                            k_cache, v_cache, block_tables, max_blocks, hq, hkv, block_size, scale_log2,
+                            sp.last == 0 ? 1 : num_splits, split, ws_o, ws_ml);
+  if (wv == 0) decode_end_list(ws_ml, b, hq, kvh, G, num_splits, split, sp.last, lane);
 }
 
 // Software-pipelined variant: a wave walks a list of work units (item = (sequence, kv head,
@@ -1045,24 +1071,23 @@ extern "C" int dli_decode_attention(void* out, const void* q, int q_stride, cons
     decode_attn_wg_kernel<<<(int)items, 64 * DEC_WAVES, 0, st>>>(
         (u16*)out, (const u16*)q, q_stride, (const u16*)k_cache, (const u16*)v_cache,
         block_tables, max_blocks, context_lens, B, hq, hkv, block_size, scale_log2);
+  } else if (hd == 128 && num_splits > 1) {
+    decode_attn_split_kernel<-1, false><<<(int)decode_split_items<DEC_WAVES>(B * hkv, num_splits), 256, 0, st>>>(
+        (u16*)out, q, q_stride, nullptr, nullptr, nullptr, (u16*)k_cache, (u16*)v_cache, block_tables,
+        max_blocks, context_lens, B, hq, hkv, block_size, scale_log2, num_splits, ws_o, ws_ml);
   } else {
-  const long listed = num_splits > 1 ? decode_split_items(B * hkv, num_splits) : items;
-  dim3 grid((int)((listed + DEC_WAVES - 1) / DEC_WAVES));
-  if (hd == 128 && num_splits > 1)
-    decode_attn_kernel<128, 3, true><<<grid, 64 * DEC_WAVES, 0, st>>>(
-        (u16*)out, (const u16*)q, q_stride, (const u16*)k_cache, (const u16*)v_cache,
-        block_tables, max_blocks, context_lens, B, hq, hkv, block_size, scale_log2, num_splits,
-        split_tokens, ws_o, ws_ml);
-  else if (hd == 128)
-    decode_attn_kernel<128, 4, false><<<grid, 64 * DEC_WAVES, 0, st>>>(
-        (u16*)out, (const u16*)q, q_stride, (const u16*)k_cache, (const u16*)v_cache,
-        block_tables, max_blocks, context_lens, B, hq, hkv, block_size, scale_log2, num_splits,
-        split_tokens, ws_o, ws_ml);
-  else
-    decode_attn_kernel<64, 1, true><<<grid, 64 * DEC_WAVES, 0, st>>>(
-        (u16*)out, (const u16*)q, q_stride, (const u16*)k_cache, (const u16*)v_cache,
-        block_tables, max_blocks, context_lens, B, hq, hkv, block_size, scale_log2, num_splits,
-        split_tokens, ws_o, ws_ml);
+    const long listed = num_splits > 1 ? decode_split_items<1>(B * hkv, num_splits) : items;
+    dim3 grid((int)((listed + DEC_WAVES - 1) / DEC_WAVES));
+    if (hd == 128)
+      decode_attn_kernel<128, 4, false><<<grid, 64 * DEC_WAVES, 0, st>>>(
+          (u16*)out, (const u16*)q, q_stride, (const u16*)k_cache, (const u16*)v_cache,
+          block_tables, max_blocks, context_lens, B, hq, hkv, block_size, scale_log2, num_splits,
+          split_tokens, ws_o, ws_ml);
+    else
+      decode_attn_kernel<64, 1, true><<<grid, 64 * DEC_WAVES, 0, st>>>(
+          (u16*)out, (const u16*)q, q_stride, (const u16*)k_cache, (const u16*)v_cache,
+          block_tables, max_blocks, context_lens, B, hq, hkv, block_size, scale_log2, num_splits,
+          split_tokens, ws_o, ws_ml);
   }
   if (num_splits > 1) {
     const int blocks = (int)(((long)B * hq + 3) / 4);
@@ -1096,9 +1121,8 @@ extern "C" int dli_decode_attention_fused(void* out, const void* ws, int splits,
   if (num_splits > 1) {
     float* ws_o = (float*)workspace;
     float* ws_ml = ws_o + (long)B * hq * num_splits * hd;
-    const long listed = decode_split_items(B * hkv, num_splits);
-    const dim3 gs((int)((listed + DEC_WAVES - 1) / DEC_WAVES));
-#define DLI_DAS(S, F) decode_attn_fused_split_kernel<S, F><<<gs, 64 * DEC_WAVES, 0, st>>>(     \
+    const dim3 gs((int)decode_split_items<DEC_WAVES>(B * hkv, num_splits));
+#define DLI_DAS(S, F) decode_attn_split_kernel<S, F><<<gs, 64 * DEC_WAVES, 0, st>>>(     \
       (u16*)out, ws, N, positions, slot_mapping, cos_sin, (u16*)k_cache, (u16*)v_cache,      \
       block_tables, max_blocks, context_lens, B, hq, hkv, block_size, scale_log2, num_splits,  \
       ws_o, ws_ml)

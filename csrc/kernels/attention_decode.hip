@@ -65,6 +65,11 @@ __device__ __forceinline__ void decode_wg_range(int from, int to, int wv, int& s
 // more than num_splits. Sequence b has max(1, ceil(context / split_tokens)) equal ones, listed sequence
 // by sequence: `pair` of that list is (b, split); b = -1 past its end. Every wave works this out for
 // itself: a few loads and scans.
+// A workgroup's split keeps 3 of a CU's 4 slots: about 768 run at once, half of one more a sequence and
+// head is rounding (24 of 500 - 8000: 57.9 us dealt to 768 and the rounding up, 960 at most; 52.6 so).
+template <int W> __host__ __device__ static inline int decode_ragged_units(int items) {
+  return W == 1 ? DEC_TARGET : items < 768 ? 768 - items / 2 : 384;
+}
 template <int W> __host__ __device__ static inline int decode_even_splits(int items) {
   int n = 1;
   while ((long)items * n < 2048 / W) n *= 2;
@@ -102,7 +107,7 @@ __device__ __forceinline__ DecSplit decode_split(const int* __restrict__ context
   longest = __builtin_amdgcn_readlane(wave_scan<true>(longest), 63);
   const int even = decode_even_splits<W>(B * hkv);
   const int share = 4l * sum >= 3l * longest * B ? (longest + even - 1) / even
-                                                 : (sum * hkv + DEC_TARGET / W - 1) / (DEC_TARGET / W);
+                                                 : (sum * hkv + decode_ragged_units<W>(B * hkv) - 1) / decode_ragged_units<W>(B * hkv);
   const int per = max(max(share, (longest + num_splits - 1) / num_splits), max(W, DEC_MIN_TILES));
   DecSplit r{-1, 0, per * DEC_TILE, 0};
   const auto find = [&](int i0, int c) {
@@ -132,7 +137,7 @@ __device__ __forceinline__ DecSplit decode_split(const int* __restrict__ context
 // units a split launch needs at most: the even splits, or DEC_TARGET and the rounding up of every
 // sequence
 template <int W> static inline long decode_split_items(int items, int num_splits) {
-  const long even = (long)items * decode_even_splits<W>(items), ragged = DEC_TARGET / W + items;
+  const long even = (long)items * decode_even_splits<W>(items), ragged = decode_ragged_units<W>(items) + items;
   const long all = (long)items * num_splits, most = even > ragged ? even : ragged;
   return all < most ? all : most;
 }

@@ -264,7 +264,10 @@ def _heuristic(M: int, N: int, K: int, epi: str) -> GemmPlan:
             pays = K > 2048 or (K >= 1024 and tiles > NUM_CUS) or N % 64 != 0   # (tile 22 takes no such N)
         else:
             pays = epi not in ("bias", "bias_gelu")
-        if (pays and splits == 1 and M >= LARGE_M and K % 128 == 0 and (K <= 8192 or M < 4096)
+        # (long K from 4096 rows on where its narrower tiles save part of a round: 4352 x 4096, K = 14336
+        # 402 us against 560)
+        if (pays and splits == 1 and M >= LARGE_M and K % 128 == 0
+                and (K <= 8192 or M < 4096 or persistent_width(M, N, epi in PAIR_EPIS) < 256)
                 and (M < 16384 or N >= 16384) and tile_ok(55, epi)):
             return GemmPlan("dli", 55, 1)
         return GemmPlan("dli", 22, splits)
@@ -437,6 +440,24 @@ def plan(M: int, N: int, K: int, epi: str) -> GemmPlan:
     # tuned and pinned plans by bucket; a fitted one by its own M (a bucket of prefill sizes spans a
     # factor of two, in which the best split differs)
     return _plan_cache.get(key) or _heuristic(M, N, K, epi)
+
+
+@functools.lru_cache(maxsize=8192)
+def persistent_width(M: int, N: int, pairs: bool) -> int:
+    """Columns of the tiles that the persistent kernel (tile 55) takes: gemm4wp.hip's width_of."""
+    best, least = 256, 0.0
+    for nj, price in ((8, 1.0), (6, 1.09 * 6 / 8), (5, 1.13 * 5 / 8)):
+        if pairs and nj & 1:
+            continue
+        whole, rest = divmod(-(-M // 256) * -(-N // (32 * nj)), NUM_CUS)
+        x = rest / NUM_CUS
+        last = 0.0 if not rest else 0.66 + 0.25 * x + 0.09 * x ** 3 if whole else 0.8 + 0.2 * x ** 3
+        c = (whole + last) * price
+        if nj == 8:
+            least = 0.97 * c
+        elif c < least:
+            best, least = 32 * nj, c
+    return best
 
 
 @functools.lru_cache(maxsize=8192)

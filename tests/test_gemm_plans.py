@@ -78,3 +78,35 @@ def test_products_on_fitted_plans(gpu, M, N, K, epi):
     got = ops.linear(x, w, bias, epi=epi)
     assert got.shape == want.shape and got.dtype == (torch.float32 if epi == "f32" else torch.bfloat16)
     assert float((got.double() - want).norm() / want.norm()) < (1e-5 if epi == "f32" else 2.0 ** -8)
+
+
+@pytest.mark.gpu
+def test_persistent_tile_widths_are_the_kernels(gpu):
+    from distributed_llm_inferencing_amd.ops import _native
+    width = _native.require_native().dli_gemm_persistent_width
+    for M in (1, 256, 257, 1290, 2112, 2816, 4352, 5000, 8199):
+        for N in (32, 160, 4096, 4100, 6144, 14336, 28672):
+            for pairs in (False, True):
+                assert G.persistent_width(M, N, pairs) == width(M, N, int(pairs)), (M, N, pairs)
+
+
+# every width of the persistent kernel's tiles, with partial tiles in both directions, two to twenty K-tiles and
+# one to three tiles a workgroup; tolerances as above
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,epi,width", [
+    (1290, 4100, 128, "f32", 160), (2300, 4090, 640, "none", 160), (4300, 4096, 256, "f32", 160), (300, 1000, 1280, "f32", 160),
+    (2810, 4104, 384, "f32", 192), (5000, 4096, 128, "none", 192), (900, 10400, 256, "f32", 192), (1270, 28672, 128, "silu_mul", 192),
+    (1270, 28704, 256, "gelu_mul", 192), (9216, 4096, 128, "f32", 256), (300, 1024, 128, "silu_mul", 192)])
+def test_persistent_tiles_of_every_width(gpu, M, N, K, epi, width):
+    pairs = epi in G.PAIR_EPIS
+    assert G.persistent_width(M, N, pairs) == width
+    g = torch.Generator(device=gpu).manual_seed(M + N)
+    x, w = (torch.randn(r, K, device=gpu, generator=g).bfloat16() for r in (M, N))
+    w = w * K ** -0.5
+    want = x.double() @ w.double().t()
+    if pairs:
+        gate, up = want.view(M, N // 32, 2, 16).unbind(2)
+        act = torch.nn.functional.silu(gate) if epi == "silu_mul" else torch.nn.functional.gelu(gate, approximate="tanh")
+        want = (act * up).reshape(M, N // 2)
+    got = ops._gemm_native(x, w, epi, plan=G.GemmPlan("dli", 55, 1)).double()
+    assert float((got - want).norm() / want.norm()) < (1e-5 if epi == "f32" else 2.0 ** -8)

@@ -7,7 +7,10 @@
 //                      xs[r] = sum_s mix[s][r] xs[s] + write[r] * y          (all r at once)
 //                  and with the next sublayer's read weights the row u = sum_s read[s] xs[s]
 //                  leaves RMS-normed times (w + w_offset) as S, or as it is in fp32 (w null).
-//                  One launch does a sublayer's write-back and the next one's read + norm.
+//                  One launch does a sublayer's write-back and the next one's read + norm. Two
+//                  finished sublayers may be handed over at once: the first one's write-back is
+//                  then formed again on the way instead of having been stored. The streams may
+//                  come from another array than they go to, also from one row for all of them.
 //  * sink_prepare  q / k RMS-normed over their whole rows (all heads at once) with a weight
 //                  per column, the first rot_dims dims of every head rotated (dimension i with
 //                  i + rot_dims/2; angle = position * freq[i] formed in double; cos and sin
@@ -31,11 +34,16 @@ constexpr int MAXS = 8;          // streams
 // split-K product: the launch and the pass of its reduce are spared. The coefficients are the same
 // for the whole launch: read as scalars, beside the rows' requests and without a barrier before them.
 // Decode step, 64 rows of 3 x 4096: 7.5 us with a reduce launch of 5.4 before it -> 6.2. Prefill is bound
-// by memory: 8199 rows 173 us, 1.0 GB at 5.8 TB/s.
+// by memory: 8199 rows 199 us with the streams stored, 126 without, 5.1 and 4.8 TB/s; two mixes of which
+// one stores 397 -> 350 us.
+// y0 / prev0 (nullable): the sublayer before y's, whose write-back was not stored (xs null then).
+// src: the streams' rows, src_row floats a token and src_stream a stream (0: one row for all).
 template <typename S, int VEC, int NS>
 __global__ void __launch_bounds__(1024) hyper_mix_kernel(
-    float* __restrict__ xs, const float* __restrict__ y, int ldy, int nsplit, long ysplit,
-    const float* __restrict__ prev, const float* __restrict__ read, const S* __restrict__ w,
+    const float* src, long src_row, long src_stream, float* xs,
+    const float* __restrict__ y0, const float* __restrict__ prev0, const float* __restrict__ y,
+    int ldy, int nsplit, long ysplit, const float* __restrict__ prev,
+    const float* __restrict__ read, const S* __restrict__ w,
     void* __restrict__ h, int ns_any, int dim, float eps, float w_offset) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
   constexpr int MS = NS ? NS : MAXS;
@@ -43,9 +51,8 @@ __global__ void __launch_bounds__(1024) hyper_mix_kernel(
   float* urow = sm;                        // [dim]
   float* red = urow + dim;                 // [16]
   const int t = blockIdx.x;
-  float* xr = xs + (long)t * ns * dim;
-  const float* wr = prev + ns;             // write weights
-  const float* mix = prev + 2 * ns;        // [from][to]
+  const float* xi = src + t * src_row;
+  float* xo = xs == nullptr ? nullptr : xs + (long)t * ns * dim;
   float ss = 0.f;
   for (int c = threadIdx.x * VEC; c < dim; c += blockDim.x * VEC) {
     float x[MS][VEC];
@@ -53,16 +60,47 @@ __global__ void __launch_bounds__(1024) hyper_mix_kernel(
     for (int s = 0; s < MS; ++s) {
       if (s < ns) {
         if (VEC == 4) {
-          const f32x4 v = *reinterpret_cast<const f32x4*>(xr + (long)s * dim + c);
+          const f32x4 v = *reinterpret_cast<const f32x4*>(xi + s * src_stream + c);
 #pragma unroll
           for (int u = 0; u < VEC; ++u) x[s][u] = v[u];
         } else {
-          x[s][0] = xr[(long)s * dim + c];
+          x[s][0] = xi[s * src_stream + c];
         }
       }
     }
+    // x <- the streams mixed by a sublayer's vector, plus its output (the same sums whether they
+    // are formed once and stored or formed again)
+    const auto write_back = [&](const float* vec, const float (&yv)[VEC]) {
+      const float* wr = vec + ns;          // write weights
+      const float* mix = vec + 2 * ns;     // [from][to]
+      float nx[MS][VEC];
+#pragma unroll
+      for (int r = 0; r < MS; ++r)
+        if (r < ns) {
+#pragma unroll
+          for (int u = 0; u < VEC; ++u) {
+            float acc = 0.f;
+#pragma unroll
+            for (int s = 0; s < MS; ++s)
+              if (s < ns) acc += mix[s * ns + r] * x[s][u];
+            nx[r][u] = acc + wr[r] * yv[u];
+          }
+        }
+#pragma unroll
+      for (int r = 0; r < MS; ++r)
+        if (r < ns) {
+#pragma unroll
+          for (int u = 0; u < VEC; ++u) x[r][u] = nx[r][u];
+        }
+    };
+    if (y0 != nullptr) {
+      float yv[VEC];
+#pragma unroll
+      for (int u = 0; u < VEC; ++u) yv[u] = y0[(long)t * dim + c + u];
+      write_back(prev0, yv);
+    }
     if (y != nullptr) {
-      float yv[VEC], nx[MS][VEC];
+      float yv[VEC];
       const float* yr = y + (long)t * ldy + c;
       if constexpr (VEC == 4) {
         f32x4 v = *reinterpret_cast<const f32x4*>(yr);
@@ -73,29 +111,17 @@ __global__ void __launch_bounds__(1024) hyper_mix_kernel(
         yv[0] = yr[0];
         for (int s = 1; s < nsplit; ++s) yv[0] += yr[s * ysplit];
       }
-#pragma unroll
-      for (int r = 0; r < MS; ++r) {
-        if (r < ns) {
-#pragma unroll
-          for (int u = 0; u < VEC; ++u) {
-            float acc = 0.f;
-#pragma unroll
-            for (int s = 0; s < MS; ++s)
-              if (s < ns) acc += mix[s * ns + r] * x[s][u];
-            nx[r][u] = acc + wr[r] * yv[u];
-          }
-          if (VEC == 4)
-            *reinterpret_cast<f32x4*>(xr + (long)r * dim + c) =
-                f32x4{nx[r][0], nx[r][VEC > 1 ? 1 : 0], nx[r][VEC > 2 ? 2 : 0], nx[r][VEC > 3 ? 3 : 0]};
-          else
-            xr[(long)r * dim + c] = nx[r][0];
-        }
-      }
+      write_back(prev, yv);
+    }
+    if (xo != nullptr) {
 #pragma unroll
       for (int r = 0; r < MS; ++r)
         if (r < ns) {
-#pragma unroll
-          for (int u = 0; u < VEC; ++u) x[r][u] = nx[r][u];
+          if (VEC == 4)
+            *reinterpret_cast<f32x4*>(xo + (long)r * dim + c) =
+                f32x4{x[r][0], x[r][VEC > 1 ? 1 : 0], x[r][VEC > 2 ? 2 : 0], x[r][VEC > 3 ? 3 : 0]};
+          else
+            xo[(long)r * dim + c] = x[r][0];
         }
     }
     if (read != nullptr) {
@@ -248,22 +274,30 @@ __global__ void __launch_bounds__(1024) sink_prepare4_kernel(
     else return (int)hipErrorInvalidValue;        \
   } while (0)
 
-// y: nsplit slabs, ysplit elements apart, whose sum is the sublayer's output (1: the output itself)
-extern "C" int dli_hyper_mix(float* xs, const float* y, int ldy, int nsplit, long ysplit,
+// src: the streams' rows ([T, ns, dim], or with one_row [T, dim] read as every stream); xs: where the
+// new streams go (src itself, another array, or null: not stored). y0 (contiguous) with prev0: a
+// finished sublayer whose write-back is not in src yet; y with prev: the one after it, nsplit slabs,
+// ysplit elements apart, whose sum is its output (1: the output itself).
+extern "C" int dli_hyper_mix(const float* src, int one_row, float* xs, const float* y0,
+                             const float* prev0, const float* y, int ldy, int nsplit, long ysplit,
                              const float* prev, const float* read, const void* w, void* h, int T,
                              int ns, int dim, float eps, float w_offset, int dt, hipStream_t st) {
   if (T <= 0) return 0;
   if (ns < 1 || ns > MAXS || dim < 1 || (y != nullptr) != (prev != nullptr) || nsplit < 1 ||
-      (read != nullptr && h == nullptr) || (read == nullptr && y == nullptr))
+      (y0 != nullptr) != (prev0 != nullptr) || src == nullptr || (one_row && src == xs) ||
+      (read != nullptr && h == nullptr) || (read == nullptr && xs == nullptr))
     return (int)hipErrorInvalidValue;
   const size_t sh = ((size_t)dim + 16) * 4;
   if (sh > 60000) return (int)hipErrorInvalidValue;
-  const bool v4 = dim % 4 == 0 && (uintptr_t)xs % 16 == 0 &&
-                  (y == nullptr || ((uintptr_t)y % 16 == 0 && ldy % 4 == 0 && ysplit % 4 == 0));
+  const bool v4 = dim % 4 == 0 &&
+                  (((uintptr_t)src | (uintptr_t)xs | (uintptr_t)y0 | (uintptr_t)y) & 15) == 0 &&
+                  (y == nullptr || (ldy % 4 == 0 && ysplit % 4 == 0));
   const int nt = (T <= 1024 && dim >= 2048) ? 1024 : 256;
+  const long row = one_row ? dim : (long)ns * dim, stream = one_row ? 0 : dim;
 #define HM_LAUNCH(S, V, N)                                                                    \
-  hyper_mix_kernel<S, V, N><<<T, nt, sh, st>>>(xs, y, ldy, nsplit, ysplit, prev, read,         \
-                                               (const S*)w, h, ns, dim, eps, w_offset)
+  hyper_mix_kernel<S, V, N><<<T, nt, sh, st>>>(src, row, stream, xs, y0, prev0, y, ldy, nsplit, \
+                                               ysplit, prev, read, (const S*)w, h, ns, dim, eps, \
+                                               w_offset)
 #define HM_STREAMS(S)                                                                         \
   (ns == 2 ? (void)HM_LAUNCH(S, 4, 2) : ns == 3 ? (void)HM_LAUNCH(S, 4, 3)                     \
    : ns == 4 ? (void)HM_LAUNCH(S, 4, 4) : (void)HM_LAUNCH(S, 4, 0))

@@ -180,19 +180,39 @@ class HybridLM(TransformerLM):
         eps, off, S = cfg.norm_eps, cfg.norm_offset, cfg.streams
         step = self._step_view(b, kv_caches.block_size)
         T, D = x.shape
-        xs = x.unsqueeze(1).expand(T, S, D).contiguous()
+        # The streams are all equal at first: read from x until they are stored. Of two write-backs
+        # one is stored: ``held`` is the sublayer whose write-back the next mix forms again (two
+        # mixes of 8199 rows of 3 x 4096: 397 -> 350 us, of 512 rows 30 -> 28, of 64 equal). Partial
+        # sums are gone after the next GEMM: theirs is stored.
+        xs, source, held = (T, S, D), x, None
         y = prev = None                     # a sublayer's output awaiting its write-back
+
+        def mix(read, norm, last=False):
+            nonlocal xs, source, held
+            out = H.rows_of(y) if not isinstance(y, (torch.Tensor, type(None))) else y
+            defer = (out is not None and held is None and not last
+                     and out.dim() == 2 and out.is_contiguous())
+            store = out is not None and not last and not defer
+            if store and isinstance(xs, tuple):
+                xs = torch.empty(T, S, D, dtype=torch.float32, device=x.device)
+            h = H.hyper_mix(xs, out, prev, read, norm, eps, off, before=held, source=source,
+                            store=store)
+            if not last:                    # a sum alone leaves what awaits its write-back
+                held = (out, prev) if defer else None
+            if store:
+                source = None
+            return h
+
         for ri, (li, _, _) in enumerate(self.runs):
             spec, lp = cfg.layer_specs[li], self.layers[li]
-            h = H.hyper_mix(xs, y, prev, lp["hc1"], lp["norm1"], eps, off)
+            h = mix(lp["hc1"], lp["norm1"])
             y, prev = MIXERS[spec.kind](spec, lp, h, step, kv_caches.entries[ri], eps), lp["hc1"]
             if spec.ff:
-                h = H.hyper_mix(xs, y, prev, lp["hc2"], lp["norm2"], eps, off)
+                h = mix(lp["hc2"], lp["norm2"])
                 y, prev = FEED_FORWARDS[spec.ff_kind](spec, lp, h), lp["hc2"]
             if self.layer_trace is not None:
-                self.layer_trace.append(H.hyper_mix(xs, y, prev, self._sum_streams, None))
-                y = prev = None
-        return H.hyper_mix(xs, y, prev, self._sum_streams, None)
+                self.layer_trace.append(mix(self._sum_streams, None, last=True))
+        return mix(self._sum_streams, None, last=True)
 
     def _sandwich_layers(self, x: torch.Tensor, b: DeviceBatch, kv_caches) -> torch.Tensor:
         """Layers with a norm before and after every sublayer."""

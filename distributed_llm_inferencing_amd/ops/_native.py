@@ -110,7 +110,7 @@ _SIGS = {
     "dli_head_gate": [P, P, P, I, I, I, I, I, P],
     "dli_logit_router": [P, P, P, I, P, P, I, I, I, I, I, P],
     # hyper-connected designs (streams.hip, recurrent_scalar.hip)
-    "dli_hyper_mix": [P, P, I, I, L, P, P, P, P, I, I, I, F, F, I, P],
+    "dli_hyper_mix": [P, I, P, P, P, P, I, I, L, P, P, P, P, I, I, I, F, F, I, P],
     "dli_sink_prepare": [P, I, P, P, F, I, I, I, I, I, I, P, F, P, P, P, P, P, I, P],
     "dli_scalar_recurrence": [P, I, I, P, P, F, P, F, P, P, P, P, P, P, I, F, I, I, I, I, I, I,
                               I, I, P, I, P],

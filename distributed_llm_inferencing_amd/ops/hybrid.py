@@ -898,23 +898,42 @@ def moe_gelu_experts_f32(x, w_up, w_down, topk_w, topk_ids, shared=None) -> torc
 
 
 # ----------------------------------------------------------------------------- hyper-connected designs
-def hyper_mix(xs, y, prev, read, w, eps: float = 0.0, w_offset: float = 0.0, dtype=None):
+def hyper_mix(xs, y, prev, read, w, eps: float = 0.0, w_offset: float = 0.0, dtype=None,
+              before=None, source=None, store: bool = True):
     """One step of hyper-connections on the fp32 streams xs [T, S, D], in place
     (``reference.hyper_mix``): with y (a sublayer's fp32 output) and ``prev`` (that sublayer's
     fp32 vector read | write | mix) the streams are mixed and receive y (or, of a GEMM's partial sums,
     see ``linear_out``, their sum); with ``read`` (the next
     sublayer's vector, or ones for the plain sum) the weighted sum of the new streams is
-    returned — RMS-normed times (w + w_offset) in the storage dtype when w is given, else fp32."""
+    returned — RMS-normed times (w + w_offset) in the storage dtype when w is given, else fp32.
+
+    ``before`` (y, prev): a sublayer before y's whose write-back xs still lacks. ``source`` fp32
+    [T, D]: read as every stream in place of xs. ``store`` False: xs stays as it is (and may be the
+    shape alone, when nothing of it is read)."""
     if not isinstance(y, (torch.Tensor, type(None))):
         y = rows_of(y)
-    if not xs.is_cuda:
-        return R.hyper_mix(xs, y, prev, read, w, eps, w_offset, dtype or (w.dtype if w is not None else None))
-    T, S, D = xs.shape
+    keeps = isinstance(xs, tuple)                    # a shape: nothing to store to
+    T, S, D = xs if keeps else xs.shape
+    if keeps and (store or source is None):
+        raise ValueError("hyper_mix needs the streams to read or to store")
+    ref = source if source is not None else xs
+    y0, prev0 = before or (None, None)
+    if not ref.is_cuda:
+        new = source.unsqueeze(1).repeat(1, S, 1) if source is not None else xs if store else xs.clone()
+        if before is not None:
+            R.hyper_mix(new, y0, prev0, None, None, eps, w_offset, None)
+        h = R.hyper_mix(new, y, prev, read, w, eps, w_offset, dtype or (w.dtype if w is not None else None))
+        if store and new is not xs:
+            xs.copy_(new)
+        return h
     h = None
     if read is not None:
-        h = torch.empty(T, D, dtype=torch.float32 if w is None else w.dtype, device=xs.device)
-    _call("dli_hyper_mix", _p(xs), _p(y), *slabs_of(y), _p(prev), _p(read), _p(w), _p(h), T, S, D, float(eps), float(w_offset),
-          _dt(w.dtype) if w is not None else 1, _st())
+        h = torch.empty(T, D, dtype=torch.float32 if w is None else w.dtype, device=ref.device)
+    # nothing to write back: the streams are what they were
+    stores = store and (source is not None or y is not None or before is not None)
+    _call("dli_hyper_mix", _p(ref), int(source is not None), _p(xs) if stores else None, _p(y0),
+          _p(prev0), _p(y), *slabs_of(y), _p(prev), _p(read), _p(w), _p(h), T, S, D, float(eps),
+          float(w_offset), _dt(w.dtype) if w is not None else 1, _st())
     return h
 
 

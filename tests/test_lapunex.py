@@ -204,6 +204,33 @@ def test_stream_mix_read_and_norm(device, dtype, S, D):
     np.testing.assert_allclose(xt.cpu().numpy(), new, atol=2e-5, rtol=2e-5)
 
 
+# streams read from one row, write-backs held and formed again, streams left as they are: the same
+# bits as one after the other (the same sums of the same numbers; the CPU path's einsum as well)
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("S,D", [(1, 64), (2, 30), (3, 4096), (4, 64), (8, 36)])
+def test_held_write_back(device, S, D):
+    rng = np.random.default_rng(S + D)
+    T, n = 5, S * (S + 2)
+    x, y1, y2 = (dev_t(rng.standard_normal((T, D)), device) for _ in range(3))
+    v = [dev_t(rng.standard_normal(n) * 0.5, device) for _ in range(3)]
+    w = dev_t(rng.standard_normal(D), device)
+    step = x.unsqueeze(1).repeat(1, S, 1)
+    h = [H.hyper_mix(step, None, None, v[0], w, 1e-5), H.hyper_mix(step, y1, v[0], v[1], w, 1e-5),
+         H.hyper_mix(step, y2, v[1], v[2], w, 1e-5)]
+    xs = torch.full((T, S, D), 7.0, device=x.device)
+    got = [H.hyper_mix((T, S, D), None, None, v[0], w, 1e-5, source=x, store=False),
+           H.hyper_mix((T, S, D), y1, v[0], v[1], w, 1e-5, source=x, store=False),
+           H.hyper_mix(xs, y2, v[1], v[2], w, 1e-5, before=(y1, v[0]), source=x)]
+    for a, b in zip(got, h):
+        assert torch.equal(a, b)
+    assert torch.equal(xs, step)
+    left = xs.clone()
+    a = H.hyper_mix(xs, y1, v[2], v[0], None, store=False)
+    assert torch.equal(xs, left) and torch.equal(a, H.hyper_mix(step, y1, v[2], v[0], None))
+    with pytest.raises(ValueError):
+        H.hyper_mix((T, S, D), y1, v[0], v[1], w, 1e-5)
+
+
 def test_yarn_frequencies_follow_their_definition():
     from distributed_llm_inferencing_amd.models.mixers import yarn_frequencies
     for r in (rot(), rot(16, 10000.0, (6.0, 1024, 24.0, 2.0)), rot(6, 7.0, None),

@@ -682,11 +682,26 @@ __global__ void __launch_bounds__(256) swa_reduce_kernel(SwaArgs a, int S) {
 int decode_splits(int num_seqs, int H, int G, long keys) {
   const int rep = H / G, hp = rep <= 4 ? 4 : 8;
   const long base = (long)num_seqs * G * ((rep + hp - 1) / hp);
-  long n = (1536 + base - 1) / base;
-  const long most = (keys + 127) / 128;            // a tile for each wave of a workgroup
-  n = n > most ? most : n;
-  n = n > 32 ? 32 : n;
-  return n < 1 ? 1 : (int)n;
+  const long keys_most = (keys + 127) / 128;       // a tile for each wave of a workgroup
+  const int most = (int)(keys_most > 32 ? 32 : keys_most);
+  // 256 units and more: to 1536 workgroups, so that long contexts among short ones are cut (contexts of
+  // 64 to 2000 keys, 32 heads on 8: 32 sequences 45 us with 6 splits, 56 whole; 64 77 with 3, 84 whole).
+  // Fewer: a CU's time goes with the keys that its workgroups read, so what counts is how evenly 512
+  // workgroups or more fill 256 CUs: ceil(base n / 256) / n of a sequence for the fullest, and 0.004 of
+  // one for every split's share of the merge. With 1536 before; us, 8 sequences of 4000 keys 53 -> 39,
+  // 16 of 2000 44 -> 36, 24 of 2000 53 -> 48; 8 of 64 to 4000 45 -> 35, 24 of 64 to 2000 40 -> 34.
+  if (base >= 256) {
+    const long n = (1536 + base - 1) / base;
+    return n > most ? most : (int)n;
+  }
+  int best = (int)((512 + base - 1) / base);
+  if (best >= most) return most < 1 ? 1 : most;
+  float least = 1e30f;
+  for (int n = best; n <= most && base * n <= 1536; ++n) {
+    const float cost = (float)((base * n + 255) / 256) / (float)n + 0.004f * (float)n;
+    if (cost < least) { least = cost; best = n; }
+  }
+  return best;
 }
 
 // key / value widths this file is built for

@@ -254,7 +254,7 @@ __global__ void __launch_bounds__(512) prefill_attn32_kernel(
     const int* __restrict__ cu_seqlens, int hq, int hkv, float scale_log2,
     const int* __restrict__ ctx_lens, const u16* __restrict__ k_cache,
     const u16* __restrict__ v_cache, const int* __restrict__ block_tables, int bt_stride,
-    int block_size) {
+    int block_size, bool paired) {
   static_assert(HD == 128, "long-sequence kernel: head_dim 128");
   constexpr int KC = HD / 16;                      // K-steps of the QK^T product
   constexpr int DBK = HD / 32;                     // 32-wide d blocks of O^T
@@ -280,9 +280,17 @@ __global__ void __launch_bounds__(512) prefill_attn32_kernel(
   if (blk >= nblk) return;                                       // workgroup-uniform
   const int nkeys = PAGED ? ctx_lens[seq] : len;
   const int qoff = nkeys - len;
-  const int wg_q0 = blk * PL_ROWS;
-  const int q0 = wg_q0 + wid * PL_QROWS;                         // this wave's first row
-  const bool active = q0 < len;
+  // Up to a workgroup for each CU there is nothing to even out the causal bounds with, and the last
+  // block's workgroup, which sees most keys, takes as long as the launch. Paired, waves 0 to 3 take a
+  // half block counted from the end and waves 4 to 7 its counterpart from the start: a SIMD, which
+  // holds one wave of each, has the long one to itself when the short one is through. 32 heads, us:
+  // 2048 tokens 78 -> 66, 1024 45 -> 40, the second 2048 of a prompt 150 -> 135, 1024 after 5000 192 -> 185.
+  // With more workgroups the longest first do it at full width: 3000 tokens 105, paired 129.
+  const int nhalf = (len + PL_ROWS / 2 - 1) / (PL_ROWS / 2), back = nhalf - 1 - (nblk - 1 - blk);
+  const int half = wid < 4 ? back : nhalf - 1 - back;
+  const int q0 = paired ? half * (PL_ROWS / 2) + (wid & 3) * PL_QROWS
+                        : blk * PL_ROWS + wid * PL_QROWS;        // this wave's first row
+  const bool active = q0 < len && (!paired || wid < 4 || half != back);
   const u16* kbase = qkv + (long)(hq + kvh) * HD;
   const u16* vbase = qkv + (long)(hq + hkv + kvh) * HD;
   const int* btab = PAGED ? block_tables + (long)seq * bt_stride : nullptr;
@@ -301,7 +309,8 @@ __global__ void __launch_bounds__(512) prefill_attn32_kernel(
   }
   const int qpos = qoff + q0 + qc;                 // position of this lane's query
   const int wq_lo = qoff + q0, wq_hi = qoff + min(q0 + PL_QROWS, len) - 1;
-  const int kend_wg = min(nkeys, qoff + min(wg_q0 + PL_ROWS, len));
+  const int wg_end = paired ? (back + 1) * (PL_ROWS / 2) : (blk + 1) * PL_ROWS;
+  const int kend_wg = min(nkeys, qoff + min(wg_end, len));
   const int ntiles = (kend_wg + PL_KT - 1) / PL_KT;
 
   f32x16 o[DBK];
@@ -487,7 +496,8 @@ static int launch_prefill(void* out, int out_stride, const void* qkv, int row_st
     const dim3 grid32 = hq <= 4 ? dim3(blocks, num_seqs, hq) : dim3(blocks * hq, num_seqs);
     prefill_attn32_kernel<128, PAGED><<<grid32, 512, 0, st>>>(
         (u16*)out, out_stride, (const u16*)qkv, row_stride, cu_seqlens, hq, hkv, sl2, ctx_lens,
-        (const u16*)k_cache, (const u16*)v_cache, block_tables, bt_stride, block_size);
+        (const u16*)k_cache, (const u16*)v_cache, block_tables, bt_stride, block_size,
+        (long)blocks * hq * num_seqs <= 256);
     DLI_RETURN_LAUNCH();
   }
   // waves per query head: pack 2 / 4 heads of one GQA group into a workgroup for short

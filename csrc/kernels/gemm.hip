@@ -88,6 +88,7 @@ extern "C" int dli_gemm(const void* A, int lda, const void* W, int ldw, void* C,
   if (epi == EPI_CLAMP && (bias == nullptr || group_off != nullptr)) return (int)hipErrorInvalidValue;
   if (splits > 1 && ws == nullptr) return (int)hipErrorInvalidValue;
   if (groups < 1) groups = 1;
+  if (epi == EPI_F32) bias = nullptr;              // (where the block maxima go: dli_gemm_head)
   const int* go = group_off;
   int r = gemm_tiles_dispatch(epi, tile_cfg, DLI_GEMM_PASS);
   if (r == DLI_NOT_MINE) r = gemm_stream_dispatch(epi, tile_cfg, DLI_GEMM_PASS);
@@ -96,4 +97,39 @@ extern "C" int dli_gemm(const void* A, int lda, const void* W, int ldw, void* C,
   if (r == DLI_NOT_MINE) r = gemm_4wp_dispatch(epi, tile_cfg, DLI_GEMM_PASS);
   if (r == DLI_NOT_MINE) r = gemm_gemv_dispatch(epi, tile_cfg, DLI_GEMM_PASS);
   return r == DLI_NOT_MINE ? (int)hipErrorInvalidValue : r;
+}
+
+extern "C" int dli_gemm_persistent_width(int M, int N, int pairs);
+
+// columns of the blocks whose maxima dli_gemm_head can write for a tile; 0: not for this one
+static int head_block(int tile_cfg, int M, int N) {
+  if (N % 4) return 0;
+  if (tile_cfg == 55) return dli_gemm_persistent_width(M, N, 0) / 2;
+  if (tile_cfg == 30 || tile_cfg == 32) return M <= 4 ? 16 : 0;
+  if (tile_cfg == 31 || tile_cfg == 33) return M <= 4 ? 32 : 0;
+  switch (tile_cfg) {                              // columns of a wave tile
+    case 60: case 66: return 32;
+    case 61: case 63: case 67: case 68: return 64;
+    case 62: case 64: case 69: case 70: case 71: case 72: return 32;
+    case 65: return 128;
+    default: return 0;
+  }
+}
+extern "C" int dli_gemm_head_block(int tile_cfg, int M, int N) { return head_block(tile_cfg, M, N); }
+
+// C = A W^T in fp32 and, in keys [M, ceil(N / block)], each row's largest value by blocks of
+// dli_gemm_head_block columns (BlockMax). Unsplit; the tiles with a block only.
+extern "C" int dli_gemm_head(const void* A, int lda, const void* W, int ldw, void* C, int ldc, int M,
+                             int N, int K, int tile_cfg, void* keys, hipStream_t st) {
+  if (M <= 0 || N <= 0) return 0;
+  if (((tile_cfg < 29 || tile_cfg > 33) && K % BK) || lda % 8 || ldw % 8 || C == nullptr ||
+      keys == nullptr || head_block(tile_cfg, M, N) == 0)
+    return (int)hipErrorInvalidValue;
+  const void* bias = keys;
+  void* ws = nullptr;
+  const int* go = nullptr;
+  const int splits = 1, groups = 1;
+  if (tile_cfg == 55) return gemm_4wp_dispatch(EPI_F32, tile_cfg, DLI_GEMM_PASS);
+  if (tile_cfg >= 60) return gemm_stream_dispatch(EPI_F32, tile_cfg, DLI_GEMM_PASS);
+  return gemm_gemv_dispatch(EPI_F32, tile_cfg, DLI_GEMM_PASS);
 }

@@ -231,12 +231,20 @@ __global__ void __launch_bounds__(256, 1) gemm4wp_kernel(
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const int row = wr0 + 16 * i + fr;
+        BlockMax top;
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
           const f32x4 val = vget(acc[i][j]);
           const int col = wc0 + 16 * j + 4 * fq;
+          if (EPI == EPI_F32 && col < N) top.take(val);
           if (row < M && col < N) store_quad<EPI>(C, ldc, row, col, N, val, bias, vec);
         }
+        if constexpr (EPI == EPI_F32)
+          if (bias != nullptr) {                   // uniform: the block's largest value (BlockMax)
+            const uint32_t key = row_key(top);
+            if (fq == 0 && row < M && wc0 < N)
+              ((uint32_t*)bias)[(long)row * ((N + 16 * NJ - 1) / (16 * NJ)) + wc0 / (16 * NJ)] = key;
+          }
       }
     }
     // the next tile's K-tiles 0 and 1 (issued in the last two K-tiles) landed for every wave

@@ -164,6 +164,30 @@ __device__ __forceinline__ void slab_quad(float* p, f32x4 v, int mode, bool vec,
   slab_quad_fp32(p, v, mode, vec, left);
 }
 
+// EPI_F32's `bias` argument (unsplit, N % 4 == 0; the other fp32 uses leave it null): the address of
+// one order-preserving key (f2key) for every row and wave tile of columns, that of the largest value
+// stored there. The LM head's sampler (sampling.hip) then reads the few column blocks that can hold a
+// candidate in place of every logit: 512 rows of 128256 64 -> 20 us. A key may be too large (a NaN, a
+// zero of either sign), never too small.
+struct BlockMax {
+  float m = -INFINITY;
+  bool nan = false;
+  __device__ __forceinline__ void take(const f32x4& v) {
+    m = fmaxf(fmaxf(m, v[0]), v[1]);
+    m = fmaxf(fmaxf(m, v[2]), v[3]);
+    nan |= __builtin_isunordered(v[0], v[1]) | __builtin_isunordered(v[2], v[3]);
+  }
+  __device__ __forceinline__ uint32_t key() const {
+    return nan ? 0xffffffffu : m == 0.f ? 0x80000000u : f2key(m);
+  }
+};
+// of the 4 lanes that hold a row's quads (16 and 32 lanes apart); all lanes of the wave call it
+__device__ __forceinline__ uint32_t row_key(const BlockMax& b) {
+  uint32_t k = b.key();
+  k = max(k, (uint32_t)__shfl_xor((int)k, 16, 64));
+  return max(k, (uint32_t)__shfl_xor((int)k, 32, 64));
+}
+
 // four consecutive output columns [col, col + 4) of one row; vec = (N % 4 == 0 && ldc % 4
 // == 0): one 16-B (fp32) / 8-B (bf16) store, else per-column stores for the row's tail
 template <int EPI>

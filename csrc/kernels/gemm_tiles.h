@@ -227,6 +227,16 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_bf16_kernel(
 #pragma unroll
   for (int i = 0; i < MI; ++i) {
     const int row = m0 + wm * TM + 16 * i + fr;
+    if constexpr (EPI == EPI_F32)
+      if (bias != nullptr) {                       // uniform: the block's largest value (BlockMax)
+        BlockMax top;
+#pragma unroll
+        for (int j = 0; j < NI; ++j)
+          if (n0 + wn * TN + 16 * j + 4 * fq < N) top.take(acc[i][j]);
+        const uint32_t key = row_key(top);
+        if (fq == 0 && row < Mg && n0 + wn * TN < N)
+          ((uint32_t*)bias)[(long)(row0 + row) * ((N + TN - 1) / TN) + n0 / TN + wn] = key;
+      }
     if (row >= Mg) continue;
 #pragma unroll
     for (int j = 0; j < NI; ++j) {

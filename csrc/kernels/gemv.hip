@@ -307,6 +307,15 @@ __global__ void __launch_bounds__(256) gemv_kernel(
     }
     return;
   }
+  if constexpr (EPI == EPI_F32 && R >= 16)
+    if (bias != nullptr && threadIdx.x < MB) {      // the block's largest value (BlockMax)
+      const int m = threadIdx.x;
+      BlockMax top;
+#pragma unroll
+      for (int j = 0; j < R; j += 4)
+        if (n_base + j < N) top.take(f32x4{res[m][j], res[m][j + 1], res[m][j + 2], res[m][j + 3]});
+      if (m < M) ((uint32_t*)bias)[(long)m * gridDim.x + blockIdx.x] = top.key();
+    }
   for (int t = threadIdx.x; t < MB * R; t += 256) {
     const int m = t / R, j = t % R, n = n_base + j;
     if (m < M && n < N) store_pair_or_one<EPI>(C, ldc, m, n, res[m][j], bias);

@@ -10,6 +10,11 @@
 //     a gather of <= CAP elements. The set is sorted, then temperature-softmax, top-p truncation
 //     (keep j while the mass of strictly larger tokens < top_p, i.e. HF's `cumsum_asc <=
 //     1-top_p` removal) and an inverse-CDF draw.
+// Where the LM head left the largest key of every block of columns (BlockMax in gemm_common.h), the
+// bound comes from these, and only the blocks that reach it are read. top_k 50 of 128k fp32 logits with
+// the head's product before them, us: 512 rows 503 -> 449, 64 212 -> 201, 24 196 -> 184; of 32k, 64
+// rows 64 -> 59. Greedy 512 rows 488 -> 430. One row of 16-column blocks 179 -> 173, where the head
+// takes a kernel of 4-column ones (which leaves none) two phases as before.
 // top_k is capped at CAP (2048). Randomness: Philox4x32-10 keyed by a per-row 64-bit seed
 // supplied by the engine (seed = f(request seed, output index)), so a request samples the
 // same tokens regardless of how it is batched.
@@ -20,10 +25,6 @@
 // candidates ranked by counting; more go through the bitonic sort
 #define SMP_RANK_MAX 128
 
-__device__ __forceinline__ uint32_t f2key(float f) {
-  uint32_t u = __float_as_uint(f);
-  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-}
 __device__ __forceinline__ float key2f(uint32_t k) {
   return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
 }
@@ -234,6 +235,34 @@ __device__ __forceinline__ void row_scan(const LT* __restrict__ x, int V, F&& f,
   row_rounds<8>(x, V, 1, f, floor...);
 }
 
+// The same over n listed blocks of bw columns (a multiple of 4; V is one too), 4 quads in flight a thread
+template <typename LT, typename F>
+__device__ __forceinline__ void block_scan_quads(const LT* __restrict__ x, int V, const int* blk, int n,
+                                                 int bw, F&& f, float lo) {
+  constexpr int U = 4;
+  const int q = bw >> 2, total = n * q;
+  for (int t0 = threadIdx.x; t0 < total; t0 += U * blockDim.x) {
+    float v[U][4];
+    int at[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int t = t0 + u * blockDim.x, b = t < total ? t / q : 0;
+      at[u] = t < total ? blk[b] * bw + (t - b * q) * 4 : V;
+      if (at[u] < V) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[u][j] = ldv(x, at[u] + j);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (at[u] < V) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (!(v[u][j] < lo)) f(v[u][j], at[u] + j);
+      }
+  }
+}
+
 // ---------------------------------------------------------------------------------------
 // Small batches (B <= SMP_SPLIT_MAX_B): one workgroup per row leaves ~255 CUs idle while it
 // walks a 128k-entry row (23 us at batch 1; two phases 18). Two phases
@@ -344,7 +373,7 @@ __global__ void __launch_bounds__(SMP_THREADS) sample_kernel(
     const float* __restrict__ temperature, const int* __restrict__ top_k,
     const float* __restrict__ top_p, const long long* __restrict__ seeds,
     const float* __restrict__ cand_v, const int* __restrict__ cand_i,
-    int* __restrict__ overflow, int ncand) {
+    int* __restrict__ overflow, int ncand, const uint32_t* __restrict__ maxima, int nblk, int bw) {
   __shared__ uint32_t hist[256];
   __shared__ uint32_t ckey[2 * SMP_CAP];      // fast path: the list of candidates
   __shared__ int cidx[2 * SMP_CAP];
@@ -354,7 +383,11 @@ __global__ void __launch_bounds__(SMP_THREADS) sample_kernel(
   __shared__ float sv[16];
   __shared__ int si[16];
   __shared__ uint32_t s_sel[3], s_tau[SMP_THREADS / 64], s_cnt;
+  constexpr int BLKS = 512;                      // blocks of columns that a pass lists
+  __shared__ int s_blk[BLKS], s_nblk;
   const int row = blockIdx.x, tid = threadIdx.x;
+  // largest key of every block of bw columns (null: none were formed)
+  const uint32_t* mx = maxima == nullptr ? nullptr : maxima + (long)row * nblk;
   const LT* xl = logits + (long)row * row_stride;
   const float* xc = nullptr;                     // two-phase mode: the row's candidate list
   const float T = temperature[row];
@@ -384,6 +417,29 @@ __global__ void __launch_bounds__(SMP_THREADS) sample_kernel(
   if (T <= 0.f || K == 1) {                                  // greedy
     ArgMax a{-INFINITY, 0x7fffffff};
     const auto larger = [&](float v, int i) { a = amax(a, ArgMax{v, i}); };
+    if (mx != nullptr) {
+      // the first block of the largest value, then its first element (a block with a NaN, which never
+      // is the largest but whose key hides the others, sends the row to the whole scan)
+      int odd = 0;
+      for (int i = tid; i < nblk; i += SMP_THREADS) {
+        const uint32_t k = mx[i];
+        odd |= k > 0xff800000u;
+        a = amax(a, ArgMax{key2f(k), i});
+      }
+      if (!__syncthreads_or(odd)) {
+        a = block_argmax(a, sv, si);
+        if (a.i < nblk) {
+          const int lo = a.i * bw, hi = min(V, lo + bw);
+          a = ArgMax{-INFINITY, 0x7fffffff};
+          for (int i = lo + tid; i < hi; i += SMP_THREADS) a = amax(a, ArgMax{ldv(xl, i), i});
+          __syncthreads();                         // sv / si are written again
+          a = block_argmax(a, sv, si);
+        }
+        if (tid == 0) out_tokens[row] = a.i < V ? a.i : 0;
+        return;
+      }
+      a = ArgMax{-INFINITY, 0x7fffffff};
+    }
     // (fewer loads in flight where more rows than CUs are walked: 512 rows of 128k bf16 logits 24 us, 27)
     if (xc != nullptr) row_scan(xc, V, larger);
     else if (sizeof(LT) == 2 || gridDim.x > 128) row_rounds<4>(xl, V, 1, larger);
@@ -443,11 +499,18 @@ __global__ void __launch_bounds__(SMP_THREADS) sample_kernel(
       row_rounds<8>(x, V, step, [&](float v, int) { mk = max(mk, f2key(v)); });
       pieces = (reinterpret_cast<uintptr_t>(x) & 15) ? V : V / (int)(16 / sizeof(*x));
     };
-    if (xc != nullptr) sample(xc);
+    const bool by_block = mx != nullptr && nblk >= 4 * Keff;   // (fewer blocks bound too loosely)
+    if (by_block) {
+      pieces = nblk;
+#pragma unroll 4
+      for (int i = tid; i < nblk; i += SMP_THREADS) mk = max(mk, mx[i]);
+    } else if (xc != nullptr) sample(xc);
     else sample(xl);
     constexpr int NWV = SMP_THREADS / 64, SLOTS = 2 * SMP_CAP / SMP_THREADS;
     const uint32_t mk1[1] = {mk};
-    const int nw = max(1, min(NWV, (pieces + 63) >> 6));   // waves that met elements
+    // waves that met elements; of a few hundred blocks only whole ones (the 8th largest of a last wave's
+    // 16 bounds too loosely: 256 rows of 400 blocks 30 us, so 18)
+    const int nw = max(1, min(NWV, by_block ? pieces >> 6 : (pieces + 63) >> 6));
     const uint32_t tw = wave_kth(mk1, (Keff + nw - 1) / nw);
     if ((tid & 63) == 0) s_tau[tid >> 6] = (tid >> 6) < nw ? tw : 0xffffffffu;
     if (tid == 0) s_cnt = 0;
@@ -481,7 +544,22 @@ __global__ void __launch_bounds__(SMP_THREADS) sample_kernel(
       // compare an element, the keys only where one of 16 bytes passes
       const float tf = key2f(tau0);
       cnt = 0;
-      if (xc != nullptr) row_scan(xc, V, hit, tf);
+      bool listed = by_block;
+      if (by_block) {
+        if (tid == 0) s_nblk = 0;
+        __syncthreads();
+#pragma unroll 4
+        for (int i = tid; i < nblk; i += SMP_THREADS)
+          if (mx[i] >= tau0) {
+            const int pos = atomicAdd(&s_nblk, 1);
+            if (pos < BLKS) s_blk[pos] = i;
+          }
+        __syncthreads();
+        listed = s_nblk <= BLKS;                  // else ties by the hundred: the whole row
+        if (listed) block_scan_quads(xl, V, s_blk, s_nblk, bw, hit, tf);
+      }
+      if (listed) {
+      } else if (xc != nullptr) row_scan(xc, V, hit, tf);
       else row_scan(xl, V, hit, tf);
       at = cnt ? atomicAdd(&s_cnt, (uint32_t)cnt) : 0u;
       dropped = __syncthreads_or(cnt > SLOTS ? 1 : 0);
@@ -756,9 +834,12 @@ extern "C" int dli_sample_set_split_max_b(int b) {
 template <typename LT>
 static int launch_sample(int* out_tokens, const LT* logits, long row_stride, int B, int V,
                          const float* temperature, const int* top_k, const float* top_p,
-                         const long long* seeds, void* ws, hipStream_t st) {
+                         const long long* seeds, void* ws, const uint32_t* maxima, int nblk,
+                         int bw, hipStream_t st) {
   if (B <= 0) return 0;
-  if (ws != nullptr && B <= g_smp_max_b) {
+  if (maxima != nullptr && (bw < 4 || bw % 4 || V % 4 || (long)nblk != ((long)V + bw - 1) / bw))
+    return (int)hipErrorInvalidValue;
+  if (maxima == nullptr && ws != nullptr && B <= g_smp_max_b) {
     // P chunks per row: >= 256 workgroups in all, each chunk <= SMP_CHUNK_MAX entries
     int P = 1;
     while (P < 64 && (B * P < 256 || (V + P - 1) / P > SMP_CHUNK_MAX)) P <<= 1;
@@ -772,12 +853,13 @@ static int launch_sample(int* out_tokens, const LT* logits, long row_stride, int
                                                           top_p);
       sample_kernel<LT><<<B, SMP_THREADS, 0, st>>>(out_tokens, logits, row_stride, V,
                                                   temperature, top_k, top_p, seeds, cand_v,
-                                                  cand_i, overflow, P * SMP_CAPC);
+                                                  cand_i, overflow, P * SMP_CAPC, nullptr, 0, 0);
       DLI_RETURN_LAUNCH();
     }
   }
   sample_kernel<LT><<<B, SMP_THREADS, 0, st>>>(out_tokens, logits, row_stride, V, temperature,
-                                              top_k, top_p, seeds, nullptr, nullptr, nullptr, 0);
+                                              top_k, top_p, seeds, nullptr, nullptr, nullptr, 0, maxima,
+                                              nblk, bw);
   DLI_RETURN_LAUNCH();
 }
 
@@ -785,7 +867,18 @@ extern "C" int dli_sample(int* out_tokens, const float* logits, long row_stride,
                           const float* temperature, const int* top_k, const float* top_p,
                           const long long* seeds, void* ws, hipStream_t st) {
   return launch_sample(out_tokens, logits, row_stride, B, V, temperature, top_k, top_p, seeds,
-                       ws, st);
+                       ws, nullptr, 0, 0, st);
+}
+
+// the same with maxima uint32 [B, nblk]: the largest key of every bw columns of these logits, as
+// dli_gemm_head leaves them
+extern "C" int dli_sample_blocks(int* out_tokens, const float* logits, long row_stride, int B, int V,
+                                 const float* temperature, const int* top_k, const float* top_p,
+                                 const long long* seeds, const void* maxima, int nblk, int bw,
+                                 hipStream_t st) {
+  if (maxima == nullptr) return (int)hipErrorInvalidValue;
+  return launch_sample(out_tokens, logits, row_stride, B, V, temperature, top_k, top_p, seeds,
+                       nullptr, static_cast<const uint32_t*>(maxima), nblk, bw, st);
 }
 
 // the same over bf16 logits (row_stride in elements)
@@ -794,7 +887,7 @@ extern "C" int dli_sample_bf16(int* out_tokens, const void* logits, long row_str
                                const float* top_p, const long long* seeds, void* ws,
                                hipStream_t st) {
   return launch_sample(out_tokens, static_cast<const u16*>(logits), row_stride, B, V,
-                       temperature, top_k, top_p, seeds, ws, st);
+                       temperature, top_k, top_p, seeds, ws, nullptr, 0, 0, st);
 }
 
 // ---------------------------------------------------------------------------------------

@@ -54,12 +54,13 @@ from typing import Dict, List, Optional
 import torch
 
 from ..engine.batch import DeviceBatch
+from .. import ops
 from ..ops import gemm as G
 from ..ops import hybrid as H
 from .configs import ModelConfig
 from .mixers import (FEED_FORWARDS, MIXERS, StepView, derive_constants,
                      prepare_feed_forward)
-from .model import TransformerLM
+from .model import _LOGITS, TransformerLM, replaced
 
 
 class HybridLM(TransformerLM):
@@ -301,15 +302,24 @@ class HybridLM(TransformerLM):
     def head_logits(self, h: torch.Tensor) -> torch.Tensor:
         return H.linear_any(h, self.params["lm_head"], out_f32=True)
 
+    def head(self, h: torch.Tensor):
+        w = self.params["lm_head"]
+        if replaced(self, "head_logits", _HEAD_LOGITS):
+            return self.head_logits(h), None
+        if h.dtype == torch.bfloat16 and H.tuned_operands(h, w):
+            return ops.head(h, w)
+        return self.head_logits(h), None
+
     def forward(self, b: DeviceBatch, kv_caches, hidden: Optional[torch.Tensor] = None,
                 return_logits: bool = False):
         """Sampled int32 tokens [S] (and the logits when asked). With ``b.logit_rows`` the
         logits of exactly those rows are returned and nothing is sampled."""
         x = self.forward_layers(self.embed(b, kv_caches), b, kv_caches)
-        lg = self.logits(x, b)
         if b.logit_rows is not None:
-            return lg
-        tok = self.sample(lg, b)
+            return self.logits(x, b)
+        lg, top = ((self.logits(x, b), None) if replaced(self, "logits", _LOGITS)
+                   else self.head(self.final_hidden(x, b)))
+        tok = self.sample_head(lg, b, top)
         return (tok, lg) if return_logits else tok
 
     # ------------------------------------------------------------------ planning
@@ -364,3 +374,6 @@ class HybridLM(TransformerLM):
                     rows = M * spec.top
                     out += [(rows, w1, epi), (rows, lp["w_down"], "none")]
         return out
+
+
+_HEAD_LOGITS = HybridLM.head_logits

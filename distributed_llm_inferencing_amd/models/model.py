@@ -258,6 +258,13 @@ class TransformerLM:
         return ops.linear(h, p["embed"] if self.cfg.tie_embeddings else p["lm_head"],
                           epi=ops.HEAD_EPI)
 
+    def head(self, h: torch.Tensor):
+        """(``head_logits``, what the sampler can use of their product: ``ops.head``)."""
+        if replaced(self, "head_logits", _HEAD_LOGITS):
+            return self.head_logits(h), None
+        p = self.params
+        return ops.head(h, p["embed"] if self.cfg.tie_embeddings else p["lm_head"])
+
     def logits(self, hidden: torch.Tensor, b: DeviceBatch) -> torch.Tensor:
         """Final norm + LM head on the last token of each sequence -> [S, V] logits."""
         return self.head_logits(self.final_hidden(hidden, b))
@@ -270,6 +277,13 @@ class TransformerLM:
     def sample(self, logits: torch.Tensor, b: DeviceBatch, generator=None) -> torch.Tensor:
         return ops.sample(logits, b.temperature, b.top_k, b.top_p, b.seeds, generator=generator)
 
+    def sample_head(self, logits: torch.Tensor, b: DeviceBatch, maxima) -> torch.Tensor:
+        """``sample`` of the logits as ``head`` returned them. A ``sample`` put in its place may
+        change them first and has them without the maxima."""
+        if maxima is None or replaced(self, "sample", _SAMPLE):
+            return self.sample(logits, b)
+        return ops.sample(logits, b.temperature, b.top_k, b.top_p, b.seeds, maxima=maxima)
+
     def forward(self, b: DeviceBatch, kv_caches, hidden: Optional[torch.Tensor] = None,
                 return_logits: bool = False):
         """Stage forward. First stage embeds ``b.input_ids``; otherwise ``hidden`` is the
@@ -281,8 +295,17 @@ class TransformerLM:
             return x
         if self.vocab_parallel:          # the LM head runs sliced on every pipeline rank
             return self.final_hidden(x, b)
-        lg = self.logits(x, b)
         if b.logit_rows is not None:     # scoring / trace replay: these rows' logits, no sampling
-            return lg
-        tok = self.sample(lg, b)
+            return self.logits(x, b)
+        lg, top = ((self.logits(x, b), None) if replaced(self, "logits", _LOGITS)
+                   else self.head(self.final_hidden(x, b)))
+        tok = self.sample_head(lg, b, top)
         return (tok, lg) if return_logits else tok
+
+
+def replaced(model, name: str, plain) -> bool:
+    """Whether a subclass, or whoever set the attribute, put a method of its own in ``plain``'s place."""
+    return getattr(getattr(model, name), "__func__", None) is not plain
+
+
+_SAMPLE, _LOGITS, _HEAD_LOGITS = TransformerLM.sample, TransformerLM.logits, TransformerLM.head_logits

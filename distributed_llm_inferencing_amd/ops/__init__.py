@@ -641,12 +641,32 @@ def _sample_ws(device, B: int, V: int):
 HEAD_EPI = "f32"
 
 
-def sample(logits, temperature, top_k, top_p, seeds, generator=None, ids=None):
+def head(h, w):
+    """(logits, maxima): the fp32 logits ``h @ w.T`` of an LM head and, where its plan's kernel can
+    leave them, (the largest key of each block of columns [M, blocks], columns of a block) for
+    ``sample`` of exactly these logits, else None."""
+    M = h.shape[0]
+    Nn = w.shape[-2]
+    if (HEAD_EPI != "f32" or isinstance(h, NormedRows) or not _use_native(h) or h.stride(-1) != 1 or w.stride(-1) != 1
+            or G.row_cut(M, Nn, h.shape[1])):
+        return linear(h, w, epi=HEAD_EPI), None
+    p = G.plan(M, Nn, h.shape[1], "f32")
+    bw = int(N.require_native().dli_gemm_head_block(p.tile, M, Nn)) if p.splits == 1 else 0
+    if not bw:
+        return linear(h, w, epi=HEAD_EPI), None
+    out = torch.empty(M, Nn, dtype=torch.float32, device=h.device)
+    keys = torch.empty(M, -(-Nn // bw), dtype=torch.int32, device=h.device)
+    _native_call("dli_gemm_head", _p(h), h.stride(0), _p(w), w.stride(-2), _p(out), Nn, M, Nn,
+                 h.shape[1], p.tile, _p(keys), _st())
+    return out, (keys, bw)
+
+
+def sample(logits, temperature, top_k, top_p, seeds, generator=None, ids=None, maxima=None):
     """logits fp32 or bf16 [B, V] -> int32 tokens [B] (every comparison on the exact fp32
     value of each logit). temperature<=0 -> greedy. With ``ids``
     [B, V] the row holds candidates (vocab-parallel LM head) in ascending token-id order,
     and the sampled column is mapped to its token id (ties then break by token id exactly
-    as over the full vocabulary)."""
+    as over the full vocabulary). ``maxima``: what ``head`` returned beside these logits."""
     if not _use_native(logits):
         return R.sample(logits, temperature, top_k, top_p, generator=generator, seeds=seeds,
                         ids=ids)
@@ -654,6 +674,12 @@ def sample(logits, temperature, top_k, top_p, seeds, generator=None, ids=None):
     out = torch.empty(B, dtype=torch.int32, device=logits.device)
     if logits.dtype not in (torch.float32, torch.bfloat16):
         logits = logits.float()
+    if maxima is not None:
+        keys, bw = maxima
+        _native_call("dli_sample_blocks", _p(out), _p(logits), logits.stride(0), B, V,
+                     _p(temperature), _p(top_k), _p(top_p), _p(seeds), _p(keys), keys.shape[1], bw,
+                     _st())
+        return out
     fn = "dli_sample_bf16" if logits.dtype == torch.bfloat16 else "dli_sample"
     _native_call(fn, _p(out), _p(logits), logits.stride(0), B, V, _p(temperature),
                  _p(top_k), _p(top_p), _p(seeds), _p(_sample_ws(logits.device, B, V)), _st())

@@ -52,11 +52,14 @@ _SIGS = {
     "dli_gemm_set_slab_store_family": [I, I],
     "dli_prefill_attention_paged": [P, I, P, I, P, P, P, P, P, I, I, I, I, I, I, I, F, P],
     "dli_sample": [P, P, L, I, I, P, P, P, P, P, P],
+    "dli_sample_blocks": [P, P, L, I, I, P, P, P, P, P, I, I, P],
     "dli_sample_workspace_bytes": [I, I],
     "dli_sample_bf16": [P, P, L, I, I, P, P, P, P, P, P],
     "dli_topk_rows_bf16": [P, P, P, L, I, I, I, I, P],
     "dli_topk_rows": [P, P, P, L, I, I, I, I, P],
     "dli_gemm": [P, I, P, I, P, I, I, I, I, I, I, I, P, P, P, I, P],
+    "dli_gemm_head": [P, I, P, I, P, I, I, I, I, I, P, P],
+    "dli_gemm_head_block": [I, I, I],
     "dli_gemm_persistent_width": [I, I, I],
     "dli_splitk_add_rmsnorm": [P, P, P, I, I, I, P, F, I, P],
     "dli_gemv_fused": [P, I, P, F, P, I, P, I, I, I, I, I, I, I, P, P],

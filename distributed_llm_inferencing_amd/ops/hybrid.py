@@ -45,6 +45,12 @@ def _st():
 
 
 # ----------------------------------------------------------------------------- GEMM
+def tuned_operands(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether bf16 operands are the tuned tiles' own (K a multiple of the K-tile, 16-byte rows)."""
+    return (x.shape[1] % 64 == 0 and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+
+
 def linear_any(x: torch.Tensor, w: torch.Tensor, out_f32: bool = True,
                out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """x [M, K] @ w [N, K]^T with fp32 accumulation -> fp32 (or the storage dtype). bf16 shapes
@@ -63,9 +69,7 @@ def linear_any(x: torch.Tensor, w: torch.Tensor, out_f32: bool = True,
     f32 = out_f32 or x.dtype == torch.float32
     if out is None:
         out = torch.empty(M, Nn, dtype=torch.float32 if f32 else x.dtype, device=x.device)
-    if (x.dtype == torch.bfloat16 and K % 64 == 0 and x.stride(0) % 8 == 0
-            and w.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
-            and out.stride(1) == 1):
+    if x.dtype == torch.bfloat16 and tuned_operands(x, w) and out.stride(1) == 1:
         from . import _gemm_native
         return _gemm_native(x, w, "f32" if f32 else "none", out=out)
     _call("dli_gemm_any", _p(x), x.stride(0), _p(w), w.stride(0), _p(out), out.stride(0), M, Nn,

@@ -329,7 +329,9 @@ __device__ __forceinline__ void decode_end_list(float* __restrict__ ws_ml, int b
 }
 
 // MINW = 4 waves per SIMD: <= 128 VGPRs, so every item of a 512-sequence batch (4096 waves)
-// is resident at once (measured 7 % faster than the 166-VGPR / 2-waves build at ctx 66)
+// is resident at once (measured 7 % faster than the 166-VGPR / 2-waves build at ctx 66). A kernel of 2
+// waves a SIMD that walked items and requested the next tile, across them too, served contexts of 768 and
+// more until the loads here went past the caches: 256 of 984 195 us, this 168; 512 of 33 to 99 36, 33
 template <int HD, int MINW, bool PIPE>
 __global__ void __launch_bounds__(256, MINW) decode_attn_kernel(
     u16* __restrict__ out, const u16* __restrict__ q, int q_stride,
@@ -710,247 +712,6 @@ __global__ void __launch_bounds__(256, 2) decode_attn_split_kernel(
   if (wv == 0) decode_end_list(ws_ml, b, hq, kvh, G, num_splits, split, sp.last, lane);
 }
 
-// Software-pipelined variant: a wave walks a list of work units (item = (sequence, kv head,
-// split), unit = one 32-token tile of it; an empty split is one empty unit) and issues the
-// loads of unit u+1 before computing unit u, across item boundaries (the next item's Q and
-// block-table window are fetched one unit ahead too). K goes to one of two register sets;
-// V goes by LDS-DMA (global_load_lds_dwordx4) straight into one of two per-wave LDS tiles
-// (256-B rows, chunk XOR swizzle for the transposed reads), so no VGPRs hold it. 2 waves per
-// SIMD and a grid of 8 waves per CU, each wave taking items gw, gw + nw, ... The
-// one-tile-per-round kernel above leaves every wave of the chip loading, then computing, in
-// lockstep: 3 exposed HBM round trips at ctx ~66.
-typedef __attribute__((address_space(3))) void dec_lds_void;
-typedef const __attribute__((address_space(1))) void dec_gbl_void;
-
-template <int HD>
-__global__ void __launch_bounds__(256, 2) decode_attn_pipe_kernel(
-    u16* __restrict__ out, const u16* __restrict__ q, int q_stride,
-    const u16* __restrict__ k_cache, const u16* __restrict__ v_cache,
-    const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ context_lens,
-    int B, int hq, int hkv, int block_size, float scale_log2, int num_splits, int split_tokens,
-    float* __restrict__ ws_o, float* __restrict__ ws_ml) {
-  static_assert(HD == 128, "pipelined decode attention: head_dim 128");
-  constexpr int KK = HD / 32, DB = HD / 16;
-  constexpr int VT_BYTES = DEC_TILE * HD * 2;                  // 8 KiB per V tile
-  __shared__ __attribute__((aligned(16))) char vt_all[DEC_WAVES][2][VT_BYTES];
-  const int wv = threadIdx.x >> 6;
-  const int lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4;
-  const int G = hq / hkv;
-  const int nitems = B * hkv * num_splits;
-  const int nw = gridDim.x * DEC_WAVES;
-  const long kv_head_stride = (long)block_size * HD;
-
-  int p_item = blockIdx.x * DEC_WAVES + wv;
-  if (p_item >= nitems) return;                                  // wave-uniform
-  auto geom = [&](int it, int& b, int& kvh, int& split, int& sb, int& se) {
-    split = it % num_splits;
-    const int bh = it / num_splits;
-    kvh = bh % hkv;
-    b = bh / hkv;
-    const int ctx = context_lens[b];
-    sb = split * split_tokens;
-    se = min(ctx, sb + split_tokens);
-  };
-  auto ntiles_of = [&](int sb, int se) { return se > sb ? (se - sb + DEC_TILE - 1) / DEC_TILE : 1; };
-  auto load_q = [&](int b, int kvh, bf16x8* dst) {
-    const bool valid = col < G;
-    const u16* qp = q + (long)b * q_stride + (long)(kvh * G + (valid ? col : 0)) * HD;
-#pragma unroll
-    for (int kk = 0; kk < KK; ++kk) {
-      uint4 v = valid ? *reinterpret_cast<const uint4*>(qp + kk * 32 + grp * 8)
-                      : make_uint4(0, 0, 0, 0);
-      dst[kk] = *reinterpret_cast<bf16x8*>(&v);
-    }
-  };
-  int pb, pkvh, psplit, psb, pse;
-  geom(p_item, pb, pkvh, psplit, psb, pse);
-  int p_tile = 0, p_nt = ntiles_of(psb, pse);
-  int p_win = psb / block_size;
-  int p_last_blk = max(pse - 1, 0) / block_size;
-  int p_bt = block_tables[(long)pb * max_blocks + min(p_win + lane, p_last_blk)];
-  bf16x8 qf_next[KK];
-  load_q(pb, pkvh, qf_next);
-
-  // V image: row r at 256 r, 16-B chunk c at physical chunk c ^ swz(r)
-  auto vswz = [](int r) { return ((r & 3) << 2) | ((r >> 2) & 3); };
-  uint4 ka[2][KK], kb[2][KK];
-  // issue the loads of the prefetch cursor's unit; returns true if it issued any
-  auto issue = [&](uint4 (&kr)[2][KK], int vbuf) -> bool {
-    if (pse <= psb) return false;                                // empty unit: no loads
-    const int t0 = psb + DEC_TILE * p_tile;
-    if ((min(t0 + DEC_TILE, pse) - 1) / block_size - p_win >= 64) {   // wave-uniform
-      p_win = t0 / block_size;
-      p_bt = block_tables[(long)pb * max_blocks + min(p_win + lane, p_last_blk)];
-    }
-    const u16* kbase = k_cache + (long)pkvh * kv_head_stride;
-    const u16* vbase = v_cache + (long)pkvh * kv_head_stride;
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int tok = min(t0 + 16 * s + col, pse - 1);
-      const int blk = __shfl(p_bt, tok / block_size - p_win, 64), off = tok % block_size;
-      const u16* kp = kbase + (long)blk * hkv * kv_head_stride + (long)off * HD;
-#pragma unroll
-      for (int kk = 0; kk < KK; ++kk)
-        kr[s][kk] = *reinterpret_cast<const uint4*>(kp + kk * 32 + grp * 8);
-    }
-    // 8 pieces of 4 rows: lane L of piece m lands at row 4m + L/16, physical chunk L%16
-#pragma unroll
-    for (int m = 0; m < DEC_TILE / 4; ++m) {
-      const int r = 4 * m + (lane >> 4);
-      const int c = (lane & 15) ^ vswz(r);
-      const int tok = min(t0 + r, pse - 1);
-      const int blk = __shfl(p_bt, tok / block_size - p_win, 64), off = tok % block_size;
-      __builtin_amdgcn_global_load_lds(
-          (dec_gbl_void*)(vbase + (long)blk * hkv * kv_head_stride + (long)off * HD + c * 8),
-          (dec_lds_void*)&vt_all[wv][vbuf][m * 1024], 16, 0, 0);
-    }
-    return true;
-  };
-  auto advance = [&]() -> bool {
-    if (++p_tile < p_nt) return true;
-    p_item += nw;
-    if (p_item >= nitems) return false;
-    geom(p_item, pb, pkvh, psplit, psb, pse);
-    p_tile = 0;
-    p_nt = ntiles_of(psb, pse);
-    p_win = psb / block_size;
-    p_last_blk = max(pse - 1, 0) / block_size;
-    p_bt = block_tables[(long)pb * max_blocks + min(p_win + lane, p_last_blk)];
-    load_q(pb, pkvh, qf_next);
-    return true;
-  };
-
-  int c_item = p_item, cb = pb, ckvh = pkvh, csplit = psplit, csb = psb, cse = pse;
-  int c_tile = 0, c_nt = p_nt;
-  bf16x8 qf[KK];
-#pragma unroll
-  for (int kk = 0; kk < KK; ++kk) qf[kk] = qf_next[kk];
-  float m_run = -INFINITY, l_part = 0.f;
-  f32x4 o_acc[DB];
-#pragma unroll
-  for (int i = 0; i < DB; ++i) o_acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  auto finalize = [&]() {
-    float l_tot = l_part + __shfl_xor(l_part, 16, 64);
-    l_tot += __shfl_xor(l_tot, 32, 64);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int h = 4 * grp + r;
-      const float lr = __shfl(l_tot, h, 64);
-      const float mr = __shfl(m_run, h, 64);
-      if (h >= G) continue;
-      const int qh = ckvh * G + h;
-      const float inv = lr > 0.f ? 1.f / lr : 0.f;
-      if (num_splits == 1) {
-        u16* op = out + ((long)cb * hq + qh) * HD;
-#pragma unroll
-        for (int i = 0; i < DB; ++i) op[16 * i + col] = f2bf(o_acc[i][r] * inv);
-      } else {
-        const long base = ((long)cb * hq + qh) * num_splits + csplit;
-        float* wo = ws_o + base * HD;
-#pragma unroll
-        for (int i = 0; i < DB; ++i) wo[16 * i + col] = o_acc[i][r] * inv;
-        if (col == 0) {
-          ws_ml[base * 2] = lr > 0.f ? mr : -INFINITY;
-          ws_ml[base * 2 + 1] = lr;
-        }
-      }
-    }
-  };
-  // compute cursor's unit from K registers kr and V tile vbuf; `later` = the next unit's
-  // loads were issued after this unit's V DMA (then vmcnt(16) retires exactly this tile:
-  // at least 16 vector-memory ops followed it; else vmcnt(0))
-  const int qrow = (lane >> 2) & 3, pcol = lane & 3;
-  auto compute = [&](uint4 (&kr)[2][KK], int vbuf, bool later) {
-    if (cse > csb) {
-      const int t0 = csb + DEC_TILE * c_tile;
-      f32x4 s_acc[2];
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        s_acc[s] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kk = 0; kk < KK; ++kk)
-          s_acc[s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              *reinterpret_cast<bf16x8*>(&kr[s][kk]), qf[kk], s_acc[s], 0, 0, 0);
-      }
-      float p[8];
-      float tmax = -INFINITY;
-#pragma unroll
-      for (int s = 0; s < 2; ++s)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int tok = t0 + 16 * s + 4 * grp + r;
-          const float v = tok < cse ? s_acc[s][r] * scale_log2 : -INFINITY;
-          p[s * 4 + r] = v;
-          tmax = fmaxf(tmax, v);
-        }
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-      const float m_new = fmaxf(m_run, tmax);
-      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);     // m_run=-inf -> 0
-      m_run = m_new;
-      float psum = 0.f;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) { p[j] = __builtin_amdgcn_exp2f(p[j] - m_new); psum += p[j]; }
-      l_part = l_part * alpha + psum;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float a = __shfl(alpha, 4 * grp + r, 64);
-#pragma unroll
-        for (int i = 0; i < DB; ++i) o_acc[i][r] *= a;
-      }
-      bf16x8 pa;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) pa[j] = (__bf16)p[j];
-      if (later) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");   // this V tile landed
-      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      const char* vt = vt_all[wv][vbuf];
-#pragma unroll
-      for (int i = 0; i < DB; ++i) {
-        // rows 4grp + qrow and 16 + 4grp + qrow, columns 16i + 4pcol .. +3
-        const int r0 = 4 * grp + qrow, r1 = 16 + r0, ch = 2 * i + (pcol >> 1);
-        s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) s16x4*)(vt + 256 * r0 + 16 * (ch ^ vswz(r0)) +
-                                                       8 * (pcol & 1)));
-        s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) s16x4*)(vt + 256 * r1 + 16 * (ch ^ vswz(r1)) +
-                                                       8 * (pcol & 1)));
-        s16x8 w = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-        o_acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa, *reinterpret_cast<bf16x8*>(&w),
-                                                          o_acc[i], 0, 0, 0);
-      }
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // reads done before restaging
-    }
-    if (++c_tile == c_nt) {                                      // item done
-      finalize();
-      c_item += nw;
-      if (c_item < nitems) {
-        geom(c_item, cb, ckvh, csplit, csb, cse);
-        c_tile = 0;
-        c_nt = ntiles_of(csb, cse);
-#pragma unroll
-        for (int kk = 0; kk < KK; ++kk) qf[kk] = qf_next[kk];
-        m_run = -INFINITY;
-        l_part = 0.f;
-#pragma unroll
-        for (int i = 0; i < DB; ++i) o_acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-      }
-    }
-  };
-
-  issue(ka, 0);
-  while (true) {
-    bool more = advance();
-    bool later = more && issue(kb, 1);
-    compute(ka, 0, later);
-    if (!more) break;
-    more = advance();
-    later = more && issue(ka, 0);
-    compute(kb, 1, later);
-    if (!more) break;
-  }
-}
-
 // out[b, h, :] = sum_s w_s o_s / sum_s w_s,  w_s = exp2(m_s - M) * l_s, over the splits before the
 // first one with l = -1; none: the row is there already. A wave per row, the splits' (m, l) one per
 // lane, up to 16 splits' outputs in flight: what another XCD wrote comes from memory, and a row has
@@ -1015,17 +776,6 @@ __global__ void __launch_bounds__(256) decode_reduce_kernel(u16* __restrict__ ou
   for (int j = 0; j < E; ++j) out[bh * HD + lane * E + j] = f2bf(acc[j] * inv);
 }
 
-// pipelined (1), one-tile-per-round (0) or automatic (2, the default) decode kernel for hd 128
-static int g_decode_pipe = 2;
-extern "C" int dli_decode_set_pipe(int v) {
-  const int old = g_decode_pipe;
-  g_decode_pipe = v;
-  return old;
-}
-
-// the mode the next dli_decode_attention call applies
-extern "C" int dli_decode_get_pipe() { return g_decode_pipe; }
-
 // a workgroup per (sequence, kv head) item while the items alone would leave most CUs idle
 // (<= 256 items: B <= 32 at 8 kv heads), else a wave per item; tests force either form with
 // dli_decode_set_form(1 = wave per item, DEC_WAVES = workgroup per item, 0 = automatic)
@@ -1056,23 +806,7 @@ extern "C" int dli_decode_attention(void* out, const void* q, int q_stride, cons
   float* ws_ml = ws_o ? ws_o + (long)B * hq * num_splits * hd : nullptr;
   const float scale_log2 = scale * 1.4426950408889634f;
   const long items = (long)B * hkv * num_splits;
-  // 2 = automatic: the pipelined kernel where a sequence is one item of up to 768 tokens or more
-  // (max_context is a bound, in a captured step the table's width): +18 % at 1000 tokens, 64 rows;
-  // within 3 % slower at 33 - 100, 512 rows, where the per-item dependent loads (context length ->
-  // block table -> K/V) rather than tile rounds bound the time. Split sequences are dealt whatever
-  // the bound: 128 rows of 100 - 1000 tokens on an 8192-token table 54 us, pipelined over the same 8
-  // static slots 231, over two 93; 24 of 500 - 8000 on 32768 64 us, 98, 304; 128 of 8000 731, 780, 755.
-  const bool use_pipe = g_decode_pipe == 1 ||
-                        (g_decode_pipe == 2 && num_splits == 1 && split_tokens >= 768);
-  if (hd == 128 && use_pipe) {
-    // 8 waves per CU x 256 CUs; each wave walks items gw, gw + nw, ...
-    const long wgs = (items + DEC_WAVES - 1) / DEC_WAVES;
-    dim3 gp((int)(wgs < 512 ? wgs : 512));
-    decode_attn_pipe_kernel<128><<<gp, 64 * DEC_WAVES, 0, st>>>(
-        (u16*)out, (const u16*)q, q_stride, (const u16*)k_cache, (const u16*)v_cache,
-        block_tables, max_blocks, context_lens, B, hq, hkv, block_size, scale_log2, num_splits,
-        split_tokens, ws_o, ws_ml);
-  } else if (hd == 128 && num_splits == 1 && wg_form(items)) {
+  if (hd == 128 && num_splits == 1 && wg_form(items)) {
     decode_attn_wg_kernel<<<(int)items, 64 * DEC_WAVES, 0, st>>>(
         (u16*)out, (const u16*)q, q_stride, (const u16*)k_cache, (const u16*)v_cache,
         block_tables, max_blocks, context_lens, B, hq, hkv, block_size, scale_log2);

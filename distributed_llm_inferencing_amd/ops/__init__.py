@@ -393,7 +393,7 @@ def linear_rope_attention(x, w, positions, slot_mapping, cos_sin, k_cache, v_cac
     attention computed by ONE kernel per layer (``dli_decode_attention_fused``) instead of
     ``linear_rope_cache`` + ``decode_attention``. Returns the attention output [B, hq*hd], or
     None where the fused kernel does not apply (the caller then runs the two-kernel path):
-    split counts other than 2 / 4, the pipelined long-context kernel, head dim != 128."""
+    split counts other than 2 / 4, head dim != 128."""
     xr = x.residual if isinstance(x, NormedRows) else x
     if hd != 128 or k_cache is None or not _use_native(xr):
         return None
@@ -402,9 +402,6 @@ def linear_rope_attention(x, w, positions, slot_mapping, cos_sin, k_cache, v_cac
         return None
     B, K = x.shape
     ns = decode_num_splits(B, hkv, max_context)
-    mode = int(N.require_native().dli_decode_get_pipe())
-    if mode == 1 or (mode == 2 and ns == 1 and -(-max_context // 32) * 32 >= 768):
-        return None                       # dli_decode_attention picks the pipelined kernel
     Nn = w.shape[0]
     fmt = 0
     slabs = p.splits * B * Nn * 4 if p is not None else 0
@@ -512,11 +509,15 @@ def prefill_attention(qkv, cu_seqlens, max_seqlen: int, hq, hkv, hd, scale, out=
     return out
 
 
+_pipelined = 2
+
+
 def decode_pipelined(v: int) -> int:
-    """Select the pipelined (1), one-tile-per-round (0) or automatic (2, the default: pipelined
-    for unsplit contexts of up to 768 tokens or more) decode attention kernel for head_dim 128. Returns the
-    previous setting (tests force either kernel with it)."""
-    return int(N.require_native().dli_decode_set_pipe(int(v)))
+    """Once chose between two decode attention kernels; one serves every setting now, which is only
+    kept and returned."""
+    global _pipelined
+    old, _pipelined = _pipelined, int(v)
+    return old
 
 
 def decode_form(v: int) -> int:

@@ -45,8 +45,6 @@ _SIGS = {
     "dli_prefill_set_min_len": [I],
     "dli_prefill_set_pack": [I],
     "dli_sample_set_split_max_b": [I],
-    "dli_decode_set_pipe": [I],
-    "dli_decode_get_pipe": [],
     "dli_decode_set_form": [I],
     "dli_gemm_set_slab_store": [I],
     "dli_gemm_set_slab_store_family": [I, I],

@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Decode attention at batch 512 (Llama-3-8B heads: 32 q / 8 kv x 128) against context
 length: the fused kernel the decode graph runs (QKV split-K fp16 slabs reduced, RoPE, k/v
-cache write and attention in one launch), and the unfused plain / pipelined attention kernels
+cache write and attention in one launch), and the unfused attention kernel
 (timed apart from the separate RoPE + cache-write kernel). Times are per call from graph replays of 16 calls each; the KV
 bytes read per call give the achieved bandwidth, and the slope / intercept of time against
 context split the per-token (streaming) cost from the fixed (prologue, launch) cost.
@@ -59,19 +59,13 @@ def main():
             ops.decode_attention(qkv, kc, vc, bt, cl, ctx, hq, hkv, hd, scale, out=out)
 
         row = {"batch": B, "ctx": ctx, "kv_MB": round(kv_mb, 1)}
-        for name, fn, mode in (("fused", fused, None), ("rope", rope, None),
-                               ("plain", attn, 0), ("pipe", attn, 1)):
-            old = ops.decode_pipelined(mode) if mode is not None else None
+        for name, fn in (("fused", fused), ("rope", rope), ("plain", attn)):
             # R calls per graph: one replay's launch latency (~10-20 us of host time that the
             # events around a replay also measure) is spread over R kernels
             def rep(fn=fn):
                 for _ in range(R):
                     fn()
-            try:
-                ms = ops.benchmark(rep, iters=a.reps, warmup=1, graph=True) / R
-            finally:
-                if old is not None:
-                    ops.decode_pipelined(old)
+            ms = ops.benchmark(rep, iters=a.reps, warmup=1, graph=True) / R
             us = ms * 1e3
             row[name + "_us"] = round(us, 2)
             if name != "rope":

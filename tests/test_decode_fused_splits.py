@@ -13,18 +13,18 @@ HD, BS, HKV = 128, 16, 8
 
 
 # one token; a split's edge and either side; a short last split; a long
-# context among short ones; a padded row (0: no slot); more sequences than one scan covers
+# context among short ones; a padded row (0: no slot); more sequences than one scan covers; as many as take no splits
 @pytest.mark.gpu
 @pytest.mark.parametrize("hq", (8, 32, 128))
 @pytest.mark.parametrize("tile,splits", ((0, 1), (0, 2), (0, 4), (30, 2)))
 @pytest.mark.parametrize("lens,limit", (
     ([1], 2048), ([64], 2048), ([65], 2048), ([129], 1024), ([2047, 0, 5, 33], 2048), ([4000] + [70] * 5, 4096),
-    ([700, 701, 690, 720], 1024), ([(7 * i) % 190 + 1 for i in range(70)], 1024)))
+    ([700, 701, 690, 720], 1024), ([(7 * i) % 190 + 1 for i in range(70)], 1024), ([(37 * i) % 901 for i in range(260)], 1024)))
 def test_fused_splits_match_separate_kernels(gpu, hq, tile, splits, lens, limit):
     B, K, N = len(lens), 512, (hq + 2 * HKV) * HD
     if tile == 30 and B > G.GEMV_MAX_M:
         pytest.skip("weight stream of up to 4 rows")
-    assert ops.decode_num_splits(B, HKV, limit) > 1
+    assert (ops.decode_num_splits(B, HKV, limit) > 1) == (B < 256)
     g = torch.Generator(device=gpu).manual_seed(hq + B)
     width = -(-limit // BS)
     need = [-(-n // BS) for n in lens]
@@ -56,10 +56,11 @@ def test_fused_splits_match_separate_kernels(gpu, hq, tile, splits, lens, limit)
         G.clear_plans()
         G._plan_cache.update(kept)
     # the rotation's products and difference may be contracted differently: a key or query element that
-    # lies between two bf16 values falls to either side, one ulp (2^-7 of it at most), the rest is equal
+    # lies between two bf16 values falls to either side, one ulp (2^-7 of it at most), the rest is equal;
+    # where the difference cancels, what is left is the products' rounding: 2^-23 of |a cos| + |b sin| <= 16
     assert torch.equal(v1, v2)
     apart = (k1.float() - k2.float()).abs()
-    assert bool((apart <= 2.0 ** -7 * k1.float().abs()).all()) and int((apart > 0).sum()) <= 2 + B * HKV * HD // 1000
+    assert bool((apart <= 2.0 ** -7 * k1.float().abs() + 2.0 ** -19).all()) and int((apart > 0).sum()) <= 2 + B * HKV * HD // 1000
     # a few elements of a score's 128 move by 2^-8: the softmax's weights by less than 1 %
     live = ctx > 0
     assert float((got[live].float() - want[live].float()).norm() / want[live].float().norm()) < 2.0 ** -8

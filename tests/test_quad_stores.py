@@ -1,0 +1,25 @@
+"""Kernels that store four columns at a time where every row takes it, and one by one elsewhere."""
+import pytest
+import torch
+
+from distributed_llm_inferencing_amd.ops import hybrid as H
+
+
+# N a multiple of 4, of 2, odd; rows of the output 16 bytes apart and not; an output that starts off 16 bytes.
+# bf16 products summed in fp32: K terms of at most |a||b|, 2^-24 each, and bf16's own rounding
+@pytest.mark.gpu
+@pytest.mark.parametrize("N", [4096, 68, 30, 33])
+@pytest.mark.parametrize("K", [32, 96, 7])
+@pytest.mark.parametrize("pad,off", [(0, 0), (4, 0), (3, 0), (4, 1)])
+@pytest.mark.parametrize("f32", [True, False])
+def test_rank_products(gpu, N, K, pad, off, f32):
+    g = torch.Generator(device=gpu).manual_seed(N + K)
+    M = 70
+    x, w = (torch.randn(r, K, device=gpu, generator=g).bfloat16() for r in (M, N))
+    whole = torch.full((M, N + pad + off), 7.0, device=gpu, dtype=torch.float32 if f32 else torch.bfloat16)
+    out = whole[:, off:off + N]
+    H.linear_any(x, w, out_f32=f32, out=out)
+    want = x.double() @ w.double().T
+    bound = (x.double().abs() @ w.double().abs().T) * K * 2.0 ** -24 + (0 if f32 else want.abs() * 2.0 ** -8)
+    assert bool(((out.double() - want).abs() <= bound).all())
+    assert bool((whole[:, :off] == 7).all()) and bool((whole[:, off + N:] == 7).all())

@@ -62,28 +62,39 @@ __global__ void __launch_bounds__(256) prev_tokens_kernel(
   if (threadIdx.x == 0 && slot >= 0) state[slot] = ids[t1 - 1];
 }
 
-template <typename S>
+// VEC = 4: whole 16-byte pieces of a row, and a row's hash once for four columns. 7200 rows of 4096 from
+// bf16 tables (0.3 GB) 155 -> 78 us.
+template <typename S, int VEC>
 __global__ void __launch_bounds__(256) embedding_bigram_kernel(
     float* __restrict__ x, S* __restrict__ xs, const int* __restrict__ ids,
     const int* __restrict__ prev, const S* __restrict__ table, const S* __restrict__ bigram,
     int T, int dim, int vocab, int buckets, long mul_prev, long mul_cur) {
   const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= (long)T * dim) return;
-  const int t = (int)(gid / dim), c = (int)(gid % dim);
+  const int w = dim / VEC;
+  if (gid >= (long)T * w) return;
+  const int t = (int)(gid / w), c = (int)(gid - (long)t * w) * VEC;
   int id = ids[t];
   id = id < 0 ? 0 : (id >= vocab ? vocab - 1 : id);
-  float v = ldf(table + (long)id * dim + c);
+  long row = buckets;                          // no previous token: the table's last row
   if (bigram != nullptr) {
     const int p = prev[t];
-    long row = buckets;                        // no previous token: the table's last row
     if (p >= 0) {
       row = ((long)p * mul_prev + (long)id * mul_cur) % buckets;
       if (row < 0) row += buckets;
     }
-    v += ldf(bigram + row * dim + c);
   }
-  x[gid] = v;
-  stf(xs + gid, v);
+  const long o = (long)t * dim + c;
+  if constexpr (VEC == 4) {
+    f32x4 v = ld4(table + (long)id * dim + c);
+    if (bigram != nullptr) v += ld4(bigram + row * dim + c);
+    *reinterpret_cast<f32x4*>(x + o) = v;
+    st4(xs + o, v);
+  } else {
+    float v = ldf(table + (long)id * dim + c);
+    if (bigram != nullptr) v += ldf(bigram + row * dim + c);
+    x[o] = v;
+    stf(xs + o, v);
+  }
 }
 
 // One workgroup per row: v = keep * x + y, y the sum of nsplit slabs of a split-K product; mean and variance (of the deviations, two passes
@@ -520,14 +531,16 @@ extern "C" int dli_embedding_bigram(float* x, void* xs, const int* ids, const in
                                     hipStream_t st) {
   if (T <= 0) return 0;
   if (bigram != nullptr && (prev == nullptr || buckets < 1)) return (int)hipErrorInvalidValue;
-  const int nb = (int)(((long)T * dim + 255) / 256);
-  DT_SWITCH(dt,
-            (embedding_bigram_kernel<u16><<<nb, 256, 0, st>>>(
-                x, (u16*)xs, ids, prev, (const u16*)table, (const u16*)bigram, T, dim, vocab,
-                buckets, (long)mul_prev, (long)mul_cur)),
-            (embedding_bigram_kernel<float><<<nb, 256, 0, st>>>(
-                x, (float*)xs, ids, prev, (const float*)table, (const float*)bigram, T, dim,
-                vocab, buckets, (long)mul_prev, (long)mul_cur)));
+  const bool vec = dim % 4 == 0 &&
+                   (((uintptr_t)x | (uintptr_t)xs | (uintptr_t)table | (uintptr_t)bigram) & 15) == 0;
+  const int nb = (int)(((long)T * (vec ? dim / 4 : dim) + 255) / 256);
+#define EB_LAUNCH(S, V)                                                                        \
+  (embedding_bigram_kernel<S, V><<<nb, 256, 0, st>>>(x, (S*)xs, ids, prev, (const S*)table,     \
+                                                     (const S*)bigram, T, dim, vocab, buckets,  \
+                                                     (long)mul_prev, (long)mul_cur))
+  if (vec) DT_SWITCH(dt, EB_LAUNCH(u16, 4), EB_LAUNCH(float, 4));
+  else DT_SWITCH(dt, EB_LAUNCH(u16, 1), EB_LAUNCH(float, 1));
+#undef EB_LAUNCH
   DLI_RETURN_LAUNCH();
 }
 

@@ -23,3 +23,20 @@ def test_rank_products(gpu, N, K, pad, off, f32):
     bound = (x.double().abs() @ w.double().abs().T) * K * 2.0 ** -24 + (0 if f32 else want.abs() * 2.0 ** -8)
     assert bool(((out.double() - want).abs() <= bound).all())
     assert bool((whole[:, :off] == 7).all()) and bool((whole[:, off + N:] == 7).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dim", [40, 30, 4096])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("hashed", [True, False])
+def test_bigram_rows(gpu, dim, dtype, hashed):
+    g = torch.Generator(device=gpu).manual_seed(dim)
+    t, b = (torch.randn(r, dim, device=gpu, generator=g).to(dtype) for r in (31, 18))
+    ids = torch.randint(0, 31, (65,), device=gpu, generator=g, dtype=torch.int32)
+    prev = torch.randint(-1, 31, (65,), device=gpu, generator=g, dtype=torch.int32)
+    x, xs = H.embedding_bigram(ids, prev if hashed else None, t, b if hashed else None, 17, 29, 5)
+    want = t[ids.long()].float()
+    if hashed:
+        row = torch.where(prev < 0, 17, (prev.long() * 29 + ids.long() * 5) % 17)
+        want = want + b[row].float()
+    assert torch.equal(x, want) and torch.equal(xs, want.to(dtype))

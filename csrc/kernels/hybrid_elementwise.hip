@@ -145,13 +145,15 @@ __global__ void __launch_bounds__(1024) resadd_groupnorm_kernel(
     }
   }
   __syncthreads();
-  if (vec4 && !h_f32 && groups == 1 && ldh % 4 == 0) {
-    const float rs = gsum[0] * gain;
+  // (8192 rows of 4096 in 4 groups, 0.47 GB: 112 us with 2-byte stores, 95 so; in a step 90 -> 77)
+  if (vec4 && !h_f32 && gl % 4 == 0 && ldh % 4 == 0) {
+    const float after = groups == 1 ? 1.f : gain;
     for (int c = threadIdx.x * 4; c < dim; c += blockDim.x * 4) {
       const f32x4 v = *reinterpret_cast<const f32x4*>(row + c);
+      const float rs = groups == 1 ? gsum[0] * gain : gsum[c / gl];
       float o[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) o[u] = v[u] * rs * (ldf(w + c + u) + w_offset);
+      for (int u = 0; u < 4; ++u) o[u] = v[u] * rs * (ldf(w + c + u) + w_offset) * after;
       S* hp = (S*)h + (long)r * ldh + c;
       if constexpr (sizeof(S) == 2) {
         uint2 pk;

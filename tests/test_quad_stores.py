@@ -40,3 +40,22 @@ def test_bigram_rows(gpu, dim, dtype, hashed):
         row = torch.where(prev < 0, 17, (prev.long() * 29 + ids.long() * 5) % 17)
         want = want + b[row].float()
     assert torch.equal(x, want) and torch.equal(xs, want.to(dtype))
+
+
+# groups of whole quads and not, against float64: the sums' and products' rounding, and the output's
+@pytest.mark.gpu
+@pytest.mark.parametrize("dim,groups", [(4096, 4), (4096, 1), (40, 2), (60, 4), (48, 3), (4096, 64), (30, 5), (36, 6)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows", [3, 1030])
+def test_grouped_norm(gpu, dim, groups, dtype, rows):
+    g = torch.Generator(device=gpu).manual_seed(dim + groups)
+    x, y = (torch.randn(rows, dim, device=gpu, generator=g) for _ in range(2))
+    w = torch.randn(dim, device=gpu, generator=g).to(dtype)
+    new = x.double() + 0.7 * y.double()
+    v = new.view(rows, groups, -1)
+    want = (v * torch.rsqrt(v.pow(2).mean(-1, keepdim=True) + 1e-5)).view(rows, dim) * (w.double() + 0.5) * 1.25
+    h = H.resadd_groupnorm(x, y, w, groups, 1e-5, mult=0.7, gain=1.25, w_offset=0.5)
+    assert torch.allclose(x.double(), new, rtol=0, atol=float(new.abs().max()) * 2.0 ** -22)
+    # a group's sum of squares: dim / groups terms of one sign, half of that in the root; five roundings after
+    rel = (dim / groups / 2 + 8) * 2.0 ** -24 + (2.0 ** -8 if dtype == torch.bfloat16 else 0)
+    assert bool(((h.double() - want).abs() <= rel * want.abs() + 2.0 ** -21 * (w.double().abs() + 0.5)).all())

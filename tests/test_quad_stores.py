@@ -2,6 +2,7 @@
 import pytest
 import torch
 
+from distributed_llm_inferencing_amd.ops import hybrid
 from distributed_llm_inferencing_amd.ops import hybrid as H
 
 
@@ -59,3 +60,53 @@ def test_grouped_norm(gpu, dim, groups, dtype, rows):
     # a group's sum of squares: dim / groups terms of one sign, half of that in the root; five roundings after
     rel = (dim / groups / 2 + 8) * 2.0 ** -24 + (2.0 ** -8 if dtype == torch.bfloat16 else 0)
     assert bool(((h.double() - want).abs() <= rel * want.abs() + 2.0 ** -21 * (w.double().abs() + 0.5)).all())
+
+
+# the pieces' form (rows 16 bytes apart) and the general one (rows 4 bytes off) against float64: the split
+# halves and the interleaved pairs, part of the tail rotated, none of it, a cache of another layer, unused slots
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,d,dr,r,rot", [(32, 128, 64, 512, 64), (3, 8, 16, 20, 8), (2, 4, 8, 4, 0), (2, 8, 12, 12, 6)])
+@pytest.mark.parametrize("half", [True, False])
+@pytest.mark.parametrize("own", [True, False])
+@pytest.mark.parametrize("pad", [0, 1])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_latent_rows(gpu, H, d, dr, r, rot, half, own, pad, dtype):
+    g = torch.Generator(device=gpu).manual_seed(d + r + rot)
+    T = 9
+    q = torch.randn(T, H * (d + dr) + 4 * pad + pad, device=gpu, generator=g)[:, pad:pad + H * (d + dr)]
+    kv = torch.randn(T, r + dr + 4 * pad + pad, device=gpu, generator=g)[:, pad:pad + r + dr] if own else None
+    w = torch.randn(r, device=gpu, generator=g).to(dtype)
+    freq = torch.rand(max(rot // 2, 1), device=gpu, generator=g).double()
+    pos = torch.randint(0, 5000, (T,), device=gpu, generator=g, dtype=torch.int32)
+    slots = torch.arange(T, device=gpu, dtype=torch.int32) * 2
+    slots[4] = -1
+    cache = torch.full((2 * T, r + dr), 7.0, device=gpu, dtype=dtype)
+    want = cache.double().cpu()
+    qn, qf = hybrid.latent_prepare(q, kv, w, 1e-5, H, d, dr, r, rot, freq, pos, slots, cache, dtype, half)
+    c = lambda t: None if t is None else t.double().cpu()  # noqa: E731
+    tail = lambda v: rotated(v, pos.double().cpu(), freq.cpu(), rot, half)  # noqa: E731
+    qq = c(q).reshape(T, H, d + dr)
+    ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -24
+    near = lambda a, b: bool(((c(a) - b).abs() <= ulp * b.abs() + 2.0 ** -20).all())  # noqa: E731
+    assert near(qn, qq[:, :, :d]) and near(qf[:, :, r:], tail(qq[:, :, d:]))
+    if own:
+        lat = c(kv)[:, :r] * torch.rsqrt(c(kv)[:, :r].pow(2).mean(-1, keepdim=True) + 1e-5) * c(w)
+        ok = (slots >= 0).cpu()
+        want[slots.cpu()[ok].long()] = torch.cat([lat, tail(c(kv)[:, None, r:])[:, 0]], 1)[ok]
+    assert near(cache, want)
+
+
+def rotated(v, pos, freq, rot, half):
+    """v float64 [T, H, dr]: the first rot dims turned by pos * freq."""
+    out = v.clone()
+    if not rot:
+        return out
+    a = pos[:, None, None] * freq[None, None, :rot // 2]
+    co, si = a.cos().float().double(), a.sin().float().double()
+    x, y = (v[..., :rot // 2], v[..., rot // 2:rot]) if half else (v[..., 0:rot:2], v[..., 1:rot:2])
+    first, second = x * co - y * si, y * co + x * si
+    if half:
+        out[..., :rot // 2], out[..., rot // 2:rot] = first, second
+    else:
+        out[..., 0:rot:2], out[..., 1:rot:2] = first, second
+    return out

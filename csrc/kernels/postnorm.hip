@@ -316,7 +316,9 @@ __global__ void __launch_bounds__(256) rmsnorm_cols_block_kernel(
 
 // The same for rows of at most 4096 columns in whole 16-byte pieces: a thread's pieces of the row, the
 // weight and the gate are all requested at once and stay in registers, so the row costs one round trip to
-// memory instead of one for each column of a thread, twice. 64 gated rows of 4096: 18.8 -> 6.3 us.
+// memory instead of one for each column of a thread, twice. 64 gated rows of 4096: 18.8 -> 6.3 us. Of many
+// rows a wave had one each, which it read twice: 600 gated rows of 4096 34 -> 15 us, 8199 125 -> 99, 4000 of
+// 1536 27.6 -> 27.3, 8199 of 1024 35 -> 28; without gates 20 -> 10, 81 -> 61.
 template <typename S>
 __global__ void __launch_bounds__(256) rmsnorm_cols_block4_kernel(
     S* __restrict__ out, const float* __restrict__ src, int lds, const S* __restrict__ w, int n,
@@ -670,7 +672,7 @@ extern "C" int dli_rmsnorm_cols(void* out, const float* src, int lds, const void
   if (n < 1 || groups < 1) return (int)hipErrorInvalidValue;
   const bool vec4 = n % 4 == 0 && lds % 4 == 0 && ldg % 4 == 0 && ldo % 4 == 0 &&
                     (((uintptr_t)out | (uintptr_t)src | (uintptr_t)w | (uintptr_t)gate) & 15) == 0;
-  if ((long)T * groups <= 512 && n >= 1024) {
+  if (((long)T * groups <= 512 || (vec4 && n <= 4096)) && n >= 1024) {
     if (vec4 && n <= 4096) {
       DT_SWITCH(dt,
                 (rmsnorm_cols_block4_kernel<u16><<<T * groups, 256, 0, st>>>(

@@ -110,3 +110,23 @@ def rotated(v, pos, freq, rot, half):
     else:
         out[..., 0:rot:2], out[..., 1:rot:2] = first, second
     return out
+
+
+# rows in a workgroup's registers (1024 to 4096 columns in quads) and the forms around it; several parts, gates
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1020, 1024, 1028, 1030, 2052, 4096, 4100])
+@pytest.mark.parametrize("groups", [1, 2])
+@pytest.mark.parametrize("rows", [3, 601])
+@pytest.mark.parametrize("gated", [False, True])
+def test_column_norm(gpu, n, groups, rows, gated):
+    g = torch.Generator(device=gpu).manual_seed(n + rows)
+    x = torch.randn(rows, n * groups, device=gpu, generator=g)
+    gate = torch.randn(rows, n * groups, device=gpu, generator=g) if gated else None
+    w = torch.randn(n * groups, device=gpu, generator=g).bfloat16()
+    got = hybrid.rmsnorm_cols(x, w, 1e-5, gate=gate, groups=groups)
+    v = x.double().view(rows, groups, n)
+    want = (v * torch.rsqrt(v.pow(2).mean(-1, keepdim=True) + 1e-5)).view(rows, -1) * w.double()
+    if gated:
+        want = want * torch.sigmoid(gate.double())
+    # bf16's rounding; the sum's and the few products' before it are 2^-24 each
+    assert bool(((got.double() - want).abs() <= (2.0 ** -8 + 2.0 ** -12) * want.abs() + 1e-30).all())

@@ -35,7 +35,8 @@ constexpr int MAXS = 8;          // streams
 // for the whole launch: read as scalars, beside the rows' requests and without a barrier before them.
 // Decode step, 64 rows of 3 x 4096: 7.5 us with a reduce launch of 5.4 before it -> 6.2. Prefill is bound
 // by memory: 8199 rows 199 us with the streams stored, 126 without, 5.1 and 4.8 TB/s; two mixes of which
-// one stores 397 -> 350 us.
+// one stores 397 -> 350 us. The outputs of sublayers are read and the streams stored past the caches, which
+// neither meets again: a mix in a step 125 -> 114 us.
 // y0 / prev0 (nullable): the sublayer before y's, whose write-back was not stored (xs null then).
 // src: the streams' rows, src_row floats a token and src_stream a stream (0: one row for all).
 template <typename S, int VEC, int NS>
@@ -95,15 +96,20 @@ __global__ void __launch_bounds__(1024) hyper_mix_kernel(
     };
     if (y0 != nullptr) {
       float yv[VEC];
+      if constexpr (VEC == 4) {
+        const f32x4 v = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(y0 + (long)t * dim + c));
 #pragma unroll
-      for (int u = 0; u < VEC; ++u) yv[u] = y0[(long)t * dim + c + u];
+        for (int u = 0; u < VEC; ++u) yv[u] = v[u];
+      } else {
+        yv[0] = y0[(long)t * dim + c];
+      }
       write_back(prev0, yv);
     }
     if (y != nullptr) {
       float yv[VEC];
       const float* yr = y + (long)t * ldy + c;
       if constexpr (VEC == 4) {
-        f32x4 v = *reinterpret_cast<const f32x4*>(yr);
+        f32x4 v = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(yr));
         for (int s = 1; s < nsplit; ++s) v += *reinterpret_cast<const f32x4*>(yr + s * ysplit);
 #pragma unroll
         for (int u = 0; u < VEC; ++u) yv[u] = v[u];
@@ -118,8 +124,9 @@ __global__ void __launch_bounds__(1024) hyper_mix_kernel(
       for (int r = 0; r < MS; ++r)
         if (r < ns) {
           if (VEC == 4)
-            *reinterpret_cast<f32x4*>(xo + (long)r * dim + c) =
-                f32x4{x[r][0], x[r][VEC > 1 ? 1 : 0], x[r][VEC > 2 ? 2 : 0], x[r][VEC > 3 ? 3 : 0]};
+            __builtin_nontemporal_store(
+                f32x4{x[r][0], x[r][VEC > 1 ? 1 : 0], x[r][VEC > 2 ? 2 : 0], x[r][VEC > 3 ? 3 : 0]},
+                reinterpret_cast<f32x4*>(xo + (long)r * dim + c));
           else
             xo[(long)r * dim + c] = x[r][0];
         }

@@ -364,17 +364,16 @@ __global__ void __launch_bounds__(256) scalar_step_kernel(ScalarRecArgs a) {
   f32x4 reg[R];
 #pragma unroll
   for (int r = 0; r < R; ++r) reg[r] = *reinterpret_cast<const f32x4*>(sp + (rg + RG * r) * D);
-  float at, bt = 1.f, em = 0.f;
+  float at, bt = 1.f, em = 0.f, m1 = 0.f;
   if (FORM == 1) {
     const float ig = a.cap * tanhf((zi + a.if_b[h]) / a.cap);
     const float fg = logsigmoid32(a.cap * tanhf((zf + a.if_b[H + h]) / a.cap));
     m0 = fresh ? 0.f : m0;
     n0 = fresh ? 0.f : n0;
-    const float m1 = fmaxf(fg + m0, ig);
+    m1 = fmaxf(fg + m0, ig);
     at = expf(fg + m0 - m1);
     bt = expf(ig - m1);
     em = expf(-m1);
-    if (tid == 0) np[D] = m1;
     if (first) { qs[i] = mine * (1.f / sqrtf((float)D)); ns[i] = n0; }
     else if (second) ks[i] = mine;
   } else {
@@ -401,6 +400,7 @@ __global__ void __launch_bounds__(256) scalar_step_kernel(ScalarRecArgs a) {
     nq = wave_sum(nq);
     inv = 1.f / (fmaxf(fabsf(at * nq + bt * kq), em) + 1e-6f);
     if (first) np[i] = at * n0 + bt * ks[i];
+    if (tid == 0) np[D] = m1;                  // (every thread has loaded it before the barrier)
   }
   f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll

@@ -667,7 +667,14 @@ def sample(logits, temperature, top_k, top_p, seeds, generator=None, ids=None, m
     value of each logit). temperature<=0 -> greedy. With ``ids``
     [B, V] the row holds candidates (vocab-parallel LM head) in ascending token-id order,
     and the sampled column is mapped to its token id (ties then break by token id exactly
-    as over the full vocabulary). ``maxima``: what ``head`` returned beside these logits."""
+    as over the full vocabulary). ``maxima``: what ``head`` returned beside these logits (fp32, without
+    ``ids``: its kernel reads rows of that type at the columns that the keys' blocks name)."""
+    if maxima is not None:
+        keys, bw = maxima
+        if (logits.dtype != torch.float32 or logits.stride(1) != 1 or ids is not None or bw < 1
+                or keys.dtype != torch.int32 or keys.device != logits.device or not keys.is_contiguous()
+                or tuple(keys.shape) != (logits.shape[0], -(-logits.shape[1] // bw))):
+            raise ValueError("sample: maxima are int32 keys [B, blocks] of fp32 logits [B, V], without ids")
     if not _use_native(logits):
         return R.sample(logits, temperature, top_k, top_p, generator=generator, seeds=seeds,
                         ids=ids)
@@ -676,7 +683,6 @@ def sample(logits, temperature, top_k, top_p, seeds, generator=None, ids=None, m
     if logits.dtype not in (torch.float32, torch.bfloat16):
         logits = logits.float()
     if maxima is not None:
-        keys, bw = maxima
         _native_call("dli_sample_blocks", _p(out), _p(logits), logits.stride(0), B, V,
                      _p(temperature), _p(top_k), _p(top_p), _p(seeds), _p(keys), keys.shape[1], bw,
                      _st())

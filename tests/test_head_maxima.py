@@ -119,3 +119,22 @@ def test_refused_shapes(gpu):
     h, w = torch.zeros(2, 512, device=gpu).bfloat16(), torch.zeros(64, 512, device=gpu).bfloat16()
     o, k = torch.zeros(2, 64, device=gpu), torch.zeros(2, 4, device=gpu, dtype=torch.int32)
     assert lib.dli_gemm_head(ops._p(h), 512, ops._p(w), 512, ops._p(o), 64, 2, 64, 512, 22, ops._p(k), ops._st())
+
+
+# logits of another type (half the bytes that the kernel would read), candidates of a sliced head, keys of other
+# rows, other blocks, another type or place
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+def test_maxima_of_other_logits_are_refused(device):
+    B, V, bw = 2, 64, 16
+    x, one = torch.randn(B, V, device=device), torch.ones(B, device=device)
+    keys = torch.zeros(B, V // bw, device=device, dtype=torch.int32)
+    args = (one, (5 * one).int(), 0.9 * one, one.long())
+    ids = torch.arange(V, device=device, dtype=torch.int32).expand(B, V)
+    for logits, top, more in ((x.bfloat16(), (keys, bw), {}), (x.half(), (keys, bw), {}), (x, (keys, bw), dict(ids=ids)),
+                              (x, (keys[:1], bw), {}), (x, (keys, 32), {}), (x, (keys, 0), {}), (x, (keys.long(), bw), {}),
+                              (x, (keys.t().contiguous().t(), bw), {}), (x.t().contiguous().t(), (keys, bw), {})):
+        with pytest.raises(ValueError):
+            ops.sample(logits, *args, maxima=top, **more)
+    if device != "cpu":
+        with pytest.raises(ValueError):
+            ops.sample(x, *args, maxima=(keys.cpu(), bw))

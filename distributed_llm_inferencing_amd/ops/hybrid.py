@@ -911,8 +911,8 @@ def hyper_mix(xs, y, prev, read, w, eps: float = 0.0, w_offset: float = 0.0, dty
     sublayer's vector, or ones for the plain sum) the weighted sum of the new streams is
     returned — RMS-normed times (w + w_offset) in the storage dtype when w is given, else fp32.
 
-    ``before`` (y, prev): a sublayer before y's whose write-back xs still lacks. ``source`` fp32
-    [T, D]: read as every stream in place of xs. ``store`` False: xs stays as it is (and may be the
+    ``before`` (y, prev): a sublayer before y's (fp32 [T, D], contiguous) whose write-back xs still lacks.
+    ``source`` fp32 [T, D], contiguous: read as every stream in place of xs. ``store`` False: xs stays as it is (and may be the
     shape alone, when nothing of it is read)."""
     if not isinstance(y, (torch.Tensor, type(None))):
         y = rows_of(y)
@@ -922,6 +922,10 @@ def hyper_mix(xs, y, prev, read, w, eps: float = 0.0, w_offset: float = 0.0, dty
         raise ValueError("hyper_mix needs the streams to read or to store")
     ref = source if source is not None else xs
     y0, prev0 = before or (None, None)
+    for name, rows in (("source", source), ("before", y0)):
+        if rows is not None and (rows.shape != (T, D) or rows.dtype != torch.float32 or rows.device != ref.device
+                                 or not rows.is_contiguous()):
+            raise ValueError(f"hyper_mix: {name} must be contiguous fp32 rows [{T}, {D}]")
     if not ref.is_cuda:
         new = source.unsqueeze(1).repeat(1, S, 1) if source is not None else xs if store else xs.clone()
         if before is not None:

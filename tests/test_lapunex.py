@@ -231,6 +231,19 @@ def test_held_write_back(device, S, D):
         H.hyper_mix((T, S, D), y1, v[0], v[1], w, 1e-5)
 
 
+# rows that the kernel would step over wrongly: apart, of another width, number or type
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+def test_held_rows_must_be_whole(device):
+    T, S, D = 5, 2, 32
+    x, v, w = torch.ones(T, D, device=device), torch.ones(S * (S + 2), device=device), torch.ones(D, device=device)
+    wide = torch.ones(T, 2 * D, device=device)
+    for bad in (wide[:, :D], wide, x[:4], x.double(), x.bfloat16()):
+        with pytest.raises(ValueError):
+            H.hyper_mix((T, S, D), x, v, v, w, 1e-5, source=bad, store=False)
+        with pytest.raises(ValueError):
+            H.hyper_mix((T, S, D), x, v, v, w, 1e-5, source=x, before=(bad, v), store=False)
+
+
 def test_yarn_frequencies_follow_their_definition():
     from distributed_llm_inferencing_amd.models.mixers import yarn_frequencies
     for r in (rot(), rot(16, 10000.0, (6.0, 1024, 24.0, 2.0)), rot(6, 7.0, None),

@@ -306,7 +306,9 @@ class HybridLM(TransformerLM):
         w = self.params["lm_head"]
         if replaced(self, "head_logits", _HEAD_LOGITS):
             return self.head_logits(h), None
-        if h.dtype == torch.bfloat16 and H.tuned_operands(h, w):
+        # (operands that do not match are for ``linear_any`` to refuse)
+        if (h.dtype == w.dtype == torch.bfloat16 and h.shape[1] == w.shape[1]
+                and h.stride(1) == w.stride(1) == 1 and H.tuned_operands(h, w)):
             return ops.head(h, w)
         return self.head_logits(h), None
 

@@ -138,3 +138,19 @@ def test_maxima_of_other_logits_are_refused(device):
     if device != "cpu":
         with pytest.raises(ValueError):
             ops.sample(x, *args, maxima=(keys.cpu(), bw))
+
+
+# operands that do not match never reach the tuned head, whose kernel takes their word for it
+def test_a_mismatched_head_weight_is_left_to_the_general_product(monkeypatch):
+    from distributed_llm_inferencing_amd.models import hybrid
+    calls = []
+    monkeypatch.setattr(hybrid.ops, "head", lambda h, w: calls.append("tuned"))
+    monkeypatch.setattr(hybrid.H, "linear_any", lambda h, w, **k: calls.append("general"))
+    m = object.__new__(hybrid.HybridLM)
+    h = torch.zeros(2, 128).bfloat16()
+    for w, want in ((torch.zeros(64, 128).bfloat16(), "tuned"), (torch.zeros(64, 128), "general"),
+                    (torch.zeros(64, 64).bfloat16(), "general"), (torch.zeros(64, 256).bfloat16(), "general"),
+                    (torch.zeros(128, 64).bfloat16().t(), "general")):
+        m.params = {"lm_head": w}
+        m.head(h)
+        assert calls.pop() == want and not calls

@@ -82,9 +82,9 @@ def linear_out(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     ``hyper_mix``, or any through ``rows_of``): [M, N], or, where the planned GEMM splits K, its partial sums
     [splits, M, N] in the shared workspace, which the add sums itself (one launch and one pass
     less). They must be consumed before the next GEMM."""
-    if (x.is_cuda and x.dtype == torch.bfloat16 and x.shape[1] % 64 == 0 and w.shape[0] % 4 == 0
-            and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and x.stride(1) == 1
-            and w.stride(1) == 1 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
+    # (operands that do not match are for ``linear_any`` to refuse)
+    if (x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and x.shape[1] == w.shape[1]
+            and w.shape[0] % 4 == 0 and x.stride(1) == w.stride(1) == 1 and tuned_operands(x, w)):
         (M, K), Nn = x.shape, w.shape[0]
         p = _gemm.plan(M, Nn, K, "f32")
         if p.splits > 1:

@@ -110,3 +110,30 @@ def test_persistent_tiles_of_every_width(gpu, M, N, K, epi, width):
         want = (act * up).reshape(M, N // 2)
     got = ops._gemm_native(x, w, epi, plan=G.GemmPlan("dli", 55, 1)).double()
     assert float((got - want).norm() / want.norm()) < (1e-5 if epi == "f32" else 2.0 ** -8)
+
+
+class OnGpu:
+    """A CPU tensor that says it is on the GPU."""
+    is_cuda = True
+
+    def __init__(self, t):
+        self.t = t
+
+    def __getattr__(self, name):
+        return getattr(self.t, name)
+
+
+# a split product's operands go to the kernel by address: those that do not match go to linear_any, which raises
+def test_partial_sums_of_mismatched_operands_are_refused(monkeypatch):
+    from distributed_llm_inferencing_amd.ops import hybrid as H
+    calls = []
+    monkeypatch.setattr(H._gemm, "plan", lambda *a: G.GemmPlan("dli", 22, 2))
+    monkeypatch.setattr(H._gemm, "workspace", lambda device, nbytes: torch.empty(nbytes, dtype=torch.uint8))
+    monkeypatch.setattr(H, "_call", lambda *a: calls.append(a[0]))
+    monkeypatch.setattr(H, "_st", lambda: None)
+    x = OnGpu(torch.zeros(8, 128).bfloat16())
+    assert H.linear_out(x, torch.zeros(64, 128).bfloat16()).shape == (2, 8, 64) and calls.pop() == "dli_gemm"
+    for w in (torch.zeros(64, 128), torch.zeros(64, 64).bfloat16(), torch.zeros(64, 256).bfloat16()):
+        with pytest.raises(ValueError):
+            H.linear_out(x, w)
+    assert not calls

@@ -467,11 +467,14 @@ def row_cut(M: int, N: int, K: int) -> int:
     bound by the weights' read. 0: all rows together. K = 4096, fp32 outputs, us together and cut: 4104 x
     4096 172 and 120, 8256 x 4096 265 and 212, 8199 x 16384 852 and 796, 1312 x 12288 172 and 121;
     8199 x 28672 (SiLU pairs) 1366 and 1332; K = 14336: 8199 x 4096 907 and 710. Not where as many rounds remain: 8199
-    x 6144 is 3.09 rounds, 355 and 307, but 4104 x 6144 1.59, 181 and 193. The last round's price is
+    x 6144 is 3.09 rounds, 355 and 307, but 4104 x 6144 1.59, 181 and 193. Nor where 512 rows would remain, which
+    run on a decode step's tiles: 513 x 28672 168 and 186, 640 x 32000 187 and 217. The last round's price is
     0.73 of a full one even if nearly empty (fewer busy CUs clock higher): 0.017 us a K on one, the other
-    side the weights at 5.5 TB/s and a launch."""
+    side the weights at 5.5 TB/s and a launch. The rows past the cut are summed in another order than those
+    before it (each order a valid fp32 one): a token's last bits depend on which side of it the step puts
+    the token. Pinned and tuned plans apply to each part by its own rows."""
     rest = M % 256
-    if M <= 512 or not 0 < rest <= STREAM_MAX_M or K % 64:
+    if M - rest <= 512 or not 0 < rest <= STREAM_MAX_M or K % 64:
         return 0
     rows, cols = M // 256, -(-N // 256)
     rounds = -(-(rows + 1) * cols // NUM_CUS) - -(-rows * cols // NUM_CUS)

@@ -97,6 +97,7 @@ def test_grouped_tiles_match_float64(gpu, tile):
 @pytest.mark.parametrize("M,N,K,cut", [
     (4104, 4096, 4096, 4096), (4224, 4096, 4096, 4096), (4225, 4096, 4096, 0), (4096, 4096, 4096, 0), (4353, 4096, 4096, 0),
     (8199, 28672, 4096, 8192), (4104, 6144, 4096, 0), (8199, 6144, 4096, 8192), (1312, 12288, 4096, 1280),
+    (513, 28672, 4096, 0), (640, 32000, 4096, 0), (769, 32000, 4096, 0), (1025, 32000, 4096, 1024),
     (513, 65536, 4096, 0), (300, 32768, 4096, 0), (2049, 128256, 4096, 0), (4104, 4096, 512, 0), (4104, 4096, 4104, 0)])
 def test_rows_that_would_begin_a_round_run_apart(M, N, K, cut):
     assert G.row_cut(M, N, K) == cut

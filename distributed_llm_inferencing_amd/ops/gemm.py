@@ -188,11 +188,14 @@ def _stream_plan(M: int, N: int, K: int, epi: str):
     20.0, 26.5 / 35.2, 28.5 / 29.0, 45 / 60, 177 / 209; 96 rows: 16.3 / 16.2, 23.8 / 24.4, 30.1 / 38.3, 31.9 / 33.0,
     47.5 / 63.5, 190 / 215. Above 96 rows the narrowest weights stay on two rows of tile 6 or one of tile 7
     (128 rows, 4096 x 4096 17.6 / 19.8, 4096 x 14336 35 / 39), from 65 rows the small ones on tile 5 (96 rows,
-    2048 x 2048 11.2 / 14.0)."""
+    2048 x 2048 11.2 / 14.0), above 96 rows all of short K (bias and GELU, 128 rows, 3072 x 768 7.7 / 10.9 on
+    tile 6, 9.8 on tile 0), from 33 rows the up to 256 columns of a low-rank factor, K = 1024 split too (64 rows, 256 x
+    1024 7.1 / 8.7 on tile 64 unsplit, 96 x 4096 8.6 / 9.2 on tile 64, 64 x 768 5.5 / 6.1)."""
     if K % 64:
         return None
     _, narrow, mid, wide, head = next(b for b in STREAM_BANDS if M <= b[0])
     fill = 3 * NUM_CUS // 4
+    few = M > 32 and N <= 256
     split = False
     if N >= 256 * NUM_CUS:
         tile = head
@@ -205,7 +208,7 @@ def _stream_plan(M: int, N: int, K: int, epi: str):
     else:
         split = True
         tile = mid
-        if M > 64 and N < 3072:
+        if M > 64 and N < 3072 or M > 96 and K <= 1024 or few:
             tile = 5
         elif M > 96 and N < 6144:
             tile = 7 if K > 8192 else 6
@@ -216,8 +219,9 @@ def _stream_plan(M: int, N: int, K: int, epi: str):
     tiles, splits = -(-M // bm) * -(-N // bn), 1
     most = 2 * NUM_CUS if tile == 5 else NUM_CUS
     # (K <= 1024: the second launch costs more than the shorter loop saves, 4096 x 1024 at 24 rows 6.1 / 7.8)
-    while (split and K > 1024 and tiles * splits * 2 <= most and K % (step * splits * 2) == 0
-           and K // (splits * 2) >= 512 and splits < 8):
+    while (split and (K > 1024 or few and K == 1024) and tiles * splits * 2 <= most
+           and K % (step * splits * 2) == 0 and K // (splits * 2) >= (256 if K == 1024 else 512)
+           and splits < 8):
         splits *= 2
     if epi == "splitk" and splits == 1 and K % (2 * step) == 0 and K >= 1024:
         splits = 2            # the fused reduce consumes partial slabs: need >= 2 slices

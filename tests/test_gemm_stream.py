@@ -18,6 +18,10 @@ from distributed_llm_inferencing_amd.ops.reference import interleave_gate_up
     (24, 128256, 4096, "f32", 62, 1), (64, 128256, 4096, "f32", 65, 1), (65, 128256, 4096, "f32", 68, 1), (129, 4096, 4096, "f32", 1, 8),
     # short K is not split, but where a fused reduce follows
     (24, 4096, 1024, "f32", 62, 1), (24, 4096, 1024, "splitk", 62, 2), (24, 4096, 768, "splitk", 62, 1),
+    # narrow weights: the 64-column tile with 3 stages
+    (97, 3072, 768, "bias_gelu", 5, 1), (128, 5120, 1024, "f32", 5, 1), (97, 4096, 1088, "f32", 6, 1), (96, 3072, 768, "f32", 70, 1),
+    (33, 256, 1024, "bias_gelu", 5, 4), (64, 96, 4096, "f32", 5, 8), (33, 64, 768, "none", 5, 1), (32, 256, 1024, "f32", 62, 1),
+    (33, 257, 1024, "f32", 64, 1), (128, 256, 2048, "f32", 5, 4),
     # up to 4 rows stay on the plain weight stream
     (5, 28672, 4096, "silu_mul", 61, 1), (4, 28672, 4096, "silu_mul", 31, 1), (4, 4096, 4096, "f32", 30, 2),
     (1, 28672, 4096, "silu_mul", 29, 1)])

@@ -30,9 +30,11 @@ constexpr int MAXS = 8;          // streams
 
 // One workgroup per token (256 threads; 1024 for the few wide rows of a decode step, which
 // are bound by latency). VEC = 4: 16-byte accesses of the fp32 rows (dim % 4 == 0). NS: the number of
-// streams where it is 2 to 4 (0: any). y may be nsplit partial sums, ysplit elements apart, of a
+// streams in the 16-byte form (0: any). y may be nsplit partial sums, ysplit elements apart, of a
 // split-K product: the launch and the pass of its reduce are spared. The coefficients are the same
 // for the whole launch: read as scalars, beside the rows' requests and without a barrier before them.
+// With the number known, 512 rows of 4096: 1 stream 14.6 -> 9.5 us, 5 29.9 ->
+// 23.9, 8 43.8 -> 32.9.
 // Decode step, 64 rows of 3 x 4096: 7.5 us with a reduce launch of 5.4 before it -> 6.2. Prefill is bound
 // by memory: 8199 rows 199 us with the streams stored, 126 without, 5.1 and 4.8 TB/s; two mixes of which
 // one stores 397 -> 350 us. The outputs of sublayers are read and the streams stored past the caches, which
@@ -306,8 +308,10 @@ extern "C" int dli_hyper_mix(const float* src, int one_row, float* xs, const flo
                                                ysplit, prev, read, (const S*)w, h, ns, dim, eps, \
                                                w_offset)
 #define HM_STREAMS(S)                                                                         \
-  (ns == 2 ? (void)HM_LAUNCH(S, 4, 2) : ns == 3 ? (void)HM_LAUNCH(S, 4, 3)                     \
-   : ns == 4 ? (void)HM_LAUNCH(S, 4, 4) : (void)HM_LAUNCH(S, 4, 0))
+  (ns == 1 ? (void)HM_LAUNCH(S, 4, 1) : ns == 2 ? (void)HM_LAUNCH(S, 4, 2)                     \
+   : ns == 3 ? (void)HM_LAUNCH(S, 4, 3) : ns == 4 ? (void)HM_LAUNCH(S, 4, 4)                   \
+   : ns == 5 ? (void)HM_LAUNCH(S, 4, 5) : ns == 6 ? (void)HM_LAUNCH(S, 4, 6)                   \
+   : ns == 7 ? (void)HM_LAUNCH(S, 4, 7) : (void)HM_LAUNCH(S, 4, 8))
   if (v4) DT_SWITCH2(dt, HM_STREAMS(u16), HM_STREAMS(float));
   else DT_SWITCH2(dt, (HM_LAUNCH(u16, 1, 0)), (HM_LAUNCH(float, 1, 0)));
 #undef HM_STREAMS

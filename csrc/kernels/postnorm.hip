@@ -63,7 +63,8 @@ __global__ void __launch_bounds__(256) prev_tokens_kernel(
 }
 
 // VEC = 4: whole 16-byte pieces of a row, and a row's hash once for four columns. 7200 rows of 4096 from
-// bf16 tables (0.3 GB) 155 -> 78 us.
+// bf16 tables (0.3 GB) 155 -> 78 us. Not below 2^19 elements, where it leaves CUs without a workgroup: 128 rows
+// of 1024 3.9 us, so 4.6.
 template <typename S, int VEC>
 __global__ void __launch_bounds__(256) embedding_bigram_kernel(
     float* __restrict__ x, S* __restrict__ xs, const int* __restrict__ ids,
@@ -318,7 +319,8 @@ __global__ void __launch_bounds__(256) rmsnorm_cols_block_kernel(
 // weight and the gate are all requested at once and stay in registers, so the row costs one round trip to
 // memory instead of one for each column of a thread, twice. 64 gated rows of 4096: 18.8 -> 6.3 us. Of many
 // rows a wave had one each, which it read twice: 600 gated rows of 4096 34 -> 15 us, 8199 125 -> 99, 4000 of
-// 1536 27.6 -> 27.3, 8199 of 1024 35 -> 28; without gates 20 -> 10, 81 -> 61.
+// 1536 27.6 -> 27.3, 8199 of 1024 35 -> 28; without gates 20 -> 10, 81 -> 61, of 1024 columns 513 rows 5.0 -> 3.7, 4000 7.8 ->
+// 8.4, 8199 17.3 -> 14.7.
 template <typename S>
 __global__ void __launch_bounds__(256) rmsnorm_cols_block4_kernel(
     S* __restrict__ out, const float* __restrict__ src, int lds, const S* __restrict__ w, int n,
@@ -604,7 +606,7 @@ extern "C" int dli_embedding_bigram(float* x, void* xs, const int* ids, const in
                                     hipStream_t st) {
   if (T <= 0) return 0;
   if (bigram != nullptr && (prev == nullptr || buckets < 1)) return (int)hipErrorInvalidValue;
-  const bool vec = dim % 4 == 0 &&
+  const bool vec = dim % 4 == 0 && (long)T * dim >= 1l << 19 &&
                    (((uintptr_t)x | (uintptr_t)xs | (uintptr_t)table | (uintptr_t)bigram) & 15) == 0;
   const int nb = (int)(((long)T * (vec ? dim / 4 : dim) + 255) / 256);
 #define EB_LAUNCH(S, V)                                                                        \

@@ -30,11 +30,13 @@ def test_rank_products(gpu, N, K, pad, off, f32):
 @pytest.mark.parametrize("dim", [40, 30, 4096])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("hashed", [True, False])
-def test_bigram_rows(gpu, dim, dtype, hashed):
+@pytest.mark.parametrize("many", [False, True])            # (from 2^19 elements in pieces)
+def test_bigram_rows(gpu, dim, dtype, hashed, many):
     g = torch.Generator(device=gpu).manual_seed(dim)
+    T = -(-(1 << 19) // dim) if many else 65
     t, b = (torch.randn(r, dim, device=gpu, generator=g).to(dtype) for r in (31, 18))
-    ids = torch.randint(0, 31, (65,), device=gpu, generator=g, dtype=torch.int32)
-    prev = torch.randint(-1, 31, (65,), device=gpu, generator=g, dtype=torch.int32)
+    ids = torch.randint(0, 31, (T,), device=gpu, generator=g, dtype=torch.int32)
+    prev = torch.randint(-1, 31, (T,), device=gpu, generator=g, dtype=torch.int32)
     x, xs = H.embedding_bigram(ids, prev if hashed else None, t, b if hashed else None, 17, 29, 5)
     want = t[ids.long()].float()
     if hashed:

@@ -285,7 +285,8 @@ __global__ void __launch_bounds__(512) prefill_attn32_kernel(
   // half block counted from the end and waves 4 to 7 its counterpart from the start: a SIMD, which
   // holds one wave of each, has the long one to itself when the short one is through. 32 heads, us:
   // 2048 tokens 78 -> 66, 1024 45 -> 40, the second 2048 of a prompt 150 -> 135, 1024 after 5000 192 -> 185.
-  // With more workgroups the longest first do it at full width: 3000 tokens 105, paired 129.
+  // With more workgroups the longest first do it at full width: 3000 tokens 105, paired 129. A sequence's only
+  // block is dealt to the SIMDs so anyway (256 tokens 16.2, paired 16.8).
   const int nhalf = (len + PL_ROWS / 2 - 1) / (PL_ROWS / 2), back = nhalf - 1 - (nblk - 1 - blk);
   const int half = wid < 4 ? back : nhalf - 1 - back;
   const int q0 = paired ? half * (PL_ROWS / 2) + (wid & 3) * PL_QROWS
@@ -497,7 +498,7 @@ static int launch_prefill(void* out, int out_stride, const void* qkv, int row_st
     prefill_attn32_kernel<128, PAGED><<<grid32, 512, 0, st>>>(
         (u16*)out, out_stride, (const u16*)qkv, row_stride, cu_seqlens, hq, hkv, sl2, ctx_lens,
         (const u16*)k_cache, (const u16*)v_cache, block_tables, bt_stride, block_size,
-        (long)blocks * hq * num_seqs <= 256);
+        blocks > 1 && (long)blocks * hq * num_seqs <= 256);
     DLI_RETURN_LAUNCH();
   }
   // waves per query head: pack 2 / 4 heads of one GQA group into a workgroup for short

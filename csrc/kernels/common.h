@@ -67,6 +67,12 @@ __device__ __forceinline__ uint4 load16_once(const u16* p) {
   return uint4{v[0], v[1], v[2], v[3]};
 }
 
+template <bool ONCE>
+__device__ __forceinline__ uint4 load16(const u16* p) {
+  if constexpr (ONCE) return load16_once(p);
+  return *reinterpret_cast<const uint4*>(p);
+}
+
 // four consecutive elements (8-byte aligned bf16, 16-byte aligned fp32)
 __device__ __forceinline__ void st4(u16* p, const f32x4 v) {
   uint2 pk;

@@ -106,3 +106,25 @@ def test_few_portions_over_many_keys_are_split():
     assert pays(1, 256, 256, 8, 8, 128, 8000) and not pays(1, 1024, 1024, 8, 8, 128, 8000)
     assert not pays(65, 576, 512, 32, 8, 128, 8000)                  # single tokens beside a portion
     assert not pays(64, 1024, 16, 32, 8, 128, 8000) and not pays(64, 64, 1, 32, 8, 128, 8000)
+
+
+# decode rows read past the caches (few keys can be seen) and through them (a bound of 2^30 keys), each kv head's
+# keys by one workgroup (up to 8 heads) and by several
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,dv", [(64, 64), (128, 128), (96, 192)])
+@pytest.mark.parametrize("heads,G", [(4, 2), (16, 2), (24, 2)])
+@pytest.mark.parametrize("bound", [301, 1 << 30])
+def test_decode_rows_past_and_through_the_caches(gpu, d, dv, heads, G, bound):
+    S, block, scale = 5, 16, d ** -0.5
+    pos = torch.tensor([0, 31, 300, 127, 7]).int()
+    g = torch.Generator().manual_seed(d + heads)
+    W = 300 // block + 1
+    bt = torch.randperm(S * W, generator=g).int().view(S, W)
+    kc, vc = (torch.randn(S * W * block, G * w, generator=g).bfloat16() for w in (d, dv))
+    q, cu = torch.randn(S, heads * d, generator=g).bfloat16(), torch.arange(S + 1).int()
+    want = R.window_attention(q, kc, vc, d, dv, heads, G, cu, pos, bt, block, 1 << 30, scale,
+                              out_dtype=torch.float32).double()
+    got = H.window_attention(q.to(gpu), kc.to(gpu), vc.to(gpu), d, dv, heads, G, cu.to(gpu), 1, pos.to(gpu),
+                             bt.to(gpu), block, bound, scale).double().cpu()
+    # weights and outputs rounded to bf16, half an ulp (2^-9) each
+    assert float((got - want).norm() / want.norm()) < 2 * 2.0 ** -9

@@ -1,8 +1,7 @@
-// Paged decode attention (one query token per sequence, GQA) on MFMA — SURVEY.md §2.4 K8.
+// Paged decode attention (one query token per sequence, GQA) on MFMA.
 //
-// Work decomposition: one wave per (sequence, kv head, KV split) item, 4 independent items per
-// workgroup; the wave walks the split's 32-token tiles. Per tile, with the GQA group of G <= 16 query
-// heads padded to 16 MFMA columns:
+// A wave walks the 32-token tiles of a (sequence, kv head) item or of a part of it. Per tile, with the GQA
+// group of G <= 16 query heads padded to 16 MFMA columns:
 //   S^T[tok, head] = K[tok, :] . Q[head, :]^T   (mfma_f32_16x16x32_bf16, K rows as the A
 //                                                operand straight from the cache: 16-B loads)
 //   online softmax along tokens (exp2 domain; max across the 4 lane groups = 2 shuffles)
@@ -12,10 +11,16 @@
 //                                                a per-wave LDS tile and read as the B operand
 //                                                with the transposing ds_read_b64_tr_b16, as
 //                                                in the prefill kernel)
-// With >1 split the per-split (m, l, O) go to a workspace merged by a second kernel.
-// decode_attn_fused_kernel (the decode-graph default) runs the same tile loop after a
-// prologue that replaces dli_splitk_rope_cache: the QKV GEMM's split-K slabs are reduced,
-// q/k rotated and k/v written to the paged cache inside the attention wave.
+// Who takes what:
+//   unsplit items, many of them     a wave each, 4 independent ones a workgroup (decode_attn_kernel)
+//   unsplit items, up to 256        a workgroup each, its waves' partial results merged in LDS
+//                                   (decode_attn_wg_kernel)
+//   KV splits, head dim 128         a workgroup each, likewise (decode_attn_split_kernel)
+//   KV splits, head dim 64          a wave each (decode_attn_kernel)
+// With splits their (m, l, O) go to a workspace merged by decode_reduce_kernel. The decode graph's default
+// are the fused forms of the first three (decode_attn_fused_kernel, decode_attn_split_kernel): the same tile
+// loop after a prologue that replaces dli_splitk_rope_cache, in which the QKV GEMM's split-K slabs are
+// reduced, q/k rotated and k/v written to the paged cache inside the attention wave.
 //
 // Layouts: q rows of stride q_stride (the fused QKV buffer), k_cache and v_cache
 // [nblk,Hkv,bs,hd] (token-major: the per-step cache write is a contiguous row),
@@ -56,12 +61,12 @@ __device__ __forceinline__ void decode_wg_range(int from, int to, int wv, int& s
   s_end = min(to, s_begin + per * DEC_TILE);
 }
 
-// KV splits of a step, from its contexts, for units of W waves (a workgroup of 4, or a wave). Ragged
-// contexts: split_tokens (whole tiles) deals the step's tiles to about DEC_TARGET waves, so that one
-// long context among short ones is cut as finely as the step can use; near-equal ones (the mean at
+// KV splits of a step, from its contexts, for units of W waves (head dim 128: a workgroup of 4; 64: a wave).
+// Ragged contexts: split_tokens (whole tiles) deals the step's tiles to about decode_ragged_units units, so
+// that one long context among short ones is cut as finely as the step can use; near-equal ones (the mean at
 // least 3/4 of the longest) are cut in the power of two that gives 2048 waves or more, which leaves no
-// short last split and CUs with equal shares (64 x 1000 tokens: 59 us, by DEC_TARGET 62; 24 of 500 -
-// 8000: 62 us, cut like equal ones 101). At least DEC_MIN_TILES tiles a split, and no sequence takes
+// short last split and CUs with equal shares (by waves, 64 x 1000 tokens: 59 us, dealt to DEC_TARGET 62; 24 of
+// 500 - 8000: 62 us, cut like equal ones 101). At least DEC_MIN_TILES tiles a split, and no sequence takes
 // more than num_splits. Sequence b has max(1, ceil(context / split_tokens)) equal ones, listed sequence
 // by sequence: `pair` of that list is (b, split); b = -1 past its end. Every wave works this out for
 // itself: a few loads and scans.
@@ -134,7 +139,7 @@ __device__ __forceinline__ DecSplit decode_split(const int* __restrict__ context
     if (find(i0, i0 + lane < B ? context_lens[i0 + lane] : 0)) return r;
   return r;
 }
-// units a split launch needs at most: the even splits, or DEC_TARGET and the rounding up of every
+// units a split launch needs at most: the even splits, or decode_ragged_units and the rounding up of every
 // sequence
 template <int W> static inline long decode_split_items(int items, int num_splits) {
   const long even = (long)items * decode_even_splits<W>(items), ragged = decode_ragged_units<W>(items) + items;
@@ -331,7 +336,9 @@ __device__ __forceinline__ void decode_end_list(float* __restrict__ ws_ml, int b
 // MINW = 4 waves per SIMD: <= 128 VGPRs, so every item of a 512-sequence batch (4096 waves)
 // is resident at once (measured 7 % faster than the 166-VGPR / 2-waves build at ctx 66). A kernel of 2
 // waves a SIMD that walked items and requested the next tile, across them too, served contexts of 768 and
-// more until the loads here went past the caches: 256 of 984 195 us, this 168; 512 of 33 to 99 36, 33
+// more until the loads here went past the caches: 256 of 984 195 us, this 168; 512 of 33 to 99 36, 33.
+// Head dim 64, whose splits come here too: pipelined and past the caches; before, 24 contexts of 1000 and 12
+// heads 27.6 us, so 23.4; 64 of 500 27.8, 24.3; 512 of 33 20.9, 17.7; one of 33 8.5, 7.3
 template <int HD, int MINW, bool PIPE>
 __global__ void __launch_bounds__(256, MINW) decode_attn_kernel(
     u16* __restrict__ out, const u16* __restrict__ q, int q_stride,
@@ -344,12 +351,14 @@ __global__ void __launch_bounds__(256, MINW) decode_attn_kernel(
   __shared__ __attribute__((aligned(16))) u16 vtile_all[DEC_WAVES][DEC_TILE * VROW];
   u16* vt = vtile_all[threadIdx.x >> 6];
   const int lane = threadIdx.x & 63;
-  // one WAVE per work item (sequence, kv head, KV split): no LDS, no barriers, so every
+  // one WAVE per work item (sequence, kv head, at head dim 64 also KV split): no barriers, so every
   // resident wave of the chip streams a different (seq, head) pair concurrently
   const int item = blockIdx.x * DEC_WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int kvh = item % hkv;
   DecSplit sp{item / hkv, 0, split_tokens, 0};
-  if (num_splits > 1) sp = decode_split<1>(context_lens, B, hkv, num_splits, item / hkv, lane);
+  // (head dim 128 with splits: decode_attn_split_kernel)
+  const bool listed = HD == 64 && num_splits > 1;
+  if (listed) sp = decode_split<1>(context_lens, B, hkv, num_splits, item / hkv, lane);
   if (sp.b < 0 || sp.b >= B) return;                           // wave-uniform exit
   const int b = sp.b, split = sp.split;
   split_tokens = sp.split_tokens;
@@ -373,8 +382,8 @@ __global__ void __launch_bounds__(256, MINW) decode_attn_kernel(
   }
   decode_attn_core<HD, PIPE>(qf, vt, lane, b, kvh, split, G, ctx, s_begin, s_end, out, k_cache,
                        v_cache, block_tables, max_blocks, hq, hkv, block_size, scale_log2,
-                       sp.last == 0 ? 1 : num_splits, ws_o, ws_ml);
-  if (num_splits > 1) decode_end_list(ws_ml, b, hq, kvh, G, num_splits, split, sp.last, lane);
+                       listed && sp.last > 0 ? num_splits : 1, ws_o, ws_ml);
+  if (listed) decode_end_list(ws_ml, b, hq, kvh, G, num_splits, split, sp.last, lane);
 }
 
 // One (sequence, kv head) item, or one KV split of it, per workgroup of WPI waves: wave wv walks the
@@ -838,9 +847,9 @@ extern "C" int dli_decode_attention(void* out, const void* q, int q_stride, cons
   DLI_RETURN_LAUNCH();
 }
 
-// Fused split-K QKV reduce + RoPE + KV-cache write + decode attention (head dim 128, RoPE models;
-// workspace as dli_decode_attention's where num_splits > 1, apart from ws): ws = the QKV GEMM's fp32 slabs [splits, B, (hq + 2 hkv) * 128], or
-// with splits == 0 the bf16 QKV rows [B, (hq + 2 hkv) * 128] of an unsplit GEMM.
+// Fused split-K QKV reduce + RoPE + KV-cache write + decode attention (head dim 128, RoPE models; workspace
+// as dli_decode_attention's where num_splits > 1, apart from ws): one launch, and the splits' merge where
+// there are some. ws = the QKV GEMM's fp32 slabs [splits, B, (hq + 2 hkv) * 128], or with splits == 0 the bf16 QKV rows [B, (hq + 2 hkv) * 128] of an unsplit GEMM.
 // fmt: 0 = fp32 slabs (or the bf16 rows when splits == 0), 1 = fp16 x 1/16 slabs (EPI_SLAB16)
 extern "C" int dli_decode_attention_fused(void* out, const void* ws, int splits,
                                           const int* positions, const int* slot_mapping,

@@ -390,8 +390,8 @@ def linear_rope_attention(x, w, positions, slot_mapping, cos_sin, k_cache, v_cac
                           block_tables, context_lens, max_context: int, hq, hkv, hd, scale):
     """Decode step, one fused pass after the QKV GEMM: the split-K slabs (or, for an unsplit
     plan, the bf16 QKV rows) are reduced, q and k rotated, k/v written to the paged cache and
-    attention computed by ONE kernel per layer (``dli_decode_attention_fused``) instead of
-    ``linear_rope_cache`` + ``decode_attention``. Returns the attention output [B, hq*hd], or
+    attention computed by one launch per layer (``dli_decode_attention_fused``), with KV splits a
+    second one that merges them, instead of ``linear_rope_cache`` + ``decode_attention``. Returns the attention output [B, hq*hd], or
     None where the fused kernel does not apply (the caller then runs the two-kernel path):
     split counts other than 2 / 4, head dim != 128."""
     xr = x.residual if isinstance(x, NormedRows) else x
@@ -513,8 +513,8 @@ _pipelined = 2
 
 
 def decode_pipelined(v: int) -> int:
-    """Once chose between two decode attention kernels; one serves every setting now, which is only
-    kept and returned."""
+    """Once chose between two decode attention kernels; one serves every setting now. Kept for callers
+    that still set it: the setting is stored and the previous one returned, nothing else."""
     global _pipelined
     old, _pipelined = _pipelined, int(v)
     return old
@@ -565,22 +565,20 @@ def prefill_attention_paged(qkv, cu_seqlens, max_seqlen: int, context_lens, bloc
 
 
 def decode_num_splits(B: int, hkv: int, max_context: int) -> int:
-    """KV split slots per sequence: 1 where the B*Hkv items (one wave each) or short contexts fill
-    the chip unsplit, else what the longest context may need."""
+    """KV split slots per sequence: 1 where the B*Hkv items fill the chip unsplit or contexts are short,
+    else what the longest context may need."""
     items = B * hkv
     splits = 1
-    # tiny batches (batch-1 latency): >= 512 tokens per split, so graphs captured for a
-    # 512-token table take the single-pass kernel with the fused QKV reduce / RoPE / cache
-    # prologue (the 4-split form cost rope + attention + merge = 23 us per layer at B = 1,
-    # profiles/r3/prof_b1_summary.txt)
+    # tiny batches (batch-1 latency): >= 512 tokens per split, so that graphs captured for a 512-token
+    # table take the unsplit kernel, which needs no merge behind it
     min_tok = 512 if B <= 4 else 128
     while items * splits < 2048 and max_context // (splits * 2) >= min_tok and splits < 64:
         splits *= 2
     if splits == 1:
         return 1
-    # slots a sequence may use, of at least 64 tokens: the kernel deals the step's actual contexts
-    # to at most max(even splits, 3072 + B * hkv) waves, fewer where contexts or slots run out, so
-    # one long context among short ones takes many slots
+    # slots a sequence may use, of at least 64 tokens: the kernel deals the step's actual contexts to the
+    # even splits or, if they differ, to about 768 workgroups (head dim 128; 3072 waves at 64), fewer where
+    # contexts or slots run out, so one long context among short ones takes many slots
     return max(splits, min(64, max_context // 64, 8192 // items))
 
 

@@ -569,18 +569,17 @@ def test_decode_attention_paged(gpu, hq, hkv, hd, bs, lens):
     scale = 1 / math.sqrt(hd)
     q = qkv[:, : hq * hd].reshape(len(lens), hq, hd)
     ref = R.decode_attention(q, kc, vc, tables, ctx, scale).reshape(len(lens), -1)
-    # pipelined and one-tile-per-round kernels; the latter unsplit at hd 128 as a workgroup
-    # per (sequence, kv head) (small batches, WPI 4) or a wave per item (WPI 1)
-    for pipe, wpi in ((1, 0), (0, 4), (0, 1)):
-        old = ops.decode_pipelined(pipe)
-        old_form = ops.decode_form(wpi)
+    # unsplit at hd 128 the automatic form, a workgroup per (sequence, kv head) (4) and a wave per item (1),
+    # which differ in their tile loop (the next tile requested behind this one's use, and in turn); with
+    # splits a workgroup each at hd 128; at hd 64 a wave each, split or not
+    for form in (0, 4, 1):
+        old_form = ops.decode_form(form)
         try:
             for splits in (1, 2, 4):
                 out = ops.decode_attention(qkv, kc, vc, tables, ctx, max(lens), hq, hkv, hd,
                                            scale, num_splits=splits)
                 close(out, ref, rtol=2e-2, atol=2e-2)
         finally:
-            ops.decode_pipelined(old)
             ops.decode_form(old_form)
 
 
@@ -1175,11 +1174,13 @@ def test_prefill_attention_long(gpu, lens, hq, hkv):
         close(out, ref, rtol=2e-2, atol=2e-2)
 
 
-def test_decode_attention_32k_context(gpu):
+@pytest.mark.parametrize("hd", [128, 64])
+def test_decode_attention_32k_context(gpu, hd):
     """Decode against a 32k-token paged context (and a short one in the same batch), with
-    the default split heuristic and forced splits."""
+    the default split heuristic, forced splits (a workgroup each at hd 128, a wave at 64) and none
+    (a workgroup or a wave per item)."""
     torch.manual_seed(22)
-    hq, hkv, hd, bs = 32, 8, 128, 16
+    hq, hkv, bs = 32, 8, 16
     lens = [32768, 77]
     nblk = sum(-(-n // bs) for n in lens) + 4
     kc = rnd(nblk, hkv, bs, hd, dev=gpu)
@@ -1198,15 +1199,15 @@ def test_decode_attention_32k_context(gpu):
     scale = 1 / math.sqrt(hd)
     q = qkv[:, : hq * hd].reshape(len(lens), hq, hd)
     ref = R.decode_attention(q, kc, vc, tables, ctx, scale).reshape(len(lens), -1)
-    for pipe in (1, 0):                      # pipelined and one-tile-per-round kernels
-        old = ops.decode_pipelined(pipe)
+    for form in (1, 4):
+        old = ops.decode_form(form)
         try:
-            for splits in (None, 8, 32):
+            for splits in (None, 1, 8, 32):
                 out = ops.decode_attention(qkv, kc, vc, tables, ctx, max(lens), hq, hkv, hd,
                                            scale, num_splits=splits)
                 close(out, ref, rtol=2e-2, atol=2e-2)
         finally:
-            ops.decode_pipelined(old)
+            ops.decode_form(old)
 
 
 @pytest.mark.parametrize("hq,hkv,hd,bs,chunks", [

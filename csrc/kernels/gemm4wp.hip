@@ -17,7 +17,7 @@
 
 // NJ: tiles of 256 x 32 NJ (wave tiles of 128 x 16 NJ). The narrower ones are for the counts of tiles
 // that 256 columns leave at little more than a round of the chip, or at little over half of one: see
-// narrowest(). Their schedule is the same with fewer MFMAs, W fragments and W pieces.
+// width_of(). Their schedule is the same with fewer MFMAs, W fragments and W pieces.
 template <int EPI, int NJ>
 __global__ void __launch_bounds__(256, 1) gemm4wp_kernel(
     const u16* __restrict__ A, int lda, const u16* __restrict__ W, int ldw,
@@ -272,7 +272,8 @@ static int cu_count() {
 // The tile width (8, 6 or 5 times 32 columns) whose rounds take least: a round's price is its width times
 // what the narrower schedule costs more (fewer MFMAs between the same barriers: 9 and 13 %), the last one's
 // by how many CUs it keeps, and little less for few of them, which clock higher. 256 columns unless
-// another is 3 % better. (7 is hardly ever best, and then by as little.) N = 4096, us at 8 / 7 / 6 / 5: 2304 rows, K = 14336 241 / 226 / 218 / 202,
+// another is 3 % better. (7 is hardly ever best, and then by as little.) N = 4096, one weight again and again, us at 8 /
+// 7 / 6 / 5 (four weights in turn, as in a step: 4352 rows, K = 14336 551 and 412, K = 4096 163 and 125): 2304 rows, K = 14336 241 / 226 / 218 / 202,
 // K = 4096 83 / 79 / 74 / 65; 4352 rows 535 / 476 / 424 / 402 and 164 / 149 / 136 / 127; 5120 rows 168 / 153 /
 // 149 / 175; 8192 rows, two whole rounds at 8, 195 / 240 / 224 / 240. N = 6144, K = 4096: 2816 rows 164 / 149 /
 // 134 / 121, 4096 rows 172 / 159 / 157 / 182. ops/gemm.py's persistent_width is its copy.

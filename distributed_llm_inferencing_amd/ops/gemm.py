@@ -268,10 +268,10 @@ def _heuristic(M: int, N: int, K: int, epi: str) -> GemmPlan:
             pays = K > 2048 or (K >= 1024 and tiles > NUM_CUS) or N % 64 != 0   # (tile 22 takes no such N)
         else:
             pays = epi not in ("bias", "bias_gelu")
-        # (long K from 4096 rows on where its narrower tiles save part of a round: 4352 x 4096, K = 14336
-        # 402 us against 560)
+        # (long K from 4096 rows on where its narrower tiles save part of a round: 4352 x 4096, K = 14336,
+        # bf16 outputs 412 us against 551, fp32 489 against 577)
         if (pays and splits == 1 and M >= LARGE_M and K % 128 == 0
-                and (K <= 8192 or M < 4096 or persistent_width(M, N, epi in PAIR_EPIS) < 256)
+                and (K <= 8192 or M < 4096 or persistent_width(M, N, epi in PAIR_EPIS, device_cus()) < 256)
                 and (M < 16384 or N >= 16384) and tile_ok(55, epi)):
             return GemmPlan("dli", 55, 1)
         return GemmPlan("dli", 22, splits)
@@ -446,15 +446,24 @@ def plan(M: int, N: int, K: int, epi: str) -> GemmPlan:
     return _plan_cache.get(key) or _heuristic(M, N, K, epi)
 
 
+@functools.lru_cache(maxsize=None)
+def device_cus() -> int:
+    """CUs of the current GPU as the kernels see them (a partition has fewer); 256 without one."""
+    if torch.cuda.is_available():
+        return torch.cuda.get_device_properties(torch.cuda.current_device()).multi_processor_count
+    return NUM_CUS
+
+
 @functools.lru_cache(maxsize=8192)
-def persistent_width(M: int, N: int, pairs: bool) -> int:
-    """Columns of the tiles that the persistent kernel (tile 55) takes: gemm4wp.hip's width_of."""
+def persistent_width(M: int, N: int, pairs: bool, cus: int = NUM_CUS) -> int:
+    """Columns of the tiles that the persistent kernel (tile 55) takes on ``cus`` CUs: gemm4wp.hip's
+    width_of."""
     best, least = 256, 0.0
     for nj, price in ((8, 1.0), (6, 1.09 * 6 / 8), (5, 1.13 * 5 / 8)):
         if pairs and nj & 1:
             continue
-        whole, rest = divmod(-(-M // 256) * -(-N // (32 * nj)), NUM_CUS)
-        x = rest / NUM_CUS
+        whole, rest = divmod(-(-M // 256) * -(-N // (32 * nj)), cus)
+        x = rest / cus
         last = 0.0 if not rest else 0.66 + 0.25 * x + 0.09 * x ** 3 if whole else 0.8 + 0.2 * x ** 3
         c = (whole + last) * price
         if nj == 8:

@@ -87,7 +87,17 @@ def test_persistent_tile_widths_are_the_kernels(gpu):
     for M in (1, 256, 257, 1290, 2112, 2816, 4352, 5000, 8199):
         for N in (32, 160, 4096, 4100, 6144, 14336, 28672):
             for pairs in (False, True):
-                assert G.persistent_width(M, N, pairs) == width(M, N, int(pairs)), (M, N, pairs)
+                assert G.persistent_width(M, N, pairs, G.device_cus()) == width(M, N, int(pairs)), (M, N, pairs)
+
+
+# 17 x 16 = 272 tiles of 256 columns: a second round of 256 CUs, hardly filled, but one of 272 and of 304
+def test_persistent_width_goes_by_the_devices_cus(monkeypatch):
+    assert [G.persistent_width(4352, 4096, False, cus) for cus in (256, 272, 304)] == [160, 256, 256]
+    for cus, tile in ((256, 55), (304, 22)):
+        monkeypatch.setattr(G, "device_cus", lambda: cus)
+        G._heuristic.cache_clear()
+        assert G._heuristic(4352, 4096, 14336, "f32").tile == tile
+    G._heuristic.cache_clear()
 
 
 # every width of the persistent kernel's tiles, with partial tiles in both directions, two to twenty K-tiles and

@@ -475,9 +475,9 @@ __global__ void __launch_bounds__(256) swa_prefill16_kernel(SwaArgs a) {
 }
 
 // One query token a sequence. Workgroup = 4 waves of one (sequence, kv head, chunk of HP heads,
-// key split); a wave takes every fourth 32-key tile of the split. ONCE: keys and values past the caches,
-// see launch_swa.
-template <int DK, int DV, int HP, bool ONCE>
+// key split); a wave takes every fourth 32-key tile of the split. PAST: what it reads past the caches (0
+// nothing, 1 the values, 2 the keys too), see launch_swa.
+template <int DK, int DV, int HP, int PAST>
 __global__ void __launch_bounds__(256) swa_decode_kernel(SwaArgs a) {
   constexpr int KK = DK / 32, LPR = DV / 8;        // lanes that cover a V row with 16 bytes each
   constexpr int KPI = 64 / LPR, NV = 32 / KPI;     // keys per V load of a wave, V loads per tile
@@ -523,7 +523,7 @@ __global__ void __launch_bounds__(256) swa_decode_kernel(SwaArgs a) {
       const long r = __shfl(row, 16 * u + fr, 64);
 #pragma unroll
       for (int kk = 0; kk < KK; ++kk) {
-        const uint4 v = load16<ONCE>(a.k + r * a.k_stride + kvh * DK + kk * 32 + fq * 8);
+        const uint4 v = load16<(PAST > 1)>(a.k + r * a.k_stride + kvh * DK + kk * 32 + fq * 8);
         kf[u][kk] = *reinterpret_cast<const bf16x8*>(&v);
       }
     }
@@ -533,7 +533,7 @@ __global__ void __launch_bounds__(256) swa_decode_kernel(SwaArgs a) {
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       const long r = __shfl(row, i * KPI + vk, 64);
-      vv[i] = load16<ONCE>(a.v + r * a.v_stride + kvh * DV + (lane % LPR) * 8);
+      vv[i] = load16<(PAST > 0)>(a.v + r * a.v_stride + kvh * DV + (lane % LPR) * 8);
     }
     f32x4 sa[2];
     float tmax = -INFINITY;
@@ -733,16 +733,20 @@ int launch_swa(SwaArgs a, int num_seqs, int max_seqlen, hipStream_t st) {
   if (max_seqlen == 1) {
     const int rep = a.H / a.G, hp = rep <= 4 ? 4 : 8;
     dim3 grid(a.G * ((rep + hp - 1) / hp), num_seqs, a.nsplit);
-    // A step's few keys and values are read past the caches. Not where they may be more than 48 MB, for contexts
-    // of different lengths (16 of 63 to 8000 keys, 8 kv heads of 128: 75 us, past the caches 89; 24 of
-    // 63 to 1000 22; equal lengths 0 to 2 % the other way), nor, from 16 MB on, where a kv head's keys are
-    // read by several workgroups (16 heads a kv head: 128 of 8000 307 us, 370; 128 of 300 35, 34).
-    // 4 of 300 12.0 us, past the caches 11.0; 32 of 64 7.3, 6.5; 8 of 1000 20.0, 19.0.
-    const long bytes = (long)num_seqs * a.G * ((long)a.window + a.keep) * (DK + DV) * 2;
-    const bool once = bytes <= (rep > hp ? 16l << 20 : 48l << 20);
-#define SWA_DECODE(HP, ONCE) swa_decode_kernel<DK, DV, HP, ONCE><<<grid, 256, 0, st>>>(a)
-    if (hp == 4) once ? (void)SWA_DECODE(4, true) : (void)SWA_DECODE(4, false);
-    else once ? (void)SWA_DECODE(8, true) : (void)SWA_DECODE(8, false);
+    // Keys and values are read past the caches: 4 of 300 keys 12.0 -> 11.0 us, 32 of 64 7.3 -> 6.5. Not the keys of
+    // few long sequences, whose rows arrive in two pieces and which the tail of a step of different lengths waits
+    // for (8 kv heads of 128, 16 of 63 to 8000 keys 89 us, the keys through the caches 77, the values too 80); from
+    // 192 (sequence, kv head) pairs on the whole chip reads, and what the keys push out of the caches costs the rest of the
+    // step more (24 of 2083 keys on 8 kv heads, two such layers of a step: 660 us, 693). Not where several
+    // workgroups read a kv head's keys and the second one would find them (16 heads a kv head: 128 of 8000 keys
+    // 370 us, 308 through the caches; 16 heads on one of 128 and 256, 64 of 1000 keys, 49 MB, 33 and 30; 4 of 8000
+    // on two, 33 MB, 36 and 45).
+    const long keys = (long)a.window + a.keep, bytes = (long)num_seqs * a.G * keys * (DK + DV) * 2;
+    const bool all = bytes <= 48l << 20 || ((long)num_seqs * a.G >= 192 && keys < 4096);
+#define SWA_DECODE(HP, PAST) swa_decode_kernel<DK, DV, HP, PAST><<<grid, 256, 0, st>>>(a)
+    if (rep > 8 && bytes > 36l << 20) SWA_DECODE(8, 0);
+    else if (hp == 4) all ? (void)SWA_DECODE(4, 2) : (void)SWA_DECODE(4, 1);
+    else all ? (void)SWA_DECODE(8, 2) : (void)SWA_DECODE(8, 1);
 #undef SWA_DECODE
     if (a.nsplit > 1) {
       const long n = (long)num_seqs * a.H * DV / 4;

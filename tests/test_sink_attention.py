@@ -108,8 +108,8 @@ def test_few_portions_over_many_keys_are_split():
     assert not pays(64, 1024, 16, 32, 8, 128, 8000) and not pays(64, 64, 1, 32, 8, 128, 8000)
 
 
-# decode rows read past the caches (few keys can be seen) and through them (a bound of 2^30 keys), each kv head's
-# keys by one workgroup (up to 8 heads) and by several
+# decode rows read past the caches (few keys can be seen) and, with a bound of 2^30 keys, the keys through them, or all
+# where a kv head's keys are read by several workgroups (more than 8 heads)
 @pytest.mark.gpu
 @pytest.mark.parametrize("d,dv", [(64, 64), (128, 128), (96, 192)])
 @pytest.mark.parametrize("heads,G", [(4, 2), (16, 2), (24, 2)])

@@ -86,6 +86,7 @@ extern "C" int dli_gemm(const void* A, int lda, const void* W, int ldw, void* C,
     return (int)hipErrorInvalidValue;
   if (epi_pairs(epi) && N % 32) return (int)hipErrorInvalidValue;
   if (epi == EPI_CLAMP && (bias == nullptr || group_off != nullptr)) return (int)hipErrorInvalidValue;
+  if ((epi == EPI_BIAS || epi == EPI_BIAS_GELU) && bias == nullptr) return (int)hipErrorInvalidValue;
   if (splits > 1 && ws == nullptr) return (int)hipErrorInvalidValue;
   if (groups < 1) groups = 1;
   if (epi == EPI_F32) bias = nullptr;              // (where the block maxima go: dli_gemm_head)

@@ -217,6 +217,8 @@ def _gemm_native(x, w, epi: str, bias=None, out=None, plan: Optional[G.GemmPlan]
     M, K = x.shape
     Nn = w.shape[-2]
     out_n = Nn // 2 if epi in G.PAIR_EPIS else Nn
+    if bias is None and epi in ("bias", "bias_gelu", "clamp_mul"):
+        raise ValueError(f"{epi} needs its bias: the kernel reads it by address")
     if out is None:
         dt = torch.float32 if epi == "f32" else x.dtype
         out = torch.empty(M, out_n, dtype=dt, device=x.device)

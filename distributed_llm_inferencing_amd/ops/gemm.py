@@ -563,7 +563,9 @@ def autotune(shapes, weights: dict, device, iters: int = 6, log=None,
                 bt = (slots // 16).to(torch.int32).unsqueeze(1).contiguous()
                 ctx = torch.ones(M, dtype=torch.int32, device=device)
                 sc = 1.0 / math.sqrt(hd)
-        bias = (torch.ones(1, dtype=torch.float32, device=device) if epi == "clamp_mul" else None)
+        # what the epilogue reads by address: clamp_mul's limit, a bias of the output's columns
+        bias = (torch.ones(1, dtype=torch.float32, device=device) if epi == "clamp_mul" else
+                torch.zeros(N, dtype=w0.dtype, device=device) if epi in ("bias", "bias_gelu") else None)
         best = None
         timed = []                                  # (ms, plan, run) of every valid candidate
         t_shape = time.perf_counter()

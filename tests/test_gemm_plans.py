@@ -147,3 +147,46 @@ def test_partial_sums_of_mismatched_operands_are_refused(monkeypatch):
         with pytest.raises(ValueError):
             H.linear_out(x, w)
     assert not calls
+
+
+# the timing of a product with a bias reads one: an address of none is a fault on the GPU (a width of K that gives
+# candidates, as GPT-2's 768 does and its tiny variant's does not)
+@pytest.mark.parametrize("epi", ["bias", "bias_gelu", "clamp_mul", "f32"])
+@pytest.mark.parametrize("M,N,K", [(1, 96, 768), (64, 96, 768), (2048, 256, 768)])
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+def test_timed_products_have_their_bias(device, monkeypatch, epi, M, N, K):
+    seen = []
+    native = ops._gemm_native
+
+    def product(x, w, epi, bias=None, plan=None, **more):
+        seen.append(None if bias is None else (bias.numel(), bias.dtype, bias.device.type))
+        if device != "cpu":
+            assert seen[-1] is not None or epi == "f32"
+            native(x, w, epi, bias=bias, plan=plan, **more)
+    monkeypatch.setattr(ops, "_gemm_native", product)
+    if device == "cpu":
+        monkeypatch.setattr(ops, "benchmark", lambda run, **k: (run(), 1.0)[1])
+    w = torch.ones(N, K, device=device).bfloat16()
+    more = dict(candidates=G.prefill_candidates) if M > 1024 else {}
+    got = G.autotune([(M, N, K, epi)], {(N, K): w}, torch.device(device), iters=1, cold_bytes=1, **more)
+    want = {"clamp_mul": (1, torch.float32, device), "f32": None}.get(epi, (N, torch.bfloat16, device))
+    assert seen and all(s == want for s in seen) and (M, N, K, epi) in got
+
+
+def test_a_missing_bias_is_refused(monkeypatch):
+    monkeypatch.setattr(ops, "_native_call", lambda *a: pytest.fail("reached the kernel"))
+    x, w = torch.zeros(8, 768).bfloat16(), torch.zeros(96, 768).bfloat16()
+    for epi in ("bias", "bias_gelu", "clamp_mul"):
+        with pytest.raises(ValueError):
+            ops._gemm_native(x, w, epi, plan=G.GemmPlan("dli", 5, 1))
+
+
+@pytest.mark.gpu
+def test_the_library_refuses_a_missing_bias(gpu):
+    from distributed_llm_inferencing_amd.ops import _native
+    lib = _native.require_native()
+    x, w, o = (torch.zeros(r, 768, device=gpu).bfloat16() for r in (8, 96, 8))
+    for tile in (0, 22, 34, 45, 30, 55, 62):
+        for epi in ("bias", "bias_gelu"):
+            assert lib.dli_gemm(ops._p(x), 768, ops._p(w), 768, ops._p(o), 96, 4, 96, 768, G.EPI[epi], tile, 1, None,
+                                None, None, 1, ops._st()) != 0

@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""Headline benchmark (BASELINE.json): output tokens/sec (whole node) + p50 request latency,
+"""Headline benchmark: output tokens/sec (whole node) + p50 request latency,
 Llama-3-8B bf16, 1/2/4/8 GPU-workers (layer-sharded pipeline over RCCL for N > 1).
 
 Workload = the reference's request shape (worker/app.py:297-305, views.py:351): synthetic

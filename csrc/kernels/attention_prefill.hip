@@ -1,4 +1,4 @@
-// Causal variable-length (packed) GQA prefill attention on MFMA — SURVEY.md §2.4 K7.
+// Causal variable-length (packed) GQA prefill attention on MFMA.
 //
 // Reads q/k/v straight out of the fused QKV activation (row stride = (Hq+2Hkv)*hd) after
 // the in-place RoPE, so no separate K/V copies exist. A workgroup = 4 waves = 64 query rows

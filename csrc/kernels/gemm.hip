@@ -1,5 +1,5 @@
 // bf16 GEMM on CDNA4 matrix cores: C[M,N] = A[M,K] . W[N,K]^T (+ fused epilogue).
-// SURVEY.md §2.4 K4/K9-K12 (dense projections) and K16 (MoE grouped GEMM).
+// Dense projections and the experts' grouped products.
 //
 // Structure (cdna_hip_programming.md §5):
 //  * WM x WN waves (2x2 = 256 threads, or 2x4 / 4x2 = 512 threads for 256-wide tiles); block
@@ -24,7 +24,7 @@
 // Files: gemm_common.h (shared epilogue / split-K pieces), gemm_tiles.hip (ids 0-21, 23-25),
 // gemm_stream.hip (60-72: few rows, weights streamed), gemm8p.hip (22, 26-28), gemm4w.h +
 // gemm4w.hip (34, 41, 45), gemm4wp.hip (55: persistent 45), gemv.hip (29-33 and the fused batch-1
-// combine). The losing 4-wave A/B variants of round 4 are documented, not built
+// combine). The losing 4-wave variants are documented, not built
 // (profiles/r4/gemm4w/).
 #include "gemm_common.h"
 

@@ -49,7 +49,7 @@ __device__ __forceinline__ uint4 buf_ld16(const void* base, int nbytes, int voff
 // Diagnostics only: 64 = no LDS-DMA in the K loop, 128 = also no barrier / waits (wrong
 // results, timing of the remaining work), 131072 = s_memtime stamps (correct results).
 // Only tiles 34 (VAR 8), 41 (8 | 32) and 45 (8 | 4096) are instantiated; the other VAR bits
-// are the round-4 A/B variants, kept for diagnostics (measurements: profiles/r4/gemm4w/).
+// are variants that lost, kept for diagnostics (measurements: profiles/r4/gemm4w/).
 template <int EPI, int VAR = 0>
 __global__ void __launch_bounds__(256, 1) gemm4w_kernel(
     const u16* __restrict__ A, int lda, const u16* __restrict__ W, int ldw,

@@ -1,5 +1,5 @@
 // Persistent form of the 4-wave two-barrier 256x256 GEMM (tile 55; tile 45 = gemm4w_kernel
-// <EPI, 8 | 4096> is its one-tile-per-workgroup form). the prefill
+// <EPI, 8 | 4096> is its one-tile-per-workgroup form). Tile by tile the prefill
 // projections pay, per 256x256 tile, a prologue (the first two K-tiles' LDS-DMA latency with
 // the matrix pipe idle) and an epilogue (the 128-256 KB store tail) that a workgroup-per-tile
 // grid cannot hide. Here one workgroup per CU walks tiles v = blockIdx.x, + gridDim.x, ...

@@ -3,8 +3,8 @@
 #include "gemm_common.h"
 
 // ---------------------------------------------------------------------------------------
-// Skinny GEMM for M <= 4 rows (batch-1 / tiny-batch decode: SURVEY.md §7.4 "the decode
-// skinny GEMM must approach the HBM roofline"): every weight byte is used M times, so the
+// Skinny GEMM for M <= 4 rows (batch-1 / tiny-batch decode, which must
+// approach the HBM roofline): every weight byte is used M times, so the
 // kernel is a weight stream, not an MFMA tile. A workgroup (4 waves) owns R = 4 * RW output
 // rows of W over one K slice; in a wave, lane l covers the 8 K-elements [8 (l + 64 s),
 // +8) of step s for its RW rows: RW 16-B nontemporal weight loads per step (the weights are

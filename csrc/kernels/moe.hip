@@ -1,4 +1,4 @@
-// Mixture-of-experts routing / permutation kernels (Mixtral) — SURVEY.md §2.4 K15/K16.
+// Mixture-of-experts routing / permutation kernels (Mixtral).
 //   route   : softmax over E router logits -> top-k -> renormalise (HF MixtralSparseMoeBlock)
 //   align   : per-expert counts, exclusive offsets, permuted position of every (token, slot)
 //   gather  : x_perm[p] = x[src[p]]            (16-B row copies)

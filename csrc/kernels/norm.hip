@@ -1,4 +1,4 @@
-// RMSNorm / LayerNorm (+ fused residual add) for gfx950 — SURVEY.md §2.4 K2/K3.
+// RMSNorm / LayerNorm (+ fused residual add) for gfx950.
 //
 // Memory-bound: one workgroup per row, 16-B vector loads (8 x bf16 per lane), the row is
 // held in registers between the reduction and the normalised write (one HBM read of x and

@@ -1,5 +1,5 @@
 // RoPE (rotate-half, HF Llama convention) applied IN PLACE to q and k inside the fused QKV
-// activation, fused with the paged KV-cache write — SURVEY.md §2.4 K5/K6.
+// activation, fused with the paged KV-cache write.
 //
 // One lane owns 8 dims of the first half of a head and the matching 8 dims of the second
 // half (16-B loads of each), so a head of 128 dims is 8 lanes and the rotation needs no

@@ -1,4 +1,4 @@
-// On-device token sampling with HF `generate` semantics — SURVEY.md §2.4 K13/K14.
+// On-device token sampling with HF `generate` semantics.
 //
 // HF warper order (transformers/generation/utils.py): Temperature -> TopK -> TopP -> softmax
 // -> multinomial. One 512-thread workgroup per row (vocab up to ~256k), no full-vocab sort:

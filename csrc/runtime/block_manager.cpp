@@ -1,7 +1,7 @@
 // Paged KV-cache block allocator + per-step metadata builders (host C++).
 //
-// Replaces HF's per-request `past_key_values` tensors (grown by torch.cat every step,
-// SURVEY.md §2.4 K6) with a fixed pool of `num_blocks` blocks of `block_size` tokens per
+// Replaces HF's per-request `past_key_values` tensors (grown by torch.cat every
+// step) with a fixed pool of `num_blocks` blocks of `block_size` tokens per
 // layer, sized from HBM at engine start (288 GB per MI355X => millions of tokens). The
 // scheduler (Python) asks this allocator for blocks; the batch builders below emit the
 // int32 block tables and slot mappings the HIP kernels consume, so per-step metadata for a

@@ -1,5 +1,4 @@
-// RCCL point-to-point for the pipeline data plane, called directly ("RCCL ...
-// called directly from a C++ comm module"; the reference has no data plane at all — its
+// RCCL point-to-point for the pipeline data plane, called directly (the reference has no data plane at all — its
 // "shards" exchange nothing, master/dashboard/views.py:318-355).
 //
 // One communicator per pipeline (ranks = stages). Sends and receives of a tick are enqueued
@@ -108,8 +107,8 @@ int dli_comm_destroy(void* comm) {
   return rc(a->comm_destroy((ncclComm_t)comm));
 }
 
-// Failure handling ("RCCL async-error polling (ncclCommGetAsyncError) with
-// communicator abort + rebuild"). dli_comm_async_error: 0 healthy, else -(ncclResult_t) of
+// Failure handling: RCCL async-error polling (ncclCommGetAsyncError) with communicator
+// abort + rebuild. dli_comm_async_error: 0 healthy, else -(ncclResult_t) of
 // the communicator's asynchronous error (a peer died, a network / xGMI fault). The pipeline
 // watchdog polls it next to the stage liveness probe. dli_comm_abort: ncclCommAbort — frees
 // the communicator WITHOUT waiting for the peers and makes its kernels still queued on a

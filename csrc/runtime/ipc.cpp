@@ -1,6 +1,6 @@
 // Device-memory mailbox transport between the processes of one node (hipIpc): the
-// pipeline / expert-parallel data plane without RCCL ("loopback transport
-// (same C++ interface): stage-ranks on one GPU exchange via device memcpy / IPC handles").
+// pipeline / expert-parallel data plane without RCCL; ranks that share
+// one GPU exchange through the same interface.
 // The reference has no data plane at all — its "shards" exchange nothing
 // (master/dashboard/views.py:318-355, worker/app.py:332-372).
 //
@@ -40,7 +40,7 @@
 // LL buffers): no XCD's L2 ever holds a copy, every load and store goes to memory. Flags are
 // written with system-scope release stores after the payload kernel and polled with
 // system-scope acquire loads. DLI_IPC_MEM = uncached (default) | fine | coarse selects the
-// allocation (coarse = the round-3 layout, for A/B only); the kind in use is reported by
+// allocation (coarse: for comparison only); the kind in use is reported by
 // dli_ipc_mem_kind.
 //
 // Every message carries a 16-byte header {sequence, bytes}. Each rank keeps a 64-bit

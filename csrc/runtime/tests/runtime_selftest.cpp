@@ -1,5 +1,5 @@
 // Host-side self-test of the C++ runtime (block allocator + safetensors parser), built with
-// AddressSanitizer on the host (SURVEY.md §5.2: sanitizers for the C++ layer; GPU ASan is
+// AddressSanitizer on the host (sanitizers for the C++ layer; GPU ASan is
 // not available on this pool). Randomised allocator stress with invariant checks, and a
 // parser fuzz: every truncation of a valid header, corrupted length fields and
 // out-of-range data offsets must be rejected without any out-of-bounds access.

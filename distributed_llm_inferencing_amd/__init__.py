@@ -1,7 +1,7 @@
 """distributed_llm_inferencing_amd — an MI355X-native (gfx950 / CDNA4) master/worker sharded
 LLM inference hub with the capabilities and HTTP API of MihirPanpatil/Distributed-LLM-Inferencing.
 
-Layers (see README.md / SURVEY.md §7):
+Layers:
     control/   Flask master: node registry, request queue, dispatcher, dashboard (API-compatible)
     worker/    per-GPU Flask worker with the reference's /health /load_model /load_shard ...
     engine/    continuous-batching scheduler, paged KV cache, hipGraph decode runner

@@ -1,7 +1,6 @@
 """In-tree native build: hipcc for gfx950, no torch headers, no JIT cache.
 
-Produces two shared objects inside the package (they travel to the GPU box with the
-repo snapshot; they are git-ignored):
+Produces two shared objects inside the package (git-ignored):
 
 * ``lib/libdli_kernels.so`` — every HIP/CDNA4 kernel in ``csrc/kernels`` behind a plain
   ``extern "C"`` ABI (called through ctypes with torch's current HIP stream).
@@ -167,7 +166,7 @@ def build(force: bool = False, jobs: int = 0, verbose: bool = True) -> dict:
     out = {}
     # --no-undefined: a kernel whose host-side handle hipcc failed to emit (it happens
     # silently, e.g. for a lambda capturing an __amdgpu_buffer_rsrc_t) fails the link here
-    # instead of the library failing to load on the GPU box
+    # instead of the library failing to load on the GPU's host
     out["kernels"] = _build_group(k_srcs, k_hdrs, k_flags, LIBDIR / "libdli_kernels.so", jobs,
                                   extra=("-Wl,--no-undefined",), kind="kernels")
     if r_srcs:

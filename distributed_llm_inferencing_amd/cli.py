@@ -1,7 +1,7 @@
 """Command-line entry: ``python -m distributed_llm_inferencing_amd.cli <command>``.
 
-Replaces the reference's ``manage.py`` (runserver / shard_model, SURVEY.md M4) and its
-docker-compose topology (X6: master + 2 worker containers + redis) with a single-node
+Replaces the reference's ``manage.py`` (runserver / shard_model) and its
+docker-compose topology (master + 2 worker containers + redis) with a single-node
 launcher for an 8-GPU MI355X box.
 
     serve-master    [--port 8000]                       Flask master (dashboard + API)
@@ -15,11 +15,10 @@ launcher for an 8-GPU MI355X box.
                     API and reports the stages as shards; --shard-dir serves the files
                     `shard-model` exported (rank r <- D/shard_<r>/)
     serve-cluster   --model M --gpus 8 --dp K [--base-port 5000] [--master URL]
-                    K data-parallel replicas, each a pipeline of gpus/K stages (SURVEY.md
-                    §2.5 "DP replicas"); every replica head registers as a node and the
+                    K data-parallel replicas, each a pipeline of gpus/K stages; every replica head registers as a node and the
                     master's dispatcher load-balances across them (least in flight)
     serve-expert    --model mixtral-8x7b --gpus N [--base-port 5000] [--master URL]
-                    expert-parallel deployment (BASELINE.json config 5): N ranks, one per
+                    expert-parallel deployment: N ranks, one per
                     GPU, each an HTTP worker on port base+rank holding experts
                     [r E/N, (r+1) E/N) and all attention weights; every rank registers
                     as a node and reports its expert shard, the master balances requests
@@ -30,7 +29,7 @@ launcher for an 8-GPU MI355X box.
     join-pipeline   --model M --shard-dir D --nodes URL0,URL1,... [--rendezvous tcp://H:P]
                     assign shard i of an export to node i over the worker API (/load_shard
                     with a "pipeline" spec): the N worker processes form one RCCL ring and
-                    node 0 serves the model (SURVEY.md §2.2 W5)
+                    node 0 serves the model
     loadgen         --master URL --model M [--requests N] [--concurrency C | --rate R]
                     end-to-end load through the master API: tokens/s, p50/p99 latency
     trace-run       --model DIR --dtype bfloat16|float32 --out DIR --max-tokens N

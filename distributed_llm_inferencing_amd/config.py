@@ -1,7 +1,7 @@
 """Process-wide configuration read from environment variables.
 
 Keeps every environment variable name the reference reads, with the same
-semantics, and adds the MI355X-specific knobs of SURVEY.md §5.6:
+semantics, and adds the MI355X-specific knobs:
 
 reference (master, ``master/master/settings.py:8-101``):
     SECRET_KEY, DEBUG, REDIS_HOST, REDIS_PORT, REDIS_DB, MODEL_CACHE_DIR

@@ -1,4 +1,4 @@
-"""Dispatcher: queue consumers that route each request to a worker node (SURVEY.md M13).
+"""Dispatcher: queue consumers that route each request to a worker node.
 
 Reference behaviour (``master/dashboard/views.py:305-455``): mark ``processing``; if loaded
 ``ModelShard`` rows exist for the model, POST ``/inference`` with ``shard_ids`` to the FIRST
@@ -14,7 +14,7 @@ and error strings here, with these fixes:
   to the health monitor, instead of failing (the reference fails over only at selection
   time, views.py:99-105,389-391);
 * the worker's bearer token is sent when ``AUTH_KEY`` is configured (the reference never
-  sends it, so enabling worker auth broke dispatch, SURVEY.md W2);
+  sends it, so enabling worker auth broke dispatch);
 * a fixed pool of consumer threads instead of one unbounded thread per submit.
 """
 from __future__ import annotations

@@ -1,4 +1,4 @@
-"""Failure detector / heartbeat monitor (SURVEY.md M14, §5.3).
+"""Failure detector / heartbeat monitor.
 
 Reference: health is probed only when the UI polls ``/api/nodes/status/``; one
 ``RequestException`` marks a node inactive FOREVER (inactive nodes are never re-probed,

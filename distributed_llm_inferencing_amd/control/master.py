@@ -1,7 +1,7 @@
 """Master HTTP service: API-compatible replacement of the reference's Django master.
 
 Routes, form fields, JSON shapes, status codes and messages follow
-``master/dashboard/urls.py:6-16`` and ``views.py`` (SURVEY.md Appendix A):
+``master/dashboard/urls.py:6-16`` and ``views.py``:
 
     GET  /                              dashboard page (counts + 5 recent)
     GET  /nodes/                        node management page

@@ -1,4 +1,4 @@
-"""Request queue with Redis-compatible semantics (SURVEY.md §2.3 X3).
+"""Request queue with Redis-compatible semantics.
 
 The reference configures Redis (``settings.py:95-97``, ``docker-compose.yml:57-63``) but
 never uses it: every submit spawns an unbounded ``threading.Thread`` (``views.py:233``).

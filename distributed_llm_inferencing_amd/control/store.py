@@ -10,7 +10,7 @@ Mirrors the Django models of the reference (``master/dashboard/models.py:4-62``)
                   status in {pending, processing, completed, failed}, created_at, completed_at)
                   with mark_completed / mark_failed.
 
-The reference has no migrations directory (SURVEY.md §2.1 M5), so its tables would not exist
+The reference has no migrations directory, so its tables would not exist
 after ``migrate``; here the schema is created on startup. One database thread owns the
 connection and serialises every access (the reference mutated sqlite from unbounded
 threads, §5.2).

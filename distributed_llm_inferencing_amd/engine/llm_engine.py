@@ -1,7 +1,7 @@
 """Single-pipeline-stage inference engine (one GPU, or CPU): the worker's model runtime.
 
-Replaces the reference worker's ``model.generate`` call path (``worker/app.py:278-308``,
-L1 in SURVEY.md §1) with: C++ paged-KV allocator + continuous-batching scheduler +
+Replaces the reference worker's ``model.generate`` call path (``worker/app.py:278-308``)
+with: C++ paged-KV allocator + continuous-batching scheduler +
 hipGraph decode on our HIP kernels. Multi-GPU pipelines use the same pieces through
 ``parallel/pipeline.py``.
 """
@@ -118,7 +118,7 @@ class LLMEngine:
                                           device=self.device)
         max_model_len = min(max_model_len, cfg.max_position)
         if num_blocks is None:
-            # KV pool sized from free HBM (SURVEY.md §5.7), optionally capped
+            # KV pool sized from free HBM, optionally capped
             num_blocks = auto_num_blocks(cfg, cfg.num_layers, block_size, self.device,
                                          kv_fraction, cap_tokens=max_kv_tokens or 0)
         self.state_slots = None

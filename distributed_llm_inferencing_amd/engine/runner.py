@@ -3,7 +3,7 @@
 Decode steps have a fixed shape per batch-size bucket, so each bucket's whole stage forward
 (all layers, and on the last stage the LM head + sampler) is captured once into a
 ``torch.cuda.CUDAGraph`` (a hipGraph on ROCm) and replayed: one graph launch per step per
-stage instead of ~10 kernel launches per layer (SURVEY.md §3.2). All per-step metadata
+stage instead of ~10 kernel launches per layer. All per-step metadata
 lives in ONE static int32 device buffer refreshed by ONE pinned H2D copy before replay.
 Padded rows (bucket > live sequences) carry slot = -1 (no KV write) and context 0.
 

@@ -1,5 +1,4 @@
-"""End-to-end load generator for the serving stack (SURVEY.md §7.1 "bench/ load generator":
-tokens/s + p50/p99 through the master's public API).
+"""End-to-end load generator for the serving stack (tokens/s + p50/p99 through the master's public API).
 
 Submits requests to a running master (``POST /api/inference/submit/``, form-encoded exactly
 as the reference UI does), polls ``/api/inference/status/<id>/`` and reports request

@@ -2,7 +2,7 @@
 
 The reference loads arbitrary HF checkpoints through ``AutoModelForCausalLM``
 (``worker/app.py:121``); offline we define the architectures ourselves from the
-public HF ``config.json`` values (SURVEY.md §2.4 table) and random-init them.
+public HF ``config.json`` values and random-init them.
 
 Names accepted by ``get_config`` are case-insensitive and include the HF hub ids
 the reference UI would send (``gpt2``, ``meta-llama/Meta-Llama-3-8B`` ...).

@@ -3,7 +3,7 @@
 One ``TransformerLM`` instance owns layers ``[layer_start, layer_end)`` of a model plus the
 embedding (first stage) and final norm + LM head + sampler (last stage). It is the
 replacement for the HF ``AutoModelForCausalLM.forward`` + ``generate`` hot loop the
-reference worker runs (``worker/app.py:297-305``; SURVEY.md §3.2), re-built on our ops:
+reference worker runs (``worker/app.py:297-305``), re-built on our ops:
 
     embed -> [ (add_)rmsnorm -> QKV GEMM -> RoPE+KV write -> attention -> O GEMM
               -> add_rmsnorm -> gate/up GEMM with fused SiLU*mul -> down GEMM ] x L

@@ -13,7 +13,7 @@ globals: embed [V, D], (gpt2) pos_embed [P, D], final_norm [D], (gpt2) final_nor
 
 Random init mirrors HF ``_init_weights`` (normal(0, 0.02), norms = 1, biases = 0) and is
 generated directly on the target device, per stage, so a 70B stage never materialises the
-full model anywhere (SURVEY.md §7.4 item 7).
+full model anywhere.
 """
 from __future__ import annotations
 

@@ -201,7 +201,7 @@ def ptr(t) -> int | None:
 
 
 # DLI_DEBUG_SYNC=1: synchronise after every native launch and name the op whose kernel
-# faulted (SURVEY.md §5.2 debug mode; pair with AMD_SERIALIZE_KERNEL=3 set before HIP init,
+# faulted (debug mode; pair with AMD_SERIALIZE_KERNEL=3 set before HIP init,
 # which utils.debug.enable_debug_sync() does). Not usable inside hipGraph capture.
 _DEBUG_SYNC = os.environ.get("DLI_DEBUG_SYNC", "0") == "1"
 

@@ -705,7 +705,7 @@ def candidate_plans(M: int, N: int, K: int, epi: str):
     # isolated decode timings (M = 512 LM head 4-7 %) but cost the step 1.8 % in a same-box
     # bench A/B (42,548 without vs 41,790 / 41,653 tok/s with, profiles/r4/bench/)
     excl_env = os.environ.get("DLI_GEMM_EXCLUDE")
-    # 34 too (round 5): the 4-wave family wins isolated cold-weight timings within the noise
+    # 34 too: the 4-wave family wins isolated cold-weight timings within the noise
     # but loses in the decode graph — down at M = 512 ran 70.4 us on tile 34 against 56.9 on
     # the 8-phase tile 22, the LM head 433 vs 407 (profiles/r5/s12/wave_summary.txt vs
     # profiles/r4/prof/llama_b512_head.wave.txt); the autotune flipped between them run to run

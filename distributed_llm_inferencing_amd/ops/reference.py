@@ -1,8 +1,8 @@
 """Pure-PyTorch reference implementations of every hot op (fp32 math).
 
-These are (a) the CPU execution path (config 1: gpt2 on a CPU worker, and every
-CPU test), and (b) the golden each HIP kernel is tested against
-(SURVEY.md §4 tier T3). They define the tensor layouts the HIP kernels share:
+These are (a) the CPU execution path (gpt2 on a CPU worker, and every CPU
+test), and (b) the golden each HIP kernel is tested against.
+They define the tensor layouts the HIP kernels share:
 
 * hidden states: ``[T, D]`` (tokens of all sequences flattened, bf16)
 * fused QKV activations: ``[T, (Hq + 2*Hkv) * hd]``
@@ -16,7 +16,7 @@ CPU test), and (b) the golden each HIP kernel is tested against
   features ``[16i, 16i+16)`` and rows ``[32i+16, 32i+32)`` the matching up
   features, so a GEMM tile owns both halves of every SiLU·mul pair.
 
-The implicit HF ops these replace are listed in SURVEY.md §2.4 (K1-K16).
+They replace the ops that HF ``generate`` runs implicitly.
 """
 from __future__ import annotations
 

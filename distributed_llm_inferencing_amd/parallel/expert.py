@@ -1,5 +1,5 @@
 """Expert parallelism for Mixtral: experts mapped to GPU ranks, all-to-all over xGMI
-(SURVEY.md §2.4 C4, §2.5 "Expert parallel"; the reference has no
+(the reference has no
 MoE at all — its compute is HF ``generate`` at ``worker/app.py:297-305``).
 
 Layout: data-parallel attention + expert-parallel MoE. Every rank holds the full attention
@@ -342,7 +342,7 @@ class ExpertParallelEngine:
         self.board = self._open_board()
         self.control_plane = "shm" if self.board is not None else "gloo"
         self.lockstep_s = 0.0
-        # liveness watchdog (ADVICE r5): a peer that dies mid-forward would leave this rank's
+        # liveness watchdog: a peer that dies mid-forward would leave this rank's
         # queue spinning in its mailbox waits for the whole wait budget; the board knows every
         # rank's pid, so a death aborts the mailboxes within ~0.2 s and the next step raises
         self.dead_peer: Optional[str] = None

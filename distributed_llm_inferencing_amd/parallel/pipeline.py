@@ -1,6 +1,6 @@
 """Layer-sharded pipeline-parallel serving: one process per MI355X, stages over RCCL.
 
-This is what the reference's "sharded inference" was meant to be (SURVEY.md §3.3: offline
+This is what the reference's "sharded inference" was meant to be (offline
 layer split ``shard_model.py:55-109``, ``metadata.json``, ``/load_shard`` at
 ``worker/app.py:139-206``, dispatch to shard holders at ``master/dashboard/views.py:318-355``;
 execution never actually coordinated the shards) — made real:
@@ -27,7 +27,7 @@ execution never actually coordinated the shards) — made real:
 
 ``LocalPipeline`` runs the same partitioned stages and tick schedule in ONE process (all
 stages on one device): the loopback transport used to test pipeline correctness on a single
-GPU or CPU (SURVEY.md §4 T5).
+GPU or CPU.
 """
 from __future__ import annotations
 
@@ -711,7 +711,7 @@ def run_stage_loop(stage: StageWorker, channel) -> None:
 # ------------------------------------------------------------------------------ shard files
 def read_shard_dir(shard_dir: str, rank: int, world: int) -> Tuple[ModelConfig, dict, Path]:
     """(config, metadata, path) of ``<shard_dir>/shard_<rank>`` as written by ``shard-model``
-    (reference layout, SURVEY.md Appendix C); the files' partition must have ``world``
+    (reference layout); the files' partition must have ``world``
     stages."""
     d = Path(shard_dir) / f"shard_{rank}"
     meta = json.loads((d / "metadata.json").read_text())

@@ -1,5 +1,4 @@
-"""Tensor parallelism (optional, for ablation against the
-layer-sharded pipeline — not the north star).
+"""Tensor parallelism (optional, beside the layer-sharded pipeline).
 
 Megatron-style split of every Llama layer over N ranks:
     wqkv   column-parallel by heads (Hq/N query heads, Hkv/N kv heads per rank)

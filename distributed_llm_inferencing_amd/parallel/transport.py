@@ -1,4 +1,4 @@
-"""Inter-stage transport for the layer-sharded pipeline (SURVEY.md §2.4 C1-C3, §5.8).
+"""Inter-stage transport for the layer-sharded pipeline.
 
 The reference has NO inter-shard data plane (its "sharded" path runs shard 0 alone,
 ``worker/app.py:334-336``). Here a pipeline step moves over two planes:
@@ -222,7 +222,7 @@ class PipeChannel:
         on a death abort the data plane AT ONCE (every wait this rank's queue holds on the
         dead peer is released, the device plane turns sticky-failed) so the next ``check``
         of the tick loop raises. Detection within ~``period_s`` instead of a wait budget or
-        the RCCL watchdog's ``DLI_PP_TIMEOUT_S``. SURVEY.md §5.3."""
+        the RCCL watchdog's ``DLI_PP_TIMEOUT_S``."""
         if self.world == 1 or self._wd is not None:
             return
         if self.ring is None and self.rccl is None:
@@ -582,7 +582,7 @@ def init_distributed(backend: Optional[str] = None, device: Optional[torch.devic
     joins a pipeline when the master assigns it a shard (``/load_shard`` with a "pipeline"
     spec, ``worker/server.py``).
 
-    Failure detection (SURVEY.md §5.3): data-plane operations get a bounded timeout
+    Failure detection: data-plane operations get a bounded timeout
     (``DLI_PP_TIMEOUT_S``, default 600 s), so a stage that dies mid-session turns a blocked
     exchange into an error: RCCL's watchdog aborts the communicator when the timeout fires
     (torch's ``TORCH_NCCL_ASYNC_ERROR_HANDLING`` default), gloo raises as soon as the dead

@@ -1,4 +1,4 @@
-"""Shard export / import in the reference's on-disk layout (SURVEY.md Appendix C):
+"""Shard export / import in the reference's on-disk layout:
 
     <output_dir>/<model_name with '/' -> '_'>/
         tokenizer/                     (reference: shard_model.py:29-33)

@@ -1,4 +1,4 @@
-"""Offline tokenizers (SURVEY.md §2.4 K17: CPU-side).
+"""Offline tokenizers (CPU-side).
 
 There is no network and no HF hub cache, so the default is a deterministic byte-level
 tokenizer that works for any vocabulary size:

@@ -1,4 +1,4 @@
-"""Debug modes (SURVEY.md §5.2): serialised kernels and per-op fault attribution.
+"""Debug modes: serialised kernels and per-op fault attribution.
 
     DLI_DEBUG_SYNC=1   every native op synchronises after launch and reports its own name
                        when a kernel faulted (ops/_native.py); graphs are disabled

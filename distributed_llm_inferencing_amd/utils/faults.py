@@ -1,4 +1,4 @@
-"""Fault injection (SURVEY.md §5.3: the reference had none).
+"""Fault injection (the reference had none).
 
 ``DLI_FAULT`` holds comma-separated rules ``site:action[:arg]``; every component calls
 ``check(site, **ctx)`` at its injection point:

@@ -1,4 +1,4 @@
-"""Structured logging (SURVEY.md §5.5): JSON lines to ``logs/<component>.log`` plus a
+"""Structured logging: JSON lines to ``logs/<component>.log`` plus a
 human-readable console handler. The reference promised ``master/logs/django.log`` and
 ``worker/logs/worker.log`` (README.md:175,185) but never configured them."""
 from __future__ import annotations

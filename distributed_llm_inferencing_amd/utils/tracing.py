@@ -1,4 +1,4 @@
-"""Tracing / profiling hooks (SURVEY.md §5.1; the reference had only ``execution_time``).
+"""Tracing / profiling hooks (the reference had only ``execution_time``).
 
 * ``trace_range(name)`` — a roctx range (``roctxRangePushA/Pop`` from the ROCm roctx library)
   when ``DLI_TRACE=1``; rocprofv3 ``--marker-trace`` then shows engine steps, prefill/decode,

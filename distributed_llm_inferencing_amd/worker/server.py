@@ -1,5 +1,5 @@
 """Worker HTTP service: one process per MI355X (or a CPU worker), API-compatible with the
-reference's Flask worker (``worker/app.py``; SURVEY.md Appendix B):
+reference's Flask worker (``worker/app.py``):
 
     GET  /health         {"status":"healthy","resources":{cpu,memory,gpu,gpu_available,device},
                           "loaded_models","loaded_tokenizers","loaded_shards"}
@@ -10,7 +10,7 @@ reference's Flask worker (``worker/app.py``):
                          -> {"status":"success","result","execution_time"}; 408 on timeout
     POST /ssh_setup      {host, port=22, username, password | key_path}
 
-Differences that fix reference defects (SURVEY.md §2.2):
+Differences that fix reference defects:
 * ``gpu`` is the real HBM-in-use fraction of this worker's device (the reference reported
   memory_allocated / max_memory_allocated, W3);
 * ``shard_id = 0`` is accepted (W5 rejected it via ``all([...])``);
@@ -167,7 +167,7 @@ class WorkerState:
             return True
 
     def join_pipeline(self, name: str, shard_id: int, path: str, spec: dict) -> bool:
-        """``/load_shard`` with a "pipeline" spec (SURVEY.md §2.2 W5: the shard's layers go
+        """``/load_shard`` with a "pipeline" spec (the shard's layers go
         onto this GPU and the worker joins the pipeline communicator). Every node of the
         ring gets one such call: rank = shard id, ``world_size`` = the shard count of the
         export (``metadata.json``), rendezvous at ``init_method`` (``tcp://host:port``). The

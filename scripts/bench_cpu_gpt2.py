@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""BASELINE config 1: gpt2 on one CPU worker. Reference strategy (HF generate, batch 1,
+"""gpt2 on one CPU worker. Reference strategy (HF generate, batch 1,
 serial) vs this framework's CPU engine (continuous batching over the PyTorch reference ops).
 Random-init GPT-2 (124M) weights shared by both; 32-token prompts, max_length 100."""
 import json

@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""The reference's execution strategy measured on MI355X (SURVEY.md §6 / BASELINE.md):
+"""The reference's execution strategy measured on MI355X:
 HF transformers AutoModelForCausalLM.generate, batch 1, requests served one at a time
 (1 sync gunicorn worker, worker/Dockerfile:45), do_sample T=0.8 top_k=50 top_p=0.95,
 max_length=100 including a 32-token synthetic prompt, random-init weights, bf16 on GPU.

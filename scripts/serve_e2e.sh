@@ -1,5 +1,5 @@
 #!/bin/bash
-# End-to-end serving on one MI355X through the public API (BASELINE.json config 2: master
+# End-to-end serving on one MI355X through the public API (master
 # dispatch -> one Llama-3-8B worker): master (Flask, sqlite store, request queue,
 # dispatcher pool) + one GPU worker (continuous batching over HTTP requests) + the load
 # generator submitting form-encoded requests exactly as the reference UI does and polling

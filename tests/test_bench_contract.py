@@ -1,6 +1,6 @@
-"""bench.py driver contract on CPU: the driver launches ``python bench.py`` for N = 1 and
-``python -m torch.distributed.run --nproc-per-node N ... bench.py --gpus N`` for N > 1 and
-parses ONE JSON line from rank 0. These runs use a tiny Llama / Mixtral so the same code
+"""bench.py's contract on CPU: started as ``python bench.py`` for N = 1 and
+``python -m torch.distributed.run --nproc-per-node N ... bench.py --gpus N`` for N > 1,
+it prints ONE JSON line on rank 0. These runs use a tiny Llama / Mixtral so the same code
 paths (single engine, layer-sharded pipeline, DP replicas, expert parallel) finish in
 seconds over gloo."""
 from __future__ import annotations
@@ -74,7 +74,7 @@ def test_bench_torchrun_two_ranks(mode, model, par, gb):
 
 
 def test_bench_spawns_its_own_ranks():
-    """The driver's plain form ``python bench.py --gpus N`` (no torchrun): bench.py starts
+    """The plain form ``python bench.py --gpus N`` (no torchrun): bench.py starts
     the N ranks itself and rank 0's line names the data plane and every rank's device."""
     rec = _run([sys.executable, "bench.py", "--gpus", "2", "--model", "llama-tiny",
                 "--mode", "pp", *COMMON])

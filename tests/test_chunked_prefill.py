@@ -1,4 +1,4 @@
-"""Chunked prefill (SURVEY.md §5.7 long context): prompts longer
+"""Chunked prefill: prompts longer
 than ``max_prefill_tokens`` are prefilled over several steps, each chunk attending over the
 paged cache (earlier chunks + itself). Outputs must be token-identical to whole-prompt
 prefill, also when chunks interleave with decode steps of running sequences and after

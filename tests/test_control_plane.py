@@ -1,6 +1,6 @@
-"""T1/T2 control-plane tests: sqlite store, queues, master API contract (Appendix A),
-worker API contract (Appendix B), and master -> worker dispatch over real HTTP on localhost
-with the CPU engine (config 1: gpt2 on a CPU worker)."""
+"""Control-plane tests: sqlite store, queues, master API contract,
+worker API contract, and master -> worker dispatch over real HTTP on localhost
+with the CPU engine (gpt2 on a CPU worker)."""
 import threading
 from pathlib import Path
 import time
@@ -384,7 +384,7 @@ def test_loadgen_end_to_end(tmp_path, master):
 
 def test_worker_health_reports_failed_pipeline(worker):
     """A pipeline head whose ring broke (PipelineService.error set) answers /health with 503,
-    so the master's heartbeat takes the node out of rotation (SURVEY.md §5.3)."""
+    so the master's heartbeat takes the node out of rotation."""
     assert worker.get("/health").status_code == 200
 
     class _Broken:

@@ -217,7 +217,7 @@ def test_mixed_steps_token_identical_on_gpu(gpu, monkeypatch):
     tiles; a decode-only step of <= 4 rows the weight-streaming GEMVs), so a request may
     differ only where the exact model is undecided: at its first differing token the fp32
     reference's top-two logits are a near tie; and at most one request of the eight differs.
-    (token identity held only on plans earlier tests had autotuned.)"""
+    (Token identity would hold only on plans that earlier tests had autotuned.)"""
     from distributed_llm_inferencing_amd.ops import gemm as G
     monkeypatch.setenv("DLI_GEMM_AUTOTUNE", "0")
     assert G.DEFER_NORM

@@ -1,4 +1,4 @@
-"""The expert-parallel lockstep control plane (VERDICT r5 item 6): the shared-memory board
+"""The expert-parallel lockstep control plane: the shared-memory board
 (``csrc/runtime/lockstep.cpp``) replaces the per-step gloo all_gather, and idle ranks sleep on
 its doorbell instead of exchanging every 2 ms. CPU, spawned processes."""
 from __future__ import annotations
@@ -186,7 +186,7 @@ def _dying_worker(rank, world, port, q):
 def test_expert_rank_death_mid_forward_fails_fast():
     """A rank that dies inside a forward (rank 0 waiting in its mailboxes for the dead rank's
     rows) is seen by the board watchdog: the mailboxes are aborted and the survivor's next
-    step raises within seconds, not after the 120 s wait budget (ADVICE r5)."""
+    step raises within seconds, not after the 120 s wait budget."""
     ctx = mp.get_context("spawn")
     q = ctx.Queue()
     port = _free_port()

@@ -1,5 +1,5 @@
-"""Expert parallelism served through the worker / master API (
-"experts mapped to worker shards"): ``cli serve-expert`` starts N EP ranks, each an HTTP
+"""Expert parallelism served through the worker / master API (experts mapped
+to worker shards): ``cli serve-expert`` starts N EP ranks, each an HTTP
 worker registered with the master as a node reporting its expert shard; requests submitted
 to ``/api/inference/submit/`` are balanced across the ranks, whose MoE layers exchange rows
 every step. Results must be token-identical to one dense engine holding every expert.

@@ -268,7 +268,7 @@ def test_expert_parallel_caps_prefill_while_peers_decode():
 def _ep_overflow_worker(rank, world, port, q):
     """Rank 0 'replays' a decode graph of bucket 8 holding 5 live rows (every row of the
     bucket is routed), rank 1 is idle (an eager forward of zero rows): rank 1 must reserve a
-    region for rank 0's whole bucket, not for its 5 announced tokens (ADVICE r3, high)."""
+    region for rank 0's whole bucket, not for its 5 announced tokens."""
     _env(rank, world, port, DLI_EP_COMM="ipc")
     import torch.distributed as dist
     from distributed_llm_inferencing_amd.parallel.expert import ExpertParallelEngine

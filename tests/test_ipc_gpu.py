@@ -1,6 +1,6 @@
-"""The device mailbox data plane (csrc/runtime/ipc.cpp) hardened for the first 8-GPU run:
+"""The device mailbox data plane (csrc/runtime/ipc.cpp) hardened:
 uncached mailboxes, per-message sequence checks, sticky failure, and a ring that notices a
-dead stage in well under the wait budget (SURVEY.md §5.3, §5.8; the reference has no data
+dead stage in well under the wait budget (the reference has no data
 plane at all: master/dashboard/views.py:318-355, worker/app.py:332-372).
 
 All ranks share cuda:0 (gloo for the control group: RCCL refuses two ranks on one GPU)."""

@@ -1,5 +1,5 @@
 """T3 kernel golden tests: every HIP kernel vs the PyTorch fp32 reference of the same op
-(ops/reference.py), on the GPU. Run on an MI355X via gpurun."""
+(ops/reference.py), on an MI355X."""
 import math
 import os
 
@@ -1155,7 +1155,7 @@ def test_ep_pack_and_combine(gpu):
 @pytest.mark.parametrize("lens,hq,hkv", [([2048, 300], 32, 8), ([8192], 8, 2),
                                           ([1000, 400, 5, 700], 32, 8)])
 def test_prefill_attention_long(gpu, lens, hq, hkv):
-    """Long prompts (SURVEY.md §5.7): 2k and 8k-token causal GQA prefill vs the fp32
+    """Long prompts: 2k and 8k-token causal GQA prefill vs the fp32
     reference (the 8k case with fewer heads so the fp32 reference's score matrix fits)."""
     torch.manual_seed(21)
     hd = 128

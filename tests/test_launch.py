@@ -1,5 +1,5 @@
 """Launchers: serve-node's worker command lines and the data-plane fields a multi-rank
-worker reports (VERDICT r4: per-GPU isolation must not defeat the peer data plane)."""
+worker reports (per-GPU isolation must not defeat the peer data plane)."""
 from __future__ import annotations
 
 import os
@@ -23,7 +23,7 @@ def test_serve_node_keeps_every_gpu_visible(monkeypatch):
 
 
 def test_serve_node_passes_the_operator_mask_through(monkeypatch):
-    """ADVICE r5 (cli.py:46): a preset mask is kept, --gpu i indexes into it, and every GPU
+    """A preset mask is kept, --gpu i indexes into it, and every GPU
     of the mask stays visible to every worker."""
     monkeypatch.setenv("HIP_VISIBLE_DEVICES", "4,5,6,7")
     for i, (cmd, env) in enumerate(cli.node_commands(4)):
@@ -32,7 +32,7 @@ def test_serve_node_passes_the_operator_mask_through(monkeypatch):
 
 
 def test_visible_gpus_never_initialises_hip(monkeypatch, tmp_path):
-    """ADVICE r5 (launch.py:134): the parent counts GPUs from the KFD topology under the
+    """The parent counts GPUs from the KFD topology under the
     visibility masks; torch's device count (hipGetDeviceCount when amdsmi is missing) is
     never called, and launch.start refuses a parent that already initialised HIP."""
     import torch

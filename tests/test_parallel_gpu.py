@@ -231,11 +231,11 @@ def _pp8_worker(rank, world, port, q):
 
 @pytest.mark.timeout(420)
 def test_pipeline_pp8_real_shape_stages_match_single_engine(gpu):
-    """The driver's 8-rank pipeline form at the real Llama-3-8B layer shapes (d 4096, 32 q /
+    """An 8-rank pipeline at the real Llama-3-8B layer shapes (d 4096, 32 q /
     8 kv heads, FFN 14336, vocab 128256), 2 layers per stage, all 8 ranks on cuda:0: default
     data plane (IPC mailboxes), vocab-parallel head, M = 11 microbatches, decode graphs with
     the captured receive / send — greedy tokens identical to one engine holding all 16
-    layers (VERDICT r5 item 2)."""
+    layers."""
     (res,) = _run(_pp8_worker, 8)
     _register_16l()
     os.environ["DLI_GEMM_AUTOTUNE"] = "0"

@@ -1,5 +1,5 @@
 """Pipeline parallelism: loopback (single process) and real multi-process rings over gloo
-must produce exactly the single-stage engine's tokens (SURVEY.md §4 T5)."""
+must produce exactly the single-stage engine's tokens."""
 import os
 import socket
 
@@ -256,7 +256,7 @@ def _dying_worker(rank, world, port, q):
 
 
 def test_pipeline_stage_death_fails_fast_and_marks_unhealthy():
-    """SURVEY.md §5.3 failure detection: a stage process that dies mid-session (injected
+    """Failure detection: a stage process that dies mid-session (injected
     hard exit) turns into an error on the head within the data-plane timeout — not a hang —
     the pending request fails, later requests fail immediately, and the service reports the
     failure (the worker's /health then answers 503)."""

@@ -1,4 +1,4 @@
-"""Automatic prefix caching (VERDICT r1 'What's missing' 7 'no prefix reuse'):
+"""Automatic prefix caching:
 full KV blocks are published under chain hashes of their tokens; a later request with the
 same prefix maps those blocks (refcounted) and prefills only its remaining tokens as a chunk
 over the paged cache. Outputs must be token-identical to an engine without the cache, also

@@ -4,7 +4,7 @@
   end stuck on a dead peer): it marks the handle dead and aborts it anyway, within its bound;
 * ``async_error()`` reports ``BUSY`` (not "healthy") while an exchange holds the handle;
 * the pipeline watchdog turns a handle that stays busy past ``DLI_PP_TIMEOUT_S`` into a dead
-  peer and aborts the data plane (ADVICE r5: runtime/__init__.py:533).
+  peer and aborts the data plane (runtime/__init__.py:533).
 """
 import threading
 import time

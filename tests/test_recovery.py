@@ -1,4 +1,4 @@
-"""Ring failure recovery and request re-dispatch (SURVEY.md §5.3).
+"""Ring failure recovery and request re-dispatch.
 
 The reference marks a failing node inactive and keeps dispatching to the next active node
 (master/dashboard/views.py:99-105,389-391); nothing in it could recover a sharded model. Here,

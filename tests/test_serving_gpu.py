@@ -1,5 +1,5 @@
-"""Multi-process serving on the GPU, every rank on cuda:0 (``DLI_SAME_DEVICE=1``: the box
-has one MI355X): the deployments the driver's 8-GPU node would run, with the data plane
+"""Multi-process serving on the GPU, every rank on cuda:0 (``DLI_SAME_DEVICE=1``, for a host
+with one MI355X): the deployments that an 8-GPU node runs, with the data plane
 each one resolves reported by the workers themselves.
 
 * ``serve-worker`` x 2 + ``join-pipeline``: a 2-stage ring formed over the worker API

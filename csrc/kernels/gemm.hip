@@ -23,26 +23,22 @@
 //
 // Files: gemm_common.h (shared epilogue / split-K pieces), gemm_tiles.hip (ids 0-21, 23-25),
 // gemm_stream.hip (60-72: few rows, weights streamed), gemm8p.hip (22, 26-28), gemm4w.h +
-// gemm4w.hip (34, 41, 45), gemm4wp.hip (55: persistent 45), gemv.hip (29-33 and the fused batch-1
-// combine). The losing 4-wave variants are documented, not built
-// (profiles/r4/gemm4w/).
+// gemm4w.hip (34, 41, 45), gemm4wp.hip (55), gemv.hip (29-33 and the fused batch-1 combine).
 #include "gemm_common.h"
 
 extern "C" int dli_gemm_set_slab_store(int mode) {
   const int old = gemm_tiles_set_slab_store(mode);
   gemm_stream_set_slab_store(mode);
   gemm_8p_set_slab_store(mode);
-  gemm_4w_set_slab_store(mode);
   return old;
 }
 
 // one family's split-K slab store (0 plain, 1 nt, 2 sc1, 3 sc0 sc1): family 0 = the generic
-// tiles (decode O / QKV), 1 = the 8-phase kernels (decode down), 2 = the 4-wave kernels
+// tiles (decode O / QKV), 1 = the 8-phase kernels (decode down)
 extern "C" int dli_gemm_set_slab_store_family(int family, int mode) {
   switch (family) {
     case 0: gemm_stream_set_slab_store(mode); return gemm_tiles_set_slab_store(mode);
     case 1: return gemm_8p_set_slab_store(mode);
-    case 2: return gemm_4w_set_slab_store(mode);
     default: return -1;
   }
 }
@@ -53,8 +49,8 @@ extern "C" int dli_gemm_set_slab_store_family(int family, int mode) {
 // 256x256, 256x128, 128x256 (2 stages) and 256x128, 128x256 (3 stages); 18/19 = 128x96 and
 // 20/21 = 128x64 with 2/3 stages; 22 = 256x256 8-phase ping-pong; 23/24 = 128x192 (3/2
 // stages), 25 = 256x192, 8 waves; 26 = 256x224 ping-pong; 29-33 = the M <= 4 weight
-// stream (16 / 32 rows per workgroup, dispatch_gemv); 55 = tile 45 persistent (one workgroup
-// per CU walks its tiles, no split-K / grouped mode); 60-72 = weight-streaming tiles
+// stream (16 / 32 rows per workgroup, dispatch_gemv); 34, 41, 45 = 256x256, 4 waves; 55 = the
+// same on tiles of 256, 192 or 160 columns (no split-K / grouped mode); 60-72 = weight-streaming tiles
 // (gemm_stream.h). ws: fp32 [splits, M, N] when splits>1.
 // group_off (nullable): int[groups+1] row offsets; M is then the max rows of any group.
 // Grouped SiLU*up GEMM whose permuted row p reads activation row arow[p] (the MoE gate/up

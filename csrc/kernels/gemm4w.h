@@ -1,582 +1,540 @@
-// The 4-wave 256x256 MFMA GEMM (gemm4w_kernel: one wave per SIMD, 128x128 wave tiles,
-// accumulators pinned in the AGPR file) and its launcher, shared by the production tiles
-// (gemm4w.hip: 34, 41, 45).
+// 256-row GEMM tiles with ONE wave per SIMD: four waves of 128 x 16 NJ, their 8 NJ 16x16 blocks
+// accumulated in the AGPR file, on a grid of at most one workgroup a CU that walks its tiles
+// (tiles 34, 41, 45: gemm4w.hip; 55: gemm4wp.hip).
+//
+// What bounds it. Bare 16x16x32 MFMAs on random data run at 2.0 GHz (2.07 PFLOP/s), which the power
+// budget sets; with this tile's 32 fragment reads and 16 LDS-DMA pieces a K-tile at 1.75 GHz and 17.6
+// cycles an MFMA (1.68, operands in the L2). So what costs is (a) cycles in which the matrix pipe waits
+// and (b) energy beside the MFMAs; a cycle saved gives about 0.6 of itself, the clock gives the rest back.
+// 32x32x16 MFMAs, half the instructions, hold 1.73 GHz and 1.81 PFLOP/s alone: not used. Consecutive MFMAs share
+// the activation fragment (a new pair of fragments each time costs 4 % of the clock).
+//
+// (a) is this schedule's business; measured amid MFMAs of 16 cycles, one wave a SIMD: an LDS-DMA piece
+// costs 2 to 4 cycles, every scalar instruction beside it 4, vector ones nothing. So a lane's offsets advance by
+// vector adds, four pieces share M0 through their immediate offsets (which move the address in memory and in LDS
+// alike: the soffset takes them back), and the pieces are spread as thinly as the ring of two buffers allows (K =
+// 14336: 1.43 PFLOP/s with a piece every 4 MFMAs, 1.54 with one every 6 or 7).
+// The tile's epilogue was 20 k of 170 k cycles at K = 4096 (bounds by branches, 8-byte stores, a division a
+// SiLU, and a wait for all of its stores): now stores of 16 bytes a lane through range-checked descriptors that
+// nothing waits for until the tile's second K-tile. Both against a schedule of reads and pieces in bursts and
+// the former epilogue, us: 16384 x 6144 x 4096 557 -> 535 (1.54 PFLOP/s), 8192 x 4096 x 4096 182 -> 176 and x 14336
+// 645 -> 626, 8192 x 28672 x 4096 with SiLU pairs 1271 -> 1230. With fp32 outputs 188 -> 186: all CUs store 67 MB at
+// once, at 6.4 TB/s, behind which the next tile's pieces wait.
 #pragma once
 #include "gemm_common.h"
 
-template <int CPOL = 0>
-__device__ __forceinline__ void buf_lds16(const void* base, int nbytes, char* lds, int voff,
-                                          int soff) {
-  const __amdgpu_buffer_rsrc_t r =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, nbytes, 0x00020000);
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)lds, 16, voff, soff, 0, CPOL);
+typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
+typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
+typedef const __attribute__((address_space(3))) bf16x8 lds_frag;
+
+template <int V> using int_c = std::integral_constant<int, V>;
+// f(0), f(1), .. f(N - 1) with compile-time arguments
+template <class F, int... U>
+__device__ __forceinline__ void unroll_seq(F f, std::integer_sequence<int, U...>) {
+  (f(int_c<U>{}), ...);
+}
+template <int N, class F> __device__ __forceinline__ void unroll(F f) {
+  unroll_seq(f, std::make_integer_sequence<int, N>{});
 }
 
-// 16-B buffer load of `base` into registers (same range-checked descriptor as buf_lds16)
-__device__ __forceinline__ uint4 buf_ld16(const void* base, int nbytes, int voff, int soff) {
-  const __amdgpu_buffer_rsrc_t r =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, nbytes, 0x00020000);
-  const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
-  return uint4{v[0], v[1], v[2], v[3]};
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* p, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
+}
+// 1 KiB of LDS-DMA (16 B a lane); IMM moves both the address in memory and the one in LDS
+template <int IMM>
+__device__ __forceinline__ void dma16(const void* base, int bytes, uint32_t lds, int voff, int soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(make_rsrc(base, bytes), (lds_void*)lds, 16, voff, soff, IMM, 0);
 }
 
-// ---------------------------------------------------------------------------------------
-// 256x256 GEMM with ONE wave per SIMD and 128x128 wave tiles ("4-wave"): the structure of
-// the library kernels the prefill projections used to fall back to (hipBLASLt's
-// MT256x256x64 solution for these shapes is 4 waves, MIWaveTile 16x4, 1 workgroup per CU).
-// Against the 8-wave ping-pong (gemm8p_kernel: 128x64 per wave, two waves per SIMD) a
-// 128x128 wave tile reads 1/3 fewer LDS bytes per MFMA (32 ds_read_b128 per 128 MFMAs per
-// K-tile instead of 24 per 64) and issues half the barrier traffic; on MI355X under DVFS the
-// energy per MFMA, not the cycle count, sets the clock the chip holds on random data
-// (cdna_hip_programming.md §5.4 rule 28), and LDS read bytes are one of the terms.
-//
-// Waves (wm, wn) = (wid >> 1, wid & 1) own rows 128 wm .. +127 and columns 128 wn .. +127:
-// acc[8][8] 16x16 blocks = 256 accumulator registers. LDS: 2 buffers x (A 256x64 + W 256x64)
-// bf16 = 128 KiB, the chunk XOR swizzle of gemm_bf16_kernel, staged by LDS-DMA (each wave
-// moves 64 rows of A and 64 rows of W per K-tile: 16 x 1 KiB). K-tile T = two 32-deep halves:
-//   half 0: ds_read the kk=1 fragments of T (F1) | 64 MFMAs on F0 (kk=0 of T)
-//   lgkmcnt(0) + vmcnt(0) (T+1 landed) + s_barrier     <- the only barrier of the K-tile
-//   half 1: LDS-DMA T+2 into T's buffer; ds_read F0 = kk=0 of T+1 | 64 MFMAs on F1
-// so the fragments a half multiplies were read during the previous half, and the barrier
-// never leaves the matrix pipe without queued work beyond its own skew.
-// VAR bits: 1 = stagger-U (workgroup t starts its K loop at K-tile t % 8 and wraps: the
-// concurrent workgroups of a wave of the grid spread over memory channels), 8 / 16 = grouped
-// tile order (GM 4 / 8 tile-rows per group, as gemm8p), 2 = all 16 next-half reads up front,
-// 4 = all 16 LDS-DMA pieces of a K-tile up front (default: one per 4 MFMAs), 32 = deep W
-// ring (3 W stages), 1024 = register staging, 2048 = sc1 loads, 4096 = the two-barrier K-tile
-// (ktile2 below; tile 45, the default 4-wave tile), 8192 / 16384 = its other barrier
-// placements, 32768 = column-major MFMA order, 65536 = per-piece voffset addressing.
-// Diagnostics only: 64 = no LDS-DMA in the K loop, 128 = also no barrier / waits (wrong
-// results, timing of the remaining work), 131072 = s_memtime stamps (correct results).
-// Only tiles 34 (VAR 8), 41 (8 | 32) and 45 (8 | 4096) are instantiated; the other VAR bits
-// are variants that lost, kept for diagnostics (measurements: profiles/r4/gemm4w/).
-template <int EPI, int VAR = 0>
+// The schedule of a K-tile: 16 NJ MFMAs, the first half on the fragments F0 (its first 32 values of K, read
+// before it began), the second on F1. After MFMA q:
+//   0 .. NF - 1         a fragment of F1 each
+//   B1                  every wave has read the buffer: a barrier frees it
+//   D, D + DS, ..       a DMA piece of the K-tile after the next into it, NP of them
+//   B2                  the next K-tile landed (the pieces just issued may fly) for every wave
+//   B2 + 1, + 3, ..     a fragment of the next K-tile's F0 each
+// Positions by measurement (8192 x 4096 x 4096, 16384 x 4096 x 14336, us): reads one or two MFMAs apart 185.9 / 187.3
+// and 1298 / 1296; pieces 5 instead of 6 apart 185.4 and 1313.
+template <int NJ> struct Sched4w {
+  static constexpr int Q = 16 * NJ, NF = 8 + NJ, NP = 8 + NJ;
+  static constexpr int B1 = NF + 3 + NJ / 3, D = B1 + 1, DS = (Q - 4 - D) / (NP - 1), DL = D + DS * (NP - 1);
+  static constexpr int B2 = Q - 1 - 2 * NF;
+  static constexpr int ahead = B2 < D ? 0 : (B2 - D) / DS + 1;      // pieces issued when B2 waits
+  static_assert(DS >= 1 && DL + 2 < Q && B2 > B1 && ahead <= NP, "the pieces fit the K-tile");
+};
+
+// EPI_F32's bias (unsplit): where the block maxima go (BlockMax). ws: the partial sums' slabs of a product
+// split over K (fp32, or fp16 with EPI_SLAB16). group_off: rows of group g are [off[g], off[g + 1]).
+template <int EPI, int NJ>
 __global__ void __launch_bounds__(256, 1) gemm4w_kernel(
     const u16* __restrict__ A, int lda, const u16* __restrict__ W, int ldw,
-    void* __restrict__ C, int ldc, int M, int N, int K, int k_split_len,
-    const u16* __restrict__ bias, float* __restrict__ ws, const int* __restrict__ group_off) {
-  constexpr int BM = 256, BN = 256;
-  constexpr int A_BYTES = BM * BK * 2, BUF = 2 * A_BYTES;
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-
-  int row0 = 0, Mg = M;
-  const u16* Wg = W;
-  if (group_off != nullptr) {
-    row0 = group_off[blockIdx.z];
-    Mg = group_off[blockIdx.z + 1] - row0;
-    Wg = W + (long)blockIdx.z * N * ldw;
-  }
-  const int tiles_m = (M + BM - 1) / BM;
-  const int tiles_n = (N + BN - 1) / BN;
-  int tile, ks;
-  split_tile(tiles_m * tiles_n, group_off != nullptr, tile, ks);
-  int tn, tm;
-  constexpr int GM = (VAR & 8) ? 4 : (VAR & 16) ? 8 : 1;
-  if (GM > 1) {
-    const int per_group = GM * tiles_n;
-    const int first_m = (tile / per_group) * GM;
-    const int gsz = min(tiles_m - first_m, GM);
-    const int in_g = tile % per_group;
-    tm = first_m + in_g % gsz;
-    tn = in_g / gsz;
-  } else {
-    tn = tile / tiles_m;
-    tm = tile % tiles_m;
-  }
-  const int m0 = tm * BM, n0 = tn * BN;
-  if (m0 >= Mg) return;
-  const int kb = ks * k_split_len;
-  const int nk = min(k_split_len, K - kb) / BK;
-  const int kst = (VAR & 1) ? (tile & 7) % max(nk, 1) : 0;   // stagger-U start K-tile
-  const u16* Ab = A + (long)row0 * lda;
+    void* __restrict__ C, int ldc, int M, int N, int K, int splits, const u16* __restrict__ bias,
+    float* __restrict__ ws, const int* __restrict__ group_off, int groups) {
+  using S = Sched4w<NJ>;
+  constexpr int BM = 256, BN = 32 * NJ, GM = 4;
+  constexpr int A_BYTES = BM * BK * 2;
+  constexpr int NF = S::NF, NP = S::NP;
+  constexpr bool PAIRS = epi_pairs(EPI);
+  // two buffers 64 KiB apart: the bit that tells them apart. The kernel has no other LDS, so it starts at 0
+  constexpr uint32_t FLIP = 0x10000;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wid >> 1, wn = wid & 1;
+  const int tiles_n = (N + BN - 1) / BN;
+  const int ksl = K / splits, nk = ksl / BK;
 
-  // ---- staging by buffer LDS-DMA: piece i (0..7) of A / W = rows 64 wid + 8 i + lane / 8 of
-  // the tile, swizzled chunk (lane & 7) ^ ((row >> 1) & 7) = (lane & 7) ^ ((lane >> 4) + 4 i)
-  // & 7: only the parity of i changes the lane's offset, the rest is the scalar soffset
-  // i * 8 rows + K-tile. Rows past the matrix read as zeros (buffer range check) instead of
-  // needing a clamped address per row, so a lane keeps 4 offset VGPRs, not 16 pointers.
-  // (the descriptors are built inside buf_lds16: a lambda capturing an
-  // __amdgpu_buffer_rsrc_t made hipcc drop the kernel's host-side handle)
-  const u16* a_base = Ab + (long)m0 * lda;
-  const u16* w_base = Wg + (long)n0 * ldw;
-  const int a_bytes = min(Mg - m0, BM) * lda * 2, w_bytes = min(N - n0, BN) * ldw * 2;
-  const int prow = 64 * wid + (lane >> 3);
-  const int ce = (lane & 7) ^ ((lane >> 4) & 7), co = (lane & 7) ^ (((lane >> 4) + 4) & 7);
-  const int a_off[2] = {prow * lda * 2 + (kb + ce * 8) * 2, prow * lda * 2 + (kb + co * 8) * 2};
-  const int w_off[2] = {prow * ldw * 2 + (kb + ce * 8) * 2, prow * ldw * 2 + (kb + co * 8) * 2};
-  // LDS: 2 stages of {A 256x64, W 256x64} (128 KiB); with VAR 32 ("deep W") 2 A stages and
-  // 3 W stages (160 KiB, the whole LDS): the weight panel, which a decode-sized GEMM streams
-  // from HBM while A is L2-resident, is fetched one K-tile further ahead (a CU's stream rate
-  // is its bytes in flight over the loaded memory latency)
-  constexpr bool DEEP = (VAR & 32) != 0;
-  auto abase = [&](int kt) -> char* {
-    return DEEP ? smem + (kt & 1) * A_BYTES : smem + (kt & 1) * BUF;
-  };
-  auto wbase = [&](int kt, int ws) -> char* {      // ws = kt % 3 (DEEP)
-    return DEEP ? smem + 2 * A_BYTES + ws * A_BYTES : smem + (kt & 1) * BUF + A_BYTES;
-  };
-  auto kpos = [&](int kt) {                        // stagger-U: physical K-tile of logical kt
-    const int kp = kt + kst;
-    return kp >= nk ? kp - nk : kp;
-  };
-  // one 1-KiB piece f (0..15: A pieces 0-7 of K-tile ka, W pieces 8-15 of K-tile kw into W
-  // slot ws); a negative K-tile skips its pieces
-  constexpr int CPOL = (VAR & 2048) ? 16 : 0;
-  // VAR 65536 (VOFF, the library kernel's addressing): every piece keeps its whole byte
-  // offset in its own VGPR (16 per lane) and the K-tile advances the descriptor's base
-  // (SALU, once per K-tile and operand) instead of a per-piece soffset SGPR
-  constexpr bool VOFF = (VAR & 65536) != 0;
-  int va[8], vw[8];
+  // ---- tiles. Dense: virtual id -> XCD remap -> (split, grouped order of GM row tiles). Grouped: a group's
+  // row tiles follow those of the groups before it, 64 groups a step, a group a lane
+  int tiles_m = (M + BM - 1) / BM;
+  int ga = 0, gb = 0, gsum = 0;                    // this lane's group: its rows, row tiles up to and with it
+  auto load_groups = [&](int g0) {
+    const int g = g0 + lane;
+    ga = g < groups ? group_off[g] : 0;
+    gb = g < groups ? group_off[g + 1] : 0;
+    gsum = (gb - ga + BM - 1) / BM;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    va[i] = VOFF ? a_off[i & 1] + i * 16 * lda : 0;
-    vw[i] = VOFF ? w_off[i & 1] + i * 16 * ldw : 0;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int up = __shfl_up(gsum, o, 64);
+      if (lane >= o) gsum += up;
+    }
+    return __builtin_amdgcn_readlane(gsum, 63);
+  };
+  if (group_off != nullptr) {
+    tiles_m = 0;
+    for (int g0 = (groups - 1) & ~63; g0 >= 0; g0 -= 64) tiles_m += load_groups(g0);
   }
-  auto stage_piece = [&](int ka, int kw, int ws, int f) {
-    const int i = f & 7;
-    if (VOFF) {
-      if (f < 8) {
-        if (ka >= 0) {
-          const int kp = kpos(ka) * BK;
-          buf_lds16<CPOL>(a_base + kp, a_bytes - kp * 2, abase(ka) + (64 * wid + 8 * i) * 128,
-                          va[i], 0);
+  const int nwg = tiles_m * tiles_n;
+  const int total = nwg * splits;
+  struct Tile { int m0, n0, ks, row0, rows; const u16* w; };
+  auto locate = [&](int v) -> Tile {
+    Tile t;
+    const int lg = xcd_remap(v, total);
+    t.ks = lg / nwg;
+    int tile = lg - t.ks * nwg, tm = tiles_m;
+    t.row0 = 0;
+    t.rows = M;
+    t.w = W;
+    if (group_off != nullptr) {
+      int before = 0;                              // row tiles of the groups before this step's
+      for (int g0 = 0; g0 < groups; g0 += 64) {
+        // (the first 64 groups' stay in registers: a load here would wait for the stores in flight)
+        const int sum = groups > 64 ? load_groups(g0) : __builtin_amdgcn_readlane(gsum, 63);
+        const unsigned long long past = __ballot((before + gsum) * tiles_n > tile);
+        if (past != 0) {
+          const int l = __builtin_ctzll(past);
+          t.row0 = __builtin_amdgcn_readlane(ga, l);
+          t.rows = __builtin_amdgcn_readlane(gb, l) - t.row0;
+          tm = (t.rows + BM - 1) / BM;
+          tile -= (before + __builtin_amdgcn_readlane(gsum, l) - tm) * tiles_n;
+          t.w = W + (long)(g0 + l) * N * ldw;
+          break;
         }
-      } else if (kw >= 0) {
-        const int kp = kpos(kw) * BK;
-        buf_lds16<CPOL>(w_base + kp, w_bytes - kp * 2, wbase(kw, ws) + (64 * wid + 8 * i) * 128,
-                        vw[i], 0);
-      }
-      return;
-    }
-    if (f < 8) {
-      if (ka >= 0)
-        buf_lds16<CPOL>(a_base, a_bytes, abase(ka) + (64 * wid + 8 * i) * 128, a_off[i & 1],
-                        i * 16 * lda + kpos(ka) * (BK * 2));
-    } else if (kw >= 0) {
-      buf_lds16<CPOL>(w_base, w_bytes, wbase(kw, ws) + (64 * wid + 8 * i) * 128, w_off[i & 1],
-                      i * 16 * ldw + kpos(kw) * (BK * 2));
-    }
-  };
-  auto stage = [&](int ka, int kw, int ws) {
-#pragma unroll
-    for (int f = 0; f < 16; ++f) stage_piece(ka, kw, ws, f);
-  };
-  // VAR 1024 (register staging): piece f of K-tile k is loaded into stg[f] (buffer_load to
-  // VGPRs, 64 per lane for a K-tile) and later written to LDS with one ds_write_b128 — the
-  // load / write pair issues in a fraction of an LDS-DMA's cost among MFMAs with ONE wave
-  // per SIMD (no partner wave hides the DMA issue, as the 8-wave ping-pong does)
-  constexpr bool RS = (VAR & 1024) != 0;
-  uint4 stg[16];
-  auto rs_load = [&](int k, int f) {
-    const int i = f & 7;
-    if (f < 8) stg[f] = buf_ld16(a_base, a_bytes, a_off[i & 1], i * 16 * lda + kpos(k) * (BK * 2));
-    else stg[f] = buf_ld16(w_base, w_bytes, w_off[i & 1], i * 16 * ldw + kpos(k) * (BK * 2));
-  };
-  auto rs_write = [&](int k, int f) {
-    const int i = f & 7;
-    char* dst = (f < 8 ? abase(k) : wbase(k, 0)) + (64 * wid + 8 * i) * 128 + lane * 16;
-    *reinterpret_cast<uint4*>(dst) = stg[f];
-  };
-
-  const int fr = lane & 15, fq = lane >> 4;
-  auto read_frag = [&](const char* part, int row, int kk) -> bf16x8 {
-    const int c = kk * 4 + fq;
-    return *reinterpret_cast<const bf16x8*>(part + row * 128 + ((c ^ ((row >> 1) & 7)) << 4));
-  };
-  const int arow = wm * 128 + fr, wrow = wn * 128 + fr;
-
-  f32x4 acc[8][8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  auto barrier = [&]() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    asm volatile("" ::: "memory");
-  };
-  // one 32-deep half: 64 MFMAs on (acur, bcur) while the next half's 16 fragments are read
-  // from (na, nw) into (anext, bnext). The MFMAs are inline asm with the accumulator pinned to
-  // the AGPR file ("+a"): with 256 accumulators per lane the compiler's own MFMA selection
-  // bounced them between VGPRs and AGPRs (1,000+ v_accvgpr moves per K-tile). hipcc pads no
-  // hazard inside an asm statement (cdna_hip_programming.md §5.7): the fragments come from
-  // ds_reads, whose completion hipcc waits for by register (lgkmcnt) before each statement;
-  // an accumulator is read only as the next MFMA's C (no wait states) until the drain after
-  // the loop. ka / kw >= 0: this half also stages those K-tiles, one LDS-DMA piece after
-  // every 4th MFMA (16 pieces issued back to back held the matrix pipe for several hundred
-  // cycles: an LDS-DMA issue costs ~60 cycles among MFMAs, /opt/skills/guides/MI355X_MICROARCH.md constants).
-  auto half = [&](const bf16x8 (&acur)[8], const bf16x8 (&bcur)[8], bf16x8 (&anext)[8],
-                  bf16x8 (&bnext)[8], const char* na, const char* nw, int nkk, bool more,
-                  int ka, int kw, int ws, int rw = -1, int rl = -1)
-      __attribute__((always_inline)) {
-    if ((VAR & 2) && more) {                       // A/B: all 16 reads up front
-#pragma unroll
-      for (int i = 0; i < 8; ++i) anext[i] = read_frag(na, arow + 16 * i, nkk);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) bnext[j] = read_frag(nw, wrow + 16 * j, nkk);
-    }
-    const bool dma = !(VAR & 4) && (ka >= 0 || kw >= 0);
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
-                     : "+a"(acc[i][j]) : "v"(bcur[j]), "v"(acur[i]));
-        const int q = 8 * i + j;
-        if (dma && (q & 3) == 1) {
-          stage_piece(ka, kw, ws, q >> 2);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-        if (RS && rw >= 0 && (q & 3) == 1) {        // write piece of rw, reload it with rl
-          rs_write(rw, q >> 2);
-          if (rl >= 0) rs_load(rl, q >> 2);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-        // one next-half fragment read after every 4th MFMA, pinned in place (the scheduler
-        // hoisted all 16 above the first MFMA, whose lgkmcnt then waited on 2 of them), in
-        // the order the next half consumes them: A0, B0..B7, A1..A7
-        if (!(VAR & 2) && more && (q & 3) == 3) {
-          const int f = q >> 2;
-          if (f >= 1 && f <= 8) bnext[f - 1] = read_frag(nw, wrow + 16 * (f - 1), nkk);
-          else { const int ia = f == 0 ? 0 : f - 8; anext[ia] = read_frag(na, arow + 16 * ia, nkk); }
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      }
-  };
-
-  // ---- prologue. Plain: K-tiles 0 and 1 in flight. DEEP: A 0-1 and W 0-2 (issue order A0 W0
-  // A1 W1 W2). Then the kk=0 fragments of K-tile 0 in registers.
-  if (RS) {                                        // K-tiles 0, 1 into LDS, 2 in registers
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      if (k < nk) {
-#pragma unroll
-        for (int f = 0; f < 16; ++f) rs_load(k, f);
-#pragma unroll
-        for (int f = 0; f < 16; ++f) rs_write(k, f);
+        before += sum;
       }
     }
-    if (nk > 2) {
-#pragma unroll
-      for (int f = 0; f < 16; ++f) rs_load(2, f);
-    }
-    __builtin_amdgcn_s_waitcnt(0xC07F);            // lgkmcnt(0): the writes landed
-    barrier();
-  } else {
-    if (nk > 0) stage(0, 0, 0);
-    if (nk > 1) stage(1, 1, 1);
-    if (DEEP && nk > 2) stage(-1, 2, 2);
-    if (DEEP && nk > 2) wait_vmcnt<24>();
-    else if (nk > 1) wait_vmcnt<16>();
-    else wait_vmcnt<0>();
-    barrier();
-  }
-  bf16x8 a0[8], b0[8], a1[8], b1[8];
-  if (nk > 0 && (VAR & 32768)) {                   // column-major MFMA order (JM below)
-    b0[0] = read_frag(wbase(0, 0), wrow, 0);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) a0[i] = read_frag(abase(0), arow + 16 * i, 0);
-#pragma unroll
-    for (int j = 1; j < 8; ++j) b0[j] = read_frag(wbase(0, 0), wrow + 16 * j, 0);
-  } else if (nk > 0) {
-    a0[0] = read_frag(abase(0), arow, 0);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) b0[j] = read_frag(wbase(0, 0), wrow + 16 * j, 0);
-#pragma unroll
-    for (int i = 1; i < 8; ++i) a0[i] = read_frag(abase(0), arow + 16 * i, 0);
-  }
-
-  // one K-tile; SA / SW (compile-time, so no branch sits inside an MFMA sequence): restage
-  // A (K-tile kt + 2) / W (kt + 2, DEEP: kt + 3) during its second half
-  int wsl = 0;                                      // W slot of kt (DEEP: kt % 3)
-  auto ktile = [&](auto SA, auto SW, int kt) __attribute__((always_inline)) {
-    constexpr bool sa = decltype(SA)::value, sw = decltype(SW)::value;
-    const int ws1 = wsl == 2 ? 0 : wsl + 1;
-    const char* ab = abase(kt);
-    const char* wb = wbase(kt, wsl);
-    // half 0: MFMAs on kk=0 of kt, reading kk=1 of kt
-    half(a0, b0, a1, b1, ab, wb, 1, true, -1, -1, 0);
-    // every wave's reads of these buffers retired; K-tile kt+1 landed for every wave: the
-    // only younger DMAs may be DEEP's W of kt+2 (issued last in the previous K-tile)
-    if (!(VAR & 128)) {
-      __builtin_amdgcn_s_waitcnt(0xC07F);          // lgkmcnt(0), seen by hipcc's counters
-      if (RS) {
-      } else if (DEEP && kt + 2 < nk) {
-        wait_vmcnt<8>();
-      } else {
-        wait_vmcnt<0>();
-      }
-      barrier();
-    }
-    // half 1: MFMAs on kk=1 of kt, reading kk=0 of kt+1; restage kt's buffers (register
-    // staging: write K-tile kt+2 from the registers, reload them with kt+3)
-    const int ka = (sa && !(VAR & 64)) ? kt + 2 : -1;
-    const int kw = (sw && !(VAR & 64)) ? kt + (DEEP ? 3 : 2) : -1;
-    if (RS) {
-      half(a1, b1, a0, b0, abase(kt + 1), wbase(kt + 1, ws1), 0, true, -1, -1, 0,
-           sa ? kt + 2 : -1, sw ? kt + 3 : -1);
-    } else {
-      if ((VAR & 4) && (ka >= 0 || kw >= 0)) stage(ka, kw, wsl);
-      half(a1, b1, a0, b0, abase(kt + 1), wbase(kt + 1, ws1), 0, true,
-           (VAR & 4) ? -1 : ka, (VAR & 4) ? -1 : kw, wsl);
-    }
-    wsl = ws1;
-  };
-  // VAR 4096 ("two barriers", the buffer-release point moved forward): one K-tile = 128
-  // MFMAs, 64 on F0 (kk=0, read during the previous K-tile) then 64 on F1:
-  //   MFMAs 0-15: one F1(kt) fragment read after each        | frees buffer kt early
-  //   after MFMA 19: lgkmcnt(0) + s_barrier (B1: every wave has read buffer kt)
-  //   MFMAs 20-95: LDS-DMA of K-tile kt+2 into buffer kt, one piece per 5 MFMAs
-  //   after MFMA 103: vmcnt(16) (K-tile kt+1 landed; kt+2 may fly) + s_barrier (B2)
-  //   MFMAs 104-119: one F0(kt+1) fragment read after each
-  // The DMA of kt+2 starts ~45 MFMAs earlier than in the one-barrier schedule and is waited
-  // for ~1.5 K-tiles later (hides ~2,400 cycles of HBM latency instead of ~1,000-2,000),
-  // and 16 DMAs spread over 80 MFMAs instead of 64. Plain (2-stage) ring only.
-  constexpr bool TWO_B = (VAR & 4096) != 0;
-  // With DEEP (3 W stages) the DMA of this K-tile is A(kt+2) and W(kt+3), both into kt's
-  // slots; B2 may leave the previous tile's W pieces in flight too (vmcnt 24).
-  static_assert(!(TWO_B && RS), "two-barrier schedule: LDS-DMA staging only");
-  // SA / SW: this K-tile stages A(kt+2) / W(kt+2, DEEP: kt+3); PW: the previous K-tile
-  // staged W (DEEP: its pieces may still fly at B2)
-  // VAR 131072 (STAMP, diagnostic build only): s_memtime stamps around the two barriers and
-  // the DMA window, summed over the K loop per segment and written by each workgroup's
-  // first lane to the workspace (read the SHARES: every stamp drains the LDS reads)
-  constexpr bool STAMP = (VAR & 131072) != 0;
-  unsigned long long sseg[6] = {0, 0, 0, 0, 0, 0};
-  unsigned long long st_prev = 0;
-  auto stamp = [&]() __attribute__((always_inline)) -> unsigned long long {
-    unsigned long long t;
-    __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_memtime %0\n\ts_waitcnt lgkmcnt(0)" : "=s"(t) :: "memory");
-    __builtin_amdgcn_sched_barrier(0);
+    const int per_group = GM * tiles_n;
+    const int first_m = (tile / per_group) * GM;
+    const int gsz = min(tm - first_m, GM);
+    const int in_g = tile % per_group;
+    t.m0 = (first_m + in_g % gsz) * BM;
+    t.n0 = (in_g / gsz) * BN;
     return t;
   };
-  auto mark = [&](int seg) __attribute__((always_inline)) {
-    if constexpr (STAMP) {
-      const unsigned long long t = stamp();
-      sseg[seg] += t - st_prev;
-      st_prev = t;
+
+  // ---- staging. LDS rows of 128 B whose 16-B chunk c of row r lies at c ^ ((r >> 1) & 7). A wave moves 64 rows
+  // of A and 8 NJ of W a K-tile, piece i the rows 8 i + lane / 8 of them: only i's parity changes the chunk
+  // that a lane fetches, the rest is the soffset's. Rows past the matrix read as zeros
+  const int prow = 64 * wid + (lane >> 3), wprow = 8 * NJ * wid + (lane >> 3);
+  const int ce = (lane & 7) ^ ((lane >> 4) & 7), co = (lane & 7) ^ (((lane >> 4) + 4) & 7);
+  // (a wave's W rows start at an odd multiple of 8 where NJ and the wave are odd)
+  const bool flip = (NJ * wid) & 1;
+  const int va0 = prow * lda * 2 + ce * 16, va1 = prow * lda * 2 + co * 16;
+  const int vw0 = wprow * ldw * 2 + (flip ? co : ce) * 16, vw1 = wprow * ldw * 2 + (flip ? ce : co) * 16;
+  int xa0, xa1, xw0, xw1;                          // those of the next K-tile to stage
+  int sofa[8], sofw[NJ];                           // a piece's soffset, less its immediate offset
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    sofa[i] = i * 16 * lda - (i & 3) * 1024;
+    asm volatile("" : "+s"(sofa[i]));
+  }
+#pragma unroll
+  for (int i = 0; i < NJ; ++i) {
+    sofw[i] = i * 16 * ldw - (i & 3) * 1024;
+    asm volatile("" : "+s"(sofw[i]));
+  }
+  const u16 *sa, *sw;                              // the staged tile's panels, and their bytes in range
+  int sab, swb;
+  auto begin_stage = [&](const Tile& t, bool any) {
+    sa = A + (long)(t.row0 + t.m0) * lda + t.ks * ksl;
+    sw = t.w + (long)t.n0 * ldw + t.ks * ksl;
+    sab = any && nk > 0 ? (min(t.rows - t.m0, BM) * lda - t.ks * ksl) * 2 : 0;
+    swb = any && nk > 0 ? (min(N - t.n0, BN) * ldw - t.ks * ksl) * 2 : 0;
+    xa0 = va0; xa1 = va1; xw0 = vw0; xw1 = vw1;
+  };
+  uint32_t da = 64 * wid * 128, dw = A_BYTES + 8 * NJ * wid * 128;
+  auto piece = [&](auto F) __attribute__((always_inline)) {
+    constexpr int f = decltype(F)::value;
+    if constexpr (f < 8)
+      dma16<(f & 3) * 1024>(sa, sab, da + (f >> 2) * 4096, f & 1 ? xa1 : xa0, sofa[f]);
+    else
+      dma16<((f - 8) & 3) * 1024>(sw, swb, dw + ((f - 8) >> 2) * 4096, f & 1 ? xw1 : xw0, sofw[f - 8]);
+  };
+  auto next_buffer = [&]() { da ^= FLIP; dw ^= FLIP; };
+  auto next_k = [&]() { xa0 += 2 * BK; xa1 += 2 * BK; xw0 += 2 * BK; xw1 += 2 * BK; };
+
+  // ---- fragments: rows 16 apart swizzle alike, so one address a half K-tile and operand
+  const int fr = lane & 15, fq = lane >> 4;
+  const int arow = wm * 128 + fr, wrow = wn * 16 * NJ + fr;
+  uint32_t ra0 = arow * 128 + ((fq ^ ((arow >> 1) & 7)) << 4);
+  uint32_t ra1 = arow * 128 + (((4 + fq) ^ ((arow >> 1) & 7)) << 4);
+  uint32_t rw0 = A_BYTES + wrow * 128 + ((fq ^ ((wrow >> 1) & 7)) << 4);
+  uint32_t rw1 = A_BYTES + wrow * 128 + (((4 + fq) ^ ((wrow >> 1) & 7)) << 4);
+  f32x4 acc[8][NJ];
+  bf16x8 a0[8], b0[NJ], a1[8], b1[NJ];
+  // in the order of their use: A's first, all of W's, A's others
+  auto read = [&](auto F, bf16x8 (&av)[8], bf16x8 (&bv)[NJ], uint32_t pa, uint32_t pw)
+      __attribute__((always_inline)) {
+    constexpr int f = decltype(F)::value;
+    if constexpr (f >= 1 && f <= NJ) {
+      bv[f - 1] = *(lds_frag*)(pw + (f - 1) * 2048);
+    } else {
+      constexpr int i = f == 0 ? 0 : f - NJ;
+      av[i] = *(lds_frag*)(pa + i * 2048);
     }
   };
-  auto ktile2 = [&](auto SA, auto SW, auto PW, bool more, int kt)
-      __attribute__((always_inline)) {
-    if constexpr (STAMP) st_prev = stamp();
-    constexpr bool sa = decltype(SA)::value, sw = decltype(SW)::value;
-    constexpr bool pw = DEEP && decltype(PW)::value;
-    constexpr bool sd = sa || sw;
-    const int ws1 = wsl == 2 ? 0 : wsl + 1;
-    const char* ab = abase(kt);
-    const char* wb = wbase(kt, wsl);
-    const char* nab = abase(kt + 1);
-    const char* nwb = wbase(kt + 1, ws1);
-    // B1 / B2 positions: default 19 / 103; VAR 8192: 25 / 111; VAR 16384: 25 / after the
-    // last MFMA with the 16 F0(kt+1) reads in one burst (the library kernel's placement)
-    constexpr int QB1 = (VAR & (8192 | 16384)) ? 25 : 19;
-    constexpr int QB2 = (VAR & 8192) ? 111 : (VAR & 16384) ? 127 : 103;
-    // VAR 32768 (JM): MFMAs column-major within a half (acc[i][j] with j outer), so the
-    // weight fragment — MFMA operand A — stays the same for 8 consecutive MFMAs (the
-    // library kernel's order); fragment f of a half is then read in the order B0, A0..A7,
-    // B1..B7 instead of A0, B0..B7, A1..A7
-    constexpr bool JM = (VAR & 32768) != 0;
-    auto read_fx = [&](int f, bf16x8 (&av)[8], bf16x8 (&bv)[8], const char* pa, const char* pw,
-                       int kk) __attribute__((always_inline)) {
-      if (JM) {
-        if (f >= 1 && f <= 8) av[f - 1] = read_frag(pa, arow + 16 * (f - 1), kk);
-        else { const int jb = f == 0 ? 0 : f - 8; bv[jb] = read_frag(pw, wrow + 16 * jb, kk); }
-      } else {
-        if (f >= 1 && f <= 8) bv[f - 1] = read_frag(pw, wrow + 16 * (f - 1), kk);
-        else { const int ia = f == 0 ? 0 : f - 8; av[ia] = read_frag(pa, arow + 16 * ia, kk); }
-      }
-    };
-    auto read_f0 = [&](int f) __attribute__((always_inline)) { read_fx(f, a0, b0, nab, nwb, 0); };
-    auto step = [&](int q) __attribute__((always_inline)) {
-      if (q < 16) {                                // F1(kt)
-        read_fx(q, a1, b1, ab, wb, 1);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      if (q == QB1 && !(VAR & 128)) {
-        mark(0);                                   // MFMAs 0..QB1 + the F1 reads
-        __builtin_amdgcn_s_waitcnt(0xC07F);        // lgkmcnt(0)
-        barrier();
-        mark(1);                                   // B1
-      }
-      if (q == QB1 + 80) mark(2);                  // the DMA window
-      if (sd && !(VAR & 64) && q > QB1 && q <= QB1 + 80 && (q - QB1 - 1) % 5 == 0) {
-        stage_piece(sa ? kt + 2 : -1, sw ? kt + (DEEP ? 3 : 2) : -1, wsl, (q - QB1 - 1) / 5);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      if (q == QB2 && more && !(VAR & 128)) {
-        mark(3);                                   // MFMAs after the DMA window
-        constexpr int fly = (VAR & 64) ? 0 : 8 * ((sa ? 1 : 0) + (sw ? 1 : 0) + (pw ? 1 : 0));
-        wait_vmcnt<fly>();
-        barrier();
-        mark(4);                                   // B2
-      }
-      if (q == 127) mark(5);                       // MFMAs after B2 + the F0 reads
-      if (more) {                                  // F0(kt+1)
-        if (QB2 == 127) {
-          if (q == 127) {
-#pragma unroll
-            for (int f = 0; f < 16; ++f) read_f0(f);
-            __builtin_amdgcn_sched_barrier(0);
-          }
-        } else if (q > QB2 && q <= QB2 + 16) {
-          read_f0(q - QB2 - 1);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      }
-    };
-#pragma unroll
-    for (int u = 0; u < 8; ++u)
-#pragma unroll
-      for (int v = 0; v < 8; ++v) {
-        const int i = JM ? v : u, j = JM ? u : v;
-        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
-                     : "+a"(acc[i][j]) : "v"(b0[j]), "v"(a0[i]));
-        step(8 * u + v);
-      }
-#pragma unroll
-    for (int u = 0; u < 8; ++u)
-#pragma unroll
-      for (int v = 0; v < 8; ++v) {
-        const int i = JM ? v : u, j = JM ? u : v;
-        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
-                     : "+a"(acc[i][j]) : "v"(b1[j]), "v"(a1[i]));
-        step(64 + 8 * u + v);
-      }
+  auto fence = [&]() __attribute__((always_inline)) { __builtin_amdgcn_sched_barrier(0); };
+  auto barrier = [&]() __attribute__((always_inline)) {
+    asm volatile("" ::: "memory");
+    fence();
+    __builtin_amdgcn_s_barrier();
+    fence();
+    asm volatile("" ::: "memory");
   };
 
-  using T_ = std::integral_constant<bool, true>;
-  using F_ = std::integral_constant<bool, false>;
-  int kt = 0;
-  if (TWO_B && DEEP) {
-    for (; kt + 3 < nk; ++kt) { ktile2(T_{}, T_{}, T_{}, true, kt); wsl = wsl == 2 ? 0 : wsl + 1; }
-    if (kt + 2 < nk) { ktile2(T_{}, F_{}, T_{}, true, kt); wsl = wsl == 2 ? 0 : wsl + 1; ++kt; }
-    for (; kt < nk; ++kt) { ktile2(F_{}, F_{}, F_{}, kt + 1 < nk, kt); wsl = wsl == 2 ? 0 : wsl + 1; }
-  } else if (TWO_B) {
-    for (; kt + 2 < nk; ++kt) ktile2(T_{}, T_{}, F_{}, true, kt);
-    for (; kt < nk; ++kt) ktile2(F_{}, F_{}, F_{}, kt + 1 < nk, kt);
-  } else if (DEEP || RS) {                         // RS: SA = write kt+2, SW = load kt+3
-    for (; kt + 3 < nk; ++kt) ktile(T_{}, T_{}, kt);
-    if (kt + 2 < nk) { ktile(T_{}, F_{}, kt); ++kt; }
-  } else {
-    for (; kt + 2 < nk; ++kt) ktile(T_{}, T_{}, kt);
-  }
-  if (!TWO_B) {
-    if (kt + 1 < nk) { ktile(F_{}, F_{}, kt); ++kt; }
-    if (nk > 0) {
-      half(a0, b0, a1, b1, abase(kt), wbase(kt, wsl), 1, true, -1, -1, 0);
-      half(a1, b1, a0, b0, smem, smem, 0, false, -1, -1, 0);
-    }
-  }
-  // MFMA results -> any other reader: the XDL write-back wait states (§5.7 item 2), tied to
-  // the last row of accumulators written so that no copy of them is hoisted above the pad
-  if constexpr ((VAR & 32768) != 0) {              // column-major order: column 7 is last
-    asm volatile("s_nop 15\n\ts_nop 15"
-                 : "+a"(acc[0][7]), "+a"(acc[1][7]), "+a"(acc[2][7]), "+a"(acc[3][7]),
-                   "+a"(acc[4][7]), "+a"(acc[5][7]), "+a"(acc[6][7]), "+a"(acc[7][7]));
-  } else {
-    asm volatile("s_nop 15\n\ts_nop 15"
-                 : "+a"(acc[7][0]), "+a"(acc[7][1]), "+a"(acc[7][2]), "+a"(acc[7][3]),
-                   "+a"(acc[7][4]), "+a"(acc[7][5]), "+a"(acc[7][6]), "+a"(acc[7][7]));
-  }
-  // accumulators leave the AGPR file by one pinned copy each, ahead of any row / column
-  // condition (an AGPR value read inside a divergent branch made hipcc move the whole
-  // accumulator set through VGPRs in the K loop)
-  auto vget = [&](const f32x4& a) -> f32x4 {
+  // one K-tile. MORE: another of the same tile follows. landed: it is in LDS already
+  auto ktile = [&](auto MORE, bool landed) __attribute__((always_inline)) {
+    constexpr bool more = decltype(MORE)::value;
+    auto after = [&](auto QC) __attribute__((always_inline)) {
+      constexpr int q = decltype(QC)::value;
+      if constexpr (q < NF) {
+        read(int_c<q>{}, a1, b1, ra1, rw1);
+        fence();
+      }
+      if constexpr (q == S::B1) {
+        __builtin_amdgcn_s_waitcnt(0xC07F);        // lgkmcnt(0)
+        barrier();
+      }
+      if constexpr (q >= S::D && q <= S::DL && (q - S::D) % S::DS == 0) {
+        piece(int_c<(q - S::D) / S::DS>{});
+        fence();
+      }
+      if constexpr (q == S::DL + 1) { next_buffer(); fence(); }
+      if constexpr (q == S::DL + 2) { next_k(); fence(); }
+      if constexpr (q == S::B2 - 1) { ra0 ^= FLIP; rw0 ^= FLIP; fence(); }
+      if constexpr (q == S::B2 && more) {
+        if (!landed) {
+          wait_vmcnt<S::ahead>();
+          barrier();
+        }
+      }
+      if constexpr (more && q > S::B2 && (q - S::B2) % 2 == 1) {
+        read(int_c<(q - S::B2) / 2>{}, a0, b0, ra0, rw0);
+        fence();
+      }
+      if constexpr (q == S::Q - 1) { ra1 ^= FLIP; rw1 ^= FLIP; fence(); }
+    };
+    // inline asm keeps the accumulators in the AGPR file ("+a"; hipcc's own selection moves them through
+    // VGPRs); it pads no hazard inside: the fragments' reads it waits for by register, the accumulators are
+    // read only as the next MFMA's C until the pad behind the loop
+    unroll<8 * NJ>([&](auto U) __attribute__((always_inline)) {
+      constexpr int u = decltype(U)::value;
+      asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
+                   : "+a"(acc[u / NJ][u % NJ]) : "v"(b0[u % NJ]), "v"(a0[u / NJ]));
+      after(U);
+    });
+    unroll<8 * NJ>([&](auto U) __attribute__((always_inline)) {
+      constexpr int u = decltype(U)::value;
+      asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
+                   : "+a"(acc[u / NJ][u % NJ]) : "v"(b1[u % NJ]), "v"(a1[u / NJ]));
+      after(int_c<8 * NJ + u>{});
+    });
+  };
+  // an accumulator leaves the AGPR file by one pinned copy, ahead of any condition
+  auto vget = [&](const f32x4& a) __attribute__((always_inline)) -> f32x4 {
     f32x4 v;
     asm volatile("" : "=v"(v) : "0"(a));
     return v;
   };
 
-  // ---- epilogue (transposed accumulators):
-  // acc[I][J][r] = C[m0 + 128 wm + 16I + fr][n0 + 128 wn + 16J + 4fq + r]
-  if constexpr (STAMP) {
-    if (threadIdx.x == 0 && ws != nullptr) {
-      unsigned long long* o = reinterpret_cast<unsigned long long*>(ws) + (long)blockIdx.x * 8;
-#pragma unroll
-      for (int k = 0; k < 6; ++k) o[k] = sseg[k];
-      o[6] = (unsigned long long)nk;
+  // ---- epilogue of a tile: acc[i][j][r] = C[m0 + 128 wm + 16 i + fr][n0 + 16 NJ wn + 16 j + 4 fq + r].
+  // ranged: whole quads (fp32, partial sums) or octets (16 bits) at aligned addresses, so that rows past the
+  // matrix fall out of the descriptor's range and columns past it get an offset out of it
+  const bool slab = splits > 1;
+  constexpr bool OUT32 = EPI == EPI_F32;
+  const int ld = slab ? N : ldc;
+  const bool ranged = [&]() {
+    const uintptr_t at = (uintptr_t)(slab ? (const void*)ws : C);
+    const bool wide = OUT32 || (slab && EPI != EPI_SLAB16);
+    const bool bias_ok = !(EPI == EPI_BIAS || EPI == EPI_BIAS_GELU) || ((uintptr_t)bias & 7) == 0;
+    return bias_ok && ld < (1 << 21) - 1024 &&
+           (wide ? ((N | ld) & 3) == 0 && (at & 15) == 0 : ((N | ld) & 7) == 0 && (at & 15) == 0);
+  }();
+  auto quad_f = [&](const f32x4& v, uint2 bq) __attribute__((always_inline)) -> f32x4 {
+    f32x4 o = v;
+    if (EPI == EPI_BIAS || EPI == EPI_BIAS_GELU) {
+      o[0] += __uint_as_float(bq.x << 16); o[1] += __uint_as_float(bq.x & 0xffff0000u);
+      o[2] += __uint_as_float(bq.y << 16); o[3] += __uint_as_float(bq.y & 0xffff0000u);
     }
-  }
-  const int wr0 = m0 + 128 * wm, wc0 = n0 + 128 * wn;
-  if (gridDim.y > 1) {
-    float* slab = ws + (long)ks * M * N;
-    const int sm = g_slab_store;
-    const bool vec = (N & 3) == 0;
+    if (EPI == EPI_BIAS_GELU) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int row = wr0 + 16 * i + fr;
-      float* srow = slab + (long)(row0 + min(row, Mg - 1)) * N;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
+      for (int r = 0; r < 4; ++r) o[r] = gelu_f(o[r]);
+    }
+    return o;
+  };
+  constexpr int OUT_OF_RANGE = (int)0x80000000;
+  // fp32 quads: logits, fp32 outputs, partial sums; returns with them in flight
+  auto store32 = [&](const Tile& t, char* base, uint32_t* keys) __attribute__((always_inline)) {
+    const int left = min(t.rows - t.m0, BM), cols = N - t.n0;
+    const auto rc = make_rsrc(base, left * ld * 4);
+    const int c0 = 16 * NJ * wn + 4 * fq, vo = ((128 * wm + fr) * ld + c0) * 4;
+    unroll<8>([&](auto I) __attribute__((always_inline)) {
+      constexpr int i = decltype(I)::value;
+      BlockMax top;
+      unroll<NJ>([&](auto J) __attribute__((always_inline)) {
+        constexpr int j = decltype(J)::value;
         const f32x4 v = vget(acc[i][j]);
-        const int col = wc0 + 16 * j + 4 * fq;
-        if (row < Mg && col < N) slab_quad_fp32(srow + col, v, sm & 3, vec, N - col);
+        const bool in = c0 + 16 * j < cols;
+        if (EPI == EPI_F32 && in) top.take(v);
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rc,
+                                               in ? vo + 64 * j : OUT_OF_RANGE, i * 16 * ld * 4, 0);
+      });
+      if constexpr (EPI == EPI_F32) {
+        if (keys != nullptr) {                     // uniform
+          const uint32_t key = row_key(top);
+          const int row = t.m0 + 128 * wm + 16 * i + fr, wc0 = t.n0 + 16 * NJ * wn;
+          if (fq == 0 && row < t.rows && wc0 < N)
+            keys[(long)row * ((N + 16 * NJ - 1) / (16 * NJ)) + wc0 / (16 * NJ)] = key;
+        }
       }
+    });
+  };
+  // 16-bit outputs: neighbouring blocks' quads change places between lanes 16 apart, so that a lane holds 8
+  // columns and a store covers 64 B of each row
+  auto store16 = [&](const Tile& t, char* base) __attribute__((always_inline)) {
+    constexpr int NO = PAIRS ? NJ / 2 : NJ;        // blocks of 16 output columns
+    const int left = min(t.rows - t.m0, BM), cols = (PAIRS ? N / 2 : N) - (PAIRS ? t.n0 / 2 : t.n0);
+    const auto rc = make_rsrc(base, left * ld * 2);
+    const int c0 = 16 * NO * wn + 16 * (fq & 1) + 8 * (fq >> 1), c1 = 16 * NO * wn + 16 * (NO - 1) + 4 * fq;
+    const int ro = (128 * wm + fr) * ld * 2;
+    uint2 bq[NJ];
+    if constexpr (EPI == EPI_BIAS || EPI == EPI_BIAS_GELU) {
+      const auto rb = make_rsrc(bias, N * 2);
+      unroll<NJ>([&](auto J) __attribute__((always_inline)) {
+        constexpr int j = decltype(J)::value;
+        const auto b = __builtin_amdgcn_raw_buffer_load_b64(rb, (t.n0 + 16 * NJ * wn + 16 * j + 4 * fq) * 2, 0, 0);
+        bq[j] = uint2{b[0], b[1]};
+      });
     }
-    return;
-  }
-  const bool vec = out_vec<EPI>(C, ldc, N, bias);
-  if (EPI == EPI_SILU) {
+    unroll<8>([&](auto I) __attribute__((always_inline)) {
+      constexpr int i = decltype(I)::value;
+      auto quad = [&](auto J) __attribute__((always_inline)) -> uint2 {
+        constexpr int j = decltype(J)::value;
+        if constexpr (PAIRS) {
+          const f32x4 g = vget(acc[i][2 * j]), u = vget(acc[i][2 * j + 1]);
+          float o[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) o[r] = pair_f<EPI>(g[r], u[r], 0.f);
+          return uint2{pack2bf(o[0], o[1]), pack2bf(o[2], o[3])};
+        } else if constexpr (EPI == EPI_SLAB16) {
+          const f32x4 v = vget(acc[i][j]);
+          return uint2{pack2h(v[0] * SLAB16_SCALE, v[1] * SLAB16_SCALE),
+                       pack2h(v[2] * SLAB16_SCALE, v[3] * SLAB16_SCALE)};
+        } else {
+          const f32x4 o = quad_f(vget(acc[i][j]), bq[j]);
+          return uint2{pack2bf(o[0], o[1]), pack2bf(o[2], o[3])};
+        }
+      };
+      unroll<NO / 2>([&](auto J) __attribute__((always_inline)) {
+        constexpr int j = 2 * decltype(J)::value;
+        const uint2 x = quad(int_c<j>{}), y = quad(int_c<j + 1>{});
+        const auto p = __builtin_amdgcn_permlane16_swap(x.x, y.x, false, false);
+        const auto q = __builtin_amdgcn_permlane16_swap(x.y, y.y, false, false);
+        __builtin_amdgcn_raw_buffer_store_b128(u32x4{p[0], q[0], p[1], q[1]}, rc,
+                                               c0 + 16 * j < cols ? ro + 2 * c0 + 32 * j : OUT_OF_RANGE,
+                                               i * 16 * ld * 2, 0);
+      });
+      if constexpr (NO & 1) {
+        const uint2 x = quad(int_c<NO - 1>{});
+        __builtin_amdgcn_raw_buffer_store_b64(u32x2{x.x, x.y}, rc, c1 < cols ? ro + 2 * c1 : OUT_OF_RANGE,
+                                              i * 16 * ld * 2, 0);
+      }
+    });
+  };
+  // any width and alignment, quad by quad
+  auto store_any = [&](const Tile& t) __attribute__((always_inline)) {
+    const int wr0 = t.m0 + 128 * wm, wc0 = t.n0 + 16 * NJ * wn;
+    const bool vec = slab ? (N & 3) == 0 : out_vec<EPI>(C, ldc, N, bias);
+    float* sl = ws + (long)t.ks * M * N;
+    unroll<8>([&](auto I) __attribute__((always_inline)) {
+      constexpr int i = decltype(I)::value;
+      const int row = wr0 + 16 * i + fr;
+      BlockMax top;
+      unroll<NJ>([&](auto J) __attribute__((always_inline)) {
+        constexpr int j = decltype(J)::value;
+        const int col = wc0 + 16 * j + 4 * fq;
+        if constexpr (PAIRS) {
+          if constexpr (j % 2 == 0) {
+            const f32x4 g = vget(acc[i][j]), u = vget(acc[i][j + 1]);
+            if (slab) {
+              float* p = sl + (long)(t.row0 + row) * N + col;
+              if (row < t.rows && col < N) slab_quad_fp32(p, g, 0, vec, N - col);
+              if (row < t.rows && col + 16 < N) slab_quad_fp32(p + 16, u, 0, vec, N - col - 16);
+            } else if (row < t.rows && col < N) {
+              store_pair_quad<EPI>(C, ldc, t.row0 + row, ((wc0 + 16 * j) >> 5) * 16 + 4 * fq, g, u, vec);
+            }
+          }
+        } else {
+          const f32x4 v = vget(acc[i][j]);
+          if (EPI == EPI_F32 && col < N) top.take(v);
+          if (row < t.rows && col < N) {
+            if (EPI == EPI_SLAB16)
+              slab_quad16(sl + (long)(t.row0 + row) * N + col, v, vec, N - col, ws);
+            else if (slab)
+              slab_quad_fp32(sl + (long)(t.row0 + row) * N + col, v, 0, vec, N - col);
+            else
+              store_quad<EPI>(C, ldc, t.row0 + row, col, N, v, bias, vec);
+          }
+        }
+      });
+      if constexpr (EPI == EPI_F32) {
+        if (!slab && bias != nullptr) {            // uniform: the block's largest value (BlockMax)
+          const uint32_t key = row_key(top);
+          if (fq == 0 && row < t.rows && wc0 < N)
+            ((uint32_t*)bias)[(long)row * ((N + 16 * NJ - 1) / (16 * NJ)) + wc0 / (16 * NJ)] = key;
+        }
+      }
+    });
+  };
+  // stores issued behind the next tile's pieces, which may fly while those are waited for (6 bits count)
+  constexpr int N32 = 8 * NJ, N16 = 8 * (((PAIRS ? NJ / 2 : NJ) + 1) / 2);
+  auto epilogue = [&](const Tile& t) __attribute__((always_inline)) {
+    if (!ranged) {
+      store_any(t);
+      asm volatile("" ::: "memory");
+      wait_vmcnt<0>();
+    } else if (EPI == EPI_F32 || (EPI != EPI_SLAB16 && slab)) {
+      char* base = slab ? (char*)(ws + ((long)t.ks * M + t.row0 + t.m0) * N + t.n0)
+                        : (char*)((float*)C + (long)(t.row0 + t.m0) * ldc + t.n0);
+      store32(t, base, EPI == EPI_F32 && !slab ? (uint32_t*)const_cast<u16*>(bias) : nullptr);
+      asm volatile("" ::: "memory");
+      wait_vmcnt<(N32 < 63 ? N32 : 63)>();
+    } else {
+      char* base = EPI == EPI_SLAB16 ? (char*)((u16*)ws + ((long)t.ks * M + t.row0 + t.m0) * N + t.n0)
+                                     : (char*)((u16*)C + (long)(t.row0 + t.m0) * ldc + (PAIRS ? t.n0 / 2 : t.n0));
+      store16(t, base);
+      asm volatile("" ::: "memory");
+      wait_vmcnt<(N16 < 63 ? N16 : 63)>();
+    }
+  };
+
+  using T_ = std::integral_constant<bool, true>;
+  using F_ = std::integral_constant<bool, false>;
+  int v = blockIdx.x;
+  if (v >= total) return;                          // wave-uniform: every wave exits
+  Tile t = locate(v);
+  // K-tiles 0 and 1 of the first tile (a K of one K-tile: the second is zeros)
+  begin_stage(t, true);
+  unroll<NP>(piece);
+  next_buffer();
+  next_k();
+  if (nk < 2) sab = swb = 0;
+  unroll<NP>(piece);
+  next_buffer();
+  next_k();
+  wait_vmcnt<0>();
+  barrier();
+
+  while (true) {                                   // every wave runs the same tiles
+    const int vn = v + (int)gridDim.x;
+    const bool has_next = vn < total;
+    Tile tn = t;
+    if (has_next) tn = locate(vn);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // the zeroed accumulators are read by inline-asm MFMAs, which hipcc pads no hazard for: pin every write
+    // ahead of a few wait states
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const int row = wr0 + 16 * i + fr;
 #pragma unroll
-      for (int j = 0; j < 8; j += 2) {
-        const f32x4 g = vget(acc[i][j]), u = vget(acc[i][j + 1]);
-        const int gcol = wc0 + 16 * j;
-        if (row < Mg && gcol < N)
-          store_pair_quad(C, ldc, row0 + row, (gcol >> 5) * 16 + 4 * fq, g, u, vec);
-      }
+      for (int j = 0; j < NJ; ++j) asm volatile("" : "+a"(acc[i][j]));
+      asm volatile("s_nop 3");
     }
-    return;
-  }
+    unroll<NF>([&](auto F) __attribute__((always_inline)) { read(F, a0, b0, ra0, rw0); });
+    // (K-tile 1 is there, and the last tile's stores need not have left: nothing to wait for in K-tile 0)
+    if (nk > 2) ktile(T_{}, true);
+    for (int kt = 1; kt + 2 < nk; ++kt) ktile(T_{}, false);
+    // the last two K-tiles stage the next tile's first two. Without a next tile they stage through an empty
+    // range (no memory traffic, zeros): one code path, since a branch doubles the unrolled tail and hipcc
+    // spills the fragments
+    begin_stage(tn, has_next);
+    ktile(T_{}, nk <= 2);
+    if (nk < 2) sab = swb = 0;
+    ktile(F_{}, false);
+    // MFMA results -> the epilogue's copies: the XDL write-back's wait states, tied to the last row of
+    // accumulators written so that no copy of them moves above the pad
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int row = wr0 + 16 * i + fr;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const f32x4 v = vget(acc[i][j]);
-      const int col = wc0 + 16 * j + 4 * fq;
-      if (row < Mg && col < N) store_quad<EPI>(C, ldc, row0 + row, col, N, v, bias, vec);
-    }
+    for (int j = 0; j < NJ; ++j) asm volatile("" : "+a"(acc[7][j]));
+    epilogue(t);       // (and its wait: the next tile's K-tiles 0 and 1 landed, also before an exit)
+    if (!has_next) break;
+    barrier();
+    v = vn;
+    t = tn;
   }
 }
 
-template <int EPI, int VAR>
-static int launch_4w(const void* A, int lda, const void* W, int ldw, void* C, int ldc, int M,
-                     int N, int K, int splits, const void* bias, void* ws, const int* group_off,
-                     int groups, hipStream_t st) {
-  if (EPI == EPI_SILU && N % 32) return (int)hipErrorInvalidValue;
-  const int tiles = ((M + 255) / 256) * ((N + 255) / 256);
-  int ksl = K / splits;
-  ksl = (ksl / BK) * BK;
-  if (ksl * splits != K) return (int)hipErrorInvalidValue;
-  constexpr size_t lds = ((VAR & 32) ? 5 : 4) * (size_t)256 * BK * 2;
-  static bool attr_done = false;
-  if (!attr_done) {
-    hipFuncSetAttribute((const void*)gemm4w_kernel<EPI, VAR>,
-                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    attr_done = true;
+static int cu_count() {
+  static int cus = 0;
+  if (!cus) {
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    if (cus <= 0) cus = 256;
   }
-  dim3 grid(tiles, splits, groups);
-  gemm4w_kernel<EPI, VAR><<<grid, 256, lds, st>>>((const u16*)A, lda, (const u16*)W, ldw, C,
-                                                  ldc, M, N, K, ksl, (const u16*)bias,
-                                                  (float*)ws, group_off);
+  return cus;
+}
+
+// M: rows, or the most rows of a group (group_off: their offsets, groups of them)
+template <int EPI, int NJ>
+static int launch_4w(const void* A, int lda, const void* W, int ldw, void* C, int ldc, int M, int N,
+                     int K, int splits, const void* bias, void* ws, const int* group_off, int groups,
+                     hipStream_t st) {
+  if (epi_pairs(EPI) && N % 32) return (int)hipErrorInvalidValue;
+  if (K % (splits * BK)) return (int)hipErrorInvalidValue;
+  constexpr size_t lds = 0x10000 + (size_t)(256 + 32 * NJ) * BK * 2;
+  static bool raised = false;
+  if (!raised) {
+    hipFuncSetAttribute((const void*)gemm4w_kernel<EPI, NJ>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                        (int)lds);
+    raised = true;
+  }
+  const int cus = cu_count();
+  const long tiles = (long)((M + 255) / 256) * ((N + 32 * NJ - 1) / (32 * NJ)) * splits *
+                     (group_off != nullptr ? groups : 1);
+  // one workgroup per CU (over 80 KiB of LDS each); a multiple of 8 keeps every workgroup's virtual tile ids
+  // on one XCD residue class
+  int grid = tiles < cus ? (int)tiles : (cus / 8) * 8;
+  if (grid < 1) grid = 1;
+  gemm4w_kernel<EPI, NJ><<<grid, 256, lds, st>>>((const u16*)A, lda, (const u16*)W, ldw, C, ldc, M, N, K, splits,
+                                                 (const u16*)bias, (float*)ws, group_off, groups);
   if (splits > 1 && C != nullptr) {
-    const int outN = (EPI == EPI_SILU) ? N / 2 : N;
+    const int outN = epi_pairs(EPI) ? N / 2 : N;
     const long total = (long)M * outN;
     splitk_reduce_kernel<EPI><<<(int)((total + 255) / 256), 256, 0, st>>>(
         C, ldc, (const float*)ws, M, N, splits, (const u16*)bias);
   }
   DLI_RETURN_LAUNCH();
 }
-

@@ -47,13 +47,10 @@ TILES = {0: (64, 64), 1: (64, 128), 2: (128, 128), 3: (128, 256), 4: (256, 128),
          # N = 4096 at M = 512 with split-K 4
          28: (256, 128),
          # 256x256, 4 waves (one per SIMD), 128x128 wave tiles, accumulators pinned in the AGPR
-         # file (gemm4w_kernel); 41 = 34 with a 3-stage weight ring (160 KiB LDS: W fetched a
-         # K-tile further ahead); 45 = 34 with two barriers per K-tile (the buffer released
-         # after 20 MFMAs, the next-next K-tile's DMA over 80 MFMAs). The losing A/B variants
-         # 35-40 / 42-44 / 46-53 are not instantiated (profiles/r4/gemm4w/)
+         # file, at most a workgroup a CU that walks its tiles (gemm4w.h)
          34: (256, 256), 41: (256, 256), 45: (256, 256),
-         # 55 = 45 persistent: one workgroup per CU walks its tiles, the next tile's first two
-         # K-tiles staged in the current tile's last two (gemm4wp.hip); no split-K / grouped
+         # 55: the same on tiles of 256, 192 or 160 columns, by rounds of the chip (gemm4wp.hip);
+         # no split-K / grouped
          55: (256, 256)}
 # weight-streaming tiles for up to 128 rows (gemm_stream.h): weights nontemporal, K loops turned from
 # tile to tile, 3 to 6 stages; (BM, BN, K-tile: a split of K holds whole ones), so kept apart

@@ -22,8 +22,8 @@
 // gate/up weight (output width N/2), 3 bias + tanh-GELU, 4 bias.
 //
 // Files: gemm_common.h (shared epilogue / split-K pieces), gemm_tiles.hip (ids 0-21, 23-25),
-// gemm_stream.hip (60-72: few rows, weights streamed), gemm8p.hip (22, 26-28), gemm4w.h +
-// gemm4w.hip (34, 41, 45), gemm4wp.hip (55), gemv.hip (29-33 and the fused batch-1 combine).
+// gemm_stream.hip (60-72: few rows, weights streamed), gemm4w.h +
+// gemm4w.hip, gemm4w_narrow.hip (22, 28, 34, 41, 45, 55), gemm8p.hip (26; 22 and 28 with the rarer epilogues), gemv.hip (29-33 and the fused batch-1 combine).
 #include "gemm_common.h"
 
 extern "C" int dli_gemm_set_slab_store(int mode) {
@@ -47,10 +47,10 @@ extern "C" int dli_gemm_set_slab_store_family(int family, int mode) {
 // tiles with 3 LDS stages (one tile in flight across the barrier); 10/11 = 192x128 with 2/3
 // stages, 12 = 160x128 (MoE experts of ~130-190 rows in one pass); 13-17 = 8-wave tiles
 // 256x256, 256x128, 128x256 (2 stages) and 256x128, 128x256 (3 stages); 18/19 = 128x96 and
-// 20/21 = 128x64 with 2/3 stages; 22 = 256x256 8-phase ping-pong; 23/24 = 128x192 (3/2
+// 20/21 = 128x64 with 2/3 stages; 22 = 256x256; 23/24 = 128x192 (3/2
 // stages), 25 = 256x192, 8 waves; 26 = 256x224 ping-pong; 29-33 = the M <= 4 weight
-// stream (16 / 32 rows per workgroup, dispatch_gemv); 34, 41, 45 = 256x256, 4 waves; 55 = the
-// same on tiles of 256, 192 or 160 columns (no split-K / grouped mode); 60-72 = weight-streaming tiles
+// stream (16 / 32 rows per workgroup, dispatch_gemv); 28 = 256x128; 34, 41, 45 = 256x256;
+// 55 = 256x256, 192 or 160 (no split-K / grouped mode); 60-72 = weight-streaming tiles
 // (gemm_stream.h). ws: fp32 [splits, M, N] when splits>1.
 // group_off (nullable): int[groups+1] row offsets; M is then the max rows of any group.
 // Grouped SiLU*up GEMM whose permuted row p reads activation row arow[p] (the MoE gate/up
@@ -89,9 +89,8 @@ extern "C" int dli_gemm(const void* A, int lda, const void* W, int ldw, void* C,
   const int* go = group_off;
   int r = gemm_tiles_dispatch(epi, tile_cfg, DLI_GEMM_PASS);
   if (r == DLI_NOT_MINE) r = gemm_stream_dispatch(epi, tile_cfg, DLI_GEMM_PASS);
-  if (r == DLI_NOT_MINE) r = gemm_8p_dispatch(epi, tile_cfg, DLI_GEMM_PASS);
   if (r == DLI_NOT_MINE) r = gemm_4w_dispatch(epi, tile_cfg, DLI_GEMM_PASS);
-  if (r == DLI_NOT_MINE) r = gemm_4wp_dispatch(epi, tile_cfg, DLI_GEMM_PASS);
+  if (r == DLI_NOT_MINE) r = gemm_8p_dispatch(epi, tile_cfg, DLI_GEMM_PASS);
   if (r == DLI_NOT_MINE) r = gemm_gemv_dispatch(epi, tile_cfg, DLI_GEMM_PASS);
   return r == DLI_NOT_MINE ? (int)hipErrorInvalidValue : r;
 }
@@ -126,7 +125,7 @@ extern "C" int dli_gemm_head(const void* A, int lda, const void* W, int ldw, voi
   void* ws = nullptr;
   const int* go = nullptr;
   const int splits = 1, groups = 1;
-  if (tile_cfg == 55) return gemm_4wp_dispatch(EPI_F32, tile_cfg, DLI_GEMM_PASS);
+  if (tile_cfg == 55) return gemm_4w_dispatch(EPI_F32, tile_cfg, DLI_GEMM_PASS);
   if (tile_cfg >= 60) return gemm_stream_dispatch(EPI_F32, tile_cfg, DLI_GEMM_PASS);
   return gemm_gemv_dispatch(EPI_F32, tile_cfg, DLI_GEMM_PASS);
 }

@@ -1,6 +1,6 @@
 // 256-row GEMM tiles with ONE wave per SIMD: four waves of 128 x 16 NJ, their 8 NJ 16x16 blocks
 // accumulated in the AGPR file, on a grid of at most one workgroup a CU that walks its tiles
-// (tiles 34, 41, 45: gemm4w.hip; 55: gemm4wp.hip).
+// (tiles 22, 28, 34, 41, 45 and 55: gemm4w.hip).
 //
 // What bounds it. Bare 16x16x32 MFMAs on random data run at 2.0 GHz (2.07 PFLOP/s), which the power
 // budget sets; with this tile's 32 fragment reads and 16 LDS-DMA pieces a K-tile at 1.75 GHz and 17.6

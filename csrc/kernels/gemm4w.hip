@@ -1,11 +1,83 @@
-// Tiles 34, 41 and 45: 256x256, split-K and grouped products (gemm4w.h). One kernel: the three ids remain from
-// kernels that differed in their schedules.
+// Tiles 22, 28, 34, 41, 45 and 55 on the 4-wave kernel (gemm4w.h): 256 columns here, narrower ones in
+// gemm4w_narrow.hip, and the rules that choose between them.
+//   34, 41, 45  256 columns (three ids from kernels that differed in their schedules)
+//   22          256 columns, or by rounds as below where the product is dense and not biased
+//   28          128 columns
+//   55          256, 192 or 160 by rounds; dense, unsplit, K a multiple of 128
+// Against the 8-phase kernels that 22 and 28 were (gemm8p.hip keeps what is not built here), us: 16384 x 6144 x 4096
+// 595 -> 533, 8192 x 4096 x 14336 664 -> 631, 8192 x 28672 with SiLU pairs 1318 -> 1231, 4096 x 2304 x 768 with
+// a bias 32 -> 23; partial sums in 16 bits of 512 rows: 6144 x 4096 in four 35.8 -> 27.0, 4096 x 4096 in four 26.5
+// (eight) -> 21.6, 4096 x 14336 in eight 60.9 -> 50.9.
 #include "gemm4w.h"
 
-template <int EPI>
-static int dispatch_4w(int tile_cfg, DLI_GEMM_ARGS) {
-  if (tile_cfg != 34 && tile_cfg != 41 && tile_cfg != 45) return DLI_NOT_MINE;
-  return launch_4w<EPI, 8>(DLI_GEMM_PASS);
+int gemm_4w_narrow(int epi, int nj, DLI_GEMM_ARGS);
+
+// The tile width, in 32 columns, whose rounds take least. A round's price is its width times what the narrower
+// schedule costs more (fewer MFMAs between the same barriers: 1.6, 5, 9 and 15 %), the last one's by how many CUs
+// it keeps, and little less for few of them, which clock higher. 256 columns unless another is 3 % better.
+// K = 4096, bf16 outputs, 16 columns of tiles, us at 256 / 224 / 192 / 160 / 128: a quarter of a round 69 / 62 / 54
+// / 48 / 40, three 80 / 74 / 64 / 57 / 47, one round 95 / 84 / 75 / 65 / 54, 1.25 155 / 139 / 122 / 106 / 88, 1.75
+// 173 / 154 / 133 / 117 / 98, two 186 / 166 / 147 / 127 / 105; K = 1024 and 14336 and fp32 outputs within 5 % of the
+// same ratios. Tile 55 chooses among 8, 6 and 5, its widths where the LM head's block maxima are laid out by them
+// (ops/gemm.py's persistent_width is its copy).
+static int width_of(int M, int N, int splits, bool pairs, bool all) {
+  const double cus = cu_count();
+  const double price[9] = {0, 0, 0, 0, 0.573, 0.684, 0.794, 0.889, 1.0};
+  int best = 8;
+  double least = 0.0;
+  for (int nj = 8; nj >= 4; --nj) {
+    if ((!all && (nj == 7 || nj == 4)) || (pairs && nj & 1)) continue;
+    const long tiles = (long)((M + 255) / 256) * ((N + 32 * nj - 1) / (32 * nj)) * splits;
+    const double whole = (double)(tiles / (long)cus), x = tiles / cus - whole;
+    const double last = x == 0 ? 0.0 : whole == 0 ? 0.72 + 0.28 * x * x * x
+                                                  : 0.60 + 0.25 * x + 0.15 * x * x * x;
+    const double c = (whole + last) * price[nj];
+    if (nj == 8) least = 0.97 * c;
+    else if (c < least) { least = c; best = nj; }
+  }
+  return best;
 }
 
-int gemm_4w_dispatch(int epi, int tile_cfg, DLI_GEMM_ARGS) { DLI_EPI_SWITCH_BASE(dispatch_4w) }
+static int launch8(int epi, DLI_GEMM_ARGS) {
+  switch (epi) {
+    case EPI_BF16: return launch_4w<EPI_BF16, 8>(DLI_GEMM_PASS);
+    case EPI_F32: return launch_4w<EPI_F32, 8>(DLI_GEMM_PASS);
+    case EPI_SILU: return launch_4w<EPI_SILU, 8>(DLI_GEMM_PASS);
+    case EPI_GELU_MUL: return launch_4w<EPI_GELU_MUL, 8>(DLI_GEMM_PASS);
+    case EPI_BIAS: return launch_4w<EPI_BIAS, 8>(DLI_GEMM_PASS);
+    case EPI_BIAS_GELU: return launch_4w<EPI_BIAS_GELU, 8>(DLI_GEMM_PASS);
+    case EPI_SLAB16: return launch_4w<EPI_SLAB16, 8>(DLI_GEMM_PASS);
+    default: return DLI_NOT_MINE;
+  }
+}
+
+int gemm_4w_dispatch(int epi, int tile_cfg, DLI_GEMM_ARGS) {
+  const bool pairs = epi_pairs(epi), bias_epi = epi == EPI_BIAS || epi == EPI_BIAS_GELU;
+  int nj = 8;
+  switch (tile_cfg) {
+    case 34: case 41: case 45:
+      if (epi == EPI_GELU_MUL || epi == EPI_SLAB16) return DLI_NOT_MINE;
+      break;
+    case 22:
+      if (pairs && N % 64) return (int)hipErrorInvalidValue;
+      if (go == nullptr && !bias_epi) nj = width_of(M, N, splits, pairs, true);
+      break;
+    case 28:
+      nj = 4;
+      break;
+    case 55:
+      if (epi == EPI_SLAB16) return DLI_NOT_MINE;
+      if (splits != 1 || go != nullptr || K % (2 * BK) || C == nullptr) return (int)hipErrorInvalidValue;
+      // (the biased epilogues, which few products take, are built in one width)
+      if (!bias_epi) nj = width_of(M, N, 1, pairs, false);
+      break;
+    default: return DLI_NOT_MINE;
+  }
+  if (epi == EPI_SLAB16 && (C != nullptr || splits < 2)) return (int)hipErrorInvalidValue;
+  return nj == 8 ? launch8(epi, DLI_GEMM_PASS) : gemm_4w_narrow(epi, nj, DLI_GEMM_PASS);
+}
+
+// the columns of the tiles that tile 55 takes for a product
+extern "C" int dli_gemm_persistent_width(int M, int N, int pairs) {
+  return 32 * width_of(M, N, 1, pairs != 0, false);
+}

@@ -1,5 +1,5 @@
-// 8-wave "8-phase ping-pong" MFMA GEMMs (tile ids 22, 26, 28): 256x256 (gemm8p_kernel),
-// 256x224 (gemm8p224_kernel) and 256x128 (gemm8p128_kernel) block tiles, two wave groups
+// 8-wave "8-phase ping-pong" MFMA GEMMs (tile id 26, and 22 and 28 with the epilogues that gemm4w.hip does not build):
+// 256x256 (gemm8p_kernel), 256x224 (gemm8p224_kernel) and 256x128 (gemm8p128_kernel) block tiles, two wave groups
 // alternating MFMA and load segments (cdna_hip_programming.md §5 'The 256² 8-phase template').
 #include "gemm_common.h"
 
@@ -910,16 +910,18 @@ static int launch_8p128(const void* A, int lda, const void* W, int ldw, void* C,
 
 template <int EPI>
 static int dispatch_8p(int tile_cfg, DLI_GEMM_ARGS) {
-  switch (tile_cfg) {
-    // 256x256 8-phase ping-pong (gemm8p_kernel)
-    case 22: return launch_8p<EPI, GEMM8P_DEFAULT>(DLI_GEMM_PASS);
-    // 256x224 ping-pong (gemm8p224_kernel): N = 28672 gate/up at M = 512 is 256 tiles
-    case 26: return launch_8p224<EPI>(DLI_GEMM_PASS);
-    // 256x128 ping-pong (gemm8p128_kernel): Mixtral grouped down (8 x 32 tiles), N = 4096 at
-    // M = 512 (64 tiles x split 4)
-    case 28: return launch_8p128<EPI>(DLI_GEMM_PASS);
-    default: return DLI_NOT_MINE;
+  // 256x224 ping-pong (gemm8p224_kernel): N = 28672 gate/up at M = 512 is 256 tiles
+  if (tile_cfg == 26) return launch_8p224<EPI>(DLI_GEMM_PASS);
+  // 256x256 (gemm8p_kernel) and 256x128 (gemm8p128_kernel) for the epilogues that the 4-wave kernel, which comes
+  // first and is faster, does not build
+  constexpr bool rest = EPI == EPI_GELU_ERF || EPI == EPI_CLAMP || EPI == EPI_RELU;
+  if constexpr (rest) {
+    if (tile_cfg == 22) return launch_8p<EPI, GEMM8P_DEFAULT>(DLI_GEMM_PASS);
   }
+  if constexpr (rest || EPI == EPI_BIAS || EPI == EPI_BIAS_GELU) {
+    if (tile_cfg == 28) return launch_8p128<EPI>(DLI_GEMM_PASS);
+  }
+  return DLI_NOT_MINE;
 }
 
 int gemm_8p_dispatch(int epi, int tile_cfg, DLI_GEMM_ARGS) { DLI_EPI_SWITCH_S16(dispatch_8p) }

@@ -339,7 +339,6 @@ int gemm_tiles_dispatch(int epi, int tile_cfg, DLI_GEMM_ARGS);
 int gemm_stream_dispatch(int epi, int tile_cfg, DLI_GEMM_ARGS);
 int gemm_8p_dispatch(int epi, int tile_cfg, DLI_GEMM_ARGS);
 int gemm_4w_dispatch(int epi, int tile_cfg, DLI_GEMM_ARGS);
-int gemm_4wp_dispatch(int epi, int tile_cfg, DLI_GEMM_ARGS);
 int gemm_gemv_dispatch(int epi, int tile_cfg, DLI_GEMM_ARGS);
 int gemm_tiles_set_slab_store(int mode);
 int gemm_stream_set_slab_store(int mode);
@@ -360,9 +359,6 @@ int gemm_8p_set_slab_store(int mode);
 #define DLI_EPI_SWITCH(FN)                                                         \
   if (epi == EPI_GELU_ERF) return FN<EPI_GELU_ERF>(tile_cfg, DLI_GEMM_PASS);       \
   DLI_EPI_SWITCH_BASE(FN)
-
-// without the exact-GELU epilogue: the 4-wave families, whose 256-accumulator epilogue does
-// not unroll with it (the accumulators would leave the AGPR file inside the K loop)
 #define DLI_EPI_SWITCH_BASE(FN)                                                    \
   switch (epi) {                                                                   \
     case EPI_BF16: return FN<EPI_BF16>(tile_cfg, DLI_GEMM_PASS);                   \

@@ -49,7 +49,7 @@ TILES = {0: (64, 64), 1: (64, 128), 2: (128, 128), 3: (128, 256), 4: (256, 128),
          # 256x256, 4 waves (one per SIMD), 128x128 wave tiles, accumulators pinned in the AGPR
          # file, at most a workgroup a CU that walks its tiles (gemm4w.h)
          34: (256, 256), 41: (256, 256), 45: (256, 256),
-         # 55: the same on tiles of 256, 192 or 160 columns, by rounds of the chip (gemm4wp.hip);
+         # 55: the same on tiles of 256, 192 or 160 columns, by rounds of the chip;
          # no split-K / grouped
          55: (256, 256)}
 # weight-streaming tiles for up to 128 rows (gemm_stream.h): weights nontemporal, K loops turned from
@@ -453,15 +453,15 @@ def device_cus() -> int:
 
 @functools.lru_cache(maxsize=8192)
 def persistent_width(M: int, N: int, pairs: bool, cus: int = NUM_CUS) -> int:
-    """Columns of the tiles that the persistent kernel (tile 55) takes on ``cus`` CUs: gemm4wp.hip's
+    """Columns of the tiles that the persistent kernel (tile 55) takes on ``cus`` CUs: gemm4w.hip's
     width_of."""
     best, least = 256, 0.0
-    for nj, price in ((8, 1.0), (6, 1.09 * 6 / 8), (5, 1.13 * 5 / 8)):
+    for nj, price in ((8, 1.0), (6, 0.794), (5, 0.684)):
         if pairs and nj & 1:
             continue
         whole, rest = divmod(-(-M // 256) * -(-N // (32 * nj)), cus)
         x = rest / cus
-        last = 0.0 if not rest else 0.66 + 0.25 * x + 0.09 * x ** 3 if whole else 0.8 + 0.2 * x ** 3
+        last = 0.0 if not rest else 0.60 + 0.25 * x + 0.15 * x ** 3 if whole else 0.72 + 0.28 * x ** 3
         c = (whole + last) * price
         if nj == 8:
             least = 0.97 * c

@@ -6,10 +6,11 @@ import torch
 
 from distributed_llm_inferencing_amd import ops
 from distributed_llm_inferencing_amd.ops import gemm as G
+from test_head_maxima import block_keys
 
 # fp32 sums of exact products of up to 1280 values: 1e-5; bf16 results are rounded once, half an ulp (2^-9) a value
 BOUND = {True: 1e-5, False: 2.0 ** -8}
-TILES = [45]
+TILES = [45, 22, 28]      # 256 columns, by rounds of the chip, 128
 
 
 def operands(gpu, M, N, K, seed, groups=1):
@@ -48,6 +49,20 @@ def test_products(gpu, M, N, K, splits, tile):
         b = bias if epi.startswith("bias") else None
         got = ops._gemm_native(x, w[0], epi, bias=b, plan=G.GemmPlan("dli", tile, splits))
         assert off(got, expected(x, w[0], epi, bias)) < BOUND[epi == "f32"], epi
+
+
+# partial sums in 16 bits on tiles of every width that tile 22 takes (a third column: the last tiles' columns); half
+# an ulp (2^-11) of each of the slices, whose squares add up to the sum's
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,splits", [(300, 15000, 256, 2), (300, 12808, 256, 2), (512, 6144, 1024, 4), (300, 10244, 384, 2),
+                                          (512, 4096, 1024, 4), (257, 1001, 512, 8)])
+@pytest.mark.parametrize("tile", [22, 28])
+def test_partial_sums_in_16_bits(gpu, M, N, K, splits, tile):
+    x, w = operands(gpu, M, N, K, M + N)
+    ws = torch.zeros(splits, M, N, device=gpu, dtype=torch.float16)
+    ops._native_call("dli_gemm", ops._p(x), K, ops._p(w), K, None, N, M, N, K, G.EPI["slab16"], tile, splits, None,
+                     ops._p(ws), None, 1, ops._st())
+    assert off(ws.double().sum(0) * 16, expected(x, w[0], "none")) < 2.0 ** -11
 
 
 # outputs inside a wider buffer, whole and odd offsets: nothing beside the product is written
@@ -94,3 +109,16 @@ def test_values_at_the_limits(gpu, tile):
     assert got[0] == float("inf") and got[3] > 2.9e38 and got[6] == 90.0 and got[7] == got[8] == 0
     assert got[1] != got[1] and got[2] != got[2]        # -inf / inf, NaN
     assert abs(got[4]) < 1e-30 and abs(got[5]) < 1e-30
+
+
+# the LM head of a plan on tile 22 writes block maxima too, as tile 55 (the same kernel); they are exact
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(300, 1000, 512), (257, 20000, 256), (300, 24000, 128), (300, 30720, 512), (300, 1000, 192)])
+def test_block_maxima_of_the_head(gpu, monkeypatch, M, N, K):
+    x, w = operands(gpu, M, N, K, M + N)
+    monkeypatch.setattr(G, "row_cut", lambda *a: 0)
+    monkeypatch.setattr(G, "plan", lambda *a, **k: G.GemmPlan("dli", 22, 1))
+    logits, top = ops.head(x, w[0])
+    assert off(logits, expected(x, w[0], "f32")) < BOUND[True]
+    assert (top is None) == (K % 128 != 0)               # tile 55 takes whole pairs of K-tiles
+    assert top is None or torch.equal(top[0], block_keys(logits, top[1]))

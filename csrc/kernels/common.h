@@ -37,8 +37,11 @@ __device__ __forceinline__ u16 f2bf(float f) {
   return *reinterpret_cast<u16*>(&b);
 }
 
+// two roundings to nearest even in one v_cvt_pk_bf16_f32 (by f2bf of each: two of them, a shift and an or)
 __device__ __forceinline__ uint32_t pack2bf(float lo, float hi) {
-  return (uint32_t)f2bf(lo) | ((uint32_t)f2bf(hi) << 16);
+  typedef float f32x2_ __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2_ __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_{lo, hi}), bf16x2_));
 }
 
 // 8 bf16 (one 16-B word) -> fp32

@@ -17,8 +17,8 @@
 // The tile's epilogue was 20 k of 170 k cycles at K = 4096 (bounds by branches, 8-byte stores, a division a
 // SiLU, and a wait for all of its stores): now stores of 16 bytes a lane through range-checked descriptors that
 // nothing waits for until the tile's second K-tile. Both against a schedule of reads and pieces in bursts and
-// the former epilogue, us: 16384 x 6144 x 4096 557 -> 535 (1.54 PFLOP/s), 8192 x 4096 x 4096 182 -> 176 and x 14336
-// 645 -> 626, 8192 x 28672 x 4096 with SiLU pairs 1271 -> 1230. With fp32 outputs 188 -> 186: all CUs store 67 MB at
+// the former epilogue, us: 16384 x 6144 x 4096 557 -> 530 (1.55 PFLOP/s), 8192 x 4096 x 4096 182 -> 175 and x 14336
+// 645 -> 625, 8192 x 28672 x 4096 with SiLU pairs 1271 -> 1217. With fp32 outputs 188 -> 185: all CUs store 67 MB at
 // once, at 6.4 TB/s, behind which the next tile's pieces wait.
 #pragma once
 #include "gemm_common.h"
@@ -39,6 +39,13 @@ template <int N, class F> __device__ __forceinline__ void unroll(F f) {
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* p, int bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
+}
+// silu(g) u, or gelu(g) u by its tanh form, with v_rcp_f32 (1 ulp) for the division's ten instructions: 128 of them a
+// lane are 5 k cycles of a tile. The rounding to bf16 behind it is 2^15 times coarser; the outputs' error against
+// 64 bits is 1.657e-3 (SiLU, 8192 x 28672 x 4096) and 1.658e-3 (GELU) with either
+template <int EPI> __device__ __forceinline__ float pair_rcp(float g, float u) {
+  const float e = EPI == EPI_GELU_MUL ? 1.5957691216057308f * (g + 0.044715f * g * g * g) : g;
+  return g * __builtin_amdgcn_rcpf(1.f + __expf(-e)) * u;
 }
 // 1 KiB of LDS-DMA (16 B a lane); IMM moves both the address in memory and the one in LDS
 template <int IMM>
@@ -212,9 +219,9 @@ __global__ void __launch_bounds__(256, 1) gemm4w_kernel(
     asm volatile("" ::: "memory");
   };
 
-  // one K-tile. MORE: another of the same tile follows. landed: it is in LDS already
-  auto ktile = [&](auto MORE, bool landed) __attribute__((always_inline)) {
-    constexpr bool more = decltype(MORE)::value;
+  // one K-tile. FIRST: its sums begin at zero; MORE: another of the same tile follows, in LDS already where landed
+  auto ktile = [&](auto FIRST, auto MORE, bool landed) __attribute__((always_inline)) {
+    constexpr bool first = decltype(FIRST)::value, more = decltype(MORE)::value;
     auto after = [&](auto QC) __attribute__((always_inline)) {
       constexpr int q = decltype(QC)::value;
       if constexpr (q < NF) {
@@ -249,8 +256,12 @@ __global__ void __launch_bounds__(256, 1) gemm4w_kernel(
     // read only as the next MFMA's C until the pad behind the loop
     unroll<8 * NJ>([&](auto U) __attribute__((always_inline)) {
       constexpr int u = decltype(U)::value;
-      asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
-                   : "+a"(acc[u / NJ][u % NJ]) : "v"(b0[u % NJ]), "v"(a0[u / NJ]));
+      if constexpr (first)
+        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0"
+                     : "=a"(acc[u / NJ][u % NJ]) : "v"(b0[u % NJ]), "v"(a0[u / NJ]));
+      else
+        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
+                     : "+a"(acc[u / NJ][u % NJ]) : "v"(b0[u % NJ]), "v"(a0[u / NJ]));
       after(U);
     });
     unroll<8 * NJ>([&](auto U) __attribute__((always_inline)) {
@@ -344,7 +355,7 @@ __global__ void __launch_bounds__(256, 1) gemm4w_kernel(
           const f32x4 g = vget(acc[i][2 * j]), u = vget(acc[i][2 * j + 1]);
           float o[4];
 #pragma unroll
-          for (int r = 0; r < 4; ++r) o[r] = pair_f<EPI>(g[r], u[r], 0.f);
+          for (int r = 0; r < 4; ++r) o[r] = pair_rcp<EPI>(g[r], u[r]);
           return uint2{pack2bf(o[0], o[1]), pack2bf(o[2], o[3])};
         } else if constexpr (EPI == EPI_SLAB16) {
           const f32x4 v = vget(acc[i][j]);
@@ -460,29 +471,31 @@ __global__ void __launch_bounds__(256, 1) gemm4w_kernel(
     const bool has_next = vn < total;
     Tile tn = t;
     if (has_next) tn = locate(vn);
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // the zeroed accumulators are read by inline-asm MFMAs, which hipcc pads no hazard for: pin every write
-    // ahead of a few wait states
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) asm volatile("" : "+a"(acc[i][j]));
-      asm volatile("s_nop 3");
-    }
     unroll<NF>([&](auto F) __attribute__((always_inline)) { read(F, a0, b0, ra0, rw0); });
-    // (K-tile 1 is there, and the last tile's stores need not have left: nothing to wait for in K-tile 0)
-    if (nk > 2) ktile(T_{}, true);
-    for (int kt = 1; kt + 2 < nk; ++kt) ktile(T_{}, false);
-    // the last two K-tiles stage the next tile's first two. Without a next tile they stage through an empty
-    // range (no memory traffic, zeros): one code path, since a branch doubles the unrolled tail and hipcc
-    // spills the fragments
+    if (nk > 2) {
+      // (K-tile 1 is there, and the last tile's stores need not have left: nothing to wait for in K-tile 0)
+      ktile(T_{}, T_{}, true);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      // these are read by inline-asm MFMAs, which hipcc pads no hazard for: every write ahead of wait states
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) asm volatile("" : "+a"(acc[i][j]));
+        asm volatile("s_nop 3");
+      }
+    }
+    for (int kt = 1; kt + 2 < nk; ++kt) ktile(F_{}, T_{}, false);
+    // the last two K-tiles stage the next tile's first two. Without a next tile they stage through an
+    // empty range (no memory traffic, zeros): one code path, since a branch doubles the unrolled tail and hipcc
+    // spills the fragments or moves the descriptors into VGPRs
     begin_stage(tn, has_next);
-    ktile(T_{}, nk <= 2);
+    ktile(F_{}, T_{}, nk <= 2);
     if (nk < 2) sab = swb = 0;
-    ktile(F_{}, false);
+    ktile(F_{}, F_{}, false);
     // MFMA results -> the epilogue's copies: the XDL write-back's wait states, tied to the last row of
     // accumulators written so that no copy of them moves above the pad
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");

@@ -33,14 +33,14 @@ constexpr bool epi_pairs(int epi) {
 typedef __attribute__((address_space(3))) void lds_void;
 typedef const __attribute__((address_space(1))) void gbl_void;
 
-__device__ __forceinline__ float silu_f(float x) { return x * __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
+__device__ __forceinline__ float silu_f(float x) { return x / (1.f + __expf(-x)); }
 // tanh-approximate GELU, branch-free: 0.5 (1 + tanh(y)) = sigmoid(2 y). tanhf's range
 // branches made a 256-accumulator epilogue too large to unroll, and the rolled loop indexed
 // the accumulators dynamically: hipcc demoted them to scratch and copied them out of the
 // AGPRs inside the K loop, where no hazard padding follows an inline-asm MFMA
 __device__ __forceinline__ float gelu_f(float x) {
   const float y2 = 1.5957691216057308f * (x + 0.044715f * x * x * x);
-  return x * __builtin_amdgcn_rcpf(1.f + __expf(-y2));
+  return x / (1.f + __expf(-y2));
 }
 
 // exact GELU x * Phi(x), branch-free (see gelu_f on why): Phi(-|x|) = erfc(|x| / sqrt 2) / 2

@@ -233,6 +233,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))
 // shortest max_seqlen that takes the 256-row kernel; below, the 64-row kernel wastes fewer
 // idle waves (settable for A/B runs and tests: dli_prefill_set_min_len)
 static int g_pl_min_len = 256;
+// shortest max_seqlen that takes waves of 64 rows (attention_prefill_long.hip; settable too:
+// dli_prefill_set_wave64_len), in launches of more than a round of workgroups: 2500 tokens 76 -> 69 us, 8 x 2000
+// 331 -> 319, 4 x 2048 162 -> 159, but 8 of 300 to 2000 174 -> 178, 16 x 1000 equal, and one round, where blocks
+// are paired, 2048 51 -> 58
+static int g_pw_min_len = 2048;
 static int g_pf_pack = 1;                          // head packing for short prompts (A/B)
 
 // Tile image: 8-row x 32-column subtiles of 512 B (cdna_hip_programming.md §5.5 T10, image
@@ -483,6 +488,11 @@ __global__ void __launch_bounds__(512) prefill_attn32_kernel(
   }
 }
 
+// attention_prefill_long.hip; ctx_lens null: keys and values in the activation's rows
+int launch_prefill_long(void* out, int out_stride, const void* qkv, int row_stride, const int* cu_seqlens, int num_seqs,
+                        int max_seqlen, int hq, int hkv, float scale_log2, const int* ctx_lens, const void* k_cache,
+                        const void* v_cache, const int* block_tables, int bt_stride, int block_size, hipStream_t st);
+
 template <bool PAGED>
 static int launch_prefill(void* out, int out_stride, const void* qkv, int row_stride,
                           const int* cu_seqlens, int num_seqs, int max_seqlen, int hq, int hkv,
@@ -492,6 +502,13 @@ static int launch_prefill(void* out, int out_stride, const void* qkv, int row_st
   if (num_seqs <= 0 || max_seqlen <= 0) return 0;
   if (hq % hkv || (hd != 64 && hd != 128)) return (int)hipErrorInvalidValue;
   const float sl2 = scale * 1.4426950408889634f;
+  // (rows at 32-bit offsets from their sequence's first, and cached blocks that hold whole rows of a piece)
+  if (hd == 128 && max_seqlen >= max(g_pw_min_len, g_pl_min_len) &&
+      (long)((max_seqlen + PL_ROWS - 1) / PL_ROWS) * hq * num_seqs > 256 &&
+      (PAGED ? block_size >= 16 && (block_size & (block_size - 1)) == 0
+             : ((long)max_seqlen + 256) * row_stride * 2 < (1L << 31)))
+    return launch_prefill_long(out, out_stride, qkv, row_stride, cu_seqlens, num_seqs, max_seqlen, hq, hkv, sl2,
+                               PAGED ? ctx_lens : nullptr, k_cache, v_cache, block_tables, bt_stride, block_size, st);
   if (hd == 128 && max_seqlen >= g_pl_min_len) {     // long sequences: 256-row workgroups
     const int blocks = (max_seqlen + PL_ROWS - 1) / PL_ROWS;
     const dim3 grid32 = hq <= 4 ? dim3(blocks, num_seqs, hq) : dim3(blocks * hq, num_seqs);
@@ -553,5 +570,11 @@ extern "C" int dli_prefill_set_pack(int on) {
 extern "C" int dli_prefill_set_min_len(int n) {
   const int old = g_pl_min_len;
   if (n > 0) g_pl_min_len = n;
+  return old;
+}
+
+extern "C" int dli_prefill_set_wave64_len(int n) {
+  const int old = g_pw_min_len;
+  if (n > 0) g_pw_min_len = n;
   return old;
 }

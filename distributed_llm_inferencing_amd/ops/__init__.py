@@ -535,6 +535,12 @@ def prefill_long_min_len(n: int = 0) -> int:
     return int(N.require_native().dli_prefill_set_min_len(int(n)))
 
 
+def prefill_wave64_min_len(n: int = 0) -> int:
+    """Shortest max_seqlen whose launches of more than 256 workgroups of 256 rows take the kernel with 64 rows a
+    wave; n > 0 sets it. Returns the previous value (A/B runs and tests)."""
+    return int(N.require_native().dli_prefill_set_wave64_len(int(n)))
+
+
 def prefill_set_pack(on: bool) -> bool:
     """Head packing of the short-prompt prefill attention kernel (2 / 4 query heads of a GQA
     group per workgroup when every prompt of the batch is <= 32 / 16 tokens); returns the

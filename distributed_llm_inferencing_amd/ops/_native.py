@@ -43,6 +43,7 @@ _SIGS = {
     "dli_decode_attention_workspace_bytes": [I, I, I, I],
     "dli_prefill_attention": [P, I, P, I, P, I, I, I, I, I, F, P],
     "dli_prefill_set_min_len": [I],
+    "dli_prefill_set_wave64_len": [I],
     "dli_prefill_set_pack": [I],
     "dli_sample_set_split_max_b": [I],
     "dli_decode_set_form": [I],

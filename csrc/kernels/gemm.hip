@@ -19,7 +19,7 @@
 //    weights W + g*N*ldw. Rows past the group end are skipped. Split-K composes with it
 //    (slab rows are the permuted rows), for long-K expert GEMMs with few row tiles.
 // Epilogues: 0 bf16 store, 1 fp32 store (logits), 2 SiLU(gate)*up over the 16-row-interleaved
-// gate/up weight (output width N/2), 3 bias + tanh-GELU, 4 bias.
+// gate/up weight (output width N/2), 3 bias + tanh-GELU, 4 bias, 16 C += (4-wave tiles).
 //
 // Files: gemm_common.h (shared epilogue / split-K pieces), gemm_tiles.hip (ids 0-21, 23-25),
 // gemm_stream.hip (60-72: few rows, weights streamed), gemm4w.h +

@@ -338,6 +338,54 @@ __global__ void __launch_bounds__(256, 1) gemm4w_kernel(
     const auto rc = make_rsrc(base, left * ld * 2);
     const int c0 = 16 * NO * wn + 16 * (fq & 1) + 8 * (fq >> 1), c1 = 16 * NO * wn + 16 * (NO - 1) + 4 * fq;
     const int ro = (128 * wm + fr) * ld * 2;
+    // What the tile is added to is requested all at once, into the fragments' registers: 128 KB a CU at the
+    // memory's rate, 3 to 7 us a round of tiles (three row blocks' requests ahead of the last K-tile changed nothing). The
+    // add behind it read and wrote twice that: ops._add_product has the times
+    if constexpr (EPI == EPI_RES) {
+      u32x4 old[8][NO / 2];
+      u32x2 odd[8];
+      auto fetch = [&](auto I) __attribute__((always_inline)) {
+        constexpr int i = decltype(I)::value;
+        unroll<NO / 2>([&](auto J) __attribute__((always_inline)) {
+          constexpr int j = 2 * decltype(J)::value;
+          old[i][j / 2] = __builtin_amdgcn_raw_buffer_load_b128(
+              rc, c0 + 16 * j < cols ? ro + 2 * c0 + 32 * j : OUT_OF_RANGE, i * 16 * ld * 2, 0);
+        });
+        if constexpr (NO & 1)
+          odd[i] = __builtin_amdgcn_raw_buffer_load_b64(rc, c1 < cols ? ro + 2 * c1 : OUT_OF_RANGE,
+                                                            i * 16 * ld * 2, 0);
+      };
+      auto sum = [](uint32_t c, float lo, float hi) __attribute__((always_inline)) -> uint32_t {
+        return pack2bf(__uint_as_float(c << 16) + lo, __uint_as_float(c & 0xffff0000u) + hi);
+      };
+      unroll<8>(fetch);
+      asm volatile("" ::: "memory");
+      unroll<8>([&](auto I) __attribute__((always_inline)) {
+        constexpr int i = decltype(I)::value;
+        unroll<NO / 2>([&](auto J) __attribute__((always_inline)) {
+          constexpr int j = 2 * decltype(J)::value;
+          const f32x4 x = vget(acc[i][j]), y = vget(acc[i][j + 1]);
+          float f[8];
+          unroll<4>([&](auto R) __attribute__((always_inline)) {
+            constexpr int k = decltype(R)::value;
+            const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(x[k]), __float_as_uint(y[k]), false, false);
+            f[k] = __uint_as_float(p[0]);
+            f[4 + k] = __uint_as_float(p[1]);
+          });
+          const u32x4 c = old[i][j / 2];
+          __builtin_amdgcn_raw_buffer_store_b128(
+              u32x4{sum(c[0], f[0], f[1]), sum(c[1], f[2], f[3]), sum(c[2], f[4], f[5]), sum(c[3], f[6], f[7])}, rc,
+              c0 + 16 * j < cols ? ro + 2 * c0 + 32 * j : OUT_OF_RANGE, i * 16 * ld * 2, 0);
+        });
+        if constexpr (NO & 1) {
+          const f32x4 x = vget(acc[i][NO - 1]);
+          const u32x2 c = odd[i];
+          __builtin_amdgcn_raw_buffer_store_b64(u32x2{sum(c[0], x[0], x[1]), sum(c[1], x[2], x[3])}, rc,
+                                                c1 < cols ? ro + 2 * c1 : OUT_OF_RANGE, i * 16 * ld * 2, 0);
+        }
+      });
+      return;
+    }
     uint2 bq[NJ];
     if constexpr (EPI == EPI_BIAS || EPI == EPI_BIAS_GELU) {
       const auto rb = make_rsrc(bias, N * 2);
@@ -430,11 +478,11 @@ __global__ void __launch_bounds__(256, 1) gemm4w_kernel(
   // stores issued behind the next tile's pieces, which may fly while those are waited for (6 bits count)
   constexpr int N32 = 8 * NJ, N16 = 8 * (((PAIRS ? NJ / 2 : NJ) + 1) / 2);
   auto epilogue = [&](const Tile& t) __attribute__((always_inline)) {
-    if (!ranged) {
+    if (EPI != EPI_RES && !ranged) {
       store_any(t);
       asm volatile("" ::: "memory");
       wait_vmcnt<0>();
-    } else if (EPI == EPI_F32 || (EPI != EPI_SLAB16 && slab)) {
+    } else if (EPI == EPI_F32 || (EPI != EPI_SLAB16 && EPI != EPI_RES && slab)) {
       char* base = slab ? (char*)(ws + ((long)t.ks * M + t.row0 + t.m0) * N + t.n0)
                         : (char*)((float*)C + (long)(t.row0 + t.m0) * ldc + t.n0);
       store32(t, base, EPI == EPI_F32 && !slab ? (uint32_t*)const_cast<u16*>(bias) : nullptr);
@@ -527,6 +575,9 @@ static int launch_4w(const void* A, int lda, const void* W, int ldw, void* C, in
                      hipStream_t st) {
   if (epi_pairs(EPI) && N % 32) return (int)hipErrorInvalidValue;
   if (K % (splits * BK)) return (int)hipErrorInvalidValue;
+  if (EPI == EPI_RES && (splits != 1 || group_off != nullptr || ((N | ldc) & 7) || ((uintptr_t)C & 15) || C == nullptr ||
+                         ldc >= (1 << 21) - 1024))
+    return (int)hipErrorInvalidValue;
   constexpr size_t lds = 0x10000 + (size_t)(256 + 32 * NJ) * BK * 2;
   static bool raised = false;
   if (!raised) {

@@ -47,6 +47,7 @@ static int launch8(int epi, DLI_GEMM_ARGS) {
     case EPI_BIAS: return launch_4w<EPI_BIAS, 8>(DLI_GEMM_PASS);
     case EPI_BIAS_GELU: return launch_4w<EPI_BIAS_GELU, 8>(DLI_GEMM_PASS);
     case EPI_SLAB16: return launch_4w<EPI_SLAB16, 8>(DLI_GEMM_PASS);
+    case EPI_RES: return launch_4w<EPI_RES, 8>(DLI_GEMM_PASS);
     default: return DLI_NOT_MINE;
   }
 }

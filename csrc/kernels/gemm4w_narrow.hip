@@ -6,6 +6,7 @@ template <int NJ> static int launch_nj(int epi, DLI_GEMM_ARGS) {
     case EPI_BF16: return launch_4w<EPI_BF16, NJ>(DLI_GEMM_PASS);
     case EPI_F32: return launch_4w<EPI_F32, NJ>(DLI_GEMM_PASS);
     case EPI_SLAB16: return launch_4w<EPI_SLAB16, NJ>(DLI_GEMM_PASS);
+    case EPI_RES: return launch_4w<EPI_RES, NJ>(DLI_GEMM_PASS);
     default: break;
   }
   if constexpr (NJ % 2 == 0) {                     // a gate block and its up block in one wave tile

@@ -24,7 +24,9 @@ enum { EPI_BF16 = 0, EPI_F32 = 1, EPI_SILU = 2, EPI_BIAS_GELU = 3, EPI_BIAS = 4,
        // relu(gate) * up over the interleaved gate/up weight
        EPI_RELU = 8,
        // tanh-approximate gelu(gate) * up over the interleaved gate/up weight
-       EPI_GELU_MUL = 9 };
+       EPI_GELU_MUL = 9,
+       // C += the product (unsplit, dense): the 4-wave kernel where rows are aligned, rounding once, and gemv.hip
+       EPI_RES = 16 };
 // epilogues that pair a gate block with the up block beside it (output width N / 2)
 constexpr bool epi_pairs(int epi) {
   return epi == EPI_SILU || epi == EPI_CLAMP || epi == EPI_RELU || epi == EPI_GELU_MUL;

@@ -154,10 +154,9 @@ __device__ __forceinline__ void gemv_core(const u16* __restrict__ A, int lda,
     }
 }
 
-// gemv-only epilogue: C is the residual, residual[m, n] = bf16(residual + bf16(acc)) (the
+// EPI_RES here: C is the residual, residual[m, n] = bf16(residual + bf16(acc)) (the
 // rounding of splitk_add_rmsnorm: the GEMM result is rounded before the add). Full K per
 // workgroup (splits 1): every output element has one writer and no slab round trip.
-constexpr int EPI_RES = 16;
 
 // The deferred RMSNorm of the consuming GEMV (PRO): x[m] = bf16(A[m] * rstd_m * nw) for the
 // MB input rows into LDS (xs: [MB][K] bf16), one block reduction per row. issue(): every row

@@ -308,6 +308,28 @@ def _splitk_plan(x, w):
     return p if p.splits > 1 else None
 
 
+def _add_product(x, w, residual, plan: Optional[G.GemmPlan]) -> bool:
+    """residual += x @ w.T inside the GEMM, rounded once, where the unsplit plan's kernel has that epilogue and the
+    rows are whole, aligned and many; whether it did. The product neither travels as bf16 to the add nor is read
+    again there. 4096 columns, us with the norm behind it, apart / so: K = 4096, 16384 rows 458 / 433, 7993 223 / 207,
+    2112 73 / 71; K = 14336 1350 / 1326, 676 / 660, 204 / 200. Few rows take split plans and their fused reduce."""
+    if not (_use_native(x) and x.dtype == w.dtype == residual.dtype == torch.bfloat16 and w.dim() == 2):
+        return False
+    (M, K), Nn = x.shape, w.shape[0]
+    if (M < G.LARGE_M or w.shape[1] != K or residual.shape != (M, Nn) or not residual.is_contiguous() or Nn % 8
+            or residual.data_ptr() % 16 or x.stride(-1) != 1 or w.stride(-1) != 1):
+        return False
+    cut = G.row_cut(M, Nn, K) if plan is None else 0
+    rows = cut or M
+    p = plan or G.plan(rows, Nn, K, "none")
+    if p.splits != 1 or p.tile not in G.RES_ADD_TILES or rows < G.LARGE_M:
+        return False
+    _gemm_native(x[:rows], w, "res_add", out=residual[:rows], plan=p)
+    if cut:
+        residual[cut:].add_(linear(x[cut:], w))
+    return True
+
+
 def linear_add_rmsnorm(x, w, residual, norm_w, eps, plan: Optional[G.GemmPlan] = None,
                        route=None):
     """residual += x @ w.T (bf16-rounded, in place); returns rmsnorm(residual) * norm_w
@@ -346,6 +368,8 @@ def linear_add_rmsnorm(x, w, residual, norm_w, eps, plan: Optional[G.GemmPlan] =
     else:
         p = plan if plan.splits > 1 else None
     if p is None:
+        if _add_product(x, w, residual, plan):
+            return None if norm_w is None else rmsnorm(residual, norm_w, eps)
         y = linear(x, w) if plan is None else _gemm_native(x, w, "none", plan=plan)
         if norm_w is None:
             residual.add_(y)             # bf16 add computes in fp32 and rounds once

@@ -120,7 +120,9 @@ def tile_ok(tile: int, epi: str) -> bool:
 # "splitk": a plain GEMM whose fp32 partial slabs feed a fused reduce (ops.linear_add_rmsnorm,
 # ops.linear_rope_cache); planned/tuned separately (a non-split winner runs unfused).
 EPI = {"none": 0, "f32": 1, "silu_mul": 2, "bias_gelu": 3, "bias": 4, "splitk": 0,
-       "slab16": 5, "gelu_erf": 6, "clamp_mul": 7, "relu_mul": 8, "gelu_mul": 9}
+       "slab16": 5, "gelu_erf": 6, "clamp_mul": 7, "relu_mul": 8, "gelu_mul": 9, "res_add": 16}
+# the 4-wave kernel's tiles, whose unsplit product can add into its output (EPI "res_add")
+RES_ADD_TILES = frozenset((22, 28, 34, 41, 45, 55))
 # epilogues over the interleaved gate/up weight: the output is half as wide
 PAIR_EPIS = ("silu_mul", "clamp_mul", "relu_mul", "gelu_mul")
 # tiles whose slab-only split-K call can store fp16 partials (EPI "slab16": the generic tile

@@ -34,7 +34,7 @@ extern "C" int dli_gemm_set_slab_store(int mode) {
 }
 
 // one family's split-K slab store (0 plain, 1 nt, 2 sc1, 3 sc0 sc1): family 0 = the generic
-// tiles (decode O / QKV), 1 = the 8-phase kernels (decode down)
+// tiles (decode O / QKV), 1 = the 8-phase kernels
 extern "C" int dli_gemm_set_slab_store_family(int family, int mode) {
   switch (family) {
     case 0: gemm_stream_set_slab_store(mode); return gemm_tiles_set_slab_store(mode);

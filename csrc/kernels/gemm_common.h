@@ -14,7 +14,7 @@
 enum { EPI_BF16 = 0, EPI_F32 = 1, EPI_SILU = 2, EPI_BIAS_GELU = 3, EPI_BIAS = 4,
        // slab-only split-K call (C == nullptr, splits > 1) whose partials are stored as fp16
        // scaled by 1/16 instead of fp32 (half the bytes the GEMM writes and its consumer
-       // reads; the scale keeps |partial| up to ~1e6 in range). Tiles and 8-phase families.
+       // reads; the scale keeps |partial| up to ~1e6 in range). Tiles, 8-phase and 4-wave families.
        EPI_SLAB16 = 5,
        // the exact (erf) GELU of the product, no bias (ungated expert feed-forwards)
        EPI_GELU_ERF = 6,
@@ -347,7 +347,7 @@ int gemm_stream_set_slab_store(int mode);
 int gemm_8p_set_slab_store(int mode);
 
 // EPI -> template argument, for a family's dispatch<EPI>(tile_cfg, ...); the families with
-// an fp16 slab store (tiles, 8-phase) take DLI_EPI_SWITCH_S16
+// an fp16 slab store (tiles, streaming, 8-phase) take DLI_EPI_SWITCH_S16
 #define DLI_EPI_SWITCH_S16(FN)                                                     \
   if (epi == EPI_CLAMP) return FN<EPI_CLAMP>(tile_cfg, DLI_GEMM_PASS);             \
   if (epi == EPI_RELU) return FN<EPI_RELU>(tile_cfg, DLI_GEMM_PASS);               \

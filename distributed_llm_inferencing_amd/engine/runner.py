@@ -270,7 +270,7 @@ class StageRunner:
 
     def autotune_prefill(self, max_tokens: int) -> None:
         """GEMM plans of prefill steps, one per power-of-two token bucket from 2048 up to the
-        bucket of ``max_tokens``: our 8-phase kernel against our 4-wave kernel, the faster pinned
+        bucket of ``max_tokens``: the 4-wave kernel's tiles of several widths, the fastest pinned
         (``ops.gemm.prefill_candidates``). Skipped like the decode autotune
         (DLI_GEMM_AUTOTUNE=0, non-GPU) and by DLI_TUNE_PREFILL=0."""
         if (os.environ.get("DLI_GEMM_AUTOTUNE", "1") != "1" or self.device.type != "cuda"

@@ -8,9 +8,8 @@ The projection GEMMs of a decode step are skinny (M = batch) and of a prefill st
   GEMM at M = 256': choose SPLITK so that tiles * SPLITK ~ 0.5-1x the CU count),
 * every GEMM runs on our kernels (no vendor-library backend): decode GEMMs (the hipGraph
   steps) on tiles autotuned at graph capture (on by default; ``DLI_GEMM_AUTOTUNE=0``
-  disables it); prefill GEMMs on our 8-phase 256x256 kernel or the one-wave-per-SIMD 256x256
-  kernel (tile 45), whichever the warmup measures faster per token bucket
-  (``prefill_candidates``).
+  disables it); prefill GEMMs on the one-wave-per-SIMD kernel (gemm4w.h), whose tile and width the
+  warmup measures per token bucket (``prefill_candidates``).
 
 Split-K partial slabs live in a grow-only per-device workspace; engines warm every shape
 up before hipGraph capture so no allocation happens inside a capture.
@@ -36,15 +35,15 @@ TILES = {0: (64, 64), 1: (64, 128), 2: (128, 128), 3: (128, 256), 4: (256, 128),
          13: (256, 256), 14: (256, 128), 15: (128, 256), 16: (256, 128), 17: (128, 256),
          # grid-filling tiles for N = 6144 / 4096 at M = 512
          18: (128, 96), 19: (128, 96), 20: (128, 64), 21: (128, 64),
-         # 256x256 8-phase ping-pong (two wave groups alternate MFMA / load segments)
+         # 4 waves, one per SIMD (gemm4w.h): 256 columns, or fewer where they leave less of a round of CUs
+         # empty (dense, not biased); the rarer epilogues on the 8-phase ping-pong kernel (gemm8p.hip)
          22: (256, 256),
          # 192-wide, 8 waves: N = 6144 is 32 column tiles (fused QKV at M = 512 fills the chip
          # with split-K 2 / 4)
          23: (128, 192), 24: (128, 192), 25: (256, 192),
          # 256x224 ping-pong: N = 28672 (Llama-3 gate/up) at M = 512 = 256 tiles on 256 CUs
          26: (256, 224),
-         # 256x128 ping-pong: Mixtral grouped down (N = 4096: 32 column tiles per expert),
-         # N = 4096 at M = 512 with split-K 4
+         # 256x128 of the same kernels: N = 4096 at M = 512 with split-K 4
          28: (256, 128),
          # 256x256, 4 waves (one per SIMD), 128x128 wave tiles, accumulators pinned in the AGPR
          # file, at most a workgroup a CU that walks its tiles (gemm4w.h)
@@ -59,13 +58,12 @@ STREAM_TILES = {60: (32, 32, 256), 61: (32, 128, 64), 62: (32, 64, 256), 63: (64
                 68: (128, 256, 64), 69: (64, 32, 256), 70: (96, 64, 64), 71: (128, 64, 64),
                 72: (128, 32, 128)}
 STREAM_MAX_M = 128
-# the 4-wave plan raced against the 8-phase one in the prefill autotune
+# the plan of 256 columns throughout, raced against tile 22's width by rounds in the prefill autotune
 PREFILL_4W_TILE = 45
 # the persistent 4-wave tile (55) raced too
 PREFILL_PERSIST = True
-# prefill-sized grouped expert GEMMs (ops.moe_mlp's eager path): Mixtral 8x7B at 32k routed
-# rows, tile 45 vs the 8-phase tile 22: down 2,895 vs 3,071-3,239 us, gate/up 5,736 vs
-# 5,898 us (profiles/r4/moe/)
+# prefill-sized grouped expert GEMMs (ops.moe_mlp's eager path): the 4-wave kernel on 256 columns, which
+# tile 22 takes too where a product is grouped
 MOE_PREFILL_TILE = 45
 # weight-streaming skinny GEMM (gemm.hip gemv_kernel) for M <= GEMV_MAX_M rows: 16 / 32 output
 # rows per workgroup (31 for the SiLU*up gate/up pairing); not an MFMA tile, so kept apart
@@ -125,9 +123,8 @@ EPI = {"none": 0, "f32": 1, "silu_mul": 2, "bias_gelu": 3, "bias": 4, "splitk": 
 RES_ADD_TILES = frozenset((22, 28, 34, 41, 45, 55))
 # epilogues over the interleaved gate/up weight: the output is half as wide
 PAIR_EPIS = ("silu_mul", "clamp_mul", "relu_mul", "gelu_mul")
-# tiles whose slab-only split-K call can store fp16 partials (EPI "slab16": the generic tile
-# family and the 8-phase kernels); the fused consumers then read half the bytes. The
-# weight-streaming GEMVs and the 4-wave family keep fp32 slabs.
+# tiles whose slab-only split-K call can store fp16 partials (EPI "slab16"); the fused consumers then
+# read half the bytes. The weight-streaming GEMVs and tiles 34, 41, 45 and 55 keep fp32 slabs.
 SLAB16_TILES = frozenset(list(range(0, 22)) + [22, 23, 24, 25, 26, 28] + list(STREAM_TILES))
 SLAB16 = os.environ.get("DLI_SLAB_FP32", "0") != "1"      # A/B: fp32 partials everywhere
 # tiles whose grouped SiLU*up GEMM can read its rows through a permutation (the generic
@@ -231,10 +228,10 @@ def _stream_plan(M: int, N: int, K: int, epi: str):
 def _heuristic(M: int, N: int, K: int, epi: str) -> GemmPlan:
     """Fitted to profiles/r1_gemm/gemm_bench.json and profiles/r1_gemm8p/ (MI355X, random
     bf16 operands): skinny decode GEMMs (M <= 512) on the 2/3-stage tiles below (autotuned
-    at capture); fat prefill GEMMs (M >= LARGE_M) on the 256x256 kernels, the 8-phase ping-pong one
-    (tile 22) or the persistent 4-wave one (tile 55), with their fused epilogues (SiLU*up, bias+GELU,
-    fp32); the prefill autotune (``prefill_candidates``) measures them per bucket."""
-    # M > 512: mixed prefill+decode steps of a full batch and prefill — 256x256 8-phase
+    at capture); fat prefill GEMMs (M >= LARGE_M) on 256-row tiles of the 4-wave kernel (22, 28, 55), with
+    their fused epilogues (SiLU*up, bias+GELU, fp32); the prefill autotune (``prefill_candidates``) measures
+    them per bucket."""
+    # M > 512: mixed prefill+decode steps of a full batch and prefill — 256-row
     # tiles (the 128-row tiles below ran a 512 + 300-token mixed step's GEMMs ~2.5x slower
     # than the tuned decode step: 26.7 ms per mixed step end to end, profiles/r3/e2e/)
     if M >= LARGE_M or M > 512:
@@ -253,22 +250,17 @@ def _heuristic(M: int, N: int, K: int, epi: str) -> GemmPlan:
             while (tiles * splits * 2 <= NUM_CUS and K % (64 * splits * 2) == 0
                    and K // (splits * 2) >= 1024 and splits < 4):
                 splits *= 2
-        # the persistent kernel hides a tile's prologue and epilogue, which counts for short K: 8192
-        # rows, K = 4096: N = 4096 / 6144 / 12288 / 28672 in 185 / 274 / 556 / 1284 us against 192 / 288 /
-        # 582 / 1337; at K = 14336 it is 5 % ahead for 1536 to 3000 rows (251 against 267) and 4 % behind
-        # from 4096 on (643 against 619 at 8192). 16384 rows: 2538 against 2672 at N = 28672, within 2 %
-        # at 6144. Its biased epilogues are slower, GELU's most (4096 x 3072, K = 768: 48 us against 33,
-        # bias alone 38 and 33; 8192 x 12288, K = 4096 684 and 637), and a pairing one pays where tiles
-        # follow each other or K is long (1024 x 8192, K = 1024, one round of 128 tiles: 27.2 against 26.3,
-        # 8192 x 8192 114 against 116; 4096 x 8192, K = 512 38.0 against 37.1). fp32 outputs of 0.8 GB and
-        # more over K <= 1024, bound by their stores, follow the order of the tiles: 0.87 to 1.17 times
-        # tile 22's time from size to size, by no line
+        # 55 and 22 run one kernel, 55 on 256, 192 or 160 columns, 22 on 224 and 128 too, with any K, with splits
+        # and, where biased, on 256. So they are equal where both choose 256 (8192 rows, K = 4096, us: N = 4096 185,
+        # 6144 275, 28672 1253), and 22 is ahead where 128 or 224 columns fill a round (1536 x 4096, K = 4096 48
+        # against 51, 1024 x 8192 pairs, K = 1024 19.9 against 20.7), 55 by the last per cents where 22 takes 224
+        # (4352 x 4096, K = 14336 380 against 391). The lines below are from kernels that differed more and cost
+        # at most that
         if epi in PAIR_EPIS:
             pays = K > 2048 or (K >= 1024 and tiles > NUM_CUS) or N % 64 != 0   # (tile 22 takes no such N)
         else:
             pays = epi not in ("bias", "bias_gelu")
-        # (long K from 4096 rows on where its narrower tiles save part of a round: 4352 x 4096, K = 14336,
-        # bf16 outputs 412 us against 551, fp32 489 against 577)
+        # (long K from 4096 rows on where its narrower tiles save part of a round: as above)
         if (pays and splits == 1 and M >= LARGE_M and K % 128 == 0
                 and (K <= 8192 or M < 4096 or persistent_width(M, N, epi in PAIR_EPIS, device_cus()) < 256)
                 and (M < 16384 or N >= 16384) and tile_ok(55, epi)):
@@ -674,13 +666,13 @@ _GRAPH_TUNE = True
 
 
 def prefill_candidates(M: int, N: int, K: int, epi: str):
-    """Prefill-sized GEMMs (M > 1024 rows): our 8-phase 256x256 kernel with the heuristic's
-    split count against our one-wave-per-SIMD 256x256 kernel (PREFILL_4W_TILE, the
-    two-barrier schedule) at the same split, 1-4 % apart on the square / QKV / gate-up /
-    down prefill shapes (profiles/r4/gemm4w/), measured per shape and bucket. At these sizes
+    """Prefill-sized GEMMs (M > 1024 rows): the one-wave-per-SIMD kernel on tile 22's width with the
+    heuristic's split count, on 256 columns (PREFILL_4W_TILE) at the same split and, unsplit, on tile 55's
+    width, measured per shape and bucket (a bucket's rows leave a part of a round empty that a step's own
+    need not). At these sizes
     the GEMM is MFMA-bound, so the autotuner times them warm (``cold_bytes`` 1)."""
     base = _heuristic(M, N, K, epi)
-    if base.tile == 55:                  # (its 8-phase and 4-wave counterparts)
+    if base.tile == 55:                  # (its counterparts of other widths)
         base = GemmPlan("dli", 22, 1)
     out = [base]
     if base.tile == 22 and PREFILL_4W_TILE > 0:
@@ -699,15 +691,8 @@ def candidate_plans(M: int, N: int, K: int, epi: str):
     # Default: 26 (256x224). It fills all 256 CUs on the gate/up GEMM and wins the isolated
     # autotune (98.8 vs ~106 us), but in the decode step it ran 97.9 vs 99.0 us per call and
     # the bench 0.3-0.7 % lower in three same-box A/B runs (profiles/r2_s2/README.md)
-    # 45 stays
-    # prefill-only too (no gain in a same-box bench A/B, profiles/r4/bench/s18_*); 41 won
-    # isolated decode timings (M = 512 LM head 4-7 %) but cost the step 1.8 % in a same-box
-    # bench A/B (42,548 without vs 41,790 / 41,653 tok/s with, profiles/r4/bench/)
     excl_env = os.environ.get("DLI_GEMM_EXCLUDE")
-    # 34 too: the 4-wave family wins isolated cold-weight timings within the noise
-    # but loses in the decode graph — down at M = 512 ran 70.4 us on tile 34 against 56.9 on
-    # the 8-phase tile 22, the LM head 433 vs 407 (profiles/r5/s12/wave_summary.txt vs
-    # profiles/r4/prof/llama_b512_head.wave.txt); the autotune flipped between them run to run
+    # 34, 41 and 45 are tile 22's kernel without its narrower widths and fp16 partial sums
     excl = {int(t) for t in (excl_env if excl_env is not None else "26,34,41,45,55").split(",")
             if t.strip()}
     # the persistent tile 55, whose stores drain under the next tile's loads, for the unsplit products of

@@ -398,7 +398,13 @@ __global__ void __launch_bounds__(256, 1) prefill_long_kernel(
     iteration(int_c<0>{});
     iteration(int_c<1>{});
   }
-  if (t < mine) iteration(int_c<0>{});
+  // (what follows reads O, hipcc's copies of it where these paths meet included: the wait states on each of them)
+  if (t < mine) {
+    iteration(int_c<0>{});
+    pad();
+  } else {
+    pad();
+  }
   // the workgroup's other tiles: this wave's share of the staging, and the barriers
   for (; t < ntiles; ++t) {
     find(t + 3);
@@ -411,7 +417,6 @@ __global__ void __launch_bounds__(256, 1) prefill_long_kernel(
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // no LDS-DMA outlives the workgroup
   if (!active) return;
-  pad();
 #pragma unroll
   for (int qb = 0; qb < 2; ++qb) {
     const auto w = __builtin_amdgcn_permlane32_swap(__float_as_uint(l_run[qb]), __float_as_uint(l_run[qb]), false, false);

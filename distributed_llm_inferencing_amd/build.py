@@ -26,10 +26,14 @@ import argparse
 import concurrent.futures as cf
 import hashlib
 import os
+import re
 import shutil
 import subprocess
 import sys
+import tempfile
 from pathlib import Path
+
+from . import asm_check
 
 PKG = Path(__file__).resolve().parent
 REPO = PKG.parent
@@ -70,8 +74,17 @@ def _digest(paths, flags) -> str:
 # compiler-made copy of their accumulators inside the K loop (a scratch spill, a rolled
 # epilogue indexing them dynamically) reads AGPRs an MFMA may still be writing. Such a
 # kernel must keep its accumulators in registers: a nonzero scratch size fails the build.
-ASM_MFMA_KERNELS = ("gemm4w_kernel",)
+# And the assembly of their sources is looked through for such copies (asm_check.py).
+ASM_MFMA_KERNELS = ("gemm4w_kernel", "prefill_long_kernel")
 _REMARKS = "-Rpass-analysis=kernel-resource-usage"
+
+
+def has_asm_mfma(src: Path) -> bool:
+    """Whether a source, or a header of the kernels that it includes, holds matrix products as asm statements."""
+    text = src.read_text()
+    texts = [text] + [(src.parent / h).read_text() for h in re.findall(r'#include "([\w.]+)"', text)
+                      if (src.parent / h).exists()]
+    return any(re.search(r'asm volatile\(\s*"v_mfma', t) for t in texts)
 
 
 def check_scratch(stderr: str, src: str) -> None:
@@ -96,15 +109,19 @@ def _compile(src: Path, obj: Path, flags, headers) -> Path:
     if obj.exists() and stamp.exists() and stamp.read_text() == dig:
         return obj
     obj.parent.mkdir(parents=True, exist_ok=True)
-    remarks = src.suffix == ".hip" and any(k.split("_")[0] in src.read_text()
-                                           for k in ASM_MFMA_KERNELS)
-    cmd = [_hipcc(), *flags, *([_REMARKS] if remarks else []), "-I", str(CSRC / "kernels"),
-           "-I", str(CSRC / "runtime"), "-c", str(src), "-o", str(obj)]
-    r = subprocess.run(cmd, capture_output=True, text=True)
-    if r.returncode != 0:
-        raise RuntimeError(f"hipcc failed for {src.name}:\n{' '.join(cmd)}\n{r.stderr[-6000:]}")
-    if remarks:
-        check_scratch(r.stderr, src.name)
+    checked = src.suffix == ".hip" and has_asm_mfma(src)
+    with tempfile.TemporaryDirectory(dir=obj.parent) as tmp:
+        # (-save-temps leaves the assembly that the object is made of beside it)
+        made = Path(tmp) / obj.name if checked else obj
+        cmd = [_hipcc(), *flags, *([_REMARKS, "-save-temps=obj"] if checked else []), "-I", str(CSRC / "kernels"),
+               "-I", str(CSRC / "runtime"), "-c", str(src), "-o", str(made)]
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        if r.returncode != 0:
+            raise RuntimeError(f"hipcc failed for {src.name}:\n{' '.join(cmd)}\n{r.stderr[-6000:]}")
+        if checked:
+            check_scratch(r.stderr, src.name)
+            asm_check.check((Path(tmp) / f"{src.stem}-hip-amdgcn-amd-amdhsa-{ARCH}.s").read_text(), src.name)
+            os.replace(made, obj)
     stamp.write_text(dig)
     return obj
 

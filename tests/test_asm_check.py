@@ -1,0 +1,54 @@
+"""The build's look through the assembly of kernels whose matrix products are asm statements, which hipcc pads nothing
+for: what it finds, what it lets pass, and the kernels themselves."""
+import subprocess
+
+import pytest
+
+from distributed_llm_inferencing_amd import asm_check, build
+
+PRODUCT = "v_mfma_f32_32x32x16_bf16 a[0:15], v[0:3], a[16:19], a[0:15]"
+SMALL = "v_mfma_f32_16x16x32_bf16 v[8:11], v[0:3], v[4:7], 0"
+
+
+def function(*lines):
+    return "\t.type\tk,@function\nk:\n" + "\n".join(lines) + "\n\ts_endpgm\n.Lfunc_end0:\n"
+
+
+# 12 wait states behind the 32x32 product, 8 behind the 16x16 one; any path counts, and so do operands written just before
+@pytest.mark.parametrize("lines,ok", [
+    ([PRODUCT, "s_nop 10", "v_accvgpr_read_b32 v0, a15"], False),
+    ([PRODUCT, "s_nop 11", "v_accvgpr_read_b32 v0, a15"], True),
+    ([PRODUCT, "s_nop 3", "v_accvgpr_read_b32 v0, a16"], True),
+    ([PRODUCT, "v_accvgpr_write_b32 a3, v9"], False),
+    ([PRODUCT, PRODUCT, "s_nop 11", "v_accvgpr_read_b32 v0, a0"], True),
+    ([PRODUCT, "v_mfma_f32_32x32x16_bf16 a[32:47], v[0:3], a[12:15], a[32:47]"], False),
+    ([SMALL, "s_nop 6", "global_store_dwordx4 v12, v[8:11], s[0:1]"], False),
+    ([SMALL, "s_nop 7", "global_store_dwordx4 v12, v[8:11], s[0:1]"], True),
+    ([PRODUCT, "s_cbranch_scc0 .LBB0_1", "s_nop 15", ".LBB0_1:", "v_accvgpr_read_b32 v0, a0"], False),
+    ([PRODUCT, "s_branch .LBB0_2", ".LBB0_1:", "v_accvgpr_read_b32 v0, a0", ".LBB0_2:", "s_nop 15"], True),
+    ([".LBB0_1:", "v_accvgpr_read_b32 v0, a0", "s_nop 15", PRODUCT, "s_cbranch_vccnz .LBB0_1"], False),
+    (["v_cvt_pk_bf16_f32 v3, v20, v21", "s_nop 0", PRODUCT], False),
+    (["v_cvt_pk_bf16_f32 v3, v20, v21", "s_nop 1", PRODUCT], True),
+])
+def test_what_is_found(lines, ok):
+    if ok:
+        asm_check.check(function(*lines), "k.hip")
+    else:
+        with pytest.raises(RuntimeError, match="k.hip: 1 hazards"):
+            asm_check.check(function(*lines), "k.hip")
+
+
+def test_kernels_with_asm_products_are_looked_through():
+    named = {s.name for s in build._group_sources("kernels")[0] if build.has_asm_mfma(s)}
+    assert {"attention_prefill_long.hip", "gemm4w.hip", "gemm4w_narrow.hip"} <= named
+    with pytest.raises(RuntimeError, match="8 B/lane"):
+        build.check_scratch("x: remark: Function Name: _Z19prefill_long_kernelILi0EEv\nx: remark: ScratchSize [bytes/lane]: 8\n", "x")
+
+
+def test_long_attention(tmp_path):
+    src, out = build.CSRC / "kernels" / "attention_prefill_long.hip", tmp_path / "k.s"
+    subprocess.run([build._hipcc(), *build.KERNEL_FLAGS, "-I", str(src.parent), "--offload-device-only", "-S", str(src), "-o", str(out)],
+                   check=True, capture_output=True)
+    text = out.read_text()
+    assert sum(fn.name.startswith("_Z19prefill_long_kernel") for fn in asm_check.functions(text)) == 2
+    asm_check.check(text, src.name)

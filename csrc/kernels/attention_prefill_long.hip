@@ -95,7 +95,12 @@ __global__ void __launch_bounds__(256, 1) prefill_long_kernel(
   // where K's and V's rows of this head begin
   const u16* const first_k = SRC ? k_cache + (long)kvh * block_size * HD : qkv + (long)s0 * row_stride + (long)(hq + kvh) * HD;
   const u16* const first_v = SRC ? v_cache + (long)kvh * block_size * HD : first_k + hkv * HD;
-  const uintptr_t heads[2] = {(uintptr_t)first_k, (uintptr_t)first_v};
+  // (in scalar registers from here on: a descriptor formed beside its request from vector ones would need wait states
+  // that nobody puts ahead of an asm statement)
+  auto uniform = [](const u16* p) __attribute__((always_inline)) -> uintptr_t {
+    return (uintptr_t)scalar((uint32_t)(uintptr_t)p) | (uintptr_t)scalar((uint32_t)((uintptr_t)p >> 32)) << 32;
+  };
+  const uintptr_t heads[2] = {uniform(first_k), uniform(first_v)};
   // Rows: one descriptor a sequence and operand, the tile in the scalar offset. Blocks: a descriptor a piece, whose
   // place and bytes V's piece, staged an iteration after K's, takes over
   const int total = __builtin_amdgcn_readfirstlane((nkeys - 1) * stride + HD * 2);                   // (the launcher keeps a sequence's below 2^31)
@@ -131,7 +136,7 @@ __global__ void __launch_bounds__(256, 1) prefill_long_kernel(
     const uint32_t so = SRC == BLOCKS_OF_16 ? 0 : scalar((uint32_t)(row_at[kv] + j * 16 * stride));
     const int lane_at = voff;
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                 :: "s"(dst), "v"(lane_at), "s"(r), "s"(so) : "memory");
+                 :: "s"(dst), "v"(lane_at), "s"(r), "s"(so) : "memory", "m0");
   };
   using K_ = int_c<0>;
   using V_ = int_c<1>;

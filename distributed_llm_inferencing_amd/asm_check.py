@@ -15,6 +15,9 @@ MFMA_RESULT = {"v_mfma_f32_16x16x32_bf16": 8, "v_mfma_f32_32x32x16_bf16": 12}
 MFMA_RESULT_MOST = 20
 # from a vector instruction to a matrix product that reads its result
 MFMA_OPERAND = 2
+# from a vector instruction's scalar result to a memory instruction that reads it
+SCALAR_TO_MEMORY = 5
+_MEMORY = ("buffer_", "global_", "flat_", "scratch_")
 
 _REG = re.compile(r"(?<![\w.])([vas])(?:(\d+)|\[(\d+):(\d+)\])(?!\w)")
 _LABEL = re.compile(r"^([.\w$]+):")
@@ -91,7 +94,8 @@ def _result_touched(result: frozenset, name: str, ops) -> bool:
 
 def _written(name: str, ops) -> frozenset:
     """The registers that a vector instruction other than a matrix product writes."""
-    return registers(ops[0]) | (registers(ops[1]) if "swap" in name else frozenset())
+    second = "swap" in name or "div_scale" in name or "_co_" in name
+    return registers(ops[0]) | (registers(ops[1]) if second else frozenset())
 
 
 def faults(fn: Code):
@@ -104,9 +108,11 @@ def faults(fn: Code):
                     yield fn.code[n][2], f"{fn.code[n][0]} {fn.code[n][1][0]} too early behind line {line}'s {name} {ops[0]}"
         elif name.startswith("v_"):
             result = _written(name, ops)
-            for n in fn.within(at, MFMA_OPERAND):
+            scalars = frozenset(r for r in result if r[0] == "s")
+            for n in fn.within(at, SCALAR_TO_MEMORY if scalars else MFMA_OPERAND):
                 to, used, where = fn.code[n]
-                if to.startswith("v_mfma") and any(result & registers(o) for o in used[1:]):
+                early = scalars if to.startswith(_MEMORY) else result if to.startswith("v_mfma") and not scalars else ()
+                if any(registers(o).intersection(early) for o in used):
                     yield where, f"{to} {used[0]} too early behind line {line}'s {name} {ops[0]}"
 
 

@@ -7,6 +7,7 @@ import pytest
 from distributed_llm_inferencing_amd import asm_check, build
 
 PRODUCT = "v_mfma_f32_32x32x16_bf16 a[0:15], v[0:3], a[16:19], a[0:15]"
+REQUEST = "buffer_load_dwordx4 v156, s[40:43], s78 offen lds"
 SMALL = "v_mfma_f32_16x16x32_bf16 v[8:11], v[0:3], v[4:7], 0"
 
 
@@ -14,7 +15,7 @@ def function(*lines):
     return "\t.type\tk,@function\nk:\n" + "\n".join(lines) + "\n\ts_endpgm\n.Lfunc_end0:\n"
 
 
-# 12 wait states behind the 32x32 product, 8 behind the 16x16 one; any path counts, and so do operands written just before
+# 12 wait states behind the 32x32 product, 8 behind the 16x16 one, on any path; 2 from an operand's write to its product
 @pytest.mark.parametrize("lines,ok", [
     ([PRODUCT, "s_nop 10", "v_accvgpr_read_b32 v0, a15"], False),
     ([PRODUCT, "s_nop 11", "v_accvgpr_read_b32 v0, a15"], True),
@@ -29,6 +30,14 @@ def function(*lines):
     ([".LBB0_1:", "v_accvgpr_read_b32 v0, a0", "s_nop 15", PRODUCT, "s_cbranch_vccnz .LBB0_1"], False),
     (["v_cvt_pk_bf16_f32 v3, v20, v21", "s_nop 0", PRODUCT], False),
     (["v_cvt_pk_bf16_f32 v3, v20, v21", "s_nop 1", PRODUCT], True),
+    # a scalar from a vector instruction: 5 to the memory instruction that reads it
+    (["v_readfirstlane_b32 s40, v148", "s_and_b32 s41, s2, 0xffff", "s_add_i32 s2, s49, s56", "s_mov_b32 m0, s2", "s_nop 0", REQUEST], False),
+    (["v_readfirstlane_b32 s40, v148", "s_nop 4", REQUEST], True),
+    (["v_readlane_b32 s78, v148, 3", "s_nop 2", REQUEST], False),
+    (["s_mov_b32 s40, s2", REQUEST], True),
+    (["v_readfirstlane_b32 s40, v148", "s_add_i32 s40, s40, s2"], True),
+    (["v_div_scale_f32 v133, s[0:1], v132, v132, 1.0", "global_store_dword v12, v133, s[4:5]"], True),
+    (["v_div_scale_f32 v133, s[4:5], v132, v132, 1.0", "global_store_dword v12, v133, s[4:5]"], False),
 ])
 def test_what_is_found(lines, ok):
     if ok:

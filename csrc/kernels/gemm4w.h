@@ -40,12 +40,15 @@ template <int N, class F> __device__ __forceinline__ void unroll(F f) {
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* p, int bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
 }
-// silu(g) u, or gelu(g) u by its tanh form, with v_rcp_f32 (1 ulp) for the division's ten instructions: 128 of them a
-// lane are 5 k cycles of a tile. The rounding to bf16 behind it is 2^15 times coarser; the outputs' error against
-// 64 bits is 1.657e-3 (SiLU, 8192 x 28672 x 4096) and 1.658e-3 (GELU) with either
-template <int EPI> __device__ __forceinline__ float pair_rcp(float g, float u) {
+// silu(g) u, or gelu(g) u by its tanh form, with a quotient that costs 6 instructions for a division's ten (128 of them
+// a lane are 5 k cycles of a tile) and equals it to the bit (by all of 2^26 random gates and as many of each range of
+// exponents; gates below 2^-124 to 2^-149). The reciprocal alone, 2 instructions, is an ulp off in a quarter of the cases.
+// g / d as (g / 4) / (d / 4), whose reciprocal is no denormal number, which v_rcp_f32 would flush; the quotient's
+// remainder corrects it, and v_div_fixup_f32 sees to infinities
+template <int EPI> __device__ __forceinline__ float pair_div(float g, float u) {
   const float e = EPI == EPI_GELU_MUL ? 1.5957691216057308f * (g + 0.044715f * g * g * g) : g;
-  return g * __builtin_amdgcn_rcpf(1.f + __expf(-e)) * u;
+  const float n = 0.25f * g, d = fmaf(0.25f, __expf(-e), 0.25f), r = __builtin_amdgcn_rcpf(d), q = n * r;
+  return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, q, n), r, q), d, n) * u;
 }
 // 1 KiB of LDS-DMA (16 B a lane); IMM moves both the address in memory and the one in LDS
 template <int IMM>
@@ -403,7 +406,7 @@ __global__ void __launch_bounds__(256, 1) gemm4w_kernel(
           const f32x4 g = vget(acc[i][2 * j]), u = vget(acc[i][2 * j + 1]);
           float o[4];
 #pragma unroll
-          for (int r = 0; r < 4; ++r) o[r] = pair_rcp<EPI>(g[r], u[r]);
+          for (int r = 0; r < 4; ++r) o[r] = pair_div<EPI>(g[r], u[r]);
           return uint2{pack2bf(o[0], o[1]), pack2bf(o[2], o[3])};
         } else if constexpr (EPI == EPI_SLAB16) {
           const f32x4 v = vget(acc[i][j]);

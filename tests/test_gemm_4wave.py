@@ -122,3 +122,28 @@ def test_block_maxima_of_the_head(gpu, monkeypatch, M, N, K):
     assert off(logits, expected(x, w[0], "f32")) < BOUND[True]
     assert (top is None) == (K % 128 != 0)               # tile 55 takes whole pairs of K-tiles
     assert top is None or torch.equal(top[0], block_keys(logits, top[1]))
+
+
+# SiLU and GELU pairs divide as the other kernels do, to the bit: 4 million gates given to 24 bits (three bf16 values each,
+# which one product adds up), of which a quotient off by an ulp of fp32 would round some 30 to another bf16 value
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("epi", ["silu_mul", "gelu_mul"])
+def test_quotients(gpu, epi, tile):
+    if tile == 45 and epi == "gelu_mul":
+        tile = 55
+    M, gates, K = 32768, 128, 512
+    g = torch.Generator(device=gpu).manual_seed(7)
+    left = torch.randn(M, gates, device=gpu, generator=g) * torch.tensor([1.0, 4.0, 40.0, 0.01], device=gpu).repeat(gates // 4)
+    x = torch.zeros(M, K, device=gpu).bfloat16()
+    for i in range(3):
+        x[:, i:3 * gates:3] = left.bfloat16()
+        left = left - x[:, i:3 * gates:3].float()
+    x[:, 3 * gates] = torch.rand(M, device=gpu, generator=g).bfloat16() + 0.5
+    w = torch.zeros(gates // 16, 2, 16, K, device=gpu).bfloat16()
+    for j in range(gates):
+        w[j // 16, 0, j % 16, 3 * j:3 * j + 3] = 1
+    w[:, 1, :, 3 * gates] = 1
+    w = w.view(2 * gates, K)
+    got, other = (ops._gemm_native(x, w, epi, plan=G.GemmPlan("dli", t, 1)) for t in (tile, 13))
+    assert torch.equal(got, other)

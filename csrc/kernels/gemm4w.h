@@ -578,6 +578,9 @@ static int launch_4w(const void* A, int lda, const void* W, int ldw, void* C, in
                      hipStream_t st) {
   if (epi_pairs(EPI) && N % 32) return (int)hipErrorInvalidValue;
   if (K % (splits * BK)) return (int)hipErrorInvalidValue;
+  // (a panel's range is its rows times their stride in 32 bits, which overlapping rows would reach past: ops/gemm.py's
+  // spaced copies those)
+  if (lda < K || ldw < K || lda >= (1 << 22) || ldw >= (1 << 22)) return (int)hipErrorInvalidValue;
   if (EPI == EPI_RES && (splits != 1 || group_off != nullptr || ((N | ldc) & 7) || ((uintptr_t)C & 15) || C == nullptr ||
                          ldc >= (1 << 21) - 1024))
     return (int)hipErrorInvalidValue;

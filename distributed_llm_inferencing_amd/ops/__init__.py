@@ -237,7 +237,8 @@ def _gemm_native(x, w, epi: str, bias=None, out=None, plan: Optional[G.GemmPlan]
     if splits > 1:
         ws = G.workspace(x.device, splits * M * Nn * 4)
     m_arg = M if group_off is None else rows_per_group
-    _native_call("dli_gemm", _p(x), x.stride(0), _p(w), w.stride(-2), _p(out), out.stride(0),
+    (x, lda), (w, ldw) = G.spaced(x, plan.tile), G.spaced(w, plan.tile)
+    _native_call("dli_gemm", _p(x), lda, _p(w), ldw, _p(out), out.stride(0),
                  m_arg, Nn, K, G.EPI[epi], plan.tile, splits, _p(bias), _p(ws), _p(group_off),
                  groups, _st())
     return out
@@ -294,7 +295,8 @@ def _slab_gemm(x, w, p: G.GemmPlan, ws) -> int:
     M, K = x.shape
     Nn = w.shape[0]
     fmt = 1 if (G.SLAB16 and p.tile in G.SLAB16_TILES and p.splits in (2, 4, 8)) else 0
-    _native_call("dli_gemm", _p(x), x.stride(0), _p(w), w.stride(-2), None, Nn, M, Nn, K,
+    (x, lda), (w, ldw) = G.spaced(x, p.tile), G.spaced(w, p.tile)
+    _native_call("dli_gemm", _p(x), lda, _p(w), ldw, None, Nn, M, Nn, K,
                  G.EPI["slab16"] if fmt else 0, p.tile, p.splits, None, _p(ws), None, 1, _st())
     return fmt
 
@@ -689,7 +691,8 @@ def head(h, w):
         return linear(h, w, epi=HEAD_EPI), None
     out = torch.empty(M, Nn, dtype=torch.float32, device=h.device)
     keys = torch.empty(M, -(-Nn // bw), dtype=torch.int32, device=h.device)
-    _native_call("dli_gemm_head", _p(h), h.stride(0), _p(w), w.stride(-2), _p(out), Nn, M, Nn,
+    (h, lda), (w, ldw) = G.spaced(h, tile), G.spaced(w, tile)
+    _native_call("dli_gemm_head", _p(h), lda, _p(w), ldw, _p(out), Nn, M, Nn,
                  h.shape[1], tile, _p(keys), _st())
     return out, (keys, bw)
 

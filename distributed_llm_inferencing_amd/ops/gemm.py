@@ -121,6 +121,22 @@ EPI = {"none": 0, "f32": 1, "silu_mul": 2, "bias_gelu": 3, "bias": 4, "splitk": 
        "slab16": 5, "gelu_erf": 6, "clamp_mul": 7, "relu_mul": 8, "gelu_mul": 9, "res_add": 16}
 # the 4-wave kernel's tiles, whose unsplit product can add into its output (EPI "res_add")
 RES_ADD_TILES = frozenset((22, 28, 34, 41, 45, 55))
+
+
+# row strides that the 4-wave kernel reaches over a tile's 256 rows by 32-bit offsets
+MAX_4W_STRIDE = 1 << 22
+
+
+def spaced(t: torch.Tensor, tile: int):
+    """(an operand, its row stride) as the tile's kernel takes them: the 4-wave kernel reads a tile's rows by offsets
+    within their range and so needs them at least their length apart, and not too far. Rows that overlap (expanded
+    ones, windows) are copied; one row has no stride."""
+    ld, n = t.stride(-2), t.shape[-1]
+    if tile not in RES_ADD_TILES or n <= ld < MAX_4W_STRIDE:
+        return t, ld
+    return (t, n) if t.shape[-2] == 1 else (t.contiguous(), n)
+
+
 # epilogues over the interleaved gate/up weight: the output is half as wide
 PAIR_EPIS = ("silu_mul", "clamp_mul", "relu_mul", "gelu_mul")
 # tiles whose slab-only split-K call can store fp16 partials (EPI "slab16"); the fused consumers then

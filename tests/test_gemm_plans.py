@@ -190,3 +190,37 @@ def test_the_library_refuses_a_missing_bias(gpu):
         for epi in ("bias", "bias_gelu"):
             assert lib.dli_gemm(ops._p(x), 768, ops._p(w), 768, ops._p(o), 96, 4, 96, 768, G.EPI[epi], tile, 1, None,
                                 None, None, 1, ops._st()) != 0
+
+
+# rows that the 4-wave kernel does not reach by its offsets (expanded, windows of a signal, very far apart) go to it as a
+# copy, one row with its length for a stride; other kernels take them as they are
+@pytest.mark.parametrize("tile,copied", [(22, True), (28, True), (45, True), (55, True), (26, False), (2, False)])
+def test_rows_of_any_stride(monkeypatch, tile, copied):
+    calls = []
+    monkeypatch.setattr(ops, "_native_call", lambda name, *a: calls.append(a[:4]))
+    monkeypatch.setattr(ops, "_st", lambda: None)
+    plan, w = G.GemmPlan("dli", tile, 1), torch.zeros(32, 128).bfloat16()
+    signal = torch.zeros(4096).bfloat16()
+    for x in (w[:1].expand(16, 128), signal.as_strided((16, 128), (40, 1)), signal.as_strided((16, 128), (200, 1)), w[:, :128]):
+        ops._gemm_native(x, w, "none", plan=plan)
+        a, lda, _, ldw = calls.pop()
+        assert (a, lda) == ((x.data_ptr(), x.stride(0)) if not copied or x.stride(0) >= 128 else (a, 128)) and ldw == 128
+        assert (a == x.data_ptr()) == (not copied or x.stride(0) >= 128)
+        ops._gemm_native(w, x[:16], "none", plan=plan)
+        assert calls.pop()[3] == (max(x.stride(0), 128) if copied else x.stride(0))
+    ops._gemm_native(signal.as_strided((1, 128), (1, 1)), w, "none", plan=plan)
+    assert calls.pop()[:2] == (signal.data_ptr(), 128 if copied else 1)
+    monkeypatch.setattr(G, "MAX_4W_STRIDE", 200)
+    assert G.spaced(signal.as_strided((16, 128), (200, 1)), tile)[1] == (128 if copied else 200)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", [22, 28, 45, 55])
+@pytest.mark.parametrize("stride", [0, 8, 40, 120])
+def test_products_of_overlapping_rows(gpu, tile, stride):
+    signal = torch.randn(300 * 120 + 128, device=gpu, generator=torch.Generator(device=gpu).manual_seed(1)).bfloat16()
+    x = signal.as_strided((300, 128), (stride, 1))
+    w = torch.randn(264, 128, device=gpu, generator=torch.Generator(device=gpu).manual_seed(2)).bfloat16()
+    plan = G.GemmPlan("dli", tile, 1)
+    for a, b in ((x, w), (w, x)):
+        assert torch.equal(ops._gemm_native(a, b, "f32", plan=plan), ops._gemm_native(a.contiguous(), b.contiguous(), "f32", plan=plan))

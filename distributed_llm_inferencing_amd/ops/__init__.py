@@ -310,16 +310,30 @@ def _splitk_plan(x, w):
     return p if p.splits > 1 else None
 
 
+def _extent(t) -> tuple:
+    """(first, past the last) byte that a tensor's elements lie in."""
+    last = sum((n - 1) * s for n, s in zip(t.shape, t.stride()))
+    return t.data_ptr(), t.data_ptr() + (last + 1) * t.element_size()
+
+
+def _apart(a, b) -> bool:
+    """Whether two tensors share no byte."""
+    (a0, a1), (b0, b1) = _extent(a), _extent(b)
+    return a1 <= b0 or b1 <= a0
+
+
 def _add_product(x, w, residual, plan: Optional[G.GemmPlan]) -> bool:
     """residual += x @ w.T inside the GEMM, rounded once, where the unsplit plan's kernel has that epilogue and the
     rows are whole, aligned and many; whether it did. The product neither travels as bf16 to the add nor is read
-    again there. 4096 columns, us with the norm behind it, apart / so: K = 4096, 16384 rows 458 / 433, 7993 223 / 207,
+    again there. Not where the residual is an operand too, in part even: tiles are stored while others are still
+    read. 4096 columns, us with the norm behind it, apart / so: K = 4096, 16384 rows 458 / 433, 7993 223 / 207,
     2112 73 / 71; K = 14336 1350 / 1326, 676 / 660, 204 / 200. Few rows take split plans and their fused reduce."""
     if not (_use_native(x) and x.dtype == w.dtype == residual.dtype == torch.bfloat16 and w.dim() == 2):
         return False
     (M, K), Nn = x.shape, w.shape[0]
     if (M < G.LARGE_M or w.shape[1] != K or residual.shape != (M, Nn) or not residual.is_contiguous() or Nn % 8
-            or residual.data_ptr() % 16 or x.stride(-1) != 1 or w.stride(-1) != 1):
+            or residual.data_ptr() % 16 or x.stride(-1) != 1 or w.stride(-1) != 1 or Nn >= G.MAX_4W_STRIDE // 2 - 1024
+            or not x.device == w.device == residual.device or not (_apart(residual, x) and _apart(residual, w))):
         return False
     cut = G.row_cut(M, Nn, K) if plan is None else 0
     rows = cut or M

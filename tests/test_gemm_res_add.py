@@ -87,3 +87,34 @@ def test_linear_add_rmsnorm(gpu, monkeypatch, M, N, K, off, taken, norm):
         assert h is None
     else:
         assert torch.equal(h, ops.rmsnorm(residual, nw, 1e-5) if taken else normed)
+
+
+# the add inside the product stores tiles while others are read: not where the residual is an operand, or shares bytes
+# with one, nor where it lies elsewhere
+@pytest.mark.parametrize("K", [1024, 4096])
+def test_operands_apart_from_the_residual(monkeypatch, K):
+    calls = []
+    monkeypatch.setattr(ops, "_use_native", lambda t: True)
+    monkeypatch.setattr(ops, "_gemm_native", lambda *a, **k: calls.append(a))
+    monkeypatch.setattr(G, "row_cut", lambda *a: 0)
+    monkeypatch.setattr(G, "plan", lambda *a: G.GemmPlan("dli", 22, 1))
+    M, N = 1024, 1024
+    held = torch.zeros(3 * M * K).bfloat16()
+    residual, w = held[:M * N].view(M, N), torch.zeros(N, K).bfloat16()
+    for at, x in ((0, held[:M * K]), (8, held[8:M * K + 8]), (M * N - 8, held[M * N - 8:M * N - 8 + M * K])):
+        assert not ops._add_product(x.view(M, K), w, residual, None) and not calls, at
+    assert not ops._add_product(torch.zeros(M, K).bfloat16(), held[M * N - 8:M * N - 8 + N * K].view(N, K), residual, None)
+    assert not ops._add_product(torch.zeros(M, K).bfloat16(), w, residual.to("meta"), None) and not calls
+    assert ops._add_product(held[M * N:M * N + M * K].view(M, K), w, residual, None) and calls
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("norm", [True, False])
+def test_a_residual_that_is_the_input(gpu, norm):
+    g = torch.Generator(device=gpu).manual_seed(3)
+    x = torch.randn(4096, 4096, device=gpu, generator=g).bfloat16()
+    w = (torch.randn(4096, 4096, device=gpu, generator=g) / 64).bfloat16()
+    nw = torch.ones(4096, device=gpu).bfloat16() if norm else None
+    want = x + ops.linear(x, w)
+    ops.linear_add_rmsnorm(x, w, x, nw, 1e-5)
+    assert torch.equal(x, want)

@@ -30,15 +30,18 @@ extern "C" int dli_gemm_set_slab_store(int mode) {
   const int old = gemm_tiles_set_slab_store(mode);
   gemm_stream_set_slab_store(mode);
   gemm_8p_set_slab_store(mode);
+  gemm_4w_set_slab_store(mode);
   return old;
 }
 
 // one family's split-K slab store (0 plain, 1 nt, 2 sc1, 3 sc0 sc1): family 0 = the generic
-// tiles (decode O / QKV), 1 = the 8-phase kernels
+// tiles (decode O / QKV), 1 = the 8-phase kernels, 2 = the 4-wave tiles (22 and 28 too), which refuse split products
+// in any but mode 0
 extern "C" int dli_gemm_set_slab_store_family(int family, int mode) {
   switch (family) {
     case 0: gemm_stream_set_slab_store(mode); return gemm_tiles_set_slab_store(mode);
     case 1: return gemm_8p_set_slab_store(mode);
+    case 2: return gemm_4w_set_slab_store(mode);
     default: return -1;
   }
 }

@@ -571,6 +571,9 @@ static int cu_count() {
   return cus;
 }
 
+// the mode that dli_gemm_set_slab_store asked for
+int gemm_4w_store_mode();
+
 // M: rows, or the most rows of a group (group_off: their offsets, groups of them)
 template <int EPI, int NJ>
 static int launch_4w(const void* A, int lda, const void* W, int ldw, void* C, int ldc, int M, int N,
@@ -581,6 +584,9 @@ static int launch_4w(const void* A, int lda, const void* W, int ldw, void* C, in
   // (a panel's range is its rows times their stride in 32 bits, which overlapping rows would reach past: ops/gemm.py's
   // spaced copies those)
   if (lda < K || ldw < K || lda >= (1 << 22) || ldw >= (1 << 22)) return (int)hipErrorInvalidValue;
+  // The kernel has one way to store fp32 partial sums (the others' probe modes would more than double its code): while
+  // another is set, split products are refused and not timed as what they are not
+  if (splits > 1 && EPI != EPI_SLAB16 && gemm_4w_store_mode() != 0) return (int)hipErrorInvalidValue;
   if (EPI == EPI_RES && (splits != 1 || group_off != nullptr || ((N | ldc) & 7) || ((uintptr_t)C & 15) || C == nullptr ||
                          ldc >= (1 << 21) - 1024))
     return (int)hipErrorInvalidValue;

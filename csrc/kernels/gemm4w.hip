@@ -9,6 +9,7 @@
 // a bias 32 -> 23; partial sums in 16 bits of 512 rows: 6144 x 4096 in four 35.8 -> 27.0, 4096 x 4096 in four 26.5
 // (eight) -> 21.6, 4096 x 14336 in eight 60.9 -> 50.9.
 #include "gemm4w.h"
+#include <utility>
 
 int gemm_4w_narrow(int epi, int nj, DLI_GEMM_ARGS);
 
@@ -51,6 +52,10 @@ static int launch8(int epi, DLI_GEMM_ARGS) {
     default: return DLI_NOT_MINE;
   }
 }
+
+static int g_store_mode = 0;
+int gemm_4w_set_slab_store(int mode) { return std::exchange(g_store_mode, mode); }
+int gemm_4w_store_mode() { return g_store_mode; }
 
 int gemm_4w_dispatch(int epi, int tile_cfg, DLI_GEMM_ARGS) {
   const bool pairs = epi_pairs(epi), bias_epi = epi == EPI_BIAS || epi == EPI_BIAS_GELU;

@@ -114,8 +114,7 @@ __device__ __forceinline__ void slab_store4(float* p, f32x4 v, int mode) {
   }
 }
 
-// the fp32 partial quad (store modes 0-3); the 4-wave family calls it directly (its
-// accumulator-pinned epilogue has no register room for the probe modes)
+// the fp32 partial quad (store modes 0-3); the 4-wave family calls it directly, always in mode 0
 __device__ __forceinline__ void slab_quad_fp32(float* p, f32x4 v, int mode, bool vec, int left) {
   if (vec) {
     slab_store4(p, v, mode);
@@ -345,6 +344,7 @@ int gemm_gemv_dispatch(int epi, int tile_cfg, DLI_GEMM_ARGS);
 int gemm_tiles_set_slab_store(int mode);
 int gemm_stream_set_slab_store(int mode);
 int gemm_8p_set_slab_store(int mode);
+int gemm_4w_set_slab_store(int mode);
 
 // EPI -> template argument, for a family's dispatch<EPI>(tile_cfg, ...); the families with
 // an fp16 slab store (tiles, streaming, 8-phase) take DLI_EPI_SWITCH_S16

@@ -27,7 +27,7 @@ def main():
     ap.add_argument("--shapes", default="o,qkv")
     ap.add_argument("--iters", type=int, default=6)
     ap.add_argument("--slab-store", type=int, default=0,
-                    help="split-K partial stores: 0 plain, 1 nt, 2 sc1, 3 sc0 sc1")
+                    help="fp32 split-K partial stores: 0 plain, 1 nt, 2 sc1, 3 sc0 sc1 (tiles 22 and 28 take 0 alone)")
     ap.add_argument("--top", type=int, default=0, help="print only the N fastest plans")
     a = ap.parse_args()
     from distributed_llm_inferencing_amd import ops

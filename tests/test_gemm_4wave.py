@@ -147,3 +147,23 @@ def test_quotients(gpu, epi, tile):
     w = w.view(2 * gates, K)
     got, other = (ops._gemm_native(x, w, epi, plan=G.GemmPlan("dli", t, 1)) for t in (tile, 13))
     assert torch.equal(got, other)
+
+
+# the kernel stores partial sums in one way: a product that should use another is refused, not run as if it did
+@pytest.mark.gpu
+@pytest.mark.parametrize("family", [None, 2])
+def test_other_store_modes_are_refused(gpu, family):
+    from distributed_llm_inferencing_amd.ops import _native
+    lib = _native.require_native()
+    x, w = operands(gpu, 300, 512, 256, 1)
+    setter = lib.dli_gemm_set_slab_store if family is None else lambda m: lib.dli_gemm_set_slab_store_family(family, m)
+    before = [ops._gemm_native(x, w[0], "f32", plan=G.GemmPlan("dli", t, 2)) for t in TILES]
+    assert setter(2) == 0
+    try:
+        for tile in TILES:
+            with pytest.raises(RuntimeError):
+                ops._gemm_native(x, w[0], "f32", plan=G.GemmPlan("dli", tile, 2))
+            ops._gemm_native(x, w[0], "f32", plan=G.GemmPlan("dli", tile, 1))
+    finally:
+        assert setter(0) == 2
+    assert all(torch.equal(b, ops._gemm_native(x, w[0], "f32", plan=G.GemmPlan("dli", t, 2))) for b, t in zip(before, TILES))

@@ -233,11 +233,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))
 // shortest max_seqlen that takes the 256-row kernel; below, the 64-row kernel wastes fewer
 // idle waves (settable for A/B runs and tests: dli_prefill_set_min_len)
 static int g_pl_min_len = 256;
-// shortest max_seqlen that takes waves of 64 rows (attention_prefill_long.hip; settable too:
-// dli_prefill_set_wave64_len), in launches of more than a round of workgroups: 2500 tokens 76 -> 69 us, 8 x 2000
-// 331 -> 319, 4 x 2048 162 -> 159, but 8 of 300 to 2000 174 -> 178, 16 x 1000 equal, and one round, where blocks
-// are paired, 2048 51 -> 58
-static int g_pw_min_len = 2048;
+constexpr int PL_ROUND = 256;                      // workgroups of a round: one a CU
+// max_seqlen from which waves of 64 rows (attention_prefill_long.hip) are considered, by the mix of lengths (takes_wave64);
+// any other length set by dli_prefill_set_wave64_len decides alone (A/B runs and tests)
+constexpr int PW_MIN_LEN = 2048;
+static int g_pw_min_len = PW_MIN_LEN;
 static int g_pf_pack = 1;                          // head packing for short prompts (A/B)
 
 // Tile image: 8-row x 32-column subtiles of 512 B (cdna_hip_programming.md §5.5 T10, image
@@ -493,20 +493,38 @@ int launch_prefill_long(void* out, int out_stride, const void* qkv, int row_stri
                         int max_seqlen, int hq, int hkv, float scale_log2, const int* ctx_lens, const void* k_cache,
                         const void* v_cache, const int* block_tables, int bt_stride, int block_size, hipStream_t st);
 
+// Whether a launch takes waves of 64 rows. They gain on long sequences (2500 tokens 75 -> 69 us, 7993 511 -> 473, 7 x
+// 2048 303 -> 289) and lose on short ones, whose last waves they leave idle (1000 tokens equal, 500 161 -> 174, 300 180
+// -> 222), and by every block, which has a CU to itself. One round of workgroups is for the other kernel, which pairs
+// blocks: 2048 51 / 58. The lengths themselves lie on the device. In the activation's rows, with T tokens, n
+// sequences and the longest L, the mean length over the tokens is at least low, that of n - 1 equal others; where low
+// covers a sequence's fixed cost this kernel is ahead (L = 2100 and 7 of about 1200 171 / 171, 7 of 350 76 / 80; L =
+// 4096 and 7 of 370 179 / 171; L = 2048 and 60 of 40 178 / 210), and where all the blocks find CUs, so that the longest
+// sequence is the launch (8 heads, L = 4096 and 7 of 300 111 / 96). Of 382 launches, 4 to 64 heads, this takes 257, 5 of
+// them slower by 1 to 2.5 %, and leaves 77 that would be slower by up to 19 % (and 32 that would gain). In the cache a few
+// rows may stand behind any number of keys, on one wave of a workgroup (2048 of 2048 and 40 of 8000 217 / 263): there
+// every sequence must have a block of rows, however the T are dealt.
+static bool takes_wave64(bool paged, long T, int n, long L, int hq, int hd, int row_stride, int block_size) {
+  if (hd != 128 || L < max(g_pw_min_len, g_pl_min_len) || (L + PL_ROWS - 1) / PL_ROWS * hq * n <= PL_ROUND) return false;
+  // (rows at 32-bit offsets from their sequence's first, and cached blocks that hold whole rows of a piece)
+  if (paged ? block_size < 16 || (block_size & (block_size - 1)) : (L + PL_ROWS) * row_stride * 2 >= (1L << 31)) return false;
+  if (g_pw_min_len != PW_MIN_LEN || n == 1) return true;
+  if (paged) return T - (n - 1) * L >= PL_ROWS;
+  if ((T / PL_ROWS + n) * hq <= 400) return true;
+  const double low = ((double)L * L + (double)(T - L) * (T - L) / (n - 1)) / T;
+  return low >= 1200.0 + 2e5 * n / T;
+}
+
 template <bool PAGED>
 static int launch_prefill(void* out, int out_stride, const void* qkv, int row_stride,
-                          const int* cu_seqlens, int num_seqs, int max_seqlen, int hq, int hkv,
+                          const int* cu_seqlens, int tokens, int num_seqs, int max_seqlen, int hq, int hkv,
                           int hd, float scale, const int* ctx_lens, const void* k_cache,
                           const void* v_cache, const int* block_tables, int bt_stride,
                           int block_size, hipStream_t st) {
   if (num_seqs <= 0 || max_seqlen <= 0) return 0;
   if (hq % hkv || (hd != 64 && hd != 128)) return (int)hipErrorInvalidValue;
   const float sl2 = scale * 1.4426950408889634f;
-  // (rows at 32-bit offsets from their sequence's first, and cached blocks that hold whole rows of a piece)
-  if (hd == 128 && max_seqlen >= max(g_pw_min_len, g_pl_min_len) &&
-      (long)((max_seqlen + PL_ROWS - 1) / PL_ROWS) * hq * num_seqs > 256 &&
-      (PAGED ? block_size >= 16 && (block_size & (block_size - 1)) == 0
-             : ((long)max_seqlen + 256) * row_stride * 2 < (1L << 31)))
+  if (takes_wave64(PAGED, tokens, num_seqs, max_seqlen, hq, hd, row_stride, block_size))
     return launch_prefill_long(out, out_stride, qkv, row_stride, cu_seqlens, num_seqs, max_seqlen, hq, hkv, sl2,
                                PAGED ? ctx_lens : nullptr, k_cache, v_cache, block_tables, bt_stride, block_size, st);
   if (hd == 128 && max_seqlen >= g_pl_min_len) {     // long sequences: 256-row workgroups
@@ -515,7 +533,7 @@ static int launch_prefill(void* out, int out_stride, const void* qkv, int row_st
     prefill_attn32_kernel<128, PAGED><<<grid32, 512, 0, st>>>(
         (u16*)out, out_stride, (const u16*)qkv, row_stride, cu_seqlens, hq, hkv, sl2, ctx_lens,
         (const u16*)k_cache, (const u16*)v_cache, block_tables, bt_stride, block_size,
-        blocks > 1 && (long)blocks * hq * num_seqs <= 256);
+        blocks > 1 && (long)blocks * hq * num_seqs <= PL_ROUND);
     DLI_RETURN_LAUNCH();
   }
   // waves per query head: pack 2 / 4 heads of one GQA group into a workgroup for short
@@ -537,10 +555,11 @@ static int launch_prefill(void* out, int out_stride, const void* qkv, int row_st
   DLI_RETURN_LAUNCH();
 }
 
+// tokens: rows of qkv, of all sequences together
 extern "C" int dli_prefill_attention(void* out, int out_stride, const void* qkv, int row_stride,
-                                     const int* cu_seqlens, int num_seqs, int max_seqlen, int hq,
+                                     const int* cu_seqlens, int tokens, int num_seqs, int max_seqlen, int hq,
                                      int hkv, int hd, float scale, hipStream_t st) {
-  return launch_prefill<false>(out, out_stride, qkv, row_stride, cu_seqlens, num_seqs,
+  return launch_prefill<false>(out, out_stride, qkv, row_stride, cu_seqlens, tokens, num_seqs,
                                max_seqlen, hq, hkv, hd, scale, nullptr, nullptr, nullptr,
                                nullptr, 0, 16, st);
 }
@@ -551,11 +570,11 @@ extern "C" int dli_prefill_attention_paged(void* out, int out_stride, const void
                                            int row_stride, const int* cu_seqlens,
                                            const int* ctx_lens, const void* k_cache,
                                            const void* v_cache, const int* block_tables,
-                                           int bt_stride, int num_seqs, int max_seqlen, int hq,
+                                           int bt_stride, int tokens, int num_seqs, int max_seqlen, int hq,
                                            int hkv, int hd, int block_size, float scale,
                                            hipStream_t st) {
   if (block_size <= 0) return (int)hipErrorInvalidValue;
-  return launch_prefill<true>(out, out_stride, qkv, row_stride, cu_seqlens, num_seqs,
+  return launch_prefill<true>(out, out_stride, qkv, row_stride, cu_seqlens, tokens, num_seqs,
                               max_seqlen, hq, hkv, hd, scale, ctx_lens, k_cache, v_cache,
                               block_tables, bt_stride, block_size, st);
 }
@@ -571,6 +590,12 @@ extern "C" int dli_prefill_set_min_len(int n) {
   const int old = g_pl_min_len;
   if (n > 0) g_pl_min_len = n;
   return old;
+}
+
+// 1 where such a launch takes waves of 64 rows (block_size 0: keys and values in the activation's rows)
+extern "C" int dli_prefill_takes_wave64(int tokens, int num_seqs, int max_seqlen, int hq, int hd, int row_stride,
+                                        int block_size) {
+  return takes_wave64(block_size > 0, tokens, num_seqs, max_seqlen, hq, hd, row_stride, block_size) ? 1 : 0;
 }
 
 extern "C" int dli_prefill_set_wave64_len(int n) {

@@ -547,7 +547,7 @@ def prefill_attention(qkv, cu_seqlens, max_seqlen: int, hq, hkv, hd, scale, out=
         out = torch.empty(T, hq * hd, dtype=qkv.dtype, device=qkv.device)
     nseq = cu_seqlens.shape[0] - 1
     _native_call("dli_prefill_attention", _p(out), out.stride(0), _p(qkv), qkv.stride(0),
-                 _p(cu_seqlens), nseq, max_seqlen, hq, hkv, hd, scale, _st())
+                 _p(cu_seqlens), T, nseq, max_seqlen, hq, hkv, hd, scale, _st())
     return out
 
 
@@ -577,7 +577,8 @@ def prefill_long_min_len(n: int = 0) -> int:
 
 def prefill_wave64_min_len(n: int = 0) -> int:
     """Shortest max_seqlen whose launches of more than 256 workgroups of 256 rows take the kernel with 64 rows a
-    wave; n > 0 sets it. Returns the previous value (A/B runs and tests)."""
+    wave; n > 0 sets it, and then whatever the other lengths are, but for the default (2048), which looks at these
+    too. Returns the previous value (A/B runs and tests)."""
     return int(N.require_native().dli_prefill_set_wave64_len(int(n)))
 
 
@@ -607,7 +608,7 @@ def prefill_attention_paged(qkv, cu_seqlens, max_seqlen: int, context_lens, bloc
     nseq = cu_seqlens.shape[0] - 1
     _native_call("dli_prefill_attention_paged", _p(out), out.stride(0), _p(qkv), qkv.stride(0),
                  _p(cu_seqlens), _p(context_lens), _p(k_cache), _p(v_cache), _p(block_tables),
-                 block_tables.stride(0), nseq, max_seqlen, hq, hkv, hd, k_cache.shape[2], scale,
+                 block_tables.stride(0), T, nseq, max_seqlen, hq, hkv, hd, k_cache.shape[2], scale,
                  _st())
     return out
 

@@ -41,15 +41,16 @@ _SIGS = {
     "dli_prefetch": [P, L, I, P, P],
     "dli_decode_attention": [P, P, I, P, P, P, I, P, I, I, I, I, I, F, I, I, P, P],
     "dli_decode_attention_workspace_bytes": [I, I, I, I],
-    "dli_prefill_attention": [P, I, P, I, P, I, I, I, I, I, F, P],
+    "dli_prefill_attention": [P, I, P, I, P, I, I, I, I, I, I, F, P],
     "dli_prefill_set_min_len": [I],
     "dli_prefill_set_wave64_len": [I],
+    "dli_prefill_takes_wave64": [I, I, I, I, I, I, I],
     "dli_prefill_set_pack": [I],
     "dli_sample_set_split_max_b": [I],
     "dli_decode_set_form": [I],
     "dli_gemm_set_slab_store": [I],
     "dli_gemm_set_slab_store_family": [I, I],
-    "dli_prefill_attention_paged": [P, I, P, I, P, P, P, P, P, I, I, I, I, I, I, I, F, P],
+    "dli_prefill_attention_paged": [P, I, P, I, P, P, P, P, P, I, I, I, I, I, I, I, I, F, P],
     "dli_sample": [P, P, L, I, I, P, P, P, P, P, P],
     "dli_sample_blocks": [P, P, L, I, I, P, P, P, P, P, I, I, P],
     "dli_sample_workspace_bytes": [I, I],

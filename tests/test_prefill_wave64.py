@@ -90,3 +90,26 @@ def test_rising_scores(gpu, both):
     qkv = qkv.bfloat16()
     new, old = both(lambda: ops.prefill_attention(qkv, cumulated(lens, gpu), 513, hq, hkv, HD, 1.0))
     assert torch.equal(new, old) and torch.isfinite(new.float()).all()
+
+
+# which launches take it: by the longest sequence and by what stands beside it (measured on both kernels, us)
+@pytest.mark.parametrize("lens,hq,paged,taken", [
+    ([2500], 32, False, True), ([2048], 32, False, False), ([2047] * 8, 32, False, False), ([2048] * 7, 32, False, True),
+    ([2100] + [353, 489, 330, 341, 433, 294, 207], 32, False, False),       # 76 / 80
+    ([2048] + [40] * 60, 32, False, False), ([2048] + [40] * 60, 8, False, False),      # 178 / 210
+    ([4096] + [300] * 7, 32, False, True), ([2100, 300], 32, False, True),              # 179 / 171, 62 / 57
+    ([2100] + [300] * 7, 8, False, True), ([2100] + [300] * 7, 64, False, False),       # 59 / 54, 136 / 145
+    ([8192] + [300] * 31, 32, False, True),
+    ([4096], 32, True, True), ([2048] * 4, 32, True, True), ([2048, 300], 32, True, True),
+    ([2048, 40], 32, True, False), ([2048] + [300] * 7, 32, True, False)])              # 217 / 263
+def test_choice_by_the_mix_of_lengths(lens, hq, paged, taken):
+    from distributed_llm_inferencing_amd.ops import _native
+    takes = _native.require_native().dli_prefill_takes_wave64
+    assert takes(sum(lens), len(lens), max(lens), hq, HD, (hq + 16) * HD, 16 if paged else 0) == taken
+    assert not takes(sum(lens), len(lens), max(lens), hq, 64, (hq + 16) * 64, 16 if paged else 0)
+    assert not paged or not takes(sum(lens), len(lens), max(lens), hq, HD, 0, 48)
+    try:
+        assert ops.prefill_wave64_min_len(1) == 2048
+        assert takes(sum(lens), len(lens), max(lens), hq, HD, (hq + 16) * HD, 16 if paged else 0) == (lens != [2048])
+    finally:
+        ops.prefill_wave64_min_len(2048)

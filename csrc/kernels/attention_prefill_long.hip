@@ -19,8 +19,6 @@
 // only barrier, once the last of V(t) is read, ends all three. Causal: a workgroup's tiles stop at its last row's
 // bound, a wave's at its own; only tiles that cross a wave's diagonal or the last key are masked.
 #include "common.h"
-#include <type_traits>
-#include <utility>
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
@@ -29,14 +27,6 @@ typedef __attribute__((address_space(3))) void lds_void;
 typedef const __attribute__((address_space(1))) void gbl_void;
 typedef const __attribute__((address_space(3))) bf16x8 lds_frag;
 
-template <int V> using int_c = std::integral_constant<int, V>;
-template <class F, int... U>
-__device__ __forceinline__ void unroll_seq(F f, std::integer_sequence<int, U...>) {
-  (f(int_c<U>{}), ...);
-}
-template <int N, class F> __device__ __forceinline__ void unroll(F f) {
-  unroll_seq(f, std::make_integer_sequence<int, N>{});
-}
 __device__ __forceinline__ float max3_raw(float a, float b, float c) {  // no canonicalise
   float r;
   asm volatile("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));

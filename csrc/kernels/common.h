@@ -13,6 +13,8 @@
 #include <hip/hip_runtime.h>
 #include <hip/hip_bf16.h>
 #include <stdint.h>
+#include <type_traits>
+#include <utility>
 
 #define DLI_WAVE 64
 
@@ -21,6 +23,16 @@ typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint16_t u16;
+
+template <int V> using int_c = std::integral_constant<int, V>;
+// f(0), f(1), .. f(N - 1) with compile-time arguments
+template <class F, int... U>
+__device__ __forceinline__ void unroll_seq(F f, std::integer_sequence<int, U...>) {
+  (f(int_c<U>{}), ...);
+}
+template <int N, class F> __device__ __forceinline__ void unroll(F f) {
+  unroll_seq(f, std::make_integer_sequence<int, N>{});
+}
 
 struct alignas(16) U16x8 { u16 v[8]; };
 struct alignas(8) U16x4 { u16 v[4]; };

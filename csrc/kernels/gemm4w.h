@@ -27,16 +27,6 @@ typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
 typedef const __attribute__((address_space(3))) bf16x8 lds_frag;
 
-template <int V> using int_c = std::integral_constant<int, V>;
-// f(0), f(1), .. f(N - 1) with compile-time arguments
-template <class F, int... U>
-__device__ __forceinline__ void unroll_seq(F f, std::integer_sequence<int, U...>) {
-  (f(int_c<U>{}), ...);
-}
-template <int N, class F> __device__ __forceinline__ void unroll(F f) {
-  unroll_seq(f, std::make_integer_sequence<int, N>{});
-}
-
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* p, int bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
 }
@@ -606,11 +596,13 @@ static int launch_4w(const void* A, int lda, const void* W, int ldw, void* C, in
   if (grid < 1) grid = 1;
   gemm4w_kernel<EPI, NJ><<<grid, 256, lds, st>>>((const u16*)A, lda, (const u16*)W, ldw, C, ldc, M, N, K, splits,
                                                  (const u16*)bias, (float*)ws, group_off, groups);
-  if (splits > 1 && C != nullptr) {
-    const int outN = epi_pairs(EPI) ? N / 2 : N;
-    const long total = (long)M * outN;
-    splitk_reduce_kernel<EPI><<<(int)((total + 255) / 256), 256, 0, st>>>(
-        C, ldc, (const float*)ws, M, N, splits, (const u16*)bias);
+  if constexpr (EPI != EPI_RES) {                  // (never split)
+    if (splits > 1 && C != nullptr) {
+      const int outN = epi_pairs(EPI) ? N / 2 : N;
+      const long total = (long)M * outN;
+      splitk_reduce_kernel<EPI><<<(int)((total + 255) / 256), 256, 0, st>>>(
+          C, ldc, (const float*)ws, M, N, splits, (const u16*)bias);
+    }
   }
   DLI_RETURN_LAUNCH();
 }

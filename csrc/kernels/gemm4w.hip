@@ -9,7 +9,6 @@
 // a bias 32 -> 23; partial sums in 16 bits of 512 rows: 6144 x 4096 in four 35.8 -> 27.0, 4096 x 4096 in four 26.5
 // (eight) -> 21.6, 4096 x 14336 in eight 60.9 -> 50.9.
 #include "gemm4w.h"
-#include <utility>
 
 int gemm_4w_narrow(int epi, int nj, DLI_GEMM_ARGS);
 

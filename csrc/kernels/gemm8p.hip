@@ -287,8 +287,7 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(
       for (int j = 0; j < 4; ++j) {
         const int col = wc0 + 16 * j + 4 * fq;
         if (col >= N) continue;
-        if (EPI == EPI_SLAB16) slab_quad16(srow + col, acc[i][j], vec, N - col, ws);
-        else slab_quad(srow + col, acc[i][j], sm, vec, N - col, ws);
+        slab_quad(srow + col, acc[i][j], sm, vec, N - col, ws);
       }
     }
     return;
@@ -774,8 +773,7 @@ __global__ void __launch_bounds__(512) gemm8p128_kernel(
       for (int j = 0; j < 4; ++j) {
         const int col = wc0 + 16 * j + 4 * fq;
         if (col >= N) continue;
-        if (EPI == EPI_SLAB16) slab_quad16(srow + col, acc[i][j], vec, N - col, ws);
-        else slab_quad(srow + col, acc[i][j], sm, vec, N - col, ws);
+        slab_quad(srow + col, acc[i][j], sm, vec, N - col, ws);
       }
     }
     return;

@@ -6,7 +6,6 @@
 // translation unit.
 #pragma once
 #include "common.h"
-#include <type_traits>
 
 
 #define BK 64

@@ -98,12 +98,12 @@ extern "C" int dli_gemm(const void* A, int lda, const void* W, int ldw, void* C,
   return r == DLI_NOT_MINE ? (int)hipErrorInvalidValue : r;
 }
 
-extern "C" int dli_gemm_persistent_width(int M, int N, int pairs);
+extern "C" int dli_gemm_4w_width(int tile_cfg, int epi, int M, int N, int splits);
 
 // columns of the blocks whose maxima dli_gemm_head can write for a tile; 0: not for this one
 static int head_block(int tile_cfg, int M, int N) {
   if (N % 4) return 0;
-  if (tile_cfg == 55) return dli_gemm_persistent_width(M, N, 0) / 2;
+  if (tile_cfg == 55) return dli_gemm_4w_width(55, EPI_F32, M, N, 1) / 2;
   if (tile_cfg == 30 || tile_cfg == 32) return M <= 4 ? 16 : 0;
   if (tile_cfg == 31 || tile_cfg == 33) return M <= 4 ? 32 : 0;
   switch (tile_cfg) {                              // columns of a wave tile

@@ -56,33 +56,37 @@ static int g_store_mode = 0;
 int gemm_4w_set_slab_store(int mode) { return std::exchange(g_store_mode, mode); }
 int gemm_4w_store_mode() { return g_store_mode; }
 
+// a tile's columns, in 32, for a product
+static int columns(int tile_cfg, int epi, int M, int N, int splits, bool grouped) {
+  if (tile_cfg == 28) return 4;
+  // (the biased epilogues, which few products take, are built in one width)
+  const bool bias_epi = epi == EPI_BIAS || epi == EPI_BIAS_GELU;
+  if ((tile_cfg != 22 && tile_cfg != 55) || grouped || bias_epi) return 8;
+  return width_of(M, N, splits, epi_pairs(epi), tile_cfg == 22);
+}
+
 int gemm_4w_dispatch(int epi, int tile_cfg, DLI_GEMM_ARGS) {
-  const bool pairs = epi_pairs(epi), bias_epi = epi == EPI_BIAS || epi == EPI_BIAS_GELU;
-  int nj = 8;
   switch (tile_cfg) {
     case 34: case 41: case 45:
       if (epi == EPI_GELU_MUL || epi == EPI_SLAB16) return DLI_NOT_MINE;
       break;
     case 22:
-      if (pairs && N % 64) return (int)hipErrorInvalidValue;
-      if (go == nullptr && !bias_epi) nj = width_of(M, N, splits, pairs, true);
+      if (epi_pairs(epi) && N % 64) return (int)hipErrorInvalidValue;
       break;
     case 28:
-      nj = 4;
       break;
     case 55:
       if (epi == EPI_SLAB16) return DLI_NOT_MINE;
       if (splits != 1 || go != nullptr || K % (2 * BK) || C == nullptr) return (int)hipErrorInvalidValue;
-      // (the biased epilogues, which few products take, are built in one width)
-      if (!bias_epi) nj = width_of(M, N, 1, pairs, false);
       break;
     default: return DLI_NOT_MINE;
   }
   if (epi == EPI_SLAB16 && (C != nullptr || splits < 2)) return (int)hipErrorInvalidValue;
+  const int nj = columns(tile_cfg, epi, M, N, splits, go != nullptr);
   return nj == 8 ? launch8(epi, DLI_GEMM_PASS) : gemm_4w_narrow(epi, nj, DLI_GEMM_PASS);
 }
 
-// the columns of the tiles that tile 55 takes for a product
-extern "C" int dli_gemm_persistent_width(int M, int N, int pairs) {
-  return 32 * width_of(M, N, 1, pairs != 0, false);
+// the columns that a tile (22, 28, 34, 41, 45 or 55) has for a dense product
+extern "C" int dli_gemm_4w_width(int tile_cfg, int epi, int M, int N, int splits) {
+  return 32 * columns(tile_cfg, epi, M, N, splits, false);
 }

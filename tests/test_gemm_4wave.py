@@ -51,31 +51,51 @@ def test_products(gpu, M, N, K, splits, tile):
         assert off(got, expected(x, w[0], epi, bias)) < BOUND[epi == "f32"], epi
 
 
-# partial sums in 16 bits on tiles of every width that tile 22 takes (a third column: the last tiles' columns); half
-# an ulp (2^-11) of each of the slices, whose squares add up to the sum's
+# partial sums in 16 bits on tiles of every width that tile 22 takes; half an ulp (2^-11) of each of the slices, whose
+# squares add up to the sum's; nothing behind the last slab
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K,splits", [(300, 15000, 256, 2), (300, 12808, 256, 2), (512, 6144, 1024, 4), (300, 10244, 384, 2),
-                                          (512, 4096, 1024, 4), (257, 1001, 512, 8)])
+@pytest.mark.parametrize("M,N,K,splits,width", [
+    (300, 15000, 256, 2, 256), (300, 12808, 256, 2, 224), (512, 6144, 1024, 4, 192), (300, 10244, 384, 2, 192),
+    (512, 4096, 1024, 4, 128), (257, 1001, 512, 8, 128), (300, 9000, 256, 2, 160)])
 @pytest.mark.parametrize("tile", [22, 28])
-def test_partial_sums_in_16_bits(gpu, M, N, K, splits, tile):
+def test_partial_sums_in_16_bits(gpu, M, N, K, splits, width, tile):
     x, w = operands(gpu, M, N, K, M + N)
-    ws = torch.zeros(splits, M, N, device=gpu, dtype=torch.float16)
+    from distributed_llm_inferencing_amd.ops import _native
+    assert _native.require_native().dli_gemm_4w_width(tile, G.EPI["slab16"], M, N, splits) == (128 if tile == 28 else width)
+    held = torch.full((splits * M + 256, N), 7.0, device=gpu, dtype=torch.float16)
+    ws, behind = held[:splits * M].view(splits, M, N), held[splits * M:]
     ops._native_call("dli_gemm", ops._p(x), K, ops._p(w), K, None, N, M, N, K, G.EPI["slab16"], tile, splits, None,
                      ops._p(ws), None, 1, ops._st())
-    assert off(ws.double().sum(0) * 16, expected(x, w[0], "none")) < 2.0 ** -11
+    assert off(ws.double().sum(0) * 16, expected(x, w[0], "none")) < 2.0 ** -11 and torch.all(behind == 7)
 
 
-# outputs inside a wider buffer, whole and odd offsets: nothing beside the product is written
+# outputs inside a wider buffer, whole and odd offsets: nothing beside the product is written, nor behind it, where a tile's
+# rows go on (up to 255 of them)
 @pytest.mark.gpu
 @pytest.mark.parametrize("tile", TILES)
-@pytest.mark.parametrize("M,N,wide,at", [(300, 264, 512, 8), (300, 264, 516, 4), (257, 260, 301, 3), (513, 512, 520, 0)])
+@pytest.mark.parametrize("M,N,wide,at", [(300, 264, 512, 8), (300, 264, 516, 4), (257, 260, 301, 3), (513, 512, 520, 0),
+                                         (1, 264, 512, 8), (17, 264, 264, 0), (300, 30000, 30000, 0), (257, 1000, 1000, 0)])
 @pytest.mark.parametrize("epi", ["none", "f32"])
 def test_outputs_inside_wider_rows(gpu, M, N, wide, at, epi, tile):
     x, w = operands(gpu, M, N, 192, M + wide)
-    whole = torch.full((M, wide), 7.0, device=gpu, dtype=torch.float32 if epi == "f32" else torch.bfloat16)
-    ops._gemm_native(x, w[0], epi, out=whole[:, at:at + N], plan=G.GemmPlan("dli", tile, 1))
-    assert off(whole[:, at:at + N], expected(x, w[0], epi)) < BOUND[epi == "f32"]
-    assert torch.all(whole[:, :at] == 7) and torch.all(whole[:, at + N:] == 7)
+    whole = torch.full((M + 256, wide), 7.0, device=gpu, dtype=torch.float32 if epi == "f32" else torch.bfloat16)
+    ops._gemm_native(x, w[0], epi, out=whole[:M, at:at + N], plan=G.GemmPlan("dli", tile, 1))
+    assert off(whole[:M, at:at + N], expected(x, w[0], epi)) < BOUND[epi == "f32"]
+    whole[:M, at:at + N] = 7
+    assert torch.all(whole == 7)
+
+
+# fp32 partial sums: nothing behind the last slab
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("M,N,K,splits", [(1, 264, 128, 2), (17, 260, 256, 4), (257, 1001, 512, 8), (300, 1000, 384, 2)])
+def test_partial_sums(gpu, M, N, K, splits, tile):
+    x, w = operands(gpu, M, N, K, M + N)
+    held = torch.full((splits * M + 256, N), 7.0, device=gpu)
+    ops._native_call("dli_gemm", ops._p(x), K, ops._p(w), K, None, N, M, N, K, G.EPI["none"], tile, splits, None,
+                     ops._p(held), None, 1, ops._st())
+    assert off(held[:splits * M].view(splits, M, N).double().sum(0), expected(x, w[0], "none")) < BOUND[True]
+    assert torch.all(held[splits * M:] == 7)
 
 
 @pytest.mark.gpu

@@ -83,11 +83,12 @@ def test_products_on_fitted_plans(gpu, M, N, K, epi):
 @pytest.mark.gpu
 def test_persistent_tile_widths_are_the_kernels(gpu):
     from distributed_llm_inferencing_amd.ops import _native
-    width = _native.require_native().dli_gemm_persistent_width
+    width = _native.require_native().dli_gemm_4w_width
     for M in (1, 256, 257, 1290, 2112, 2816, 4352, 5000, 8199):
         for N in (32, 160, 4096, 4100, 6144, 14336, 28672):
             for pairs in (False, True):
-                assert G.persistent_width(M, N, pairs, G.device_cus()) == width(M, N, int(pairs)), (M, N, pairs)
+                assert G.persistent_width(M, N, pairs, G.device_cus()) == width(
+                    55, G.EPI["silu_mul" if pairs else "none"], M, N, 1), (M, N, pairs)
 
 
 # 17 x 16 = 272 tiles of 256 columns: a second round of 256 CUs, hardly filled, but one of 272 and of 304

@@ -23,18 +23,29 @@ def close(got, x, w, before):
     return bool(((got.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + (x.shape[1] + 1) * 2.0 ** -24 * size).all())
 
 
-# edges of the 256-row tile and its waves, of 16 columns and each tile width, K of one, two, three and more K-tiles
+SIZES = [(1, 8, 64), (17, 24, 128), (128, 264, 64), (129, 136, 192), (255, 248, 256), (256, 256, 128), (257, 1000, 128),
+         (300, 520, 640), (700, 4104, 256), (2112, 4096, 128), (257, 24008, 192), (300, 28008, 128), (513, 32776, 64)]
+
+
+# the sizes below are on tiles of every width that the kernel has
+def test_widths():
+    from distributed_llm_inferencing_amd.ops import _native as N
+    width = lambda tile: {N.require_native().dli_gemm_4w_width(tile, G.EPI["res_add"], m, n, 1) for m, n, _ in SIZES}
+    assert width(22) == {128, 160, 192, 224, 256} and width(55) == {160, 192, 256} and width(28) == {128} and width(45) == {256}
+
+
+# edges of the 256-row tile and its waves, of 16 columns and each tile width, K of one, two, three and more K-tiles.
+# A tile's rows past the product's, up to 255, are kept off what follows it by a descriptor's range
 @pytest.mark.gpu
 @pytest.mark.parametrize("tile", [45, 22, 28, 55])
-@pytest.mark.parametrize("M,N,K", [(1, 8, 64), (17, 24, 128), (128, 264, 64), (129, 136, 192), (255, 248, 256), (256, 256, 128),
-                                   (257, 1000, 128), (300, 520, 640), (700, 4104, 256), (2112, 4096, 128)])
+@pytest.mark.parametrize("M,N,K", SIZES)
 def test_sums(gpu, tile, M, N, K):
     if tile == 55 and K % 128:
         K += 64
     g = torch.Generator(device=gpu).manual_seed(M)
     x = torch.randn(M, K, device=gpu, generator=g).bfloat16()
     w = torch.randn(N, K, device=gpu, generator=g).bfloat16()
-    held = torch.randn(M + 2, N + 16, device=gpu, generator=g).bfloat16()
+    held = torch.randn(M + 257, N + 16, device=gpu, generator=g).bfloat16()
     before = held.clone()
     assert call(x, w, held[1:, 8:], tile) == 0
     assert close(held[1:M + 1, 8:N + 8], x, w, before[1:M + 1, 8:N + 8])

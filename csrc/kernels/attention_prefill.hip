@@ -493,8 +493,8 @@ int launch_prefill_long(void* out, int out_stride, const void* qkv, int row_stri
                         int max_seqlen, int hq, int hkv, float scale_log2, const int* ctx_lens, const void* k_cache,
                         const void* v_cache, const int* block_tables, int bt_stride, int block_size, hipStream_t st);
 
-// Whether a launch takes waves of 64 rows. They gain on long sequences (2500 tokens 75 -> 69 us, 7993 511 -> 473, 7 x
-// 2048 303 -> 289) and lose on short ones, whose last waves they leave idle (1000 tokens equal, 500 161 -> 174, 300 180
+// Whether a launch takes waves of 64 rows. They gain on long sequences (2500 tokens 77 -> 69.5 us, 7993 516 -> 471, 7
+// x 2048 306 -> 291) and lose on short ones, whose last waves they leave idle (1000 tokens equal, 500 161 -> 174, 300 180
 // -> 222), and by every block, which has a CU to itself. One round of workgroups is for the other kernel, which pairs
 // blocks: 2048 51 / 58. The lengths themselves lie on the device. In the activation's rows, with T tokens, n
 // sequences and the longest L, the mean length over the tokens is at least low, that of n - 1 equal others; where low

@@ -11,8 +11,8 @@
 // max3, 48 LDS reads, 8 LDS-DMA pieces; none alone is worth more than 10 %). The kernel of 8 waves of 32 rows, which
 // met at a barrier a tile, read K and V from LDS twice as often and did products and softmax by turns. Here the
 // products S(t + 1) run beside the exponentials of tile t, the products with V(t) beside the last of them and the
-// maxima of t + 1. 32 heads on 8, us, that kernel / this one: 3000 tokens 88 / 81, 7993 511 / 473, 16000 1941 / 1775, 4 x 4096
-// 587 / 539, 4096 of 8192 cached 416 / 389. Outputs are equal to the bit.
+// maxima of t + 1. 32 heads on 8, us, that kernel / this one: 3000 tokens 97 / 87, 7993 516 / 471 (1.11 PFLOP/s), 16000 1930 / 1718, 4
+// x 4096 577 / 525; on another card 4096 of 8192 cached 416 / 389. Outputs are equal to the bit.
 //
 // K and V tiles come by LDS-DMA into rings of three slots, rows past the keys as zeros (range-checked descriptors).
 // In iteration t K(t + 1) and V(t) are read, K(t + 2) and V(t + 1) land, K(t + 3) and V(t + 2) are requested; the

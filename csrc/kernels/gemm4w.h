@@ -17,9 +17,9 @@
 // The tile's epilogue was 20 k of 170 k cycles at K = 4096 (bounds by branches, 8-byte stores, a division a
 // SiLU, and a wait for all of its stores): now stores of 16 bytes a lane through range-checked descriptors that
 // nothing waits for until the tile's second K-tile. Both against a schedule of reads and pieces in bursts and
-// the former epilogue, us: 16384 x 6144 x 4096 557 -> 530 (1.55 PFLOP/s), 8192 x 4096 x 4096 182 -> 175 and x 14336
-// 645 -> 625, 8192 x 28672 x 4096 with SiLU pairs 1271 -> 1217. With fp32 outputs 188 -> 185: all CUs store 67 MB at
-// once, at 6.4 TB/s, behind which the next tile's pieces wait.
+// the former epilogue, us, one card (others run 3 to 4 % faster): 16384 x 6144 x 4096 570 -> 540 (1.53 PFLOP/s), 8192 x
+// 4096 x 4096 191 -> 182 and x 14336 655 -> 629, 8192 x 28672 x 4096 with SiLU pairs 1295 -> 1249 (1.54). fp32 outputs
+// of 8192 x 4096 x 4096 gain nothing (189): all CUs store 67 MB at once, at 6.4 TB/s, behind which the next tile's pieces wait.
 #pragma once
 #include "gemm_common.h"
 
@@ -53,8 +53,8 @@ __device__ __forceinline__ void dma16(const void* base, int bytes, uint32_t lds,
 //   D, D + DS, ..       a DMA piece of the K-tile after the next into it, NP of them
 //   B2                  the next K-tile landed (the pieces just issued may fly) for every wave
 //   B2 + 1, + 3, ..     a fragment of the next K-tile's F0 each
-// Positions by measurement (8192 x 4096 x 4096, 16384 x 4096 x 14336, us): reads one or two MFMAs apart 185.9 / 187.3
-// and 1298 / 1296; pieces 5 instead of 6 apart 185.4 and 1313.
+// Positions by measurement, times of 8192 x 4096 x 4096 and 16384 x 4096 x 14336 against these: reads one MFMA apart
+// instead of two -0.7 % and +0.2 %, pieces 5 instead of 6 apart -1.0 % and +1.3 %.
 template <int NJ> struct Sched4w {
   static constexpr int Q = 16 * NJ, NF = 8 + NJ, NP = 8 + NJ;
   static constexpr int B1 = NF + 3 + NJ / 3, D = B1 + 1, DS = (Q - 4 - D) / (NP - 1), DL = D + DS * (NP - 1);

@@ -4,10 +4,10 @@
 //   22          256 columns, or by rounds as below where the product is dense and not biased
 //   28          128 columns
 //   55          256, 192 or 160 by rounds; dense, unsplit, K a multiple of 128
-// Against the 8-phase kernels that 22 and 28 were (gemm8p.hip keeps what is not built here), us: 16384 x 6144 x 4096
-// 595 -> 533, 8192 x 4096 x 14336 664 -> 631, 8192 x 28672 with SiLU pairs 1318 -> 1231, 4096 x 2304 x 768 with
-// a bias 32 -> 23; partial sums in 16 bits of 512 rows: 6144 x 4096 in four 35.8 -> 27.0, 4096 x 4096 in four 26.5
-// (eight) -> 21.6, 4096 x 14336 in eight 60.9 -> 50.9.
+// Against the 8-phase kernels that 22 and 28 were (gemm8p.hip keeps what is not built here), us, on gemm4w.h's card:
+// 16384 x 6144 x 4096 591 -> 540, 8192 x 4096 x 14336 663 -> 632, 8192 x 28672 with SiLU pairs 1348 -> 1248, 4096 x
+// 2304 x 768 with a bias 33 -> 24.5; partial sums in 16 bits of 512 rows: 6144 x 4096 in four 32.4 -> 26.0, 4096 x
+// 4096 in four 23.0 (tile 28) -> 19.5, 4096 x 14336 in eight 52 -> 47.
 #include "gemm4w.h"
 
 int gemm_4w_narrow(int epi, int nj, DLI_GEMM_ARGS);

@@ -838,10 +838,11 @@ def moe_mlp(x, w_gu, w_down, topk_w, topk_ids, expert_offset: int = 0,
         return _H.act_mul(a, Fa, x.dtype, "clamp_swish", rows=offsets[E_local:], limit=limit)
     if n >= _MOE_PREFILL_ROWS * E_local and not torch.cuda.is_current_stream_capturing():
         # prefill-sized expert GEMMs (thousands of rows per expert) are compute-bound: a
-        # grouped 256x256 kernel (G.MOE_PREFILL_TILE: the two-barrier 4-wave tile, grid.z =
-        # expert) with the fused SiLU*up epilogue. The largest expert's row count bounds the
-        # grid (one host read of the offsets per MoE layer, eager prefill only) instead of n,
-        # which would launch ~8x more (empty) row tiles per expert.
+        # grouped 256x256 kernel (G.MOE_PREFILL_TILE: the 4-wave kernel, whose workgroups walk the
+        # experts' tiles) with the fused SiLU*up epilogue. The largest expert's row count (one host
+        # read of the offsets per MoE layer, eager prefill only) bounds the grid where it is below
+        # a workgroup a CU, and the row tiles of the 8-phase kernel, an expert a grid.z, where
+        # n would launch ~8x more (empty) ones.
         xp = torch.empty(max(n, 1), D, dtype=x.dtype, device=dev)
         _native_call("dli_moe_gather", _p(xp), _p(x), _p(src), n, D, _p(offsets[E_local:]),
                      _st())

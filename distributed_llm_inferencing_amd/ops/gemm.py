@@ -81,9 +81,10 @@ GEMV_PRO_TILES = {"silu_mul": (29, 31, 33, 58, 59), "splitk": (30, 32, 56, 57),
                   "none": (30, 32, 56, 57)}
 GEMV_PRO_M1_ONLY = (32, 33)
 DEFER_NORM = os.environ.get("DLI_DEFER_NORM", "1") == "1"
+# waves down and across a tile where they are not 2 x 2
 TILE_WAVES = {13: (2, 4), 14: (4, 2), 15: (2, 4), 16: (4, 2), 17: (2, 4),
-              22: (2, 4), 23: (2, 4), 24: (2, 4), 25: (4, 2),
-              26: (4, 2), 28: (4, 2), 60: (2, 1), 66: (1, 4), 68: (2, 4), 69: (4, 1), 72: (4, 1)}
+              23: (2, 4), 24: (2, 4), 25: (4, 2),
+              26: (4, 2), 60: (2, 1), 66: (1, 4), 68: (2, 4), 69: (4, 1), 72: (4, 1)}
 
 
 def tile_shape(tile: int):
@@ -266,12 +267,11 @@ def _heuristic(M: int, N: int, K: int, epi: str) -> GemmPlan:
             while (tiles * splits * 2 <= NUM_CUS and K % (64 * splits * 2) == 0
                    and K // (splits * 2) >= 1024 and splits < 4):
                 splits *= 2
-        # 55 and 22 run one kernel, 55 on 256, 192 or 160 columns, 22 on 224 and 128 too, with any K, with splits
-        # and, where biased, on 256. So they are equal where both choose 256 (8192 rows, K = 4096, us: N = 4096 185,
-        # 6144 275, 28672 1253), and 22 is ahead where 128 or 224 columns fill a round (1536 x 4096, K = 4096 48
-        # against 51, 1024 x 8192 pairs, K = 1024 19.9 against 20.7), 55 by the last per cents where 22 takes 224
-        # (4352 x 4096, K = 14336 380 against 391). The lines below are from kernels that differed more and cost
-        # at most that
+        # 55 and 22 run one kernel (gemm4w.h), 55 on 256, 192 or 160 columns, 22 on 224 and 128 too, with any K, with
+        # splits and, where biased, on 256. So they are equal where both choose one width (8192 x 6144, K = 4096 268
+        # us, 4352 x 4096, K = 14336 371), and 22 is ahead where 128 or 224 columns fill a round better (1536 x 4096,
+        # K = 4096 48 against 53, 1024 x 8192 pairs, K = 1024 18 against 22). The lines below are from kernels that
+        # differed more: they cost up to that where they name 55
         if epi in PAIR_EPIS:
             pays = K > 2048 or (K >= 1024 and tiles > NUM_CUS) or N % 64 != 0   # (tile 22 takes no such N)
         else:

@@ -86,7 +86,7 @@ def test_gemm_bf16_all_tiles(gpu, M, N, K):
 @pytest.mark.parametrize("M,N,K,epi", [(512, 28672, 4096, "silu_mul"), (500, 2240, 14336, "none"),
                                        (1000, 7168, 1024, "f32"), (512, 4096, 14336, "none")])
 def test_gemm_256x224_pingpong(gpu, M, N, K, epi, tile):
-    """Tiles 26 (256x224 ping-pong) and 28 (256x128 ping-pong) at the Llama-3 gate/up and
+    """Tiles 26 (256x224 ping-pong) and 28 (256x128, 4 waves) at the Llama-3 gate/up and
     down decode shapes and with long K / partial M tiles, against the fp32 reference."""
     torch.manual_seed(5)
     x, w = rnd(M, K, dev=gpu), rnd(N, K, dev=gpu, scale=0.05)
@@ -107,7 +107,7 @@ def test_gemm_256x224_pingpong(gpu, M, N, K, epi, tile):
                                        (1100, 4096, 14336, "none"), (777, 50257, 4096, "f32"),
                                        (300, 2304, 768, "bias_gelu")])
 def test_gemm_4wave_persistent(gpu, M, N, K, epi):
-    """Tile 55: the two-barrier 4-wave kernel as a persistent grid (one workgroup per CU walks
+    """Tile 55: the 4-wave kernel as a persistent grid (one workgroup per CU walks
     tiles; the next tile's first K-tiles are staged in the current tile's last two). Shapes
     with one tile per workgroup (M = 2048 QKV: 192 tiles), many (gate/up at 8192: 3,584
     tiles, 14 per workgroup), partial row / column tiles and every epilogue, against the fp32
@@ -300,7 +300,7 @@ def test_gemv_norm_prologue(gpu, M, N, K, epi):
 
 def test_prefill_autotune_pins_a_correct_plan(gpu):
     """StageRunner.autotune_prefill's measurement (ops.gemm.autotune over prefill_candidates:
-    our 8-phase kernel vs hipBLASLt) pins one plan per shape, and whichever it pins computes
+    the 4-wave kernel's widths) pins one plan per shape, and whichever it pins computes
     each consumer (plain, SiLU*up, add + RMSNorm) like the fp32 reference."""
     torch.manual_seed(14)
     G.clear_plans()
@@ -868,8 +868,8 @@ def test_grouped_gemm_all_tiles_and_splitk(gpu, epi):
 @pytest.mark.parametrize("tile", [22, 45])
 def test_moe_mlp_prefill_grouped_path(gpu, monkeypatch, tile):
     """Prefill-sized MoE (rows per expert above the threshold) takes the grouped 256x256
-    path (grid bounded by the largest expert's rows) on the 8-phase (22) or the two-barrier
-    4-wave tile (45, the default); same result as the reference."""
+    path (grid bounded by the largest expert's rows) of the 4-wave kernel
+    by either of its ids (22, or 45, the default); same result as the reference."""
     monkeypatch.setattr(ops, "_MOE_PREFILL_ROWS", 16)
     monkeypatch.setattr(ops.G, "MOE_PREFILL_TILE", tile)
     torch.manual_seed(13)

@@ -272,7 +272,7 @@ def test_decode_core_matches_python_scheduler():
 
 
 def test_prefill_gemm_plan_is_own_kernel(monkeypatch):
-    """Prefill-sized GEMMs plan onto the 8-phase MFMA kernel (tile 22); every plan the
+    """Prefill-sized GEMMs plan onto the 4-wave MFMA kernel (tile 22); every plan the
     planner or the autotune can produce is one of our kernels (no library backend left)."""
     from distributed_llm_inferencing_amd.ops import gemm as G
     G.clear_plans()
@@ -286,7 +286,7 @@ def test_prefill_gemm_plan_is_own_kernel(monkeypatch):
     assert G.plan(1024, 4096, 4096, "splitk") == G.GemmPlan("dli", 22, 4)      # 64 tiles
     assert G.plan(1200, 28672, 4096, "silu_mul").splits == 1
     assert all(p.backend == "dli" for p in G.candidate_plans(512, 4096, 4096, "none"))
-    # mixed prefill+decode steps of a full batch (512 < M < 1024): 8-phase tiles, and one
+    # mixed prefill+decode steps of a full batch (512 < M < 1024): 256-row tiles, and one
     # plan-cache bucket per 128 rows (tuned when serving: StageRunner.autotune_mixed)
     assert G.plan(800, 28672, 4096, "silu_mul") == G.GemmPlan("dli", 22, 1)
     assert G.plan(600, 4096, 14336, "splitk").tile == 22
@@ -305,9 +305,8 @@ def test_prefill_gemm_plan_is_own_kernel(monkeypatch):
     assert not any(p.tile == 29 for p in G.candidate_plans(1, 4096, 4096, "splitk"))
     assert not any(p.tile == 29 for p in G.candidate_plans(8, 28672, 4096, "silu_mul"))
     G.clear_plans()
-    # prefill autotune (StageRunner.autotune_prefill): our 8-phase plan vs our 4-wave plan at
-    # the same split
-    # (and the persistent 4-wave tile 55 where the plan is unsplit and K an even K-tile count)
+    # prefill autotune (StageRunner.autotune_prefill): tile 22's width vs 256 columns at the same split
+    # (and tile 55's where the plan is unsplit and K an even K-tile count)
     c = G.prefill_candidates(16384, 28672, 4096, "silu_mul")
     t4 = G.PREFILL_4W_TILE
     assert c == [G.GemmPlan("dli", 22, 1), G.GemmPlan("dli", t4, 1), G.GemmPlan("dli", 55, 1)]

@@ -237,7 +237,7 @@ def _gemm_native(x, w, epi: str, bias=None, out=None, plan: Optional[G.GemmPlan]
     if splits > 1:
         ws = G.workspace(x.device, splits * M * Nn * 4)
     m_arg = M if group_off is None else rows_per_group
-    (x, lda), (w, ldw) = G.spaced(x, plan.tile), G.spaced(w, plan.tile)
+    x, lda, w, ldw = G.spaced(x, w, plan.tile)
     _native_call("dli_gemm", _p(x), lda, _p(w), ldw, _p(out), out.stride(0),
                  m_arg, Nn, K, G.EPI[epi], plan.tile, splits, _p(bias), _p(ws), _p(group_off),
                  groups, _st())
@@ -295,7 +295,7 @@ def _slab_gemm(x, w, p: G.GemmPlan, ws) -> int:
     M, K = x.shape
     Nn = w.shape[0]
     fmt = 1 if (G.SLAB16 and p.tile in G.SLAB16_TILES and p.splits in (2, 4, 8)) else 0
-    (x, lda), (w, ldw) = G.spaced(x, p.tile), G.spaced(w, p.tile)
+    x, lda, w, ldw = G.spaced(x, w, p.tile)
     _native_call("dli_gemm", _p(x), lda, _p(w), ldw, None, Nn, M, Nn, K,
                  G.EPI["slab16"] if fmt else 0, p.tile, p.splits, None, _p(ws), None, 1, _st())
     return fmt
@@ -310,16 +310,10 @@ def _splitk_plan(x, w):
     return p if p.splits > 1 else None
 
 
-def _extent(t) -> tuple:
-    """(first, past the last) byte that a tensor's elements lie in."""
-    last = sum((n - 1) * s for n, s in zip(t.shape, t.stride()))
-    return t.data_ptr(), t.data_ptr() + (last + 1) * t.element_size()
-
-
-def _apart(a, b) -> bool:
-    """Whether two tensors share no byte."""
-    (a0, a1), (b0, b1) = _extent(a), _extent(b)
-    return a1 <= b0 or b1 <= a0
+def _apart(whole, t) -> bool:
+    """Whether a contiguous bf16 tensor shares no byte with a bf16 matrix, whose columns lie side by side."""
+    a, b = whole.data_ptr(), t.data_ptr()
+    return a + 2 * whole.numel() <= b or b + 2 * ((t.shape[0] - 1) * t.stride(0) + t.shape[1]) <= a
 
 
 def _add_product(x, w, residual, plan: Optional[G.GemmPlan]) -> bool:
@@ -328,10 +322,10 @@ def _add_product(x, w, residual, plan: Optional[G.GemmPlan]) -> bool:
     again there. Not where the residual is an operand too, in part even: tiles are stored while others are still
     read. 4096 columns, us with the norm behind it, apart / so: K = 4096, 16384 rows 458 / 433, 7993 223 / 207,
     2112 73 / 71; K = 14336 1350 / 1326, 676 / 660, 204 / 200. Few rows take split plans and their fused reduce."""
-    if not (_use_native(x) and x.dtype == w.dtype == residual.dtype == torch.bfloat16 and w.dim() == 2):
-        return False
     (M, K), Nn = x.shape, w.shape[0]
-    if (M < G.LARGE_M or w.shape[1] != K or residual.shape != (M, Nn) or not residual.is_contiguous() or Nn % 8
+    if M < G.LARGE_M or not (_use_native(x) and x.dtype == w.dtype == residual.dtype == torch.bfloat16 and w.dim() == 2):
+        return False
+    if (w.shape[1] != K or residual.shape != (M, Nn) or not residual.is_contiguous() or Nn % 8
             or residual.data_ptr() % 16 or x.stride(-1) != 1 or w.stride(-1) != 1 or Nn >= G.MAX_4W_STRIDE // 2 - 1024
             or not x.device == w.device == residual.device or not (_apart(residual, x) and _apart(residual, w))):
         return False
@@ -340,9 +334,11 @@ def _add_product(x, w, residual, plan: Optional[G.GemmPlan]) -> bool:
     p = plan or G.plan(rows, Nn, K, "none")
     if p.splits != 1 or p.tile not in G.RES_ADD_TILES or rows < G.LARGE_M:
         return False
-    _gemm_native(x[:rows], w, "res_add", out=residual[:rows], plan=p)
     if cut:
+        _gemm_native(x[:cut], w, "res_add", out=residual[:cut], plan=p)
         residual[cut:].add_(linear(x[cut:], w))
+    else:
+        _gemm_native(x, w, "res_add", out=residual, plan=p)
     return True
 
 
@@ -706,7 +702,7 @@ def head(h, w):
         return linear(h, w, epi=HEAD_EPI), None
     out = torch.empty(M, Nn, dtype=torch.float32, device=h.device)
     keys = torch.empty(M, -(-Nn // bw), dtype=torch.int32, device=h.device)
-    (h, lda), (w, ldw) = G.spaced(h, tile), G.spaced(w, tile)
+    h, lda, w, ldw = G.spaced(h, w, tile)
     _native_call("dli_gemm_head", _p(h), lda, _p(w), ldw, _p(out), Nn, M, Nn,
                  h.shape[1], tile, _p(keys), _st())
     return out, (keys, bw)

@@ -128,14 +128,18 @@ RES_ADD_TILES = frozenset((22, 28, 34, 41, 45, 55))
 MAX_4W_STRIDE = 1 << 22
 
 
-def spaced(t: torch.Tensor, tile: int):
-    """(an operand, its row stride) as the tile's kernel takes them: the 4-wave kernel reads a tile's rows by offsets
-    within their range and so needs them at least their length apart, and not too far. Rows that overlap (expanded
-    ones, windows) are copied; one row has no stride."""
-    ld, n = t.stride(-2), t.shape[-1]
-    if tile not in RES_ADD_TILES or n <= ld < MAX_4W_STRIDE:
-        return t, ld
-    return (t, n) if t.shape[-2] == 1 else (t.contiguous(), n)
+def spaced(x: torch.Tensor, w: torch.Tensor, tile: int):
+    """(x, its row stride, w, its row stride) as the tile's kernel takes them: the 4-wave kernel reads a tile's rows by
+    offsets within their range and so needs them at least their length apart, and not too far. Rows that overlap
+    (expanded ones, windows) are copied; one row has no stride."""
+    lda, ldw = x.stride(0), w.stride(-2)
+    if tile in RES_ADD_TILES:
+        n = x.shape[1]
+        if not n <= lda < MAX_4W_STRIDE:
+            x, lda = (x, n) if x.shape[0] == 1 else (x.contiguous(), n)
+        if not n <= ldw < MAX_4W_STRIDE:
+            w, ldw = (w, w.shape[-1]) if w.shape[-2] == 1 else (w.contiguous(), w.shape[-1])
+    return x, lda, w, ldw
 
 
 # epilogues over the interleaved gate/up weight: the output is half as wide

@@ -89,7 +89,7 @@ def linear_out(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         p = _gemm.plan(M, Nn, K, "f32")
         if p.splits > 1:
             ws = _gemm.workspace(x.device, p.splits * M * Nn * 4)
-            (x, lda), (w, ldw) = _gemm.spaced(x, p.tile), _gemm.spaced(w, p.tile)
+            x, lda, w, ldw = _gemm.spaced(x, w, p.tile)
             _call("dli_gemm", _p(x), lda, _p(w), ldw, None, Nn, M, Nn, K,
                   _gemm.EPI["f32"], p.tile, p.splits, None, _p(ws), None, 1, _st())
             return ws[:p.splits * M * Nn * 4].view(torch.float32).view(p.splits, M, Nn)

@@ -6,8 +6,8 @@
 // budget sets; with this tile's 32 fragment reads and 16 LDS-DMA pieces a K-tile at 1.75 GHz and 17.6
 // cycles an MFMA (1.68, operands in the L2). So what costs is (a) cycles in which the matrix pipe waits
 // and (b) energy beside the MFMAs; a cycle saved gives about 0.6 of itself, the clock gives the rest back.
-// 32x32x16 MFMAs, half the instructions, hold 1.73 GHz and 1.81 PFLOP/s alone: not used. Consecutive MFMAs share
-// the activation fragment (a new pair of fragments each time costs 4 % of the clock).
+// 32x32x16 MFMAs, half the instructions, hold 1.73 GHz and 1.81 PFLOP/s alone: not used. The order in which a wave
+// takes its blocks (Walk4w) is about (b) alone.
 //
 // (a) is this schedule's business; measured amid MFMAs of 16 cycles, one wave a SIMD: an LDS-DMA piece
 // costs 2 to 4 cycles, every scalar instruction beside it 4, vector ones nothing. So a lane's offsets advance by
@@ -61,6 +61,21 @@ template <int NJ> struct Sched4w {
   static constexpr int B2 = Q - 1 - 2 * NF;
   static constexpr int ahead = B2 < D ? 0 : (B2 - D) / DS + 1;      // pieces issued when B2 waits
   static_assert(DS >= 1 && DL + 2 < Q && B2 > B1 && ahead <= NP, "the pieces fit the K-tile");
+};
+
+// The u-th block of a half K-tile: two rows of blocks down, then up, column after column, and back on the next two,
+// so that each MFMA shares one of its two fragments with the one before and each of both is taken anew every other
+// time (the first columns need W's first fragments and A's first two, in the order in which they are read). The sums are
+// the same. us against row after row, a step as much as 4 % ahead of a new pair each time, one card: 8192 x 28672 x 4096
+// with SiLU pairs 1250 -> 1226 (1.57 PFLOP/s), 8192 x 6144 x 4096 272 -> 268, 8192 x 4096 x 14336 642 -> 634, 512 x
+// 128256 x 4096 421 -> 409. Rows back and forth give 0.8 %, columns likewise 0.8, three rows at a time 1.4, four
+// 1.2, two columns 1.6 and a Hilbert curve 1.7, against this one's 1.6.
+template <int NJ> struct Walk4w {
+  static constexpr int col_of(int u) {
+    const int j = u % (2 * NJ) / 2;
+    return u / (2 * NJ) % 2 ? NJ - 1 - j : j;
+  }
+  static constexpr int row_of(int u) { return u / (2 * NJ) * 2 + ((u ^ u % (2 * NJ) / 2) & 1); }
 };
 
 // EPI_F32's bias (unsplit): where the block maxima go (BlockMax). ws: the partial sums' slabs of a product
@@ -248,19 +263,19 @@ __global__ void __launch_bounds__(256, 1) gemm4w_kernel(
     // VGPRs); it pads no hazard inside: the fragments' reads it waits for by register, the accumulators are
     // read only as the next MFMA's C until the pad behind the loop
     unroll<8 * NJ>([&](auto U) __attribute__((always_inline)) {
-      constexpr int u = decltype(U)::value;
+      constexpr int u = decltype(U)::value, i = Walk4w<NJ>::row_of(u), j = Walk4w<NJ>::col_of(u);
       if constexpr (first)
         asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0"
-                     : "=a"(acc[u / NJ][u % NJ]) : "v"(b0[u % NJ]), "v"(a0[u / NJ]));
+                     : "=a"(acc[i][j]) : "v"(b0[j]), "v"(a0[i]));
       else
         asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
-                     : "+a"(acc[u / NJ][u % NJ]) : "v"(b0[u % NJ]), "v"(a0[u / NJ]));
+                     : "+a"(acc[i][j]) : "v"(b0[j]), "v"(a0[i]));
       after(U);
     });
     unroll<8 * NJ>([&](auto U) __attribute__((always_inline)) {
-      constexpr int u = decltype(U)::value;
+      constexpr int u = decltype(U)::value, i = Walk4w<NJ>::row_of(u), j = Walk4w<NJ>::col_of(u);
       asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
-                   : "+a"(acc[u / NJ][u % NJ]) : "v"(b1[u % NJ]), "v"(a1[u / NJ]));
+                   : "+a"(acc[i][j]) : "v"(b1[j]), "v"(a1[i]));
       after(int_c<8 * NJ + u>{});
     });
   };
@@ -537,11 +552,11 @@ __global__ void __launch_bounds__(256, 1) gemm4w_kernel(
     ktile(F_{}, T_{}, nk <= 2);
     if (nk < 2) sab = swb = 0;
     ktile(F_{}, F_{}, false);
-    // MFMA results -> the epilogue's copies: the XDL write-back's wait states, tied to the last row of
+    // MFMA results -> the epilogue's copies: the XDL write-back's wait states, tied to the last rows of
     // accumulators written so that no copy of them moves above the pad
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) asm volatile("" : "+a"(acc[7][j]));
+    for (int j = 0; j < NJ; ++j) asm volatile("" : "+a"(acc[6][j]), "+a"(acc[7][j]));
     epilogue(t);       // (and its wait: the next tile's K-tiles 0 and 1 landed, also before an exit)
     if (!has_next) break;
     barrier();

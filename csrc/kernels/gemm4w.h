@@ -1,6 +1,6 @@
-// 256-row GEMM tiles with ONE wave per SIMD: four waves of 128 x 16 NJ, their 8 NJ 16x16 blocks
-// accumulated in the AGPR file, on a grid of at most one workgroup a CU that walks its tiles
-// (tiles 22, 28, 34, 41, 45 and 55: gemm4w.hip).
+// GEMM tiles of 32 MI x 32 NJ (256 rows, MI = 8, where a comment says no other) with ONE wave per SIMD: four waves of
+// 16 MI x 16 NJ, their MI NJ 16x16 blocks accumulated in the AGPR file, on a grid of at most one workgroup a CU that
+// walks its tiles (tiles 22, 28, 34, 41, 45 and 55: gemm4w.hip).
 //
 // What bounds it. Bare 16x16x32 MFMAs on random data run at 2.0 GHz (2.07 PFLOP/s), which the power
 // budget sets; with this tile's 32 fragment reads and 16 LDS-DMA pieces a K-tile at 1.75 GHz and 17.6
@@ -46,7 +46,7 @@ __device__ __forceinline__ void dma16(const void* base, int bytes, uint32_t lds,
   __builtin_amdgcn_raw_ptr_buffer_load_lds(make_rsrc(base, bytes), (lds_void*)lds, 16, voff, soff, IMM, 0);
 }
 
-// The schedule of a K-tile: 16 NJ MFMAs, the first half on the fragments F0 (its first 32 values of K, read
+// The schedule of a K-tile: 2 MI NJ MFMAs, the first half on the fragments F0 (its first 32 values of K, read
 // before it began), the second on F1. After MFMA q:
 //   0 .. NF - 1         a fragment of F1 each
 //   B1                  every wave has read the buffer: a barrier frees it
@@ -55,8 +55,8 @@ __device__ __forceinline__ void dma16(const void* base, int bytes, uint32_t lds,
 //   B2 + 1, + 3, ..     a fragment of the next K-tile's F0 each
 // Positions by measurement, times of 8192 x 4096 x 4096 and 16384 x 4096 x 14336 against these: reads one MFMA apart
 // instead of two -0.7 % and +0.2 %, pieces 5 instead of 6 apart -1.0 % and +1.3 %.
-template <int NJ> struct Sched4w {
-  static constexpr int Q = 16 * NJ, NF = 8 + NJ, NP = 8 + NJ;
+template <int NJ, int MI> struct Sched4w {
+  static constexpr int Q = 2 * MI * NJ, NF = MI + NJ, NP = MI + NJ;
   static constexpr int B1 = NF + 3 + NJ / 3, D = B1 + 1, DS = (Q - 4 - D) / (NP - 1), DL = D + DS * (NP - 1);
   static constexpr int B2 = Q - 1 - 2 * NF;
   static constexpr int ahead = B2 < D ? 0 : (B2 - D) / DS + 1;      // pieces issued when B2 waits
@@ -80,18 +80,19 @@ template <int NJ> struct Walk4w {
 
 // EPI_F32's bias (unsplit): where the block maxima go (BlockMax). ws: the partial sums' slabs of a product
 // split over K (fp32, or fp16 with EPI_SLAB16). group_off: rows of group g are [off[g], off[g + 1]).
-template <int EPI, int NJ>
+template <int EPI, int NJ, int MI>
 __global__ void __launch_bounds__(256, 1) gemm4w_kernel(
     const u16* __restrict__ A, int lda, const u16* __restrict__ W, int ldw,
     void* __restrict__ C, int ldc, int M, int N, int K, int splits, const u16* __restrict__ bias,
     float* __restrict__ ws, const int* __restrict__ group_off, int groups) {
-  using S = Sched4w<NJ>;
-  constexpr int BM = 256, BN = 32 * NJ, GM = 4;
+  using S = Sched4w<NJ, MI>;
+  constexpr int BM = 32 * MI, BN = 32 * NJ, GM = 4;
   constexpr int A_BYTES = BM * BK * 2;
   constexpr int NF = S::NF, NP = S::NP;
   constexpr bool PAIRS = epi_pairs(EPI);
   // two buffers 64 KiB apart: the bit that tells them apart. The kernel has no other LDS, so it starts at 0
   constexpr uint32_t FLIP = 0x10000;
+  static_assert(MI % 2 == 0 && (BM + BN) * BK * 2 <= (int)FLIP && MI * NJ <= 64, "a K-tile's buffer, and accumulators");
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -157,19 +158,19 @@ __global__ void __launch_bounds__(256, 1) gemm4w_kernel(
     return t;
   };
 
-  // ---- staging. LDS rows of 128 B whose 16-B chunk c of row r lies at c ^ ((r >> 1) & 7). A wave moves 64 rows
+  // ---- staging. LDS rows of 128 B whose 16-B chunk c of row r lies at c ^ ((r >> 1) & 7). A wave moves 8 MI rows
   // of A and 8 NJ of W a K-tile, piece i the rows 8 i + lane / 8 of them: only i's parity changes the chunk
-  // that a lane fetches, the rest is the soffset's. Rows past the matrix read as zeros
-  const int prow = 64 * wid + (lane >> 3), wprow = 8 * NJ * wid + (lane >> 3);
+  // (MI is even) that a lane fetches, the rest is the soffset's. Rows past the matrix read as zeros
+  const int prow = 8 * MI * wid + (lane >> 3), wprow = 8 * NJ * wid + (lane >> 3);
   const int ce = (lane & 7) ^ ((lane >> 4) & 7), co = (lane & 7) ^ (((lane >> 4) + 4) & 7);
   // (a wave's W rows start at an odd multiple of 8 where NJ and the wave are odd)
   const bool flip = (NJ * wid) & 1;
   const int va0 = prow * lda * 2 + ce * 16, va1 = prow * lda * 2 + co * 16;
   const int vw0 = wprow * ldw * 2 + (flip ? co : ce) * 16, vw1 = wprow * ldw * 2 + (flip ? ce : co) * 16;
   int xa0, xa1, xw0, xw1;                          // those of the next K-tile to stage
-  int sofa[8], sofw[NJ];                           // a piece's soffset, less its immediate offset
+  int sofa[MI], sofw[NJ];                           // a piece's soffset, less its immediate offset
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
+  for (int i = 0; i < MI; ++i) {
     sofa[i] = i * 16 * lda - (i & 3) * 1024;
     asm volatile("" : "+s"(sofa[i]));
   }
@@ -187,28 +188,28 @@ __global__ void __launch_bounds__(256, 1) gemm4w_kernel(
     swb = any && nk > 0 ? (min(N - t.n0, BN) * ldw - t.ks * ksl) * 2 : 0;
     xa0 = va0; xa1 = va1; xw0 = vw0; xw1 = vw1;
   };
-  uint32_t da = 64 * wid * 128, dw = A_BYTES + 8 * NJ * wid * 128;
+  uint32_t da = 8 * MI * wid * 128, dw = A_BYTES + 8 * NJ * wid * 128;
   auto piece = [&](auto F) __attribute__((always_inline)) {
     constexpr int f = decltype(F)::value;
-    if constexpr (f < 8)
+    if constexpr (f < MI)
       dma16<(f & 3) * 1024>(sa, sab, da + (f >> 2) * 4096, f & 1 ? xa1 : xa0, sofa[f]);
     else
-      dma16<((f - 8) & 3) * 1024>(sw, swb, dw + ((f - 8) >> 2) * 4096, f & 1 ? xw1 : xw0, sofw[f - 8]);
+      dma16<((f - MI) & 3) * 1024>(sw, swb, dw + ((f - MI) >> 2) * 4096, f & 1 ? xw1 : xw0, sofw[f - MI]);
   };
   auto next_buffer = [&]() { da ^= FLIP; dw ^= FLIP; };
   auto next_k = [&]() { xa0 += 2 * BK; xa1 += 2 * BK; xw0 += 2 * BK; xw1 += 2 * BK; };
 
   // ---- fragments: rows 16 apart swizzle alike, so one address a half K-tile and operand
   const int fr = lane & 15, fq = lane >> 4;
-  const int arow = wm * 128 + fr, wrow = wn * 16 * NJ + fr;
+  const int arow = wm * 16 * MI + fr, wrow = wn * 16 * NJ + fr;
   uint32_t ra0 = arow * 128 + ((fq ^ ((arow >> 1) & 7)) << 4);
   uint32_t ra1 = arow * 128 + (((4 + fq) ^ ((arow >> 1) & 7)) << 4);
   uint32_t rw0 = A_BYTES + wrow * 128 + ((fq ^ ((wrow >> 1) & 7)) << 4);
   uint32_t rw1 = A_BYTES + wrow * 128 + (((4 + fq) ^ ((wrow >> 1) & 7)) << 4);
-  f32x4 acc[8][NJ];
-  bf16x8 a0[8], b0[NJ], a1[8], b1[NJ];
+  f32x4 acc[MI][NJ];
+  bf16x8 a0[MI], b0[NJ], a1[MI], b1[NJ];
   // in the order of their use: A's first, all of W's, A's others
-  auto read = [&](auto F, bf16x8 (&av)[8], bf16x8 (&bv)[NJ], uint32_t pa, uint32_t pw)
+  auto read = [&](auto F, bf16x8 (&av)[MI], bf16x8 (&bv)[NJ], uint32_t pa, uint32_t pw)
       __attribute__((always_inline)) {
     constexpr int f = decltype(F)::value;
     if constexpr (f >= 1 && f <= NJ) {
@@ -262,7 +263,7 @@ __global__ void __launch_bounds__(256, 1) gemm4w_kernel(
     // inline asm keeps the accumulators in the AGPR file ("+a"; hipcc's own selection moves them through
     // VGPRs); it pads no hazard inside: the fragments' reads it waits for by register, the accumulators are
     // read only as the next MFMA's C until the pad behind the loop
-    unroll<8 * NJ>([&](auto U) __attribute__((always_inline)) {
+    unroll<MI * NJ>([&](auto U) __attribute__((always_inline)) {
       constexpr int u = decltype(U)::value, i = Walk4w<NJ>::row_of(u), j = Walk4w<NJ>::col_of(u);
       if constexpr (first)
         asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0"
@@ -272,11 +273,11 @@ __global__ void __launch_bounds__(256, 1) gemm4w_kernel(
                      : "+a"(acc[i][j]) : "v"(b0[j]), "v"(a0[i]));
       after(U);
     });
-    unroll<8 * NJ>([&](auto U) __attribute__((always_inline)) {
+    unroll<MI * NJ>([&](auto U) __attribute__((always_inline)) {
       constexpr int u = decltype(U)::value, i = Walk4w<NJ>::row_of(u), j = Walk4w<NJ>::col_of(u);
       asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
                    : "+a"(acc[i][j]) : "v"(b1[j]), "v"(a1[i]));
-      after(int_c<8 * NJ + u>{});
+      after(int_c<MI * NJ + u>{});
     });
   };
   // an accumulator leaves the AGPR file by one pinned copy, ahead of any condition
@@ -286,7 +287,7 @@ __global__ void __launch_bounds__(256, 1) gemm4w_kernel(
     return v;
   };
 
-  // ---- epilogue of a tile: acc[i][j][r] = C[m0 + 128 wm + 16 i + fr][n0 + 16 NJ wn + 16 j + 4 fq + r].
+  // ---- epilogue of a tile: acc[i][j][r] = C[m0 + 16 MI wm + 16 i + fr][n0 + 16 NJ wn + 16 j + 4 fq + r].
   // ranged: whole quads (fp32, partial sums) or octets (16 bits) at aligned addresses, so that rows past the
   // matrix fall out of the descriptor's range and columns past it get an offset out of it
   const bool slab = splits > 1;
@@ -296,7 +297,7 @@ __global__ void __launch_bounds__(256, 1) gemm4w_kernel(
     const uintptr_t at = (uintptr_t)(slab ? (const void*)ws : C);
     const bool wide = OUT32 || (slab && EPI != EPI_SLAB16);
     const bool bias_ok = !(EPI == EPI_BIAS || EPI == EPI_BIAS_GELU) || ((uintptr_t)bias & 7) == 0;
-    return bias_ok && ld < (1 << 21) - 1024 &&
+    return bias_ok && ld < (int)((1u << 31) / (4 * BM)) - 1024 &&
            (wide ? ((N | ld) & 3) == 0 && (at & 15) == 0 : ((N | ld) & 7) == 0 && (at & 15) == 0);
   }();
   auto quad_f = [&](const f32x4& v, uint2 bq) __attribute__((always_inline)) -> f32x4 {
@@ -316,8 +317,8 @@ __global__ void __launch_bounds__(256, 1) gemm4w_kernel(
   auto store32 = [&](const Tile& t, char* base, uint32_t* keys) __attribute__((always_inline)) {
     const int left = min(t.rows - t.m0, BM), cols = N - t.n0;
     const auto rc = make_rsrc(base, left * ld * 4);
-    const int c0 = 16 * NJ * wn + 4 * fq, vo = ((128 * wm + fr) * ld + c0) * 4;
-    unroll<8>([&](auto I) __attribute__((always_inline)) {
+    const int c0 = 16 * NJ * wn + 4 * fq, vo = ((16 * MI * wm + fr) * ld + c0) * 4;
+    unroll<MI>([&](auto I) __attribute__((always_inline)) {
       constexpr int i = decltype(I)::value;
       BlockMax top;
       unroll<NJ>([&](auto J) __attribute__((always_inline)) {
@@ -331,7 +332,7 @@ __global__ void __launch_bounds__(256, 1) gemm4w_kernel(
       if constexpr (EPI == EPI_F32) {
         if (keys != nullptr) {                     // uniform
           const uint32_t key = row_key(top);
-          const int row = t.m0 + 128 * wm + 16 * i + fr, wc0 = t.n0 + 16 * NJ * wn;
+          const int row = t.m0 + 16 * MI * wm + 16 * i + fr, wc0 = t.n0 + 16 * NJ * wn;
           if (fq == 0 && row < t.rows && wc0 < N)
             keys[(long)row * ((N + 16 * NJ - 1) / (16 * NJ)) + wc0 / (16 * NJ)] = key;
         }
@@ -345,13 +346,13 @@ __global__ void __launch_bounds__(256, 1) gemm4w_kernel(
     const int left = min(t.rows - t.m0, BM), cols = (PAIRS ? N / 2 : N) - (PAIRS ? t.n0 / 2 : t.n0);
     const auto rc = make_rsrc(base, left * ld * 2);
     const int c0 = 16 * NO * wn + 16 * (fq & 1) + 8 * (fq >> 1), c1 = 16 * NO * wn + 16 * (NO - 1) + 4 * fq;
-    const int ro = (128 * wm + fr) * ld * 2;
+    const int ro = (16 * MI * wm + fr) * ld * 2;
     // What the tile is added to is requested all at once, into the fragments' registers: 128 KB a CU at the
     // memory's rate, 3 to 7 us a round of tiles (three row blocks' requests ahead of the last K-tile changed nothing). The
     // add behind it read and wrote twice that: ops._add_product has the times
     if constexpr (EPI == EPI_RES) {
-      u32x4 old[8][NO / 2];
-      u32x2 odd[8];
+      u32x4 old[MI][NO / 2];
+      u32x2 odd[MI];
       auto fetch = [&](auto I) __attribute__((always_inline)) {
         constexpr int i = decltype(I)::value;
         unroll<NO / 2>([&](auto J) __attribute__((always_inline)) {
@@ -366,9 +367,9 @@ __global__ void __launch_bounds__(256, 1) gemm4w_kernel(
       auto sum = [](uint32_t c, float lo, float hi) __attribute__((always_inline)) -> uint32_t {
         return pack2bf(__uint_as_float(c << 16) + lo, __uint_as_float(c & 0xffff0000u) + hi);
       };
-      unroll<8>(fetch);
+      unroll<MI>(fetch);
       asm volatile("" ::: "memory");
-      unroll<8>([&](auto I) __attribute__((always_inline)) {
+      unroll<MI>([&](auto I) __attribute__((always_inline)) {
         constexpr int i = decltype(I)::value;
         unroll<NO / 2>([&](auto J) __attribute__((always_inline)) {
           constexpr int j = 2 * decltype(J)::value;
@@ -403,7 +404,7 @@ __global__ void __launch_bounds__(256, 1) gemm4w_kernel(
         bq[j] = uint2{b[0], b[1]};
       });
     }
-    unroll<8>([&](auto I) __attribute__((always_inline)) {
+    unroll<MI>([&](auto I) __attribute__((always_inline)) {
       constexpr int i = decltype(I)::value;
       auto quad = [&](auto J) __attribute__((always_inline)) -> uint2 {
         constexpr int j = decltype(J)::value;
@@ -440,10 +441,10 @@ __global__ void __launch_bounds__(256, 1) gemm4w_kernel(
   };
   // any width and alignment, quad by quad
   auto store_any = [&](const Tile& t) __attribute__((always_inline)) {
-    const int wr0 = t.m0 + 128 * wm, wc0 = t.n0 + 16 * NJ * wn;
+    const int wr0 = t.m0 + 16 * MI * wm, wc0 = t.n0 + 16 * NJ * wn;
     const bool vec = slab ? (N & 3) == 0 : out_vec<EPI>(C, ldc, N, bias);
     float* sl = ws + (long)t.ks * M * N;
-    unroll<8>([&](auto I) __attribute__((always_inline)) {
+    unroll<MI>([&](auto I) __attribute__((always_inline)) {
       constexpr int i = decltype(I)::value;
       const int row = wr0 + 16 * i + fr;
       BlockMax top;
@@ -484,7 +485,7 @@ __global__ void __launch_bounds__(256, 1) gemm4w_kernel(
     });
   };
   // stores issued behind the next tile's pieces, which may fly while those are waited for (6 bits count)
-  constexpr int N32 = 8 * NJ, N16 = 8 * (((PAIRS ? NJ / 2 : NJ) + 1) / 2);
+  constexpr int N32 = MI * NJ, N16 = MI * (((PAIRS ? NJ / 2 : NJ) + 1) / 2);
   auto epilogue = [&](const Tile& t) __attribute__((always_inline)) {
     if (EPI != EPI_RES && !ranged) {
       store_any(t);
@@ -533,12 +534,12 @@ __global__ void __launch_bounds__(256, 1) gemm4w_kernel(
       ktile(T_{}, T_{}, true);
     } else {
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
+      for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
       // these are read by inline-asm MFMAs, which hipcc pads no hazard for: every write ahead of wait states
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
+      for (int i = 0; i < MI; ++i) {
 #pragma unroll
         for (int j = 0; j < NJ; ++j) asm volatile("" : "+a"(acc[i][j]));
         asm volatile("s_nop 3");
@@ -556,7 +557,7 @@ __global__ void __launch_bounds__(256, 1) gemm4w_kernel(
     // accumulators written so that no copy of them moves above the pad
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) asm volatile("" : "+a"(acc[6][j]), "+a"(acc[7][j]));
+    for (int j = 0; j < NJ; ++j) asm volatile("" : "+a"(acc[MI - 2][j]), "+a"(acc[MI - 1][j]));
     epilogue(t);       // (and its wait: the next tile's K-tiles 0 and 1 landed, also before an exit)
     if (!has_next) break;
     barrier();
@@ -579,8 +580,11 @@ static int cu_count() {
 // the mode that dli_gemm_set_slab_store asked for
 int gemm_4w_store_mode();
 
+// the stride of a tile's 32 L rows from which its offsets no longer fit 31 bits, to a power of two
+template <int L> constexpr int MAX_LD = L > 8 ? 1 << 21 : 1 << 22;
+
 // M: rows, or the most rows of a group (group_off: their offsets, groups of them)
-template <int EPI, int NJ>
+template <int EPI, int NJ, int MI = 8>
 static int launch_4w(const void* A, int lda, const void* W, int ldw, void* C, int ldc, int M, int N,
                      int K, int splits, const void* bias, void* ws, const int* group_off, int groups,
                      hipStream_t st) {
@@ -588,28 +592,28 @@ static int launch_4w(const void* A, int lda, const void* W, int ldw, void* C, in
   if (K % (splits * BK)) return (int)hipErrorInvalidValue;
   // (a panel's range is its rows times their stride in 32 bits, which overlapping rows would reach past: ops/gemm.py's
   // spaced copies those)
-  if (lda < K || ldw < K || lda >= (1 << 22) || ldw >= (1 << 22)) return (int)hipErrorInvalidValue;
+  if (lda < K || ldw < K || lda >= MAX_LD<MI> || ldw >= MAX_LD<NJ>) return (int)hipErrorInvalidValue;
   // The kernel has one way to store fp32 partial sums (the others' probe modes would more than double its code): while
   // another is set, split products are refused and not timed as what they are not
   if (splits > 1 && EPI != EPI_SLAB16 && gemm_4w_store_mode() != 0) return (int)hipErrorInvalidValue;
   if (EPI == EPI_RES && (splits != 1 || group_off != nullptr || ((N | ldc) & 7) || ((uintptr_t)C & 15) || C == nullptr ||
                          ldc >= (1 << 21) - 1024))
     return (int)hipErrorInvalidValue;
-  constexpr size_t lds = 0x10000 + (size_t)(256 + 32 * NJ) * BK * 2;
+  constexpr size_t lds = 0x10000 + (size_t)(32 * MI + 32 * NJ) * BK * 2;
   static bool raised = false;
   if (!raised) {
-    hipFuncSetAttribute((const void*)gemm4w_kernel<EPI, NJ>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    hipFuncSetAttribute((const void*)gemm4w_kernel<EPI, NJ, MI>, hipFuncAttributeMaxDynamicSharedMemorySize,
                         (int)lds);
     raised = true;
   }
   const int cus = cu_count();
-  const long tiles = (long)((M + 255) / 256) * ((N + 32 * NJ - 1) / (32 * NJ)) * splits *
+  const long tiles = (long)((M + 32 * MI - 1) / (32 * MI)) * ((N + 32 * NJ - 1) / (32 * NJ)) * splits *
                      (group_off != nullptr ? groups : 1);
   // one workgroup per CU (over 80 KiB of LDS each); a multiple of 8 keeps every workgroup's virtual tile ids
   // on one XCD residue class
   int grid = tiles < cus ? (int)tiles : (cus / 8) * 8;
   if (grid < 1) grid = 1;
-  gemm4w_kernel<EPI, NJ><<<grid, 256, lds, st>>>((const u16*)A, lda, (const u16*)W, ldw, C, ldc, M, N, K, splits,
+  gemm4w_kernel<EPI, NJ, MI><<<grid, 256, lds, st>>>((const u16*)A, lda, (const u16*)W, ldw, C, ldc, M, N, K, splits,
                                                  (const u16*)bias, (float*)ws, group_off, groups);
   if constexpr (EPI != EPI_RES) {                  // (never split)
     if (splits > 1 && C != nullptr) {
@@ -620,4 +624,20 @@ static int launch_4w(const void* A, int lda, const void* W, int ldw, void* C, in
     }
   }
   DLI_RETURN_LAUNCH();
+}
+
+// the epilogues of the tiles that gemm4w.hip chooses by rounds
+template <int NJ, int MI = 8> static int launch_nj(int epi, DLI_GEMM_ARGS) {
+  switch (epi) {
+    case EPI_BF16: return launch_4w<EPI_BF16, NJ, MI>(DLI_GEMM_PASS);
+    case EPI_F32: return launch_4w<EPI_F32, NJ, MI>(DLI_GEMM_PASS);
+    case EPI_SLAB16: return launch_4w<EPI_SLAB16, NJ, MI>(DLI_GEMM_PASS);
+    case EPI_RES: return launch_4w<EPI_RES, NJ, MI>(DLI_GEMM_PASS);
+    default: break;
+  }
+  if constexpr (NJ % 2 == 0) {                     // a gate block and its up block in one wave tile
+    if (epi == EPI_SILU) return launch_4w<EPI_SILU, NJ, MI>(DLI_GEMM_PASS);
+    if (epi == EPI_GELU_MUL) return launch_4w<EPI_GELU_MUL, NJ, MI>(DLI_GEMM_PASS);
+  }
+  return DLI_NOT_MINE;
 }

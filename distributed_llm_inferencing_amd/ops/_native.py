@@ -61,6 +61,7 @@ _SIGS = {
     "dli_gemm_head": [P, I, P, I, P, I, I, I, I, I, P, P],
     "dli_gemm_head_block": [I, I, I],
     "dli_gemm_4w_width": [I, I, I, I, I],
+    "dli_gemm_4w_rows": [I, I, I, I, I, I],
     "dli_splitk_add_rmsnorm": [P, P, P, I, I, I, P, F, I, P],
     "dli_gemv_fused": [P, I, P, F, P, I, P, I, I, I, I, I, I, I, P, P],
     "dli_splitk_rope_cache": [P, P, I, I, I, P, P, P, P, P, I, I, I, I, I, I, P],

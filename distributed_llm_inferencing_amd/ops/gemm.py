@@ -35,8 +35,9 @@ TILES = {0: (64, 64), 1: (64, 128), 2: (128, 128), 3: (128, 256), 4: (256, 128),
          13: (256, 256), 14: (256, 128), 15: (128, 256), 16: (256, 128), 17: (128, 256),
          # grid-filling tiles for N = 6144 / 4096 at M = 512
          18: (128, 96), 19: (128, 96), 20: (128, 64), 21: (128, 64),
-         # 4 waves, one per SIMD (gemm4w.h): 256 columns, or fewer where they leave less of a round of CUs
-         # empty (dense, not biased); the rarer epilogues on the 8-phase ping-pong kernel (gemm8p.hip)
+         # 4 waves, one per SIMD (gemm4w.h): 256 columns, or fewer, or rows of 192 or 320, where they leave
+         # less of a round of CUs empty (dense, not biased; gemm4w.hip's shape_of); the rarer epilogues on the
+         # 8-phase ping-pong kernel (gemm8p.hip)
          22: (256, 256),
          # 192-wide, 8 waves: N = 6144 is 32 column tiles (fused QKV at M = 512 fills the chip
          # with split-K 2 / 4)
@@ -48,8 +49,8 @@ TILES = {0: (64, 64), 1: (64, 128), 2: (128, 128), 3: (128, 256), 4: (256, 128),
          # 256x256, 4 waves (one per SIMD), 128x128 wave tiles, accumulators pinned in the AGPR
          # file, at most a workgroup a CU that walks its tiles (gemm4w.h)
          34: (256, 256), 41: (256, 256), 45: (256, 256),
-         # 55: the same on tiles of 256, 192 or 160 columns, by rounds of the chip;
-         # no split-K / grouped
+         # 55: the same on tiles of 256, 192 or 160 columns by rounds of the chip, or of other
+         # rows as 22; no split-K / grouped
          55: (256, 256)}
 # weight-streaming tiles for up to 128 rows (gemm_stream.h): weights nontemporal, K loops turned from
 # tile to tile, 3 to 6 stages; (BM, BN, K-tile: a split of K holds whole ones), so kept apart

@@ -4,7 +4,7 @@
 // mixing — those run window_attention_mfma.hip). The sink and the head's gate only touch the epilogue
 // and cost nothing: 5 prompts of 900 to 2601 tokens, 32 heads of 128 on 8 kv heads, took 2.12 ms in
 // window_attention_mfma.hip (16 queries x 8 heads a workgroup, barrier-separated phases) and take
-// 0.25 ms here; decode of 64 rows at 984 keys 59 us instead of 252.
+// 0.2 ms here; decode of 64 rows at 984 keys 59 us instead of 252.
 // Position i sees j <= i with i - j < window or j < keep.
 //
 // The keys that a group of queries can see are at most two runs, [0, kf) and [lo, last], walked
@@ -15,8 +15,8 @@
 //  * swa_prefill32  8 waves x 32 query rows of one head: v_mfma_f32_32x32x16_bf16 on swapped
 //                   products (S^T = K . Q^T, O^T = V^T . P^T), so that a lane owns one query and
 //                   the softmax is lane-local but for one exchange; K / V tiles of 64 keys by
-//                   LDS-DMA into three buffers, one barrier a tile; the list's cache rows looked
-//                   up once (LDS). The structure of attention_prefill.hip's long-prompt kernel.
+//                   LDS-DMA into three buffers, one barrier a tile; the list's cache rows (of
+//                   every sixteenth, where 16 lie together) looked up once (LDS). The structure of attention_prefill.hip's long-prompt kernel.
 //                   Latent attention runs it too, expanded: [k_h | shared rotated key] rows of 192.
 //  * swa_prefill16  4 waves x 16 query rows: portions shorter than the above is worth
 //  * swa_decode     one query token a sequence: a workgroup per (sequence, kv head, key split).
@@ -50,6 +50,7 @@ struct SwaArgs {
   int H, G, window, keep;
   float scale_log2;
   int table_cap;                       // prefill32: list entries that fit the LDS table
+  int block_shift;                     // log2 of a block's rows, where they are a power of two
   int nsplit;                          // decode: key splits
   float* ws;                           // decode, nsplit > 1: [nsplit][S][H][2], [nsplit][S][H][HD]
   // shared tail of queries and keys (prefill32 with DR > 0): head h of token t has its DR dims at q2 +
@@ -87,6 +88,15 @@ struct KeyList {
     n = last - skip + 1;
   }
   __device__ int key(int x) const { return x < kf ? x : x + skip; }
+  // The same with both runs widened to whole groups of 16 keys, whose rows lie in one cache block each; the keys
+  // that no query sees are masked as those of other queries are
+  __device__ void widen(int last) {
+    const int lo = kf + skip & ~15;
+    kf = kf + 15 & ~15;
+    skip = kf < lo ? lo - kf : 0;
+    if (skip == 0) kf = 0;
+    n = last - skip + 1;
+  }
 };
 
 __device__ __forceinline__ float max3(float a, float b, float c) {
@@ -96,6 +106,9 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
 constexpr int KT = 64;                 // keys a tile
 constexpr int LROWS = 256;             // query rows of a long-form workgroup
 constexpr float RESCALE_THR = 8.f;     // log2 units: the running max moves only by more than this
+
+// a value that is the same in all lanes, in a scalar register
+__device__ __forceinline__ uint32_t scalar(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
 
 // One tile of rows (D wide) by LDS-DMA: 1-KiB pieces of two subtiles in a row, wave w of 8 takes
 // pieces w, w + 8, ... The DMA writes lane-linearly, so each lane loads the logical chunk that
@@ -118,9 +131,43 @@ __device__ __forceinline__ void stage_rows(const u16* src, long stride, const u1
   }
 }
 
+// The same tile from rows that lie together, by sixteens (TOGETHER = 16) or all 64 of it. Nothing of an address is left
+// to the lanes but their place among those rows (voff, of each piece), and what is past the last row lands as zeros.
+// rows: the descriptor of sixteen g's (tail: of the second matrix's)
+__device__ __forceinline__ u32x4 rows_at(uintptr_t first, int bytes) {
+  return {scalar((uint32_t)first), scalar((uint32_t)(first >> 32) & 0xffff), scalar((uint32_t)bytes), 0x00020000};
+}
+template <int D, int D1, typename Rows>
+__device__ __forceinline__ void stage_together(uint32_t dst, int wid, const int (&voff)[(D / 8 + 7) / 8], const Rows& rows) {
+  constexpr int NP = D / 8;
+#pragma unroll
+  for (int j = 0; j < (NP + 7) / 8; ++j) {
+    const int piece = wid + 8 * j;
+    if (NP % 8 != 0 && piece >= NP) break;                     // wave-uniform
+    const bool tail = D1 < D && piece * 1024 % (D * 16) / 16 >= D1;
+    const u32x4 rsrc = rows(piece * 64 / D >> 1, tail);
+    const uint32_t to = scalar(dst + piece * 1024);
+    // (inline asm: behind the builtins hipcc waits for every LDS-DMA in flight ahead of the transposing reads, this
+    // tile's among them. The wait states are a vector instruction's that wrote one of the scalars)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                 :: "s"(to), "v"(voff[j]), "s"(rsrc) : "memory", "m0");
+  }
+}
+template <int D, int D1, int TOGETHER>
+__device__ __forceinline__ void piece_offsets(int (&voff)[(D / 8 + 7) / 8], long stride, long stride2, int wid, int lane) {
+#pragma unroll
+  for (int j = 0; j < (D / 8 + 7) / 8; ++j) {
+    const int b = (wid + 8 * j) * 1024 + lane * 16, in = b % (D * 16);
+    const int r = 8 * (b / (D * 16)) + ((lane & 31) >> 2), c = 4 * (in / 512) + ((lane & 3) ^ ((r >> 2) & 3));
+    const bool tail = D1 < D && c * 8 >= D1;
+    voff[j] = r % TOGETHER * (int)(tail ? stride2 : stride) * 2 + (tail ? c * 8 - D1 : c * 8) * 2;
+  }
+}
+
 // Tile image: 8-row x 32-column subtiles of 512 B with the chunks of a row rotated by its row
 // group: conflict-free for row reads and for transposed reads. DK, DR, DV: multiples of 32.
-template <int DK, int DR, int DV>
+// GROUPS: cache blocks are powers of two of at least 16 rows (or the rows a plain matrix's), staged by stage_together
+template <int DK, int DR, int DV, bool GROUPS>
 __global__ void __launch_bounds__(512) swa_prefill32_kernel(SwaArgs a) {
   constexpr int KW = DK + DR, KC = KW / 16, DBK = DV / 32;
   constexpr int RGK = KW * 16, RGV = DV * 16;                  // bytes of an 8-row group
@@ -144,7 +191,9 @@ __global__ void __launch_bounds__(512) swa_prefill32_kernel(SwaArgs a) {
   const int p0 = a.positions[t0];
   const int q0 = wg_q0 + wid * 32;
   const bool active = q0 < len;
-  const KeyList kl(p0 + wg_q0, p0 + min(wg_q0 + LROWS, len) - 1, a.window, a.keep);
+  const int last = p0 + min(wg_q0 + LROWS, len) - 1;
+  KeyList kl(p0 + wg_q0, last, a.window, a.keep);
+  if (GROUPS && !DR) kl.widen(last);           // (a plain matrix has no row ahead of the first key)
   const int ntiles = (kl.n + KT - 1) / KT;
   const int* bt = DR ? nullptr : a.block_tables + (long)s * a.bt_stride;
   const int base = DR ? a.cu_ctx[s + 1] - (p0 + len) : 0;
@@ -152,9 +201,15 @@ __global__ void __launch_bounds__(512) swa_prefill32_kernel(SwaArgs a) {
     const int j = kl.key(x);
     return DR ? base + j : bt[j / a.block_size] * a.block_size + j % a.block_size;
   };
-  const bool use_table = !DR && kl.n <= a.table_cap;
+  // the list's cache rows (GROUPS: of every sixteenth)
+  const bool use_table = !DR && !GROUPS && kl.n <= a.table_cap;
   if (use_table)
     for (int x = tid; x < kl.n; x += 512) table[x] = row_of(x);
+  if (GROUPS && !DR)
+    for (int x = tid; x < 4 * ntiles; x += 512) {
+      const int j = kl.key(min(16 * x, kl.n - 1 & ~15));
+      table[x] = (bt[j >> a.block_shift] << a.block_shift) + (j & (a.block_size - 1));
+    }
 
   bf16x8 qf[KC];
   {
@@ -181,7 +236,38 @@ __global__ void __launch_bounds__(512) swa_prefill32_kernel(SwaArgs a) {
     x = min(x, kl.n - 1);
     return use_table ? table[x] : row_of(x);
   };
+  int vk[(KW / 8 + 7) / 8], vv[(DV / 8 + 7) / 8];
+  if constexpr (GROUPS) {
+    piece_offsets<KW, DK, DR ? KT : 16>(vk, a.k_stride, a.k2_stride, wid, lane);
+    piece_offsets<DV, DV, DR ? KT : 16>(vv, a.v_stride, 0, wid, lane);
+  }
+  // GROUPS: where the next tile's rows begin (of a plain matrix; else the cache's first), and the bytes of a row
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_void*)lds;
+  const int row_k = (int)a.k_stride * 2, row_v = (int)a.v_stride * 2, row_k2 = (int)a.k2_stride * 2;
+  const long row0 = DR ? base + kl.skip : 0;
+  uintptr_t at_k = (uintptr_t)(a.k + kvh * DK) + row0 * row_k, at_v = (uintptr_t)(a.v + kvh * DV) + row0 * row_v,
+            at_k2 = (uintptr_t)a.k2 + row0 * row_k2;
   const auto stage = [&](int buf, int x0) {
+    if constexpr (GROUPS) {
+      const uint32_t to = lds0 + buf * TILE_B;
+      const int left = kl.n - x0;                              // (only the last tile's are fewer than its rows)
+      if constexpr (DR != 0) {
+        const int n = left < KT ? left : KT;
+        const u32x4 head = rows_at(at_k, n * row_k), tail = rows_at(at_k2, n * row_k2), vals = rows_at(at_v, n * row_v);
+        stage_together<KW, DK>(to, wid, vk, [&](int, bool t) { return t ? tail : head; });
+        stage_together<DV, DV>(to + TILE_K, wid, vv, [&](int, bool) { return vals; });
+        at_k += KT * row_k, at_k2 += KT * row_k2, at_v += KT * row_v;
+      } else {
+        const int rows4 = table[(x0 >> 4) + (lane & 3)];
+        const auto rows = [&](uintptr_t m, int row, int g) {
+          const int n = left - 16 * g;
+          return rows_at(m + (long)__builtin_amdgcn_readlane(rows4, g) * row, n >= 16 ? 16 * row : n > 0 ? n * row : 0);
+        };
+        stage_together<KW, DK>(to, wid, vk, [&](int g, bool) { return rows(at_k, row_k, g); });
+        stage_together<DV, DV>(to + TILE_K, wid, vv, [&](int g, bool) { return rows(at_v, row_v, g); });
+      }
+      return;
+    }
     char* kd = lds + buf * TILE_B;
     stage_rows<KW, DK>(a.k + kvh * DK, a.k_stride, a.k2, a.k2_stride, kd, x0, wid, lane, row_in_list);
     stage_rows<DV, DV>(a.v + kvh * DV, a.v_stride, nullptr, 0, kd + TILE_K, x0, wid, lane, row_in_list);
@@ -197,6 +283,10 @@ __global__ void __launch_bounds__(512) swa_prefill32_kernel(SwaArgs a) {
     asm volatile("" ::: "memory");
   };
   stage(0, 0);
+  // the queries are there from here on: hipcc would wait for them where it first uses them, in every tile, and so for the
+  // DMA in flight, which it does not count
+#pragma unroll
+  for (int c = 0; c < KC; ++c) asm volatile("" : "+v"(qf[c]));
   if (ntiles > 1) {
     stage(1, KT);
     wait_one_tile();
@@ -235,7 +325,16 @@ __global__ void __launch_bounds__(512) swa_prefill32_kernel(SwaArgs a) {
         }
       }
       // only tiles that cross this wave's diagonal or the window's far edge are masked
-      if (kt1 > wq_lo || wq_hi - kt0 >= a.window) {
+      if (kt0 >= a.keep && (kt1 > wq_lo || wq_hi - kt0 >= a.window)) {
+        // (one run of keys: those seen are the window's that end at the query)
+        const int first = kt0 + 4 * hi - (qpos - a.window + 1);
+#pragma unroll
+        for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            sacc[sub][r] = (unsigned)(first + 32 * sub + (r & 3) + 8 * (r >> 2)) < (unsigned)a.window ? sacc[sub][r]
+                                                                                                     : -INFINITY;
+      } else if (kt1 > wq_lo || wq_hi - kt0 >= a.window) {
 #pragma unroll
         for (int sub = 0; sub < 2; ++sub)
 #pragma unroll
@@ -708,15 +807,11 @@ int decode_splits(int num_seqs, int H, int G, long keys) {
 // key / value widths this file is built for
 #define SWA_WIDTHS(F) F(64, 64) F(128, 128) F(64, 128) F(96, 192) F(128, 256)
 
-template <int DK, int DR, int DV>
-int launch_prefill32(SwaArgs a, int num_seqs, int max_seqlen, hipStream_t st) {
-  const long list = (long)a.window + LROWS + a.keep;
-  constexpr int TILES = 3 * KT * (DK + DR + DV) * 2;
-  a.table_cap = !DR && list <= 6144 && TILES + list * 4 + 16 <= 160 * 1024 ? (int)list : 0;
-  const int sh = TILES + a.table_cap * 4 + 16;
+template <int DK, int DR, int DV, bool GROUPS>
+int launch_prefill32(SwaArgs a, int sh, int num_seqs, int max_seqlen, hipStream_t st) {
   static bool raised = false;
   if (!raised) {
-    const hipError_t e = hipFuncSetAttribute((const void*)swa_prefill32_kernel<DK, DR, DV>,
+    const hipError_t e = hipFuncSetAttribute((const void*)swa_prefill32_kernel<DK, DR, DV, GROUPS>,
                                              hipFuncAttributeMaxDynamicSharedMemorySize,
                                              160 * 1024);
     if (e != hipSuccess) return (int)e;
@@ -724,8 +819,32 @@ int launch_prefill32(SwaArgs a, int num_seqs, int max_seqlen, hipStream_t st) {
   }
   const int blocks = (max_seqlen + LROWS - 1) / LROWS;
   const dim3 grid = a.H <= 4 ? dim3(blocks, num_seqs, a.H) : dim3(blocks * a.H, num_seqs);
-  swa_prefill32_kernel<DK, DR, DV><<<grid, 512, sh, st>>>(a);
+  swa_prefill32_kernel<DK, DR, DV, GROUPS><<<grid, 512, sh, st>>>(a);
   DLI_RETURN_LAUNCH();
+}
+
+template <int DK, int DR, int DV>
+int launch_prefill32(SwaArgs a, int num_seqs, int max_seqlen, hipStream_t st) {
+  constexpr int TILES = 3 * KT * (DK + DR + DV) * 2, MOST = 160 * 1024;
+  const long list = (long)a.window + LROWS + a.keep;
+  const int bs = a.block_size;
+  // Rows that lie together, by 31-bit offsets, apart from one another, and a table of the list's sixteens beside the tiles
+  // (at 128 + 128 wide it has room for 260 thousand keys). Row by row otherwise, the former way, through a table of rows
+  // or the block table itself, whose loads wait for all DMA in flight. That way and its mask, by runs and key by key,
+  // against this one and the mask of one run, us, 32 heads of 128 on 8 with a sink and a gate a head: 5 portions of
+  // 900 to 2601 tokens 285 -> 203, in windows of 1024 217 -> 171, 8000 tokens 767 -> 567 (0.92 PFLOP/s); expanded latent
+  // heads, 6 of 301 to 3000 222 -> 199, in windows of 1024 187 -> 158. The mask is 13 % of the first and all of the last
+  const auto fits = [](long stride, int wide) { return stride >= wide && stride < (1l << 31) / (2 * (DR ? KT : 16)); };
+  if (fits(a.k_stride, DK) && fits(a.v_stride, DV) && (DR == 0 || fits(a.k2_stride, DR))) {
+    if (DR) return launch_prefill32<DK, DR, DV, true>(a, TILES, num_seqs, max_seqlen, st);
+    const long sixteens = (list + 32 + 63) / KT * 4;
+    if (bs >= 16 && (bs & (bs - 1)) == 0 && TILES + sixteens * 4 <= MOST) {
+      a.block_shift = __builtin_ctz(bs);
+      return launch_prefill32<DK, DR, DV, true>(a, TILES + (int)sixteens * 4, num_seqs, max_seqlen, st);
+    }
+  }
+  a.table_cap = !DR && list <= 6144 && TILES + list * 4 + 16 <= MOST ? (int)list : 0;
+  return launch_prefill32<DK, DR, DV, false>(a, TILES + a.table_cap * 4 + 16, num_seqs, max_seqlen, st);
 }
 
 template <int DK, int DV>
@@ -818,7 +937,7 @@ extern "C" int dli_shared_tail_attention(const void* q, int ldq, const void* q2,
     return (int)hipErrorNotSupported;
   SwaArgs a{(const u16*)q, ldq, (const u16*)k, k_stride, (const u16*)v, v_stride, (u16*)out, ldo,
             gate, ldg, gate != nullptr, nullptr, 1.f, cu, positions, nullptr, 0, 1, H, H, window, 0,
-            scale * LOG2E, 0, 1, nullptr, (const u16*)q2, ldq2, q2_head, (const u16*)k2, k2_stride, cu_ctx};
+            scale * LOG2E, 0, 0, 1, nullptr, (const u16*)q2, ldq2, q2_head, (const u16*)k2, k2_stride, cu_ctx};
   return launch_prefill32<128, 64, 128>(a, num_seqs, max_seqlen, st);
 }
 
@@ -852,7 +971,7 @@ extern "C" int dli_swa_attention(const void* q, int ldq, const void* k, long k_s
     return (int)hipErrorNotSupported;
   SwaArgs a{(const u16*)q, ldq, (const u16*)k, k_stride, (const u16*)v, v_stride, (u16*)out, ldo,
             gate, ldg, head_gate != 0, sink, out_scale, cu, positions, block_tables, bt_stride, block_size, H, G, window, keep,
-            scale * LOG2E, 0, 1, (float*)ws, nullptr, 0, 0, nullptr, 0, nullptr};
+            scale * LOG2E, 0, 0, 1, (float*)ws, nullptr, 0, 0, nullptr, 0, nullptr};
   if (max_seqlen == 1) {
     a.nsplit = decode_splits(num_seqs, H, G, (long)window + keep);
     if (a.nsplit > 1 && ws == nullptr) return (int)hipErrorInvalidValue;

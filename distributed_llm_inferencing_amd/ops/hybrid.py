@@ -411,11 +411,13 @@ def window_attention(q, k_cache, v_cache, dq, dv, H, G, cu_seqlens, max_seqlen, 
             nb = lib.dli_swa_attention_workspace_bytes(S, int(max_seqlen), H, G, dv, int(window),
                                                        int(keep_first))
             ws = _gemm.workspace(q.device, nb) if nb else None
+            # (a portion's keys are in its blocks: with a bound to them the kernel's table of them fits)
+            reach = int(window) if int(max_seqlen) == 1 else max(1, min(int(window), block_tables.shape[1] * block_size))
             rc = lib.dli_swa_attention(
                 _p(q), q.stride(0), _p(k_cache), k_cache.stride(0), _p(v_cache),
                 v_cache.stride(0), _p(out), out.stride(0), _p(cu_seqlens), _p(positions),
                 _p(block_tables), block_tables.stride(0), block_size, S, int(max_seqlen), H, G, dq,
-                dv, int(window), int(keep_first), float(scale), _p(gate),
+                dv, reach, int(keep_first), float(scale), _p(gate),
                 gate.stride(0) if gate is not None else 0, hg, _p(sink), float(out_scale), _p(ws),
                 _st())
             if rc == 0:

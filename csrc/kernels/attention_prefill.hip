@@ -24,10 +24,9 @@
 // workgroup packs 2 / 4 query heads of one GQA group (2 / 1 waves each): the K/V tiles it
 // stages serve every packed head, and no wave idles past a 32-token prompt (the bench's
 // 512 x 32-token prefill ran 16,384 half-idle workgroups).
-#include "common.h"
+#include "lds_dma.h"
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) void lds_void;
 typedef const __attribute__((address_space(1))) void gbl_void;
 typedef short s16x8 __attribute__((ext_vector_type(8)));
 #define PF_WAVES 4
@@ -253,14 +252,20 @@ __device__ __forceinline__ float pl_max3(float a, float b, float c) {  // no can
 }
 #define PL_RESCALE_THR 8.f      // log2 units: a running max is raised only by more than this
 
-template <int HD, bool PAGED>
+// SRC: the activation's rows; cache blocks of a power of two of at least 16 tokens, whose rows lie together by sixteens
+// and are staged through scalar descriptors (lds_dma.h); other blocks, row by row, whose table every lane reads, behind
+// all DMA in flight. 2048 queries of 4096 keys 133 -> 126 us, 1024 of 6000 174 -> 163, 6 x 400 of 2400 147 -> 138. The
+// activation's rows gain nothing so (4 x 1000 62.2 and 61.9, 2048 51.4 and 51.6)
+enum { ROWS_OF_QKV = 0, BLOCKS_OF_16 = 1, BLOCKS = 2 };
+template <int HD, int SRC>
 __global__ void __launch_bounds__(512) prefill_attn32_kernel(
     u16* __restrict__ out, int out_stride, const u16* __restrict__ qkv, int row_stride,
     const int* __restrict__ cu_seqlens, int hq, int hkv, float scale_log2,
     const int* __restrict__ ctx_lens, const u16* __restrict__ k_cache,
     const u16* __restrict__ v_cache, const int* __restrict__ block_tables, int bt_stride,
-    int block_size, bool paired) {
+    int block_size, int block_shift, bool paired) {
   static_assert(HD == 128, "long-sequence kernel: head_dim 128");
+  constexpr bool PAGED = SRC != ROWS_OF_QKV;
   constexpr int KC = HD / 16;                      // K-steps of the QK^T product
   constexpr int DBK = HD / 32;                     // 32-wide d blocks of O^T
   constexpr int TILE_B = PL_KT * HD * 2;           // bytes per K (or V) tile image
@@ -330,7 +335,27 @@ __global__ void __launch_bounds__(512) prefill_attn32_kernel(
   // tile image is 16 pieces of 1 KiB (= subtiles 2hp, 2hp+1 of 8-row group rg); wave w
   // stages pieces w and w + 8 of K and of V. The DMA writes lane-linearly (lane L at byte
   // 16L of the piece), so each lane loads the logical chunk that lands there.
+  constexpr int ROW = HD * 2;                        // bytes of a cache row
+  int voff[2];                                       // BLOCKS_OF_16: a lane's place in its piece's sixteen
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int r = 8 * ((wid + 8 * j) >> 1) + ((lane & 31) >> 2);
+    voff[j] = (r & 15) * ROW + 64 * (2 * (wid & 1) + (lane >> 5)) + 16 * ((lane & 3) ^ ((r >> 2) & 3));
+  }
   auto stage = [&](int buf, int k0) {
+    if constexpr (SRC == BLOCKS_OF_16) {
+      const uint32_t to = lds_address(&lds[buf][0][0]);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int first = k0 + 16 * ((wid >> 2) + 2 * j), n = nkeys - first;
+        const int id = __builtin_amdgcn_readfirstlane(btab[min(first, nkeys - 1) >> block_shift]);
+        const long at = (long)id * ((long)hkv * block_size * ROW) + (first & (block_size - 1)) * ROW;
+        const int bytes = (n < 16 ? max(n, 0) : 16) * ROW;
+        dma_piece(to + (wid + 8 * j) * 1024, voff[j], bytes_at((uintptr_t)(k_cache + head_off) + at, bytes));
+        dma_piece(to + TILE_B + (wid + 8 * j) * 1024, voff[j], bytes_at((uintptr_t)(v_cache + head_off) + at, bytes));
+      }
+      return;
+    }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int piece = wid + 8 * j;
@@ -357,6 +382,12 @@ __global__ void __launch_bounds__(512) prefill_attn32_kernel(
   };
 
   stage(0, 0);
+  // the queries are there from here on: hipcc would wait for them where it first uses them, in every tile, and so for the
+  // DMA in flight, which it does not count
+  if (SRC == BLOCKS_OF_16) {
+#pragma unroll
+    for (int c = 0; c < KC; ++c) asm volatile("" : "+v"(qf[c]));
+  }
   if (ntiles > 1) {
     stage(1, PL_KT);
     asm volatile("s_waitcnt vmcnt(4)" ::: "memory");             // tile 0 landed
@@ -530,10 +561,14 @@ static int launch_prefill(void* out, int out_stride, const void* qkv, int row_st
   if (hd == 128 && max_seqlen >= g_pl_min_len) {     // long sequences: 256-row workgroups
     const int blocks = (max_seqlen + PL_ROWS - 1) / PL_ROWS;
     const dim3 grid32 = hq <= 4 ? dim3(blocks, num_seqs, hq) : dim3(blocks * hq, num_seqs);
-    prefill_attn32_kernel<128, PAGED><<<grid32, 512, 0, st>>>(
-        (u16*)out, out_stride, (const u16*)qkv, row_stride, cu_seqlens, hq, hkv, sl2, ctx_lens,
-        (const u16*)k_cache, (const u16*)v_cache, block_tables, bt_stride, block_size,
-        blocks > 1 && (long)blocks * hq * num_seqs <= PL_ROUND);
+    const bool paired = blocks > 1 && (long)blocks * hq * num_seqs <= PL_ROUND;
+    const bool by16 = PAGED && block_size >= 16 && (block_size & (block_size - 1)) == 0;
+    const int shift = by16 ? __builtin_ctz(block_size) : 0;
+#define PL_ARGS (u16*)out, out_stride, (const u16*)qkv, row_stride, cu_seqlens, hq, hkv, sl2, ctx_lens, \
+                (const u16*)k_cache, (const u16*)v_cache, block_tables, bt_stride, block_size, shift, paired
+    if (by16) prefill_attn32_kernel<128, BLOCKS_OF_16><<<grid32, 512, 0, st>>>(PL_ARGS);
+    else prefill_attn32_kernel<128, PAGED ? BLOCKS : ROWS_OF_QKV><<<grid32, 512, 0, st>>>(PL_ARGS);
+#undef PL_ARGS
     DLI_RETURN_LAUNCH();
   }
   // waves per query head: pack 2 / 4 heads of one GQA group into a workgroup for short

@@ -24,12 +24,10 @@
 //                   of the group are the columns); the value sum in fp32 FMAs, a lane owning 8
 //                   dims of every head of the group: at one row per head it is far below the
 //                   time the bytes take, and V needs no transpose.
-#include "common.h"
+#include "lds_dma.h"
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) void lds_void;
 typedef const __attribute__((address_space(1))) void gbl_void;
 
 namespace {
@@ -107,9 +105,6 @@ constexpr int KT = 64;                 // keys a tile
 constexpr int LROWS = 256;             // query rows of a long-form workgroup
 constexpr float RESCALE_THR = 8.f;     // log2 units: the running max moves only by more than this
 
-// a value that is the same in all lanes, in a scalar register
-__device__ __forceinline__ uint32_t scalar(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
-
 // One tile of rows (D wide) by LDS-DMA: 1-KiB pieces of two subtiles in a row, wave w of 8 takes
 // pieces w, w + 8, ... The DMA writes lane-linearly, so each lane loads the logical chunk that
 // lands at its place. Columns from D1 on come from a second matrix (its rows alike).
@@ -131,12 +126,9 @@ __device__ __forceinline__ void stage_rows(const u16* src, long stride, const u1
   }
 }
 
-// The same tile from rows that lie together, by sixteens (TOGETHER = 16) or all 64 of it. Nothing of an address is left
-// to the lanes but their place among those rows (voff, of each piece), and what is past the last row lands as zeros.
-// rows: the descriptor of sixteen g's (tail: of the second matrix's)
-__device__ __forceinline__ u32x4 rows_at(uintptr_t first, int bytes) {
-  return {scalar((uint32_t)first), scalar((uint32_t)(first >> 32) & 0xffff), scalar((uint32_t)bytes), 0x00020000};
-}
+// The same tile from rows that lie together, by sixteens (TOGETHER = 16) or all 64 of it: a lane's offset (voff, of each
+// piece) is its place among those rows, and rows past the last land as zeros. rows: the descriptor of sixteen g's (tail:
+// of the second matrix's)
 template <int D, int D1, typename Rows>
 __device__ __forceinline__ void stage_together(uint32_t dst, int wid, const int (&voff)[(D / 8 + 7) / 8], const Rows& rows) {
   constexpr int NP = D / 8;
@@ -145,12 +137,7 @@ __device__ __forceinline__ void stage_together(uint32_t dst, int wid, const int 
     const int piece = wid + 8 * j;
     if (NP % 8 != 0 && piece >= NP) break;                     // wave-uniform
     const bool tail = D1 < D && piece * 1024 % (D * 16) / 16 >= D1;
-    const u32x4 rsrc = rows(piece * 64 / D >> 1, tail);
-    const uint32_t to = scalar(dst + piece * 1024);
-    // (inline asm: behind the builtins hipcc waits for every LDS-DMA in flight ahead of the transposing reads, this
-    // tile's among them. The wait states are a vector instruction's that wrote one of the scalars)
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-                 :: "s"(to), "v"(voff[j]), "s"(rsrc) : "memory", "m0");
+    dma_piece(dst + piece * 1024, voff[j], rows(piece * 64 / D >> 1, tail));
   }
 }
 template <int D, int D1, int TOGETHER>
@@ -242,7 +229,7 @@ __global__ void __launch_bounds__(512) swa_prefill32_kernel(SwaArgs a) {
     piece_offsets<DV, DV, DR ? KT : 16>(vv, a.v_stride, 0, wid, lane);
   }
   // GROUPS: where the next tile's rows begin (of a plain matrix; else the cache's first), and the bytes of a row
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_void*)lds;
+  const uint32_t lds0 = lds_address(lds);
   const int row_k = (int)a.k_stride * 2, row_v = (int)a.v_stride * 2, row_k2 = (int)a.k2_stride * 2;
   const long row0 = DR ? base + kl.skip : 0;
   uintptr_t at_k = (uintptr_t)(a.k + kvh * DK) + row0 * row_k, at_v = (uintptr_t)(a.v + kvh * DV) + row0 * row_v,
@@ -253,7 +240,7 @@ __global__ void __launch_bounds__(512) swa_prefill32_kernel(SwaArgs a) {
       const int left = kl.n - x0;                              // (only the last tile's are fewer than its rows)
       if constexpr (DR != 0) {
         const int n = left < KT ? left : KT;
-        const u32x4 head = rows_at(at_k, n * row_k), tail = rows_at(at_k2, n * row_k2), vals = rows_at(at_v, n * row_v);
+        const u32x4 head = bytes_at(at_k, n * row_k), tail = bytes_at(at_k2, n * row_k2), vals = bytes_at(at_v, n * row_v);
         stage_together<KW, DK>(to, wid, vk, [&](int, bool t) { return t ? tail : head; });
         stage_together<DV, DV>(to + TILE_K, wid, vv, [&](int, bool) { return vals; });
         at_k += KT * row_k, at_k2 += KT * row_k2, at_v += KT * row_v;
@@ -261,7 +248,7 @@ __global__ void __launch_bounds__(512) swa_prefill32_kernel(SwaArgs a) {
         const int rows4 = table[(x0 >> 4) + (lane & 3)];
         const auto rows = [&](uintptr_t m, int row, int g) {
           const int n = left - 16 * g;
-          return rows_at(m + (long)__builtin_amdgcn_readlane(rows4, g) * row, n >= 16 ? 16 * row : n > 0 ? n * row : 0);
+          return bytes_at(m + (long)__builtin_amdgcn_readlane(rows4, g) * row, n >= 16 ? 16 * row : n > 0 ? n * row : 0);
         };
         stage_together<KW, DK>(to, wid, vk, [&](int g, bool) { return rows(at_k, row_k, g); });
         stage_together<DV, DV>(to + TILE_K, wid, vv, [&](int g, bool) { return rows(at_v, row_v, g); });

@@ -1,7 +1,7 @@
-// LDS-DMA of 1-KiB pieces through descriptors in scalar registers, for kernels that count what is in flight themselves.
-// Nothing of an address is left to the lanes but a constant offset each, and what is out of a descriptor's range lands as
-// zeros. The request is inline asm: behind the builtins hipcc waits for every LDS-DMA in flight ahead of a transposing LDS
-// read, the youngest tile's among them (s_waitcnt vmcnt(0) in the middle of a tile). It has no result; what it has written is
+// LDS-DMA of 1-KiB pieces, for kernels that count what is in flight themselves; through descriptors in scalar registers
+// nothing of an address is left to the lanes but a constant offset each, and what is out of a descriptor's range lands as
+// zeros. The requests are inline asm: behind the builtins hipcc waits for every LDS-DMA in flight ahead of a transposing LDS
+// read, the youngest tile's among them (s_waitcnt vmcnt(0) in the middle of a tile). They have no result; what they have written is
 // read behind counted waits and a barrier.
 #pragma once
 #include "common.h"
@@ -24,4 +24,9 @@ __device__ __forceinline__ void dma_piece(uint32_t to, int voff, const u32x4 rsr
   const uint32_t m = scalar(to);
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
                :: "s"(m), "v"(voff), "s"(rsrc) : "memory", "m0");
+}
+// the same from an address of each lane's own
+__device__ __forceinline__ void dma_lanes(uint32_t to, const void* from) {
+  const uint32_t m = scalar(to);
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" :: "s"(m), "v"(from) : "memory", "m0");
 }

@@ -18,11 +18,11 @@
 // waves of a SIMD, in the same phase, wait for each other; the registers allow no third.
 // 4 x 2048 tokens, window 1024: the general form, which stages all heads' keys behind barriers, loads
 // the queries for every tile and transposes the values by 2-byte stores, 2264 us; this 147 + 496.
-// 8000 tokens, window 4096: 8141 -> 2052 us; 64 single ones at 1000 keys 306 -> 167.
-#include "common.h"
+// 8000 tokens, window 4096: 8141 -> 2052 us; 64 single ones at 1000 keys 306 -> 167. Since then a tile's values are
+// requested a whole tile ahead (they were just ahead of the wait for the next keys, which hipcc makes a wait for both):
+// both launches 562 -> 540, 8000 tokens, window 4000, 1787 -> 1704, the single ones 152 -> 135, to the bit.
+#include "lds_dma.h"
 
-typedef __attribute__((address_space(3))) void mix_lds_void;
-typedef const __attribute__((address_space(1))) void mix_gbl_void;
 typedef short mix_s16x4 __attribute__((ext_vector_type(4)));
 typedef short mix_s16x8 __attribute__((ext_vector_type(8)));
 
@@ -57,11 +57,12 @@ struct MixArgs {
 // 16-byte chunk of row r's values at c ^ swz(r): the transposed reads take 32 bytes of 4 rows
 __device__ __forceinline__ int swz(int r) { return ((r >> 1) & 3) << 1; }
 
-template <bool STATS>
+// NV: value tiles of a wave in LDS
+template <bool STATS, int NV>
 __global__ void __launch_bounds__(STATS ? 256 : 512) mix_attention_kernel(MixArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  u16* Vt = (u16*)smem;                            // [NW][TK][DVW]
-  u16* Pm = Vt + (STATS ? 0 : NW * TK * DVW);      // [TK * TQ][PROW]
+  u16* Vt = (u16*)smem;                            // [NW][NV][TK][DVW]
+  u16* Pm = Vt + (STATS ? 0 : NW * NV * TK * DVW); // [TK * TQ][PROW]
   u16* Wm = Pm + (STATS ? 0 : TK * TQ * PROW);     // [H * TQ][WROW]
   int* slot = (int*)(Wm + (STATS ? 0 : H * TQ * WROW));
   const int tid = threadIdx.x, lane = tid & 63;
@@ -127,25 +128,31 @@ __global__ void __launch_bounds__(STATS ? 256 : 512) mix_attention_kernel(MixArg
 #pragma unroll
     for (int kk = 0; kk < HD / 32; ++kk) kf[kb][kk] = *reinterpret_cast<const bf16x8*>(kr + kk * 32);
   };
-  u16* vt = Vt + wave * TK * DVW;
+  const u16* const vts = Vt + wave * NV * TK * DVW;
   const auto load_v = [&](int tile) {              // 8 rows of 128 bytes an instruction
+    const uint32_t to = lds_address(vts + tile % NV * TK * DVW);
 #pragma unroll
     for (int p = 0; p < TK / 8; ++p) {
       const int r = p * 8 + (lane >> 3), c = (lane & 7) ^ swz(r);
-      __builtin_amdgcn_global_load_lds(
-          (mix_gbl_void*)(a.v + (long)slot[tile * TK + r] * a.v_stride + grp * HD + dvo + c * 8),
-          (mix_lds_void*)(vt + p * 8 * DVW), 16, 0, 0);
+      dma_lanes(to + p * 8 * DVW * 2, a.v + (long)slot[tile * TK + r] * a.v_stride + grp * HD + dvo + c * 8);
     }
   };
+  // A tile's values are requested ahead of its keys, whose wait then is for both: with two value tiles a whole tile ahead.
+  // (hipcc counts the keys alone. With one value tile its requests follow the next keys', and the wait for those is for
+  // values that were requested just before)
+  if constexpr (!STATS) load_v(0);
   load_k(0, 0);
   load_k(0, 1);
-  asm volatile("" ::: "memory");                   // keys first, as in the loop: they are waited for
-  if constexpr (!STATS) load_v(0);                 // with the values in flight
 
   for (int tile = 0; tile < ntiles; ++tile) {
     const int j0 = lo + tile * TK;
     // (rows past the last query keep m = l = 0 or are not stored: whatever they hold stays theirs)
     const bool interior = j0 + TK - 1 <= p0 && j0 > p_last - a.window;
+    if constexpr (!STATS && NV == 2) {             // (behind hipcc's wait for the keys, which would be for these too)
+#pragma unroll
+      for (int kk = 0; kk < HD / 32; ++kk) asm volatile("" : "+v"(kf[0][kk]), "+v"(kf[1][kk]));
+      if (tile + 1 < ntiles) load_v(tile + 1);
+    }
     f32x4 sc[2][HW];
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {
@@ -234,9 +241,7 @@ __global__ void __launch_bounds__(STATS ? 256 : 512) mix_attention_kernel(MixArg
           }
       }
       __syncthreads();                             // mixed weights; the weights are read
-      // this tile's values were requested before the next tile's 8 key rows
-      if (tile + 1 < ntiles) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      const u16* vt = vts + tile % NV * TK * DVW;
       bf16x8 wf[HW];
 #pragma unroll
       for (int h = 0; h < HW; ++h)
@@ -258,7 +263,7 @@ __global__ void __launch_bounds__(STATS ? 256 : 512) mix_attention_kernel(MixArg
           o[h][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, wf[h], o[h][b], 0, 0, 0);
       }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // reads done before the tile is replaced
-      if (tile + 1 < ntiles) load_v(tile + 1);
+      if (NV == 1 && tile + 1 < ntiles) load_v(tile + 1);
     }
   }
 
@@ -332,11 +337,18 @@ extern "C" int dli_mix_attention(const void* q, int ldq, const void* k, long k_s
             ldg, slopes, talk, cu, positions, block_tables, bt_stride, block_size, G, window, qtiles,
             scale, out_scale, head_gate, (float*)ws};
   const size_t tables = (size_t)slots * 4;
-  const size_t sh = (size_t)(NW * TK * DVW + TK * TQ * PROW + H * TQ * WROW) * 2 + tables;
-  static const hipError_t raised = hipFuncSetAttribute(
-      (const void*)mix_attention_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+  const size_t vts = (size_t)NW * TK * DVW * 2, sh = vts + (TK * TQ * PROW + H * TQ * WROW) * 2 + tables;
+  // (two value tiles a wave to windows of 4064)
+  const bool two = sh + vts <= 160 * 1024;
+  static const hipError_t raised = [] {
+    const hipError_t e = hipFuncSetAttribute((const void*)mix_attention_kernel<false, 1>,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    return e != hipSuccess ? e : hipFuncSetAttribute((const void*)mix_attention_kernel<false, 2>,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+  }();
   if (raised != hipSuccess) return (int)raised;
-  mix_attention_kernel<true><<<2 * qtiles * num_seqs, 256, tables, st>>>(a);
-  mix_attention_kernel<false><<<2 * qtiles * num_seqs, 512, sh, st>>>(a);
+  mix_attention_kernel<true, 1><<<2 * qtiles * num_seqs, 256, tables, st>>>(a);
+  if (two) mix_attention_kernel<false, 2><<<2 * qtiles * num_seqs, 512, sh + vts, st>>>(a);
+  else mix_attention_kernel<false, 1><<<2 * qtiles * num_seqs, 512, sh, st>>>(a);
   DLI_RETURN_LAUNCH();
 }

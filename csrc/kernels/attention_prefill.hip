@@ -520,7 +520,7 @@ __global__ void __launch_bounds__(512) prefill_attn32_kernel(
 }
 
 // attention_prefill_long.hip; ctx_lens null: keys and values in the activation's rows
-int launch_prefill_long(void* out, int out_stride, const void* qkv, int row_stride, const int* cu_seqlens, int num_seqs,
+int launch_prefill_long(bool paired, void* out, int out_stride, const void* qkv, int row_stride, const int* cu_seqlens, int num_seqs,
                         int max_seqlen, int hq, int hkv, float scale_log2, const int* ctx_lens, const void* k_cache,
                         const void* v_cache, const int* block_tables, int bt_stride, int block_size, hipStream_t st);
 
@@ -546,6 +546,16 @@ static bool takes_wave64(bool paged, long T, int n, long L, int hq, int hd, int 
   return low >= 1200.0 + 2e5 * n / T;
 }
 
+// Whether a launch of up to a workgroup a CU takes waves of 64 rows in pairs of half blocks (attention_prefill_long.hip):
+// wherever that kernel can read the rows. It is ahead from 257 tokens on: 300 14.7 / 14.6 us, 400 18.8 / 16.0, 300 of 300
+// cached 15.5 / 15.5, 2048 of 8048 250 / 217 (54 mixes of lengths, contexts and heads: 0.80 to 1.00 of the time). Other
+// lengths than the default set by dli_prefill_set_wave64_len leave such launches to waves of 32 rows.
+static bool pairs_wave64(bool paged, int n, long L, int hq, int hd, int row_stride, int block_size) {
+  const long blocks = (L + PL_ROWS - 1) / PL_ROWS;
+  if (hd != 128 || L < g_pl_min_len || blocks < 2 || blocks * hq * n > PL_ROUND || g_pw_min_len != PW_MIN_LEN) return false;
+  return paged ? block_size >= 16 && !(block_size & (block_size - 1)) : (L + PL_ROWS) * row_stride * 2 < (1L << 31);
+}
+
 template <bool PAGED>
 static int launch_prefill(void* out, int out_stride, const void* qkv, int row_stride,
                           const int* cu_seqlens, int tokens, int num_seqs, int max_seqlen, int hq, int hkv,
@@ -555,8 +565,11 @@ static int launch_prefill(void* out, int out_stride, const void* qkv, int row_st
   if (num_seqs <= 0 || max_seqlen <= 0) return 0;
   if (hq % hkv || (hd != 64 && hd != 128)) return (int)hipErrorInvalidValue;
   const float sl2 = scale * 1.4426950408889634f;
-  if (takes_wave64(PAGED, tokens, num_seqs, max_seqlen, hq, hd, row_stride, block_size))
-    return launch_prefill_long(out, out_stride, qkv, row_stride, cu_seqlens, num_seqs, max_seqlen, hq, hkv, sl2,
+  // (their queries come by 16-byte LDS-DMA, as keys and values in the activation's rows do)
+  const bool whole = !PAGED || (row_stride % 8 == 0 && ((uintptr_t)qkv & 15) == 0);
+  const bool pairs = whole && pairs_wave64(PAGED, num_seqs, max_seqlen, hq, hd, row_stride, block_size);
+  if (pairs || (whole && takes_wave64(PAGED, tokens, num_seqs, max_seqlen, hq, hd, row_stride, block_size)))
+    return launch_prefill_long(pairs, out, out_stride, qkv, row_stride, cu_seqlens, num_seqs, max_seqlen, hq, hkv, sl2,
                                PAGED ? ctx_lens : nullptr, k_cache, v_cache, block_tables, bt_stride, block_size, st);
   if (hd == 128 && max_seqlen >= g_pl_min_len) {     // long sequences: 256-row workgroups
     const int blocks = (max_seqlen + PL_ROWS - 1) / PL_ROWS;
@@ -631,6 +644,11 @@ extern "C" int dli_prefill_set_min_len(int n) {
 extern "C" int dli_prefill_takes_wave64(int tokens, int num_seqs, int max_seqlen, int hq, int hd, int row_stride,
                                         int block_size) {
   return takes_wave64(block_size > 0, tokens, num_seqs, max_seqlen, hq, hd, row_stride, block_size) ? 1 : 0;
+}
+
+// 1 where it takes them in pairs of half blocks
+extern "C" int dli_prefill_pairs_wave64(int num_seqs, int max_seqlen, int hq, int hd, int row_stride, int block_size) {
+  return pairs_wave64(block_size > 0, num_seqs, max_seqlen, hq, hd, row_stride, block_size) ? 1 : 0;
 }
 
 extern "C" int dli_prefill_set_wave64_len(int n) {

@@ -14,6 +14,17 @@
 // maxima of t + 1. 32 heads on 8, us, that kernel / this one: 3000 tokens 97 / 87, 7993 516 / 471 (1.11 PFLOP/s), 16000 1930 / 1718, 4
 // x 4096 577 / 525; on another card 4096 of 8192 cached 416 / 389. Outputs are equal to the bit.
 //
+// A workgroup's fixed cost was 11 k cycles ahead of the first product and 6 k behind the last: queries read a row a
+// lane, outputs stored 8 bytes a row, 32 rows a request. Both go through a tile image a wave in LDS now, in whole rows;
+// and a cached tile's 130 scalar instructions (four cycles each beside the products) are 40 and 24 lane reads: 4 x 2048
+// tokens 160 -> 150 us, 8000 473 -> 460, 2 x 2048 of 4096 cached 208 -> 193, 4096 of 8192 384 -> 367.
+//
+// PAIRED (launches of up to a workgroup a CU): a wave's 64 rows are 32 of a half block counted from a sequence's start and
+// 32 of its counterpart from the end. Once the former see no more keys the wave goes on with the latter alone, an iteration
+// of half the products (2.1 k cycles a tile, 3.2 k with both): the workgroups' work is nearly equal, where whole
+// blocks would wait for the last. 32 heads on 8, us, the other kernel's pairs / these: 1024 tokens 30.1 / 25.0, 2048 51.9
+// / 44.7, 512 of 2560 cached 77.8 / 66.0, 2048 of 4096 121 / 106, 8 heads and 8000 tokens 163 / 139. Equal to the bit.
+//
 // K and V tiles come by LDS-DMA into rings of three slots, rows past the keys as zeros (range-checked descriptors).
 // In iteration t K(t + 1) and V(t) are read, K(t + 2) and V(t + 1) land, K(t + 3) and V(t + 2) are requested; the
 // only barrier, once the last of V(t) is read, ends all three. Causal: a workgroup's tiles stop at its last row's
@@ -23,6 +34,7 @@
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) void lds_void;
 typedef const __attribute__((address_space(1))) void gbl_void;
 typedef const __attribute__((address_space(3))) bf16x8 lds_frag;
@@ -44,14 +56,14 @@ constexpr float RESCALE_THR = 8.f;                 // log2 units: a running max 
 // tokens (others take the kernel of 8 waves).
 enum { ROWS_OF_QKV = 0, BLOCKS_OF_16 = 1 };
 
-template <int SRC>
+template <int SRC, bool PAIRED>
 __global__ void __launch_bounds__(256, 1) prefill_long_kernel(
     u16* __restrict__ out, int out_stride, const u16* __restrict__ qkv, int row_stride,
     const int* __restrict__ cu_seqlens, int hq, int hkv, float scale_log2,
     const int* __restrict__ ctx_lens, const u16* __restrict__ k_cache,
     const u16* __restrict__ v_cache, const int* __restrict__ block_tables, int bt_stride,
     int block_size, int block_shift) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];        // 3 K slots, 3 V slots, from address 0
+  extern __shared__ __attribute__((aligned(16))) char smem[];        // 3 K slots, 3 V slots, from address 0; a tile image a wave
   // Workgroups of a sequence: key heads fastest (round-robin over the XCDs: with 8 of them one L2
   // holds one head's K and V), then the query heads of a group, then row blocks, longest first over
   // all heads. Up to 4 heads leave too few of a sequence's blocks in flight before its empty ones come; there a
@@ -69,11 +81,17 @@ __global__ void __launch_bounds__(256, 1) prefill_long_kernel(
   if (blk >= nblk) return;                                           // workgroup-uniform
   const int nkeys = SRC ? __builtin_amdgcn_readfirstlane(ctx_lens[seq]) : len;
   const int qoff = nkeys - len;
-  const int q0 = blk * ROWS + wid * 64;                              // this wave's first row
-  const bool active = q0 < len;
-  const int wq_lo = qoff + q0, wq_hi = qoff + min(q0 + 64, len) - 1; // its first and last position
-  const int kend = min(nkeys, qoff + min((blk + 1) * ROWS, len));
-  const int ntiles = (kend + KT - 1) / KT, mine = active ? wq_hi / KT + 1 : 0;
+  // this wave's two blocks of 32 rows: their first rows, and the tiles that both take part in, and one of them. Paired,
+  // they are of a half block counted from the start and its counterpart from the end (the middle one of an odd number alone)
+  const int nhalf = (len + ROWS / 2 - 1) / (ROWS / 2), front = nblk - 1 - blk, back = nhalf - 1 - front;
+  const int row0[2] = {PAIRED ? front * (ROWS / 2) + wid * 32 : blk * ROWS + wid * 64,
+                       PAIRED ? back * (ROWS / 2) + wid * 32 : blk * ROWS + wid * 64 + 32};
+  const bool has0 = (!PAIRED || front != back) && row0[0] < len, active = has0 || (PAIRED && row0[1] < len);
+  const int end1 = (qoff + min(row0[1] + 32, len) - 1) / KT + 1;     // (unpaired, a wave's last block is behind its first)
+  const int both = !has0 ? 0 : PAIRED ? (qoff + min(row0[0] + 32, len) - 1) / KT + 1 : end1;
+  const int mine = PAIRED && row0[1] < len ? max(both, end1) : both;
+  const int kend = min(nkeys, qoff + min(PAIRED ? (back + 1) * (ROWS / 2) : (blk + 1) * ROWS, len));
+  const int ntiles = (kend + KT - 1) / KT;
 
   // ---- staging: a tile is 16 pieces of 1 KiB (two of the 8-row x 32-column subtiles of 512 B, the XOR image
   // of attention_prefill.hip's pl_off); wave w moves pieces w + 4 j of K and of V, j = 0..3: rows 16 j + rw
@@ -91,24 +109,30 @@ __global__ void __launch_bounds__(256, 1) prefill_long_kernel(
     return (uintptr_t)scalar((uint32_t)(uintptr_t)p) | (uintptr_t)scalar((uint32_t)((uintptr_t)p >> 32)) << 32;
   };
   const uintptr_t heads[2] = {uniform(first_k), uniform(first_v)};
-  // Rows: one descriptor a sequence and operand, the tile in the scalar offset. Blocks: a descriptor a piece, whose
-  // place and bytes V's piece, staged an iteration after K's, takes over
+  // Rows: one descriptor a sequence and operand, the tile in the scalar offset. Blocks: a descriptor a piece, of sixteen
+  // rows; a lane holds those of a sixteen (scalar arithmetic costs issue cycles beside the MFMAs), for 15 tiles at a time
+  // and the one before them, which V's pieces are of
   const int total = __builtin_amdgcn_readfirstlane((nkeys - 1) * stride + HD * 2);                   // (the launcher keeps a sequence's below 2^31)
   int row_at[2] = {0, 0};                                            // [K's tile, V's tile]
-  long at[2][4] = {};
-  int bytes[2][4] = {};
-  // the tile that K's pieces are of next, V's that which K's were of last
+  int held = 0, place = 0, held_bytes = 0;                           // lane 0's sixteen, the lane of the first of K's tile
+  uint32_t held_lo[2] = {0, 0}, held_hi[2] = {0, 0};
+  auto hold = [&](int from) __attribute__((always_inline)) {
+    held = from;
+    const int first = 16 * (held + lane);
+    const int id = btab[min(first, nkeys - 1) >> block_shift];
+    const long at = (long)id * ((long)hkv * block_size * HD * 2) + (first & (block_size - 1)) * (HD * 2);
+#pragma unroll
+    for (int kv = 0; kv < 2; ++kv) {
+      held_lo[kv] = (uint32_t)(heads[kv] + at);
+      held_hi[kv] = (uint32_t)((heads[kv] + at) >> 32) & 0xffff;
+    }
+    held_bytes = min(max(nkeys - first, 0), 16) * (HD * 2);
+  };
+  // the tile that K's pieces are of next; V's are of the one before
   auto find = [&](int t) __attribute__((always_inline)) {
     if constexpr (SRC == BLOCKS_OF_16) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        at[1][j] = at[0][j];
-        bytes[1][j] = bytes[0][j];
-        const int first = t * KT + 16 * j;
-        const int id = __builtin_amdgcn_readfirstlane(btab[min(first, nkeys - 1) >> block_shift]);
-        bytes[0][j] = __builtin_amdgcn_readfirstlane(min(max(nkeys - first, 0), 16) * (HD * 2));
-        at[0][j] = (long)id * ((long)hkv * block_size * HD * 2) + (first & (block_size - 1)) * (HD * 2);
-      }
+      if (4 * t + 4 - held > 64) hold(4 * t - 4);                    // wave-uniform
+      place = 4 * t - held;
     } else {
       row_at[1] = row_at[0];
       row_at[0] = t * (KT * stride);
@@ -116,44 +140,66 @@ __global__ void __launch_bounds__(256, 1) prefill_long_kernel(
   };
   // (inline asm: behind the builtin hipcc waits for every LDS-DMA in flight ahead of a transposing read. It has no
   // result, and what it has written is read behind counted waits and a barrier)
-  auto piece = [&](auto J, auto KV, uint32_t slot) __attribute__((always_inline)) {
+  // (beside the products every scalar instruction costs; elsewhere the wait states of a descriptor out of vector registers)
+  auto dma = [&](auto BESIDE, uint32_t dst, auto FURTHER, int lane_at, const u32x4& r, uint32_t so) __attribute__((always_inline)) {
+    if constexpr (decltype(BESIDE)::value)
+      asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds"
+                   :: "s"(dst), "i"(decltype(FURTHER)::value), "v"(lane_at), "s"(r), "s"(so) : "memory", "m0", "scc");
+    else
+      asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 4\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds"
+                   :: "s"(dst), "i"(decltype(FURTHER)::value), "v"(lane_at), "s"(r), "s"(so) : "memory", "m0", "scc");
+  };
+  auto descriptor = [&](uintptr_t base, int bytes) __attribute__((always_inline)) -> u32x4 {
+    return u32x4{scalar((uint32_t)base), scalar((uint32_t)(base >> 32) & 0xffff), scalar((uint32_t)bytes), 0x00020000};
+  };
+  // a piece's descriptor, and the piece to the slot at dst - wid KiB
+  auto where = [&](auto J, auto KV) __attribute__((always_inline)) -> u32x4 {
     constexpr int j = decltype(J)::value, kv = decltype(KV)::value;
-    const uintptr_t base = SRC == BLOCKS_OF_16 ? heads[kv] + at[kv][j] : heads[kv];
-    // (a row past the last is out of range whatever its columns: rows are at least 256 bytes apart)
-    const u32x4 r = {scalar((uint32_t)base), scalar((uint32_t)(base >> 32) & 0xffff),
-                     scalar((uint32_t)(SRC == BLOCKS_OF_16 ? bytes[kv][j] : total)), 0x00020000};
-    const uint32_t dst = scalar(slot + (wid + 4 * j) * 1024);
-    const uint32_t so = SRC == BLOCKS_OF_16 ? 0 : scalar((uint32_t)(row_at[kv] + j * 16 * stride));
-    const int lane_at = voff;
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                 :: "s"(dst), "v"(lane_at), "s"(r), "s"(so) : "memory", "m0");
+    if constexpr (SRC == BLOCKS_OF_16) {
+      const int l = place - 4 * kv + j;
+      return u32x4{(uint32_t)__builtin_amdgcn_readlane((int)held_lo[kv], l), (uint32_t)__builtin_amdgcn_readlane((int)held_hi[kv], l),
+                   (uint32_t)__builtin_amdgcn_readlane(held_bytes, l), 0x00020000};
+    } else {
+      return descriptor(heads[kv], total);
+    }
+  };
+  auto piece = [&](auto J, auto KV, auto BESIDE, uint32_t dst, const u32x4& r) __attribute__((always_inline)) {
+    constexpr int j = decltype(J)::value, kv = decltype(KV)::value;
+    dma(BESIDE, dst, int_c<4096 * j>{}, voff, r,
+        SRC == BLOCKS_OF_16 ? 0 : scalar((uint32_t)(row_at[kv] + j * 16 * stride)));
   };
   using K_ = int_c<0>;
   using V_ = int_c<1>;
-  constexpr uint32_t V0 = 3 * SLOT;
+  constexpr uint32_t V0 = 3 * SLOT, Q0 = 6 * SLOT;
   auto stage = [&](auto KV, uint32_t slot) __attribute__((always_inline)) {
-    unroll<4>([&](auto J) __attribute__((always_inline)) { piece(J, KV, slot); });
+    const uint32_t dst = scalar(slot + wid * 1024);
+    unroll<4>([&](auto J) __attribute__((always_inline)) { piece(J, KV, int_c<0>{}, dst, where(J, KV)); });
   };
-  // Q^T operand: lane (query qc, half hi) holds Q[q][16 c + 8 hi .. + 7]
-  bf16x8 qf[2][8];
-#pragma unroll
-  for (int qb = 0; qb < 2; ++qb) {
-    const u16* qp = qkv + (long)(s0 + min(q0 + 32 * qb + qc, len - 1)) * row_stride + (long)h * HD + 8 * hi;
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      const uint4 v = *reinterpret_cast<const uint4*>(qp + 16 * c);
-      asm volatile("" : "=a"(qf[qb][c]) : "0"(__builtin_bit_cast(bf16x8, v)));
-    }
-  }
+  if constexpr (SRC == BLOCKS_OF_16) hold(0);
   find(0);
   stage(K_{}, 0);
+  // this wave's queries, to a tile image of their own (a row a lane would take 32 rows a request)
+  const uint32_t mine_at = scalar(Q0 + wid * SLOT);
+  unroll<2>([&](auto QB) __attribute__((always_inline)) {
+    constexpr int qb = decltype(QB)::value;
+    const int left = min(max(len - row0[qb], 0), 32), rl = (lane & 31) >> 2;
+    const u32x4 r = descriptor((uintptr_t)(qkv + (long)(s0 + row0[qb]) * row_stride + (long)h * HD),
+                               left > 0 ? (left - 1) * row_stride * 2 + HD * 2 : 0);
+    const int at = rl * row_stride * 2 + 64 * (lane >> 5);
+    const int even = at + 16 * ((lane & 3) ^ (rl >> 2)), odd = at + 16 * ((lane & 3) ^ (2 + (rl >> 2)));
+    unroll<8>([&](auto I) __attribute__((always_inline)) {
+      constexpr int i = decltype(I)::value;
+      dma(int_c<0>{}, mine_at, int_c<8192 * qb + 1024 * i>{}, (i >> 1) & 1 ? odd : even, r,
+          scalar((uint32_t)((i >> 1) * 8 * row_stride * 2 + 128 * (i & 1))));
+    });
+  });
   find(1);
   stage(V_{}, V0);
   stage(K_{}, SLOT);
   find(2);
   stage(V_{}, V0 + SLOT);
   stage(K_{}, 2 * SLOT);
-  asm volatile("s_waitcnt vmcnt(8)" ::: "memory");                   // K(0), V(0) and K(1) landed
+  asm volatile("s_waitcnt vmcnt(16)" ::: "memory");                  // K(0) and Q landed
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
 
@@ -169,6 +215,15 @@ __global__ void __launch_bounds__(256, 1) prefill_long_kernel(
     vb[0] = V0 + 64 * (4 * hi + q4) + 16 * (cl ^ hi) + 8 * (p4 & 1);
     vb[1] = V0 + 2048 + 64 * (4 * hi + q4) + 16 * (cl ^ (hi ^ 2)) + 8 * (p4 & 1);
   }
+  // Q^T operand: lane (query qc, half hi) holds Q[q][16 c + 8 hi .. + 7]
+  bf16x8 qf[2][8];
+#pragma unroll
+  for (int qb = 0; qb < 2; ++qb)
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      const bf16x8 v = *(lds_frag*)(kb[c & 1] + mine_at + 8192 * qb + 512 * (c >> 1));
+      asm volatile("" : "=a"(qf[qb][c]) : "0"(v));
+    }
   // the slots of tiles t, t + 1 and t + 2: K(t + 3) goes to the first, V(t + 2) to the last
   uint32_t slot[3] = {0, SLOT, 2 * SLOT};
   auto turn = [&]() {
@@ -215,8 +270,10 @@ __global__ void __launch_bounds__(256, 1) prefill_long_kernel(
 
   // The products are inline asm, O and Q in the AGPR file; what reads their results stands many MFMAs behind them or
   // behind a pad of wait states, and fences keep it there
-  auto mma_s = [&](f32x16& d, const bf16x8& a, const bf16x8& b, auto FIRST) __attribute__((always_inline)) {
-    if constexpr (decltype(FIRST)::value)
+  auto mma_s = [&](f32x16& d, const bf16x8& a, const bf16x8& b, auto FIRST, auto FROM) __attribute__((always_inline)) {
+    if constexpr (decltype(FIRST)::value && decltype(FROM)::value)     // (its registers may have been written just before)
+      asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(d) : "v"(a), "a"(b));
+    else if constexpr (decltype(FIRST)::value)
       asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(d) : "v"(a), "a"(b));
     else
       asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(d) : "v"(a), "a"(b));
@@ -226,14 +283,14 @@ __global__ void __launch_bounds__(256, 1) prefill_long_kernel(
     asm volatile("s_nop 15\n\ts_nop 7" ::: "memory");
     fence();
   };
-  // scores of keys that a lane's queries do not see
-  auto mask = [&](auto P, int t) __attribute__((always_inline)) {
-    constexpr int p = decltype(P)::value;
+  // scores of keys that a lane's queries (from query block FROM on) do not see
+  auto mask = [&](auto P, auto FROM, int t) __attribute__((always_inline)) {
+    constexpr int p = decltype(P)::value, from = decltype(FROM)::value;
     const int k0 = t * KT;
-    if (k0 + KT - 1 > wq_lo || k0 + KT > nkeys) {
-      unroll<2>([&](auto QB) __attribute__((always_inline)) {
-        constexpr int qb = decltype(QB)::value;
-        const int last = min(wq_lo + 32 * qb + qc, nkeys - 1) - k0 - 4 * hi;   // in steps of this lane's keys
+    if (k0 + KT - 1 > qoff + row0[from] || k0 + KT > nkeys) {
+      unroll<2 - from>([&](auto QB) __attribute__((always_inline)) {
+        constexpr int qb = from + decltype(QB)::value;
+        const int last = min(qoff + row0[qb] + qc, nkeys - 1) - k0 - 4 * hi;   // in steps of this lane's keys
         unroll<32>([&](auto R) __attribute__((always_inline)) {
           constexpr int sub = decltype(R)::value >> 4, r = decltype(R)::value & 15;
           if (32 * sub + (r & 3) + 8 * (r >> 2) > last) s[p][sub][qb][r] = -INFINITY;
@@ -256,9 +313,9 @@ __global__ void __launch_bounds__(256, 1) prefill_long_kernel(
   // P <= 2^8 and O^T is rescaled for few tiles
   float rise[2];
   bool up[2];
-  auto running_max = [&](auto I) __attribute__((always_inline)) {
+  auto running_max = [&](auto I, auto FROM) __attribute__((always_inline)) {
 #pragma unroll
-    for (int qb = 0; qb < 2; ++qb) {
+    for (int qb = decltype(FROM)::value; qb < 2; ++qb) {
       constexpr int i = decltype(I)::value;
       if constexpr (i == 0) {
         const auto w = __builtin_amdgcn_permlane32_swap(__float_as_uint(top[qb]), __float_as_uint(top[qb]), false, false);
@@ -286,32 +343,34 @@ __global__ void __launch_bounds__(256, 1) prefill_long_kernel(
     unroll<16>([&](auto F) __attribute__((always_inline)) {
       constexpr int f = decltype(F)::value;
       const bf16x8 a = kfrag(F);
-      mma_s(s[0][f & 1][0], a, qf[0][f >> 1], std::integral_constant<bool, (f < 2)>{});
-      mma_s(s[0][f & 1][1], a, qf[1][f >> 1], std::integral_constant<bool, (f < 2)>{});
+      mma_s(s[0][f & 1][0], a, qf[0][f >> 1], std::integral_constant<bool, (f < 2)>{}, int_c<0>{});
+      mma_s(s[0][f & 1][1], a, qf[1][f >> 1], std::integral_constant<bool, (f < 2)>{}, int_c<0>{});
     });
     pad();
-    mask(int_c<0>{}, 0);
+    mask(int_c<0>{}, int_c<0>{}, 0);
     unroll<32>([&](auto I) __attribute__((always_inline)) { max_step(int_c<0>{}, I); });
-    unroll<5>(running_max);
-    k_base(SLOT);
-    unroll<DEEP>([&](auto F) __attribute__((always_inline)) { kf[decltype(F)::value] = kfrag(F); });
+    unroll<5>([&](auto I) __attribute__((always_inline)) { running_max(I, int_c<0>{}); });
   }
-  // every wave has read K(0), whose slot K(3) takes
+  // every wave has read K(0), whose slot K(3) takes; V(0) and K(1) landed
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_waitcnt(0xC07F);
+  asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
+  k_base(SLOT);
+  unroll<DEEP>([&](auto F) __attribute__((always_inline)) { kf[decltype(F)::value] = kfrag(F); });
 
   int t = 0;
-  // iteration t of parity P (the last one's scores and maxima are of no tile and no use: one code path)
-  auto iteration = [&](auto P) __attribute__((always_inline)) {
-    constexpr int p = decltype(P)::value;
+  // iteration t of parity P (the last one's scores and maxima are of no tile and no use: one code path), of the query
+  // blocks from FROM on
+  auto iteration = [&](auto P, auto FROM) __attribute__((always_inline)) {
+    constexpr int p = decltype(P)::value, from = decltype(FROM)::value, blocks = 2 - from;
     float sum[2] = {0.f, 0.f}, e_even = 0.f;
     uint32_t pw[2][16];
-    // element e: 16 a k-step of 16 keys, 8 a query block of these (pinned: hipcc sinks all of it past the branches
-    // below, to where it is used)
+    // element e: 16 (or 8) a k-step of 16 keys, 8 a query block of these (pinned: hipcc sinks all of it past the
+    // branches below, to where it is used)
     auto element = [&](auto E) __attribute__((always_inline)) {
-      constexpr int e = decltype(E)::value, ks = e >> 4, qb = (e >> 3) & 1, j = e & 7;
+      constexpr int e = decltype(E)::value, ks = e / (8 * blocks), qb = from ? 1 : (e >> 3) & 1, j = e & 7;
       float x = __builtin_amdgcn_exp2f(fmaf(s[p][ks >> 1][qb][8 * (ks & 1) + j], scale_log2, -mc[qb]));
       sum[qb] += x;
       asm volatile("" : "+v"(x), "+v"(sum[qb]));
@@ -322,17 +381,20 @@ __global__ void __launch_bounds__(256, 1) prefill_long_kernel(
         e_even = x;
       }
     };
-    constexpr int FRONT = 40;                      // elements beside the products with K
-    // ---- S(t + 1), elements 0..39
+    const uint32_t k_to = scalar(slot[0] + wid * 1024), v_to = scalar(V0 + slot[2] + wid * 1024);
+    u32x4 from_where;
+    constexpr int ALL = 32 * blocks, FRONT = 20 * blocks;              // elements, those beside the products with K
+    // ---- S(t + 1), elements 0..FRONT - 1
     unroll<32>([&](auto Q) __attribute__((always_inline)) {
       constexpr int q = decltype(Q)::value, f = q >> 1;
-      mma_s(s[1 - p][f & 1][q & 1], kf[f % DEEP], qf[q & 1][f >> 1], std::integral_constant<bool, (f < 2)>{});
+      if constexpr ((q & 1) >= from)
+        mma_s(s[1 - p][f & 1][q & 1], kf[f % DEEP], qf[q & 1][f >> 1], std::integral_constant<bool, (f < 2)>{}, FROM);
       if constexpr (q % 2 == 1 && f + DEEP < 16) kf[f % DEEP] = kfrag(int_c<(f + DEEP < 16 ? f + DEEP : 0)>{});
       if constexpr (q == 1) {
-        if (__ballot(alpha[0] != 1.f || alpha[1] != 1.f)) {
+        if (__ballot((from == 0 && alpha[0] != 1.f) || alpha[1] != 1.f)) {
           pad();
 #pragma unroll
-          for (int qb = 0; qb < 2; ++qb)
+          for (int qb = from; qb < 2; ++qb)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
               f32x16 v;
@@ -346,10 +408,14 @@ __global__ void __launch_bounds__(256, 1) prefill_long_kernel(
       }
       if constexpr (q == 31 - DEEP) v_base(slot[0]);
       if constexpr (q == 2) find(t + 3);
-      if constexpr (q >= 6 && q < 30 && q % 3 == 0) {
-        constexpr int n = q / 3 - 2;
-        if constexpr (n < 4) piece(int_c<n>{}, K_{}, slot[0]);
-        else piece(int_c<n - 4>{}, V_{}, V0 + slot[2]);
+      if constexpr (q >= 5 && q < 30) {                        // a piece, and two steps ahead of it where it is from
+        constexpr int n = (q + 1) / 3 - 2;
+        using KV = int_c<n / 4>;
+        if constexpr (q % 3 == 2 && n < 8) {
+          from_where = where(int_c<n % 4>{}, KV{});
+          if constexpr (SRC == BLOCKS_OF_16) asm volatile("" : "+s"(from_where));
+        }
+        if constexpr (q % 3 == 0) piece(int_c<n % 4>{}, KV{}, int_c<1>{}, n < 4 ? k_to : v_to, from_where);
       }
       if constexpr (q >= 32 - DEEP) vf[q - 32 + DEEP] = vfrag(int_c<(q >= 32 - DEEP ? q - 32 + DEEP : 0)>{});
       constexpr int e0 = q * FRONT / 32, e1 = (q + 1) * FRONT / 32;
@@ -360,17 +426,20 @@ __global__ void __launch_bounds__(256, 1) prefill_long_kernel(
     const float alpha_t[2] = {alpha[0], alpha[1]};
     unroll<32>([&](auto Q) __attribute__((always_inline)) {
       constexpr int q = decltype(Q)::value, f = q >> 1, ks = f >> 2, qb = q & 1;
-      const u32x4 w = {pw[qb][4 * ks], pw[qb][4 * ks + 1], pw[qb][4 * ks + 2], pw[qb][4 * ks + 3]};
-      asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0"
-                   : "+a"(o[qb][f & 3]) : "v"(vf[f % DEEP]), "v"(w));
-      if constexpr (q % 2 == 1 && f + DEEP < 16) vf[f % DEEP] = vfrag(int_c<(f + DEEP < 16 ? f + DEEP : 0)>{});
-      if constexpr (q < 64 - FRONT) element(int_c<(q < 64 - FRONT ? FRONT + q : 0)>{});
-      if constexpr (q == 4) mask(int_c<1 - p>{}, t + 1);       // (four products behind the last of S(t + 1))
-      if constexpr (q >= 4 && q < 20) {
-        max_step(int_c<1 - p>{}, int_c<2 * (q - 4)>{});
-        max_step(int_c<1 - p>{}, int_c<2 * (q - 4) + 1>{});
+      if constexpr (qb >= from) {
+        const u32x4 w = {pw[qb][4 * ks], pw[qb][4 * ks + 1], pw[qb][4 * ks + 2], pw[qb][4 * ks + 3]};
+        asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0"
+                     : "+a"(o[qb][f & 3]) : "v"(vf[f % DEEP]), "v"(w));
       }
-      if constexpr (q >= 20 && q < 25) running_max(int_c<q - 20>{});
+      if constexpr (q % 2 == 1 && f + DEEP < 16) vf[f % DEEP] = vfrag(int_c<(f + DEEP < 16 ? f + DEEP : 0)>{});
+      if constexpr (q < ALL - FRONT) element(int_c<(q < ALL - FRONT ? FRONT + q : 0)>{});
+      constexpr int M = 4 * (1 + from);                        // (four products behind the last of S(t + 1))
+      if constexpr (q == M) mask(int_c<1 - p>{}, FROM, t + 1);
+      if constexpr (q >= M && q < M + 16) {
+        if constexpr (from == 0) max_step(int_c<1 - p>{}, int_c<2 * (q - M)>{});
+        max_step(int_c<1 - p>{}, int_c<2 * (q - M) + 1>{});
+      }
+      if constexpr (q >= M + 16 && q < M + 21) running_max(int_c<q - M - 16>{}, FROM);
       if constexpr (q == 24) {
         turn();
         __builtin_amdgcn_s_waitcnt(0xC07F);        // lgkmcnt(0): V(t) is read
@@ -385,20 +454,38 @@ __global__ void __launch_bounds__(256, 1) prefill_long_kernel(
     });
     static_assert(24 + DEEP < 32 && 2 * (15 - DEEP) + 1 < 24);
 #pragma unroll
-    for (int qb = 0; qb < 2; ++qb) l_run[qb] = l_run[qb] * alpha_t[qb] + sum[qb];
+    for (int qb = from; qb < 2; ++qb) l_run[qb] = l_run[qb] * alpha_t[qb] + sum[qb];
     ++t;
   };
+  using TWO = int_c<0>;
+  using LAST = int_c<1>;
   // (with an exit between the two hipcc moves O between register files on the way round)
-  while (t + 1 < mine) {
-    iteration(int_c<0>{});
-    iteration(int_c<1>{});
+  while (t + 1 < both) {
+    iteration(int_c<0>{}, TWO{});
+    iteration(int_c<1>{}, TWO{});
   }
   // (what follows reads O, hipcc's copies of it where these paths meet included: the wait states on each of them)
-  if (t < mine) {
-    iteration(int_c<0>{});
+  if (t < both) {
+    iteration(int_c<0>{}, TWO{});
     pad();
+    if (PAIRED && t < mine) {
+      iteration(int_c<1>{}, LAST{});
+      pad();
+    }
   } else {
     pad();
+  }
+  if constexpr (PAIRED) {                          // t is even, or all of them
+    while (t + 1 < mine) {
+      iteration(int_c<0>{}, LAST{});
+      iteration(int_c<1>{}, LAST{});
+    }
+    if (t < mine) {
+      iteration(int_c<0>{}, LAST{});
+      pad();
+    } else {
+      pad();
+    }
   }
   // the workgroup's other tiles: this wave's share of the staging, and the barriers
   for (; t < ntiles; ++t) {
@@ -412,52 +499,63 @@ __global__ void __launch_bounds__(256, 1) prefill_long_kernel(
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // no LDS-DMA outlives the workgroup
   if (!active) return;
+  // O through the queries' image, 256-byte rows whose 16-byte chunk c lies at c ^ (row & 15): stores of whole rows (8
+  // bytes a lane, of 32 rows a store, took 6 k cycles)
 #pragma unroll
   for (int qb = 0; qb < 2; ++qb) {
     const auto w = __builtin_amdgcn_permlane32_swap(__float_as_uint(l_run[qb]), __float_as_uint(l_run[qb]), false, false);
     const float l = __uint_as_float(w[0]) + __uint_as_float(w[1]);
     const float inv = l > 0.f ? 1.f / l : 0.f;
-    const int qr = q0 + 32 * qb + qc;
-    u16* op = out + (long)(s0 + qr) * out_stride + (long)h * HD;
+    const uint32_t to = mine_at + 8192 * qb + 256 * qc + 8 * hi;
 #pragma unroll
     for (int db = 0; db < 4; ++db) {
       f32x16 v;
       asm volatile("" : "=v"(v) : "0"(o[qb][db]));
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const uint2 x = {pack2bf(v[4 * g] * inv, v[4 * g + 1] * inv), pack2bf(v[4 * g + 2] * inv, v[4 * g + 3] * inv)};
-        if (qr < len) *reinterpret_cast<uint2*>(op + 32 * db + 8 * g + 4 * hi) = x;
-      }
+      for (int g = 0; g < 4; ++g)
+        *(__attribute__((address_space(3))) u32x2*)(to + 16 * ((4 * db + g) ^ (qc & 15))) =
+            u32x2{pack2bf(v[4 * g] * inv, v[4 * g + 1] * inv), pack2bf(v[4 * g + 2] * inv, v[4 * g + 3] * inv)};
     }
+  }
+  asm volatile("" ::: "memory");
+  const int r4 = lane >> 4, c16 = lane & 15;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int qb = i >> 3, row = 4 * (i & 7) + r4, qr = row0[qb] + row;
+    const u32x4 x = *(const __attribute__((address_space(3))) u32x4*)(mine_at + 8192 * qb + 256 * row + 16 * (c16 ^ (row & 15)));
+    if (qr < len && (qb == 1 || has0))
+      *reinterpret_cast<u32x4*>(out + (long)(s0 + qr) * out_stride + (long)h * HD + 8 * c16) = x;
   }
 }
 
-template <int SRC>
+template <int SRC, bool PAIRED>
 static int launch_src(dim3 grid, void* out, int out_stride, const void* qkv, int row_stride, const int* cu_seqlens,
                       int hq, int hkv, float scale_log2, const int* ctx_lens, const void* k_cache, const void* v_cache,
                       const int* block_tables, int bt_stride, int block_size, int shift, hipStream_t st) {
-  constexpr int lds = 6 * SLOT;
+  constexpr int lds = 10 * SLOT;
   static bool raised = false;
   if (!raised) {
-    hipFuncSetAttribute((const void*)prefill_long_kernel<SRC>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    hipFuncSetAttribute((const void*)prefill_long_kernel<SRC, PAIRED>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     raised = true;
   }
-  prefill_long_kernel<SRC><<<grid, 256, lds, st>>>((u16*)out, out_stride, (const u16*)qkv, row_stride, cu_seqlens, hq,
-                                                   hkv, scale_log2, ctx_lens, (const u16*)k_cache, (const u16*)v_cache,
-                                                   block_tables, bt_stride, block_size, shift);
+  prefill_long_kernel<SRC, PAIRED><<<grid, 256, lds, st>>>((u16*)out, out_stride, (const u16*)qkv, row_stride, cu_seqlens,
+                                                           hq, hkv, scale_log2, ctx_lens, (const u16*)k_cache,
+                                                           (const u16*)v_cache, block_tables, bt_stride, block_size, shift);
   DLI_RETURN_LAUNCH();
 }
 
 // ctx_lens null: keys and values in the activation's rows. scale_log2: the scores' scale times log2 e
-int launch_prefill_long(void* out, int out_stride, const void* qkv, int row_stride, const int* cu_seqlens, int num_seqs,
+int launch_prefill_long(bool paired, void* out, int out_stride, const void* qkv, int row_stride, const int* cu_seqlens, int num_seqs,
                         int max_seqlen, int hq, int hkv, float scale_log2, const int* ctx_lens, const void* k_cache,
                         const void* v_cache, const int* block_tables, int bt_stride, int block_size, hipStream_t st) {
   const int blocks = (max_seqlen + ROWS - 1) / ROWS;
   const dim3 grid = hq <= 4 ? dim3(blocks, num_seqs, hq) : dim3(blocks * hq, num_seqs);
 #define DLI_ARGS out, out_stride, qkv, row_stride, cu_seqlens, hq, hkv, scale_log2, ctx_lens, k_cache, v_cache, \
                  block_tables, bt_stride, block_size
-  if (ctx_lens == nullptr) return launch_src<ROWS_OF_QKV>(grid, DLI_ARGS, 0, st);
+  if (ctx_lens == nullptr)
+    return paired ? launch_src<ROWS_OF_QKV, true>(grid, DLI_ARGS, 0, st) : launch_src<ROWS_OF_QKV, false>(grid, DLI_ARGS, 0, st);
   if (block_size < 16 || (block_size & (block_size - 1))) return (int)hipErrorInvalidValue;
-  return launch_src<BLOCKS_OF_16>(grid, DLI_ARGS, __builtin_ctz(block_size), st);
+  const int shift = __builtin_ctz(block_size);
+  return paired ? launch_src<BLOCKS_OF_16, true>(grid, DLI_ARGS, shift, st) : launch_src<BLOCKS_OF_16, false>(grid, DLI_ARGS, shift, st);
 #undef DLI_ARGS
 }

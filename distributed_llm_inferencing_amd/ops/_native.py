@@ -45,6 +45,7 @@ _SIGS = {
     "dli_prefill_set_min_len": [I],
     "dli_prefill_set_wave64_len": [I],
     "dli_prefill_takes_wave64": [I, I, I, I, I, I, I],
+    "dli_prefill_pairs_wave64": [I, I, I, I, I, I],
     "dli_prefill_set_pack": [I],
     "dli_sample_set_split_max_b": [I],
     "dli_decode_set_form": [I],

@@ -255,7 +255,10 @@ __device__ __forceinline__ float pl_max3(float a, float b, float c) {  // no can
 // SRC: the activation's rows; cache blocks of a power of two of at least 16 tokens, whose rows lie together by sixteens
 // and are staged through scalar descriptors (lds_dma.h); other blocks, row by row, whose table every lane reads, behind
 // all DMA in flight. 2048 queries of 4096 keys 133 -> 126 us, 1024 of 6000 174 -> 163, 6 x 400 of 2400 147 -> 138. The
-// activation's rows gain nothing so (4 x 1000 62.2 and 61.9, 2048 51.4 and 51.6)
+// activation's rows gain nothing so (4 x 1000 62.2 and 61.9, 2048 51.4 and 51.6).
+// whole: queries at 16-byte addresses. They come, and outputs leave, through a row image a wave in LDS: row by row a lane each
+// request took 32 rows, 10 k cycles a workgroup in all. 32 heads on 8, us: 8 x 256 tokens 19.0 -> 15.4, 20 x 400 81 -> 73, 8 of
+// 300 to 2000 125 -> 114, 5 x 1500 132 -> 126, 8 x 1000 of 2000 cached 238 -> 232. Equal to the bit.
 enum { ROWS_OF_QKV = 0, BLOCKS_OF_16 = 1, BLOCKS = 2 };
 template <int HD, int SRC>
 __global__ void __launch_bounds__(512) prefill_attn32_kernel(
@@ -263,7 +266,7 @@ __global__ void __launch_bounds__(512) prefill_attn32_kernel(
     const int* __restrict__ cu_seqlens, int hq, int hkv, float scale_log2,
     const int* __restrict__ ctx_lens, const u16* __restrict__ k_cache,
     const u16* __restrict__ v_cache, const int* __restrict__ block_tables, int bt_stride,
-    int block_size, int block_shift, bool paired) {
+    int block_size, int block_shift, bool paired, bool whole) {
   static_assert(HD == 128, "long-sequence kernel: head_dim 128");
   constexpr bool PAGED = SRC != ROWS_OF_QKV;
   constexpr int KC = HD / 16;                      // K-steps of the QK^T product
@@ -271,6 +274,7 @@ __global__ void __launch_bounds__(512) prefill_attn32_kernel(
   constexpr int TILE_B = PL_KT * HD * 2;           // bytes per K (or V) tile image
   constexpr int NBUF = 3;
   __shared__ __attribute__((aligned(16))) char lds[NBUF][2][TILE_B];   // [buf][K/V]
+  __shared__ __attribute__((aligned(16))) char rows_lds[PL_WAVES][PL_QROWS * HD * 2];   // a wave's queries, then its outputs
   // Workgroups of a sequence: key heads fastest (round-robin over the XCDs: with 8 of them one L2
   // holds one head's K and V), then the query heads of a group, then row blocks, longest first over
   // all heads. With the blocks of a head fastest the last heads' long blocks started when other CUs
@@ -291,7 +295,8 @@ __global__ void __launch_bounds__(512) prefill_attn32_kernel(
   const int nkeys = PAGED ? ctx_lens[seq] : len;
   const int qoff = nkeys - len;
   // Up to a workgroup for each CU there is nothing to even out the causal bounds with, and the last
-  // block's workgroup, which sees most keys, takes as long as the launch. Paired, waves 0 to 3 take a
+  // block's workgroup, which sees most keys, takes as long as the launch (where the kernel with 64 rows a wave cannot read
+  // the rows, which is ahead there: pairs_wave64). Paired, waves 0 to 3 take a
   // half block counted from the end and waves 4 to 7 its counterpart from the start: a SIMD, which
   // holds one wave of each, has the long one to itself when the short one is through. 32 heads, us:
   // 2048 tokens 78 -> 66, 1024 45 -> 40, the second 2048 of a prompt 150 -> 135, 1024 after 5000 192 -> 185.
@@ -307,9 +312,18 @@ __global__ void __launch_bounds__(512) prefill_attn32_kernel(
   const int* btab = PAGED ? block_tables + (long)seq * bt_stride : nullptr;
   const long head_off = (long)kvh * block_size * HD;
 
-  // Q^T operand: lane (query qc, half hi) holds Q[q][16c + 8hi .. +7]
+  // Q^T operand: lane (query qc, half hi) holds Q[q][16c + 8hi .. +7]. Rows at 16-byte addresses come as a tile image (a row
+  // a lane takes 32 rows a request, 4 k cycles ahead of the first tile)
   bf16x8 qf[KC];
-  {
+  if (whole) {
+    const int rl = (lane & 31) >> 2;
+    const uint32_t to = lds_address(&rows_lds[wid][0]);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int r = 8 * (i >> 1) + rl, c = 4 * (2 * (i & 1) + (lane >> 5)) + ((lane & 3) ^ ((r >> 2) & 3));
+      dma_lanes(to + 1024 * i, qkv + (long)(s0 + min(q0 + r, len - 1)) * row_stride + (long)h * HD + c * 8);
+    }
+  } else {
     const int qr = min(q0 + qc, len - 1);
     const u16* qp = qkv + (long)(s0 + qr) * row_stride + (long)h * HD + 8 * hi;
 #pragma unroll
@@ -384,7 +398,7 @@ __global__ void __launch_bounds__(512) prefill_attn32_kernel(
   stage(0, 0);
   // the queries are there from here on: hipcc would wait for them where it first uses them, in every tile, and so for the
   // DMA in flight, which it does not count
-  if (SRC == BLOCKS_OF_16) {
+  if (SRC == BLOCKS_OF_16 && !whole) {
 #pragma unroll
     for (int c = 0; c < KC; ++c) asm volatile("" : "+v"(qf[c]));
   }
@@ -406,6 +420,13 @@ __global__ void __launch_bounds__(512) prefill_attn32_kernel(
     const int cl = 2 * (g16 & 1) + (p4 >> 1);
     vbase_off[0] = 64 * (4 * hi + q4) + 16 * (cl ^ hi) + 8 * (p4 & 1);
     vbase_off[1] = 2048 + 64 * (4 * hi + q4) + 16 * (cl ^ (hi ^ 2)) + 8 * (p4 & 1);
+  }
+  if (whole) {
+#pragma unroll
+    for (int c = 0; c < KC; ++c) {
+      qf[c] = *reinterpret_cast<const bf16x8*>(&rows_lds[wid][kbase_off[c & 1] + 512 * (c >> 1)]);
+      asm volatile("" : "+v"(qf[c]));
+    }
   }
   // One barrier per tile: tile t+2 is DMA'd into the buffer tile t-1 used while tile t is
   // computed; the counted vmcnt + barrier closing iteration t retire tile t+1. (A variant
@@ -504,18 +525,22 @@ __global__ void __launch_bounds__(512) prefill_attn32_kernel(
   if (!active) return;
   const float l_tot = l_part + __shfl_xor(l_part, 32, 64);
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-  const int qr = q0 + qc;
-  if (qr < len) {
-    u16* op = out + (long)(s0 + qr) * out_stride + (long)h * HD;
+  // through the wave's rows in LDS, whose 16-byte chunk c lies at c ^ (row & 15): stores of whole rows
+  char* const rows = rows_lds[wid];
 #pragma unroll
-    for (int db = 0; db < DBK; ++db)
+  for (int db = 0; db < DBK; ++db)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        U16x4 v;
+    for (int g = 0; g < 4; ++g) {
+      U16x4 v;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v.v[r] = f2bf(o[db][4 * g + r] * inv);
-        *reinterpret_cast<U16x4*>(op + 32 * db + 8 * g + 4 * hi) = v;
-      }
+      for (int r = 0; r < 4; ++r) v.v[r] = f2bf(o[db][4 * g + r] * inv);
+      *reinterpret_cast<U16x4*>(rows + 256 * qc + 16 * ((4 * db + g) ^ (qc & 15)) + 8 * hi) = v;
+    }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int r = 4 * i + (lane >> 4), c = lane & 15;
+    const uint4 v = *reinterpret_cast<const uint4*>(rows + 256 * r + 16 * (c ^ (r & 15)));
+    if (q0 + r < len) *reinterpret_cast<uint4*>(out + (long)(s0 + q0 + r) * out_stride + (long)h * HD + c * 8) = v;
   }
 }
 
@@ -565,10 +590,10 @@ static int launch_prefill(void* out, int out_stride, const void* qkv, int row_st
   if (num_seqs <= 0 || max_seqlen <= 0) return 0;
   if (hq % hkv || (hd != 64 && hd != 128)) return (int)hipErrorInvalidValue;
   const float sl2 = scale * 1.4426950408889634f;
-  // (their queries come by 16-byte LDS-DMA, as keys and values in the activation's rows do)
-  const bool whole = !PAGED || (row_stride % 8 == 0 && ((uintptr_t)qkv & 15) == 0);
-  const bool pairs = whole && pairs_wave64(PAGED, num_seqs, max_seqlen, hq, hd, row_stride, block_size);
-  if (pairs || (whole && takes_wave64(PAGED, tokens, num_seqs, max_seqlen, hq, hd, row_stride, block_size)))
+  // queries come by 16-byte LDS-DMA, as keys and values in the activation's rows do
+  const bool whole = row_stride % 8 == 0 && ((uintptr_t)qkv & 15) == 0;
+  const bool pairs = (whole || !PAGED) && pairs_wave64(PAGED, num_seqs, max_seqlen, hq, hd, row_stride, block_size);
+  if (pairs || ((whole || !PAGED) && takes_wave64(PAGED, tokens, num_seqs, max_seqlen, hq, hd, row_stride, block_size)))
     return launch_prefill_long(pairs, out, out_stride, qkv, row_stride, cu_seqlens, num_seqs, max_seqlen, hq, hkv, sl2,
                                PAGED ? ctx_lens : nullptr, k_cache, v_cache, block_tables, bt_stride, block_size, st);
   if (hd == 128 && max_seqlen >= g_pl_min_len) {     // long sequences: 256-row workgroups
@@ -578,7 +603,7 @@ static int launch_prefill(void* out, int out_stride, const void* qkv, int row_st
     const bool by16 = PAGED && block_size >= 16 && (block_size & (block_size - 1)) == 0;
     const int shift = by16 ? __builtin_ctz(block_size) : 0;
 #define PL_ARGS (u16*)out, out_stride, (const u16*)qkv, row_stride, cu_seqlens, hq, hkv, sl2, ctx_lens, \
-                (const u16*)k_cache, (const u16*)v_cache, block_tables, bt_stride, block_size, shift, paired
+                (const u16*)k_cache, (const u16*)v_cache, block_tables, bt_stride, block_size, shift, paired, whole
     if (by16) prefill_attn32_kernel<128, BLOCKS_OF_16><<<grid32, 512, 0, st>>>(PL_ARGS);
     else prefill_attn32_kernel<128, PAGED ? BLOCKS : ROWS_OF_QKV><<<grid32, 512, 0, st>>>(PL_ARGS);
 #undef PL_ARGS

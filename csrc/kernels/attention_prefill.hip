@@ -33,7 +33,11 @@ typedef short s16x8 __attribute__((ext_vector_type(8)));
 #define PF_QROWS 16
 #define PF_KT 64
 
-template <int HD, bool PAGED>
+// KT: keys of a tile, 32 where no sequence has more: half of a tile of 64 was copies of the last row. There outputs leave
+// through LDS in whole rows (two bytes a lane are 32 B of four rows a store; with tiles of 64 that changes
+// nothing: 64 x 128 tokens 53.9 and 55.3 us). 32 heads on 8: 512 x 32 tokens 92.7 -> 83.4 us (330 MB, 4.0 TB/s), 512 of 17 to
+// 32 75.6 -> 66.4, 512 x 16 45.6 -> 39; head dim 64 54.5 -> 46.4. Equal to the bit.
+template <int HD, bool PAGED, int KT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) prefill_attn_kernel(
     u16* __restrict__ out, int out_stride, const u16* __restrict__ qkv, int row_stride,
     const int* __restrict__ cu_seqlens, int hq, int hkv, float scale_log2,
@@ -48,9 +52,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))
   constexpr int KROW = HD + 16;
   constexpr int VROW = HD + 16;                    // V row in LDS (u16): hd*2 + 32 B
   constexpr int CH = HD / 8;                       // 16-B chunks per row
-  constexpr int PER = PF_KT * CH / 256;            // chunks per thread per tile (K or V)
-  __shared__ __attribute__((aligned(16))) u16 ktile[PF_KT * KROW];
-  __shared__ __attribute__((aligned(16))) u16 vtile[PF_KT * VROW];
+  constexpr int PER = KT * CH / 256;            // chunks per thread per tile (K or V)
+  static_assert(KROW == VROW && 2 * KT >= PF_WAVES * PF_QROWS, "the outputs' rows in the tiles' place");
+  __shared__ __attribute__((aligned(16))) u16 tiles[2 * KT * KROW];
+  u16 *const ktile = tiles, *const vtile = tiles + KT * KROW;
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const int seq = blockIdx.y, h = blockIdx.z * (PF_WAVES / wph) + wid / wph;
   const int col = lane & 15, grp = lane >> 4;
@@ -89,7 +94,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))
   // the next K/V tile in flight in registers: named values, not arrays — uint4 kreg[PER]
   // indexed in a loop was promoted to LDS by the compiler (a second staging copy through
   // LDS, its bank conflicts counted with the tile's: profiles/r6/README.md §12)
-  static_assert(PER == 2 || PER == 4, "tile staging assumes 2 or 4 chunks per thread");
+  static_assert(PER == 1 || PER == 2 || PER == 4, "tile staging assumes 1, 2 or 4 chunks per thread");
   uint4 kr0, kr1, kr2, kr3, vr0, vr1, vr2, vr3;
   auto load1 = [&](int j, int k0, uint4& kr, uint4& vr) {
     const int i = tid + 256 * j;
@@ -108,7 +113,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))
   };
   auto load_tile = [&](int k0) {
     load1(0, k0, kr0, vr0);
-    load1(1, k0, kr1, vr1);
+    if constexpr (PER >= 2) load1(1, k0, kr1, vr1);
     if constexpr (PER == 4) {
       load1(2, k0, kr2, vr2);
       load1(3, k0, kr3, vr3);
@@ -122,21 +127,21 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))
   };
   load_tile(0);
   const int qrow = (lane >> 2) & 3, pcol = lane & 3;
-  for (int k0 = 0; k0 < kend_wg; k0 += PF_KT) {
+  for (int k0 = 0; k0 < kend_wg; k0 += KT) {
     __syncthreads();                                             // previous tile fully read
     store1(0, kr0, vr0);
-    store1(1, kr1, vr1);
+    if constexpr (PER >= 2) store1(1, kr1, vr1);
     if constexpr (PER == 4) {
       store1(2, kr2, vr2);
       store1(3, kr3, vr3);
     }
     __syncthreads();                                             // tile visible to all waves
-    if (k0 + PF_KT < kend_wg) load_tile(k0 + PF_KT);             // in flight during compute
+    if (k0 + KT < kend_wg) load_tile(k0 + KT);             // in flight during compute
     if (!active || k0 >= kend_w) continue;                       // tile above this wave's rows
-    // ---- S^T = K . Q^T over four 16-key subtiles
-    f32x4 s_acc[4];
+    // ---- S^T = K . Q^T over 16-key subtiles
+    f32x4 s_acc[KT / 16];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
+    for (int s = 0; s < KT / 16; ++s) {
       const u16* kp = ktile + (16 * s + col) * KROW;
       s_acc[s] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -144,9 +149,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))
         s_acc[s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
             *reinterpret_cast<const bf16x8*>(kp + kk * 32 + grp * 8), qf[kk], s_acc[s], 0, 0, 0);
     }
-    float p[16], tmax = -INFINITY;
+    float p[KT / 4], tmax = -INFINITY;
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
+    for (int s = 0; s < KT / 16; ++s)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int key = k0 + 16 * s + 4 * grp + r;
@@ -163,7 +168,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))
     m_run = m_new;
     float psum = 0.f;
 #pragma unroll
-    for (int j = 0; j < 16; ++j) { p[j] = exp2f(p[j] - m_use); psum += p[j]; }
+    for (int j = 0; j < KT / 4; ++j) { p[j] = exp2f(p[j] - m_use); psum += p[j]; }
     l_part = l_part * alpha + psum;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -171,10 +176,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))
 #pragma unroll
       for (int i = 0; i < DB; ++i) o_acc[i][r] *= a;
     }
-    // ---- O += P . V, two 32-key halves; B operand rows: keys 32h + 4grp + q and
+    // ---- O += P . V, by 32 keys; B operand rows: keys 32h + 4grp + q and
     // 32h + 16 + 4grp + q (the p[] key order), cols 16i + 4p via tr16 reads
 #pragma unroll
-    for (int hh = 0; hh < 2; ++hh) {
+    for (int hh = 0; hh < KT / 32; ++hh) {
       bf16x8 pa;
 #pragma unroll
       for (int j = 0; j < 8; ++j) pa[j] = (__bf16)p[8 * hh + j];
@@ -192,18 +197,28 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))
       }
     }
   }
+  if constexpr (KT == 32) __syncthreads();                       // the last tile fully read
   if (!active) return;
   float l_tot = l_part + __shfl_xor(l_part, 16, 64);
   l_tot += __shfl_xor(l_tot, 32, 64);
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+  u16* const ot = tiles + wid * PF_QROWS * KROW;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const float iv = __shfl(inv, 4 * grp + r, 64);
     const int qr = q0 + 4 * grp + r;
-    if (qr < len) {
-      u16* op = out + (long)(s0 + qr) * out_stride + (long)h * HD;
+    if (KT == 32 || qr < len) {
+      u16* op = KT == 32 ? ot + (4 * grp + r) * KROW : out + (long)(s0 + qr) * out_stride + (long)h * HD;
 #pragma unroll
       for (int i = 0; i < DB; ++i) op[16 * i + col] = f2bf(o_acc[i][r] * iv);
+    }
+  }
+  if constexpr (KT == 32) {
+#pragma unroll
+    for (int j = 0; j < PF_QROWS * CH / 64; ++j) {
+      const int r = (lane + 64 * j) / CH, c = (lane + 64 * j) % CH;
+      const uint4 v = *reinterpret_cast<const uint4*>(ot + r * KROW + 8 * c);
+      if (q0 + r < len) *reinterpret_cast<uint4*>(out + (long)(s0 + q0 + r) * out_stride + (long)h * HD + 8 * c) = v;
     }
   }
 }
@@ -617,14 +632,16 @@ static int launch_prefill(void* out, int out_stride, const void* qkv, int row_st
   else if (g_pf_pack && max_seqlen <= 2 * PF_QROWS && G % 2 == 0) wph = 2;
   const int rows_per_wg = wph * PF_QROWS;
   dim3 grid((max_seqlen + rows_per_wg - 1) / rows_per_wg, num_seqs, hq * wph / PF_WAVES);
-  if (hd == 128)
-    prefill_attn_kernel<128, PAGED><<<grid, 256, 0, st>>>(
-        (u16*)out, out_stride, (const u16*)qkv, row_stride, cu_seqlens, hq, hkv, sl2, ctx_lens,
-        (const u16*)k_cache, (const u16*)v_cache, block_tables, bt_stride, block_size, wph);
-  else
-    prefill_attn_kernel<64, PAGED><<<grid, 256, 0, st>>>(
-        (u16*)out, out_stride, (const u16*)qkv, row_stride, cu_seqlens, hq, hkv, sl2, ctx_lens,
-        (const u16*)k_cache, (const u16*)v_cache, block_tables, bt_stride, block_size, wph);
+#define PF_ARGS (u16*)out, out_stride, (const u16*)qkv, row_stride, cu_seqlens, hq, hkv, sl2, ctx_lens, (const u16*)k_cache, \
+                (const u16*)v_cache, block_tables, bt_stride, block_size, wph
+  if (!PAGED && max_seqlen <= 32) {
+    if (hd == 128) prefill_attn_kernel<128, false, 32><<<grid, 256, 0, st>>>(PF_ARGS);
+    else prefill_attn_kernel<64, false, 32><<<grid, 256, 0, st>>>(PF_ARGS);
+  } else {
+    if (hd == 128) prefill_attn_kernel<128, PAGED, PF_KT><<<grid, 256, 0, st>>>(PF_ARGS);
+    else prefill_attn_kernel<64, PAGED, PF_KT><<<grid, 256, 0, st>>>(PF_ARGS);
+  }
+#undef PF_ARGS
   DLI_RETURN_LAUNCH();
 }
 

@@ -559,10 +559,11 @@ __global__ void __launch_bounds__(512) prefill_attn32_kernel(
   }
 }
 
-// attention_prefill_long.hip; ctx_lens null: keys and values in the activation's rows
-int launch_prefill_long(bool paired, void* out, int out_stride, const void* qkv, int row_stride, const int* cu_seqlens, int num_seqs,
-                        int max_seqlen, int hq, int hkv, float scale_log2, const int* ctx_lens, const void* k_cache,
-                        const void* v_cache, const int* block_tables, int bt_stride, int block_size, hipStream_t st);
+// attention_prefill_long.hip and attention_prefill_pairs.hip; ctx_lens null: keys and values in the activation's rows
+using launch_wave64 = int(void* out, int out_stride, const void* qkv, int row_stride, const int* cu_seqlens, int num_seqs,
+                          int max_seqlen, int hq, int hkv, float scale_log2, const int* ctx_lens, const void* k_cache,
+                          const void* v_cache, const int* block_tables, int bt_stride, int block_size, hipStream_t st);
+launch_wave64 launch_prefill_long, launch_prefill_pairs;
 
 // Whether a launch takes waves of 64 rows. They gain on long sequences (2500 tokens 77 -> 69.5 us, 7993 516 -> 471, 7
 // x 2048 306 -> 291) and lose on short ones, whose last waves they leave idle (1000 tokens equal, 500 161 -> 174, 300 180
@@ -586,7 +587,7 @@ static bool takes_wave64(bool paged, long T, int n, long L, int hq, int hd, int 
   return low >= 1200.0 + 2e5 * n / T;
 }
 
-// Whether a launch of up to a workgroup a CU takes waves of 64 rows in pairs of half blocks (attention_prefill_long.hip):
+// Whether a launch of up to a workgroup a CU takes waves of 64 rows in pairs of half blocks (attention_prefill_pairs.hip):
 // wherever that kernel can read the rows. It is ahead from 257 tokens on: 300 14.7 / 14.6 us, 400 18.8 / 16.0, 300 of 300
 // cached 15.5 / 15.5, 2048 of 8048 250 / 217 (54 mixes of lengths, contexts and heads: 0.80 to 1.00 of the time). Other
 // lengths than the default set by dli_prefill_set_wave64_len leave such launches to waves of 32 rows.
@@ -609,8 +610,9 @@ static int launch_prefill(void* out, int out_stride, const void* qkv, int row_st
   const bool whole = row_stride % 8 == 0 && ((uintptr_t)qkv & 15) == 0;
   const bool pairs = (whole || !PAGED) && pairs_wave64(PAGED, num_seqs, max_seqlen, hq, hd, row_stride, block_size);
   if (pairs || ((whole || !PAGED) && takes_wave64(PAGED, tokens, num_seqs, max_seqlen, hq, hd, row_stride, block_size)))
-    return launch_prefill_long(pairs, out, out_stride, qkv, row_stride, cu_seqlens, num_seqs, max_seqlen, hq, hkv, sl2,
-                               PAGED ? ctx_lens : nullptr, k_cache, v_cache, block_tables, bt_stride, block_size, st);
+    return (pairs ? launch_prefill_pairs : launch_prefill_long)(
+        out, out_stride, qkv, row_stride, cu_seqlens, num_seqs, max_seqlen, hq, hkv, sl2, PAGED ? ctx_lens : nullptr,
+        k_cache, v_cache, block_tables, bt_stride, block_size, st);
   if (hd == 128 && max_seqlen >= g_pl_min_len) {     // long sequences: 256-row workgroups
     const int blocks = (max_seqlen + PL_ROWS - 1) / PL_ROWS;
     const dim3 grid32 = hq <= 4 ? dim3(blocks, num_seqs, hq) : dim3(blocks * hq, num_seqs);

@@ -13,18 +13,18 @@
 //     o_i = (A_i q_i)^T S + sum_{j <= i} P_ij v_j,   P_ij = sum_c q_ic k_jc prod_{j < t <= i} a_tc
 //     S  <- diag(G) S + sum_j (B_j k_j) v_j^T
 // are four products of v_mfma_f32_16x16x4_f32. A block's 72 MFMAs of 32 cycles a wave at d = 128 are its
-// floor (1.9 us with two waves a SIMD); it takes 4 to 7 us, the rest being the gates and the LDS image.
+// floor (1.9 us with two waves a SIMD); it takes 4 to 6 us, the rest being the gates and the LDS image.
 // The walk's floor is one token after another: 0.5 to 1.2 us each.
 //
 // A workgroup fills a CU, and there are as many as heads times sequences. Where that leaves CUs idle the
 // portions are cut in segments: a first launch forms each segment's state from nothing (no read-outs:
 // less than half the work), the second starts every segment from the fold of the states before it.
 //
-// d = dv = 128, HGRN2 / GLA / FIXED of 32 heads / MLSTM of 16, us; the walk, whole portions, segments:
-//   4 x 2048 tokens     1667  2342   976  1938     621   704   517   895     483   523   403   326
-//   998 to 2601 (5)                                768   891   650  1133     551   587   478   392
-//   1 x 8000                                      2325  2688  1972  3441     462   523   419   525
-//   32 x 256             680   824   508   423     354   397   295   240    (not cut)        211
+// d = dv = 128, HGRN2 / GLA / FIXED of 32 heads / MLSTM of 16, us; the walk, whole portions (before LONG), and what runs:
+//   4 x 2048 tokens     1667  2342   976  1938     621   704   517   895     382   424   345   294
+//   998 to 2601 (5)                                768   891   650  1133     553   615   511   395
+//   1 x 8000                                      2325  2688  1972  3441     402   445   366   491
+//   32 x 256 (not cut)   680   824   508   423     354   397   295   240     300   333   256   193
 //
 // One workgroup of 8 waves per (head, sequence, 128 state columns); a wave owns 16 columns and all d
 // rows of S in its accumulators for the whole portion. The summation index of an MFMA may be permuted
@@ -43,7 +43,14 @@
 // buffered), requests the rows of block b + 2, runs block b's products, finishes block b - 1 (sums P,
 // adds P V, squares for the norm), writes block b - 2 and forms the gates of block b + 2; half of the
 // waves run the products before the finishing, half after it, so that a SIMD's two waves keep the
-// matrix pipe and the vector unit busy at the same time.
+// matrix pipe and the vector unit busy at the same time (per-channel decays: the former ahead of the staging too).
+//
+// A step of the loop was up to 93 basic blocks (a bound a token, a head's widths) and waited for LDS at each of 8
+// tiles' operands. LONG takes the steps whose blocks are full, of heads of 128 channels and columns, through a copy
+// without bounds, with scalar row addresses; the next tile's operands are read ahead of a tile's products; with
+// per-channel decays the wave that has products to issue goes first (the others lose 1 to 2 % by it). Before that and
+// with it, one card: 4 x 2048 HGRN2 441 -> 382 us, GLA 501 -> 424; 1 x 8000 FIXED 417 -> 366, MLSTM 523 -> 491; 998 to
+// 2601 596 -> 553, 677 -> 615, 551 -> 511 and 425 -> 395. Equal to the bit.
 #include "common.h"
 
 namespace {
@@ -58,8 +65,7 @@ template <> __device__ __forceinline__ void stf<float>(float* p, float v) { *p =
 // exp, reciprocal and sigmoid to about an ulp in a few instructions: 2^(x log2 e) with the product's
 // rounding carried to first order, and one Newton step. Infinities saturate, NaN stays.
 __device__ __forceinline__ float exp1(float x) {
-  x = x > 88.f ? 88.f : x;
-  x = x < -104.f ? -104.f : x;
+  x = __builtin_elementwise_maximum(__builtin_elementwise_minimum(x, 88.f), -104.f);
   const float hi = x * 0x1.715476p+0f;
   const float lo = fmaf(x, 0x1.4ae0bfp-26f, fmaf(x, 0x1.715476p+0f, -hi));
   const float r = __builtin_amdgcn_exp2f(hi);
@@ -156,7 +162,7 @@ template <int ND, bool STATE> struct Smem {
 };
 template <int ND, bool STATE> struct ChannelSmem {          // per-channel decays
   float G[2][ND * 16];              // over the block
-  float part[2][4][ND * 16];        // over 4 tokens
+  float part[17][ND * 16];          // over 4 tokens: rows 3 to 6 and 10 to 13, ones between and around them
   float raw[2][STATE ? 1 : ND * 16][3 * TB + 4];  // q, k and decays of a channel below MIN_DECAY
   float xP[2][STATE ? 2 : 256];     // such channels' share of P, [j][i]
   unsigned long long bad[2][2];     // which channels
@@ -168,7 +174,8 @@ template <int ND> struct ScalarSmem {           // one decay a token
 
 // ND * 16 >= d
 // STATE: only the states after the segments that have a successor
-template <typename S, int ND, int MODE, bool STATE>
+// LONG: with a loop for the full blocks of whole heads beside the general one, which pays from MIN_LONG tokens on
+template <typename S, int ND, int MODE, bool STATE, bool LONG>
 __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
   constexpr bool CHANNEL = MODE == HGRN2 || MODE == GLA;
   constexpr int DP = ND * 16, LQ = DP + 8;
@@ -187,7 +194,7 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
   const int t1 = seg + 1 < a.nseg && end - t0 > a.seg_tokens ? t0 + a.seg_tokens : end;
   const bool last = t1 == end, cut = end - first > a.seg_tokens;
   if (STATE && (last || slot < 0)) return;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, w = MODE == MLSTM ? tid >> 6 : __builtin_amdgcn_readfirstlane(tid >> 6);
   const int fr = lane & 15, q = lane >> 4;
   const int col = c0 + w * 16 + fr;             // this lane's state column
   const bool on = col < dv, wave_on = c0 + w * 16 < dv;
@@ -272,7 +279,7 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
   if (MODE == MLSTM && w < ND && q == 0) gm.n[nc] = n0;
   float G_seg = 1.f;                            // STATE: this thread's channel's, or the gate wave's
   // staging: thread = (channel sc and column sc of the block's 128, tokens 4 tg .. 4 tg + 3)
-  const int sc = tid & 127, tg = tid >> 7;
+  const int sc = tid & 127, tg = w >> 1;
   const bool chan = sc < d, scol = c0 + sc < dv;
   float bias = 0.f, low = 0.f;
   if (CHANNEL && chan) {
@@ -283,10 +290,30 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
   constexpr int GW = 7;                                         // the gate wave
   const int nb = (t1 - t0 + TB - 1) / TB;
   auto tokens = [&](int b) { return min(TB, t1 - t0 - b * TB); };
+  // FULL: a head of 128 channels and columns, and blocks of 16 tokens (the loop says which). A lane's places in a
+  // block of rows are then constant and the rows' start is scalar, without a bound or a branch a token
+  const bool whole = ND == 8 && d == DP && c0 + COLS <= dv && a.ldp < 1 << 24 && a.ldz < 1 << 24 && a.ldo < 1 << 24;
+  const uint32_t pat = 4u * (4 * tg * a.ldp + sc), zat = 4u * (4 * tg * a.ldz + sc);
+  const uint32_t gat = 4u * (4 * q * a.ldp + w * 16 + fr);
+  const uint32_t oat = sizeof(S) * (4 * q * a.ldo + w * 16 + fr);
+  const auto at = [](const float* base, uint32_t bytes) { return *(const float*)((const char*)base + bytes); };
   float rq[4], rk[4], rz[4], rv[4], ra[4];
   f32x4 gin = {1.f, 0.f, 0.f, 0.f};
-  auto load = [&](int b) {
+  auto load = [&](int b, auto FULL) __attribute__((always_inline)) {
     const int tc = t0 + b * TB, n = tokens(b);
+    if constexpr (decltype(FULL)::value) {
+      const float* rows = a.proj + (long)tc * a.ldp + h * d;
+      const float* vals = a.proj + (long)tc * a.ldp + 2 * H * d + h * dv + c0;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const uint32_t ro = pat + 4u * u * a.ldp;
+        if (!STATE) rq[u] = at(rows, ro);
+        rk[u] = at(rows + H * d, ro);
+        if (MODE == GLA) rz[u] = at(a.z + (long)tc * a.ldz + h * d, zat + 4u * u * a.ldz);
+        rv[u] = at(vals, ro);
+      }
+      return;
+    }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int t = 4 * tg + u;
@@ -307,11 +334,11 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
       gin = *reinterpret_cast<const f32x4*>(a.gates + ((long)(t0 + b * TB + fr) * H + h) * 4);
   };
   // per-channel decays of the block in the registers, and their products over 4 tokens
-  auto channel_gates = [&](int b) {
+  auto channel_gates = [&](int b, auto FULL) __attribute__((always_inline)) {
     const int n = tokens(b);
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const bool real = 4 * tg + u < n && chan;
+      const bool real = decltype(FULL)::value || (4 * tg + u < n && chan);
       if (MODE == HGRN2) {
         ra[u] = real ? low + (1.f - low) * sigmoid1(rk[u] + bias) : 1.f;
         rk[u] = real ? 1.f - ra[u] : 0.f;
@@ -319,7 +346,7 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
         ra[u] = real ? decay_pow(rz[u] + bias, a.inv_tau) : 1.f;
       }
     }
-    if (sc < DP) cm.part[b & 1][tg][sc] = (ra[0] * ra[1]) * (ra[2] * ra[3]);
+    if (decltype(FULL)::value || sc < DP) cm.part[3 + 7 * (b & 1) + tg][sc] = (ra[0] * ra[1]) * (ra[2] * ra[3]);
   };
   // scalar tables of a block of n tokens (one wave; lane t of every row of 16 holds token t)
   auto scalar_gates = [&](int n, Gates& gt) {
@@ -384,20 +411,18 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
     G_seg *= G;
   };
   // fixed decays: table 0 for full blocks, 1 for a shorter last one
-  auto table = [&](int b) -> Gates& { return gm.g[MODE == FIXED ? int(tokens(b) < TB) : (b & 3)]; };
+  auto table = [&](int b, auto FULL) __attribute__((always_inline)) -> Gates& {
+    return gm.g[MODE == FIXED ? !decltype(FULL)::value && tokens(b) < TB : (b & 3)];
+  };
   // a block's LDS image from the registers
-  auto stage = [&](int b) {
+  auto stage = [&](int b, auto FULL) __attribute__((always_inline)) {
     const int buf = b & 1;
     f32x4 kb, vv;
-    if (sc < DP) {
+    if (decltype(FULL)::value || sc < DP) {
       if constexpr (CHANNEL) {
-        float A[4], B[4], pre = 1.f, post = 1.f;
-#pragma unroll
-        for (int x = 0; x < 4; ++x) {
-          const float px = cm.part[buf][x][sc];
-          if (x < tg) pre *= px;
-          if (x > tg) post *= px;
-        }
+        float A[4], B[4];
+        const float* const around = &cm.part[7 * buf + tg][sc];
+        const float pre = around[0] * around[DP] * around[2 * DP], post = around[4 * DP] * around[5 * DP] * around[6 * DP];
         A[0] = pre * ra[0]; A[1] = A[0] * ra[1]; A[2] = A[1] * ra[2]; A[3] = A[2] * ra[3];
         B[3] = post; B[2] = B[3] * ra[3]; B[1] = B[2] * ra[2]; B[0] = B[1] * ra[1];
         const float G = A[3] * post;
@@ -423,7 +448,7 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
           }
         }
       } else {
-        const f32x4 kw = *reinterpret_cast<const f32x4*>(table(b).kb + 4 * tg);
+        const f32x4 kw = *reinterpret_cast<const f32x4*>(table(b, FULL).kb + 4 * tg);
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           const int t = 4 * tg + u;
@@ -445,7 +470,7 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
   unsigned long long bad0 = 0, bad1 = 0, bad0n = 0, bad1n = 0;
   f32x4 vf = {0.f, 0.f, 0.f, 0.f}, acc = vf, vfn = vf, accn = vf;
   // block b: P's partial sums to LDS, the read-out of the state before it to accn, the state after it
-  auto products = [&](int b) {
+  auto products = [&](int b, auto FULL) __attribute__((always_inline)) {
     const int buf = b & 1;
     const float* Q = sm.Q[buf];
     if (w < ND && (!STATE || MODE == MLSTM)) {  // this wave's 16 channels of P^T
@@ -468,7 +493,7 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
         float y = (kb[0] + kb[1]) + (kb[2] + kb[3]);
         y += __shfl_xor(y, 16, 64);
         y += __shfl_xor(y, 32, 64);
-        if (q == 0) gm.n[16 * w + fr] = table(b).G[0] * gm.n[16 * w + fr] + y;
+        if (q == 0) gm.n[16 * w + fr] = table(b, FULL).G[0] * gm.n[16 * w + fr] + y;
       }
     }
     if constexpr (CHANNEL && !STATE) {
@@ -489,21 +514,30 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
         cm.xP[buf][tid] = x;
       }
     }
-    if (wave_on) {
+    if (decltype(FULL)::value || wave_on) {
       vfn = *reinterpret_cast<const f32x4*>(sm.V[buf] + (16 * w + fr) * LT + 4 * q);
       f32x4 part[4];                            // short sums round less than one of d terms
 #pragma unroll
       for (int t = 0; t < 4; ++t) part[t] = f32x4{0.f, 0.f, 0.f, 0.f};
       float Gs = 0.f, Gl = 0.f;
-      if constexpr (!CHANNEL) Gs = table(b).G[0];
-      if (MODE == FIXED) Gl = table(b).G[1];
+      if constexpr (!CHANNEL) Gs = table(b, FULL).G[0];
+      if (MODE == FIXED) Gl = table(b, FULL).G[1];
+      f32x4 qf, kb, Gt, qn, kn, Gn;
+      if constexpr (CHANNEL) __builtin_amdgcn_s_setprio(1);
+      const auto read = [&](int t) __attribute__((always_inline)) {
+        if (!STATE) qn = *reinterpret_cast<const f32x4*>(Q + fr * LQ + 16 * t + 4 * q);
+        kn = *reinterpret_cast<const f32x4*>(sm.Kb[buf] + (16 * t + fr) * LT + 4 * q);
+        if constexpr (CHANNEL) Gn = *reinterpret_cast<const f32x4*>(cm.G[buf] + 16 * t + 4 * q);
+      };
+      read(0);
 #pragma unroll
       for (int t = 0; t < ND; ++t) {            // tile t's read-out and update side by side
-        f32x4 qf;
-        if (!STATE) qf = *reinterpret_cast<const f32x4*>(Q + fr * LQ + 16 * t + 4 * q);
-        const f32x4 kb = *reinterpret_cast<const f32x4*>(sm.Kb[buf] + (16 * t + fr) * LT + 4 * q);
+        qf = qn; kb = kn; Gt = Gn;
+        // the next tile's operands on their way ahead of this one's products; hipcc reads them where they are used
+        if (t + 1 < ND) read(t + 1);
+        __builtin_amdgcn_sched_barrier(0x6);    // (vector and scalar arithmetic may pass)
         f32x4 sn;
-        if constexpr (CHANNEL) sn = st[t] * *reinterpret_cast<const f32x4*>(cm.G[buf] + 16 * t + 4 * q);
+        if constexpr (CHANNEL) sn = st[t] * Gt;
         else sn = st[t] * Gs;
         if (MODE == FIXED) sn += st[t] * Gl;
 #pragma unroll
@@ -514,6 +548,7 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
         }
         st[t] = sn;
       }
+      if constexpr (CHANNEL) __builtin_amdgcn_s_setprio(0);
       accn = (part[0] + part[1]) + (part[2] + part[3]);
     }
   };
@@ -521,17 +556,24 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
   float nw = 0.f;
   if (!STATE && MODE != FIXED && on) nw = ldf((const S*)a.norm_w + (MODE == MLSTM ? h * dv + col : col));
   // o = the read-outs of block b (rows 4 q + r, this lane's column) from vf, acc and P
-  auto finish = [&](int b) {
+  auto finish = [&](int b, auto FULL) __attribute__((always_inline)) {
     const int buf = b & 1;
-    if (MODE == GLA || MODE == MLSTM) {
+    if ((MODE == GLA || MODE == MLSTM) && decltype(FULL)::value) {
+      const float* rows = a.proj + (long)(t0 + b * TB) * a.ldp + 2 * H * d + H * dv + h * dv + c0;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) gate[r] = at(rows, gat + 4u * r * a.ldp);
+    } else if (MODE == GLA || MODE == MLSTM) {
       const int n = tokens(b);
 #pragma unroll
       for (int r = 0; r < 4; ++r)
         if (on && 4 * q + r < n) gate[r] = a.proj[(long)(t0 + b * TB + 4 * q + r) * a.ldp + goff];
     }
-    f32x4 p = {0.f, 0.f, 0.f, 0.f};             // P_ij, i = fr, j = 4 q + r
+    f32x4 p = {0.f, 0.f, 0.f, 0.f}, ps[ND];     // P_ij, i = fr, j = 4 q + r
 #pragma unroll
-    for (int x = 0; x < ND; ++x) p += *reinterpret_cast<const f32x4*>(&sm.P[buf][x][4 * lane]);
+    for (int x = 0; x < ND; ++x) ps[x] = *reinterpret_cast<const f32x4*>(&sm.P[buf][x][4 * lane]);
+    __builtin_amdgcn_sched_barrier(0x6);
+#pragma unroll
+    for (int x = 0; x < ND; ++x) p += ps[x];
     float inv = 0.f;
     if constexpr (CHANNEL) {
       const bool extra = (bad0 | bad1) != 0;
@@ -541,7 +583,7 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
         p[r] = 4 * q + r <= fr ? p[r] : 0.f;
       }
     } else {
-      const Gates& gt = table(b);
+      const Gates& gt = table(b, FULL);
       const f32x4 D = *reinterpret_cast<const f32x4*>(gt.D + fr * LT + 4 * q);
 #pragma unroll
       for (int r = 0; r < 4; ++r) p[r] = 4 * q + r <= fr ? p[r] * D[r] : 0.f;
@@ -584,75 +626,95 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
       }
     }
   };
-  auto write_out = [&](int b) {
+  auto write_out = [&](int b, auto FULL) __attribute__((always_inline)) {
     const int n = tokens(b);
     float rs = 0.f;
     if (MODE != FIXED) {                        // row fr's
       const float* sq = sm.ss[b & 1][fr];
       const f32x4 x = *reinterpret_cast<const f32x4*>(sq), y = *reinterpret_cast<const f32x4*>(sq + 4);
-      rs = 1.f / sqrtf((((x[0] + x[1]) + (x[2] + x[3])) + ((y[0] + y[1]) + (y[2] + y[3]))) / (float)dv + a.eps);
+      const float n_cols = decltype(FULL)::value ? (float)COLS : (float)dv;
+      rs = 1.f / sqrtf((((x[0] + x[1]) + (x[2] + x[3])) + ((y[0] + y[1]) + (y[2] + y[3]))) / n_cols + a.eps);
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int i = 4 * q + r;
       const float rr = MODE != FIXED ? __shfl(rs, i, 64) : 0.f;
-      if (i >= n || !on) continue;
+      if (!decltype(FULL)::value && (i >= n || !on)) continue;
       const long t = (long)t0 + b * TB + i;
+      char* const rows = (char*)((S*)a.out + (long)(t0 + b * TB) * a.ldo + h * dv + c0);      // FULL: row 0's
       if (MODE == FIXED) {
-        outf[t * a.ldo + h * dv + col] = o[r];
+        if (decltype(FULL)::value) *(float*)(rows + oat + sizeof(S) * r * a.ldo) = o[r];
+        else outf[t * a.ldo + h * dv + col] = o[r];
         continue;
       }
       float v = o[r] * rr * nw;
       if (MODE == GLA) v *= silu1(gate[r]);
       if (MODE == MLSTM) v *= sigmoid1(gate[r]) * a.out_scale;
-      stf(out + t * a.ldo + h * dv + col, v);
+      stf(decltype(FULL)::value ? (S*)(rows + oat + sizeof(S) * r * a.ldo) : out + t * a.ldo + h * dv + col, v);
     }
   };
 
-  load(0);
+  using Any = std::integral_constant<bool, false>;
+  load(0, Any{});
   load_gates(0);
   if constexpr (CHANNEL) {
-    channel_gates(0);
+    if (tid < DP)
+#pragma unroll
+      for (int x = 0; x < 9; ++x) cm.part[x + x / 3 * 4][tid] = 1.f;
+    channel_gates(0, Any{});
   } else if (w == GW) {
-    scalar_gates(tokens(0), table(0));
+    scalar_gates(tokens(0), table(0, Any{}));
     if (MODE == FIXED) {
-      if (nb > 1) scalar_gates(tokens(nb - 1), table(nb - 1));
+      if (nb > 1) scalar_gates(tokens(nb - 1), table(nb - 1, Any{}));
     } else if (nb > 1) {
       load_gates(1);
-      scalar_gates(tokens(1), table(1));
+      scalar_gates(tokens(1), table(1, Any{}));
     }
     load_gates(2);
   }
   __syncthreads();
-  stage(0);
+  stage(0, Any{});
   if (nb > 1) {
-    load(1);
-    if constexpr (CHANNEL) channel_gates(1);
+    load(1, Any{});
+    if constexpr (CHANNEL) channel_gates(1, Any{});
   }
   __syncthreads();
-#pragma unroll 1
-  for (int b = 0; b < nb + (STATE ? 0 : 2); ++b) {
-    if (b + 1 < nb) stage(b + 1);
-    if (b + 2 < nb) {
-      load(b + 2);
+  // FULL: blocks b - 2 to b + 2 are there, and full
+  auto step = [&](int b, auto FULL) __attribute__((always_inline)) {
+    constexpr bool full = decltype(FULL)::value;
+
+    if (!STATE && CHANNEL && w < 4 && (full || b < nb)) products(b, FULL);
+    if (full || b + 1 < nb) stage(b + 1, FULL);
+    if (full || b + 2 < nb) {
+      load(b + 2, FULL);
       if (MODE == MLSTM && w == GW) {
-        scalar_gates(tokens(b + 2), table(b + 2));
+        scalar_gates(full ? TB : tokens(b + 2), table(b + 2, FULL));
         load_gates(b + 3);
       }
     }
     if constexpr (STATE) {
-      products(b);
+      products(b, FULL);
     } else {
-      if (w < 4 && b < nb) products(b);
-      if (b >= 2) write_out(b - 2);
-      if (b >= 1 && b <= nb) finish(b - 1);
-      if (w >= 4 && b < nb) products(b);
+      if (!CHANNEL && w < 4 && (full || b < nb)) products(b, FULL);
+      if (full || b >= 2) write_out(b - 2, FULL);
+      if (full || (b >= 1 && b <= nb)) finish(b - 1, FULL);
+      if (w >= 4 && (full || b < nb)) products(b, FULL);
       vf = vfn; acc = accn; bad0 = bad0n; bad1 = bad1n;
     }
     if constexpr (CHANNEL) {
-      if (b + 2 < nb) channel_gates(b + 2);
+      if (full || b + 2 < nb) channel_gates(b + 2, FULL);
     }
     lds_barrier();
+  };
+  const int full_to = whole ? (t1 - t0) / TB - 2 : 0;
+#pragma unroll 1
+  for (int b = 0; b < nb + (STATE ? 0 : 2); ++b) {
+    if constexpr (LONG) {
+      if (STATE || b >= 2)
+#pragma unroll 1
+        for (; b < full_to; ++b) step(b, std::integral_constant<bool, true>{});
+    }
+    step(b, Any{});
   }
   if constexpr (STATE) {
     store_state(seg_st(seg));
@@ -714,34 +776,40 @@ __global__ void __launch_bounds__(512) mlstm_gates_kernel(ChunkArgs a, float* ga
   if (tid == 0) *mp = m[0];
 }
 
-template <typename S, int ND, int MODE, bool STATE>
-int launch_chunks(const ChunkArgs& a, int num_seqs, hipStream_t st) {
+template <typename S, int ND, int MODE, bool STATE, bool LONG>
+int launch_one(const ChunkArgs& a, int num_seqs, hipStream_t st) {
   constexpr size_t sh = sizeof(Smem<ND, STATE>) +
                         (MODE <= GLA ? sizeof(ChannelSmem<ND, STATE>) : sizeof(ScalarSmem<ND>));
   static_assert(sh <= 160 * 1024 && sizeof(Smem<ND, STATE>) % 16 == 0, "LDS image");
   if (sh > 48 * 1024) {
-    hipError_t e = hipFuncSetAttribute((const void*)recurrence_chunk_kernel<S, ND, MODE, STATE>,
+    hipError_t e = hipFuncSetAttribute((const void*)recurrence_chunk_kernel<S, ND, MODE, STATE, LONG>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh);
     if (e != hipSuccess) return (int)e;
   }
   dim3 grid(a.H, num_seqs * (STATE ? a.nseg - 1 : a.nseg), (a.dv + COLS - 1) / COLS);
-  recurrence_chunk_kernel<S, ND, MODE, STATE><<<grid, NTH, sh, st>>>(a);
+  recurrence_chunk_kernel<S, ND, MODE, STATE, LONG><<<grid, NTH, sh, st>>>(a);
   DLI_RETURN_LAUNCH();
 }
 template <typename S, int ND, int MODE>
-int launch_chunks(const ChunkArgs& a, int num_seqs, hipStream_t st) {
+int launch_chunks(const ChunkArgs& a, int num_seqs, int max_seqlen, hipStream_t st) {
+  // Blocks b - 2 to b + 2 are full for the first time in a portion of 5 blocks. 64 portions of 80 / 96 / 128 tokens, us, without
+  // and with that loop: HGRN2 235 / 273 / 345 and 242 / 275 / 338, GLA 273 / 319 / 412 and 276 / 309 / 379, FIXED
+  // 211 / 242 / 302 and 209 / 237 / 293, MLSTM 144 / 174 / 220 and 150 / 180 / 219. Segments have 128 tokens and more.
+  constexpr bool WIDE = ND == 8;
+  constexpr int MIN_LONG = MODE == MLSTM ? 128 : 96;
   if (a.nseg > 1) {
-    const int rc = launch_chunks<S, ND, MODE, true>(a, num_seqs, st);
+    const int rc = launch_one<S, ND, MODE, true, WIDE>(a, num_seqs, st);
     if (rc) return rc;
   }
-  return launch_chunks<S, ND, MODE, false>(a, num_seqs, st);
+  if (WIDE && max_seqlen >= MIN_LONG) return launch_one<S, ND, MODE, false, WIDE>(a, num_seqs, st);
+  return launch_one<S, ND, MODE, false, false>(a, num_seqs, st);
 }
 
 template <typename S, int MODE>
-int launch_by_width(const ChunkArgs& a, int num_seqs, hipStream_t st) {
-  if (a.d <= 32) return launch_chunks<S, 2, MODE>(a, num_seqs, st);
-  if (a.d <= 64) return launch_chunks<S, 4, MODE>(a, num_seqs, st);
-  return launch_chunks<S, 8, MODE>(a, num_seqs, st);
+int launch_by_width(const ChunkArgs& a, int num_seqs, int max_seqlen, hipStream_t st) {
+  if (a.d <= 32) return launch_chunks<S, 2, MODE>(a, num_seqs, max_seqlen, st);
+  if (a.d <= 64) return launch_chunks<S, 4, MODE>(a, num_seqs, max_seqlen, st);
+  return launch_chunks<S, 8, MODE>(a, num_seqs, max_seqlen, st);
 }
 
 // Segments of a portion of at most max_seqlen tokens (T in all): a CU takes one workgroup, so few heads
@@ -820,17 +888,20 @@ extern "C" int dli_recurrence_chunks(int mode, const float* proj, int ldp, const
   switch (mode) {
     case HGRN2:
       if (bias == nullptr || lower == nullptr || norm_w == nullptr) break;
-      return dt == 0 ? launch_by_width<u16, HGRN2>(a, num_seqs, st) : launch_by_width<float, HGRN2>(a, num_seqs, st);
+      return dt == 0 ? launch_by_width<u16, HGRN2>(a, num_seqs, max_seqlen, st)
+                     : launch_by_width<float, HGRN2>(a, num_seqs, max_seqlen, st);
     case GLA:
       if (z == nullptr || bias == nullptr || norm_w == nullptr) break;
-      return dt == 0 ? launch_by_width<u16, GLA>(a, num_seqs, st) : launch_by_width<float, GLA>(a, num_seqs, st);
+      return dt == 0 ? launch_by_width<u16, GLA>(a, num_seqs, max_seqlen, st)
+                     : launch_by_width<float, GLA>(a, num_seqs, max_seqlen, st);
     case FIXED:
       if (decays == nullptr) break;
-      return launch_by_width<float, FIXED>(a, num_seqs, st);
+      return launch_by_width<float, FIXED>(a, num_seqs, max_seqlen, st);
     case MLSTM:
       if (if_b == nullptr || norm_w == nullptr || nstate == nullptr || !(cap > 0.f) || ws == nullptr) break;
       mlstm_gates_kernel<<<dim3(H, num_seqs), 512, 0, st>>>(a, gates);
-      return dt == 0 ? launch_by_width<u16, MLSTM>(a, num_seqs, st) : launch_by_width<float, MLSTM>(a, num_seqs, st);
+      return dt == 0 ? launch_by_width<u16, MLSTM>(a, num_seqs, max_seqlen, st)
+                     : launch_by_width<float, MLSTM>(a, num_seqs, max_seqlen, st);
   }
   return (int)hipErrorInvalidValue;
 }

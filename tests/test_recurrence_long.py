@@ -1,0 +1,24 @@
+"""Portions whose full blocks take a loop of their own (heads of 128 channels, column blocks of 128), against the float64 walk:
+portions around the shortest that take it, last blocks of 1, 15 and 16 tokens behind it, shorter portions beside
+them, a whole column block beside a narrower one, and decays that leave the range of fp32."""
+import pytest
+import torch
+
+from test_recurrence_chunks import check
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["hgrn2", "gla", "lightning", "mlstm"])
+@pytest.mark.parametrize("lens", [[95, 80], [96, 64, 97], [127, 3], [128, 16, 81], [129, 112, 143]])
+@pytest.mark.parametrize("strong", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_around_the_shortest(gpu, mode, lens, strong, dtype):
+    n = len(lens)
+    check(gpu, mode, 128, 128, strong, dtype, lens, [4, 1, 0][:n], [0, 1, 0][:n])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dv", [200, 256])
+@pytest.mark.parametrize("lens", [[131, 20], [700]])
+def test_column_blocks(gpu, dv, lens):
+    check(gpu, "lightning", 128, dv, False, torch.float32, lens, [2, 5][:len(lens)], [0, 1][:len(lens)])

@@ -21,10 +21,10 @@
 // less than half the work), the second starts every segment from the fold of the states before it.
 //
 // d = dv = 128, HGRN2 / GLA / FIXED of 32 heads / MLSTM of 16, us; the walk, whole portions (before LONG), and what runs:
-//   4 x 2048 tokens     1667  2342   976  1938     621   704   517   895     382   424   345   294
-//   998 to 2601 (5)                                768   891   650  1133     553   615   511   395
-//   1 x 8000                                      2325  2688  1972  3441     402   445   366   491
-//   32 x 256 (not cut)   680   824   508   423     354   397   295   240     300   333   256   193
+//   4 x 2048 tokens     1667  2342   976  1938     621   704   517   895     382   424   345   253
+//   998 to 2601 (5)                                768   891   650  1133     553   615   511   344
+//   1 x 8000                                      2325  2688  1972  3441     402   445   366   342
+//   32 x 256 (not cut)   680   824   508   423     354   397   295   240     300   333   256   189
 //
 // One workgroup of 8 waves per (head, sequence, 128 state columns); a wave owns 16 columns and all d
 // rows of S in its accumulators for the whole portion. The summation index of an MFMA may be permuted
@@ -50,7 +50,7 @@
 // without bounds, with scalar row addresses; the next tile's operands are read ahead of a tile's products; with
 // per-channel decays the wave that has products to issue goes first (the others lose 1 to 2 % by it). Before that and
 // with it, one card: 4 x 2048 HGRN2 441 -> 382 us, GLA 501 -> 424; 1 x 8000 FIXED 417 -> 366, MLSTM 523 -> 491; 998 to
-// 2601 596 -> 553, 677 -> 615, 551 -> 511 and 425 -> 395. Equal to the bit.
+// 2601 596 -> 553, 677 -> 615, 551 -> 511 and 425 -> 395. Equal to the bit. (MLSTM with its gates as they were then.)
 #include "common.h"
 
 namespace {
@@ -730,37 +730,65 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
 }
 
 // MLSTM's gates: a_t = exp(f_t + m_{t-1} - m_t), b_t = exp(i_t - m_t) and exp(-m_t) of every token of a
-// (head, sequence), and the state's m after the portion. Only m is a walk, of an addition and a maximum
-// a token (2600 tokens some 20 us); inside the products' launch, where one wave did this for a block
+// (head, sequence), and the state's m after the portion. Inside the products' launch, where one wave did this for a block
 // beside its share of the products, it was what the other waves waited for.
+//
+// m_t = max(f_t + m_{t-1}, i_t) is a map m -> max(F + m, I), and such maps compose. A lane of one wave composes the
+// maps of 33 tokens (an odd stride in LDS), a prefix over the lanes gives the m ahead of each, and every lane walks
+// its own: where one walk of all the tokens bound this launch, 64 go side by side. 16 heads, us, that walk / this:
+// 5 portions of 900 to 2601 tokens 68 / 17, 1 x 8000 195 / 38, 64 x 33 9.6 / 6.6. The walk within a lane matters: where
+// no i_t wins, a_t is one, and a prefix over single tokens, whose a_t round about it, lost up to half a digit against
+// 64 bits. So does the prefix in double: read-outs and states are as near as those of the one walk (1.9e-7 and
+// 1.2e-7 at forget biases of 3), m nearer where few i_t win (bias 6, 4000 tokens: 1.5e-6 -> 1.2e-7).
 __global__ void __launch_bounds__(512) mlstm_gates_kernel(ChunkArgs a, float* gates) {
-  constexpr int N = 1024;
+  constexpr int OWN = 33, N = 64 * OWN, EACH = (N + 511) / 512;
   __shared__ float ig[N], fg[N], m[N + 1];
   const int h = blockIdx.x, s = blockIdx.y, H = a.H, tid = threadIdx.x, lane = tid & 63;
   const int slot = a.slots[s], first = a.cu[s], end = a.cu[s + 1];
   if (slot < 0 || end <= first || end - first < a.min_len) return;
   float* mp = a.nstate + ((long)slot * H + h) * (a.d + 1) + a.d;
-  const int ioff = 2 * H * a.d + 2 * H * a.dv + h;
+  const float* col = a.proj + 2 * H * a.d + 2 * H * a.dv + h;
+  const float bi = a.if_b[h], bf = a.if_b[H + h];
   if (tid == 0) m[0] = a.positions[first] == 0 ? 0.f : *mp;
   for (int t0 = first; t0 < end; t0 += N) {
     const int n = min(N, end - t0);
-    for (int t = tid; t < n; t += 512) {
-      const float* row = a.proj + (long)(t0 + t) * a.ldp + ioff;
-      ig[t] = a.cap * tanhf((row[0] + a.if_b[h]) / a.cap);
-      fg[t] = logsigmoid32(a.cap * tanhf((row[H] + a.if_b[H + h]) / a.cap));
+    float ri[EACH], rf[EACH];
+#pragma unroll
+    for (int x = 0; x < EACH; ++x) {
+      const int t = min(tid + 512 * x, n - 1);
+      ri[x] = col[(long)(t0 + t) * a.ldp];
+      rf[x] = col[(long)(t0 + t) * a.ldp + H];
+    }
+#pragma unroll
+    for (int x = 0; x < EACH; ++x) {
+      const int t = tid + 512 * x;
+      if (t >= n) break;
+      ig[t] = a.cap * tanhf((ri[x] + bi) / a.cap);
+      fg[t] = logsigmoid32(a.cap * tanhf((rf[x] + bf) / a.cap));
     }
     __syncthreads();
-    if (tid < 64) {
-      float run = m[0];
-      for (int t = 0; t < n; t += 64) {
-        const float i = t + lane < n ? ig[t + lane] : -INFINITY, f = t + lane < n ? fg[t + lane] : 0.f;
-        float own = 0.f;
+    if (tid < 64 && lane * OWN < n) {           // (what the last of them makes of rows past the portion, nothing reads)
+      const float *il = ig + lane * OWN, *fl = fg + lane * OWN;
+      double F = 0.0, I = -INFINITY;
 #pragma unroll
-        for (int u = 0; u < 64; ++u) {
-          run = fmaxf(from_lane(f, u) + run, from_lane(i, u));
-          own = lane == u ? run : own;
+      for (int u = 0; u < OWN; ++u) {
+        I = fmax(fl[u] + I, (double)il[u]);
+        F += fl[u];
+      }
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const double Fb = __shfl_up(F, o, 64), Ib = __shfl_up(I, o, 64);
+        if (lane >= o) {
+          I = fmax(F + Ib, I);
+          F += Fb;
         }
-        if (t + lane < n) m[t + lane + 1] = own;
+      }
+      const double Fb = __shfl_up(F, 1, 64), Ib = __shfl_up(I, 1, 64);
+      float run = lane == 0 ? m[0] : (float)fmax(Fb + m[0], Ib);
+#pragma unroll
+      for (int u = 0; u < OWN; ++u) {
+        run = fmaxf(fl[u] + run, il[u]);
+        m[lane * OWN + u + 1] = run;
       }
     }
     __syncthreads();

@@ -1,6 +1,7 @@
 """Portions whose full blocks take a loop of their own (heads of 128 channels, column blocks of 128), against the float64 walk:
 portions around the shortest that take it, last blocks of 1, 15 and 16 tokens behind it, shorter portions beside
-them, a whole column block beside a narrower one, and decays that leave the range of fp32."""
+them, a whole column block beside a narrower one, and decays that leave the range of fp32; and the matrix memory's gates
+at the edges of a lane's tokens and of a pass."""
 import pytest
 import torch
 
@@ -22,3 +23,12 @@ def test_around_the_shortest(gpu, mode, lens, strong, dtype):
 @pytest.mark.parametrize("lens", [[131, 20], [700]])
 def test_column_blocks(gpu, dv, lens):
     check(gpu, "lightning", 128, dv, False, torch.float32, lens, [2, 5][:len(lens)], [0, 1][:len(lens)])
+
+
+# the gates' maximum: 33 tokens a lane, 2112 a pass
+@pytest.mark.gpu
+@pytest.mark.parametrize("strong", [False, True])
+@pytest.mark.parametrize("lens", [[2112, 33], [2113, 34, 1], [32, 66, 67], [512, 513]])
+def test_gates_of_the_matrix_memory(gpu, strong, lens):
+    n = len(lens)
+    check(gpu, "mlstm", 128, 128, strong, torch.float32, lens, [3, 0, 2][:n], [0, 1, 0][:n])

@@ -21,10 +21,10 @@
 // less than half the work), the second starts every segment from the fold of the states before it.
 //
 // d = dv = 128, HGRN2 / GLA / FIXED of 32 heads / MLSTM of 16, us; the walk, whole portions (before LONG), and what runs:
-//   4 x 2048 tokens     1667  2342   976  1938     621   704   517   895     382   424   345   253
-//   998 to 2601 (5)                                768   891   650  1133     553   615   511   344
-//   1 x 8000                                      2325  2688  1972  3441     402   445   366   342
-//   32 x 256 (not cut)   680   824   508   423     354   397   295   240     300   333   256   189
+//   4 x 2048 tokens     1667  2342   976  1938     621   704   517   895     385   425   345   244
+//   998 to 2601 (5)                                768   891   650  1133     474   522   432   307
+//   1 x 8000                                      2325  2688  1972  3441     384   423   345   277
+//   32 x 256 (not cut)   680   824   508   423     354   397   295   240     302   335   256   190
 //
 // One workgroup of 8 waves per (head, sequence, 128 state columns); a wave owns 16 columns and all d
 // rows of S in its accumulators for the whole portion. The summation index of an MFMA may be permuted
@@ -48,9 +48,8 @@
 // A step of the loop was up to 93 basic blocks (a bound a token, a head's widths) and waited for LDS at each of 8
 // tiles' operands. LONG takes the steps whose blocks are full, of heads of 128 channels and columns, through a copy
 // without bounds, with scalar row addresses; the next tile's operands are read ahead of a tile's products; with
-// per-channel decays the wave that has products to issue goes first (the others lose 1 to 2 % by it). Before that and
-// with it, one card: 4 x 2048 HGRN2 441 -> 382 us, GLA 501 -> 424; 1 x 8000 FIXED 417 -> 366, MLSTM 523 -> 491; 998 to
-// 2601 596 -> 553, 677 -> 615, 551 -> 511 and 425 -> 395. Equal to the bit. (MLSTM with its gates as they were then.)
+// per-channel decays the wave that has products to issue goes first (the others lose 1 to 2 % by it). 4 x 2048 tokens
+// without and with it, one card: HGRN2 441 / 382 us, GLA 501 / 424, FIXED 396 / 345, MLSTM 326 / 294. Equal to the bit.
 #include "common.h"
 
 namespace {
@@ -212,16 +211,31 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
   float* sp = a.state + ((long)slot * H + h) * d * dv + col;
   float* np = MODE == MLSTM ? a.nstate + ((long)slot * H + h) * (d + 1) : nullptr;
   const auto unit = [&](int k) { return ((long)s * a.nseg + k) * H + h; };
-  const auto seg_st = [&](int k) { return a.seg_state + unit(k) * d * dv + col; };
+  // Segments' states lie as the accumulators hold them, 8 requests of 1 KiB a wave; row by row a lane took 32, each a quarter
+  // wave's 64 bytes, for every segment folded. us, row by row / so: GLA 301 to 3000 (6) 534 / 491, FIXED 900 to
+  // 2601 (5) 445 / 395, MLSTM 322 / 289, 1 x 8000 FIXED 368 / 343, MLSTM 331 / 273
+  const auto seg_st = [&](int k) {
+    return (f32x4*)a.seg_state + ((unit(k) * gridDim.z + blockIdx.z) * 8 + w) * ND * 64 + lane;
+  };
   f32x4 st[ND];
-  const auto load_state = [&](const float* p, auto&& put) {
+  const auto load_state = [&](const float* p) {
 #pragma unroll
     for (int t = 0; t < ND; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int c = 16 * t + 4 * q + r;
-        put(t, r, p != nullptr && on && c < d ? p[(long)c * dv] : 0.f);
+        st[t][r] = p != nullptr && on && c < d ? p[(long)c * dv] : 0.f;
       }
+  };
+  const auto load_segment = [&](int k) __attribute__((always_inline)) {
+    const f32x4* p = seg_st(k);
+#pragma unroll
+    for (int t = 0; t < ND; ++t) st[t] = p[t * 64];
+  };
+  const auto store_segment = [&](int k) __attribute__((always_inline)) {
+    f32x4* p = seg_st(k);
+#pragma unroll
+    for (int t = 0; t < ND; ++t) p[t * 64] = st[t];
   };
   const auto store_state = [&](float* p) {
     if (on) {
@@ -241,15 +255,16 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
   float n0 = 0.f;
   if (seg == 0) {
     const bool copied = !STATE && cut;
-    load_state(fresh ? nullptr : copied ? seg_st(a.nseg - 1) : sp,
-               [&](int t, int r, float x) { st[t][r] = x; });
+    if (copied && !fresh) load_segment(a.nseg - 1);
+    else load_state(fresh ? nullptr : sp);
     if (MODE == MLSTM && !fresh && nc < d) n0 = copied ? a.seg_n[unit(a.nseg - 1) * UNIT + nc] : np[nc];
     if (STATE && !fresh) {
-      store_state(seg_st(a.nseg - 1));
+      store_segment(a.nseg - 1);
       if (MODE == MLSTM && q == 0 && nc < d) a.seg_n[unit(a.nseg - 1) * UNIT + nc] = n0;
     }
   } else {
-    load_state(STATE ? nullptr : seg_st(0), [&](int t, int r, float x) { st[t][r] = x; });
+    if (STATE) load_state(nullptr);
+    else load_segment(0);
     if (!STATE) {
       if (MODE == MLSTM && nc < d) n0 = a.seg_n[unit(0) * UNIT + nc];
       float Gs = 0.f, Gl = 0.f;
@@ -262,6 +277,7 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
       }
       for (int k = 1; k < seg; ++k) {
         const float* dec = a.seg_decay + unit(k) * UNIT;
+        const f32x4* own = seg_st(k);
         if (MODE == MLSTM) {
           Gs = dec[0];
           if (nc < d) n0 = Gs * n0 + a.seg_n[unit(k) * UNIT + nc];
@@ -271,8 +287,8 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
           if (CHANNEL) st[t] *= *reinterpret_cast<const f32x4*>(dec + 16 * t + 4 * q);
           else if (MODE == FIXED) st[t] = st[t] * Gs + st[t] * Gl;
           else st[t] *= Gs;
+          st[t] += own[t * 64];
         }
-        load_state(seg_st(k), [&](int t, int r, float x) { st[t][r] += x; });
       }
     }
   }
@@ -717,7 +733,7 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
     step(b, Any{});
   }
   if constexpr (STATE) {
-    store_state(seg_st(seg));
+    store_segment(seg);
     if (CHANNEL && tg == 0 && blockIdx.z == 0) a.seg_decay[unit(seg) * UNIT + sc] = sc < DP ? G_seg : 1.f;
     if (MODE == MLSTM) {
       if (w < ND && q == 0 && nc < d) a.seg_n[unit(seg) * UNIT + nc] = gm.n[nc];
@@ -845,7 +861,9 @@ int launch_by_width(const ChunkArgs& a, int num_seqs, int max_seqlen, hipStream_
 // Cut, every segment but the last runs twice, the first time (states only, several workgroups a CU) at
 // some 0.4 of a block's time. In block times, with 3 to fill and drain a workgroup and the fold. The
 // segments' states take at most 256 MB of scratch.
-static size_t unit_floats(int d, int dv) { return (size_t)d * dv + 2 * UNIT; }
+static size_t unit_floats(int d, int dv) {      // the state, in whole tiles, decays and normaliser
+  return (size_t)(d <= 32 ? 32 : d <= 64 ? 64 : 128) * ((dv + COLS - 1) / COLS) * COLS + 2 * UNIT;
+}
 static int pick_segments(int H, int d, int dv, int num_seqs, int max_seqlen, int T, int min_len) {
   // the sequences that min_len leaves count for nothing: beside the longest at most this many others
   const int others = (T - max_seqlen) / (min_len > 1 ? min_len : 1);
@@ -859,7 +877,9 @@ static int pick_segments(int H, int d, int dv, int num_seqs, int max_seqlen, int
     if (len < 128) break;
     const int k = (max_seqlen + len - 1) / len;
     if ((size_t)num_seqs * k * H * unit_floats(d, dv) > (64u << 20)) break;
-    const long all = (long)seqs * k, most = T / len + seqs, units = all < most ? all : most;
+    // (a ragged portion's last segment is half full on average: with a whole one counted for each, 5 of 516 to 1032 tokens 274
+    // us and 218 so, 4 of 556 to 1112 215 and 185, 6 of 301 to 3000 496 and 453; 24 mixes, none slower)
+    const long all = (long)seqs * k, most = T / len + (seqs + 1) / 2, units = all < most ? all : most;
     const float cost = rounds(units) * (len / 16 + 3.f) * 1.4f + 0.4f * k;
     if (cost < best) { best = cost; pick = k; }
   }

@@ -137,9 +137,9 @@ __global__ void __launch_bounds__(STATS ? 256 : 512) mix_attention_kernel(MixArg
       dma_lanes(to + p * 8 * DVW * 2, a.v + (long)slot[tile * TK + r] * a.v_stride + grp * HD + dvo + c * 8);
     }
   };
-  // A tile's values are requested ahead of its keys, whose wait then is for both: with two value tiles a whole tile ahead.
-  // (hipcc counts the keys alone. With one value tile its requests follow the next keys', and the wait for those is for
-  // values that were requested just before)
+  // With two value tiles a tile's values are requested a whole tile ahead, ahead of its keys; with one, behind the next
+  // keys. hipcc waits for the keys, and does not count the values: the loop waits for both itself, where it needs the
+  // keys and nothing else is in flight
   if constexpr (!STATS) load_v(0);
   load_k(0, 0);
   load_k(0, 1);
@@ -148,6 +148,7 @@ __global__ void __launch_bounds__(STATS ? 256 : 512) mix_attention_kernel(MixArg
     const int j0 = lo + tile * TK;
     // (rows past the last query keep m = l = 0 or are not stored: whatever they hold stays theirs)
     const bool interior = j0 + TK - 1 <= p0 && j0 > p_last - a.window;
+    if constexpr (!STATS) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // keys and values of this tile landed
     if constexpr (!STATS && NV == 2) {             // (behind hipcc's wait for the keys, which would be for these too)
 #pragma unroll
       for (int kk = 0; kk < HD / 32; ++kk) asm volatile("" : "+v"(kf[0][kk]), "+v"(kf[1][kk]));

@@ -1,5 +1,6 @@
 """The build's look through the assembly of kernels whose matrix products are asm statements, which hipcc pads nothing
 for: what it finds, what it lets pass, and the kernels themselves."""
+import re
 import subprocess
 
 import pytest
@@ -54,10 +55,41 @@ def test_kernels_with_asm_products_are_looked_through():
         build.check_scratch("x: remark: Function Name: _Z19prefill_long_kernelILi0EEv\nx: remark: ScratchSize [bytes/lane]: 8\n", "x")
 
 
-def test_long_attention(tmp_path):
-    src, out = build.CSRC / "kernels" / "attention_prefill_long.hip", tmp_path / "k.s"
+def assembly(name, tmp_path):
+    src, out = build.CSRC / "kernels" / name, tmp_path / "k.s"
     subprocess.run([build._hipcc(), *build.KERNEL_FLAGS, "-I", str(src.parent), "--offload-device-only", "-S", str(src), "-o", str(out)],
                    check=True, capture_output=True)
-    text = out.read_text()
+    return out.read_text()
+
+
+def test_long_attention(tmp_path):
+    text = assembly("attention_prefill_long.hip", tmp_path)
     assert sum(fn.name.startswith("_Z19prefill_long_kernel") for fn in asm_check.functions(text)) == 2
-    asm_check.check(text, src.name)
+    asm_check.check(text, "attention_prefill_long.hip")
+
+
+# hipcc does not count LDS-DMA that is asked for in asm statements: what it waits for, and where, is only its own loads' business. So
+# the source itself waits for a tile's values between their request and the transposed reads of them, in every iteration
+def test_values_of_the_mixing_attention_are_waited_for(tmp_path):
+    text = assembly("mix_attention.hip", tmp_path)
+    asked = re.sub(r"#ASMSTART\n\ts_waitcnt vmcnt\(0\)", "#ASMSTART\n\ts_asked", text)
+    forms = [fn for fn in asm_check.functions(asked) if "mix_attention_kernelILb0E" in fn.name]
+    assert len(forms) == 2                                  # one value tile a wave, and two
+
+    def unwaited(fn, at):
+        """The transposed reads that can follow ``at`` without such a wait."""
+        seen, todo = set(), list(fn.following(at))
+        while todo:
+            n = todo.pop()
+            if n not in seen and fn.code[n][0] != "s_asked":
+                seen.add(n)
+                todo += fn.following(n)
+        return {n for n in seen if fn.code[n][0].startswith("ds_read_b64_tr")}
+
+    for fn in forms:
+        where = lambda name: [n for n, c in enumerate(fn.code) if c[0].startswith(name)]  # noqa: E731
+        reads, requests = where("ds_read_b64_tr"), where("global_load_lds")
+        assert reads and requests and not unwaited(fn, 0)
+        assert all(min(unwaited(fn, n), default=n + 1) > n for n in reads)      # (nor once round the loop)
+        if "ILb0ELi1E" in fn.name:                          # (two tiles: the reads behind a request are of the other one)
+            assert not any(unwaited(fn, n) for n in requests)

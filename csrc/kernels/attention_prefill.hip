@@ -565,6 +565,13 @@ using launch_wave64 = int(void* out, int out_stride, const void* qkv, int row_st
                           const void* v_cache, const int* block_tables, int bt_stride, int block_size, hipStream_t st);
 launch_wave64 launch_prefill_long, launch_prefill_pairs;
 
+// Whether the kernel with 64 rows a wave can read the rows: at 31-bit offsets from their sequence's first, or, with keys and
+// values in the cache, from a wave's first of 32; and cached blocks that hold whole rows of a piece
+static bool wave64_reads(bool paged, long L, int row_stride, int block_size) {
+  if (!paged) return (L + PL_ROWS) * row_stride * 2 < (1L << 31);
+  return row_stride < 1 << 25 && block_size >= 16 && !(block_size & (block_size - 1));
+}
+
 // Whether a launch takes waves of 64 rows. They gain on long sequences (2500 tokens 77 -> 69.5 us, 7993 516 -> 471, 7
 // x 2048 306 -> 291) and lose on short ones, whose last waves they leave idle (1000 tokens equal, 500 161 -> 174, 300 180
 // -> 222), and by every block, which has a CU to itself. One round of workgroups is for the other kernel, which pairs
@@ -578,8 +585,7 @@ launch_wave64 launch_prefill_long, launch_prefill_pairs;
 // every sequence must have a block of rows, however the T are dealt.
 static bool takes_wave64(bool paged, long T, int n, long L, int hq, int hd, int row_stride, int block_size) {
   if (hd != 128 || L < max(g_pw_min_len, g_pl_min_len) || (L + PL_ROWS - 1) / PL_ROWS * hq * n <= PL_ROUND) return false;
-  // (rows at 32-bit offsets from their sequence's first, and cached blocks that hold whole rows of a piece)
-  if (paged ? block_size < 16 || (block_size & (block_size - 1)) : (L + PL_ROWS) * row_stride * 2 >= (1L << 31)) return false;
+  if (!wave64_reads(paged, L, row_stride, block_size)) return false;
   if (g_pw_min_len != PW_MIN_LEN || n == 1) return true;
   if (paged) return T - (n - 1) * L >= PL_ROWS;
   if ((T / PL_ROWS + n) * hq <= 400) return true;
@@ -594,7 +600,7 @@ static bool takes_wave64(bool paged, long T, int n, long L, int hq, int hd, int 
 static bool pairs_wave64(bool paged, int n, long L, int hq, int hd, int row_stride, int block_size) {
   const long blocks = (L + PL_ROWS - 1) / PL_ROWS;
   if (hd != 128 || L < g_pl_min_len || blocks < 2 || blocks * hq * n > PL_ROUND || g_pw_min_len != PW_MIN_LEN) return false;
-  return paged ? block_size >= 16 && !(block_size & (block_size - 1)) : (L + PL_ROWS) * row_stride * 2 < (1L << 31);
+  return wave64_reads(paged, L, row_stride, block_size);
 }
 
 template <bool PAGED>

@@ -106,3 +106,13 @@ def test_rising_scores(gpu):
     ([512] * 4, 32, 32, True), ([512] * 5, 32, 32, False), ([2048], 32, 8, False), ([2048], 32, 24, False)])
 def test_choice(lens, hq, block, expected):
     assert taken(lens, hq, (hq + 16) * HD, block) == expected
+
+
+# rows so far apart that 32 of them, a wave's queries, leave the kernel's 32-bit offsets are the other kernel's
+@pytest.mark.parametrize("block", [0, 16])
+def test_rows_far_apart(block):
+    from distributed_llm_inferencing_amd.ops import _native
+    lib = _native.require_native()
+    assert taken([300], 4, 1 << 20, block) and not taken([300], 4, 1 << 25, block)
+    assert lib.dli_prefill_takes_wave64(4100, 1, 4100, 32, HD, 1 << 17, block)
+    assert not lib.dli_prefill_takes_wave64(4100, 1, 4100, 32, HD, 1 << 25, block)

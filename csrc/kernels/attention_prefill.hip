@@ -271,7 +271,7 @@ __device__ __forceinline__ float pl_max3(float a, float b, float c) {  // no can
 // and are staged through scalar descriptors (lds_dma.h); other blocks, row by row, whose table every lane reads, behind
 // all DMA in flight. 2048 queries of 4096 keys 133 -> 126 us, 1024 of 6000 174 -> 163, 6 x 400 of 2400 147 -> 138. The
 // activation's rows gain nothing so (4 x 1000 62.2 and 61.9, 2048 51.4 and 51.6).
-// whole: queries at 16-byte addresses. They come, and outputs leave, through a row image a wave in LDS: row by row a lane each
+// dwords: queries at addresses of whole dwords. They come, and outputs leave, through a row image a wave in LDS: row by row a lane each
 // request took 32 rows, 10 k cycles a workgroup in all. 32 heads on 8, us: 8 x 256 tokens 19.0 -> 15.4, 20 x 400 81 -> 73, 8 of
 // 300 to 2000 125 -> 114, 5 x 1500 132 -> 126, 8 x 1000 of 2000 cached 238 -> 232. Equal to the bit.
 enum { ROWS_OF_QKV = 0, BLOCKS_OF_16 = 1, BLOCKS = 2 };
@@ -281,7 +281,7 @@ __global__ void __launch_bounds__(512) prefill_attn32_kernel(
     const int* __restrict__ cu_seqlens, int hq, int hkv, float scale_log2,
     const int* __restrict__ ctx_lens, const u16* __restrict__ k_cache,
     const u16* __restrict__ v_cache, const int* __restrict__ block_tables, int bt_stride,
-    int block_size, int block_shift, bool paired, bool whole) {
+    int block_size, int block_shift, bool paired, bool dwords) {
   static_assert(HD == 128, "long-sequence kernel: head_dim 128");
   constexpr bool PAGED = SRC != ROWS_OF_QKV;
   constexpr int KC = HD / 16;                      // K-steps of the QK^T product
@@ -327,10 +327,10 @@ __global__ void __launch_bounds__(512) prefill_attn32_kernel(
   const int* btab = PAGED ? block_tables + (long)seq * bt_stride : nullptr;
   const long head_off = (long)kvh * block_size * HD;
 
-  // Q^T operand: lane (query qc, half hi) holds Q[q][16c + 8hi .. +7]. Rows at 16-byte addresses come as a tile image (a row
+  // Q^T operand: lane (query qc, half hi) holds Q[q][16c + 8hi .. +7]. Rows of whole dwords come as a tile image (a row
   // a lane takes 32 rows a request, 4 k cycles ahead of the first tile)
   bf16x8 qf[KC];
-  if (whole) {
+  if (dwords) {
     const int rl = (lane & 31) >> 2;
     const uint32_t to = lds_address(&rows_lds[wid][0]);
 #pragma unroll
@@ -413,7 +413,7 @@ __global__ void __launch_bounds__(512) prefill_attn32_kernel(
   stage(0, 0);
   // the queries are there from here on: hipcc would wait for them where it first uses them, in every tile, and so for the
   // DMA in flight, which it does not count
-  if (SRC == BLOCKS_OF_16 && !whole) {
+  if (SRC == BLOCKS_OF_16 && !dwords) {
 #pragma unroll
     for (int c = 0; c < KC; ++c) asm volatile("" : "+v"(qf[c]));
   }
@@ -436,7 +436,7 @@ __global__ void __launch_bounds__(512) prefill_attn32_kernel(
     vbase_off[0] = 64 * (4 * hi + q4) + 16 * (cl ^ hi) + 8 * (p4 & 1);
     vbase_off[1] = 2048 + 64 * (4 * hi + q4) + 16 * (cl ^ (hi ^ 2)) + 8 * (p4 & 1);
   }
-  if (whole) {
+  if (dwords) {
 #pragma unroll
     for (int c = 0; c < KC; ++c) {
       qf[c] = *reinterpret_cast<const bf16x8*>(&rows_lds[wid][kbase_off[c & 1] + 512 * (c >> 1)]);
@@ -566,10 +566,13 @@ using launch_wave64 = int(void* out, int out_stride, const void* qkv, int row_st
 launch_wave64 launch_prefill_long, launch_prefill_pairs;
 
 // Whether the kernel with 64 rows a wave can read the rows: at 31-bit offsets from their sequence's first, or, with keys and
-// values in the cache, from a wave's first of 32; and cached blocks that hold whole rows of a piece
-static bool wave64_reads(bool paged, long L, int row_stride, int block_size) {
+// values in the cache, from a wave's first of 32; and cached blocks that hold whole rows of a piece. Queries come by LDS-DMA,
+// from whole dwords: those at other addresses are the other kernel's, which can read them by plain loads (in the
+// activation's rows keys and values are at the same addresses and come by LDS-DMA on either)
+static bool by_dwords(const void* qkv, int row_stride) { return row_stride % 2 == 0 && ((uintptr_t)qkv & 3) == 0; }
+static bool wave64_reads(bool paged, long L, const void* qkv, int row_stride, int block_size) {
   if (!paged) return (L + PL_ROWS) * row_stride * 2 < (1L << 31);
-  return row_stride < 1 << 25 && block_size >= 16 && !(block_size & (block_size - 1));
+  return by_dwords(qkv, row_stride) && row_stride < 1 << 25 && block_size >= 16 && !(block_size & (block_size - 1));
 }
 
 // Whether a launch takes waves of 64 rows. They gain on long sequences (2500 tokens 77 -> 69.5 us, 7993 516 -> 471, 7
@@ -583,9 +586,9 @@ static bool wave64_reads(bool paged, long L, int row_stride, int block_size) {
 // them slower by 1 to 2.5 %, and leaves 77 that would be slower by up to 19 % (and 32 that would gain). In the cache a few
 // rows may stand behind any number of keys, on one wave of a workgroup (2048 of 2048 and 40 of 8000 217 / 263): there
 // every sequence must have a block of rows, however the T are dealt.
-static bool takes_wave64(bool paged, long T, int n, long L, int hq, int hd, int row_stride, int block_size) {
+static bool takes_wave64(bool paged, long T, int n, long L, int hq, int hd, const void* qkv, int row_stride, int block_size) {
   if (hd != 128 || L < max(g_pw_min_len, g_pl_min_len) || (L + PL_ROWS - 1) / PL_ROWS * hq * n <= PL_ROUND) return false;
-  if (!wave64_reads(paged, L, row_stride, block_size)) return false;
+  if (!wave64_reads(paged, L, qkv, row_stride, block_size)) return false;
   if (g_pw_min_len != PW_MIN_LEN || n == 1) return true;
   if (paged) return T - (n - 1) * L >= PL_ROWS;
   if ((T / PL_ROWS + n) * hq <= 400) return true;
@@ -597,10 +600,10 @@ static bool takes_wave64(bool paged, long T, int n, long L, int hq, int hd, int 
 // wherever that kernel can read the rows. It is ahead from 257 tokens on: 300 14.7 / 14.6 us, 400 18.8 / 16.0, 300 of 300
 // cached 15.5 / 15.5, 2048 of 8048 250 / 217 (54 mixes of lengths, contexts and heads: 0.80 to 1.00 of the time). Other
 // lengths than the default set by dli_prefill_set_wave64_len leave such launches to waves of 32 rows.
-static bool pairs_wave64(bool paged, int n, long L, int hq, int hd, int row_stride, int block_size) {
+static bool pairs_wave64(bool paged, int n, long L, int hq, int hd, const void* qkv, int row_stride, int block_size) {
   const long blocks = (L + PL_ROWS - 1) / PL_ROWS;
   if (hd != 128 || L < g_pl_min_len || blocks < 2 || blocks * hq * n > PL_ROUND || g_pw_min_len != PW_MIN_LEN) return false;
-  return wave64_reads(paged, L, row_stride, block_size);
+  return wave64_reads(paged, L, qkv, row_stride, block_size);
 }
 
 template <bool PAGED>
@@ -612,10 +615,8 @@ static int launch_prefill(void* out, int out_stride, const void* qkv, int row_st
   if (num_seqs <= 0 || max_seqlen <= 0) return 0;
   if (hq % hkv || (hd != 64 && hd != 128)) return (int)hipErrorInvalidValue;
   const float sl2 = scale * 1.4426950408889634f;
-  // queries come by 16-byte LDS-DMA, as keys and values in the activation's rows do
-  const bool whole = row_stride % 8 == 0 && ((uintptr_t)qkv & 15) == 0;
-  const bool pairs = (whole || !PAGED) && pairs_wave64(PAGED, num_seqs, max_seqlen, hq, hd, row_stride, block_size);
-  if (pairs || ((whole || !PAGED) && takes_wave64(PAGED, tokens, num_seqs, max_seqlen, hq, hd, row_stride, block_size)))
+  const bool pairs = pairs_wave64(PAGED, num_seqs, max_seqlen, hq, hd, qkv, row_stride, block_size);
+  if (pairs || takes_wave64(PAGED, tokens, num_seqs, max_seqlen, hq, hd, qkv, row_stride, block_size))
     return (pairs ? launch_prefill_pairs : launch_prefill_long)(
         out, out_stride, qkv, row_stride, cu_seqlens, num_seqs, max_seqlen, hq, hkv, sl2, PAGED ? ctx_lens : nullptr,
         k_cache, v_cache, block_tables, bt_stride, block_size, st);
@@ -626,7 +627,8 @@ static int launch_prefill(void* out, int out_stride, const void* qkv, int row_st
     const bool by16 = PAGED && block_size >= 16 && (block_size & (block_size - 1)) == 0;
     const int shift = by16 ? __builtin_ctz(block_size) : 0;
 #define PL_ARGS (u16*)out, out_stride, (const u16*)qkv, row_stride, cu_seqlens, hq, hkv, sl2, ctx_lens, \
-                (const u16*)k_cache, (const u16*)v_cache, block_tables, bt_stride, block_size, shift, paired, whole
+                (const u16*)k_cache, (const u16*)v_cache, block_tables, bt_stride, block_size, shift, paired, \
+                by_dwords(qkv, row_stride)
     if (by16) prefill_attn32_kernel<128, BLOCKS_OF_16><<<grid32, 512, 0, st>>>(PL_ARGS);
     else prefill_attn32_kernel<128, PAGED ? BLOCKS : ROWS_OF_QKV><<<grid32, 512, 0, st>>>(PL_ARGS);
 #undef PL_ARGS
@@ -693,12 +695,12 @@ extern "C" int dli_prefill_set_min_len(int n) {
 // 1 where such a launch takes waves of 64 rows (block_size 0: keys and values in the activation's rows)
 extern "C" int dli_prefill_takes_wave64(int tokens, int num_seqs, int max_seqlen, int hq, int hd, int row_stride,
                                         int block_size) {
-  return takes_wave64(block_size > 0, tokens, num_seqs, max_seqlen, hq, hd, row_stride, block_size) ? 1 : 0;
+  return takes_wave64(block_size > 0, tokens, num_seqs, max_seqlen, hq, hd, nullptr, row_stride, block_size) ? 1 : 0;
 }
 
 // 1 where it takes them in pairs of half blocks
 extern "C" int dli_prefill_pairs_wave64(int num_seqs, int max_seqlen, int hq, int hd, int row_stride, int block_size) {
-  return pairs_wave64(block_size > 0, num_seqs, max_seqlen, hq, hd, row_stride, block_size) ? 1 : 0;
+  return pairs_wave64(block_size > 0, num_seqs, max_seqlen, hq, hd, nullptr, row_stride, block_size) ? 1 : 0;
 }
 
 extern "C" int dli_prefill_set_wave64_len(int n) {

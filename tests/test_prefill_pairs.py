@@ -73,15 +73,16 @@ def test_blocks_of_the_cache(gpu, lens, before, block, hq, hkv):
             caches[:, table[i, b], :, :n] = torch.randn(2, hkv, n, HD, device=gpu, generator=g).bfloat16()
     qkv = torch.randn(sum(lens), (hq + 2 * hkv) * HD, device=gpu, generator=g).bfloat16()
     assert taken(lens, hq, qkv.stride(0), block) == (block in (16, 64, 256))
-    # rows that are not 16-byte aligned are the other kernel's too
-    odd = torch.zeros(sum(lens), qkv.shape[1] + 4, device=gpu).bfloat16()[:, 4:]
-    odd.copy_(qkv)
     call = lambda x: ops.prefill_attention_paged(x, cumulated(lens, gpu), max(lens),  # noqa: E731
                                                  torch.tensor(ctx, device=gpu, dtype=torch.int32), table.to(gpu), caches[0],
                                                  caches[1], hq, hkv, HD, HD ** -0.5)
     new = call(qkv)
     assert torch.equal(new, other(lambda: call(qkv))) and torch.isfinite(new.float()).all()
-    assert torch.equal(new, call(odd))
+    for at in (4, 2, 1):                                    # rows of whole dwords, and of none: the other kernel's too
+        odd = torch.zeros(sum(lens), qkv.shape[1] + at, device=gpu).bfloat16()[:, at:]
+        odd.copy_(qkv)
+        assert taken(lens, hq, odd.stride(0), block) == (block in (16, 64, 256) and at > 1)
+        assert torch.equal(new, call(odd))
 
 
 # scores whose maximum rises by more than the threshold in tile after tile, falls, and is equal, on both blocks of rows
@@ -106,6 +107,12 @@ def test_rising_scores(gpu):
     ([512] * 4, 32, 32, True), ([512] * 5, 32, 32, False), ([2048], 32, 8, False), ([2048], 32, 24, False)])
 def test_choice(lens, hq, block, expected):
     assert taken(lens, hq, (hq + 16) * HD, block) == expected
+
+
+# in the cache's launches rows of whole dwords, however they are aligned; in the activation's, whatever keys and values are read by
+@pytest.mark.parametrize("more,paged", [(0, True), (4, True), (2, True), (1, False)])
+def test_alignment(more, paged):
+    assert taken([300], 32, 48 * HD + more, 16) == paged and taken([300], 32, 48 * HD + more, 0)
 
 
 # rows so far apart that 32 of them, a wave's queries, leave the kernel's 32-bit offsets are the other kernel's

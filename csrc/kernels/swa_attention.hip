@@ -47,7 +47,6 @@ struct SwaArgs {
   const int* block_tables; int bt_stride; int block_size;
   int H, G, window, keep;
   float scale_log2;
-  int table_cap;                       // prefill32: list entries that fit the LDS table
   int block_shift;                     // log2 of a block's rows, where they are a power of two
   int nsplit;                          // decode: key splits
   float* ws;                           // decode, nsplit > 1: [nsplit][S][H][2], [nsplit][S][H][HD]
@@ -153,9 +152,15 @@ __device__ __forceinline__ void piece_offsets(int (&voff)[(D / 8 + 7) / 8], long
 
 // Tile image: 8-row x 32-column subtiles of 512 B with the chunks of a row rotated by its row
 // group: conflict-free for row reads and for transposed reads. DK, DR, DV: multiples of 32.
-// GROUPS: cache blocks are powers of two of at least 16 rows (or the rows a plain matrix's), staged by stage_together
-template <int DK, int DR, int DV, bool GROUPS>
+// How a tile's rows are found: SIXTEENS, cache blocks are powers of two of at least 16 rows (or the rows a plain matrix's), staged by
+// stage_together; ROWS, a table in LDS of the list's cache rows; BLOCKS, by the block table (or a plain matrix's first row).
+// Each a kernel of its own: with the choice between the latter two and both masks in one, it spilled registers at 128 + 256
+// wide. In BLOCKS, whose waves wait for the block table, the mask is key by key alone. 16 heads on 4, 8-row blocks, us, one
+// kernel / these: 128 + 256 4000 tokens 294 / 193, 513 of 6513 422 / 294, 96 + 192 the latter 325 / 271; in ROWS 2 to 7 % less
+enum { BLOCKS = 0, ROWS = 1, SIXTEENS = 2 };
+template <int DK, int DR, int DV, int FOUND>
 __global__ void __launch_bounds__(512) swa_prefill32_kernel(SwaArgs a) {
+  constexpr bool GROUPS = FOUND == SIXTEENS;
   constexpr int KW = DK + DR, KC = KW / 16, DBK = DV / 32;
   constexpr int RGK = KW * 16, RGV = DV * 16;                  // bytes of an 8-row group
   constexpr int TILE_K = KT * KW * 2, TILE_B = KT * (KW + DV) * 2, NBUF = 3;
@@ -189,8 +194,7 @@ __global__ void __launch_bounds__(512) swa_prefill32_kernel(SwaArgs a) {
     return DR ? base + j : bt[j / a.block_size] * a.block_size + j % a.block_size;
   };
   // the list's cache rows (GROUPS: of every sixteenth)
-  const bool use_table = !DR && !GROUPS && kl.n <= a.table_cap;
-  if (use_table)
+  if (FOUND == ROWS)
     for (int x = tid; x < kl.n; x += 512) table[x] = row_of(x);
   if (GROUPS && !DR)
     for (int x = tid; x < 4 * ntiles; x += 512) {
@@ -221,7 +225,7 @@ __global__ void __launch_bounds__(512) swa_prefill32_kernel(SwaArgs a) {
 
   const auto row_in_list = [&](int x) -> long {
     x = min(x, kl.n - 1);
-    return use_table ? table[x] : row_of(x);
+    return FOUND == ROWS ? table[x] : row_of(x);
   };
   int vk[(KW / 8 + 7) / 8], vv[(DV / 8 + 7) / 8];
   if constexpr (GROUPS) {
@@ -272,8 +276,9 @@ __global__ void __launch_bounds__(512) swa_prefill32_kernel(SwaArgs a) {
   stage(0, 0);
   // the queries are there from here on: hipcc would wait for them where it first uses them, in every tile, and so for the
   // DMA in flight, which it does not count
+  if constexpr (GROUPS)
 #pragma unroll
-  for (int c = 0; c < KC; ++c) asm volatile("" : "+v"(qf[c]));
+    for (int c = 0; c < KC; ++c) asm volatile("" : "+v"(qf[c]));
   if (ntiles > 1) {
     stage(1, KT);
     wait_one_tile();
@@ -312,7 +317,7 @@ __global__ void __launch_bounds__(512) swa_prefill32_kernel(SwaArgs a) {
         }
       }
       // only tiles that cross this wave's diagonal or the window's far edge are masked
-      if (kt0 >= a.keep && (kt1 > wq_lo || wq_hi - kt0 >= a.window)) {
+      if (FOUND != BLOCKS && kt0 >= a.keep && (kt1 > wq_lo || wq_hi - kt0 >= a.window)) {
         // (one run of keys: those seen are the window's that end at the query)
         const int first = kt0 + 4 * hi - (qpos - a.window + 1);
 #pragma unroll
@@ -794,11 +799,11 @@ int decode_splits(int num_seqs, int H, int G, long keys) {
 // key / value widths this file is built for
 #define SWA_WIDTHS(F) F(64, 64) F(128, 128) F(64, 128) F(96, 192) F(128, 256)
 
-template <int DK, int DR, int DV, bool GROUPS>
+template <int DK, int DR, int DV, int FOUND>
 int launch_prefill32(SwaArgs a, int sh, int num_seqs, int max_seqlen, hipStream_t st) {
   static bool raised = false;
   if (!raised) {
-    const hipError_t e = hipFuncSetAttribute((const void*)swa_prefill32_kernel<DK, DR, DV, GROUPS>,
+    const hipError_t e = hipFuncSetAttribute((const void*)swa_prefill32_kernel<DK, DR, DV, FOUND>,
                                              hipFuncAttributeMaxDynamicSharedMemorySize,
                                              160 * 1024);
     if (e != hipSuccess) return (int)e;
@@ -806,7 +811,7 @@ int launch_prefill32(SwaArgs a, int sh, int num_seqs, int max_seqlen, hipStream_
   }
   const int blocks = (max_seqlen + LROWS - 1) / LROWS;
   const dim3 grid = a.H <= 4 ? dim3(blocks, num_seqs, a.H) : dim3(blocks * a.H, num_seqs);
-  swa_prefill32_kernel<DK, DR, DV, GROUPS><<<grid, 512, sh, st>>>(a);
+  swa_prefill32_kernel<DK, DR, DV, FOUND><<<grid, 512, sh, st>>>(a);
   DLI_RETURN_LAUNCH();
 }
 
@@ -823,15 +828,17 @@ int launch_prefill32(SwaArgs a, int num_seqs, int max_seqlen, hipStream_t st) {
   // heads, 6 of 301 to 3000 222 -> 199, in windows of 1024 187 -> 158. The mask is 13 % of the first and all of the last
   const auto fits = [](long stride, int wide) { return stride >= wide && stride < (1l << 31) / (2 * (DR ? KT : 16)); };
   if (fits(a.k_stride, DK) && fits(a.v_stride, DV) && (DR == 0 || fits(a.k2_stride, DR))) {
-    if (DR) return launch_prefill32<DK, DR, DV, true>(a, TILES, num_seqs, max_seqlen, st);
+    if (DR) return launch_prefill32<DK, DR, DV, SIXTEENS>(a, TILES, num_seqs, max_seqlen, st);
     const long sixteens = (list + 32 + 63) / KT * 4;
     if (bs >= 16 && (bs & (bs - 1)) == 0 && TILES + sixteens * 4 <= MOST) {
       a.block_shift = __builtin_ctz(bs);
-      return launch_prefill32<DK, DR, DV, true>(a, TILES + (int)sixteens * 4, num_seqs, max_seqlen, st);
+      return launch_prefill32<DK, DR, DV, SIXTEENS>(a, TILES + (int)sixteens * 4, num_seqs, max_seqlen, st);
     }
   }
-  a.table_cap = !DR && list <= 6144 && TILES + list * 4 + 16 <= MOST ? (int)list : 0;
-  return launch_prefill32<DK, DR, DV, false>(a, TILES + a.table_cap * 4 + 16, num_seqs, max_seqlen, st);
+  if constexpr (DR == 0)
+    if (list <= 6144 && TILES + list * 4 <= MOST)
+      return launch_prefill32<DK, DR, DV, ROWS>(a, TILES + (int)list * 4, num_seqs, max_seqlen, st);
+  return launch_prefill32<DK, DR, DV, BLOCKS>(a, TILES, num_seqs, max_seqlen, st);
 }
 
 template <int DK, int DV>
@@ -924,7 +931,7 @@ extern "C" int dli_shared_tail_attention(const void* q, int ldq, const void* q2,
     return (int)hipErrorNotSupported;
   SwaArgs a{(const u16*)q, ldq, (const u16*)k, k_stride, (const u16*)v, v_stride, (u16*)out, ldo,
             gate, ldg, gate != nullptr, nullptr, 1.f, cu, positions, nullptr, 0, 1, H, H, window, 0,
-            scale * LOG2E, 0, 0, 1, nullptr, (const u16*)q2, ldq2, q2_head, (const u16*)k2, k2_stride, cu_ctx};
+            scale * LOG2E, 0, 1, nullptr, (const u16*)q2, ldq2, q2_head, (const u16*)k2, k2_stride, cu_ctx};
   return launch_prefill32<128, 64, 128>(a, num_seqs, max_seqlen, st);
 }
 
@@ -958,7 +965,7 @@ extern "C" int dli_swa_attention(const void* q, int ldq, const void* k, long k_s
     return (int)hipErrorNotSupported;
   SwaArgs a{(const u16*)q, ldq, (const u16*)k, k_stride, (const u16*)v, v_stride, (u16*)out, ldo,
             gate, ldg, head_gate != 0, sink, out_scale, cu, positions, block_tables, bt_stride, block_size, H, G, window, keep,
-            scale * LOG2E, 0, 0, 1, (float*)ws, nullptr, 0, 0, nullptr, 0, nullptr};
+            scale * LOG2E, 0, 1, (float*)ws, nullptr, 0, 0, nullptr, 0, nullptr};
   if (max_seqlen == 1) {
     a.nsplit = decode_splits(num_seqs, H, G, (long)window + keep);
     if (a.nsplit > 1 && ws == nullptr) return (int)hipErrorInvalidValue;

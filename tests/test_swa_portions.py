@@ -1,8 +1,12 @@
 """Portions of sliding-window attention whose tiles are staged by sixteens of cache rows: windows and kept tokens at every
 alignment to them, blocks that the form takes and that it does not, cache rows behind a sequence's last that hold NaN."""
+import re
+import subprocess
+
 import pytest
 import torch
 
+from distributed_llm_inferencing_amd import build
 from distributed_llm_inferencing_amd.ops import hybrid as H
 from distributed_llm_inferencing_amd.ops import reference as R
 
@@ -90,3 +94,14 @@ def test_shared_tails(gpu, lens, before, window):
         p = sc.masked_fill(((far < 0) | (far >= window))[None], float("-inf")).softmax(-1)
         want = (p @ v[r].view(-1, heads, d).double().permute(1, 0, 2).contiguous()).permute(1, 0, 2).reshape(n, -1)
         assert float((out[t].double() - want).norm() / want.norm()) < 2 * 2.0 ** -9
+
+
+# no form spills registers, whose traffic would pass the counted waits for the tiles (11 to 14 % where one did), but that of the row
+# table at 128 + 256 wide, which is ahead of the general mask in windows even so
+def test_registers(tmp_path):
+    src = build.CSRC / "kernels" / "swa_attention.hip"
+    r = subprocess.run([build._hipcc(), *build.KERNEL_FLAGS, build._REMARKS, "-I", str(src.parent), "--offload-device-only", "-S", str(src),
+                        "-o", str(tmp_path / "k.s")], check=True, capture_output=True, text=True)
+    scratch = dict(re.findall(r"Function Name: (\S+).*?ScratchSize \[bytes/lane\]: (\d+)", r.stderr, re.S))
+    assert sum("swa_prefill32" in k for k in scratch) >= 11
+    assert [k for k, n in scratch.items() if n != "0" and "swa_prefill32_kernelILi128ELi0ELi256ELi1E" not in k] == []

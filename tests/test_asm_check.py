@@ -93,3 +93,21 @@ def test_values_of_the_mixing_attention_are_waited_for(tmp_path):
         assert all(min(unwaited(fn, n), default=n + 1) > n for n in reads)      # (nor once round the loop)
         if "ILb0ELi1E" in fn.name:                          # (two tiles: the reads behind a request are of the other one)
             assert not any(unwaited(fn, n) for n in requests)
+
+
+# an output gate's four rows are asked for together: hipcc waits for all loads in flight ahead of each where a condition stands before it
+def test_gate_rows_of_the_matrix_memory(tmp_path):
+    text = assembly("recurrent_chunk.hip", tmp_path)
+    forms = [fn for fn in asm_check.functions(text) if re.search(r"recurrence_chunk_kernelI[tf]Li\d+ELi3ELb0ELb0E", fn.name)]
+    assert len(forms) == 6                                  # three widths, outputs in 16 and in 32 bits
+    for fn in forms:
+        starts, waited = set(fn.labels.values()), 0
+        loop = [n for n, c in enumerate(fn.code) if c[0] == "s_barrier"][1]
+        for n, (name, _, _) in enumerate(fn.code):
+            if n < loop or not name.startswith("global_load"):
+                continue
+            n -= 1
+            while fn.code[n][0] != "s_waitcnt" and n + 1 not in starts and not fn.code[n][0].startswith(("s_cbranch", "global_", "ds_")):
+                n -= 1
+            waited += fn.code[n][0] == "s_waitcnt" and "vmcnt(0)" in " ".join(fn.code[n][1])
+        assert waited <= 1, fn.name

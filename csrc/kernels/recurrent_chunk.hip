@@ -699,8 +699,9 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
   // FULL: blocks b - 2 to b + 2 are there, and full
   auto step = [&](int b, auto FULL) __attribute__((always_inline)) {
     constexpr bool full = decltype(FULL)::value;
-
-    if (!STATE && CHANNEL && w < 4 && (full || b < nb)) products(b, FULL);
+    // (per-channel decays of wide heads that are no whole tile: GLA, 32 x 256 tokens, 16 heads of 112 198 us, behind it 192)
+    constexpr bool FIRST = CHANNEL && (LONG || ND < 8);
+    if (!STATE && FIRST && w < 4 && (full || b < nb)) products(b, FULL);
     if (full || b + 1 < nb) stage(b + 1, FULL);
     if (full || b + 2 < nb) {
       load(b + 2, FULL);
@@ -712,7 +713,7 @@ __global__ void __launch_bounds__(NTH) recurrence_chunk_kernel(ChunkArgs a) {
     if constexpr (STATE) {
       products(b, FULL);
     } else {
-      if (!CHANNEL && w < 4 && (full || b < nb)) products(b, FULL);
+      if (!FIRST && w < 4 && (full || b < nb)) products(b, FULL);
       if (full || b >= 2) write_out(b - 2, FULL);
       if (full || (b >= 1 && b <= nb)) finish(b - 1, FULL);
       if (w >= 4 && (full || b < nb)) products(b, FULL);
@@ -835,19 +836,23 @@ int launch_one(const ChunkArgs& a, int num_seqs, hipStream_t st) {
   recurrence_chunk_kernel<S, ND, MODE, STATE, LONG><<<grid, NTH, sh, st>>>(a);
   DLI_RETURN_LAUNCH();
 }
+// Whether portions of at most max_seqlen tokens take the kernels with a loop for full blocks. Blocks b - 2 to b + 2 are full
+// for the first time in a portion of 5 blocks. 64 portions of 80 / 96 / 128 tokens, us, without and with that loop: HGRN2 235 /
+// 273 / 345 and 242 / 275 / 338, GLA 273 / 319 / 412 and 276 / 309 / 379, FIXED 211 / 242 / 302 and 209 / 237 / 293, MLSTM
+// 144 / 174 / 220 and 150 / 180 / 219. Segments have 128 tokens and more. Only where the heads can run that loop: the general one
+// beside it costs more than by itself (4 x 2048 tokens, HGRN2, 32 heads of 96 534 / 432 us, GLA, 16 of 112 328 / 262)
+bool takes_long(int mode, int max_seqlen, int d, int dv, int ldp, int ldz, int ldo) {
+  return d == 128 && dv >= COLS && ldp < 1 << 24 && ldz < 1 << 24 && ldo < 1 << 24 && max_seqlen >= (mode == MLSTM ? 128 : 96);
+}
 template <typename S, int ND, int MODE>
 int launch_chunks(const ChunkArgs& a, int num_seqs, int max_seqlen, hipStream_t st) {
-  // Blocks b - 2 to b + 2 are full for the first time in a portion of 5 blocks. 64 portions of 80 / 96 / 128 tokens, us, without
-  // and with that loop: HGRN2 235 / 273 / 345 and 242 / 275 / 338, GLA 273 / 319 / 412 and 276 / 309 / 379, FIXED
-  // 211 / 242 / 302 and 209 / 237 / 293, MLSTM 144 / 174 / 220 and 150 / 180 / 219. Segments have 128 tokens and more.
   constexpr bool WIDE = ND == 8;
-  constexpr int MIN_LONG = MODE == MLSTM ? 128 : 96;
+  const bool lng = WIDE && takes_long(MODE, max_seqlen, a.d, a.dv, a.ldp, a.ldz, a.ldo);
   if (a.nseg > 1) {
-    const int rc = launch_one<S, ND, MODE, true, WIDE>(a, num_seqs, st);
+    const int rc = lng ? launch_one<S, ND, MODE, true, WIDE>(a, num_seqs, st) : launch_one<S, ND, MODE, true, false>(a, num_seqs, st);
     if (rc) return rc;
   }
-  if (WIDE && max_seqlen >= MIN_LONG) return launch_one<S, ND, MODE, false, WIDE>(a, num_seqs, st);
-  return launch_one<S, ND, MODE, false, false>(a, num_seqs, st);
+  return lng ? launch_one<S, ND, MODE, false, WIDE>(a, num_seqs, st) : launch_one<S, ND, MODE, false, false>(a, num_seqs, st);
 }
 
 template <typename S, int MODE>
@@ -953,4 +958,9 @@ extern "C" int dli_recurrence_chunks(int mode, const float* proj, int ldp, const
                      : launch_by_width<float, MLSTM>(a, num_seqs, max_seqlen, st);
   }
   return (int)hipErrorInvalidValue;
+}
+
+// 1 where portions of whole sequences take the loop for full blocks
+extern "C" int dli_recurrence_long(int mode, int max_seqlen, int d, int dv, int ldp, int ldz, int ldo) {
+  return takes_long(mode, max_seqlen, d, dv, ldp, ldz, ldo) ? 1 : 0;
 }

@@ -103,6 +103,7 @@ _SIGS = {
     # portions of the linear recurrences (recurrent_chunk.hip)
     "dli_recurrence_chunks": [I, P, I, P, I, P, P, F, F, P, P, F, P, F, P, P, P, P, P, P, I, F, I, I, I,
                               I, I, I, I, I, P, P],
+    "dli_recurrence_long": [I, I, I, I, I, I, I],
     "dli_recurrence_workspace_bytes": [I, I, I, I, I, I, I, I],
     # post-norm designs (postnorm.hip)
     "dli_prev_tokens": [P, P, P, P, P, P, I, I, P],

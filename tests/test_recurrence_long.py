@@ -1,7 +1,7 @@
 """Portions whose full blocks take a loop of their own (heads of 128 channels, column blocks of 128), against the float64 walk:
 portions around the shortest that take it, last blocks of 1, 15 and 16 tokens behind it, shorter portions beside
-them, a whole column block beside a narrower one, and decays that leave the range of fp32; and the matrix memory's gates
-at the edges of a lane's tokens and of a pass."""
+them, a whole column block beside a narrower one, and decays that leave the range of fp32; heads that cannot take it; and the
+matrix memory's gates at the edges of a lane's tokens and of a pass."""
 import pytest
 import torch
 
@@ -32,3 +32,23 @@ def test_column_blocks(gpu, dv, lens):
 def test_gates_of_the_matrix_memory(gpu, strong, lens):
     n = len(lens)
     check(gpu, "mlstm", 128, 128, strong, torch.float32, lens, [3, 0, 2][:n], [0, 1, 0][:n])
+
+
+# narrower heads, columns short of a block and rows past 24 bits keep the kernels of the general loop alone
+@pytest.mark.parametrize("mode,tokens,d,dv,stride,expected", [
+    (0, 96, 128, 128, 4096, 1), (0, 95, 128, 128, 4096, 0), (3, 127, 128, 128, 4096, 0), (3, 128, 128, 128, 4096, 1),
+    (2, 4000, 128, 200, 4096, 1), (0, 4000, 96, 96, 4096, 0), (1, 4000, 112, 128, 4096, 0), (0, 4000, 128, 64, 4096, 0),
+    (3, 4000, 100, 100, 4096, 0), (1, 4000, 128, 128, 1 << 24, 0)])
+def test_choice(mode, tokens, d, dv, stride, expected):
+    from distributed_llm_inferencing_amd.ops import _native
+    assert _native.require_native().dli_recurrence_long(mode, tokens, d, dv, stride, 4096, 4096) == expected
+
+
+# wide heads that are no whole tile, portions cut and whole
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["hgrn2", "gla", "lightning", "mlstm"])
+@pytest.mark.parametrize("d,dv", [(96, 96), (112, 128), (128, 64)])
+@pytest.mark.parametrize("lens", [[129, 33, 144], [700, 5]])
+def test_wide_heads_of_no_whole_tile(gpu, mode, d, dv, lens):
+    n = len(lens)
+    check(gpu, mode, d, dv, True, torch.float32, lens, [2, 0, 4][:n], [0, 1, 0][:n])

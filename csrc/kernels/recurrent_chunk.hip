@@ -21,10 +21,10 @@
 // less than half the work), the second starts every segment from the fold of the states before it.
 //
 // d = dv = 128, HGRN2 / GLA / FIXED of 32 heads / MLSTM of 16, us; the walk, whole portions (before LONG), and what runs:
-//   4 x 2048 tokens     1667  2342   976  1938     621   704   517   895     385   425   345   244
-//   998 to 2601 (5)                                768   891   650  1133     474   522   432   307
-//   1 x 8000                                      2325  2688  1972  3441     384   423   345   277
-//   32 x 256 (not cut)   680   824   508   423     354   397   295   240     302   335   256   190
+//   4 x 2048 tokens     1667  2342   976  1938     621   704   517   895     386   424   346   241
+//   998 to 2601 (5)                                768   891   650  1133     461   503   410   305
+//   1 x 8000                                      2325  2688  1972  3441     384   421   345   274
+//   32 x 256 (not cut)   680   824   508   423     354   397   295   240     307   332   258   183
 //
 // One workgroup of 8 waves per (head, sequence, 128 state columns); a wave owns 16 columns and all d
 // rows of S in its accumulators for the whole portion. The summation index of an MFMA may be permuted
@@ -865,8 +865,14 @@ int launch_by_width(const ChunkArgs& a, int num_seqs, int max_seqlen, hipStream_
 // Segments of a portion of at most max_seqlen tokens (T in all): a CU takes one workgroup, so few heads
 // and sequences, or ragged ones, leave most of the chip idle for as long as the longest portion takes.
 // Cut, every segment but the last runs twice, the first time (states only, several workgroups a CU) at
-// some 0.4 of a block's time. In block times, with 3 to fill and drain a workgroup and the fold. The
-// segments' states take at most 256 MB of scratch.
+// some 0.3 of a block's time. In block times, with 3 to fill and drain a workgroup. The segments' states take at most 256
+// MB of scratch.
+// A portion may end in a segment of any length, and the lengths are on the device: rounds of workgroups count a whole one for
+// each. But where they differ the shorter ones fill the CUs that others leave, so that no more than the work of a CU, half
+// a last segment a portion, and part of a workgroup counts. Over 1400 mixes of 1 to 24 portions, 4 to 32 heads of 32 to 128 and all
+// four recurrences, every number of segments timed, this is 1.039 of the best one's time (geometric mean), rounds of whole last
+// segments alone 1.052; it is more than 3 % behind those on 5 mixes and ahead on 97. Rounds of half last segments are 1.051, and
+// behind on 136: 4 of 1994 to 3988 tokens, HGRN2, 16 heads of 32, in 5 segments 225 us, in 9 143.
 static size_t unit_floats(int d, int dv) {      // the state, in whole tiles, decays and normaliser
   return (size_t)(d <= 32 ? 32 : d <= 64 ? 64 : 128) * ((dv + COLS - 1) / COLS) * COLS + 2 * UNIT;
 }
@@ -875,18 +881,23 @@ static int pick_segments(int H, int d, int dv, int num_seqs, int max_seqlen, int
   const int others = (T - max_seqlen) / (min_len > 1 ? min_len : 1);
   const int seqs = others < 0 ? 1 : others < num_seqs ? 1 + others : num_seqs;
   const long wg = (long)H * ((dv + COLS - 1) / COLS);
-  const auto rounds = [&](long units) { return (units * wg + 255) / 256; };
-  float best = 0.9f * rounds(seqs) * (max_seqlen / 16 + 3.f);
+  const bool ragged = T < (long)seqs * max_seqlen;
+  // what `units` workgroups a head of at most len tokens take that hold as much as `filled` whole ones' overhead and T tokens
+  const auto time = [&](long units, long filled, int len, float behind) {
+    const float one = len / 16.f + 3.f, even = (units * wg + 255) / 256 * one;
+    if (!ragged || units * wg <= 256) return even;
+    const float each = (T / 16.f + 3.f * filled) * wg / 256;
+    return fminf(even, fmaxf(one, each) + behind * one);
+  };
+  float best = time(seqs, seqs, max_seqlen, 0.4f);
   int pick = 1;
   for (int n = 2; n <= 16 && (long)num_seqs * n <= 65535; ++n) {
     const int len = ((max_seqlen + n - 1) / n + TB - 1) / TB * TB;
     if (len < 128) break;
     const int k = (max_seqlen + len - 1) / len;
     if ((size_t)num_seqs * k * H * unit_floats(d, dv) > (64u << 20)) break;
-    // (a ragged portion's last segment is half full on average: with a whole one counted for each, 5 of 516 to 1032 tokens 274
-    // us and 218 so, 4 of 556 to 1112 215 and 185, 6 of 301 to 3000 496 and 453; 24 mixes, none slower)
-    const long all = (long)seqs * k, most = T / len + (seqs + 1) / 2, units = all < most ? all : most;
-    const float cost = rounds(units) * (len / 16 + 3.f) * 1.4f + 0.4f * k;
+    const long all = (long)seqs * k, whole = T / len + seqs, half = T / len + (seqs + 1) / 2;
+    const float cost = time(all < whole ? all : whole, all < half ? all : half, len, 0.7f) * 1.3f + 0.1f * k;
     if (cost < best) { best = cost; pick = k; }
   }
   return pick;

@@ -310,8 +310,8 @@ __global__ void __launch_bounds__(512) prefill_attn32_kernel(
   const int nkeys = PAGED ? ctx_lens[seq] : len;
   const int qoff = nkeys - len;
   // Up to a workgroup for each CU there is nothing to even out the causal bounds with, and the last
-  // block's workgroup, which sees most keys, takes as long as the launch (where the kernel with 64 rows a wave cannot read
-  // the rows, which is ahead there: pairs_wave64). Paired, waves 0 to 3 take a
+  // block's workgroup, which sees most keys, takes as long as the launch (fewer than 600 tokens, and rows that
+  // the kernel with 64 rows a wave cannot read: pairs_wave64). Paired, waves 0 to 3 take a
   // half block counted from the end and waves 4 to 7 its counterpart from the start: a SIMD, which
   // holds one wave of each, has the long one to itself when the short one is through. 32 heads, us:
   // 2048 tokens 78 -> 66, 1024 45 -> 40, the second 2048 of a prompt 150 -> 135, 1024 after 5000 192 -> 185.
@@ -596,14 +596,17 @@ static bool takes_wave64(bool paged, long T, int n, long L, int hq, int hd, cons
   return low >= 1200.0 + 2e5 * n / T;
 }
 
-// Whether a launch of up to a workgroup a CU takes waves of 64 rows in pairs of half blocks (attention_prefill_pairs.hip):
-// wherever that kernel can read the rows. It is ahead from 257 tokens on: 300 14.7 / 14.6 us, 400 18.8 / 16.0, 300 of 300
-// cached 15.5 / 15.5, 2048 of 8048 250 / 217 (54 mixes of lengths, contexts and heads: 0.80 to 1.00 of the time). Other
+// Whether a launch of up to a workgroup a CU takes waves of 64 rows in pairs of half blocks (attention_prefill_pairs.hip).
+// Of prompts alone it is ahead from some 600 tokens on, below them the other kernel, whose workgroups begin and end sooner.
+// 32 heads on 8, us, this one / that one in its pairs: 257 14.1 / 12.6, 400 16.6 / 15.9, 512 17.7 / 17.6, 576 18.5 / 18.4, 640
+// 19.5 / 19.8, 1024 25.3 / 27.2, 2048 44.1 / 49.3; 4 of 300 15.5 / 13.8; 8 heads and 4 within 2 % of the same ratios. Behind
+// cached tokens, whose number the host does not know, 257 with 64 of them 16.6 / 14.9, 512 27.1 / 26.4, 1024 39.0 / 39.4, 6000
+// 154 / 167; 512 21.0 / 20.1, 31.2 / 31.6, 43.2 / 45.1, 160 / 181: taken from the first length of two blocks on. Other
 // lengths than the default set by dli_prefill_set_wave64_len leave such launches to waves of 32 rows.
 static bool pairs_wave64(bool paged, int n, long L, int hq, int hd, const void* qkv, int row_stride, int block_size) {
   const long blocks = (L + PL_ROWS - 1) / PL_ROWS;
   if (hd != 128 || L < g_pl_min_len || blocks < 2 || blocks * hq * n > PL_ROUND || g_pw_min_len != PW_MIN_LEN) return false;
-  return wave64_reads(paged, L, qkv, row_stride, block_size);
+  return (paged || L >= 600) && wave64_reads(paged, L, qkv, row_stride, block_size);
 }
 
 template <bool PAGED>

@@ -26,8 +26,9 @@ def cumulated(lens, gpu):
     return torch.tensor([0, *lens]).cumsum(0).to(gpu, torch.int32)
 
 
-# one half block and two, an odd and an even number of them, one row in the last wave, half block and block
-LENS = [[257], [300, 1, 64], [383, 384], [385, 32, 33, 129], [512, 511], [513, 640], [700, 256, 255], [1025], [2048]]
+# an odd and an even number of half blocks, one row in the last wave, half block and block; beside the longest, one half block,
+# two and three
+LENS = [[600], [700, 300, 1, 64], [640, 383, 384], [641, 32, 33, 129], [768, 257], [769, 512], [700, 256, 255], [1025], [2048]]
 
 
 @pytest.mark.gpu
@@ -103,7 +104,7 @@ def test_rising_scores(gpu):
 
 
 @pytest.mark.parametrize("lens,hq,block,expected", [
-    ([257], 32, 0, True), ([256], 32, 0, False), ([2048], 32, 16, True), ([2049], 32, 16, False), ([2048], 32, 0, True),
+    ([257], 32, 16, True), ([256], 32, 16, False), ([600], 32, 0, True), ([599], 32, 0, False), ([2048], 32, 16, True), ([2049], 32, 16, False), ([2048], 32, 0, True),
     ([512] * 4, 32, 32, True), ([512] * 5, 32, 32, False), ([2048], 32, 8, False), ([2048], 32, 24, False)])
 def test_choice(lens, hq, block, expected):
     assert taken(lens, hq, (hq + 16) * HD, block) == expected
@@ -112,7 +113,7 @@ def test_choice(lens, hq, block, expected):
 # in the cache's launches rows of whole dwords, however they are aligned; in the activation's, whatever keys and values are read by
 @pytest.mark.parametrize("more,paged", [(0, True), (4, True), (2, True), (1, False)])
 def test_alignment(more, paged):
-    assert taken([300], 32, 48 * HD + more, 16) == paged and taken([300], 32, 48 * HD + more, 0)
+    assert taken([300], 32, 48 * HD + more, 16) == paged and taken([600], 32, 48 * HD + more, 0)
 
 
 # rows so far apart that 32 of them, a wave's queries, leave the kernel's 32-bit offsets are the other kernel's
@@ -120,6 +121,6 @@ def test_alignment(more, paged):
 def test_rows_far_apart(block):
     from distributed_llm_inferencing_amd.ops import _native
     lib = _native.require_native()
-    assert taken([300], 4, 1 << 20, block) and not taken([300], 4, 1 << 25, block)
+    assert taken([600], 4, 1 << 20, block) and not taken([600], 4, 1 << 25, block)
     assert lib.dli_prefill_takes_wave64(4100, 1, 4100, 32, HD, 1 << 17, block)
     assert not lib.dli_prefill_takes_wave64(4100, 1, 4100, 32, HD, 1 << 25, block)

@@ -815,30 +815,41 @@ int launch_prefill32(SwaArgs a, int sh, int num_seqs, int max_seqlen, hipStream_
   DLI_RETURN_LAUNCH();
 }
 
+// How a launch's tiles are found, and its LDS
+struct Form {
+  int found, lds;
+};
 template <int DK, int DR, int DV>
-int launch_prefill32(SwaArgs a, int num_seqs, int max_seqlen, hipStream_t st) {
+Form portion_form(long k_stride, long v_stride, long k2_stride, int block_size, int window, int keep) {
   constexpr int TILES = 3 * KT * (DK + DR + DV) * 2, MOST = 160 * 1024;
-  const long list = (long)a.window + LROWS + a.keep;
-  const int bs = a.block_size;
+  const long list = (long)window + LROWS + keep;
   // Rows that lie together, by 31-bit offsets, apart from one another, and a table of the list's sixteens beside the tiles
-  // (at 128 + 128 wide it has room for 260 thousand keys). Row by row otherwise, the former way, through a table of rows
+  // (at 128 + 128 wide it has room for 260 thousand keys, at 128 + 256 for 65 thousand). Row by row otherwise, the former way, through a table of rows
   // or the block table itself, whose loads wait for all DMA in flight. That way and its mask, by runs and key by key,
   // against this one and the mask of one run, us, 32 heads of 128 on 8 with a sink and a gate a head: 5 portions of
   // 900 to 2601 tokens 285 -> 203, in windows of 1024 217 -> 171, 8000 tokens 767 -> 567 (0.92 PFLOP/s); expanded latent
   // heads, 6 of 301 to 3000 222 -> 199, in windows of 1024 187 -> 158. The mask is 13 % of the first and all of the last
   const auto fits = [](long stride, int wide) { return stride >= wide && stride < (1l << 31) / (2 * (DR ? KT : 16)); };
-  if (fits(a.k_stride, DK) && fits(a.v_stride, DV) && (DR == 0 || fits(a.k2_stride, DR))) {
-    if (DR) return launch_prefill32<DK, DR, DV, SIXTEENS>(a, TILES, num_seqs, max_seqlen, st);
+  if (fits(k_stride, DK) && fits(v_stride, DV) && (DR == 0 || fits(k2_stride, DR))) {
+    if (DR) return {SIXTEENS, TILES};
     const long sixteens = (list + 32 + 63) / KT * 4;
-    if (bs >= 16 && (bs & (bs - 1)) == 0 && TILES + sixteens * 4 <= MOST) {
-      a.block_shift = __builtin_ctz(bs);
-      return launch_prefill32<DK, DR, DV, SIXTEENS>(a, TILES + (int)sixteens * 4, num_seqs, max_seqlen, st);
-    }
+    if (block_size >= 16 && (block_size & (block_size - 1)) == 0 && TILES + sixteens * 4 <= MOST)
+      return {SIXTEENS, TILES + (int)sixteens * 4};
+  }
+  if (DR == 0 && list <= 6144 && TILES + list * 4 <= MOST) return {ROWS, TILES + (int)list * 4};
+  return {BLOCKS, TILES};
+}
+
+template <int DK, int DR, int DV>
+int launch_prefill32(SwaArgs a, int num_seqs, int max_seqlen, hipStream_t st) {
+  const Form f = portion_form<DK, DR, DV>(a.k_stride, a.v_stride, a.k2_stride, a.block_size, a.window, a.keep);
+  if (f.found == SIXTEENS) {
+    a.block_shift = __builtin_ctz(a.block_size);
+    return launch_prefill32<DK, DR, DV, SIXTEENS>(a, f.lds, num_seqs, max_seqlen, st);
   }
   if constexpr (DR == 0)
-    if (list <= 6144 && TILES + list * 4 <= MOST)
-      return launch_prefill32<DK, DR, DV, ROWS>(a, TILES + (int)list * 4, num_seqs, max_seqlen, st);
-  return launch_prefill32<DK, DR, DV, BLOCKS>(a, TILES, num_seqs, max_seqlen, st);
+    if (f.found == ROWS) return launch_prefill32<DK, DR, DV, ROWS>(a, f.lds, num_seqs, max_seqlen, st);
+  return launch_prefill32<DK, DR, DV, BLOCKS>(a, f.lds, num_seqs, max_seqlen, st);
 }
 
 template <int DK, int DV>
@@ -974,4 +985,13 @@ extern "C" int dli_swa_attention(const void* q, int ldq, const void* k, long k_s
   SWA_WIDTHS(SWA_TRY)
 #undef SWA_TRY
   return (int)hipErrorNotSupported;
+}
+
+// How portions of 192 tokens and more find their tiles: 2 by sixteens of rows, 1 by a table of rows, 0 by the block table; -1 where
+// other kernels take them
+extern "C" int dli_swa_portion_form(int dk, int dv, long k_stride, long v_stride, int block_size, int window, int keep) {
+#define SWA_FORM(K, V) if (dk == K && dv == V) return portion_form<K, 0, V>(k_stride, v_stride, 0, block_size, window, keep).found;
+  SWA_WIDTHS(SWA_FORM)
+#undef SWA_FORM
+  return -1;
 }

@@ -123,6 +123,7 @@ _SIGS = {
     # rotated designs (rotary.hip, retention.hip, swa_attention.hip)
     "dli_swa_attention": [P, I, P, L, P, L, P, I, P, P, P, I, I, I, I, I, I, I, I, I, I, F, P, I, I,
                           P, F, P, P],
+    "dli_swa_portion_form": [I, I, L, L, I, I, I],
     "dli_swa_attention_workspace_bytes": [I, I, I, I, I, I, I],
     "dli_gather_context": [P, P, I, P, P, P, P, I, I, I, I, P],
     "dli_shared_tail_attention": [P, I, P, L, I, P, L, P, L, P, L, P, I, P, P, P, I, I, I, I, I, I, I, F,

@@ -61,10 +61,22 @@ def test_widths(gpu, d, dv, window, keep):
     run(gpu, [200, 333], [10, 77], 16, window, keep, d, dv, wide=8)
 
 
-# contexts past the rows that the table beside the tiles has room for (widest: 192 KB of tiles leave none of a million keys)
+def form(block, width, window, keep, d=128, dv=128, G=2):
+    """How the kernel finds its tiles: 2 by sixteens of rows, 1 by a table of rows, 0 by the block table."""
+    from distributed_llm_inferencing_amd.ops import _native
+    return _native.require_native().dli_swa_portion_form(d, dv, G * d, G * dv, block, min(window, width * block), keep)
+
+
+# contexts past the tables beside the tiles: 6144 keys row by row (fewer at 128 + 256 wide), 65536 by sixteens at 128 + 256; and to them
 @pytest.mark.gpu
-def test_long_contexts(gpu):
-    run(gpu, [192], [70000], 16, 1 << 30, 0)
+@pytest.mark.parametrize("block,before,window,keep,d,dv,found", [
+    (16, 70000, 1 << 30, 0, 128, 128, 2), (16, 70000, 1 << 30, 0, 128, 256, 0), (256, 64000, 1 << 30, 0, 128, 256, 2), (24, 5600, 1 << 30, 0, 128, 128, 1),
+    (24, 6500, 1 << 30, 0, 128, 128, 0), (8, 7000, 1 << 30, 0, 64, 64, 0), (8, 7000, 1 << 30, 70, 96, 192, 0), (24, 9000, 6000, 20, 64, 128, 0),
+    (8, 3500, 1 << 30, 0, 128, 256, 1), (8, 4100, 1 << 30, 5, 128, 256, 0), (1, 300, 250, 40, 128, 128, 1)])
+def test_long_contexts(gpu, block, before, window, keep, d, dv, found):
+    lens = [260, 193]
+    assert form(block, -(-(before + 260) // block), window, keep, d, dv) == found
+    run(gpu, lens, [before, before // 3], block, window, keep, d, dv)
 
 
 # the expanded latent form's rows: NaN behind each sequence's, windows at every alignment

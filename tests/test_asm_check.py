@@ -50,7 +50,8 @@ def test_what_is_found(lines, ok):
 
 def test_kernels_with_asm_products_are_looked_through():
     named = {s.name for s in build._group_sources("kernels")[0] if build.has_asm_mfma(s)}
-    assert {"attention_prefill_long.hip", "gemm4w.hip", "gemm4w_narrow.hip"} <= named
+    assert {"attention_prefill_long.hip", "attention_prefill_pairs.hip", "gemm4w.hip", "gemm4w_narrow.hip", "gemm4w_rows192.hip",
+            "gemm4w_rows320.hip"} <= named
     with pytest.raises(RuntimeError, match="8 B/lane"):
         build.check_scratch("x: remark: Function Name: _Z19prefill_long_kernelILi0EEv\nx: remark: ScratchSize [bytes/lane]: 8\n", "x")
 
@@ -62,10 +63,11 @@ def assembly(name, tmp_path):
     return out.read_text()
 
 
-def test_long_attention(tmp_path):
-    text = assembly("attention_prefill_long.hip", tmp_path)
+@pytest.mark.parametrize("src", ["attention_prefill_long.hip", "attention_prefill_pairs.hip"])
+def test_long_attention(src, tmp_path):
+    text = assembly(src, tmp_path)
     assert sum(fn.name.startswith("_Z19prefill_long_kernel") for fn in asm_check.functions(text)) == 2
-    asm_check.check(text, "attention_prefill_long.hip")
+    asm_check.check(text, src)
 
 
 # hipcc does not count LDS-DMA that is asked for in asm statements: what it waits for, and where, is only its own loads' business. So

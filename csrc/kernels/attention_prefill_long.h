@@ -30,14 +30,11 @@
 // only barrier, once the last of V(t) is read, ends all three. Causal: a workgroup's tiles stop at its last row's
 // bound, a wave's at its own; only tiles that cross a wave's diagonal or the last key are masked.
 #pragma once
-#include "common.h"
+#include "lds_dma.h"
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(3))) void lds_void;
-typedef const __attribute__((address_space(1))) void gbl_void;
 typedef const __attribute__((address_space(3))) bf16x8 lds_frag;
 
 __device__ __forceinline__ float max3_raw(float a, float b, float c) {  // no canonicalise
@@ -45,9 +42,6 @@ __device__ __forceinline__ float max3_raw(float a, float b, float c) {  // no ca
   asm volatile("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
   return r;
 }
-
-// a value that is the same in all lanes, in a scalar register
-__device__ __forceinline__ uint32_t scalar(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
 
 constexpr int HD = 128, KT = 64, ROWS = 256;
 constexpr int SLOT = KT * HD * 2;                  // bytes of a K (or V) tile
@@ -150,9 +144,6 @@ __global__ void __launch_bounds__(256, 1) prefill_long_kernel(
       asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 4\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds"
                    :: "s"(dst), "i"(decltype(FURTHER)::value), "v"(lane_at), "s"(r), "s"(so) : "memory", "m0", "scc");
   };
-  auto descriptor = [&](uintptr_t base, int bytes) __attribute__((always_inline)) -> u32x4 {
-    return u32x4{scalar((uint32_t)base), scalar((uint32_t)(base >> 32) & 0xffff), scalar((uint32_t)bytes), 0x00020000};
-  };
   // a piece's descriptor, and the piece to the slot at dst - wid KiB
   auto where = [&](auto J, auto KV) __attribute__((always_inline)) -> u32x4 {
     constexpr int j = decltype(J)::value, kv = decltype(KV)::value;
@@ -161,7 +152,7 @@ __global__ void __launch_bounds__(256, 1) prefill_long_kernel(
       return u32x4{(uint32_t)__builtin_amdgcn_readlane((int)held_lo[kv], l), (uint32_t)__builtin_amdgcn_readlane((int)held_hi[kv], l),
                    (uint32_t)__builtin_amdgcn_readlane(held_bytes, l), 0x00020000};
     } else {
-      return descriptor(heads[kv], total);
+      return bytes_at(heads[kv], total);
     }
   };
   auto piece = [&](auto J, auto KV, auto BESIDE, uint32_t dst, const u32x4& r) __attribute__((always_inline)) {
@@ -184,7 +175,7 @@ __global__ void __launch_bounds__(256, 1) prefill_long_kernel(
   unroll<2>([&](auto QB) __attribute__((always_inline)) {
     constexpr int qb = decltype(QB)::value;
     const int left = min(max(len - row0[qb], 0), 32), rl = (lane & 31) >> 2;
-    const u32x4 r = descriptor((uintptr_t)(qkv + (long)(s0 + row0[qb]) * row_stride + (long)h * HD),
+    const u32x4 r = bytes_at((uintptr_t)(qkv + (long)(s0 + row0[qb]) * row_stride + (long)h * HD),
                                left > 0 ? (left - 1) * row_stride * 2 + HD * 2 : 0);
     const int at = rl * row_stride * 2 + 64 * (lane >> 5);
     const int even = at + 16 * ((lane & 3) ^ (rl >> 2)), odd = at + 16 * ((lane & 3) ^ (2 + (rl >> 2)));

@@ -269,8 +269,8 @@ __device__ __forceinline__ float pl_max3(float a, float b, float c) {  // no can
 
 // SRC: the activation's rows; cache blocks of a power of two of at least 16 tokens, whose rows lie together by sixteens
 // and are staged through scalar descriptors (lds_dma.h); other blocks, row by row, whose table every lane reads, behind
-// all DMA in flight. 2048 queries of 4096 keys 133 -> 126 us, 1024 of 6000 174 -> 163, 6 x 400 of 2400 147 -> 138. The
-// activation's rows gain nothing so (4 x 1000 62.2 and 61.9, 2048 51.4 and 51.6).
+// all DMA in flight. 6 x 400 queries of 2400 keys 147 -> 138 us. The activation's rows gain nothing so (4 x 1000 62.2 and
+// 61.9).
 // dwords: queries at addresses of whole dwords. They come, and outputs leave, through a row image a wave in LDS: row by row a lane each
 // request took 32 rows, 10 k cycles a workgroup in all. 32 heads on 8, us: 8 x 256 tokens 19.0 -> 15.4, 20 x 400 81 -> 73, 8 of
 // 300 to 2000 125 -> 114, 5 x 1500 132 -> 126, 8 x 1000 of 2000 cached 238 -> 232. Equal to the bit.
@@ -577,8 +577,8 @@ static bool wave64_reads(bool paged, long L, const void* qkv, int row_stride, in
 
 // Whether a launch takes waves of 64 rows. They gain on long sequences (2500 tokens 77 -> 69.5 us, 7993 516 -> 471, 7
 // x 2048 306 -> 291) and lose on short ones, whose last waves they leave idle (1000 tokens equal, 500 161 -> 174, 300 180
-// -> 222), and by every block, which has a CU to itself. One round of workgroups is for the other kernel, which pairs
-// blocks: 2048 51 / 58. The lengths themselves lie on the device. In the activation's rows, with T tokens, n
+// -> 222), and by every block, which has a CU to itself. (Figures of both kernels before queries and outputs passed through LDS,
+// which took 3 to 10 % of either.) Launches of up to a round of workgroups are pairs_wave64's. The lengths lie on the device. In the activation's rows, with T tokens, n
 // sequences and the longest L, the mean length over the tokens is at least low, that of n - 1 equal others; where low
 // covers a sequence's fixed cost this kernel is ahead (L = 2100 and 7 of about 1200 171 / 171, 7 of 350 76 / 80; L =
 // 4096 and 7 of 370 179 / 171; L = 2048 and 60 of 40 178 / 210), and where all the blocks find CUs, so that the longest
@@ -695,13 +695,14 @@ extern "C" int dli_prefill_set_min_len(int n) {
   return old;
 }
 
-// 1 where such a launch takes waves of 64 rows (block_size 0: keys and values in the activation's rows)
+// 1 where such a launch of more than a round of workgroups takes waves of 64 rows (block_size 0: keys and values in the
+// activation's rows); queries aligned as their stride says
 extern "C" int dli_prefill_takes_wave64(int tokens, int num_seqs, int max_seqlen, int hq, int hd, int row_stride,
                                         int block_size) {
   return takes_wave64(block_size > 0, tokens, num_seqs, max_seqlen, hq, hd, nullptr, row_stride, block_size) ? 1 : 0;
 }
 
-// 1 where it takes them in pairs of half blocks
+// 1 where a launch of up to a round takes them, in pairs of half blocks
 extern "C" int dli_prefill_pairs_wave64(int num_seqs, int max_seqlen, int hq, int hd, int row_stride, int block_size) {
   return pairs_wave64(block_size > 0, num_seqs, max_seqlen, hq, hd, nullptr, row_stride, block_size) ? 1 : 0;
 }

@@ -339,7 +339,7 @@ extern "C" int dli_mix_attention(const void* q, int ldq, const void* k, long k_s
             scale, out_scale, head_gate, (float*)ws};
   const size_t tables = (size_t)slots * 4;
   const size_t vts = (size_t)NW * TK * DVW * 2, sh = vts + (TK * TQ * PROW + H * TQ * WROW) * 2 + tables;
-  // (two value tiles a wave to windows of 4064)
+  // (two value tiles a wave to windows of 4081)
   const bool two = sh + vts <= 160 * 1024;
   static const hipError_t raised = [] {
     const hipError_t e = hipFuncSetAttribute((const void*)mix_attention_kernel<false, 1>,

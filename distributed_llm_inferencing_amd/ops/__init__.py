@@ -574,7 +574,8 @@ def prefill_long_min_len(n: int = 0) -> int:
 def prefill_wave64_min_len(n: int = 0) -> int:
     """Shortest max_seqlen whose launches of more than 256 workgroups of 256 rows take the kernel with 64 rows a
     wave; n > 0 sets it, and then whatever the other lengths are, but for the default (2048), which looks at these
-    too. Returns the previous value (A/B runs and tests)."""
+    too. Launches of up to 256 workgroups take that kernel from 600 tokens on (257 behind cached ones) with the
+    default alone, and not with any other value. Returns the previous value (A/B runs and tests)."""
     return int(N.require_native().dli_prefill_set_wave64_len(int(n)))
 
 

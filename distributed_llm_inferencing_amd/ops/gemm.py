@@ -489,15 +489,17 @@ def persistent_width(M: int, N: int, pairs: bool, cus: int = NUM_CUS) -> int:
 def row_cut(M: int, N: int, K: int) -> int:
     """Rows of a large product that run by themselves, in whole 256-row tiles, where the up to 128 rows
     past them would begin a round of the chip that they cannot fill; those then run on a streaming tile,
-    bound by the weights' read. 0: all rows together. K = 4096, fp32 outputs, us together and cut: 4104 x
-    4096 172 and 120, 8256 x 4096 265 and 212, 8199 x 16384 852 and 796, 1312 x 12288 172 and 121;
-    8199 x 28672 (SiLU pairs) 1366 and 1332; K = 14336: 8199 x 4096 907 and 710. Not where as many rounds remain: 8199
-    x 6144 is 3.09 rounds, 355 and 307, but 4104 x 6144 1.59, 181 and 193. Nor where 512 rows would remain, which
-    run on a decode step's tiles: 513 x 28672 168 and 186, 640 x 32000 187 and 217. The last round's price is
+    bound by the weights' read. 0: all rows together. Reckoned in 256 x 256 tiles, of which the last round's price is
     0.73 of a full one even if nearly empty (fewer busy CUs clock higher): 0.017 us a K on one, the other
-    side the weights at 5.5 TB/s and a launch. The rows past the cut are summed in another order than those
-    before it (each order a valid fp32 one): a token's last bits depend on which side of it the step puts
-    the token. Pinned and tuned plans apply to each part by its own rows."""
+    side the weights at 5.5 TB/s and a launch. Not where as many rounds remain: 8199 x 6144 is 3.09 rounds, 4104 x
+    6144 1.59. Nor where 512 rows would remain, which run on a decode step's tiles: 513 x 28672 168 and 186, 640 x 32000
+    187 and 217. K = 4096, us together and cut: 4104 x 4096 109 and 107, 8199 x 4096 207 and 196, 8256 x 12288 608 and
+    583, 8199 x 16384 803 and 775, 8199 x 28672 (SiLU pairs) 1302 and 1272; K = 14336: 4104 x 4096 356 and 332, 8199 x 4096
+    736 and 659. The kernel's tiles of 192 and 320 rows, which this does not know, fill some such rounds as
+    well or better: 1100 x 16384 129 and 140, 1537 x 28672 248 and 295, 3080 x 16384 313 and 329, 9220 x 28672 1440 and
+    1497; of 53 sizes it cuts 21 lose by it, 3 % in the mean, and 32 gain 4. The rows past the cut are
+    summed in another order than those before it (each order a valid fp32 one): a token's last bits depend on which
+    side of it the step puts the token. Pinned and tuned plans apply to each part by its own rows."""
     rest = M % 256
     if M - rest <= 512 or not 0 < rest <= STREAM_MAX_M or K % 64:
         return 0

@@ -77,15 +77,15 @@ static int columns(int tile_cfg, int epi, int M, int N, int splits, bool grouped
 // tiles of 256 rows leave up to a quarter of the last row of tiles or of the last round empty; tiles of 192 or 320 rows,
 // at their own price of a full round (measured as above, 16 x 16 tiles; 192 x 320 columns 0.947, x 256 0.779, x 192 0.610, x
 // 128 0.456, 320 x 192 0.935, x 128 0.675), are taken where by the same reckoning they cost 3 % less; 6 % with 8192 and
-// more of K. In launches of up to a round, or of two rows of tiles, 7 %: there few tiles share what each reads, and two shapes that
+// more of K. In launches of up to a round, or of two rows of tiles, the smaller ones 7 %: there few tiles share what each reads, and two shapes that
 // move as many bytes take as long however many products they have (so 128 columns are 8 % dearer with such K, 320 x 128
 // another 5). us, the best of 256 rows and the one taken: 2112 rows, 6144 x 4096 81 -> 77, 4096 x 4096 60 -> 55, 4096 x 14336 187 ->
 // 173, 28672 x 4096 344 -> 331; 1100 rows 4096 x 4096 44 -> 39, 4096 x 14336 137 -> 123; 600 rows 41 -> 37, 41 -> 37, 126 ->
 // 113, 118 -> 106; 5000 rows, 4096 x 14336 453 -> 406; fp32 outputs, 7623 x 12288 x 4096 562 -> 554, 8199 x 16384 x
 // 4096 844 -> 822, 9000 x 4096 x 14336 829 -> 769. Of 629 products of 260 to 16384 rows that 3 % alone would have moved, 33
 // were slower by over 1 %, by up to 14 (820 x 8192 x 5120 with SiLU pairs 60 -> 65, 640 x 14336 x 14336 229 -> 248); of the
-// 480 that this takes 3 are, by up to 3. 684 others, drawn and a grid, take 0.903 of the former time in the mean, 16 of them over
-// 1 % more, the worst 4 (520 x 11008 x 14336). Every
+// 480 that this takes 3 are, by up to 3. 1247 others, drawn and on a grid, take 0.90 of the former time in the mean, 26 of
+// them over 1 % more, the worst 6 (520 x 11008 x 11008). Every
 // shape adds a product's terms in one order, so that the choice does not change a bit. Not for short K, whose tiles are mostly
 // epilogue, nor where block maxima are laid out by the width or rows lie too far apart for 320 of them (such a
 // product is not a plain one).
@@ -101,7 +101,7 @@ static Shape shape_of(int tile_cfg, int epi, int M, int N, int K, int splits) {
   for (const auto& o : other) {
     const long rows = (M + 32 * o.mi - 1) / (32 * o.mi), cols = (N + 32 * o.nj - 1) / (32 * o.nj);
     const bool few = rows * cols * splits <= cu_count() || rows <= 2;
-    double c = cost_of(M, N, splits, o.mi, o.nj, o.price) / (few ? 0.93 : deep ? 0.94 : 0.97);
+    double c = cost_of(M, N, splits, o.mi, o.nj, o.price) / (few && o.mi * o.nj < 60 ? 0.93 : !few && deep ? 0.94 : 0.97);
     if (few && o.nj == 4) c *= (o.mi == 10 ? 1.05 : 1.0) * (deep ? 1.08 : 1.0);
     if (c < least) { least = c; best = {o.mi, o.nj}; }
   }
